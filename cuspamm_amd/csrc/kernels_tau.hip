@@ -5,144 +5,396 @@
 //    so their bit patterns order like the values; a 3-pass radix select
 //    (11 + 11 + 10 bits, most significant first) over the nbM*nbN*nbK products,
 //    recomputed from the norm maps in every pass, finds the want-th largest.
-//  - count:  number of products >= a threshold and their sum, the two
-//    quantities one round of the reference's bisection needs.
+//  - count:  number of products >= a threshold and their sum.
+//  - bisect: the reference's bisection, four of its rounds per launch: the
+//    thresholds that four rounds can visit form a binary tree of 15 nodes, one
+//    walk over the products counts all of them, and the path actually taken is
+//    followed afterwards.
+//
+// What bounds these: a selection at 2048^3 / tile 32 is 2.6e5 products, at N = 16384
+// / tile 64 1.7e7 -- a few microseconds of arithmetic -- so the time is launches,
+// round trips to memory that all CUs share, and the host's wait.  Every pass
+// therefore ends in the launch that counted: the workgroup that finishes last
+// combines the others' results and takes the pass's decision (a separate one-thread
+// walk over the 2048 bins took 30-160 us of dependent loads per pass, and
+// double-precision atomics on one address are compare-and-swap loops: 15 us of 256
+// workgroups' time at 2.6e5 products).  The decision is written straight to pinned
+// host memory, so the host waits for the stream once and copies nothing.
+// Whole calls, norm maps and the multiply behind them included: 5024 x 4128 x 3168 at
+// tile 32 to a kept fraction 667 -> 142 us, the reference's tuned 2048^3 (8 of at most
+// 20 rounds) 381 -> 118 us.
 #include "spamm_internal.h"
 
 namespace spamm {
 
-__device__ __forceinline__ uint32_t product_key(float a, float b) {
-    const float p = a * b;
-    return p > 0.0f ? __builtin_bit_cast(uint32_t, p) : 0u;       // NaN and -0 count as 0
-}
+constexpr int TAU_NTH = 1024;               // threads per workgroup
+constexpr int TAU_NW = TAU_NTH / 64;
+constexpr int TAU_MAXB = 256;               // one workgroup per CU at most: every one of them adds its part to the same few words
+constexpr int TAU_JB = 16;                  // output columns whose products share one load of nA
+constexpr int TAU_COPIES = 2;               // global copies of a histogram: workgroups that add to one copy queue on its busy bins
+constexpr int TAU_NODES = 15;               // thresholds of four rounds
 
-// Histogram of the `nbits`-wide digit at `shift` over the products whose
-// higher bits equal state->prefix.  One workgroup per (i, 16 consecutive j).
-__global__ __launch_bounds__(256) void k_tau_hist(const float *__restrict__ nA, const float *__restrict__ nBt,
-                                                  int nbM, int nbK, int nbN, int shift, int nbits, int hi_bits,
-                                                  const TauState *__restrict__ state,
-                                                  unsigned long long *__restrict__ hist) {
-    __shared__ unsigned int lh[2048];
-    const int nbins = 1 << nbits;
-    for (int b = threadIdx.x; b < nbins; b += 256) lh[b] = 0;
-    __syncthreads();
-    const int jb = (nbN + 15) / 16;
-    const int i = blockIdx.x / jb, j0 = (blockIdx.x % jb) * 16;
-    const uint32_t prefix = hi_bits ? state->prefix : 0u;
-    for (int jj = 0; jj < 16; jj++) {
-        const int j = j0 + jj;
-        if (j >= nbN) break;
-        for (int k = threadIdx.x; k < nbK; k += 256) {
-            const uint32_t key = product_key(nA[(int64_t)i * nbK + k], nBt[(int64_t)j * nbK + k]);
-            if (hi_bits == 0 || (key >> (shift + nbits)) == prefix) atomicAdd(&lh[(key >> shift) & (nbins - 1)], 1u);
-        }
+struct TauTune {
+    double norm, up, down, rate;
+    int rounds, done;
+};
+
+struct TauWorkspace {
+    TauState st;
+    TauTune tune;
+    unsigned int ticket;                    // workgroups of the running pass that have finished
+    unsigned int pad_;
+    unsigned long long zeros;               // products that are not positive
+    unsigned long long hist[3][TAU_COPIES][2048];   // one per pass: cleared together, beforehand
+    unsigned long long part[TAU_MAXB][16];  // per workgroup: counts of a pass, or {count, bits of the sum}
+};
+
+size_t tau_workspace_bytes() { return sizeof(TauWorkspace); }
+
+// Every product once: a wave takes one tile row i, 16 tile columns and 64 k, lane = k.  f(product,
+// live) runs in all lanes; `live` is false in lanes beyond the last k.  A wave's step is one round trip
+// of 17 loads and some hundred instructions, so the steps are kept small and spread over as many waves
+// as there are (whole rows of k per wave: 22 us instead of 15 for the last pass over 1.7e7 products).
+template <typename F>
+__device__ __forceinline__ void for_products(const float *__restrict__ nA, const float *__restrict__ nBt, int nbM, int nbK,
+                                             int nbN, F &&f) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int jb = (nbN + TAU_JB - 1) / TAU_JB, kb = (nbK + 63) / 64;
+    const int64_t units = (int64_t)nbM * jb * kb;
+    for (int64_t u = (int64_t)blockIdx.x * TAU_NW + wave; u < units; u += (int64_t)gridDim.x * TAU_NW) {
+        // (nbM * jb <= 65535 * 4096; the 64-bit division is a long routine that small problems need not run)
+        const int ij = units <= 0x7fffffff ? (int)u / kb : (int)(u / kb);
+        const int k0 = (int)(u - (int64_t)ij * kb) * 64;
+        const int i = ij / jb, j0 = (ij % jb) * TAU_JB;
+        const bool live = k0 + lane < nbK;
+        const int k = live ? k0 + lane : nbK - 1;
+        const float a = nA[(int64_t)i * nbK + k];
+        float b[TAU_JB];
+#pragma unroll
+        for (int jj = 0; jj < TAU_JB; jj++) b[jj] = nBt[(int64_t)(j0 + jj < nbN ? j0 + jj : nbN - 1) * nbK + k];
+#pragma unroll
+        for (int jj = 0; jj < TAU_JB; jj++)
+            if (j0 + jj < nbN) f(a * b[jj], live);
     }
-    __syncthreads();
-    for (int b = threadIdx.x; b < nbins; b += 256)
-        if (lh[b]) atomicAdd(&hist[b], (unsigned long long)lh[b]);
 }
 
-// Walks the histogram from the top bin down to the one holding the wanted
-// rank, extends the prefix, clears the histogram for the next pass.
-__global__ __launch_bounds__(256) void k_tau_pick(TauState *state, unsigned long long *hist, int nbits, int first,
-                                                  int last, unsigned long long want0) {
-    const int nbins = 1 << nbits;
+template <typename T>
+__device__ __forceinline__ T agent_load(const T *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void agent_store(T *p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// True in every thread of the workgroup that finishes last.  What workgroups hand to it goes through
+// agent-scope atomics only, which are performed where all XCDs see them: once a wave's have returned
+// (the wait on the counter) and the workgroup has met, one relaxed add on the ticket says so.  (A
+// release fence writes the XCD's whole L2 back: in every wave it took 25 us of a pass of 1100 waves,
+// in one thread per workgroup still 2.)  The ticket is put back for the next launch.
+__device__ __forceinline__ bool last_workgroup(unsigned int *ticket) {
+    __shared__ unsigned int s_last;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
     if (threadIdx.x == 0) {
-        unsigned long long want = first ? want0 : state->want;
-        if (first) state->greater = 0;
-        unsigned long long above = 0;
-        int bin = nbins - 1;
-        for (; bin > 0; bin--) {
-            if (above + hist[bin] >= want) break;
-            above += hist[bin];
-        }
-        state->greater += above;
-        state->want = want - above;           // rank inside `bin`
-        state->prefix = first ? (uint32_t)bin : ((state->prefix << nbits) | (uint32_t)bin);
-        if (last) {
-            state->tau_bits = state->prefix;
-            state->kept = state->greater + hist[bin];
-        }
+        const unsigned int t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = t == gridDim.x - 1;
+        if (s_last) agent_store(ticket, 0u);
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < nbins; b += 256) hist[b] = 0;
+    return s_last != 0;
 }
 
-// count of products with (double)p >= thr, count of products > 0, and the
-// double sum of all products (tool.cu:448-463).
-__global__ __launch_bounds__(256) void k_tau_count(const float *__restrict__ nA, const float *__restrict__ nBt,
-                                                   int nbM, int nbK, int nbN, double thr,
-                                                   unsigned long long *__restrict__ out_count,
-                                                   unsigned long long *__restrict__ out_pos,
-                                                   double *__restrict__ out_sum) {
-    __shared__ unsigned long long s_cnt, s_pos;
-    __shared__ double s_sum;
-    if (threadIdx.x == 0) { s_cnt = 0; s_pos = 0; s_sum = 0.0; }
+// One digit of the select: histogram of the PASS-th digit over the products whose higher bits equal
+// the prefix found so far, then (last workgroup) the bin that holds the wanted rank.  Zero products
+// are counted apart and never enter the histogram: sparse data would otherwise queue on one bin.
+// Neighbouring k have neighbouring exponents, so the lanes of a wave meet on few bins: four copies of
+// every bin, side by side, quarter the queue (one copy: 28 us for the first digit of 1.7e7 products).
+template <int PASS>
+__global__ __launch_bounds__(TAU_NTH) void k_tau_hist(const float *__restrict__ nA, const float *__restrict__ nBt, int nbM,
+                                                      int nbK, int nbN, unsigned long long total, unsigned long long want0,
+                                                      TauWorkspace *__restrict__ ws, TauState *__restrict__ host_out) {
+    constexpr int BITS = PASS == 2 ? 10 : 11, SHIFT = PASS == 0 ? 21 : (PASS == 1 ? 10 : 0);
+    constexpr int NB = 1 << BITS, COPIES = 4, PER = NB / TAU_NTH;
+    __shared__ unsigned int lh[NB * COPIES];
+    __shared__ unsigned long long s_sum[TAU_NW];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int b = threadIdx.x; b < NB * COPIES; b += TAU_NTH) lh[b] = 0;
     __syncthreads();
-    const int jb = (nbN + 15) / 16;
-    const int i = blockIdx.x / jb, j0 = (blockIdx.x % jb) * 16;
-    unsigned long long c = 0, pz = 0;
+    TauState prev = {};
+    if (PASS) prev = ws->st;
+    const uint32_t prefix = prev.prefix;
+    unsigned long long zeros = 0;
+    for_products(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
+        const bool pos = live && p > 0.0f;                        // NaN counts as 0
+        const uint32_t key = __builtin_bit_cast(uint32_t, p);
+        if (PASS == 0) zeros += __builtin_popcountll(__ballot(live && !(p > 0.0f)));
+        bool in = pos;
+        if constexpr (PASS > 0) in = pos && (key >> (SHIFT + BITS)) == prefix;
+        if (in) atomicAdd(&lh[((key >> SHIFT) & (NB - 1)) * COPIES + (lane & (COPIES - 1))], 1u);
+    });
+    __syncthreads();
+    for (int b = threadIdx.x; b < NB; b += TAU_NTH) {
+        unsigned long long c = 0;
+#pragma unroll
+        for (int r = 0; r < COPIES; r++) c += lh[b * COPIES + r];
+        if (c) atomicAdd(&ws->hist[PASS][blockIdx.x % TAU_COPIES][b], c);
+    }
+    if (PASS == 0 && lane == 0 && zeros) atomicAdd(&ws->zeros, zeros);
+    if (!last_workgroup(&ws->ticket)) return;
+
+    // thread t takes bins NB - 1 - t * PER downwards; `above` = products in the bins over its own.
+    // (The loads of this step are independent and go out together: a round trip that bypasses the L2
+    // is over a microsecond, and five of them one after the other were half of this kernel's time.)
+    unsigned long long h[PER], mine = 0, part[PER][TAU_COPIES];
+#pragma unroll
+    for (int e = 0; e < PER; e++)
+#pragma unroll
+        for (int r = 0; r < TAU_COPIES; r++) part[e][r] = agent_load(&ws->hist[PASS][r][NB - 1 - (int)threadIdx.x * PER - e]);
+    const unsigned long long n_zero = PASS == 0 ? agent_load(&ws->zeros) : 0ull;
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+        h[e] = 0;
+#pragma unroll
+        for (int r = 0; r < TAU_COPIES; r++) h[e] += part[e][r];
+        mine += h[e];
+    }
+    unsigned long long incl = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const unsigned long long o = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += o;
+    }
+    if (lane == 63) s_sum[wave] = incl;
+    __syncthreads();
+    unsigned long long above = incl - mine;
+    for (int w = 0; w < wave; w++) above += s_sum[w];
+    unsigned long long want = prev.want;
+    if (PASS == 0) {
+        const unsigned long long positive = total - n_zero;
+        want = want0 < positive ? want0 : positive;               // zero tail: settle for the smallest positive product
+        if (positive == 0 && threadIdx.x == 0) {                  // nothing but zeros: only tau = 0 keeps anything
+            TauState z = {};
+            z.kept = total;
+            ws->st = z;
+        }
+    }
+    if (want == 0) {                                              // (the passes after such a first one)
+        if (PASS == 2 && threadIdx.x == 0) *host_out = prev;
+        return;
+    }
+    if (above < want && want <= above + mine) {
+#pragma unroll
+        for (int e = 0; e < PER; e++) {
+            if (above < want && want <= above + h[e]) {
+                TauState st;
+                st.want = want - above;                           // rank inside the bin
+                st.greater = prev.greater + above;
+                st.prefix = (prefix << (PASS ? BITS : 0)) | (uint32_t)(NB - 1 - (int)threadIdx.x * PER - e);
+                st.tau_bits = st.prefix;
+                st.kept = st.greater + h[e];
+                ws->st = st;
+                if (PASS == 2) *host_out = st;
+            }
+            above += h[e];
+        }
+    }
+}
+
+// The two numbers that a round of the bisection starts from (tool.cu:448-463), and with `tune` its
+// first round: products with (double)p >= thr and the double sum of all products.  Sums of a
+// workgroup and of the whole are added in a fixed order: the same norm maps give the same sum.
+__global__ __launch_bounds__(TAU_NTH) void k_tau_count(const float *__restrict__ nA, const float *__restrict__ nBt, int nbM,
+                                                       int nbK, int nbN, double thr, unsigned long long total, int tune,
+                                                       double expected, double tol, int max_rounds,
+                                                       TauWorkspace *__restrict__ ws, TauCounts *__restrict__ host_out,
+                                                       TauResult *__restrict__ host_tune) {
+    __shared__ unsigned long long s_cnt[TAU_NW];
+    __shared__ double s_sum[TAU_NW];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    unsigned long long cnt = 0;
     double sum = 0.0;
-    for (int jj = 0; jj < 16; jj++) {
-        const int j = j0 + jj;
-        if (j >= nbN) break;
-        for (int k = threadIdx.x; k < nbK; k += 256) {
-            const float p = nA[(int64_t)i * nbK + k] * nBt[(int64_t)j * nbK + k];
-            if ((double)p >= thr) c++;
-            if (p > 0.0f) pz++;
-            sum += (double)p;
-        }
+    for_products(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
+        cnt += __builtin_popcountll(__ballot(live && (double)p >= thr));
+        sum += live ? (double)p : 0.0;
+    });
+    auto block_sum = [&]() {                                      // of sum and the waves' cnt, in thread 0
+        for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off, 64);
+        if (lane == 0) { s_cnt[wave] = cnt; s_sum[wave] = sum; }
+        __syncthreads();
+        cnt = 0;
+        sum = 0.0;
+        for (int w = 0; w < TAU_NW; w++) { cnt += s_cnt[w]; sum += s_sum[w]; }
+    };
+    block_sum();
+    if (threadIdx.x == 0) {
+        agent_store(&ws->part[blockIdx.x][0], cnt);
+        agent_store(&ws->part[blockIdx.x][1], __builtin_bit_cast(unsigned long long, sum));
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        c += __shfl_down(c, off, 64);
-        pz += __shfl_down(pz, off, 64);
-        sum += __shfl_down(sum, off, 64);
+    if (!last_workgroup(&ws->ticket)) return;
+    const bool have = threadIdx.x < gridDim.x;                    // gridDim.x <= TAU_MAXB <= TAU_NTH
+    cnt = have ? agent_load(&ws->part[threadIdx.x][0]) : 0ull;
+    sum = have ? __builtin_bit_cast(double, agent_load(&ws->part[threadIdx.x][1])) : 0.0;
+    for (int off = 32; off > 0; off >>= 1) cnt += __shfl_down(cnt, off, 64);
+    block_sum();
+    if (threadIdx.x != 0) return;
+    TauCounts tc;
+    tc.count = cnt;
+    tc.sum = sum;
+    *host_out = tc;
+    if (tune) {
+        TauTune t;
+        t.rate = (double)((float)cnt / (float)total);             // round 0 measures at tau = 0 ...
+        t.norm = t.up = t.down = 0.0;
+        t.done = fabs(t.rate - expected) < tol;
+        if (!t.done) t.norm = t.up = sum / (double)total;         // ... and moves to the mean product (tool.cu:445-468)
+        t.rounds = 1;
+        if (t.rounds >= max_rounds) t.done = 1;
+        ws->tune = t;
+        TauResult r = {t.norm, t.rate, t.done};
+        *host_tune = r;
     }
-    if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&s_cnt, c);
-        atomicAdd(&s_pos, pz);
-        atomicAdd(&s_sum, sum);
+}
+
+// One step of the bisection away from a measured rate (tool.cu:469-486).
+__device__ __forceinline__ void bisect_step(TauTune &t, bool above) {
+    if (above) {
+        if (t.up == t.norm) t.up *= 2;
+        t.down = t.norm;
+        t.norm = (t.norm + t.up) / 2;
+    } else {
+        t.up = t.norm;
+        t.norm = (t.norm + t.down) / 2;
+    }
+}
+
+// Four rounds of the bisection.  Node n of the tree (heap order, node 1 = the round to come) is the
+// threshold after the answers that n's bits below the leading one spell, most significant first:
+// 1 = the kept rate was above the target.  (double)p >= thr over fp32 p is p >= the smallest fp32
+// value that is not below thr.
+__global__ __launch_bounds__(TAU_NTH) void k_tau_tree(const float *__restrict__ nA, const float *__restrict__ nBt, int nbM,
+                                                      int nbK, int nbN, unsigned long long total, double expected, double tol,
+                                                      int max_rounds, TauWorkspace *__restrict__ ws,
+                                                      TauResult *__restrict__ host_tune) {
+    if (ws->tune.done) return;
+    __shared__ unsigned long long s_tot[TAU_NW][16];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float node_thr;
+    {
+        TauTune t = ws->tune;
+        const int n = (lane & 15) == 0 ? 1 : (lane & 15);
+        for (int bit = 30 - __builtin_clz(n); bit >= 0; bit--) bisect_step(t, (n >> bit) & 1);
+        node_thr = (float)t.norm;
+        if ((double)node_thr < t.norm) node_thr = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, node_thr) + 1u);   // thresholds are >= 0
+    }
+    float thr[TAU_NODES];
+    unsigned long long cnt[TAU_NODES];
+#pragma unroll
+    for (int n = 0; n < TAU_NODES; n++) {
+        thr[n] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, node_thr), n + 1));
+        cnt[n] = 0;
+    }
+    for_products(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
+        const float q = live ? p : -1.0f;
+#pragma unroll
+        for (int n = 0; n < TAU_NODES; n++) cnt[n] += __builtin_popcountll(__ballot(q >= thr[n]));
+    });
+    // workgroup totals: a wave's counts (uniform) by lane 0, then one thread per node
+#pragma unroll
+    for (int n = 0; n < TAU_NODES; n++)
+        if (lane == 0) s_tot[wave][n + 1] = cnt[n];
+    __syncthreads();
+    if (threadIdx.x >= 1 && threadIdx.x < 16) {
+        unsigned long long c = 0;
+        for (int w = 0; w < TAU_NW; w++) c += s_tot[w][threadIdx.x];
+        agent_store(&ws->part[blockIdx.x][threadIdx.x], c);
+    }
+    if (!last_workgroup(&ws->ticket)) return;
+    {
+        const int n = threadIdx.x & 15;
+        unsigned long long c = 0;
+        if (n)
+            for (unsigned b = threadIdx.x >> 4; b < gridDim.x; b += TAU_NTH / 16) c += agent_load(&ws->part[b][n]);
+        c += __shfl_xor(c, 16, 64);
+        c += __shfl_xor(c, 32, 64);
+        if (lane < 16) s_tot[wave][n] = c;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        atomicAdd(out_count, s_cnt);
-        atomicAdd(out_pos, s_pos);
-        atomicAdd(out_sum, s_sum);
+    if (threadIdx.x < 16)
+        for (int r = 1; r < TAU_NW; r++) s_tot[0][threadIdx.x] += s_tot[r][threadIdx.x];
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    TauTune t = ws->tune;
+    int n = 1;
+    for (int level = 0; level < 4 && !t.done; level++) {
+        t.rate = (double)((float)s_tot[0][n] / (float)total);
+        if (fabs(t.rate - expected) < tol) {
+            t.done = 1;
+            break;
+        }
+        const bool above = t.rate > expected;
+        bisect_step(t, above);
+        n = 2 * n + (above ? 1 : 0);
+        if (++t.rounds >= max_rounds) t.done = 1;
+    }
+    ws->tune = t;
+    TauResult r = {t.norm, t.rate, t.done};
+    *host_tune = r;
+}
+
+__global__ __launch_bounds__(256) void k_tau_clear(TauWorkspace *ws, int hist) {
+    const int b = blockIdx.x * 256 + threadIdx.x;                 // one workgroup, or 8 per histogram copy
+    if (hist) (&ws->hist[0][0][0])[b] = 0;
+    if (b == 0) {
+        ws->ticket = 0;
+        ws->zeros = 0;
     }
 }
 
-__global__ void k_tau_clear(unsigned long long *p, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0;
+static unsigned tau_grid(int64_t nbM, int64_t nbK, int64_t nbN) {
+    const int64_t units = nbM * ((nbN + TAU_JB - 1) / TAU_JB) * ((nbK + 63) / 64);
+    const int64_t blocks = (units + TAU_NW - 1) / TAU_NW;
+    return (unsigned)(blocks < TAU_MAXB ? blocks : TAU_MAXB);
 }
 
-size_t tau_workspace_bytes() { return sizeof(TauState) + 2048 * 8 + 64; }
-
-// workspace layout: [TauState][pad to 64][hist 2048 x u64][count, pos, sum]
 hipError_t launch_tau_select(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN,
-                             unsigned long long want, void *workspace, hipStream_t s) {
-    TauState *st = (TauState *)workspace;
-    unsigned long long *hist = (unsigned long long *)((char *)workspace + 64);
-    const int jb = (int)((nbN + 15) / 16);
-    const unsigned grid = (unsigned)(nbM * jb);
-    k_tau_clear<<<(2048 + 8 + 255) / 256, 256, 0, s>>>((unsigned long long *)workspace, 8 + 2048);
-    const int bits[3] = {11, 11, 10};
-    int shift = 32;
-    for (int pass = 0; pass < 3; pass++) {
-        shift -= bits[pass];
-        k_tau_hist<<<grid, 256, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, shift, bits[pass], pass, st, hist);
-        k_tau_pick<<<1, 256, 0, s>>>(st, hist, bits[pass], pass == 0, pass == 2, want);
-    }
+                             unsigned long long want, void *workspace, TauState *host_out, hipStream_t s) {
+    TauWorkspace *ws = (TauWorkspace *)workspace;
+    unsigned grid = tau_grid(nbM, nbK, nbN);
+    const unsigned long long total = (unsigned long long)nbM * nbK * nbN;
+    // a workgroup counts in 32 bits (2e9 products each is N = 262144 at tile 32)
+    if (total >> 31 > grid / 2) grid = (unsigned)(total >> 30);
+    k_tau_clear<<<3 * TAU_COPIES * 2048 / 256, 256, 0, s>>>(ws, 1);
+    k_tau_hist<0><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out);
+    k_tau_hist<1><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out);
+    k_tau_hist<2><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out);
     return hipGetLastError();
 }
 
 hipError_t launch_tau_count(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double thr,
-                            void *workspace, hipStream_t s) {
-    unsigned long long *out = (unsigned long long *)((char *)workspace + 64 + 2048 * 8);
-    const int jb = (int)((nbN + 15) / 16);
-    k_tau_clear<<<1, 256, 0, s>>>(out, 3);
-    k_tau_count<<<(unsigned)(nbM * jb), 256, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, thr, out, out + 1,
-                                                    (double *)(out + 2));
+                            void *workspace, TauCounts *host_out, hipStream_t s) {
+    TauWorkspace *ws = (TauWorkspace *)workspace;
+    k_tau_clear<<<1, 256, 0, s>>>(ws, 0);
+    k_tau_count<<<tau_grid(nbM, nbK, nbN), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, thr,
+                                                       (unsigned long long)nbM * nbK * nbN, 0, 0.0, 0.0, 0, ws, host_out, nullptr);
+    return hipGetLastError();
+}
+
+hipError_t launch_tau_tune(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double expected,
+                           double tol, int max_rounds, bool first, int passes, void *workspace, TauCounts *host_counts,
+                           TauResult *host_out, hipStream_t s) {
+    TauWorkspace *ws = (TauWorkspace *)workspace;
+    const unsigned grid = tau_grid(nbM, nbK, nbN);
+    const unsigned long long total = (unsigned long long)nbM * nbK * nbN;
+    if (first) {
+        k_tau_clear<<<1, 256, 0, s>>>(ws, 0);
+        k_tau_count<<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, 0.0, total, 1, expected, tol, max_rounds,
+                                             ws, host_counts, host_out);
+    }
+    for (int p = 0; p < passes; p++)
+        k_tau_tree<<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, expected, tol, max_rounds, ws, host_out);
     return hipGetLastError();
 }
 

@@ -38,6 +38,13 @@ struct DevBuf {
 
 }  // namespace
 
+// Pinned host memory of a context, written by kernels.
+struct HostResults {
+    TauState select;
+    TauCounts counts;
+    TauResult tune;
+};
+
 // Everything a multiply leaves behind: the shape it ran at, what is valid, and
 // the device buffers.  A context holds two of these: its own (hipMalloc'd, grown
 // on demand) and one carved out of the library's fixed device array for
@@ -80,6 +87,7 @@ struct spamm_ctx : Workspace {
 
     DevBuf staging;   // read-back staging / decay table
     DevBuf tauws;     // tau selection workspace
+    HostResults *results = nullptr;   // pinned: small results that a kernel writes and the host reads after a wait
 
     hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
     bool timing = false;        // events of the last multiply are valid
@@ -271,6 +279,7 @@ int spamm_destroy(spamm_ctx *c) {
     free_workspace(c->parked);
     if (c->staging.p) (void)hipFree(c->staging.p);
     if (c->tauws.p) (void)hipFree(c->tauws.p);
+    if (c->results) (void)hipHostFree(c->results);
     for (int i = 0; i < 5; i++)
         if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
     if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
@@ -734,13 +743,12 @@ static int tau_prepare(spamm_ctx *c, Shape *s) {
     int rc = set_device(c);
     if (rc) return rc;
     *s = shape_of(c);
+    if (!c->results) {
+        void *p = nullptr;
+        HIPCHK(c, hipHostMalloc(&p, sizeof(HostResults), hipHostMallocDefault));
+        c->results = (HostResults *)p;
+    }
     return ensure(c, c->tauws, tau_workspace_bytes());
-}
-
-static int tau_count(spamm_ctx *c, const Shape &s, double thr, TauCounts *out) {
-    HIPCHK(c, launch_tau_count((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, thr,
-                               c->tauws.p, c->stream));
-    return copy_out(c, (char *)c->tauws.p + tau_counts_offset(), out, sizeof(*out));
 }
 
 int spamm_count_kept(spamm_ctx *c, double threshold, int64_t *count_out, double *sum_out) {
@@ -748,10 +756,11 @@ int spamm_count_kept(spamm_ctx *c, double threshold, int64_t *count_out, double 
     Shape s;
     int rc = tau_prepare(c, &s);
     if (rc) return rc;
-    TauCounts tc;
-    if ((rc = tau_count(c, s, threshold, &tc))) return rc;
-    if (count_out) *count_out = (int64_t)tc.count;
-    if (sum_out) *sum_out = tc.sum;
+    HIPCHK(c, launch_tau_count((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, threshold,
+                               c->tauws.p, &c->results->counts, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (count_out) *count_out = (int64_t)c->results->counts.count;
+    if (sum_out) *sum_out = c->results->counts.sum;
     return SPAMM_OK;
 }
 
@@ -761,21 +770,13 @@ int spamm_tau_for_ratio(spamm_ctx *c, double ratio, float *tau_out, double *achi
     int rc = tau_prepare(c, &s);
     if (rc) return rc;
     const unsigned long long total = (unsigned long long)s.nbM * s.nbK * s.nbN;
-    TauCounts tc;
-    if ((rc = tau_count(c, s, 0.0, &tc))) return rc;
     double w = ceil(ratio * (double)total);
     unsigned long long want = w < 1.0 ? 1ull : (unsigned long long)w;
     if (want > total) want = total;
-    if (tc.positive == 0) {                 // nothing but zeros: only tau = 0 keeps anything
-        *tau_out = 0.0f;
-        if (achieved_out) *achieved_out = 1.0;
-        return SPAMM_OK;
-    }
-    if (want > tc.positive) want = tc.positive;     // zero tail: settle for the smallest positive product
     HIPCHK(c, launch_tau_select((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, want,
-                                c->tauws.p, c->stream));
-    TauState st;
-    if ((rc = copy_out(c, c->tauws.p, &st, sizeof(st)))) return rc;
+                                c->tauws.p, &c->results->select, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    const TauState st = c->results->select;
     memcpy(tau_out, &st.tau_bits, 4);
     if (achieved_out) *achieved_out = (double)st.kept / (double)total;
     return SPAMM_OK;
@@ -787,29 +788,20 @@ int spamm_tune_bisect(spamm_ctx *c, double expected, double tol, int max_rounds,
     Shape s;
     int rc = tau_prepare(c, &s);
     if (rc) return rc;
-    const long long total = (long long)(s.nbM * s.nbK * s.nbN);
-    double Norm = 0, up = 0, down = 0, rate = 0;
-    for (int Ti = 0; Ti < max_rounds; Ti++) {       // tool.cu:445-486
-        TauCounts tc;
-        if ((rc = tau_count(c, s, Norm, &tc))) return rc;
-        rate = (double)((float)tc.count / (float)total);
-        if (fabs(rate - expected) < tol) break;
-        if (Ti == 0) {
-            Norm = tc.sum / (double)total;
-            up = Norm;
-            continue;
-        }
-        if (rate > expected) {
-            if (up == Norm) up *= 2;
-            down = Norm;
-            Norm = (Norm + up) / 2;
-        } else {
-            up = Norm;
-            Norm = (Norm + down) / 2;
-        }
-    }
-    *tau_out = (float)Norm;
-    if (achieved_out) *achieved_out = rate;
+    // the rounds run on the device (tool.cu:445-486); the reference's 20 are one wait, beyond that the
+    // host looks every 20 whether they have ended
+    int left = (max_rounds - 1 + 3) / 4;
+    bool first = true;
+    do {
+        const int passes = left < 5 ? left : 5;
+        HIPCHK(c, launch_tau_tune((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, expected, tol,
+                                  max_rounds, first, passes, c->tauws.p, &c->results->counts, &c->results->tune, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        left -= passes;
+        first = false;
+    } while (left > 0 && !c->results->tune.done);
+    *tau_out = (float)c->results->tune.norm;
+    if (achieved_out) *achieved_out = c->results->tune.rate;
     return SPAMM_OK;
 }
 

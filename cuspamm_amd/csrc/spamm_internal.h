@@ -136,15 +136,22 @@ struct TauState {
 };
 struct TauCounts {
     unsigned long long count;     // products with (double)p >= threshold
-    unsigned long long positive;  // products > 0
     double sum;                   // sum of all products
 };
+struct TauResult {                // of the bisection so far
+    double norm, rate;
+    int done;
+};
 size_t tau_workspace_bytes();
-inline size_t tau_counts_offset() { return 64 + 2048 * 8; }
+// Results go to *host_out, pinned host memory: valid once the stream has been waited for.
 hipError_t launch_tau_select(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN,
-                             unsigned long long want, void *workspace, hipStream_t s);
+                             unsigned long long want, void *workspace, TauState *host_out, hipStream_t s);
 hipError_t launch_tau_count(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN,
-                            double thr, void *workspace, hipStream_t s);
+                            double thr, void *workspace, TauCounts *host_out, hipStream_t s);
+// the bisection: `first` starts it (its round 0), then 4 rounds per pass until done
+hipError_t launch_tau_tune(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double expected,
+                           double tol, int max_rounds, bool first, int passes, void *workspace, TauCounts *host_counts,
+                           TauResult *host_out, hipStream_t s);
 
 hipError_t gemm_init();   // one-time kernel attribute set-up
 hipError_t launch_gemm(const void *packedA, const void *packedB, const GateBuffers &g, int64_t M,

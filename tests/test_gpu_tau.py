@@ -101,3 +101,27 @@ def test_full_size_selection(orc, ctx):
     tau_o, ach_o = orc.tau_for_ratio(ctx.get_normmap(0), ctx.get_normmap(1), 0.10)
     assert np.float32(tau_g) == np.float32(tau_o) and ach_g == ach_o
     assert abs(ach_g - 0.10) < 1e-4
+
+
+@pytest.mark.parametrize("shape", [(1, 63, 16), (3, 64, 17), (2, 65, 15), (129, 65, 33), (40, 1, 300), (1, 1000, 1)])
+def test_selection_at_the_edges_of_its_work_units(orc, ctx, shape):
+    # units of 16 columns x 64 k: remainders of both, one product more or less; ties, zeros and the wanted rank
+    # at the ends of a digit's bin.  tau and kept counts are whole-number results: exact
+    rng = np.random.default_rng(sum(shape))
+    nA, nB = _maps(rng, *shape, zero_frac=0.3)
+    total = shape[0] * shape[1] * shape[2]
+    for a, b in ((nA, nB), (np.full_like(nA, 3.0), np.full_like(nB, 0.5)), (np.round(nA * 4), np.round(nB * 4))):
+        ctx.set_normmaps(a, b, 32)
+        for ratio in (1.0 / total, 0.37, 0.5, 1.0 - 1.0 / total, 1.0):
+            got, want = ctx.tau_for_ratio(ratio), orc.tau_for_ratio(a, b, ratio)
+            assert np.float32(got[0]) == np.float32(want[0]) and got[1] == want[1], (ratio, got, want)
+
+
+@pytest.mark.parametrize("rounds", [1, 2, 4, 5, 6, 9, 20, 21, 22, 45])
+def test_bisection_stops_at_any_round(orc, ctx, rounds):
+    # four rounds per launch, twenty per wait: every remainder of both, on a target that is never met (the kept
+    # fractions of 6 products are sixths), so that exactly `rounds` rounds run; sums of these values are exact
+    nA, nB = np.array([[1.0, 2.0, 4.0], [0.5, 8.0, 16.0]], np.float32), np.ones((3, 1), np.float32)
+    ctx.set_normmaps(nA, nB, 32)
+    got, want = ctx.tune_bisect(0.4, 0.01, rounds), orc.tune_bisect(nA, nB, 0.4, 0.01, rounds)
+    assert np.float32(got[0]) == np.float32(want[0]) and got[1] == want[1]
