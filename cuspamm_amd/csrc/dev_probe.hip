@@ -9,36 +9,35 @@
 namespace {
 
 // ---- matrix-pipeline ceiling: a grid of one workgroup per CU (4 waves, one per SIMD) that issues
-// nothing but independent 32x32x16 fp16 MFMAs on 16 accumulator blocks per wave.  On this part the
+// nothing but independent 16x16x32 fp16 MFMAs (the GEMM's) on 64 accumulator blocks per wave.  On this part the
 // sustained clock under MFMA load depends on the operand values (power management), so the rate
 // measured here with operands like the workload's is the ceiling a GEMM can reach, below the
 // datasheet peak.  trace[2 b] = 100 MHz wall ticks, trace[2 b + 1] = shader clocks of workgroup b.
 typedef _Float16 ceil_half8 __attribute__((ext_vector_type(8)));
-typedef float ceil_f32x16 __attribute__((ext_vector_type(16)));
+typedef float ceil_f32x4 __attribute__((ext_vector_type(4)));
 __global__ __launch_bounds__(256) void k_mfma_ceiling(const ceil_half8 *__restrict__ in, float *__restrict__ out,
                                                       unsigned long long *__restrict__ trace, int iters) {
-    ceil_half8 a[4], b[4];
-    for (int i = 0; i < 4; i++) {
-        a[i] = in[(i * 256 + threadIdx.x) % 2048];
-        b[i] = in[((i + 4) * 256 + threadIdx.x) % 2048];
+    ceil_half8 a[8], b[8];
+    for (int i = 0; i < 8; i++) {
+        a[i] = in[(i * 256 + threadIdx.x) % 4096];
+        b[i] = in[((i + 8) * 256 + threadIdx.x) % 4096];
     }
-    ceil_f32x16 acc[4][4];
-    for (int r = 0; r < 4; r++)
-        for (int c = 0; c < 4; c++)
-            for (int i = 0; i < 16; i++) acc[r][c][i] = 0.0f;
+    ceil_f32x4 acc[8][8];
+    for (int r = 0; r < 8; r++)
+        for (int c = 0; c < 8; c++) acc[r][c] = ceil_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const unsigned long long w0 = wall_clock64(), c0 = clock64();
     for (int it = 0; it < iters; it++) {
 #pragma unroll
-        for (int r = 0; r < 4; r++)
+        for (int r = 0; r < 8; r++)
 #pragma unroll
-            for (int c = 0; c < 4; c++)
-                acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[r], b[c], acc[r][c], 0, 0, 0);
+            for (int c = 0; c < 8; c++)
+                acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[r], b[c], acc[r][c], 0, 0, 0);
     }
     const unsigned long long c1 = clock64(), w1 = wall_clock64();
     float s = 0.0f;
-    for (int r = 0; r < 4; r++)
-        for (int c = 0; c < 4; c++)
-            for (int i = 0; i < 16; i++) s += acc[r][c][i];
+    for (int r = 0; r < 8; r++)
+        for (int c = 0; c < 8; c++)
+            for (int i = 0; i < 4; i++) s += acc[r][c][i];
     out[blockIdx.x * 256 + threadIdx.x] = s;
     if (threadIdx.x == 0) {
         trace[blockIdx.x * 2] = w1 - w0;
@@ -128,8 +127,8 @@ extern "C" int spamm_dev_mfma_ceiling(int device, int random_operands, int iters
     int n_wg = 0;
     DEVCHK(hipDeviceGetAttribute(&n_wg, hipDeviceAttributeMultiprocessorCount, device));
     if (n_wg <= 0 || n_wg > 4096) return -1;
-    // operands: 2048 vectors of 8 halves, zeros or uniform in [-1, 1) (a fixed LCG sequence)
-    std::vector<_Float16> h(2048 * 8);
+    // operands: 4096 vectors of 8 halves, zeros or uniform in [-1, 1) (a fixed LCG sequence)
+    std::vector<_Float16> h(4096 * 8);
     uint32_t x = 12345u;
     for (size_t i = 0; i < h.size(); i++) {
         x = x * 1664525u + 1013904223u;
@@ -156,7 +155,7 @@ extern "C" int spamm_dev_mfma_ceiling(int device, int random_operands, int iters
         best_clk = k / n_wg;
     }
     if (best_ns <= 0.0) return -1;
-    const double flops = (double)iters * 16.0 * 32768.0 * 4.0 * n_wg;   // per MFMA 2*32*32*16, 4 waves per workgroup
+    const double flops = (double)iters * 64.0 * 16384.0 * 4.0 * n_wg;   // per MFMA 2*16*16*32, 4 waves per workgroup
     *tflops = flops / best_ns * 1e-3;
     *clock_ghz = best_clk / best_ns;
     return 0;

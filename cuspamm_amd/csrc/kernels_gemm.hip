@@ -5,7 +5,7 @@
 // accumulation, ascending k.  The reference gives each 32x32 output tile its
 // own block and re-fetches both operand tiles per product (16 flop/byte).
 // Here one workgroup (4 waves, 2 x 2) owns a macro tile of 256 x 256 elements
-// of C; each wave owns a quarter of it, 128 x 128 elements (4 x 4 MFMA 32x32x16
+// of C; each wave owns a quarter of it, 128 x 128 elements (8 x 8 MFMA 16x16x32
 // accumulators = 256 fp32 registers per lane): the tiles in tile rows wr, wr + 2,
 // ... and tile columns wc, wc + 2, ... of the macro tile (for tiles of 128 that is
 // one tile).  Interleaved, because the tiles that keep a k at the edge of a band
@@ -19,7 +19,16 @@
 //
 // Operands come in the packed layout of spamm_internal.h: a tile's bytes are
 // already in MFMA operand order, so staging is a straight copy and every
-// ds_read_b128 is 512 contiguous bytes per half wave.
+// ds_read_b128 is 256 contiguous bytes per quarter wave (16 rows of one k-group).
+//
+// What bounds it: the chip's power, spent on the matrix cores, on the LDS reads and on
+// the path from L2 to LDS.  An issue loop of nothing but MFMAs on random operands runs
+// at 1.65 PFLOP/s with 32x32x16 and at 1.93 with 16x16x32 (which reads and writes half
+// the accumulator bytes per flop; on zeros both reach 2.43), hence the smaller
+// instruction; it sums the same products in the same order, C is the same bit for
+// bit.  Dense 8192^3 at tile 64: 872 us with the 32x32x16 form of this kernel,
+// 785 now (1.40 PFLOP/s); without the LDS reads 651, without the loads 663, without
+// both 536.  N = 16384, 10 % kept: 872 -> 837 us.
 #include <stdlib.h>
 
 #include <type_traits>
@@ -34,6 +43,16 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// f(integral_constant 0), ..., f(integral_constant N - 1)
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F &&f) {
+    static_for_(f, std::make_integer_sequence<int, N>{});
+}
+
 template <int B>
 struct GemmCfg {
     static constexpr int SUB = 128 / B;              // tiles per wave per dimension
@@ -45,7 +64,7 @@ struct GemmCfg {
     static constexpr int A_BYTES = MT * SLOT_BYTES;  // 256 rows x KS = 16 KiB
     static constexpr int STAGE_BYTES = 2 * A_BYTES;  // 32 KiB
     static constexpr int TILE_BYTES = B * B * 2;
-    static constexpr int RB = B / 32;                // MFMA blocks per tile per dimension
+    static constexpr int RB = B / 16;                // MFMA blocks per tile per dimension
     static constexpr int CHW = MT * CPS / 4;          // 1 KiB chunks per wave per operand per stage
     static constexpr int GS = CPS < 4 ? CPS : 4;     // chunks per load group (share a tile)
     static constexpr int NG = CHW / GS;
@@ -76,11 +95,12 @@ __device__ __forceinline__ void dma_load(const unsigned char *sbase, uint32_t vo
 }
 
 // One workgroup per macro tile.  The k loop walks stages of 32 k (a list entry
-// is B/32 stages); stage t lives in LDS buffer t % NBUF.  Ring protocol, with
-// "sync(t)" = every wave waits for its own loads of stage t+1, then a
-// workgroup barrier: after sync(t) stage t+1 is readable by all waves and no
-// wave reads stage t any more, so the loads of stage t+NBUF go into stage t's
-// buffer.  NBUF-1 stages are in flight while one is multiplied.
+// is B/32 stages); stage t lives in LDS buffer t % NBUF.  Stage t is multiplied
+// from registers that were read from LDS while stage t-1 was.  Ring protocol, with
+// "sync(t)" = every wave waits for its own loads of stage t+1 and its own LDS reads
+// of stage t, then a workgroup barrier: after sync(t) stage t+1 is readable by all
+// waves and no wave reads stage t from LDS any more, so the loads of stage t+NBUF go
+// into stage t's buffer.
 // PERSIST: the same macro tiles by workgroups that stay -- one per CU -- and take the next item of
 // their XCD's sequence from a ticket counter (what the hardware dispatcher does with one workgroup
 // per item, without ending and starting workgroups): the ticket after the current one is asked for
@@ -176,13 +196,18 @@ __global__ __launch_bounds__(256) void k_gemm(const unsigned char *__restrict__ 
     }
     if constexpr (PERSIST) tk_next = request();
 
-    f32x16 acc[4][4];
+    f32x4 acc[8][8];
 #pragma unroll
-    for (int r = 0; r < 4; r++)
+    for (int r = 0; r < 8; r++)
 #pragma unroll
-        for (int c = 0; c < 4; c++)
+        for (int c = 0; c < 8; c++) acc[r][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // The accumulators fill the accumulation registers exactly; naming them here makes the compiler
+    // keep each in one place.  (Left alone it moves some of them around in every stage, up to 200
+    // copies of them at tile 32.)
 #pragma unroll
-            for (int i = 0; i < 16; i++) acc[r][c][i] = 0.0f;
+    for (int r = 0; r < 8; r++)
+#pragma unroll
+        for (int c = 0; c < 8; c++) asm volatile("" : "+a"(acc[r][c]));
 
     {
         // ---- staging: each wave copies CHW consecutive 1 KiB chunks of the A
@@ -265,7 +290,6 @@ __global__ __launch_bounds__(256) void k_gemm(const unsigned char *__restrict__ 
             SPAMM_ISSUE(sa, 0); SPAMM_ISSUE(sa, 1); SPAMM_ISSUE(sa, 2); SPAMM_ISSUE(sa, 3);
             SPAMM_ISSUE(sa, 4); SPAMM_ISSUE(sa, 5); SPAMM_ISSUE(sa, 6); SPAMM_ISSUE(sa, 7);
         };
-        auto issue_head = [&](const StageAddr &sa) { SPAMM_ISSUE(sa, 0); SPAMM_ISSUE(sa, 1); };
         // every wave: own loads of the next stage landed and own LDS reads
         // done; then the barrier makes both true for the whole workgroup.
         // INVARIANT behind the hand-counted vmcnt: between the prologue and
@@ -283,149 +307,117 @@ __global__ __launch_bounds__(256) void k_gemm(const unsigned char *__restrict__ 
         };
 
         // LDS byte offset (inside the A or B part of a stage) of this lane's
-        // operand vector for MFMA block `blk` (32 of the wave's 128
-        // rows/columns: block blk lies in the wave's (blk * 32 / B)-th tile
-        // row/column) at k step kk (0 or 1) of the stage.
-        auto frag_off = [&](int wsel, int blk, int kk) -> int {
-            const int slot = wsel + 2 * ((blk * 32) / B);      // the wave's tile rows / columns: wsel, wsel + 2, ...
-            const int ro = (blk * 32) % B;
-            return slot * G::SLOT_BYTES + (((2 * kk + (lane >> 5)) * B) + ro + (lane & 31)) * 16;
+        // operand vector for MFMA block `blk` (16 of the wave's 128
+        // rows/columns: block blk lies in the wave's (blk * 16 / B)-th tile
+        // row/column): row lane % 16, the stage's k-group lane / 16.
+        auto frag_off = [&](int wsel, int blk) -> int {
+            const int slot = wsel + 2 * ((blk * 16) / B);      // the wave's tile rows / columns: wsel, wsel + 2, ...
+            const int ro = (blk * 16) % B;
+            return slot * G::SLOT_BYTES + ((lane >> 4) * B + ro + (lane & 15)) * 16;
         };
-        auto load_frags = [&](half8 (&af)[4], half8 (&bf)[4], int t, int kk) {
+        // operand vectors of a stage: 8 row blocks of A, 8 column blocks of B
+        struct Frags {
+            half8 a[8], b[8];
+        };
+        // read i (0..15) of a stage's vectors, in the order of their first use
+        auto load_frag = [&](Frags &f, int t, auto idx) {
+            constexpr int i = decltype(idx)::value;
             const unsigned char *bufA = smem + (t % NBUF) * G::STAGE_BYTES;
-            const unsigned char *bufB = bufA + G::A_BYTES;
-#pragma unroll
-            for (int r = 0; r < 4; r++) af[r] = *reinterpret_cast<const half8 *>(bufA + frag_off(wr, r, kk));
-#pragma unroll
-            for (int c = 0; c < 4; c++) bf[c] = *reinterpret_cast<const half8 *>(bufB + frag_off(wc, c, kk));
+            if constexpr (i == 0) f.a[0] = *reinterpret_cast<const half8 *>(bufA + frag_off(wr, 0));
+            else if constexpr (i <= 8) f.b[i - 1] = *reinterpret_cast<const half8 *>(bufA + G::A_BYTES + frag_off(wc, i - 1));
+            else f.a[i - 8] = *reinterpret_cast<const half8 *>(bufA + frag_off(wr, i - 8));
+        };
+        auto load_frags = [&](Frags &f, int t) {
+            static_for<16>([&](auto i) { load_frag(f, t, i); });
         };
 
-        // ---- prologue: stages 0..NBUF-2 and the first two loads of stage
-        // NBUF-1 (the "head"; its "tail" of six follows inside the loops, and
-        // so on for every later stage); wait for stage 0
+        // ---- prologue: stages 0..NBUF-1; wait for stage 0 and read its vectors
 #pragma unroll
-        for (int t = 0; t < NBUF - 1; t++) issue_all(stage_addr(t, stage_k(t)));
-        StageAddr sa_tail = stage_addr(NBUF - 1, stage_k(NBUF - 1));
-        issue_head(sa_tail);
-        __builtin_amdgcn_s_waitcnt(waitcnt_imm(G::LPW * (NBUF - 2) + 2, 0));
+        for (int t = 0; t < NBUF; t++) issue_all(stage_addr(t, stage_k(t)));
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm(G::LPW * (NBUF - 1), 0));
         __syncthreads();
         int t = 0;
-        // ---- loop 1: entries kept by all tiles of the macro tile; no
-        // branches.  Operand vectors are double buffered in registers (a0/b0:
-        // k step 0, a1/b1: k step 1) and every LDS read is issued 8+ MFMAs
-        // before its first use.  The sync sits in the middle of k step 1 so
-        // that the first LDS reads of the next stage overlap its second half.
-        // Global->LDS loads are spread out: one after every fourth MFMA.
-        // sched_barrier(0) pins the issue order written here.
-#define SPAMM_MFMA(A, Bv, r, c) acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[r], Bv[c], acc[r][c], 0, 0, 0)
 #define SPAMM_FENCE() __builtin_amdgcn_sched_barrier(0)
-#define SPAMM_LDA(dst, blk, kk) dst = *reinterpret_cast<const half8 *>(bufA + frag_off(wr, blk, kk))
-#define SPAMM_LDB(dst, blk, kk) dst = *reinterpret_cast<const half8 *>(bufB + frag_off(wc, blk, kk))
-        half8 a0[4], b0[4], a1[4], b1[4];
-        load_frags(a0, b0, 0, 0);
-        if (Sfull > 0) {
-            uint32_t knext = stage_k(NBUF);
-            for (; t < Sfull; t++) {
-                // address of the stage issued after this iteration's sync, computed early so that
-                // only the scalar load of the next k sits between the barrier and the MFMAs
-                const StageAddr sa_new = stage_addr(t + NBUF, knext);
-                SPAMM_FENCE();
-                {
-                    const unsigned char *bufA = smem + (t % NBUF) * G::STAGE_BYTES;
-                    const unsigned char *bufB = bufA + G::A_BYTES;
-                    // k step 0 (16 MFMA) with the 8 reads of k step 1 in between
-                    SPAMM_MFMA(a0, b0, 0, 0); SPAMM_MFMA(a0, b0, 0, 1); SPAMM_LDA(a1[0], 0, 1); SPAMM_FENCE();
-                    SPAMM_MFMA(a0, b0, 0, 2); SPAMM_MFMA(a0, b0, 0, 3); SPAMM_LDB(b1[0], 0, 1); SPAMM_FENCE();
-                    SPAMM_ISSUE(sa_tail, 2); SPAMM_FENCE();
-                    SPAMM_MFMA(a0, b0, 1, 0); SPAMM_MFMA(a0, b0, 1, 1); SPAMM_LDB(b1[1], 1, 1); SPAMM_FENCE();
-                    SPAMM_MFMA(a0, b0, 1, 2); SPAMM_MFMA(a0, b0, 1, 3); SPAMM_LDB(b1[2], 2, 1); SPAMM_FENCE();
-                    SPAMM_ISSUE(sa_tail, 3); SPAMM_FENCE();
-                    SPAMM_MFMA(a0, b0, 2, 0); SPAMM_MFMA(a0, b0, 2, 1); SPAMM_LDB(b1[3], 3, 1); SPAMM_FENCE();
-                    SPAMM_MFMA(a0, b0, 2, 2); SPAMM_MFMA(a0, b0, 2, 3); SPAMM_LDA(a1[1], 1, 1); SPAMM_FENCE();
-                    SPAMM_ISSUE(sa_tail, 4); SPAMM_FENCE();
-                    SPAMM_MFMA(a0, b0, 3, 0); SPAMM_MFMA(a0, b0, 3, 1); SPAMM_LDA(a1[2], 2, 1); SPAMM_FENCE();
-                    SPAMM_MFMA(a0, b0, 3, 2); SPAMM_MFMA(a0, b0, 3, 3); SPAMM_LDA(a1[3], 3, 1); SPAMM_FENCE();
-                    SPAMM_ISSUE(sa_tail, 5); SPAMM_FENCE();
-                    // first half of k step 1
-                    SPAMM_MFMA(a1, b1, 0, 0); SPAMM_MFMA(a1, b1, 0, 1); SPAMM_MFMA(a1, b1, 0, 2); SPAMM_MFMA(a1, b1, 0, 3);
-                    SPAMM_FENCE();
-                    SPAMM_ISSUE(sa_tail, 6); SPAMM_FENCE();
-                    SPAMM_MFMA(a1, b1, 1, 0); SPAMM_MFMA(a1, b1, 1, 1); SPAMM_MFMA(a1, b1, 1, 2); SPAMM_MFMA(a1, b1, 1, 3);
-                    SPAMM_FENCE();
-                    SPAMM_ISSUE(sa_tail, 7); SPAMM_FENCE();
-                }
-                sync_next();
-                SPAMM_FENCE();
-                // scalar load placed here so that no LDS wait follows it closely
-                knext = stage_k(t + 1 + NBUF);
-                sa_tail = sa_new;
-                SPAMM_FENCE();
-                {
-                    const unsigned char *bufA = smem + ((t + 1) % NBUF) * G::STAGE_BYTES;
-                    const unsigned char *bufB = bufA + G::A_BYTES;
-                    // second half of k step 1 with the 8 reads of the next stage's k step 0
-                    SPAMM_MFMA(a1, b1, 2, 0); SPAMM_LDA(a0[0], 0, 0); SPAMM_FENCE();
-                    SPAMM_ISSUE(sa_tail, 0); SPAMM_FENCE();
-                    SPAMM_MFMA(a1, b1, 2, 1); SPAMM_LDB(b0[0], 0, 0); SPAMM_FENCE();
-                    SPAMM_MFMA(a1, b1, 2, 2); SPAMM_LDB(b0[1], 1, 0); SPAMM_FENCE();
-                    SPAMM_MFMA(a1, b1, 2, 3); SPAMM_LDB(b0[2], 2, 0); SPAMM_FENCE();
-                    SPAMM_MFMA(a1, b1, 3, 0); SPAMM_LDB(b0[3], 3, 0); SPAMM_FENCE();
-                    SPAMM_ISSUE(sa_tail, 1); SPAMM_FENCE();
-                    SPAMM_MFMA(a1, b1, 3, 1); SPAMM_LDA(a0[1], 1, 0); SPAMM_FENCE();
-                    SPAMM_MFMA(a1, b1, 3, 2); SPAMM_LDA(a0[2], 2, 0); SPAMM_FENCE();
-                    SPAMM_MFMA(a1, b1, 3, 3); SPAMM_LDA(a0[3], 3, 0); SPAMM_FENCE();
-                }
-            }
+        Frags f0, f1;
+        load_frags(f0, 0);
+        // ---- loop 1: entries kept by all tiles of the macro tile; no branches.  One stage = one k step of
+        // 64 MFMAs on the vectors that the stage before has read; meanwhile the next stage's 16 vectors are
+        // read (one after every third MFMA, so that the last is there before the sync) and the 8 loads of
+        // the stage that takes over this stage's buffer are issued (one after every eighth).
+        // sched_barrier(0) pins the order written here.
+        uint32_t knext = stage_k(NBUF);
+        auto full_stage = [&](const Frags &cur, Frags &nxt) {
+            sync_next();
+            const StageAddr sa = stage_addr(t + NBUF, knext);
+            knext = stage_k(t + 1 + NBUF);
+            SPAMM_FENCE();
+            static_for<64>([&](auto idx) {
+                constexpr int i = decltype(idx)::value, r = i / 8, c = i % 8, read = i / 3;
+                acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cur.a[r], cur.b[c], acc[r][c], 0, 0, 0);
+                if constexpr (i % 3 == 0 && read < 16) { load_frag(nxt, t + 1, std::integral_constant<int, read>{}); SPAMM_FENCE(); }
+                if constexpr (i % 8 == 4) { issue_one(sa, std::integral_constant<int, i / 8>{}); SPAMM_FENCE(); }
+            });
+            SPAMM_FENCE();
+            t++;
+        };
+        // (two at a time, one per register set; an odd last one -- tile 32 only -- is left to loop 2,
+        // which takes it as an entry whose bits are all set)
+        while (__builtin_expect(t + 1 < Sfull, 1)) {
+            full_stage(f0, f1);
+            full_stage(f1, f0);
         }
         // ---- loop 2: entries kept by some tiles only; a wave multiplies
-        // exactly the (tile row, tile column) pairs whose bit is set.  Same
-        // register double buffering as loop 1: on entry a0/b0 hold k step 0
-        // of stage t; k step 1 is read while step 0 multiplies, and the next
-        // stage's step 0 (readable after the sync) while step 1 multiplies.
-        auto mul_kept = [&](const half8 (&af)[4], const half8 (&bf)[4], uint32_t sb) {
+        // exactly the (tile row, tile column) pairs whose bit is set.
+        // Pairs are walked in chunks, with the next stage's reads and the issued stage's loads shared
+        // out behind the chunks, so that neither waits for all of the other.
+        constexpr int NP = G::SUB * G::SUB, NCH = NP < 4 ? 4 : NP;      // chunks per stage
+        auto mul_chunk = [&](const Frags &f, auto chunk) {
+            constexpr int ch = decltype(chunk)::value, pr = ch * NP / NCH, sub = ch % (NCH / NP);
+            constexpr int a = pr / G::SUB, b = pr % G::SUB, RR = G::RB / (NCH / NP);
 #pragma unroll
-            for (int a = 0; a < G::SUB; a++)
+            for (int r = sub * RR; r < (sub + 1) * RR; r++)
 #pragma unroll
-                for (int b = 0; b < G::SUB; b++) {
-                    if ((sb >> (a * G::SUB + b)) & 1u) {
-#pragma unroll
-                        for (int r = 0; r < G::RB; r++)
-#pragma unroll
-                            for (int c = 0; c < G::RB; c++)
-                                acc[a * G::RB + r][b * G::RB + c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                                    af[a * G::RB + r], bf[b * G::RB + c], acc[a * G::RB + r][b * G::RB + c], 0, 0, 0);
-                    }
-                }
+                for (int c = 0; c < G::RB; c++)
+                    acc[a * G::RB + r][b * G::RB + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                        f.a[a * G::RB + r], f.b[b * G::RB + c], acc[a * G::RB + r][b * G::RB + c], 0, 0, 0);
         };
-        uint32_t need_tail = 0xffffu;     // the stage whose head was issued by loop 1 / the prologue: all slots
-        for (; t < S; t++) {
-            const uint64_t kn = stage_kn(t + NBUF);
-            SPAMM_ISSUE_N(sa_tail, need_tail, 2); SPAMM_ISSUE_N(sa_tail, need_tail, 3); SPAMM_ISSUE_N(sa_tail, need_tail, 4);
-            SPAMM_ISSUE_N(sa_tail, need_tail, 5); SPAMM_ISSUE_N(sa_tail, need_tail, 6); SPAMM_ISSUE_N(sa_tail, need_tail, 7);
-            const u32x4 cur = ents[t / G::NSPE];
-            const uint64_t mask = ((uint64_t)cur.w << 32) | cur.z;
-            uint32_t sb = 0;
-#pragma unroll
-            for (int a = 0; a < G::SUB; a++)
-#pragma unroll
-                for (int b = 0; b < G::SUB; b++) {
-                    const int bit = (wr + 2 * a) * G::MT + wc + 2 * b;
-                    sb |= (uint32_t)((mask >> bit) & 1ull) << (a * G::SUB + b);
-                }
-            load_frags(a1, b1, t, 1);
-            mul_kept(a0, b0, sb);
+        // the tile bits of an entry (an 8-byte scalar load of exactly the words that are used: a load
+        // with a dead word makes the next writer of that register wait for it)
+        auto stage_mask = [&](int t) -> uint64_t {
+            const int tc = t < S ? t : S - 1;
+            return *(entry_kn_ptr)(uintptr_t)(reinterpret_cast<const unsigned char *>(macro_list + (int64_t)macro * nbK + tc / G::NSPE) + 8);
+        };
+        uint64_t kn = stage_kn(t + NBUF), mask = stage_mask(t);
+        auto partial_stage = [&](const Frags &cur, Frags &nxt) {
             sync_next();
-            sa_tail = stage_addr(t + NBUF, (uint32_t)kn);
+            // tile pairs of this wave that the stage's entry keeps (none beyond the last stage)
+            const uint64_t mk = t < S ? mask >> (wr * G::MT + wc) : 0ull;
+            const StageAddr sa = stage_addr(t + NBUF, (uint32_t)kn);
             // stages past the end repeat the last entry and are never read: nothing to fetch
-            need_tail = t + NBUF < S ? (uint32_t)(kn >> 32) : 0u;
-            SPAMM_ISSUE_N(sa_tail, need_tail, 0); SPAMM_ISSUE_N(sa_tail, need_tail, 1);
-            load_frags(a0, b0, t + 1, 0);
-            mul_kept(a1, b1, sb);
+            const uint32_t need = t + NBUF < S ? (uint32_t)(kn >> 32) : 0u;
+            kn = stage_kn(t + 1 + NBUF);
+            mask = stage_mask(t + 1);
+            SPAMM_FENCE();
+            static_for<NCH>([&](auto chunk) {
+                constexpr int ch = decltype(chunk)::value, pr = ch * NP / NCH;
+                constexpr int bit = 2 * (pr / G::SUB) * G::MT + 2 * (pr % G::SUB), per = 32 / NCH;
+                if ((mk >> bit) & 1ull) mul_chunk(cur, chunk);
+                SPAMM_FENCE();
+                static_for<per>([&](auto j) {                       // the 16 reads, behind the first half of the chunks
+                    constexpr int i = ch * per + decltype(j)::value;
+                    if constexpr (i < 16) load_frag(nxt, t + 1, std::integral_constant<int, i>{});
+                });
+                if constexpr (NCH == 4) { SPAMM_ISSUE_N(sa, need, 2 * ch); SPAMM_ISSUE_N(sa, need, 2 * ch + 1); }
+                else if constexpr (ch % 2 == 0) SPAMM_ISSUE_N(sa, need, ch / 2);
+                SPAMM_FENCE();
+            });
+            t++;
+        };
+        while (__builtin_expect(t < S, 1)) {
+            partial_stage(f0, f1);
+            partial_stage(f1, f0);
         }
-#undef SPAMM_MFMA
 #undef SPAMM_FENCE
-#undef SPAMM_LDA
-#undef SPAMM_LDB
 #undef SPAMM_ISSUE
 #undef SPAMM_ISSUE_N
         // the ring still holds clamped loads: let them land before the
@@ -436,26 +428,36 @@ __global__ __launch_bounds__(256) void k_gemm(const unsigned char *__restrict__ 
     if constexpr (PERSIST) q_next = publish(tk_next);
 
     // ---- epilogue: C[row, col], row-major, ld N (cuSpAMM.cu:391).  MFMA
-    // 32x32 result register i of lane l is row 8*(i/4) + 4*(l/32) + i%4,
-    // column l%32 of the block: every store instruction writes two full
-    // 128-byte row segments.  C is written once and not read again here:
-    // non-temporal stores leave the L2 to the operand panels.  (Swapping the
-    // MFMA operands would give float4 stores, but each then touches 32 rows
-    // with 32 bytes -- measured slower.)
+    // 16x16 result register i of lane l is row 4*(l/16) + i, column l%16 of the
+    // block.  Stored as they are (or, with the MFMA operands swapped, as float4)
+    // the results leave in 64-byte row segments, which costs more than the smaller
+    // instruction gains (N = 16384, 10 % kept: 881 us).  So the odd 16-lane rows of a
+    // column block's register are swapped with the even ones of its right neighbour's:
+    // each register is then two rows of 32 columns, two full 128-byte segments per
+    // store.  C is written once and not read again here: non-temporal stores leave
+    // the L2 to the operand panels.  The stores are written out because the compiler
+    // gives each a 64-bit vector address of its own.
     int lane_e = lane;
     if constexpr (PERSIST) asm volatile("" : "+v"(lane_e));     // (as in zero_fill)
+    const uint32_t lane_off = (uint32_t)(32 * (lane_e >> 5)) * (uint32_t)N + 4 * (lane_e & 31);     // bytes
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int64_t row0 = (int64_t)mi * 256 + (wr + 2 * (r / G::RB)) * B + (r % G::RB) * 32;
+    for (int r = 0; r < 8; r++) {
+        const int64_t row0 = (int64_t)mi * 256 + (wr + 2 * (r / G::RB)) * B + (r % G::RB) * 16;
         if (row0 >= M) continue;
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const int64_t col0 = (int64_t)mj * 256 + (wc + 2 * (c / G::RB)) * B + (c % G::RB) * 32;
+        for (int c = 0; c < 8; c += 2) {
+            const int64_t col0 = (int64_t)mj * 256 + (wc + 2 * (c / G::RB)) * B + (c % G::RB) * 16;
             if (col0 >= N) continue;
-            float *out = C + (row0 + 4 * (lane_e >> 5)) * N + col0 + (lane_e & 31);
+            asm volatile("" : "+a"(acc[r][c]), "+a"(acc[r][c + 1]));      // (keeps the results where they are until here)
 #pragma unroll
-            for (int i = 0; i < 16; i++)
-                __builtin_nontemporal_store(acc[r][c][i], &out[(int64_t)(8 * (i / 4) + (i % 4)) * N]);
+            for (int i = 0; i < 4; i++) {
+                const float x = acc[r][c][i], y = acc[r][c + 1][i];
+                const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+                float *out = C + (row0 + i) * N + col0;
+                asm volatile("global_store_dword %0, %1, %2 nt" :: "v"(lane_off), "v"(sw[0]), "s"(out) : "memory");
+                asm volatile("global_store_dword %0, %1, %2 nt" :: "v"(lane_off), "v"(sw[1]), "s"(out + 4 * N) : "memory");
+            }
+            __builtin_amdgcn_sched_barrier(0);      // (or all 256 results are moved to vector registers first)
         }
     }
     if constexpr (!PERSIST) return;
@@ -716,9 +718,9 @@ __global__ __launch_bounds__(128 * NWR, NWR == 2 ? 2 : 1) void k_gemm_w64(const 
 #pragma unroll
                         for (int r = 0; r < H::RBR; r++)
 #pragma unroll
-                            for (int c = 0; c < G::RB; c++)
-                                acc[a * H::RBR + r][b * G::RB + c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                                    af[a * H::RBR + r], bf[b * G::RB + c], acc[a * H::RBR + r][b * G::RB + c], 0, 0, 0);
+                            for (int c = 0; c < (B / 32); c++)
+                                acc[a * H::RBR + r][b * (B / 32) + c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                                    af[a * H::RBR + r], bf[b * (B / 32) + c], acc[a * H::RBR + r][b * (B / 32) + c], 0, 0, 0);
                     }
                 }
         };

@@ -14,7 +14,7 @@ namespace spamm {
 // of B) and contraction index k (column of A / row of B) sits at
 //     ((k / 8) * b + r) * 8 + (k % 8)          [units: halves]
 // i.e. [k-group][r][8]: a 16-byte vector holds 8 consecutive k of one r, which
-// is exactly one lane's share of an MFMA 32x32x16 operand, and 32 consecutive
+// is exactly one lane's share of an MFMA 16x16x32 (or 32x32x16) operand, and 32 consecutive
 // r are 512 contiguous bytes.  Tile order: A tile (I,Kt) at I*nbK + Kt,
 // B tile (Kt,J) at J*nbK + Kt, so that the k tiles of one output tile are
 // consecutive in memory for both operands.

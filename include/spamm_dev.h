@@ -22,7 +22,7 @@ extern "C" {
 #endif
 
 /* The rate the matrix pipeline of `device` sustains when every CU issues
- * nothing but independent fp16 32x32x16 MFMAs (iters x 16 per wave, one wave
+ * nothing but independent fp16 16x16x32 MFMAs (iters x 64 per wave, one wave
  * per SIMD), with all-zero operands (random_operands = 0) or uniform [-1,1)
  * operands (1).  The sustained clock under MFMA load depends on the operand
  * values, so the second figure is the ceiling a GEMM on real data can
