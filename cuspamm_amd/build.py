@@ -14,7 +14,7 @@ LIB_PATH = os.path.join(HERE, "libspamm_gfx950.so")
 DEV_LIB_PATH = os.path.join(HERE, "libspamm_dev_gfx950.so")   # measurement aids (csrc/dev_probe.hip), not the engine
 MAIN_PATH = os.path.join(HERE, "spamm_main")     # the reference's main() on top of the C ABI (csrc/spamm_main.cpp)
 
-SOURCES = ["kernels_normmap.hip", "kernels_gate.hip", "kernels_gemm.hip", "kernels_tau.hip", "kernels_tools.hip",
+SOURCES = ["kernels_normmap.hip", "kernels_gate.hip", "kernels_gemm.hip", "kernels_small.hip", "kernels_tau.hip", "kernels_tools.hip",
            "spamm_api.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -33,7 +33,7 @@ CFLAGS = [
 ]
 
 
-# kernels_gemm.hip only.  M0 is listed as clobbered by its global->LDS loads and clang remarks on every
+# The multiply kernels.  M0 is listed as clobbered by its global->LDS loads and clang remarks on every
 # instance that M0 is reserved (it never allocates it anyway).  The ticket of the workgroups that stay is
 # drawn by one lane with a returning atomic that is asked for early and looked at late; the compiler's
 # rewrite of atomics in divergent code (one lane adds for all, then a broadcast) would wait for it at once.
@@ -61,7 +61,7 @@ def _check_no_scratch(log, src):
         if m:
             name = m.group(1)
         m = re.search(r"ScratchSize \[bytes/lane\]: (\d+)", line)
-        if m and name and "k_gemm" in name and int(m.group(1)) != 0:
+        if m and name and ("k_gemm" in name or "k_small" in name) and int(m.group(1)) != 0:
             raise RuntimeError("%s: kernel %s spills %s bytes/lane to scratch" % (src, name, m.group(1)))
 
 
@@ -73,7 +73,7 @@ def build_library(verbose=False):
 
     def compile_one(pair):
         src, obj = pair
-        extra = ["-Rpass-analysis=kernel-resource-usage"] + GEMM_FLAGS if src == "kernels_gemm.hip" else []
+        extra = ["-Rpass-analysis=kernel-resource-usage"] + GEMM_FLAGS if src in ("kernels_gemm.hip", "kernels_small.hip") else []
         log = _run([HIPCC] + CFLAGS + extra + ["-c", os.path.join(CSRC, src), "-o", obj])
         if extra:
             _check_no_scratch(log, src)

@@ -20,9 +20,7 @@
 // The reference's compacted per-tile list (offset[], :315-325) is the bitmap's
 // set bits in ascending order; nothing downstream reads it, so it is produced
 // from the bitmap only when asked for (k_klist).
-#include <type_traits>
-
-#include "spamm_internal.h"
+#include "gemm_device.h"
 
 namespace spamm {
 
@@ -297,12 +295,7 @@ __global__ __launch_bounds__(NTH) void k_gate(GateBuffers g, int nbM, int nbK, i
     // tile run together on one XCD, and walking k from a common start keeps
     // them on the same A row panels and B column panels at the same time.
     {
-        const int sm = mi / SUPER_M, sn = mj / SUPER_N;
-        const float ic = ((sm * SUPER_M + 0.5f * SUPER_M) * MT) / (float)nbM;
-        const float jc = ((sn * SUPER_N + 0.5f * SUPER_N) * MT) / (float)nbN;
-        const float fa = 0.5f * (ic + jc) * (float)nbK - 0.5f * SUPER_N * MT;
-        int anchor = (int)fa;
-        anchor = anchor < 0 ? 0 : (anchor > nbK - 1 ? nbK - 1 : anchor);
+        const int anchor = list_anchor(mi, mj, MT, nbM, nbK, nbN);
         const int wa = anchor >> 6, ba = anchor & 63;
         const uint64_t u = luf[2 * wa], f = luf[2 * wa + 1];
         const uint64_t below = (1ull << ba) - 1ull;

@@ -31,27 +31,9 @@
 // both 536.  N = 16384, 10 % kept: 872 -> 837 us.
 #include <stdlib.h>
 
-#include <type_traits>
-#include <utility>
-
-#include "spamm_internal.h"
+#include "gemm_device.h"
 
 namespace spamm {
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// f(integral_constant 0), ..., f(integral_constant N - 1)
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_(F &&f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F &&f) {
-    static_for_(f, std::make_integer_sequence<int, N>{});
-}
 
 template <int B>
 struct GemmCfg {
@@ -70,29 +52,6 @@ struct GemmCfg {
     static constexpr int NG = CHW / GS;
     static constexpr int LPW = 2 * CHW;              // load instructions per wave per stage
 };
-
-// s_waitcnt immediates (gfx9 encoding: vmcnt [3:0]+[15:14], expcnt [6:4], lgkmcnt [11:8])
-constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | 0x70 | ((lgkm & 15) << 8); }
-
-// One 1 KiB wave-load straight from global memory into LDS: lane l's 16 bytes
-// land at lds_addr + IMM + 16*l, read from sbase + IMM + voff (the instruction
-// offset applies to the global and to the LDS address alike).  Written as
-// inline assembly so that the compiler's wait-count insertion does not see an
-// LDS write it cannot disambiguate (it would put a full vmcnt(0) wait before
-// every LDS read and serialise the staging ring); completion is awaited
-// explicitly with s_waitcnt vmcnt before the workgroup barrier.  M0 carries
-// the LDS address and is declared clobbered, so the compiler keeps nothing
-// live in it across a load.  Both scalar operands must come from scalar
-// instructions (as all callers' do): a VALU-written SGPR (v_readfirstlane)
-// read by a vector-memory instruction within five instructions is a hazard
-// the compiler does not see inside inline assembly.
-template <int IMM>
-__device__ __forceinline__ void dma_load(const unsigned char *sbase, uint32_t voff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:%3"
-                 :
-                 : "s"(lds_addr), "v"(voff), "s"(sbase), "n"(IMM)
-                 : "memory", "m0");
-}
 
 // One workgroup per macro tile.  The k loop walks stages of 32 k (a list entry
 // is B/32 stages); stage t lives in LDS buffer t % NBUF.  Stage t is multiplied

@@ -58,13 +58,24 @@ __device__ __forceinline__ float butterfly64(float v) {
 //           canonical reduction.
 // (The phased fp32 A role is held to three waves per SIMD: it gains more from a third resident
 // workgroup than it loses to a few spilled registers; the B role would spill far more.)
-template <int B, int ROLE, int SW, bool IN16, int PH = 1, int NWV = 4>
-__global__ __launch_bounds__(64 * NWV, (PH > 1 && ROLE == 0 && !IN16 && NWV == 4) ? 3 : 1) void k_normmap(const void *__restrict__ Xv, int64_t ld, int64_t cols,
-                                                 int64_t nbr, int64_t nbc, int64_t nstrip,
-                                                 uint4 *__restrict__ packed, float *__restrict__ nm,
-                                                 float *__restrict__ nmT, uint4 *__restrict__ packed2,
-                                                 float *__restrict__ nm2, const float *__restrict__ rowmax,
-                                                 float tau_skip) {
+template <int B, int SW, int PH>
+struct NormCfg {
+    static constexpr int TPP = SW / B / PH;          // tiles resident in LDS together
+    static constexpr int QN = B / 8;                 // k-groups per tile
+    static constexpr int QS = B * 16 + 16;           // bytes per k-group segment in LDS (padded)
+    static constexpr int TS = QN * QS;               // bytes per tile in LDS
+    static constexpr int PITCH = QN + 1;             // padded row of the chunk-sum table
+    static constexpr int CH = B * PITCH;             // floats per tile in the chunk-sum table
+};
+
+// `strip`: which strip of the operand; s_pack / s_chunk / s_skip: NormCfg's TPP * TS bytes, TPP * CH floats, TPP ints of LDS
+template <int B, int ROLE, int SW, bool IN16, int PH, int NWV>
+__device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64_t ld, int64_t cols, int64_t nbr, int64_t nbc,
+                                              int64_t nstrip, uint4 *__restrict__ packed, float *__restrict__ nm,
+                                              float *__restrict__ nmT, uint4 *__restrict__ packed2, float *__restrict__ nm2,
+                                              const float *__restrict__ rowmax, float tau_skip, unsigned strip,
+                                              unsigned char *s_pack, float *s_chunk, int *s_skip) {
+    using L = NormCfg<B, SW, PH>;
     constexpr int TPS = SW / B;           // tiles per strip
     constexpr int TPP = TPS / PH;         // tiles per phase (resident in LDS together)
     static_assert(TPP * PH == TPS && TPP >= 1, "phases must divide the strip's tiles");
@@ -79,21 +90,14 @@ __global__ __launch_bounds__(64 * NWV, (PH > 1 && ROLE == 0 && !IN16 && NWV == 4
     constexpr int GSTEP = NWV;                         // 8-row groups between a lane's groups (one per wave)
     static_assert(B % (8 * NWV) == 0, "every wave takes whole 8-row groups");
     static_assert(PH == 1 || PH == 2 || PH == 4, "phases are made of whole waves");
-    constexpr int QN = B / 8;             // k-groups per tile
+    constexpr int QN = L::QN, QS = L::QS, TS = L::TS, PITCH = L::PITCH, CH = L::CH;
     constexpr int VPT = B * B / 8;        // 16-byte vectors per tile
-    constexpr int QS = B * 16 + 16;       // bytes per k-group segment in LDS (padded)
-    constexpr int TS = QN * QS;           // bytes per tile in LDS
-    constexpr int PITCH = QN + 1;         // padded row of the chunk-sum table
-    constexpr int CH = B * PITCH;         // floats per tile in the chunk-sum table
     constexpr int NGW = B / (8 * GSTEP);  // 8-row groups per lane
     constexpr int STEPS = VPT / 64;
-    __shared__ __attribute__((aligned(16))) unsigned char s_pack[TPP * TS];
-    __shared__ float s_chunk[TPP * CH];
-
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    const int64_t I = blockIdx.x / nstrip;            // tile row of the strip
-    const int64_t sc = blockIdx.x % nstrip;
+    const int64_t I = strip / nstrip;                 // tile row of the strip
+    const int64_t sc = strip % nstrip;
     const int64_t col0 = sc * SW;
     const int cl = EPL * lane;                        // first column of this lane inside the strip
     const int g0 = wave;                              // first 8-row group of this lane; then every GSTEP-th
@@ -245,7 +249,6 @@ __global__ __launch_bounds__(64 * NWV, (PH > 1 && ROLE == 0 && !IN16 && NWV == 4
         }
     };
     // packed tiles out (256 threads x 16 bytes = 4 KiB per step, contiguous per tile)
-    __shared__ int s_skip[TPP];
     auto copy_out = [&](int ph, bool as_b, uint4 *__restrict__ pk, bool prune) {
 #pragma unroll
         for (int i = 0; i < TPP * VPT / (64 * NWV); i++) {
@@ -314,6 +317,43 @@ __global__ __launch_bounds__(64 * NWV, (PH > 1 && ROLE == 0 && !IN16 && NWV == 4
         __syncthreads();
         emit_role(true, packed2, nm2, nmT, prune);
     }
+}
+
+template <int B, int ROLE, int SW, bool IN16, int PH = 1, int NWV = 4>
+__global__ __launch_bounds__(64 * NWV, (PH > 1 && ROLE == 0 && !IN16 && NWV == 4) ? 3 : 1) void k_normmap(
+    const void *__restrict__ Xv, int64_t ld, int64_t cols, int64_t nbr, int64_t nbc, int64_t nstrip, uint4 *__restrict__ packed,
+    float *__restrict__ nm, float *__restrict__ nmT, uint4 *__restrict__ packed2, float *__restrict__ nm2,
+    const float *__restrict__ rowmax, float tau_skip, int64_t *__restrict__ kept) {
+    using L = NormCfg<B, SW, PH>;
+    __shared__ __attribute__((aligned(16))) unsigned char s_pack[L::TPP * L::TS];
+    __shared__ float s_chunk[L::TPP * L::CH];
+    __shared__ int s_skip[L::TPP];
+    // (the multiply's kept-product total, which k_small adds to: cleared by the passes that run before it)
+    if (blockIdx.x == 0 && threadIdx.x == 0) *kept = 0;
+    normmap_strip<B, ROLE, SW, IN16, PH, NWV>(Xv, ld, cols, nbr, nbc, nstrip, packed, nm, nmT, packed2, nm2, rowmax, tau_skip,
+                                              blockIdx.x, s_pack, s_chunk, s_skip);
+}
+
+// Both operands in one launch: the first n_b workgroups are B's strips, the others A's.  One after the other,
+// small passes are a few microseconds of memory latency each; together they share it (and neither sees the
+// other's norms: a tau-aware call then leaves out tiles of norm zero only, in both copies).
+template <int B, int SW, bool IN16, int PH, int NWV>
+__global__ __launch_bounds__(64 * NWV) void k_normmap_pair(const void *__restrict__ A, const void *__restrict__ Bm, int64_t nbM,
+                                                           int64_t nbK, int64_t nbN, unsigned n_b, int64_t strips_a, int64_t strips_b,
+                                                           uint4 *__restrict__ packedA, uint4 *__restrict__ packedB,
+                                                           float *__restrict__ nmA, float *__restrict__ nmB,
+                                                           float *__restrict__ nmBt, float tau_skip, int64_t *__restrict__ kept) {
+    using L = NormCfg<B, SW, PH>;
+    __shared__ __attribute__((aligned(16))) unsigned char s_pack[L::TPP * L::TS];
+    __shared__ float s_chunk[L::TPP * L::CH];
+    __shared__ int s_skip[L::TPP];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *kept = 0;
+    if (blockIdx.x < n_b)
+        normmap_strip<B, 1, SW, IN16, PH, NWV>(Bm, nbN * B, nbN * B, nbK, nbN, strips_b, packedB, nmB, nmBt, nullptr, nullptr,
+                                               nullptr, tau_skip, blockIdx.x, s_pack, s_chunk, s_skip);
+    else
+        normmap_strip<B, 0, SW, IN16, PH, NWV>(A, nbK * B, nbK * B, nbM, nbK, strips_a, packedA, nmA, nullptr, nullptr, nullptr,
+                                               nullptr, tau_skip, blockIdx.x - n_b, s_pack, s_chunk, s_skip);
 }
 
 // rowmax[k] = max_j nB[k, j] (nB row-major [nbK x nbN]); one wave per row.  NaNs are ignored:
@@ -401,7 +441,7 @@ __global__ __launch_bounds__(256) void k_fill_decay(float *__restrict__ X, int64
 // ---------------------------------------------------------------- launchers
 template <int ROLE, bool IN16>
 static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int tile, void *packed, float *nm,
-                                 float *nmT, hipStream_t s, void *packed2 = nullptr, float *nm2 = nullptr,
+                                 float *nmT, int64_t *kept, hipStream_t s, void *packed2 = nullptr, float *nm2 = nullptr,
                                  const float *rowmax = nullptr, float tau_skip = 0.0f) {
     const int64_t nbr = rows / tile, nbc = cols / tile;
     constexpr int SW = IN16 ? 512 : 256;              // strip width: a wave-wide load is 1 KiB of one row
@@ -409,35 +449,71 @@ static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int 
     const unsigned grid = (unsigned)(nbr * nstrip);
     // phases: tiles of a strip resident in LDS together take ~42 KiB at most (three workgroups per CU)
     switch (tile) {
-        case 32: k_normmap<32, ROLE, SW, IN16, 1><<<grid, 256, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip); break;
+        case 32: k_normmap<32, ROLE, SW, IN16, 1><<<grid, 256, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept); break;
         case 64:
             // tile 64: eight waves per workgroup on fp16 input (tau-aware passes at N = 16384: 0.156 / 0.138 ->
             // 0.152 / 0.129 ms) and, on fp32 input, for small grids (N = 8192: 0.066 / 0.058 -> 0.063 / 0.056 ms;
             // at N = 16384 four waves are as fast or 1 % faster)
             if (IN16 || grid <= 8192u) {
-                k_normmap<64, ROLE, SW, IN16, IN16 ? 2 : 1, 8><<<grid, 512, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip);
+                k_normmap<64, ROLE, SW, IN16, IN16 ? 2 : 1, 8><<<grid, 512, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept);
                 break;
             }
-            k_normmap<64, ROLE, SW, IN16, IN16 ? 2 : 1><<<grid, 256, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip); break;
+            k_normmap<64, ROLE, SW, IN16, IN16 ? 2 : 1><<<grid, 256, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept); break;
         // tile 128: eight waves per workgroup (two 8-row groups per lane instead of four: no register
         // spills, more loads in flight) where that measured faster -- the fp32 A role (3.36 -> 3.07 ms at
         // N = 65536) and both roles on fp16 input (2.02 -> 1.85, 1.95 -> 1.90 ms) -- but not the fp32 B
         // role (3.26 -> 3.93 ms) nor, by extension, the single pass for A = B
         case 128:
             if constexpr (IN16 || ROLE == 0) {
-                k_normmap<128, ROLE, SW, IN16, IN16 ? 4 : 2, 8><<<grid, 512, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip);
+                k_normmap<128, ROLE, SW, IN16, IN16 ? 4 : 2, 8><<<grid, 512, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept);
                 break;
             }
-            k_normmap<128, ROLE, SW, IN16, IN16 ? 4 : 2><<<grid, 256, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip); break;
+            k_normmap<128, ROLE, SW, IN16, IN16 ? 4 : 2><<<grid, 256, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
 
 hipError_t launch_normmap_a(const void *X, bool in16, int64_t rows, int64_t cols, int tile, void *packed,
-                            float *nm, const float *rowmax, float tau_skip, hipStream_t s) {
-    return in16 ? launch_normmap<0, true>(X, rows, cols, tile, packed, nm, nullptr, s, nullptr, nullptr, rowmax, tau_skip)
-                : launch_normmap<0, false>(X, rows, cols, tile, packed, nm, nullptr, s, nullptr, nullptr, rowmax, tau_skip);
+                            float *nm, const float *rowmax, float tau_skip, int64_t *kept, hipStream_t s) {
+    return in16 ? launch_normmap<0, true>(X, rows, cols, tile, packed, nm, nullptr, kept, s, nullptr, nullptr, rowmax, tau_skip)
+                : launch_normmap<0, false>(X, rows, cols, tile, packed, nm, nullptr, kept, s, nullptr, nullptr, rowmax, tau_skip);
+}
+
+template <int B, int PH, int NWV, bool IN16>
+static void launch_pair(const void *A, const void *Bm, int64_t nbM, int64_t nbK, int64_t nbN, void *packedA, void *packedB,
+                        float *nmA, float *nmB, float *nmBt, float tau_skip, int64_t *kept, hipStream_t s) {
+    constexpr int SW = IN16 ? 512 : 256;
+    const int64_t strips_a = (nbK * B + SW - 1) / SW, strips_b = (nbN * B + SW - 1) / SW;
+    const unsigned n_b = (unsigned)(nbK * strips_b), n_a = (unsigned)(nbM * strips_a);
+    k_normmap_pair<B, SW, IN16, PH, NWV><<<n_a + n_b, 64 * NWV, 0, s>>>(A, Bm, nbM, nbK, nbN, n_b, strips_a, strips_b, (uint4 *)packedA,
+                                                                        (uint4 *)packedB, nmA, nmB, nmBt, tau_skip, kept);
+}
+
+// Where the two passes are worth running as one (strips of both operands).  Whole multiplies, two passes -> one:
+// 256^3 14.6 -> 10.7 us, 2048^3 28.3 -> 23.9, 4096^3 87.2 -> 83.9, 6144^3 184 -> 182, 8192^3 912.5 -> 909.5; tile 64
+// beyond that runs four waves per workgroup in passes of their own.  A tau-aware A pass of its own (behind k_rowmax)
+// writes less: 3 us less at 4096^3, where the second launch and k_rowmax cost 8, and 13 us less at 8192^3.
+bool normmap_pair_fits(bool in16, bool tau_aware, int64_t M, int64_t K, int64_t N, int tile) {
+    const int64_t sw = in16 ? 512 : 256;
+    const int64_t strips = (M / tile) * ((K + sw - 1) / sw) + (K / tile) * ((N + sw - 1) / sw);
+    return strips <= (tau_aware ? 4096 : 16384);
+}
+
+hipError_t launch_normmap_pair(const void *A, const void *Bm, bool in16, int64_t M, int64_t K, int64_t N, int tile, void *packedA,
+                               float *nmA, void *packedB, float *nmB, float *nmBt, float tau_skip, int64_t *kept, hipStream_t s) {
+    const int64_t nbM = M / tile, nbK = K / tile, nbN = N / tile;
+#define SPAMM_PAIR(T, PH16, NWV, PH32)                                                                                          \
+    if (in16) launch_pair<T, PH16, NWV, true>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, kept, s);        \
+    else launch_pair<T, PH32, NWV, false>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, kept, s)
+    switch (tile) {
+        case 32: SPAMM_PAIR(32, 1, 4, 1); break;
+        case 64: SPAMM_PAIR(64, 2, 8, 1); break;
+        case 128: SPAMM_PAIR(128, 4, 8, 2); break;
+        default: return hipErrorInvalidValue;
+    }
+#undef SPAMM_PAIR
+    return hipGetLastError();
 }
 
 hipError_t launch_rowmax(const float *nB, int64_t nbK, int64_t nbN, float *rowmax, hipStream_t s) {
@@ -446,15 +522,15 @@ hipError_t launch_rowmax(const float *nB, int64_t nbK, int64_t nbN, float *rowma
 }
 
 hipError_t launch_normmap_ab(const void *X, bool in16, int64_t n, int tile, void *packedA, float *nmA,
-                             void *packedB, float *nmB, float *nmBt, float tau_skip, hipStream_t s) {
-    return in16 ? launch_normmap<2, true>(X, n, n, tile, packedA, nmA, nmBt, s, packedB, nmB, nullptr, tau_skip)
-                : launch_normmap<2, false>(X, n, n, tile, packedA, nmA, nmBt, s, packedB, nmB, nullptr, tau_skip);
+                             void *packedB, float *nmB, float *nmBt, float tau_skip, int64_t *kept, hipStream_t s) {
+    return in16 ? launch_normmap<2, true>(X, n, n, tile, packedA, nmA, nmBt, kept, s, packedB, nmB, nullptr, tau_skip)
+                : launch_normmap<2, false>(X, n, n, tile, packedA, nmA, nmBt, kept, s, packedB, nmB, nullptr, tau_skip);
 }
 
 hipError_t launch_normmap_b(const void *X, bool in16, int64_t rows, int64_t cols, int tile, void *packed,
-                            float *nm, float *nmT, float tau_skip, hipStream_t s) {
-    return in16 ? launch_normmap<1, true>(X, rows, cols, tile, packed, nm, nmT, s, nullptr, nullptr, nullptr, tau_skip)
-                : launch_normmap<1, false>(X, rows, cols, tile, packed, nm, nmT, s, nullptr, nullptr, nullptr, tau_skip);
+                            float *nm, float *nmT, float tau_skip, int64_t *kept, hipStream_t s) {
+    return in16 ? launch_normmap<1, true>(X, rows, cols, tile, packed, nm, nmT, kept, s, nullptr, nullptr, nullptr, tau_skip)
+                : launch_normmap<1, false>(X, rows, cols, tile, packed, nm, nmT, kept, s, nullptr, nullptr, nullptr, tau_skip);
 }
 
 hipError_t launch_unpack(const void *packed, int64_t rows, int64_t cols, int tile, int role,

@@ -1,0 +1,423 @@
+// Stages 2 and 3 in one launch, for outputs that leave the chip half empty.
+//
+// Where C has few macro tiles the gate (k_gate), the schedule (k_order) and the
+// gated GEMM are each a few microseconds of latency on a mostly idle chip, and the
+// GEMM's 256-wide work units leave most CUs without any.  Here one workgroup owns a
+// unit of U x U elements of C (U = 128 or 64) and does all three for it: it forms the
+// tau mask of its output tiles from the norm maps, lists the k tiles they keep in
+// LDS, and multiplies along that list.  What the gate leaves for the caller -- mask,
+// counts, kept total -- is written on the way out; the macro tiles' work lists, which
+// nothing reads after this kernel, are built by k_gate if somebody asks for them.
+//
+// The order of the sum is k_gemm's: entries that every tile of the unit's MACRO tile
+// keeps come first, then the others, each group in ascending k rotated to the
+// macro tile's anchor.  So a unit looks at the norms of its whole macro tile, and C is
+// the same bit for bit whichever kernel runs.
+//
+// What bounds it: a chain of latencies -- norms in, first stages in, one sync per 32 k,
+// results out -- of which units of 128 (16 KiB a stage, two workgroups per CU) make
+// the k loop shortest and units of 64 spread a small C over more CUs.  Gate, schedule
+// and GEMM as launches of their own -> this kernel, whole multiplies: 256^3 24.6 -> 14.7 us
+// (10.7 with one launch for both norm-map passes), 1056 x 1568 x 1312 38.2 -> 22.8 (18.4),
+// 2048^3 at tile 32, 5 % kept, 38.5 -> 26.3 (24.8), 2048^3 dense 63 -> 38, 1024 rows
+// against a resident 8192^2 50.3 -> 36.5.
+#include "gemm_device.h"
+
+namespace spamm {
+
+template <int B, int U>
+struct SmallCfg {
+    static constexpr int MT = 256 / B;                       // tiles per macro tile per dimension
+    static constexpr int PD = 256 / U;                       // units per macro tile per dimension
+    static constexpr int TU = U / B > 0 ? U / B : 1;         // tiles (slots) per unit per dimension
+    static constexpr int TT = TU * TU;
+    static constexpr int RS = B < U ? B : U;                 // rows of a slot
+    static constexpr int NSPE = B / 32;                      // stages of 32 k per list entry
+    static constexpr int TILE_BYTES = B * B * 2;
+    static constexpr int OP_BYTES = U * 64;                  // one operand's part of a stage
+    static constexpr int STAGE_BYTES = 2 * OP_BYTES;         // 16 or 8 KiB
+    static constexpr int NBUF = U == 128 ? 4 : 6;
+    static constexpr int CPS = RS / 16;                      // 1 KiB chunks per slot
+    static constexpr int CHW = U / 64;                       // chunks per wave per operand per stage (in one slot)
+    static constexpr int LPW = 2 * CHW;
+    static constexpr int NB = U / 32;                        // 16-wide MFMA blocks per wave per dimension
+    static constexpr int NP = TU > 1 ? TU / 2 : 1;           // tiles per wave per dimension
+    static constexpr int RB = NB / NP;                       // MFMA blocks per tile and wave per dimension
+    static constexpr uint32_t ROW_BITS = (1u << TU) - 1u;
+    static constexpr uint32_t COL_BITS = TU == 4 ? 0x1111u : (TU == 2 ? 0x5u : 0x1u);
+    static_assert(CHW == 1 || CPS >= 2, "a wave's two chunks lie in one slot, one after the other");
+};
+
+// LDS behind the ring: list entries, bitmap words of the unit's tiles, {full, partial} words, tile bits per k
+size_t small_lds_bytes_(int stage_bytes, int nbuf, int tt, int64_t nbK) {
+    const size_t words = (size_t)((nbK + 63) / 64);
+    return (size_t)stage_bytes * nbuf + words * 64 * 4 + words * tt * 8 + words * 16 + words * 64 * 2;
+}
+
+template <int B, int U>
+__global__ __launch_bounds__(256, 2) void k_small(const unsigned char *__restrict__ pA, const unsigned char *__restrict__ pB,
+                                                  GateBuffers g, int nbM, int nbK, int nbN, int nMacN, int n_units, int n_xcd,
+                                                  int mode, float tau, int64_t M, int64_t N, float *__restrict__ C) {
+    using H = SmallCfg<B, U>;
+    constexpr int NBUF = H::NBUF, MT = H::MT, TU = H::TU, TT = H::TT, NB = H::NB;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int words = (nbK + 63) >> 6;
+    uint32_t *s_list = reinterpret_cast<uint32_t *>(smem + NBUF * H::STAGE_BYTES);   // k | tile bits << 16
+    uint64_t *s_word = reinterpret_cast<uint64_t *>(s_list + words * 64);            // [words][TT]
+    uint64_t *s_fp = s_word + words * TT;                                            // [words][2]
+    uint16_t *s_bits = reinterpret_cast<uint16_t *>(s_fp + 2 * words);               // [words * 64]
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wr = wave >> 1, wc = wave & 1;
+    // consecutive units (neighbours share operand panels) in equal chunks, one per XCD
+    const int chunk = (n_units + n_xcd - 1) / n_xcd;
+    const int unit = ((int)blockIdx.x % n_xcd) * chunk + (int)blockIdx.x / n_xcd;
+    if (unit >= n_units) return;
+    const int macro = unit / (H::PD * H::PD), part = unit % (H::PD * H::PD);
+    const int mi = macro / nMacN, mj = macro % nMacN, ui = part / H::PD, uj = part % H::PD;
+    const int64_t urow = (int64_t)mi * 256 + ui * U, ucol = (int64_t)mj * 256 + uj * U;
+    if (urow >= M || ucol >= N) return;
+    const int ti0 = (int)(urow / B), tj0 = (int)(ucol / B);            // first tile of the unit
+
+    // ---- gate: a wave takes 64 k at a time, lane = k, and holds the norms of the macro tile's rows and
+    // columns (loads unconditional, from clamped addresses)
+    const bool interior = (mi + 1) * MT <= nbM && (mj + 1) * MT <= nbN;
+    for (int w = wave; w < words; w += 4) {
+        const int k = w * 64 + lane, kc = k < nbK ? k : nbK - 1;
+        const bool live = k < nbK;
+        float a[MT], b[MT], au[TU], bu[TU];
+#pragma unroll
+        for (int x = 0; x < MT; x++) {
+            const int i = mi * MT + x, j = mj * MT + x;
+            a[x] = g.nA[(int64_t)(i < nbM ? i : nbM - 1) * nbK + kc];
+            b[x] = g.nBt[(int64_t)(j < nbN ? j : nbN - 1) * nbK + kc];
+        }
+#pragma unroll
+        for (int x = 0; x < TU; x++) {
+            au[x] = g.nA[(int64_t)(ti0 + x < nbM ? ti0 + x : nbM - 1) * nbK + kc];
+            bu[x] = g.nBt[(int64_t)(tj0 + x < nbN ? tj0 + x : nbN - 1) * nbK + kc];
+        }
+        uint32_t ub = 0;
+#pragma unroll
+        for (int x = 0; x < TU; x++)
+#pragma unroll
+            for (int y = 0; y < TU; y++) {
+                const bool inside = ti0 + x < nbM && tj0 + y < nbN;
+                if (inside && live && au[x] * bu[y] >= tau) ub |= 1u << (x * TU + y);
+            }
+        // kept by every tile of the macro tile: rounding is monotone, so the product of the smallest norms
+        // decides -- unless one is not finite (inf * 0 and NaN are never kept): then all products are looked at
+        float amin = a[0], bmin = b[0];
+        bool finite = true;
+#pragma unroll
+        for (int x = 0; x < MT; x++) {
+            finite = finite && __builtin_isfinite(a[x]) && __builtin_isfinite(b[x]);
+            amin = fminf(amin, a[x]);
+            bmin = fminf(bmin, b[x]);
+        }
+        bool full = amin * bmin >= tau;
+        if (__ballot(!finite) != 0ull) {
+            full = true;
+#pragma unroll
+            for (int x = 0; x < MT; x++)
+#pragma unroll
+                for (int y = 0; y < MT; y++) full = full && a[x] * b[y] >= tau;
+        }
+        full = full && live && interior;
+        const uint64_t F = __ballot(full), P = __ballot(ub != 0u && !full);
+        uint64_t mine = 0;                                             // lane t: bitmap word of tile t
+#pragma unroll
+        for (int t = 0; t < TT; t++) {
+            const uint64_t m = __ballot((ub >> t) & 1u);
+            mine = lane == t ? m : mine;
+        }
+        if (lane < TT) s_word[w * TT + lane] = mine;
+        if (lane == 0) {
+            s_fp[2 * w] = F;
+            s_fp[2 * w + 1] = P;
+        }
+        s_bits[k] = (uint16_t)ub;
+    }
+    __syncthreads();
+    // ---- list: every wave scans the words' counts (at most 64 words), then places its own words' entries
+    const uint64_t Fl = lane < words ? s_fp[2 * lane] : 0ull, Pl = lane < words ? s_fp[2 * lane + 1] : 0ull;
+    int bf = __builtin_popcountll(Fl), bp = __builtin_popcountll(Pl);
+    const int own_f = bf, own_p = bp;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int tf = __shfl_up(bf, off, 64), tp = __shfl_up(bp, off, 64);
+        if (lane >= off) { bf += tf; bp += tp; }
+    }
+    const int n_full = __builtin_amdgcn_readlane(bf, 63), n_part = __builtin_amdgcn_readlane(bp, 63);
+    bf -= own_f;
+    bp -= own_p;
+    const int anchor = list_anchor(mi, mj, MT, nbM, nbK, nbN);
+    const uint64_t below_a = (1ull << (anchor & 63)) - 1ull;
+    const int rot_f = __builtin_amdgcn_readlane(bf + __builtin_popcountll(Fl & below_a), anchor >> 6);
+    const int rot_p = __builtin_amdgcn_readlane(bp + __builtin_popcountll(Pl & below_a), anchor >> 6);
+    for (int w = wave; w < words; w += 4) {
+        const uint64_t F = s_fp[2 * w], P = s_fp[2 * w + 1], below = (1ull << lane) - 1ull;
+        const int base_f = __builtin_amdgcn_readlane(bf, w), base_p = __builtin_amdgcn_readlane(bp, w);
+        int pos = -1;
+        if ((F >> lane) & 1ull) {
+            pos = base_f + __builtin_popcountll(F & below) - rot_f;
+            if (pos < 0) pos += n_full;
+        } else if ((P >> lane) & 1ull) {
+            pos = base_p + __builtin_popcountll(P & below) - rot_p;
+            if (pos < 0) pos += n_part;
+            pos += n_full;
+        }
+        if (pos >= 0) s_list[pos] = (uint32_t)(w * 64 + lane) | (uint32_t)s_bits[w * 64 + lane] << 16;
+    }
+    __syncthreads();
+    const int S = (n_full + n_part) * H::NSPE, Sfull = n_full * H::NSPE;
+
+    // what the gate leaves behind (a tile shared by several units is written by the first)
+    auto store_gate = [&]() {
+        if (!(mode & SMALL_GATE) || (ui * U) % B != 0 || (uj * U) % B != 0) return;
+        for (int e = threadIdx.x; e < TT * words; e += 256) {
+            const int t = e / words, w = e - t * words, i = ti0 + t / TU, j = tj0 + t % TU;
+            if (i < nbM && j < nbN) g.mask[((int64_t)i * nbN + j) * words + w] = s_word[w * TT + t];
+        }
+        if (wave == 0) {
+            int cnt = 0;
+            if (lane < TT) {
+                for (int w = 0; w < words; w++) cnt += __builtin_popcountll(s_word[w * TT + lane]);
+                const int i = ti0 + lane / TU, j = tj0 + lane % TU;
+                if (i < nbM && j < nbN) g.counts[(int64_t)i * nbN + j] = cnt;
+            }
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
+            if (lane == 0 && cnt) atomicAdd(reinterpret_cast<unsigned long long *>(g.kept_total), (unsigned long long)cnt);
+        }
+    };
+
+    if (!(mode & SMALL_MULTIPLY)) {
+        store_gate();
+        return;
+    }
+    if (S == 0) {
+        constexpr int LPR = U / 4;                                     // lanes per row
+        const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+        const int64_t c0 = ucol + (lane % LPR) * 4;
+        if (c0 < N)
+            for (int r = wave * (64 / LPR) + lane / LPR; r < U && urow + r < M; r += 4 * (64 / LPR))
+                __builtin_nontemporal_store(zero, reinterpret_cast<f32x4 *>(C + (urow + r) * N + c0));
+        store_gate();
+        return;
+    }
+
+    f32x4 acc[NB][NB];
+#pragma unroll
+    for (int r = 0; r < NB; r++)
+#pragma unroll
+        for (int c = 0; c < NB; c++) acc[r][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    {
+        // ---- staging: a wave copies CHW consecutive 1 KiB chunks of the A part and of the B part of a stage
+        // (the ring protocol and its hand-counted waits are k_gemm's)
+        const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
+        const int chunk0 = wave * H::CHW, slot = chunk0 / H::CPS, vec = (chunk0 % H::CPS) * 64;
+        int ti = ti0 + slot, tj = tj0 + slot;
+        ti = ti < nbM ? ti : nbM - 1;
+        tj = tj < nbN ? tj : nbN - 1;
+        const int within = (vec / H::RS) * B + vec % H::RS;            // 16-byte vector inside the tile's 4 k-groups
+        const unsigned char *rowA = pA + (int64_t)ti * nbK * H::TILE_BYTES + (within + (ui * U) % B) * 16;
+        const unsigned char *rowB = pB + (int64_t)tj * nbK * H::TILE_BYTES + (within + (uj * U) % B) * 16;
+        const uint32_t ldsA = lds_base + chunk0 * 1024, ldsB = ldsA + H::OP_BYTES;
+        const uint32_t needA = (H::ROW_BITS << (slot * TU)) << 16, needB = (H::COL_BITS << slot) << 16;   // entry bits that read this slot
+        const uint32_t voff = lane * 16;
+
+        // entry of a stage (stages beyond the last repeat the last entry: loaded, never multiplied)
+        auto entry_at = [&](int t) -> uint32_t { return s_list[(t < S ? t : S - 1) / H::NSPE]; };
+        auto issue = [&](int t, uint32_t ent, auto idx) {
+            constexpr int i = decltype(idx)::value, j = i % H::CHW;
+            const int64_t koff = (int64_t)(ent & 0xffffu) * H::TILE_BYTES + ((t < S ? t : S - 1) % H::NSPE) * (B * 64);
+            const uint32_t boff = (uint32_t)(t % NBUF) * H::STAGE_BYTES;
+            // a slot that no tile pair of the entry reads is not fetched: its load goes to one place that is
+            // cache resident, so that the number of loads in flight stays fixed
+            if constexpr (i < H::CHW) {
+                const int64_t on = (ent & needA) ? -1ll : 0ll;
+                dma_load<j * 1024>(pA + (((rowA - pA) + koff) & on), voff, ldsA + boff);
+            } else {
+                const int64_t on = (ent & needB) ? -1ll : 0ll;
+                dma_load<j * 1024>(pB + (((rowB - pB) + koff) & on), voff, ldsB + boff);
+            }
+        };
+        auto sync_next = [&]() {
+            __builtin_amdgcn_s_waitcnt(waitcnt_imm(H::LPW * (NBUF - 2), 0));
+            __syncthreads();
+        };
+        auto frag_off = [&](int wsel, int blk) -> int {
+            const int s = TU > 1 ? wsel + 2 * (blk * 16 / H::RS) : 0;
+            const int ro = TU > 1 ? (blk * 16) % H::RS : wsel * (U / 2) + blk * 16;
+            return s * H::RS * 64 + ((lane >> 4) * H::RS + ro + (lane & 15)) * 16;
+        };
+        struct Frags {
+            half8 a[NB], b[NB];
+        };
+        auto load_frag = [&](Frags &f, int t, auto idx) {
+            constexpr int i = decltype(idx)::value;
+            const unsigned char *bufA = smem + (t % NBUF) * H::STAGE_BYTES;
+            if constexpr (i == 0) f.a[0] = *reinterpret_cast<const half8 *>(bufA + frag_off(wr, 0));
+            else if constexpr (i <= NB) f.b[i - 1] = *reinterpret_cast<const half8 *>(bufA + H::OP_BYTES + frag_off(wc, i - 1));
+            else f.a[i - NB] = *reinterpret_cast<const half8 *>(bufA + frag_off(wr, i - NB));
+        };
+        // ---- prologue
+#pragma unroll
+        for (int t = 0; t < NBUF; t++) {
+            const uint32_t e = __builtin_amdgcn_readfirstlane(entry_at(t));
+            static_for<H::LPW>([&](auto i) { issue(t, e, i); });
+        }
+        int t = 0;
+        uint32_t e_cur = entry_at(0), e_new = entry_at(NBUF);
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm(H::LPW * (NBUF - 1), 0));
+        __syncthreads();
+        Frags f0, f1;
+        static_for<2 * NB>([&](auto i) { load_frag(f0, 0, i); });
+#define SPAMM_FENCE() __builtin_amdgcn_sched_barrier(0)
+        auto full_stage = [&](const Frags &cur, Frags &nxt) {
+            sync_next();
+            const uint32_t en = __builtin_amdgcn_readfirstlane(e_new);
+            e_cur = entry_at(t + 1);
+            e_new = entry_at(t + 1 + NBUF);
+            SPAMM_FENCE();
+            static_for<NB * NB>([&](auto idx) {
+                constexpr int i = decltype(idx)::value, r = i / NB, c = i % NB;
+                acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cur.a[r], cur.b[c], acc[r][c], 0, 0, 0);
+                if constexpr (i < 2 * NB) load_frag(nxt, t + 1, idx);
+                if constexpr (NB == 4 ? (i >= 8 && i % 2 == 0) : i >= 2) issue(t + NBUF, en, std::integral_constant<int, NB == 4 ? (i >= 8 ? (i - 8) / 2 : 0) : (i >= 2 ? i - 2 : 0)>{});
+                SPAMM_FENCE();
+            });
+            t++;
+        };
+        while (__builtin_expect(t + 1 < Sfull, 1)) {
+            full_stage(f0, f1);
+            full_stage(f1, f0);
+        }
+        auto partial_stage = [&](const Frags &cur, Frags &nxt) {
+            sync_next();
+            const uint32_t en = t + NBUF < S ? __builtin_amdgcn_readfirstlane(e_new) : (__builtin_amdgcn_readfirstlane(e_new) & 0xffffu);
+            const uint32_t ec = t < S ? (__builtin_amdgcn_readfirstlane(e_cur) >> 16) >> (TU > 1 ? wr * TU + wc : 0) : 0u;
+            e_cur = entry_at(t + 1);
+            e_new = entry_at(t + 1 + NBUF);
+            SPAMM_FENCE();
+            static_for<H::NP * H::NP>([&](auto pair) {
+                constexpr int p = decltype(pair)::value, px = p / H::NP, py = p % H::NP, bit = 2 * px * TU + 2 * py;
+                if ((ec >> bit) & 1u) {
+#pragma unroll
+                    for (int r = 0; r < H::RB; r++)
+#pragma unroll
+                        for (int c = 0; c < H::RB; c++)
+                            acc[px * H::RB + r][py * H::RB + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                cur.a[px * H::RB + r], cur.b[py * H::RB + c], acc[px * H::RB + r][py * H::RB + c], 0, 0, 0);
+                }
+                if constexpr (p == 0) {
+                    SPAMM_FENCE();
+                    static_for<2 * NB>([&](auto i) { load_frag(nxt, t + 1, i); });
+                    static_for<H::LPW>([&](auto i) { issue(t + NBUF, en, i); });
+                    SPAMM_FENCE();
+                }
+            });
+            SPAMM_FENCE();
+            t++;
+        };
+        while (__builtin_expect(t < S, 1)) {
+            partial_stage(f0, f1);
+            partial_stage(f1, f0);
+        }
+#undef SPAMM_FENCE
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));                 // the ring still holds clamped loads
+    }
+
+    // ---- epilogue: as k_gemm's
+    const uint32_t lane_off = (uint32_t)(32 * (lane >> 5)) * (uint32_t)N + 4 * (lane & 31);     // bytes
+#pragma unroll
+    for (int r = 0; r < NB; r++) {
+        const int64_t row0 = urow + (TU > 1 ? (wr + 2 * (r * 16 / B)) * B + (r * 16) % B : wr * (U / 2) + r * 16);
+        if (row0 >= M) continue;
+#pragma unroll
+        for (int c = 0; c < NB; c += 2) {
+            const int64_t col0 = ucol + (TU > 1 ? (wc + 2 * (c * 16 / B)) * B + (c * 16) % B : wc * (U / 2) + c * 16);
+            if (col0 >= N) continue;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float x = acc[r][c][i], y = acc[r][c + 1][i];
+                const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+                float *out = C + (row0 + i) * N + col0;
+                asm volatile("global_store_dword %0, %1, %2 nt" :: "v"(lane_off), "v"(sw[0]), "s"(out) : "memory");
+                asm volatile("global_store_dword %0, %1, %2 nt" :: "v"(lane_off), "v"(sw[1]), "s"(out + 4 * N) : "memory");
+            }
+        }
+    }
+    store_gate();
+}
+
+__global__ void k_clear_kept(int64_t *kept) { *kept = 0; }
+
+hipError_t launch_clear_kept(int64_t *kept, hipStream_t s) {
+    k_clear_kept<<<1, 1, 0, s>>>(kept);
+    return hipGetLastError();
+}
+
+// Unit by units of 128 in C: with half a unit per CU or more the wide one is faster (256 units: 10 % kept 26.4 -> 24.0 us,
+// dense 51.7 -> 37.6; 144 units: dense 34.8 -> 29.4, 10 % 19.2 -> 20.5), below it the narrow one (99 units: 20.1 -> 18.4,
+// 64 units: 15.4 -> 13.1 and, dense, 21.7 -> 20.6).
+static int small_unit(int64_t M, int64_t N) {
+    const int64_t units128 = ((M + 127) / 128) * ((N + 127) / 128);
+    return units128 >= 128 ? 128 : 64;
+}
+
+template <int B, int U>
+static hipError_t launch_small_(const void *pA, const void *pB, const GateBuffers &g, int64_t M, int64_t K, int64_t N,
+                                int mode, float tau, float *C, int n_xcd, hipStream_t s) {
+    using H = SmallCfg<B, U>;
+    const int nbM = (int)(M / B), nbK = (int)(K / B), nbN = (int)(N / B);
+    const int nMacM = (nbM + H::MT - 1) / H::MT, nMacN = (nbN + H::MT - 1) / H::MT;
+    const int n_units = nMacM * nMacN * H::PD * H::PD;
+    const unsigned grid = (unsigned)((n_units + n_xcd - 1) / n_xcd * n_xcd);
+    k_small<B, U><<<grid, 256, small_lds_bytes_(H::STAGE_BYTES, H::NBUF, H::TT, nbK), s>>>(
+        (const unsigned char *)pA, (const unsigned char *)pB, g, nbM, nbK, nbN, nMacN, n_units, n_xcd, mode, tau, M, N, C);
+    return hipGetLastError();
+}
+
+template <int B, int U>
+static hipError_t small_attr() {
+    using H = SmallCfg<B, U>;
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(&k_small<B, U>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)small_lds_bytes_(H::STAGE_BYTES, H::NBUF, H::TT, SMALL_MAX_NBK));
+}
+
+hipError_t small_init() {
+    hipError_t e;
+    if ((e = small_attr<32, 128>()) != hipSuccess || (e = small_attr<32, 64>()) != hipSuccess) return e;
+    if ((e = small_attr<64, 128>()) != hipSuccess || (e = small_attr<64, 64>()) != hipSuccess) return e;
+    if ((e = small_attr<128, 128>()) != hipSuccess) return e;
+    return small_attr<128, 64>();
+}
+
+// Whole multiplies, gate and GEMM apart -> this kernel, by units of 128 in C (tile 64 unless said): 484 units, dense
+// 88.3 -> 71.2 us, 10 % kept 59.2 -> 44.1; 512 units, dense 118 -> 101; 576 units, dense 94.4 -> 95.1, 10 % at tile 32
+// 63.9 -> 50.1; 1024 units, dense 156 -> 180, 40 % 115 -> 121, 10 % 84.4 -> 77.8.  Up to 512 units run at once; beyond
+// that the 256-wide units' thriftier staging wins the more is kept, and how much that is the host does not know, but
+// for tau <= 0 (everything).
+bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau) {
+    const int64_t units128 = ((M + 127) / 128) * ((N + 127) / 128);
+    return units128 <= (tau > 0.0f ? 640 : 512) && K / tile <= SMALL_MAX_NBK;
+}
+
+hipError_t launch_small(const void *packedA, const void *packedB, const GateBuffers &g, int64_t M, int64_t K, int64_t N,
+                        int tile, int mode, float tau, float *C, int n_xcd, hipStream_t s) {
+    const bool wide = small_unit(M, N) == 128;
+    switch (tile) {
+        case 32: return wide ? launch_small_<32, 128>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s)
+                             : launch_small_<32, 64>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s);
+        case 64: return wide ? launch_small_<64, 128>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s)
+                             : launch_small_<64, 64>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s);
+        case 128: return wide ? launch_small_<128, 128>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s)
+                              : launch_small_<128, 64>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace spamm

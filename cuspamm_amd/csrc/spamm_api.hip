@@ -54,6 +54,7 @@ struct Workspace {
     int64_t M = 0, K = 0, N = 0;
     int tile = 0;
     bool have_a = false, have_b = false, have_gate = false;
+    bool have_lists = false;    // of the gate: the GEMM's work lists and schedule are built (see build_lists)
     // nA / nB+nBt hold norm maps of the current M x K / K x N at the current tile
     bool nm_a = false, nm_b = false;
     float tau = 0.0f;
@@ -255,7 +256,7 @@ int spamm_create(spamm_ctx **out, int device) {
     c->stream = c->own_stream;
     for (int i = 0; i < 5 && rc == SPAMM_OK; i++)
         if (hipEventCreate(&c->ev[i]) != hipSuccess) rc = SPAMM_EHIP;
-    if (rc == SPAMM_OK && (gemm_init() != hipSuccess || gate_init() != hipSuccess)) rc = SPAMM_EHIP;
+    if (rc == SPAMM_OK && (gemm_init() != hipSuccess || gate_init() != hipSuccess || small_init() != hipSuccess)) rc = SPAMM_EHIP;
     if (rc == SPAMM_OK) {
         // this device's copy of the fixed workspace array (each GPU has its own, at its own address)
         void *sp = nullptr;
@@ -344,6 +345,8 @@ static int normmap_any(spamm_ctx *c, int role, const void *dX, bool in16, int64_
     if (c->tile != tile) reset_shape(c, tile);
     const size_t nt = (size_t)(rows / tile) * (size_t)(cols / tile);
     c->have_gate = false;
+    if ((rc = ensure(c, c->kept_total, 16))) return rc;
+    int64_t *kept = (int64_t *)c->kept_total.p;
     if (role == SPAMM_ROLE_A) {
         // a new A invalidates B (fp16 copy and norm map alike) only if the shared dimension K
         // changes; A itself is invalid until its pass has been launched
@@ -362,7 +365,7 @@ static int normmap_any(spamm_ctx *c, int role, const void *dX, bool in16, int64_
         }
         if (c->timing) HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
         HIPCHK(c, launch_normmap_a(dX, in16, rows, cols, tile, c->packedA.p, (float *)c->nA.p,
-                                   prune ? (const float *)c->rowmaxB.p : nullptr, prune ? *prune_tau : 0.0f, c->stream));
+                                   prune ? (const float *)c->rowmaxB.p : nullptr, prune ? *prune_tau : 0.0f, kept, c->stream));
         if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[2], c->stream)); c->ev_a = true; }
         c->have_a = c->nm_a = true;
         c->a_pruned = prune;
@@ -380,7 +383,7 @@ static int normmap_any(spamm_ctx *c, int role, const void *dX, bool in16, int64_
         if (c->timing) HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
         const bool prune = prune_tau != nullptr && *prune_tau > 0.0f;
         HIPCHK(c, launch_normmap_b(dX, in16, rows, cols, tile, c->packedB.p, (float *)c->nB.p,
-                                   (float *)c->nBt.p, prune ? *prune_tau : 0.0f, c->stream));
+                                   (float *)c->nBt.p, prune ? *prune_tau : 0.0f, kept, c->stream));
         if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[1], c->stream)); c->ev_b = true; }
         c->have_b = c->nm_b = true;
         c->b_pruned = prune;
@@ -424,13 +427,9 @@ int spamm_set_normmaps(spamm_ctx *c, const float *nA, const float *nB, int64_t n
     return SPAMM_OK;
 }
 
-int spamm_gate(spamm_ctx *c, float tau) {
-    if (!c) return SPAMM_EINVAL;
-    if (static_stale(c)) return SPAMM_ESTATE;
-    if (!c->tile || !c->M || !c->K || !c->N || !c->nm_a || !c->nm_b) return SPAMM_ESTATE;   // both norm maps, same K and tile
-    if (tau != tau) return SPAMM_EINVAL;   // NaN
-    int rc = set_device(c);
-    if (rc) return rc;
+// Mask, counts, kept total and the GEMM's work lists and schedule at `tau` (k_gate and k_order).
+static int build_lists(spamm_ctx *c, float tau) {
+    int rc;
     const Shape s = shape_of(c);
     if (gate_lds_bytes(c->tile, s.nbK) > gate_lds_limit()) return SPAMM_EINVAL;   // (defensive: the gate walks long K in chunks that fit)
     if (order_lds_bytes(c->tile, s.nbM, s.nbN) > order_lds_limit()) return SPAMM_EINVAL;   // more than 8192 super tiles of C
@@ -443,8 +442,46 @@ int spamm_gate(spamm_ctx *c, float tau) {
     if ((rc = ensure(c, c->order, (size_t)sched_rounds(c->tile, s.nbM, s.nbN) * MAX_XCD * SUPER_M * SUPER_N * 4))) return rc;
     if ((rc = ensure(c, c->sched, SCHED_WORDS * 4))) return rc;
     if ((rc = ensure(c, c->kept_total, 16))) return rc;
-    if (c->timing && !c->ev_a) HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
     HIPCHK(c, launch_gate(gate_buffers(c), s.nbM, s.nbK, s.nbN, c->tile, tau, c->n_xcd, c->gate_chunk_cap, c->stream));
+    c->have_lists = true;
+    return SPAMM_OK;
+}
+
+// Small outputs are gated and multiplied by a kernel of their own (kernels_small.hip); a caller who fixes
+// the work unit or the gate's chunks gets the gate and the GEMM.
+static bool is_small(const spamm_ctx *c, float tau) {
+    return c->gemm_shape == 0 && c->gate_chunk_cap == 0 && small_fits(c->M, c->K, c->N, c->tile, tau);
+}
+
+// Its gate, its multiply (dC), or both.  kept_clear: a norm-map pass of this call has cleared the kept total.
+static int run_small(spamm_ctx *c, int mode, float tau, bool kept_clear, float *dC) {
+    int rc;
+    const Shape s = shape_of(c);
+    const size_t nt = (size_t)s.nbM * s.nbN;
+    if ((rc = ensure(c, c->counts, nt * 4))) return rc;
+    if ((rc = ensure(c, c->mask, nt * s.words * 8))) return rc;
+    if ((rc = ensure(c, c->kept_total, 16))) return rc;
+    if ((mode & SMALL_GATE) && !kept_clear) HIPCHK(c, launch_clear_kept((int64_t *)c->kept_total.p, c->stream));
+    HIPCHK(c, launch_small(c->packedA.p, c->packedB.p, gate_buffers(c), c->M, c->K, c->N, c->tile, mode, tau, dC, c->n_xcd, c->stream));
+    if (mode & SMALL_GATE) {
+        c->tau = tau;
+        c->have_gate = true;
+        c->have_lists = false;
+    }
+    return SPAMM_OK;
+}
+
+int spamm_gate(spamm_ctx *c, float tau) {
+    if (!c) return SPAMM_EINVAL;
+    if (static_stale(c)) return SPAMM_ESTATE;
+    if (!c->tile || !c->M || !c->K || !c->N || !c->nm_a || !c->nm_b) return SPAMM_ESTATE;   // both norm maps, same K and tile
+    if (tau != tau) return SPAMM_EINVAL;   // NaN
+    int rc = set_device(c);
+    if (rc) return rc;
+    if (c->timing && !c->ev_a) HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
+    if (is_small(c, tau)) rc = run_small(c, SMALL_GATE, tau, false, nullptr);
+    else rc = build_lists(c, tau);
+    if (rc) return rc;
     if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[3], c->stream)); c->ev_gate = true; }
     c->tau = tau;
     c->have_gate = true;
@@ -459,9 +496,15 @@ int spamm_gemm_gated(spamm_ctx *c, float *dC) {
     if (c->b_pruned && !(c->tau > 0.0f)) return SPAMM_ESTATE;               // B's copy lacks its zero tiles
     int rc = set_device(c);
     if (rc) return rc;
+    const bool small = is_small(c, c->tau);
+    if (!small && !c->have_lists && (rc = build_lists(c, c->tau))) return rc;    // (the work unit was fixed after a small gate)
     if (c->timing && !c->ev_gate) HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
-    HIPCHK(c, launch_gemm(c->packedA.p, c->packedB.p, gate_buffers(c), c->M, c->K, c->N, c->tile, dC,
-                          c->n_xcd, c->n_cu, c->gemm_ring, gemm_shape_for(c), c->stream));
+    if (small) {
+        if ((rc = run_small(c, SMALL_MULTIPLY, c->tau, true, dC))) return rc;
+    } else {
+        HIPCHK(c, launch_gemm(c->packedA.p, c->packedB.p, gate_buffers(c), c->M, c->K, c->N, c->tile, dC,
+                              c->n_xcd, c->n_cu, c->gemm_ring, gemm_shape_for(c), c->stream));
+    }
     if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[4], c->stream)); c->ev_gemm = true; }
     return SPAMM_OK;
 }
@@ -492,29 +535,37 @@ static int multiply_any(spamm_ctx *c, const spamm_params *p, const void *dA, con
     // than the two passes (1.44 against 1.34 ms per multiply at N = 16384): the flag then only asserts
     // dA == dB, and the two ordinary passes (with their full tau-aware pruning) run
     if (a_eq_b && p->tile == 128) a_eq_b = false;
-    if (a_eq_b) {
-        // one read of the matrix feeds both operand roles (the reference's A = B runs convert and
-        // norm the same data twice)
-        if (reuse_a || reuse_b || dA != dB || p->M != p->K || p->K != p->N) return SPAMM_EINVAL;
+    const bool prune = (p->flags & SPAMM_FLAG_PRUNE) != 0 && p->tau > 0.0f;
+    const bool pair = !a_eq_b && !reuse_a && !reuse_b && normmap_pair_fits(in16, prune, p->M, p->K, p->N, p->tile);
+    if (a_eq_b || pair) {
+        // one launch for both operand roles: one read of the matrix where A = B (the reference's A = B runs
+        // convert and norm the same data twice), else both operands' strips side by side
         if (c->tile != p->tile) reset_shape(c, p->tile);
-        const int64_t n = p->M;
-        if (n / p->tile > 65535) return SPAMM_EINVAL;
+        if (p->M / p->tile > 65535 || p->K / p->tile > 65535 || p->N / p->tile > 65535) return SPAMM_EINVAL;
         if ((rc = set_device(c))) return rc;
-        const size_t nt = (size_t)(n / p->tile) * (size_t)(n / p->tile);
+        const size_t ta = (size_t)(p->M / p->tile) * (size_t)(p->K / p->tile), tb = (size_t)(p->K / p->tile) * (size_t)(p->N / p->tile);
         // nothing of the old contents is valid until the pass has been launched
         c->have_a = c->have_b = c->have_gate = false;
         c->nm_a = c->nm_b = false;
         c->a_pruned = c->b_pruned = false;
-        if ((rc = ensure(c, c->packedA, (size_t)n * n * 2))) return rc;
-        if ((rc = ensure(c, c->packedB, (size_t)n * n * 2))) return rc;
-        if ((rc = ensure(c, c->nA, nt * 4))) return rc;
-        if ((rc = ensure(c, c->nB, nt * 4))) return rc;
-        if ((rc = ensure(c, c->nBt, nt * 4))) return rc;
-        c->M = c->K = c->N = n;
+        if ((rc = ensure(c, c->packedA, (size_t)p->M * p->K * 2))) return rc;
+        if ((rc = ensure(c, c->packedB, (size_t)p->K * p->N * 2))) return rc;
+        if ((rc = ensure(c, c->nA, ta * 4))) return rc;
+        if ((rc = ensure(c, c->nB, tb * 4))) return rc;
+        if ((rc = ensure(c, c->nBt, tb * 4))) return rc;
+        if ((rc = ensure(c, c->kept_total, 16))) return rc;
+        c->M = p->M;
+        c->K = p->K;
+        c->N = p->N;
         if (c->timing) HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
-        const bool prune = (p->flags & SPAMM_FLAG_PRUNE) != 0 && p->tau > 0.0f;
-        HIPCHK(c, launch_normmap_ab(dA, in16, n, p->tile, c->packedA.p, (float *)c->nA.p, c->packedB.p,
-                                    (float *)c->nB.p, (float *)c->nBt.p, prune ? p->tau : 0.0f, c->stream));
+        const float tau_skip = prune ? p->tau : 0.0f;
+        int64_t *kept = (int64_t *)c->kept_total.p;
+        if (a_eq_b)
+            HIPCHK(c, launch_normmap_ab(dA, in16, p->M, p->tile, c->packedA.p, (float *)c->nA.p, c->packedB.p,
+                                        (float *)c->nB.p, (float *)c->nBt.p, tau_skip, kept, c->stream));
+        else
+            HIPCHK(c, launch_normmap_pair(dA, dB, in16, p->M, p->K, p->N, p->tile, c->packedA.p, (float *)c->nA.p, c->packedB.p,
+                                          (float *)c->nB.p, (float *)c->nBt.p, tau_skip, kept, c->stream));
         if (c->timing) {
             HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
             HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
@@ -522,29 +573,33 @@ static int multiply_any(spamm_ctx *c, const spamm_params *p, const void *dA, con
         }
         c->have_a = c->have_b = true;
         c->nm_a = c->nm_b = true;
-        c->a_pruned = c->b_pruned = prune;       // both copies lack their tiles of norm zero:
-        c->a_pruned_tau = 1.0e-45f;              // they serve any tau > 0 (smallest positive float)
+        c->a_pruned = c->b_pruned = prune;       // both copies lack their tiles of norm zero: they serve any tau > 0
+        c->a_pruned_tau = a_eq_b ? 1.0e-45f : p->tau;   // (smallest positive float; as after the pass of its own)
         c->have_gate = false;
     } else if (!reuse_b) {
-        const bool prune = (p->flags & SPAMM_FLAG_PRUNE) != 0;
         if ((rc = normmap_any(c, SPAMM_ROLE_B, dB, in16, p->K, p->N, p->tile, prune ? &p->tau : nullptr))) return rc;
     } else if (c->timing) {
         HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
         HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
         c->ev_b = true;
     }
-    if (a_eq_b) {
+    if (a_eq_b || pair) {
         // done above
     } else if (!reuse_a) {
-        const bool prune = (p->flags & SPAMM_FLAG_PRUNE) != 0;
         if ((rc = normmap_any(c, SPAMM_ROLE_A, dA, in16, p->M, p->K, p->tile, prune ? &p->tau : nullptr))) return rc;
     } else if (c->timing) {
         HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
         c->ev_a = true;
     }
+    if (is_small(c, p->tau)) {
+        // one launch for both stages (the gate's interval is empty)
+        if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[3], c->stream)); c->ev_gate = true; }
+        if ((rc = run_small(c, SMALL_GATE | SMALL_MULTIPLY, p->tau, !(reuse_a && reuse_b), dC))) return rc;
+        if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[4], c->stream)); c->ev_gemm = true; }
+        return SPAMM_OK;
+    }
     if ((rc = spamm_gate(c, p->tau))) return rc;
-    if ((rc = spamm_gemm_gated(c, dC))) return rc;
-    return SPAMM_OK;
+    return spamm_gemm_gated(c, dC);
 }
 
 // Gives every buffer a multiply of this shape needs its place in the fixed array (base != null) and
@@ -879,7 +934,9 @@ int spamm_get_macro_counts(spamm_ctx *c, int32_t *host_counts, int32_t *host_sch
     if (static_stale(c)) return SPAMM_ESTATE;
     if (!c->have_gate) return SPAMM_ESTATE;
     const Shape s = shape_of(c);
-    int rc = copy_out(c, c->macro_count.p, host_counts, (size_t)s.n_macro * 8);
+    int rc = set_device(c);
+    if (rc == SPAMM_OK && !c->have_lists) rc = build_lists(c, c->tau);     // the last multiply ran without them
+    if (rc == SPAMM_OK) rc = copy_out(c, c->macro_count.p, host_counts, (size_t)s.n_macro * 8);
     if (rc == SPAMM_OK && host_sched) rc = copy_out(c, c->sched.p, host_sched, 2 * MAX_XCD * 4);
     return rc;
 }

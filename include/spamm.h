@@ -77,7 +77,9 @@ typedef struct spamm_params {
 typedef struct spamm_stats {
     int64_t total_products;   /* (M/b)(N/b)(K/b) */
     int64_t kept_products;    /* number of (i,j,k) that passed the gate */
-    float ms_normmap_a;       /* valid when SPAMM_FLAG_TIMING was set */
+    float ms_normmap_a;       /* valid when SPAMM_FLAG_TIMING was set.  Where one launch does the work of two stages its
+                               * time is the later one's: both norm-map passes of a small call are reported as
+                               * ms_normmap_b, gate and multiply of a small C as ms_gemm */
     float ms_normmap_b;
     float ms_gate;
     float ms_gemm;
@@ -103,9 +105,10 @@ SPAMM_API int spamm_destroy(spamm_ctx *ctx);
  *   SPAMM_OPT_GEMM_SHAPE: work unit of the gated GEMM: 1 = a workgroup of four waves per 256 x 256
  *     macro tile of C (one workgroup per CU), 2 = four waves per 128 x 256 half (two workgroups per
  *     CU), 3 = eight waves per macro tile, 4 = shape 1 by workgroups that stay on their CU and draw
- *     macro tiles from a ticket counter per XCD; 0 = chosen per call (halves when C has at most
- *     half a macro tile per CU, else 1).  All walk the same lists in the same order: C is
- *     bit-identical.
+ *     macro tiles from a ticket counter per XCD; 0 = chosen per call (a small C -- at most 640
+ *     blocks of 128 x 128, 512 for tau <= 0 -- is gated and multiplied by one kernel in units of 128
+ *     or 64; otherwise 1, or halves when C has at most half a macro tile per CU).  All add in the same
+ *     order: C is bit-identical.
  * SPAMM_EINVAL for an unknown option or a value outside its range.  The reference has no such
  * knobs: its launch shapes are compile-time constants (main.h:32-73). */
 #define SPAMM_OPT_NUM_XCD 1

@@ -232,3 +232,41 @@ def test_schedule_for_other_xcd_counts_gives_the_same_product(orc, ctx, n_xcd):
         _check(orc, other, orc.fill_decay(768, 1024, tab, 3), orc.fill_decay(1024, 640, tab, 4), 64, 0.3)
     finally:
         other.close()
+
+
+@pytest.mark.parametrize("M,K,N,tile", [(32, 32, 32, 32), (256, 256, 256, 32), (96, 2080, 224, 32), (416, 160, 736, 32),
+                                        (1056, 1568, 1312, 32), (2048, 4096, 1024, 32), (256, 65536, 288, 32),
+                                        (64, 64, 64, 64), (320, 8192, 448, 64), (1152, 640, 2112, 64), (1024, 8192, 4096, 64),
+                                        (128, 128, 128, 128), (384, 1280, 640, 128), (1920, 512, 2176, 128)])
+def test_small_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N, tile):
+    """Small outputs are gated and multiplied by one kernel, in units of 128 or 64: same mask, counts, kept total
+    and, bit for bit, the same C as the gate and the GEMM apart -- units cut by the edges of C, units smaller
+    than a tile, one to many 64-k words, empty, sparse, half-full and full lists, both input types."""
+    import torch
+    import cuspamm_amd as sp
+    apart = sp.SpammContext(0)
+    apart.set_option(sp.OPT_GEMM_SHAPE, 1)
+    try:
+        tab = orc.decay_table("exp", max(M, K, N), 12.0 / max(M, K, N))
+        dA = torch.empty((M, K), dtype=torch.float32, device="cuda")
+        dB = torch.empty((K, N), dtype=torch.float32, device="cuda")
+        ctx.fill_decay(dA, tab, 1)
+        ctx.fill_decay(dB, tab, 2)
+        ctx.normmap_f32(1, dB, tile)
+        ctx.normmap_f32(0, dA, tile)
+        for tau in (0.0, float("inf"), ctx.tau_for_ratio(0.03)[0], ctx.tau_for_ratio(0.4)[0]):
+            for a, b in ((dA, dB), (dA.half(), dB.half())):
+                want = apart.multiply(a, b, tile, tau)
+                got = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+                ctx.multiply(a, b, tile, tau, C=got)
+                assert torch.equal(got, want), tau
+                assert np.array_equal(ctx.get_mask(), apart.get_mask()) and np.array_equal(ctx.get_counts(), apart.get_counts())
+                assert ctx.get_stats().kept_products == apart.get_stats().kept_products
+        # once more on the operands that lie there (no pass runs), then the stages of their own on that gate
+        ctx.multiply(dA.half(), dB.half(), tile, tau, C=got, reuse_a=True, reuse_b=True)
+        assert torch.equal(got, want) and ctx.get_stats().kept_products == apart.get_stats().kept_products
+        assert np.array_equal(ctx.get_macro_counts()[0], apart.get_macro_counts()[0])
+        got.fill_(float("nan"))
+        assert torch.equal(ctx.gemm_gated(got), want)
+    finally:
+        apart.close()

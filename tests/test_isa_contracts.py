@@ -248,3 +248,24 @@ def test_gemm_k_loops_issue_no_other_vector_memory_instruction(tmp_path):
             assert not any(mn.startswith("scratch_") for mn in mns), name
         else:
             assert not atomics, name
+
+
+def test_small_output_kernel_keeps_the_same_contracts(tmp_path):
+    # kernels_small.hip: three tile sizes x units of 128 and 64, the same assembly blocks and hand-counted waits
+    text = _isa("kernels_small.hip", tmp_path)
+    ins = _instructions(text)
+    for reader in ("global_load_lds_dwordx4", "global_store_dword"):
+        found, checked = _hazards(ins, reader, 5)
+        assert not found and checked > 20, (reader, [ins[i] for pair in found for i in pair])
+    found, checked = _hazards(_instructions(_isa("kernels_gemm.hip", tmp_path)), "global_store_dword", 5)
+    assert not found and checked > 20
+    kernels = re.findall(r"^(_ZN5spamm7k_smallILi\d+ELi\d+EEE\w+):[^\n]*\n(.*?)s_endpgm", text, flags=re.S | re.M)
+    assert len(kernels) == 6
+    for name, body in kernels:
+        mns = [mn for mn, _, _ in _instructions(body)]
+        dma = [i for i, mn in enumerate(mns) if mn == "global_load_lds_dwordx4"]
+        assert len(dma) >= 12, name
+        other = [mn for mn in mns[dma[0]:dma[-1] + 1]
+                 if mn.startswith(("global_", "flat_", "buffer_", "scratch_")) and mn != "global_load_lds_dwordx4"]
+        assert not other, "%s: %s between the first and the last global->LDS load" % (name, sorted(set(other)))
+        assert not any(mn.startswith("scratch_") for mn in mns), name
