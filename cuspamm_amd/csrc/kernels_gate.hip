@@ -345,42 +345,68 @@ __global__ __launch_bounds__(NTH) void k_gate(GateBuffers g, int nbM, int nbK, i
 // Output: order[x * P + q] = macro tile id of XCD x's q-th workgroup for
 // q < sched[8 + x] (entries beyond are not written), sched[x] = number of
 // computing items, sched[8 + x] = number of all items.
-// One workgroup; O(n^2) ranking over at most a few thousand super tiles.
+// What bounds it: one workgroup on an idle chip, so its time is latencies one after the other.
+// The macro tiles' results are read once, by all threads; what the later steps need of them
+// -- a length and a set of computing macro tiles per super tile -- stays in LDS, ranks come from
+// prefix sums where the key is only "holds work", the serial deals run in one wave on lane
+// moves inside a row (DPP) instead of trips through LDS, and every thread writes its own part of
+// the sequences.  By the kernel trace, before -> now: 8192^2 of C (32 super tiles, 10 % kept, dealt
+// greedily) 12.2 -> 9.2 us, 16384^2 (128, band) 16.6 -> 12.1, 10048^2 (50, greedy) 19.5 -> 12.5, 32768^2 (512,
+// band) 52.9 -> 24.3.
+__device__ __forceinline__ int order_origin(int sid, int nSupN) {     // first macro tile row, column
+    return ((sid / nSupN) * SUPER_M) << 16 | ((sid % nSupN) * SUPER_N);
+}
+template <int CTRL>
+__device__ __forceinline__ int dpp(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+
 __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nMacN, int nSupN,
                                                 int n_super, int rounds, int n_xcd) {
-    extern __shared__ __attribute__((aligned(16))) int swork[];               // [n_super] length, then [n_super] super tile origin by rank,
-    int *srank_id = swork + n_super;             // then (greedy deal only) [n_xcd][rounds] rank of each XCD's r-th super tile
-    uint16_t *sdeal = reinterpret_cast<uint16_t *>(srank_id + n_super);
+    extern __shared__ __attribute__((aligned(16))) int swork[];               // [n_super + 8] length; at the end, computing macro tiles before an XCD's r-th super tile
+    int *sempty = swork + n_super + MAX_XCD;                                  // [n_super + 8] at the end: empty macro tiles before it
+    uint32_t *scomp = reinterpret_cast<uint32_t *>(sempty + n_super + MAX_XCD);  // [n_super] computing macro tiles (bit: slot)
+    int *srank_id = reinterpret_cast<int *>(scomp + n_super);                 // [n_super] super tile origin by rank,
+    uint16_t *sdeal = reinterpret_cast<uint16_t *>(srank_id + n_super);      // then (dealt by table) [n_xcd][rounds] rank of each XCD's r-th super tile
     __shared__ unsigned long long total;
-    __shared__ int s_nonempty;
+    __shared__ int s_count[16], s_len[64], s_orig[64];
+    __shared__ int s_cnt[MAX_XCD], s_before[MAX_XCD], s_nall[MAX_XCD];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint64_t below = (1ull << lane) - 1ull;
     const int P = rounds * SUPER_M * SUPER_N;
-    if (threadIdx.x == 0) { total = 0; s_nonempty = 0; }
-    // (this kernel is one workgroup on an idle GPU: its run time is memory round trips and
-    // instruction fetch, so every thread takes one macro tile row of one super tile -- all loads
-    // of the kernel's first step are in flight at once -- and the code is kept small)
-    for (int sid = threadIdx.x; sid < n_super; sid += blockDim.x) swork[sid] = 0;
+    if (threadIdx.x == 0) total = 0;
+    // every thread takes one macro tile row of one super tile: all loads of a step are in flight at once
+    for (int sid = threadIdx.x; sid < n_super; sid += blockDim.x) { swork[sid] = 0; scomp[sid] = 0u; }
     __syncthreads();
     unsigned long long mine = 0;
     for (int e = threadIdx.x; e < n_super * SUPER_M; e += blockDim.x) {
         const int sid = e / SUPER_M, a = e % SUPER_M;
         const int mi = (sid / nSupN) * SUPER_M + a, mj0 = (sid % nSupN) * SUPER_N;
-        int w = 0, len = 0;
+        int w[SUPER_N], l[SUPER_N], len = 0;
+        uint32_t bits = 0;
 #pragma unroll
-        for (int b = 0; b < SUPER_N; b++)
-            if (mi < nMacM && mj0 + b < nMacN) {
-                w += g.macro_work[mi * nMacN + mj0 + b];
-                len += g.macro_count[2 * (mi * nMacN + mj0 + b)];
-            }
+        for (int b = 0; b < SUPER_N; b++) {
+            const bool in = mi < nMacM && mj0 + b < nMacN;
+            w[b] = in ? g.macro_work[mi * nMacN + mj0 + b] : 0;
+            l[b] = in ? g.macro_count[2 * (mi * nMacN + mj0 + b)] : 0;
+        }
+#pragma unroll
+        for (int b = 0; b < SUPER_N; b++) {
+            len += l[b];
+            bits |= w[b] > 0 ? 1u << b : 0u;
+            mine += (unsigned long long)w[b];
+        }
         if (len) atomicAdd(&swork[sid], len);
-        mine += (unsigned long long)w;
+        if (bits) atomicOr(&scomp[sid], bits << (a * SUPER_N));
     }
-    if (mine) atomicAdd(&total, mine);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) mine += __shfl_xor(mine, off, 64);
+    if (lane == 0 && mine) atomicAdd(&total, mine);
     __syncthreads();
-    // How the super tiles are dealt to the XCDs (sdeal, or the snake formula in macro_at):
+    // How the super tiles are dealt to the XCDs (sdeal, or the snake formula in dealt):
     //   DEAL_LPT    few super tiles hold work: ranked by length, each goes to the XCD with the
-    //               least length so far (pure balance; ~0.2 us of serial work per super tile);
-    //   DEAL_BAND   at most BAND_DEAL_MAX super tiles hold work (the deal is serial, ~1.2 us
-    //               per group; at N = 65536 it cost more than it gained) and they are at most
+    //               least length so far (pure balance);
+    //   DEAL_BAND   at most BAND_DEAL_MAX super tiles hold work and they are at most
     //               60 % of all (a narrow band): ranked in
     //               row-major order, those with work first; every group of n_xcd consecutive
     //               ones -- neighbours along the band that read the same operand panels -- runs
@@ -396,223 +422,258 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
     //               ones in row-major order (neighbours along a row share the A panel) in equal
     //               chunks, one per XCD; no ranking (the problem is a few microseconds long).
     enum { DEAL_LPT, DEAL_BAND, DEAL_SNAKE, DEAL_FLAT };
-    {
-        int ne = 0;
-        for (int sid = threadIdx.x; sid < n_super; sid += blockDim.x) ne += swork[sid] > 0;
-        if (ne) atomicAdd(&s_nonempty, ne);
+    if (n_super < n_xcd) {                      // DEAL_FLAT: one round of at most 28 macro tiles per XCD
+        const int chunk = (nMacM * nMacN + n_xcd - 1) / n_xcd;
+        if (wave < n_xcd) {
+            const int m = wave * chunk + lane;
+            const bool in = lane < chunk && m < nMacM * nMacN;
+            const bool comp = in && g.macro_work[in ? m : 0] > 0;
+            const uint64_t bi = __ballot(in), bc = __ballot(comp), be = bi & ~bc;
+            const int nall = __builtin_popcountll(bi);
+            if (comp) g.order[wave * P + __builtin_popcountll(bc & below)] = m;
+            else if (in) g.order[wave * P + nall - 1 - __builtin_popcountll(be & below)] = m;
+            if (lane == 0) {
+                g.sched[wave] = __builtin_popcountll(bc);
+                g.sched[MAX_XCD + wave] = nall;
+                g.sched[2 * MAX_XCD + wave] = 0;
+            }
+        }
+        if (threadIdx.x == 0) g.kept_total[0] = (int64_t)total;
+        return;
     }
-    __syncthreads();
-    const int n_ne = s_nonempty;
-    const int deal = n_super < n_xcd ? DEAL_FLAT
-                     : n_super > LPT_MAX_SUPER ? DEAL_SNAKE
+    int n_ne = 0;                               // super tiles with work
+    for (int sid0 = 0; sid0 < n_super; sid0 += blockDim.x) {
+        const int sid = sid0 + threadIdx.x;
+        const uint64_t m = __ballot(sid < n_super && swork[sid < n_super ? sid : 0] > 0);
+        if (lane == 0) s_count[wave] = __builtin_popcountll(m);
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < 16; v++) n_ne += s_count[v];
+        __syncthreads();
+    }
+    const int deal = n_super > LPT_MAX_SUPER ? DEAL_SNAKE
                      : (n_ne <= LPT_GREEDY_MAX ? DEAL_LPT
                         : (n_ne <= BAND_DEAL_MAX && 5 * n_ne <= 3 * n_super ? DEAL_BAND : DEAL_SNAKE));
-    const int flat_chunk = (nMacM * nMacN + n_xcd - 1) / n_xcd;      // <= P: n_super < n_xcd super tiles of 32
-    // Ranking: larger key first, equal keys by smaller index; the key is the length, or in the
-    // band deal just "holds work".  srank_id[rank] becomes the super tile's origin.
-    //   up to RANK_SORT_MIN super tiles: rank = number of super tiles that come first, n_super^2
-    //   comparisons with the j range cut into `parts` pieces so that all 1024 threads take part
-    //   (partial ranks meet in srank_id, used as a counter first);
-    //   beyond: a bitonic sort of the indices in LDS (padded to a power of two with indices
-    //   >= n_super, which sort last): log^2 steps of one compare-exchange per thread instead of
-    //   n_super comparisons per super tile on this one CU (150 us at 2048 super tiles).
+    // Ranking: super tiles with work before those without; in the snake and the greedy deal by
+    // descending length, equal lengths by index, in the band deal by index.  srank_id[rank] becomes
+    // the super tile's origin.
     constexpr int RANK_SORT_MIN = 512;
-    if (deal == DEAL_FLAT) {
-        // nothing to rank
+    if (deal != DEAL_SNAKE) {
+        // by index first: prefix sums of "holds work" (the lengths move to their ranks)
+        constexpr int STEPS = LPT_MAX_SUPER / 1024;
+        int len_[STEPS], rank_[STEPS], ne = 0;
+#pragma unroll
+        for (int n = 0; n < STEPS; n++) {
+            const int sid = n * 1024 + threadIdx.x;
+            const int len = sid < n_super ? swork[sid] : 0;
+            const uint64_t m = __ballot(len > 0);
+            if (lane == 0) s_count[wave] = __builtin_popcountll(m);
+            __syncthreads();
+            int before = ne, here = ne;
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                before += v < wave ? s_count[v] : 0;
+                here += s_count[v];
+            }
+            before += __builtin_popcountll(m & below);
+            len_[n] = len;
+            rank_[n] = len > 0 ? before : n_ne + (sid - before);
+            ne = here;
+            __syncthreads();
+        }
+#pragma unroll
+        for (int n = 0; n < STEPS; n++) {
+            const int sid = n * 1024 + threadIdx.x;
+            if (sid >= n_super) break;
+            const int rank = rank_[n], origin = order_origin(sid, nSupN);
+            swork[rank] = len_[n];
+            srank_id[rank] = origin;
+            if (deal == DEAL_LPT && rank < n_ne) { s_len[rank] = len_[n]; s_orig[rank] = origin; }
+        }
+        __syncthreads();
+        if (wave == 0 && deal == DEAL_LPT) {
+            // the (at most 64) super tiles with work by length: lane = one of them
+            int len = lane < n_ne ? s_len[lane] : 0, rank = 0;
+            const int origin = lane < n_ne ? s_orig[lane] : 0;
+            for (int j = 0; j < n_ne; j++) {
+                const int lj = __builtin_amdgcn_readlane(len, j);
+                rank += lj > len || (lj == len && j < lane);
+            }
+            if (lane < n_ne) { s_len[rank] = len; srank_id[rank] = origin; }
+            __builtin_amdgcn_wave_barrier();
+            len = lane < n_ne ? *const_cast<volatile int *>(&s_len[lane]) : 0;
+            // lane x < n_xcd keeps XCD x's length so far and its number of super tiles; the
+            // least-loaded XCD with room is the minimum of (length, lane) over eight lanes
+            // (lengths stay far below 2^28: at most LPT_GREEDY_MAX super tiles of 32 lists)
+            const int x = lane;
+            uint32_t load = 0;
+            int cnt = 0;
+            for (int r = 0; r < n_ne; r++) {
+                uint32_t key = (x < n_xcd && cnt < rounds) ? (load << 3) | (uint32_t)x : ~0u, o;
+                o = (uint32_t)dpp<0xB1>((int)key); key = o < key ? o : key;        // lane ^ 1
+                o = (uint32_t)dpp<0x4E>((int)key); key = o < key ? o : key;        // lane ^ 2
+                o = (uint32_t)dpp<0x141>((int)key); key = o < key ? o : key;       // 7 - lane: the other four
+                if ((int)(key & 7u) == x) {
+                    sdeal[x * rounds + cnt] = (uint16_t)r;
+                    cnt++;
+                    load += (uint32_t)__builtin_amdgcn_readlane(len, r);
+                }
+            }
+            if (x < MAX_XCD) s_cnt[x] = cnt;
+        }
+        if (wave == 0 && deal == DEAL_BAND) {
+            // lanes 0..7 (and again 8..15, so that a rotation by row of 16 is one by 8): the group's i-th
+            // super tile and XCD i's length so far.  Ranks are counts over seven rotations of keys that
+            // carry the index; XCD x takes the super tile whose rank (heaviest first) is its own (shortest
+            // first).
+            const int x = lane & 7;
+            int load = 0, cnt = 0;
+            const int ngroups = (n_ne + n_xcd - 1) / n_xcd;
+            auto weight = [&](int g2) -> int { const int r = g2 * n_xcd + x; return x < n_xcd && r < n_ne ? swork[r] : -1; };     // -1: no super tile
+            int w = weight(0);
+            for (int g2 = 0; g2 < ngroups; g2++) {
+                const int wn = weight(g2 + 1);
+                const int wkey = (w + 1) * 8 + 7 - x, lkey = x < n_xcd ? load * 8 + x : 0x7ffffff0 + x;
+                int wrank = 0, xrank = 0;
+                static_for<7>([&](auto i) {
+                    constexpr int ROR = 0x121 + decltype(i)::value;
+                    wrank += dpp<ROR>(wkey) > wkey;
+                    xrank += dpp<ROR>(lkey) < lkey;
+                });
+                const int pk = (w + 1) << 6 | x << 3 | wrank;
+                int sel = wrank == xrank ? pk : 0;
+                static_for<7>([&](auto i) {
+                    const int o = dpp<0x121 + decltype(i)::value>(pk);
+                    sel = (o & 7) == xrank ? o : sel;
+                });
+                const int wm = (sel >> 6) - 1;
+                if (x < n_xcd && wm > 0) {       // (the last group may have fewer super tiles than XCDs)
+                    if (lane < MAX_XCD) sdeal[x * rounds + cnt] = (uint16_t)(g2 * n_xcd + ((sel >> 3) & 7));
+                    cnt++;
+                    load += wm;
+                }
+                w = wn;
+            }
+            if (lane < MAX_XCD) s_cnt[x] = cnt;
+        }
+        __syncthreads();
+        // super tiles with nothing kept (ranks n_ne ..) fill the XCDs' remaining slots in order
+        if (threadIdx.x < n_xcd) {
+            int before = 0;
+            for (int v = 0; v < (int)threadIdx.x; v++) before += rounds - s_cnt[v];
+            s_before[threadIdx.x] = before;
+        }
     } else if (n_super <= RANK_SORT_MIN) {
-        const bool band = deal == DEAL_BAND;
+        // rank = number of super tiles that come first, n_super^2 comparisons with the j range cut
+        // into `parts` pieces so that all 1024 threads take part
         int parts = 2;
         while (parts < 32 && n_super * parts * 2 <= (int)blockDim.x) parts *= 2;
         for (int sid = threadIdx.x; sid < n_super; sid += blockDim.x) srank_id[sid] = 0;
         __syncthreads();
         const int chunk = (n_super + parts - 1) / parts;
-        // (two copies of the loop, one per key, so that the inner loop is a read, two compares and an add)
-        auto count_first = [&](auto key) {
-            for (int e = threadIdx.x; e < n_super * parts; e += blockDim.x) {
-                const int sid = e % n_super, part = e / n_super;
-                const int w = key(swork[sid]);
-                const int j1 = (part + 1) * chunk < n_super ? (part + 1) * chunk : n_super;
-                int rank = 0;
-                for (int j = part * chunk; j < j1; j++) {
-                    const int kj = key(swork[j]);
-                    rank += (kj > w) || (kj == w && j < sid);
-                }
-                if (rank) atomicAdd(&srank_id[sid], rank);
+        for (int e = threadIdx.x; e < n_super * parts; e += blockDim.x) {
+            const int sid = e % n_super, part = e / n_super;
+            const int w = swork[sid];
+            const int j1 = (part + 1) * chunk < n_super ? (part + 1) * chunk : n_super;
+            int rank = 0;
+            for (int j = part * chunk; j < j1; j++) {
+                const int kj = swork[j];
+                rank += (kj > w) || (kj == w && j < sid);
             }
-        };
-        if (band) count_first([](int v) { return (int)(v > 0); });
-        else count_first([](int v) { return v; });
+            if (rank) atomicAdd(&srank_id[sid], rank);
+        }
         __syncthreads();
         const int sid = threadIdx.x;              // n_super <= RANK_SORT_MIN < blockDim.x: one super tile per thread
         const int rank = sid < n_super ? srank_id[sid] : 0;
         __syncthreads();
-        if (sid < n_super) {
-            srank_id[rank] = ((sid / nSupN) * SUPER_M) << 16 | ((sid % nSupN) * SUPER_N);   // first macro tile row, column
-            if (deal != DEAL_SNAKE) sdeal[sid] = (uint16_t)rank;       // parked: rank of super tile sid (read back below)
-        }
+        if (sid < n_super) srank_id[rank] = order_origin(sid, nSupN);
     } else {
+        // a bitonic sort of the indices in LDS (padded to a power of two with indices >= n_super,
+        // which sort last): log^2 steps of one compare-exchange per thread instead of n_super
+        // comparisons per super tile on this one CU (150 us at 2048 super tiles)
         int np2 = 2 * RANK_SORT_MIN;
         while (np2 < n_super) np2 <<= 1;
-        int *sidx = srank_id;                     // [np2]: runs into sdeal's space, which is not in use yet
+        int *sidx = srank_id;                     // [np2]
         for (int i = threadIdx.x; i < np2; i += blockDim.x) sidx[i] = i;
         __syncthreads();
-        auto sort_by = [&](auto key) {
-            for (int k = 2; k <= np2; k <<= 1)
-                for (int j = k >> 1; j > 0; j >>= 1) {
-                    for (int t = threadIdx.x; t < np2 / 2; t += blockDim.x) {
-                        const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1)), l = i | j;
-                        const int a = sidx[i], b = sidx[l];
-                        const int ka = a < n_super ? key(swork[a]) : -1, kb = b < n_super ? key(swork[b]) : -1;
-                        const bool a_first = ka > kb || (ka == kb && a < b);
-                        if (a_first != ((i & k) == 0)) { sidx[i] = b; sidx[l] = a; }
-                    }
-                    __syncthreads();
+        for (int k = 2; k <= np2; k <<= 1)
+            for (int j = k >> 1; j > 0; j >>= 1) {
+                for (int t = threadIdx.x; t < np2 / 2; t += blockDim.x) {
+                    const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1)), l = i | j;
+                    const int a = sidx[i], b = sidx[l];
+                    const int ka = a < n_super ? swork[a] : -1, kb = b < n_super ? swork[b] : -1;
+                    const bool a_first = ka > kb || (ka == kb && a < b);
+                    if (a_first != ((i & k) == 0)) { sidx[i] = b; sidx[l] = a; }
                 }
-        };
-        if (deal == DEAL_BAND) sort_by([](int v) { return (int)(v > 0); });
-        else sort_by([](int v) { return v; });
+                __syncthreads();
+            }
         // sidx[rank] = super tile; every thread turns its own slots into origins
-        for (int r = threadIdx.x; r < n_super; r += blockDim.x) {
-            const int sid = sidx[r];
-            srank_id[r] = ((sid / nSupN) * SUPER_M) << 16 | ((sid % nSupN) * SUPER_N);
-            if (deal != DEAL_SNAKE) sdeal[sid] = (uint16_t)r;
-        }
+        for (int r = threadIdx.x; r < n_super; r += blockDim.x) srank_id[r] = order_origin(sidx[r], nSupN);
     }
     __syncthreads();
-    if (deal != DEAL_SNAKE && deal != DEAL_FLAT) {
-        // lengths by rank, then the deal by one wave
-        int mylen[(LPT_MAX_SUPER + 1023) / 1024], myrank[(LPT_MAX_SUPER + 1023) / 1024];
-        int n = 0;
-        for (int sid = threadIdx.x; sid < n_super; sid += blockDim.x) { mylen[n] = swork[sid]; myrank[n] = sdeal[sid]; n++; }
-        __syncthreads();
-        n = 0;
-        for (int sid = threadIdx.x; sid < n_super; sid += blockDim.x) { swork[myrank[n]] = mylen[n]; n++; }
-        __syncthreads();
-        if (threadIdx.x < 64 && deal == DEAL_LPT) {
-            // lane x < n_xcd keeps XCD x's length so far and its number of super tiles; the
-            // least-loaded XCD with room is the minimum of (length, lane) over the lanes
-            // (lengths stay far below 2^28: at most LPT_GREEDY_MAX super tiles of 32 lists)
-            const int x = threadIdx.x;
-            uint32_t load = 0;
-            int cnt = 0;
-            for (int r = 0; r < n_ne; r++) {
-                uint32_t key = (x < n_xcd && cnt < rounds) ? (load << 3) | (uint32_t)x : ~0u;
-#pragma unroll
-                for (int off = 1; off < MAX_XCD; off <<= 1) {
-                    const uint32_t o = (uint32_t)__shfl_xor((int)key, off, 64);
-                    key = o < key ? o : key;
-                }
-                if ((int)(key & 7u) == x) {
-                    sdeal[x * rounds + cnt] = (uint16_t)r;
-                    cnt++;
-                    load += (uint32_t)swork[r];
-                }
-            }
-            // super tiles with nothing kept (ranks n_ne ..) fill the XCDs' remaining slots in lane order
-            const int room = x < n_xcd ? rounds - cnt : 0;
-            int before = room;
-#pragma unroll
-            for (int off = 1; off < MAX_XCD; off <<= 1) {
-                const int o = __shfl_up(before, off, 64);
-                if (x >= off) before += o;
-            }
-            before -= room;
-            for (int c = 0; c < room; c++) {
-                const int r = n_ne + before + c;
-                sdeal[x * rounds + cnt + c] = r < n_super ? (uint16_t)r : (uint16_t)0xffffu;   // 0xffff: no super tile
-            }
-        }
-        if (threadIdx.x < 64 && deal == DEAL_BAND) {
-            // lane x < 8 holds the x-th super tile of the group and the length of XCD x so far; the
-            // 64 lanes compare all pairs at once (lane 8 i + j: i against j), so that the ranks of
-            // the eight super tiles (heaviest first) and of the eight XCDs (shortest first) are
-            // byte-wise popcounts of two ballots, and the match -- the super tile whose rank is the
-            // XCD's rank -- the lowest set bit of a third
-            const int x = threadIdx.x;
-            const int pi = x >> 3, pj = x & 7;
-            int load = 0, cnt = 0;
-            const int ngroups = (n_ne + n_xcd - 1) / n_xcd;
-            for (int g2 = 0; g2 < ngroups; g2++) {
-                const int r = g2 * n_xcd + x;
-                const int w = (x < n_xcd && r < n_ne) ? swork[r] : -1;           // -1: no super tile
-                const int wi = __shfl(w, pi, 64), wj = __shfl(w, pj, 64);
-                const int li = __shfl(load, pi, 64), lj = __shfl(load, pj, 64);
-                const uint64_t heavier = __ballot((wj > wi) || (wj == wi && pj < pi));
-                const uint64_t shorter = __ballot(pj < n_xcd && ((lj < li) || (lj == li && pj < pi)));
-                const int irank_j = __builtin_popcountll((heavier >> (8 * pj)) & 0xffull);
-                const int xrank_i = __builtin_popcountll((shorter >> (8 * pi)) & 0xffull);
-                const uint64_t match = __ballot(pi < n_xcd && pj < n_xcd && irank_j == xrank_i);
-                const uint32_t mybyte = (uint32_t)((match >> (8 * (x & 7))) & 0xffull);     // lanes x < 8: row x
-                const int mine = mybyte ? __builtin_ctz(mybyte) : 0;
-                const int wm = __shfl(w, mine, 64);
-                if (x < n_xcd && mybyte && wm > 0) {   // (the last group may have fewer super tiles than XCDs)
-                    sdeal[x * rounds + cnt] = (uint16_t)(g2 * n_xcd + mine);
-                    cnt++;
-                    load += wm;
-                }
-            }
-            // super tiles with nothing kept (ranks n_ne ..) fill the XCDs' remaining slots in lane order
-            const int room = x < n_xcd ? rounds - cnt : 0;
-            int before = room;
-#pragma unroll
-            for (int off = 1; off < MAX_XCD; off <<= 1) {
-                const int o = __shfl_up(before, off, 64);
-                if (x >= off) before += o;
-            }
-            before -= room;
-            for (int c = 0; c < room; c++) {
-                const int r = n_ne + before + c;
-                sdeal[x * rounds + cnt + c] = r < n_super ? (uint16_t)r : (uint16_t)0xffffu;   // 0xffff: no super tile
-            }
-        }
-        __syncthreads();
-    }
 
-    // macro tile of XCD x at raw position p (round-major, then slot inside the super tile), or -1
-    auto macro_at = [&](int x, int p) -> int {
-        const int round = p / (SUPER_M * SUPER_N), slot = p % (SUPER_M * SUPER_N);
-        if (p >= P) return -1;
-        if (deal == DEAL_FLAT) return (p < flat_chunk && x * flat_chunk + p < nMacM * nMacN) ? x * flat_chunk + p : -1;
-        const int sr = deal != DEAL_SNAKE ? (int)sdeal[x * rounds + round] : round * n_xcd + ((round & 1) ? n_xcd - 1 - x : x);
-        if (sr >= n_super) return -1;
-        const int origin = srank_id[sr];
-        const int mi = (origin >> 16) + slot / SUPER_N, mj = (origin & 0xffff) + slot % SUPER_N;
-        return (mi < nMacM && mj < nMacN) ? mi * nMacN + mj : -1;
+    // rank of XCD x's r-th super tile; n_super and beyond: none
+    auto dealt = [&](int x, int r) -> int {
+        if (deal == DEAL_SNAKE) return r * n_xcd + ((r & 1) ? n_xcd - 1 - x : x);
+        return r < s_cnt[x] ? (int)sdeal[x * rounds + r] : n_ne + s_before[x] + r - s_cnt[x];
     };
-    // one wave per XCD: computing macro tiles to the front in raw order, empty ones from the back
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    auto sid_of = [&](int origin) -> int { return (origin >> 16) / SUPER_M * nSupN + (origin & 0xffff) / SUPER_N; };
+    // computing macro tiles go to the front of the XCD's sequence in order, empty ones to the back: one wave
+    // per XCD adds up how many of each come before its r-th super tile
     if (wave < n_xcd) {
         const int x = wave;
-        int nall = 0;                            // macro tiles in this XCD's sequence (no memory access)
-        for (int p0 = 0; p0 < P; p0 += 64) nall += __builtin_popcountll(__ballot(macro_at(x, p0 + lane) >= 0));
         int nc = 0, ne = 0;
-        const uint64_t below = (1ull << lane) - 1ull;
-        // (loads of UN chunks are issued together: the wave is alone here and each one is an L2 round trip)
-        constexpr int UN = 8;
-        for (int p0 = 0; p0 < P; p0 += 64 * UN) {
-            int mm[UN], ww[UN];
-#pragma unroll
-            for (int u = 0; u < UN; u++) {
-                mm[u] = macro_at(x, p0 + u * 64 + lane);
-                ww[u] = mm[u] >= 0 ? g.macro_work[mm[u]] : 0;
+        for (int r0 = 0; r0 < rounds; r0 += 64) {
+            const int r = r0 + lane, sr = r < rounds ? dealt(x, r) : n_super;
+            int c = 0, e = 0;
+            if (sr < n_super) {
+                const int origin = srank_id[sr], hm = nMacM - (origin >> 16), wn = nMacN - (origin & 0xffff);
+                c = __builtin_popcount(scomp[sid_of(origin)]);
+                e = (hm < SUPER_M ? hm : SUPER_M) * (wn < SUPER_N ? wn : SUPER_N) - c;
             }
+            uint32_t incl = (uint32_t)c | (uint32_t)e << 16;              // (64 super tiles: at most 2048 of each)
+            const uint32_t own = incl;
 #pragma unroll
-            for (int u = 0; u < UN; u++) {
-                const bool comp = mm[u] >= 0 && ww[u] > 0, empty = mm[u] >= 0 && ww[u] <= 0;
-                const uint64_t bc = __ballot(comp), be = __ballot(empty);
-                if (comp) g.order[x * P + nc + __builtin_popcountll(bc & below)] = mm[u];
-                if (empty) g.order[x * P + nall - 1 - (ne + __builtin_popcountll(be & below))] = mm[u];
-                nc += __builtin_popcountll(bc);
-                ne += __builtin_popcountll(be);
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t o = __shfl_up(incl, off, 64);
+                if (lane >= off) incl += o;
             }
+            const uint32_t last = __builtin_amdgcn_readlane(incl, 63), first = incl - own;
+            if (r < rounds) {
+                swork[x * rounds + r] = nc + (int)(first & 0xffffu);
+                sempty[x * rounds + r] = ne + (int)(first >> 16);
+            }
+            nc += (int)(last & 0xffffu);
+            ne += (int)(last >> 16);
         }
         if (lane == 0) {
+            s_nall[x] = nc + ne;
             g.sched[x] = nc;
-            g.sched[MAX_XCD + x] = nall;
+            g.sched[MAX_XCD + x] = nc + ne;
             g.sched[2 * MAX_XCD + x] = 0;      // ticket counter of the persistent GEMM
         }
     }
     if (threadIdx.x == 0) g.kept_total[0] = (int64_t)total;
+    __syncthreads();
+    // the sequences, all waves: XCD x by 16 / n_xcd of them, half a wave per super tile, lane = macro tile
+    {
+        const int x = wave % n_xcd, per = 2 * 16 / n_xcd, slot = lane % (SUPER_M * SUPER_N);
+        const int nall = s_nall[x], cnt = deal == DEAL_SNAKE ? 0 : s_cnt[x], rest = deal == DEAL_SNAKE ? 0 : n_ne + s_before[x] - cnt;
+        const uint32_t before = (1u << slot) - 1u;
+        for (int r = wave / n_xcd * 2 + lane / (SUPER_M * SUPER_N); r < rounds; r += per) {
+            const int sr = deal == DEAL_SNAKE ? r * n_xcd + ((r & 1) ? n_xcd - 1 - x : x) : (r < cnt ? (int)sdeal[x * rounds + r] : rest + r);
+            if (sr >= n_super) continue;
+            const int origin = srank_id[sr], oi = origin >> 16, oj = origin & 0xffff;
+            const int mi = oi + slot / SUPER_N, mj = oj + slot % SUPER_N;
+            if (mi >= nMacM || mj >= nMacN) continue;
+            const uint32_t comp = scomp[sid_of(origin)];
+            const int c = __builtin_popcount(comp & before);
+            const int wn = nMacN - oj < SUPER_N ? nMacN - oj : SUPER_N;       // (slots before this one that exist, less the computing ones)
+            const int q = (comp >> slot) & 1u ? swork[x * rounds + r] + c
+                                              : nall - 1 - (sempty[x * rounds + r] + (slot / SUPER_N) * wn + slot % SUPER_N - c);
+            g.order[x * P + q] = mi * nMacN + mj;
+        }
+    }
 }
 
 // Per-tile ascending list of kept k (the reference's offset[], cuSpAMM.cu:315-325)

@@ -115,16 +115,18 @@ inline size_t order_lds_bytes(int tile, int64_t nbM, int64_t nbN) {
     const int MT = 256 / tile;
     const int64_t nMacM = (nbM + MT - 1) / MT, nMacN = (nbN + MT - 1) / MT;
     const size_t n_super = (size_t)(((nMacM + SUPER_M - 1) / SUPER_M) * ((nMacN + SUPER_N - 1) / SUPER_N));
-    // length + origin by rank, and for the greedy deal a table of at most MAX_XCD x rounds (or
-    // n_super parked ranks) 16-bit entries; beyond 512 super tiles the ranking sorts indices
-    // padded to a power of two in the second array's place
+    // two positions (first: the length) and the set of computing macro tiles by super tile, origin by rank, for the
+    // table deals 16-bit entries; beyond 512 super tiles the ranking may sort indices padded to a power of
+    // two in the place of the last two
     size_t np2 = 1024;
     while (np2 < n_super) np2 *= 2;
-    const size_t tables = n_super * 2 * sizeof(int) + (n_super <= (size_t)LPT_MAX_SUPER ? (n_super + 2 * MAX_XCD) * sizeof(uint16_t) * 2 : 0);
-    const size_t sorting = n_super > 512 ? (n_super + np2) * sizeof(int) : 0;
-    return tables > sorting ? tables : sorting;
+    const size_t fixed = (3 * n_super + 2 * MAX_XCD) * sizeof(int);
+    const size_t tables = n_super * sizeof(int) + (n_super <= (size_t)LPT_MAX_SUPER ? (n_super + 2 * MAX_XCD) * sizeof(uint16_t) : 0);
+    const size_t sorting = n_super > 512 ? np2 * sizeof(int) : 0;
+    return fixed + (tables > sorting ? tables : sorting);
 }
-inline size_t order_lds_limit() { return 64 * 1024; }
+constexpr int ORDER_MAX_SUPER = 8192;
+inline size_t order_lds_limit() { return (size_t)(4 * ORDER_MAX_SUPER + 2 * MAX_XCD) * sizeof(int); }
 hipError_t gate_init();   // one-time kernel attribute set-up
 hipError_t launch_gate(const GateBuffers &g, int64_t nbM, int64_t nbK, int64_t nbN, int tile,
                        float tau, int n_xcd, int chunk_cap, hipStream_t s);
