@@ -23,7 +23,7 @@
 // Whole calls, norm maps and the multiply behind them included: 5024 x 4128 x 3168 at
 // tile 32 to a kept fraction 667 -> 142 us, the reference's tuned 2048^3 (8 of at most
 // 20 rounds) 381 -> 118 us.
-#include "spamm_internal.h"
+#include "reduce_device.h"
 
 namespace spamm {
 
@@ -77,33 +77,6 @@ __device__ __forceinline__ void for_products(const float *__restrict__ nA, const
         for (int jj = 0; jj < TAU_JB; jj++)
             if (j0 + jj < nbN) f(a * b[jj], live);
     }
-}
-
-template <typename T>
-__device__ __forceinline__ T agent_load(const T *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ void agent_store(T *p, T v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// True in every thread of the workgroup that finishes last.  What workgroups hand to it goes through
-// agent-scope atomics only, which are performed where all XCDs see them: once a wave's have returned
-// (the wait on the counter) and the workgroup has met, one relaxed add on the ticket says so.  (A
-// release fence writes the XCD's whole L2 back: in every wave it took 25 us of a pass of 1100 waves,
-// in one thread per workgroup still 2.)  The ticket is put back for the next launch.
-__device__ __forceinline__ bool last_workgroup(unsigned int *ticket) {
-    __shared__ unsigned int s_last;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const unsigned int t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_last = t == gridDim.x - 1;
-        if (s_last) agent_store(ticket, 0u);
-    }
-    __syncthreads();
-    return s_last != 0;
 }
 
 // One digit of the select: histogram of the PASS-th digit over the products whose higher bits equal

@@ -1,0 +1,35 @@
+// Results that all workgroups of a launch contribute to, finished by the one that ends last
+// (kernels_tau.hip, kernels_tools.hip).
+#pragma once
+#include "spamm_internal.h"
+
+namespace spamm {
+
+template <typename T>
+__device__ __forceinline__ T agent_load(const T *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void agent_store(T *p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// True in every thread of the workgroup that finishes last.  What workgroups hand to it goes through
+// agent-scope atomics only, which are performed where all XCDs see them: once a wave's have returned
+// (the wait on the counter) and the workgroup has met, one relaxed add on the ticket says so.  (A
+// release fence writes the XCD's whole L2 back: in every wave it took 25 us of a pass of 1100 waves,
+// in one thread per workgroup still 2.)  The ticket is put back for the next launch.
+__device__ __forceinline__ bool last_workgroup(unsigned int *ticket) {
+    __shared__ unsigned int s_last;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned int t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = t == gridDim.x - 1;
+        if (s_last) agent_store(ticket, 0u);
+    }
+    __syncthreads();
+    return s_last != 0;
+}
+
+}  // namespace spamm

@@ -38,11 +38,15 @@ struct DevBuf {
 
 }  // namespace
 
+// Per-tile results up to this many are written to pinned host memory by the kernel itself; more are copied.
+static constexpr size_t TILE_RESULTS_MAX = 65536;
+
 // Pinned host memory of a context, written by kernels.
 struct HostResults {
     TauState select;
     TauCounts counts;
     TauResult tune;
+    double report[3];
 };
 
 // Everything a multiply leaves behind: the shape it ran at, what is valid, and
@@ -88,6 +92,9 @@ struct spamm_ctx : Workspace {
 
     DevBuf staging;   // read-back staging / decay table
     DevBuf tauws;     // tau selection workspace
+    DevBuf reportws;  // error report workspace
+    double *tile_results = nullptr;   // pinned, TILE_RESULTS_MAX doubles at most: per-tile results of small outputs
+    size_t tile_results_cap = 0;
     HostResults *results = nullptr;   // pinned: small results that a kernel writes and the host reads after a wait
 
     hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -280,6 +287,8 @@ int spamm_destroy(spamm_ctx *c) {
     free_workspace(c->parked);
     if (c->staging.p) (void)hipFree(c->staging.p);
     if (c->tauws.p) (void)hipFree(c->tauws.p);
+    if (c->reportws.p) (void)hipFree(c->reportws.p);
+    if (c->tile_results) (void)hipHostFree(c->tile_results);
     if (c->results) (void)hipHostFree(c->results);
     for (int i = 0; i < 5; i++)
         if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
@@ -670,6 +679,24 @@ int spamm_multiply_f16(spamm_ctx *c, const spamm_params *p, const void *dAh, con
     return multiply_any(c, p, dAh, dBh, true, dC);
 }
 
+static int ensure_results(spamm_ctx *c) {
+    if (c->results) return SPAMM_OK;
+    void *p = nullptr;
+    HIPCHK(c, hipHostMalloc(&p, sizeof(HostResults), hipHostMallocDefault));
+    c->results = (HostResults *)p;
+    return SPAMM_OK;
+}
+
+static int report_prepare(spamm_ctx *c, int64_t rows) {
+    int rc = ensure_results(c);
+    if (rc) return rc;
+    const size_t bytes = report_workspace_bytes(rows, c->N, c->n_cu);
+    if (c->reportws.cap >= bytes) return SPAMM_OK;
+    if ((rc = ensure(c, c->reportws, bytes))) return rc;
+    HIPCHK(c, launch_clear_report(c->reportws.p, c->stream));
+    return SPAMM_OK;
+}
+
 int spamm_error_vs_dense_f64(spamm_ctx *c, const float *dC, int64_t row0, int64_t row1, double *out3) {
     if (!c || !dC || !out3) return SPAMM_EINVAL;
     if (static_stale(c)) return SPAMM_ESTATE;
@@ -678,12 +705,11 @@ int spamm_error_vs_dense_f64(spamm_ctx *c, const float *dC, int64_t row0, int64_
         return SPAMM_EINVAL;
     int rc = set_device(c);
     if (rc) return rc;
-    if ((rc = ensure(c, c->tauws, tau_workspace_bytes()))) return rc;
-    double *d = (double *)c->tauws.p;
-    HIPCHK(c, launch_error_vs_dense(c->packedA.p, c->packedB.p, c->M, c->K, c->N, c->tile, dC, row0, row1, d,
-                                    c->stream));
-    double sq[3];
-    if ((rc = copy_out(c, d, sq, sizeof(sq)))) return rc;
+    if ((rc = report_prepare(c, row1 - row0))) return rc;
+    double *sq = c->results->report;
+    HIPCHK(c, launch_error_vs_dense(c->packedA.p, c->packedB.p, c->K, c->N, c->tile, dC, row0, row1, c->n_cu, c->reportws.p,
+                                    sq, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
     for (int i = 0; i < 3; i++) out3[i] = sqrt(sq[i]);
     return SPAMM_OK;
 }
@@ -691,18 +717,15 @@ int spamm_error_vs_dense_f64(spamm_ctx *c, const float *dC, int64_t row0, int64_
 int spamm_dropped_bound(spamm_ctx *c, float tau, double *out) {
     if (!c || !out || tau != tau) return SPAMM_EINVAL;
     if (static_stale(c)) return SPAMM_ESTATE;
-    Shape s;
     if (!c->tile || !c->M || !c->K || !c->N || !c->nm_a || !c->nm_b) return SPAMM_ESTATE;   // both norm maps, same K and tile
     int rc = set_device(c);
     if (rc) return rc;
-    s = shape_of(c);
-    if ((rc = ensure(c, c->tauws, tau_workspace_bytes()))) return rc;
-    double *d = (double *)c->tauws.p;
-    HIPCHK(c, launch_dropped_bound((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, tau, d,
-                                   nullptr, c->stream));
-    double sq;
-    if ((rc = copy_out(c, d, &sq, sizeof(sq)))) return rc;
-    *out = sqrt(sq);
+    const Shape s = shape_of(c);
+    if ((rc = report_prepare(c, 0))) return rc;
+    HIPCHK(c, launch_dropped_bound((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, tau, c->reportws.p,
+                                   c->results->report, nullptr, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    *out = sqrt(c->results->report[0]);
     return SPAMM_OK;
 }
 
@@ -714,11 +737,23 @@ int spamm_dropped_bound_tiles(spamm_ctx *c, float tau, double *host_out) {
     if (rc) return rc;
     const Shape s = shape_of(c);
     const size_t nt = (size_t)s.nbM * s.nbN;
-    if ((rc = ensure(c, c->tauws, tau_workspace_bytes()))) return rc;
-    if ((rc = ensure(c, c->staging, nt * 8))) return rc;
-    HIPCHK(c, launch_dropped_bound((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, tau,
-                                   (double *)c->tauws.p, (double *)c->staging.p, c->stream));
-    return copy_out(c, c->staging.p, host_out, nt * 8);
+    const bool pinned = nt <= TILE_RESULTS_MAX;
+    if (pinned && c->tile_results_cap < nt) {
+        if (c->tile_results) (void)hipHostFree(c->tile_results);
+        c->tile_results = nullptr;
+        c->tile_results_cap = 0;
+        void *p = nullptr;
+        HIPCHK(c, hipHostMalloc(&p, nt * 8, hipHostMallocDefault));
+        c->tile_results = (double *)p;
+        c->tile_results_cap = nt;
+    }
+    if (!pinned && (rc = ensure(c, c->staging, nt * 8))) return rc;
+    HIPCHK(c, launch_dropped_bound((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, tau, nullptr, nullptr,
+                                   pinned ? c->tile_results : (double *)c->staging.p, c->stream));
+    if (!pinned) return copy_out(c, c->staging.p, host_out, nt * 8);
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    memcpy(host_out, c->tile_results, nt * 8);
+    return SPAMM_OK;
 }
 
 // ---- input adapters (host side; getMatrixFromCSV / getMatrixFromMTX, tool.cu:282-366)
@@ -798,11 +833,7 @@ static int tau_prepare(spamm_ctx *c, Shape *s) {
     int rc = set_device(c);
     if (rc) return rc;
     *s = shape_of(c);
-    if (!c->results) {
-        void *p = nullptr;
-        HIPCHK(c, hipHostMalloc(&p, sizeof(HostResults), hipHostMallocDefault));
-        c->results = (HostResults *)p;
-    }
+    if ((rc = ensure_results(c))) return rc;
     return ensure(c, c->tauws, tau_workspace_bytes());
 }
 

@@ -91,13 +91,15 @@ hipError_t launch_normmap_ab(const void *X, bool in16, int64_t n, int tile, void
 bool normmap_pair_fits(bool in16, bool tau_aware, int64_t M, int64_t K, int64_t N, int tile);
 hipError_t launch_normmap_pair(const void *A, const void *Bm, bool in16, int64_t M, int64_t K, int64_t N, int tile, void *packedA,
                                float *nmA, void *packedB, float *nmB, float *nmBt, float tau_skip, int64_t *kept, hipStream_t s);
-// error report tooling (kernels_tools.hip)
-hipError_t launch_error_vs_dense(const void *packedA, const void *packedB, int64_t M, int64_t K, int64_t N,
-                                 int tile, const float *C, int64_t row0, int64_t row1, double *out3,
-                                 hipStream_t s);
-// out1 += sum over tiles of s_ij^2, s_ij = sum_{k dropped} nA[i,k]*nB[k,j]; per_tile (optional): s_ij
-hipError_t launch_dropped_bound(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN,
-                                float tau, double *out1, double *per_tile, hipStream_t s);
+// error report tooling (kernels_tools.hip).  Results go to host_out, pinned host memory: valid once the stream has been
+// waited for.  The workspace's ticket is zero between launches (launch_clear_report once after allocation).
+size_t report_workspace_bytes(int64_t rows, int64_t N, int n_cu);      // rows = 0: the bound only
+hipError_t launch_clear_report(void *workspace, hipStream_t s);
+hipError_t launch_error_vs_dense(const void *packedA, const void *packedB, int64_t K, int64_t N, int tile, const float *C,
+                                 int64_t row0, int64_t row1, int n_cu, void *workspace, double *host_out3, hipStream_t s);
+// *host_out (optional) = sum over tiles of s_ij^2, s_ij = sum_{k dropped} nA[i,k]*nB[k,j]; per_tile (optional): s_ij
+hipError_t launch_dropped_bound(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, float tau,
+                                void *workspace, double *host_out, double *per_tile, hipStream_t s);
 hipError_t launch_unpack(const void *packed, int64_t rows, int64_t cols, int tile, int role,
                          uint16_t *out, hipStream_t s);
 hipError_t launch_transpose_normmap(const float *nB, int64_t nbK, int64_t nbN, float *nBt,
