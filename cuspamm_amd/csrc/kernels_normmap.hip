@@ -40,8 +40,9 @@ __device__ __forceinline__ float butterfly64(float v) {
     return v;
 }
 
-// One workgroup (4 waves) per strip of B rows x SW columns (SW/B tiles; SW = 256 for fp32 input,
-// 512 for fp16 input: a strip row is 1 KiB either way and is read by one wave-wide load).  The
+// One workgroup per strip of B rows x SW columns (SW/B tiles; SW = 256 for fp32 input,
+// 512 for fp16 input: a strip row is 1 KiB either way and is read by one wave-wide load; tiles of 128
+// mostly SW = 128, one tile per strip, two or four rows per load).  The
 // tiles of a strip pass through LDS in PH phases of SW/B/PH tiles each, sized so that at most
 // ~42 KiB are resident and three workgroups fit a CU; all loads are issued before the first phase.
 //   load    a lane takes whole 8-row groups (wave w: groups w, w + 4, ...); all loads of a lane
@@ -56,8 +57,6 @@ __device__ __forceinline__ float butterfly64(float v) {
 //   store   after one barrier: the tiles are copied out with contiguous 1 KiB wave stores (a
 //           packed tile is one contiguous block in memory), and one wave per tile applies the
 //           canonical reduction.
-// (The phased fp32 A role is held to three waves per SIMD: it gains more from a third resident
-// workgroup than it loses to a few spilled registers; the B role would spill far more.)
 template <int B, int SW, int PH>
 struct NormCfg {
     static constexpr int TPP = SW / B / PH;          // tiles resident in LDS together
@@ -83,12 +82,17 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
     // columns (4 floats, or 8 halves for fp16 input: the strip is then 512 columns wide); wave w
     // takes the 8-row groups w, w + 4, ...  A lane's columns lie in one tile; with PH > 1 the tiles
     // pass through LDS PH phases one after the other and in phase ph only the lanes of that
-    // phase's tiles stage their data.  (Tile 128 used to split the waves between its two tiles at
-    // load time -- 512-byte row segments -- which measured 0-4 % slower than whole rows.)
+    // phase's tiles stage their data.  Tiles of 128 as strips of several in as many phases put up to
+    // 128 KiB in registers per workgroup, staged, copied and reduced in turns with little else on the CU
+    // to read meanwhile; as single tiles (SW = B: a load is rows of several 8-row groups) a workgroup is
+    // what it is at tile 64.  Both passes, phased -> single: fp32 1024^2 18.6 -> 5.6 us, 4096^2 50 -> 36,
+    // A = B in one read 8192^2 145 -> 90; fp16 1024^2 13 -> 4.6, 16384^2 tau-aware 302 -> 276.
     constexpr int EPL = IN16 ? 8 : 4;                  // columns per lane
-    static_assert(SW == 64 * EPL, "a strip row is one wave-wide load");
-    constexpr int GSTEP = NWV;                         // 8-row groups between a lane's groups (one per wave)
-    static_assert(B % (8 * NWV) == 0, "every wave takes whole 8-row groups");
+    constexpr int LPR = SW / EPL;                      // lanes per strip row
+    constexpr int GPW = 64 / LPR;                      // 8-row groups a wave-wide load touches (a row of each)
+    static_assert(LPR * GPW == 64 && (GPW == 1 || PH == 1), "a wave-wide load is whole strip rows");
+    constexpr int GSTEP = NWV * GPW;                   // 8-row groups between a lane's groups
+    static_assert(B % (8 * GSTEP) == 0, "every wave takes whole 8-row groups");
     static_assert(PH == 1 || PH == 2 || PH == 4, "phases are made of whole waves");
     constexpr int QN = L::QN, QS = L::QS, TS = L::TS, PITCH = L::PITCH, CH = L::CH;
     constexpr int VPT = B * B / 8;        // 16-byte vectors per tile
@@ -99,8 +103,8 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
     const int64_t I = strip / nstrip;                 // tile row of the strip
     const int64_t sc = strip % nstrip;
     const int64_t col0 = sc * SW;
-    const int cl = EPL * lane;                        // first column of this lane inside the strip
-    const int g0 = wave;                              // first 8-row group of this lane; then every GSTEP-th
+    const int cl = EPL * (lane % LPR);                // first column of this lane inside the strip
+    const int g0 = wave * GPW + lane / LPR;           // first 8-row group of this lane; then every GSTEP-th
     const int t = cl / B, cin = cl % B;               // tile of the strip, column inside the tile
     const bool valid = col0 + cl < cols;
     const int64_t eoff = (I * B) * ld + col0 + cl;
@@ -320,7 +324,7 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
 }
 
 template <int B, int ROLE, int SW, bool IN16, int PH = 1, int NWV = 4>
-__global__ __launch_bounds__(64 * NWV, (PH > 1 && ROLE == 0 && !IN16 && NWV == 4) ? 3 : 1) void k_normmap(
+__global__ __launch_bounds__(64 * NWV, 1) void k_normmap(
     const void *__restrict__ Xv, int64_t ld, int64_t cols, int64_t nbr, int64_t nbc, int64_t nstrip, uint4 *__restrict__ packed,
     float *__restrict__ nm, float *__restrict__ nmT, uint4 *__restrict__ packed2, float *__restrict__ nm2,
     const float *__restrict__ rowmax, float tau_skip, int64_t *__restrict__ kept) {
@@ -459,16 +463,21 @@ static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int 
                 break;
             }
             k_normmap<64, ROLE, SW, IN16, IN16 ? 2 : 1><<<grid, 256, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept); break;
-        // tile 128: eight waves per workgroup (two 8-row groups per lane instead of four: no register
-        // spills, more loads in flight) where that measured faster -- the fp32 A role (3.36 -> 3.07 ms at
-        // N = 65536) and both roles on fp16 input (2.02 -> 1.85, 1.95 -> 1.90 ms) -- but not the fp32 B
-        // role (3.26 -> 3.93 ms) nor, by extension, the single pass for A = B
+        // tile 128: strips of one tile.  Only the fp32 B role of a large matrix keeps strips of two tiles in two phases by
+        // four waves: N = 32768 830 against 867 us, 16384 225 / 231, 12800 159 / 158, 8192 72 / 67.
         case 128:
-            if constexpr (IN16 || ROLE == 0) {
-                k_normmap<128, ROLE, SW, IN16, IN16 ? 4 : 2, 8><<<grid, 512, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept);
-                break;
+            if constexpr (IN16) {
+                if constexpr (ROLE == 2) return hipErrorInvalidValue;      // (two passes, or the pair, are faster)
+                else k_normmap<128, ROLE, 128, true, 1, 4><<<(unsigned)(nbr * nbc), 256, 0, s>>>(X, cols, cols, nbr, nbc, nbc, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept);
+            } else {
+                if constexpr (ROLE == 1)
+                    if (grid > 6000u) {
+                        k_normmap<128, ROLE, SW, false, 2, 4><<<grid, 256, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept);
+                        break;
+                    }
+                k_normmap<128, ROLE, 128, false, 1, 8><<<(unsigned)(nbr * nbc), 512, 0, s>>>(X, cols, cols, nbr, nbc, nbc, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept);
             }
-            k_normmap<128, ROLE, SW, IN16, IN16 ? 4 : 2><<<grid, 256, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept); break;
+            break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -480,10 +489,9 @@ hipError_t launch_normmap_a(const void *X, bool in16, int64_t rows, int64_t cols
                 : launch_normmap<0, false>(X, rows, cols, tile, packed, nm, nullptr, kept, s, nullptr, nullptr, rowmax, tau_skip);
 }
 
-template <int B, int PH, int NWV, bool IN16>
+template <int B, int SW, int PH, int NWV, bool IN16>
 static void launch_pair(const void *A, const void *Bm, int64_t nbM, int64_t nbK, int64_t nbN, void *packedA, void *packedB,
                         float *nmA, float *nmB, float *nmBt, float tau_skip, int64_t *kept, hipStream_t s) {
-    constexpr int SW = IN16 ? 512 : 256;
     const int64_t strips_a = (nbK * B + SW - 1) / SW, strips_b = (nbN * B + SW - 1) / SW;
     const unsigned n_b = (unsigned)(nbK * strips_b), n_a = (unsigned)(nbM * strips_a);
     k_normmap_pair<B, SW, IN16, PH, NWV><<<n_a + n_b, 64 * NWV, 0, s>>>(A, Bm, nbM, nbK, nbN, n_b, strips_a, strips_b, (uint4 *)packedA,
@@ -503,13 +511,16 @@ bool normmap_pair_fits(bool in16, bool tau_aware, int64_t M, int64_t K, int64_t 
 hipError_t launch_normmap_pair(const void *A, const void *Bm, bool in16, int64_t M, int64_t K, int64_t N, int tile, void *packedA,
                                float *nmA, void *packedB, float *nmB, float *nmBt, float tau_skip, int64_t *kept, hipStream_t s) {
     const int64_t nbM = M / tile, nbK = K / tile, nbN = N / tile;
-#define SPAMM_PAIR(T, PH16, NWV, PH32)                                                                                          \
-    if (in16) launch_pair<T, PH16, NWV, true>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, kept, s);        \
-    else launch_pair<T, PH32, NWV, false>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, kept, s)
+#define SPAMM_PAIR(T, PH16, NWV, SW32)                                                                                          \
+    if (in16) launch_pair<T, 512, PH16, NWV, true>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, kept, s);        \
+    else launch_pair<T, SW32, 1, NWV, false>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, kept, s)
     switch (tile) {
-        case 32: SPAMM_PAIR(32, 1, 4, 1); break;
-        case 64: SPAMM_PAIR(64, 2, 8, 1); break;
-        case 128: SPAMM_PAIR(128, 4, 8, 2); break;
+        case 32: SPAMM_PAIR(32, 1, 4, 256); break;
+        case 64: SPAMM_PAIR(64, 2, 8, 256); break;
+        case 128:
+            if (in16) launch_pair<128, 128, 1, 4, true>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, kept, s);
+            else launch_pair<128, 128, 1, 8, false>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, kept, s);
+            break;
         default: return hipErrorInvalidValue;
     }
 #undef SPAMM_PAIR

@@ -540,11 +540,10 @@ static int multiply_any(spamm_ctx *c, const spamm_params *p, const void *dA, con
     if (reuse_b && !(c->have_b && c->tile == p->tile && c->K == p->K && c->N == p->N)) return SPAMM_ESTATE;
     bool a_eq_b = (p->flags & SPAMM_FLAG_A_EQ_B) != 0;
     if (a_eq_b && (reuse_a || reuse_b || dA != dB || p->M != p->K || p->K != p->N)) return SPAMM_EINVAL;
-    // tile 128: the single pass for both roles needs every register of a SIMD for one wave and is slower
-    // than the two passes (1.44 against 1.34 ms per multiply at N = 16384): the flag then only asserts
-    // dA == dB, and the two ordinary passes (with their full tau-aware pruning) run
-    if (a_eq_b && p->tile == 128) a_eq_b = false;
     const bool prune = (p->flags & SPAMM_FLAG_PRUNE) != 0 && p->tau > 0.0f;
+    // tile 128 on fp16 input, and tau-aware: the flag only asserts dA == dB, and the ordinary passes (with
+    // their full tau-aware pruning) run
+    if (a_eq_b && p->tile == 128 && (in16 || prune)) a_eq_b = false;
     const bool pair = !a_eq_b && !reuse_a && !reuse_b && normmap_pair_fits(in16, prune, p->M, p->K, p->N, p->tile);
     if (a_eq_b || pair) {
         // one launch for both operand roles: one read of the matrix where A = B (the reference's A = B runs
