@@ -19,10 +19,13 @@
 // walk over the 2048 bins took 30-160 us of dependent loads per pass, and
 // double-precision atomics on one address are compare-and-swap loops: 15 us of 256
 // workgroups' time at 2.6e5 products).  The decision is written straight to pinned
-// host memory, so the host waits for the stream once and copies nothing.
+// host memory, where the host looks for it, and every launch leaves the counters
+// at zero.  Few products (k_tau_small_*) are held by one workgroup, and all passes
+// are one launch.
 // Whole calls, norm maps and the multiply behind them included: 5024 x 4128 x 3168 at
-// tile 32 to a kept fraction 667 -> 142 us, the reference's tuned 2048^3 (8 of at most
-// 20 rounds) 381 -> 118 us.
+// tile 32 to a kept fraction 667 -> 138 us, the reference's tuned 2048^3 (8 of at most
+// 20 rounds) 381 -> 93 us.
+#include "gemm_device.h"
 #include "reduce_device.h"
 
 namespace spamm {
@@ -30,9 +33,11 @@ namespace spamm {
 constexpr int TAU_NTH = 1024;               // threads per workgroup
 constexpr int TAU_NW = TAU_NTH / 64;
 constexpr int TAU_MAXB = 256;               // one workgroup per CU at most: every one of them adds its part to the same few words
-constexpr int TAU_JB = 16;                  // output columns whose products share one load of nA
+constexpr int TAU_JB_COUNT = 16;            // output columns whose products share one load of nA
+constexpr int TAU_JB_TREE = 4;              // (where a product is much work: more waves, and code that is fetched sooner)
 constexpr int TAU_COPIES = 2;               // global copies of a histogram: workgroups that add to one copy queue on its busy bins
 constexpr int TAU_NODES = 15;               // thresholds of four rounds
+constexpr int64_t TAU_SMALL_MAX = 24 * TAU_NTH;   // products that one workgroup holds
 
 struct TauTune {
     double norm, up, down, rate;
@@ -55,7 +60,7 @@ size_t tau_workspace_bytes() { return sizeof(TauWorkspace); }
 // live) runs in all lanes; `live` is false in lanes beyond the last k.  A wave's step is one round trip
 // of 17 loads and some hundred instructions, so the steps are kept small and spread over as many waves
 // as there are (whole rows of k per wave: 22 us instead of 15 for the last pass over 1.7e7 products).
-template <typename F>
+template <int TAU_JB, typename F>
 __device__ __forceinline__ void for_products(const float *__restrict__ nA, const float *__restrict__ nBt, int nbM, int nbK,
                                              int nbN, F &&f) {
     const int lane = threadIdx.x & 63;
@@ -87,7 +92,8 @@ __device__ __forceinline__ void for_products(const float *__restrict__ nA, const
 template <int PASS>
 __global__ __launch_bounds__(TAU_NTH) void k_tau_hist(const float *__restrict__ nA, const float *__restrict__ nBt, int nbM,
                                                       int nbK, int nbN, unsigned long long total, unsigned long long want0,
-                                                      TauWorkspace *__restrict__ ws, TauState *__restrict__ host_out) {
+                                                      TauWorkspace *__restrict__ ws, TauState *__restrict__ host_out,
+                                                      unsigned long long *__restrict__ host_seq, unsigned long long seq) {
     constexpr int BITS = PASS == 2 ? 10 : 11, SHIFT = PASS == 0 ? 21 : (PASS == 1 ? 10 : 0);
     constexpr int NB = 1 << BITS, COPIES = 4, PER = NB / TAU_NTH;
     __shared__ unsigned int lh[NB * COPIES];
@@ -99,7 +105,7 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_hist(const float *__restrict__ 
     if (PASS) prev = ws->st;
     const uint32_t prefix = prev.prefix;
     unsigned long long zeros = 0;
-    for_products(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
+    for_products<TAU_JB_COUNT>(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
         const bool pos = live && p > 0.0f;                        // NaN counts as 0
         const uint32_t key = __builtin_bit_cast(uint32_t, p);
         if (PASS == 0) zeros += __builtin_popcountll(__ballot(live && !(p > 0.0f)));
@@ -126,6 +132,12 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_hist(const float *__restrict__ 
 #pragma unroll
         for (int r = 0; r < TAU_COPIES; r++) part[e][r] = agent_load(&ws->hist[PASS][r][NB - 1 - (int)threadIdx.x * PER - e]);
     const unsigned long long n_zero = PASS == 0 ? agent_load(&ws->zeros) : 0ull;
+    // what this pass counted in is zero again for the next selection
+#pragma unroll
+    for (int e = 0; e < PER; e++)
+#pragma unroll
+        for (int r = 0; r < TAU_COPIES; r++)
+            if (part[e][r]) agent_store(&ws->hist[PASS][r][NB - 1 - (int)threadIdx.x * PER - e], 0ull);
 #pragma unroll
     for (int e = 0; e < PER; e++) {
         h[e] = 0;
@@ -145,6 +157,7 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_hist(const float *__restrict__ 
     for (int w = 0; w < wave; w++) above += s_sum[w];
     unsigned long long want = prev.want;
     if (PASS == 0) {
+        if (threadIdx.x == 0) agent_store(&ws->zeros, 0ull);      // (all threads have read it: the barrier above)
         const unsigned long long positive = total - n_zero;
         want = want0 < positive ? want0 : positive;               // zero tail: settle for the smallest positive product
         if (positive == 0 && threadIdx.x == 0) {                  // nothing but zeros: only tau = 0 keeps anything
@@ -154,7 +167,7 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_hist(const float *__restrict__ 
         }
     }
     if (want == 0) {                                              // (the passes after such a first one)
-        if (PASS == 2 && threadIdx.x == 0) *host_out = prev;
+        if (PASS == 2 && threadIdx.x == 0) publish_result(host_out, prev, host_seq, seq);
         return;
     }
     if (above < want && want <= above + mine) {
@@ -168,11 +181,24 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_hist(const float *__restrict__ 
                 st.tau_bits = st.prefix;
                 st.kept = st.greater + h[e];
                 ws->st = st;
-                if (PASS == 2) *host_out = st;
+                if (PASS == 2) publish_result(host_out, st, host_seq, seq);
             }
             above += h[e];
         }
     }
+}
+
+// Round 0 of the bisection measures at tau = 0 and moves to the mean product (tool.cu:445-468).
+__device__ __forceinline__ TauTune first_round(unsigned long long cnt, double sum, unsigned long long total, double expected, double tol,
+                                               int max_rounds) {
+    TauTune t;
+    t.rate = (double)((float)cnt / (float)total);
+    t.norm = t.up = t.down = 0.0;
+    t.done = fabs(t.rate - expected) < tol;
+    if (!t.done) t.norm = t.up = sum / (double)total;
+    t.rounds = 1;
+    if (t.rounds >= max_rounds) t.done = 1;
+    return t;
 }
 
 // The two numbers that a round of the bisection starts from (tool.cu:448-463), and with `tune` its
@@ -182,13 +208,14 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_count(const float *__restrict__
                                                        int nbK, int nbN, double thr, unsigned long long total, int tune,
                                                        double expected, double tol, int max_rounds,
                                                        TauWorkspace *__restrict__ ws, TauCounts *__restrict__ host_out,
-                                                       TauResult *__restrict__ host_tune) {
+                                                       TauResult *__restrict__ host_tune, unsigned long long *__restrict__ host_seq,
+                                                       unsigned long long seq) {
     __shared__ unsigned long long s_cnt[TAU_NW];
     __shared__ double s_sum[TAU_NW];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     unsigned long long cnt = 0;
     double sum = 0.0;
-    for_products(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
+    for_products<TAU_JB_COUNT>(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
         cnt += __builtin_popcountll(__ballot(live && (double)p >= thr));
         sum += live ? (double)p : 0.0;
     });
@@ -215,15 +242,9 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_count(const float *__restrict__
     TauCounts tc;
     tc.count = cnt;
     tc.sum = sum;
-    *host_out = tc;
+    if (!tune) publish_result(host_out, tc, host_seq, seq);
     if (tune) {
-        TauTune t;
-        t.rate = (double)((float)cnt / (float)total);             // round 0 measures at tau = 0 ...
-        t.norm = t.up = t.down = 0.0;
-        t.done = fabs(t.rate - expected) < tol;
-        if (!t.done) t.norm = t.up = sum / (double)total;         // ... and moves to the mean product (tool.cu:445-468)
-        t.rounds = 1;
-        if (t.rounds >= max_rounds) t.done = 1;
+        const TauTune t = first_round(cnt, sum, total, expected, tol, max_rounds);
         ws->tune = t;
         TauResult r = {t.norm, t.rate, t.done};
         *host_tune = r;
@@ -269,7 +290,7 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_tree(const float *__restrict__ 
         thr[n] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, node_thr), n + 1));
         cnt[n] = 0;
     }
-    for_products(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
+    for_products<TAU_JB_TREE>(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
         const float q = live ? p : -1.0f;
 #pragma unroll
         for (int n = 0; n < TAU_NODES; n++) cnt[n] += __builtin_popcountll(__ballot(q >= thr[n]));
@@ -295,9 +316,12 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_tree(const float *__restrict__ 
         if (lane < 16) s_tot[wave][n] = c;
     }
     __syncthreads();
-    if (threadIdx.x < 16)
-        for (int r = 1; r < TAU_NW; r++) s_tot[0][threadIdx.x] += s_tot[r][threadIdx.x];
-    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    unsigned long long node_cnt = 0;                              // lane n: node n
+#pragma unroll
+    for (int r = 0; r < TAU_NW; r++) node_cnt += s_tot[r][lane & 15];
+    if (lane < 16) s_tot[0][lane] = node_cnt;
+    __builtin_amdgcn_wave_barrier();
     if (threadIdx.x != 0) return;
     TauTune t = ws->tune;
     int n = 1;
@@ -317,57 +341,240 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_tree(const float *__restrict__ 
     *host_tune = r;
 }
 
-__global__ __launch_bounds__(256) void k_tau_clear(TauWorkspace *ws, int hist) {
-    const int b = blockIdx.x * 256 + threadIdx.x;                 // one workgroup, or 8 per histogram copy
-    if (hist) (&ws->hist[0][0][0])[b] = 0;
+// Small problems by one workgroup that holds every product in registers: E per thread, 1024 threads.  All
+// passes of a selection and all rounds of a bisection are then one launch, with a barrier between them.
+// Whole calls, launches of their own -> this: 528 products to a kept fraction 66 -> 42 us, tuned 69 -> 50; 21952
+// products 49 and 59.  At 64 per thread the one CU is the slower: 32768 products tuned 83 against 75 us, 64000 to a
+// kept fraction 72.5 against 71, hence TAU_SMALL_MAX.
+template <int E>
+__device__ __forceinline__ void load_products(const float *__restrict__ nA, const float *__restrict__ nBt, int nbK, int nbN, int total,
+                                              float (&p)[E]) {
+    // product idx = (i * nbN + j) * nbK + k; thread t has t, t + 1024, ...
+    int idx = threadIdx.x, k = idx % nbK, j = idx / nbK % nbN, i = idx / nbK / nbN;
+    const int dk = TAU_NTH % nbK, dj = TAU_NTH / nbK % nbN, di = TAU_NTH / nbK / nbN;
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const bool live = idx < total;
+        const float a = nA[live ? i * nbK + k : 0], b = nBt[live ? j * nbK + k : 0];
+        p[e] = live ? a * b : -1.0f;
+        idx += TAU_NTH;
+        k += dk;
+        if (k >= nbK) { k -= nbK; j++; }
+        j += dj;
+        if (j >= nbN) { j -= nbN; i++; }
+        i += di;
+    }
+}
+
+template <int E>
+__global__ __launch_bounds__(TAU_NTH) void k_tau_small_select(const float *__restrict__ nA, const float *__restrict__ nBt, int nbK, int nbN,
+                                                              int total, unsigned int want0, TauState *__restrict__ host_out,
+                                                              unsigned long long *__restrict__ host_seq, unsigned long long seq) {
+    constexpr int COPIES = 4;
+    __shared__ __attribute__((aligned(16))) unsigned int lh[2048 * COPIES];
+    __shared__ unsigned int s_sum[TAU_NW], s_found[3];            // prefix, rank inside the bin, products above it
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float p[E];
+    load_products<E>(nA, nBt, nbK, nbN, total, p);
+    for (int b = threadIdx.x; b < 2048 * COPIES; b += TAU_NTH) lh[b] = 0;
+    unsigned int positive = 0;
+#pragma unroll
+    for (int e = 0; e < E; e++) positive += (unsigned int)__builtin_popcountll(__ballot(p[e] > 0.0f));    // NaN counts as 0
+    if (lane == 0) s_sum[wave] = positive;
+    __syncthreads();
+    positive = 0;
+#pragma unroll
+    for (int w = 0; w < TAU_NW; w++) positive += s_sum[w];
+    unsigned int want = want0 < positive ? want0 : positive, prefix = 0, greater = 0;     // zero tail: settle for the smallest positive product
+    TauState st = {};
+    if (want == 0) {                                              // nothing but zeros: only tau = 0 keeps anything
+        st.kept = (unsigned long long)total;
+        if (threadIdx.x == 0) publish_result(host_out, st, host_seq, seq);
+        return;
+    }
+    static_for<3>([&](auto pass) {
+        constexpr int PASS = decltype(pass)::value, BITS = PASS == 2 ? 10 : 11, SHIFT = PASS == 0 ? 21 : (PASS == 1 ? 10 : 0);
+        constexpr int NB = 1 << BITS, PER = NB / TAU_NTH;
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const uint32_t key = __builtin_bit_cast(uint32_t, p[e]);
+            bool in = p[e] > 0.0f;
+            if constexpr (PASS > 0) in = in && (key >> (SHIFT + BITS)) == prefix;
+            if (in) atomicAdd(&lh[((key >> SHIFT) & (NB - 1)) * COPIES + (lane & (COPIES - 1))], 1u);
+        }
+        __syncthreads();
+        // thread t takes bins NB - 1 - t * PER downwards; `above` = products in the bins over its own
+        unsigned int h[PER], mine = 0;
+#pragma unroll
+        for (int e = 0; e < PER; e++) {
+            uint4 *bin = reinterpret_cast<uint4 *>(&lh[(NB - 1 - (int)threadIdx.x * PER - e) * COPIES]);
+            const uint4 c = *bin;
+            *bin = make_uint4(0u, 0u, 0u, 0u);
+            h[e] = c.x + c.y + c.z + c.w;
+            mine += h[e];
+        }
+        unsigned int incl = mine;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const unsigned int o = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += o;
+        }
+        if (lane == 63) s_sum[wave] = incl;
+        __syncthreads();
+        unsigned int above = incl - mine;
+#pragma unroll
+        for (int w = 0; w < TAU_NW; w++) above += w < wave ? s_sum[w] : 0u;
+#pragma unroll
+        for (int e = 0; e < PER; e++) {
+            if (above < want && want <= above + h[e]) {           // exactly one thread and bin
+                s_found[0] = (prefix << (PASS ? BITS : 0)) | (uint32_t)(NB - 1 - (int)threadIdx.x * PER - e);
+                s_found[1] = want - above;
+                s_found[2] = greater + above;
+                if constexpr (PASS == 2) {
+                    st.want = want - above;
+                    st.greater = greater + above;
+                    st.prefix = st.tau_bits = s_found[0];
+                    st.kept = st.greater + h[e];
+                    publish_result(host_out, st, host_seq, seq);
+                }
+            }
+            above += h[e];
+        }
+        if constexpr (PASS < 2) {
+            __syncthreads();
+            prefix = s_found[0];
+            want = s_found[1];
+            greater = s_found[2];
+        }
+    });
+}
+
+template <int E>
+__global__ __launch_bounds__(TAU_NTH) void k_tau_small_tune(const float *__restrict__ nA, const float *__restrict__ nBt, int nbK, int nbN,
+                                                            int total, double expected, double tol, int max_rounds,
+                                                            TauResult *__restrict__ host_out, unsigned long long *__restrict__ host_seq,
+                                                            unsigned long long seq) {
+    __shared__ unsigned int s_cnt[2][TAU_NW];
+    __shared__ double s_sum[TAU_NW];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float p[E];
+    load_products<E>(nA, nBt, nbK, nbN, total, p);
+    double sum = 0.0;
+#pragma unroll
+    for (int e = 0; e < E; e++) sum += (int)threadIdx.x + e * TAU_NTH < total ? (double)p[e] : 0.0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off, 64);
+    if (lane == 0) s_sum[wave] = sum;
+    int turn = 0;
+    // products >= thr, of all waves; (double)p >= thr over fp32 p is p >= the smallest fp32 value not below thr
+    auto count = [&](double thr) -> unsigned int {
+        float f = (float)thr;
+        if ((double)f < thr) f = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, f) + 1u);        // thresholds are >= 0
+        unsigned int c = 0;
+#pragma unroll
+        for (int e = 0; e < E; e++) c += (unsigned int)__builtin_popcountll(__ballot(p[e] >= f));
+        if (lane == 0) s_cnt[turn][wave] = c;
+        __syncthreads();
+        c = 0;
+#pragma unroll
+        for (int w = 0; w < TAU_NW; w++) c += s_cnt[turn][w];
+        turn ^= 1;             // (the next count writes the other half: no wave is two counts ahead of another)
+        return c;
+    };
+    // every thread follows the bisection by itself
+    const unsigned int positive = count(0.0);
+    sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < TAU_NW; w++) sum += s_sum[w];
+    TauTune t = first_round(positive, sum, (unsigned long long)total, expected, tol, max_rounds);
+    while (!t.done) {
+        t.rate = (double)((float)count(t.norm) / (float)total);
+        if (fabs(t.rate - expected) < tol) break;
+        bisect_step(t, t.rate > expected);
+        if (++t.rounds >= max_rounds) break;
+    }
+    if (threadIdx.x == 0) {
+        const TauResult res = {t.norm, t.rate, 1};
+        publish_result(host_out, res, host_seq, seq);
+    }
+}
+
+// once after allocation: every launch leaves the ticket and the histograms as it found them
+__global__ __launch_bounds__(256) void k_tau_clear(TauWorkspace *ws) {
+    const int b = blockIdx.x * 256 + threadIdx.x;                 // 8 workgroups per histogram copy
+    (&ws->hist[0][0][0])[b] = 0;
     if (b == 0) {
         ws->ticket = 0;
         ws->zeros = 0;
     }
 }
 
-static unsigned tau_grid(int64_t nbM, int64_t nbK, int64_t nbN) {
-    const int64_t units = nbM * ((nbN + TAU_JB - 1) / TAU_JB) * ((nbK + 63) / 64);
+hipError_t launch_tau_clear(void *workspace, hipStream_t s) {
+    k_tau_clear<<<3 * TAU_COPIES * 2048 / 256, 256, 0, s>>>((TauWorkspace *)workspace);
+    return hipGetLastError();
+}
+
+static int64_t tau_products(int64_t nbM, int64_t nbK, int64_t nbN) { return nbM * nbK * nbN; }
+
+bool tau_tune_small(int64_t nbM, int64_t nbK, int64_t nbN) { return tau_products(nbM, nbK, nbN) <= TAU_SMALL_MAX; }
+
+static unsigned tau_grid(int64_t nbM, int64_t nbK, int64_t nbN, int jb = TAU_JB_COUNT) {
+    const int64_t units = nbM * ((nbN + jb - 1) / jb) * ((nbK + 63) / 64);
     const int64_t blocks = (units + TAU_NW - 1) / TAU_NW;
     return (unsigned)(blocks < TAU_MAXB ? blocks : TAU_MAXB);
 }
 
 hipError_t launch_tau_select(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN,
-                             unsigned long long want, void *workspace, TauState *host_out, hipStream_t s) {
+                             unsigned long long want, void *workspace, TauState *host_out, unsigned long long *host_seq,
+                             unsigned long long seq, hipStream_t s) {
     TauWorkspace *ws = (TauWorkspace *)workspace;
+    const int64_t n = tau_products(nbM, nbK, nbN);
+    if (n <= TAU_SMALL_MAX) {
+#define SPAMM_SELECT(E) k_tau_small_select<E><<<1, TAU_NTH, 0, s>>>(nA, nBt, (int)nbK, (int)nbN, (int)n, (unsigned int)want, host_out, host_seq, seq)
+        if (n <= 8 * TAU_NTH) SPAMM_SELECT(8);
+        else SPAMM_SELECT(24);
+#undef SPAMM_SELECT
+        return hipGetLastError();
+    }
     unsigned grid = tau_grid(nbM, nbK, nbN);
-    const unsigned long long total = (unsigned long long)nbM * nbK * nbN;
+    const unsigned long long total = (unsigned long long)n;
     // a workgroup counts in 32 bits (2e9 products each is N = 262144 at tile 32)
     if (total >> 31 > grid / 2) grid = (unsigned)(total >> 30);
-    k_tau_clear<<<3 * TAU_COPIES * 2048 / 256, 256, 0, s>>>(ws, 1);
-    k_tau_hist<0><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out);
-    k_tau_hist<1><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out);
-    k_tau_hist<2><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out);
+    k_tau_hist<0><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out, host_seq, seq);
+    k_tau_hist<1><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out, host_seq, seq);
+    k_tau_hist<2><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out, host_seq, seq);
     return hipGetLastError();
 }
 
 hipError_t launch_tau_count(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double thr,
-                            void *workspace, TauCounts *host_out, hipStream_t s) {
+                            void *workspace, TauCounts *host_out, unsigned long long *host_seq, unsigned long long seq, hipStream_t s) {
     TauWorkspace *ws = (TauWorkspace *)workspace;
-    k_tau_clear<<<1, 256, 0, s>>>(ws, 0);
     k_tau_count<<<tau_grid(nbM, nbK, nbN), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, thr,
-                                                       (unsigned long long)nbM * nbK * nbN, 0, 0.0, 0.0, 0, ws, host_out, nullptr);
+                                                       (unsigned long long)nbM * nbK * nbN, 0, 0.0, 0.0, 0, ws, host_out, nullptr,
+                                                       host_seq, seq);
+    return hipGetLastError();
+}
+
+hipError_t launch_tau_tune_small(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double expected, double tol,
+                                 int max_rounds, TauResult *host_out, unsigned long long *host_seq, unsigned long long seq, hipStream_t s) {
+    const int64_t n = tau_products(nbM, nbK, nbN);
+#define SPAMM_TUNE(E) k_tau_small_tune<E><<<1, TAU_NTH, 0, s>>>(nA, nBt, (int)nbK, (int)nbN, (int)n, expected, tol, max_rounds, host_out, host_seq, seq)
+    if (n <= 8 * TAU_NTH) SPAMM_TUNE(8);
+    else SPAMM_TUNE(24);
+#undef SPAMM_TUNE
     return hipGetLastError();
 }
 
 hipError_t launch_tau_tune(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double expected,
-                           double tol, int max_rounds, bool first, int passes, void *workspace, TauCounts *host_counts,
-                           TauResult *host_out, hipStream_t s) {
+                           double tol, int max_rounds, bool first, int passes, void *workspace, TauResult *host_out, hipStream_t s) {
     TauWorkspace *ws = (TauWorkspace *)workspace;
-    const unsigned grid = tau_grid(nbM, nbK, nbN);
     const unsigned long long total = (unsigned long long)nbM * nbK * nbN;
-    if (first) {
-        k_tau_clear<<<1, 256, 0, s>>>(ws, 0);
-        k_tau_count<<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, 0.0, total, 1, expected, tol, max_rounds,
-                                             ws, host_counts, host_out);
-    }
+    if (first)
+        k_tau_count<<<tau_grid(nbM, nbK, nbN), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, 0.0, total, 1, expected, tol,
+                                                           max_rounds, ws, nullptr, host_out, nullptr, 0);
     for (int p = 0; p < passes; p++)
-        k_tau_tree<<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, expected, tol, max_rounds, ws, host_out);
+        k_tau_tree<<<tau_grid(nbM, nbK, nbN, TAU_JB_TREE), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, expected, tol,
+                                                                       max_rounds, ws, host_out);
     return hipGetLastError();
 }
 

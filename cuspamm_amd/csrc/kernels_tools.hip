@@ -32,7 +32,8 @@ struct ReportWorkspace {
 // Sums of all workgroups' N values, by the workgroup that finishes last, to host_out (pinned host memory): in a
 // fixed order, so that a repeated call gives the same number.  `own`: the workgroup's values, in thread i the i-th.
 template <int N>
-__device__ __forceinline__ void finish_sums(ReportWorkspace *ws, double own, double *host_out) {
+__device__ __forceinline__ void finish_sums(ReportWorkspace *ws, double own, ReportSums *host_out, unsigned long long *host_seq,
+                                            unsigned long long seq) {
     __shared__ double s_fin[4][N];
     if (threadIdx.x < N)
         agent_store(reinterpret_cast<unsigned long long *>(&ws->part[(size_t)blockIdx.x * N + threadIdx.x]), __builtin_bit_cast(unsigned long long, own));
@@ -51,7 +52,11 @@ __device__ __forceinline__ void finish_sums(ReportWorkspace *ws, double own, dou
         if (lane == 0) s_fin[wave][i] = v[i];
     }
     __syncthreads();
-    if (threadIdx.x < N) host_out[threadIdx.x] = s_fin[0][threadIdx.x] + s_fin[1][threadIdx.x] + s_fin[2][threadIdx.x] + s_fin[3][threadIdx.x];
+    if (threadIdx.x != 0) return;
+    ReportSums out = {};
+#pragma unroll
+    for (int i = 0; i < N; i++) out.v[i] = s_fin[0][i] + s_fin[1][i] + s_fin[2][i] + s_fin[3][i];
+    publish_result(host_out, out, host_seq, seq);
 }
 
 // A wave owns NBR x NBC blocks of v_mfma_f64_16x16x4_f64 (4 accumulator doubles per lane each), four waves (2 x 2) a
@@ -63,7 +68,8 @@ template <int NBR, int NBC>
 __global__ __launch_bounds__(256, NBR * NBC > 8 ? 2 : 3) void k_error_dense(const _Float16 *__restrict__ pA, const _Float16 *__restrict__ pB,
                                                                         int64_t K, int64_t N, int tile, const float *__restrict__ C,
                                                                         int64_t row0, int64_t row1, int nwg_n,
-                                                                        ReportWorkspace *__restrict__ ws, double *__restrict__ host_out) {
+                                                                        ReportWorkspace *__restrict__ ws, ReportSums *__restrict__ host_out,
+                                                                        unsigned long long *__restrict__ host_seq, unsigned long long seq) {
     __shared__ double red[4][3];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wr = wave >> 1, wc = wave & 1;
@@ -153,7 +159,7 @@ __global__ __launch_bounds__(256, NBR * NBC > 8 ? 2 : 3) void k_error_dense(cons
     __syncthreads();
     double own = 0.0;
     if (threadIdx.x < 3) own = red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
-    finish_sums<3>(ws, own, host_out);
+    finish_sums<3>(ws, own, host_out, host_seq, seq);
 }
 
 // Dropped norm products of every output tile: a wave takes one tile row and BOUND_JB tile columns, lane = k, so that a
@@ -165,7 +171,8 @@ constexpr unsigned BOUND_MAX_WG = 2048;
 
 __global__ __launch_bounds__(256) void k_dropped_bound(const float *__restrict__ nA, const float *__restrict__ nBt,
                                                        int nbM, int nbK, int nbN, float tau, ReportWorkspace *__restrict__ ws,
-                                                       double *__restrict__ host_out, double *__restrict__ per_tile) {
+                                                       ReportSums *__restrict__ host_out, unsigned long long *__restrict__ host_seq,
+                                                       unsigned long long seq, double *__restrict__ per_tile) {
     __shared__ double red[4];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int jb = (nbN + BOUND_JB - 1) / BOUND_JB;
@@ -202,7 +209,7 @@ __global__ __launch_bounds__(256) void k_dropped_bound(const float *__restrict__
     if (!host_out) return;
     if (lane == 0) red[wave] = sum;
     __syncthreads();
-    finish_sums<1>(ws, threadIdx.x == 0 ? red[0] + red[1] + red[2] + red[3] : 0.0, host_out);
+    finish_sums<1>(ws, threadIdx.x == 0 ? red[0] + red[1] + red[2] + red[3] : 0.0, host_out, host_seq, seq);
 }
 
 __global__ void k_clear_report(ReportWorkspace *ws) { ws->ticket = 0; }
@@ -244,23 +251,25 @@ size_t report_workspace_bytes(int64_t rows, int64_t N, int n_cu) {
 }
 
 hipError_t launch_error_vs_dense(const void *packedA, const void *packedB, int64_t K, int64_t N, int tile, const float *C,
-                                 int64_t row0, int64_t row1, int n_cu, void *workspace, double *host_out3, hipStream_t s) {
+                                 int64_t row0, int64_t row1, int n_cu, void *workspace, ReportSums *host_out,
+                                 unsigned long long *host_seq, unsigned long long seq, hipStream_t s) {
     int64_t n_wg = 0;
     const int shape = error_shape(row1 - row0, N, n_cu, &n_wg);
     const _Float16 *pA = (const _Float16 *)packedA, *pB = (const _Float16 *)packedB;
     ReportWorkspace *ws = (ReportWorkspace *)workspace;
     const int nwg_n = (int)((N + 32 * ERROR_SHAPES[shape].nbc - 1) / (32 * ERROR_SHAPES[shape].nbc));
-    if (shape == 0) k_error_dense<4, 4><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out3);
-    else if (shape == 1) k_error_dense<4, 2><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out3);
-    else k_error_dense<2, 2><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out3);
+    if (shape == 0) k_error_dense<4, 4><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out, host_seq, seq);
+    else if (shape == 1) k_error_dense<4, 2><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out, host_seq, seq);
+    else k_error_dense<2, 2><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out, host_seq, seq);
     return hipGetLastError();
 }
 
 hipError_t launch_dropped_bound(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, float tau,
-                                void *workspace, double *host_out, double *per_tile, hipStream_t s) {
+                                void *workspace, ReportSums *host_out, unsigned long long *host_seq, unsigned long long seq,
+                                double *per_tile, hipStream_t s) {
     const int64_t wg = (nbM * ((nbN + BOUND_JB - 1) / BOUND_JB) + 3) / 4;
     k_dropped_bound<<<wg < (int64_t)BOUND_MAX_WG ? (unsigned)wg : BOUND_MAX_WG, 256, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, tau,
-                                                                                (ReportWorkspace *)workspace, host_out, per_tile);
+                                                                                (ReportWorkspace *)workspace, host_out, host_seq, seq, per_tile);
     return hipGetLastError();
 }
 

@@ -32,4 +32,20 @@ __device__ __forceinline__ bool last_workgroup(unsigned int *ticket) {
     return s_last != 0;
 }
 
+// A result for the host, which waits for `seq` to appear (pinned, coherent memory): by one thread, the
+// result's words first.
+template <typename T>
+__device__ __forceinline__ void publish_result(T *host_out, const T &v, unsigned long long *host_seq, unsigned long long seq) {
+    static_assert(sizeof(T) % 8 == 0, "results are whole 64-bit words");
+    struct Words {
+        unsigned long long w[sizeof(T) / 8];
+    };
+    const Words words = __builtin_bit_cast(Words, v);
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 8; i++)
+        __hip_atomic_store(reinterpret_cast<unsigned long long *>(host_out) + i, words.w[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __hip_atomic_store(host_seq, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 }  // namespace spamm

@@ -46,7 +46,8 @@ struct HostResults {
     TauState select;
     TauCounts counts;
     TauResult tune;
-    double report[3];
+    ReportSums report;
+    unsigned long long seq;       // of the last result
 };
 
 // Everything a multiply leaves behind: the shape it ran at, what is valid, and
@@ -95,7 +96,9 @@ struct spamm_ctx : Workspace {
     DevBuf reportws;  // error report workspace
     double *tile_results = nullptr;   // pinned, TILE_RESULTS_MAX doubles at most: per-tile results of small outputs
     size_t tile_results_cap = 0;
-    HostResults *results = nullptr;   // pinned: small results that a kernel writes and the host reads after a wait
+    HostResults *results = nullptr;   // pinned: small results that a kernel writes and the host waits for
+    unsigned long long seq = 0;       // of the last result asked for
+    bool tauws_clean = false;         // the tau workspace's counters are zero, as every completed call leaves them
 
     hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
     bool timing = false;        // events of the last multiply are valid
@@ -683,7 +686,19 @@ static int ensure_results(spamm_ctx *c) {
     void *p = nullptr;
     HIPCHK(c, hipHostMalloc(&p, sizeof(HostResults), hipHostMallocDefault));
     c->results = (HostResults *)p;
+    c->results->seq = 0;
     return SPAMM_OK;
+}
+
+// Waits for result `seq`, which the last kernel of the call writes when it has done all else: a few microseconds
+// sooner than the stream is reported idle.  If the stream ends, or fails, without it, the call has failed.  (A
+// bisection in several launches waits for the stream: what has ended it may have launches behind it that still
+// look at the workspace.)
+static int wait_result(spamm_ctx *c, unsigned long long seq) {
+    for (int i = 0; i < 50000; i++)           // (some 100 us)
+        if (__atomic_load_n(&c->results->seq, __ATOMIC_ACQUIRE) == seq) return SPAMM_OK;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return __atomic_load_n(&c->results->seq, __ATOMIC_ACQUIRE) == seq ? SPAMM_OK : SPAMM_EHIP;
 }
 
 static int report_prepare(spamm_ctx *c, int64_t rows) {
@@ -705,11 +720,11 @@ int spamm_error_vs_dense_f64(spamm_ctx *c, const float *dC, int64_t row0, int64_
     int rc = set_device(c);
     if (rc) return rc;
     if ((rc = report_prepare(c, row1 - row0))) return rc;
-    double *sq = c->results->report;
+    const unsigned long long seq = ++c->seq;
     HIPCHK(c, launch_error_vs_dense(c->packedA.p, c->packedB.p, c->K, c->N, c->tile, dC, row0, row1, c->n_cu, c->reportws.p,
-                                    sq, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int i = 0; i < 3; i++) out3[i] = sqrt(sq[i]);
+                                    &c->results->report, &c->results->seq, seq, c->stream));
+    if ((rc = wait_result(c, seq))) return rc;
+    for (int i = 0; i < 3; i++) out3[i] = sqrt(c->results->report.v[i]);
     return SPAMM_OK;
 }
 
@@ -721,10 +736,11 @@ int spamm_dropped_bound(spamm_ctx *c, float tau, double *out) {
     if (rc) return rc;
     const Shape s = shape_of(c);
     if ((rc = report_prepare(c, 0))) return rc;
+    const unsigned long long seq = ++c->seq;
     HIPCHK(c, launch_dropped_bound((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, tau, c->reportws.p,
-                                   c->results->report, nullptr, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    *out = sqrt(c->results->report[0]);
+                                   &c->results->report, &c->results->seq, seq, nullptr, c->stream));
+    if ((rc = wait_result(c, seq))) return rc;
+    *out = sqrt(c->results->report.v[0]);
     return SPAMM_OK;
 }
 
@@ -747,7 +763,7 @@ int spamm_dropped_bound_tiles(spamm_ctx *c, float tau, double *host_out) {
         c->tile_results_cap = nt;
     }
     if (!pinned && (rc = ensure(c, c->staging, nt * 8))) return rc;
-    HIPCHK(c, launch_dropped_bound((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, tau, nullptr, nullptr,
+    HIPCHK(c, launch_dropped_bound((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, tau, nullptr, nullptr, nullptr, 0,
                                    pinned ? c->tile_results : (double *)c->staging.p, c->stream));
     if (!pinned) return copy_out(c, c->staging.p, host_out, nt * 8);
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -833,7 +849,10 @@ static int tau_prepare(spamm_ctx *c, Shape *s) {
     if (rc) return rc;
     *s = shape_of(c);
     if ((rc = ensure_results(c))) return rc;
-    return ensure(c, c->tauws, tau_workspace_bytes());
+    if (c->tauws.p && c->tauws_clean) return SPAMM_OK;
+    if ((rc = ensure(c, c->tauws, tau_workspace_bytes()))) return rc;
+    HIPCHK(c, launch_tau_clear(c->tauws.p, c->stream));
+    return SPAMM_OK;
 }
 
 int spamm_count_kept(spamm_ctx *c, double threshold, int64_t *count_out, double *sum_out) {
@@ -841,9 +860,12 @@ int spamm_count_kept(spamm_ctx *c, double threshold, int64_t *count_out, double 
     Shape s;
     int rc = tau_prepare(c, &s);
     if (rc) return rc;
+    const unsigned long long seq = ++c->seq;
+    c->tauws_clean = false;
     HIPCHK(c, launch_tau_count((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, threshold,
-                               c->tauws.p, &c->results->counts, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+                               c->tauws.p, &c->results->counts, &c->results->seq, seq, c->stream));
+    if ((rc = wait_result(c, seq))) return rc;
+    c->tauws_clean = true;
     if (count_out) *count_out = (int64_t)c->results->counts.count;
     if (sum_out) *sum_out = c->results->counts.sum;
     return SPAMM_OK;
@@ -858,9 +880,12 @@ int spamm_tau_for_ratio(spamm_ctx *c, double ratio, float *tau_out, double *achi
     double w = ceil(ratio * (double)total);
     unsigned long long want = w < 1.0 ? 1ull : (unsigned long long)w;
     if (want > total) want = total;
+    const unsigned long long seq = ++c->seq;
+    c->tauws_clean = false;
     HIPCHK(c, launch_tau_select((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, want,
-                                c->tauws.p, &c->results->select, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+                                c->tauws.p, &c->results->select, &c->results->seq, seq, c->stream));
+    if ((rc = wait_result(c, seq))) return rc;
+    c->tauws_clean = true;
     const TauState st = c->results->select;
     memcpy(tau_out, &st.tau_bits, 4);
     if (achieved_out) *achieved_out = (double)st.kept / (double)total;
@@ -873,18 +898,30 @@ int spamm_tune_bisect(spamm_ctx *c, double expected, double tol, int max_rounds,
     Shape s;
     int rc = tau_prepare(c, &s);
     if (rc) return rc;
-    // the rounds run on the device (tool.cu:445-486); the reference's 20 are one wait, beyond that the
-    // host looks every 20 whether they have ended
+    // the rounds run on the device (tool.cu:445-486)
+    if (tau_tune_small(s.nbM, s.nbK, s.nbN)) {
+        const unsigned long long seq = ++c->seq;
+        HIPCHK(c, launch_tau_tune_small((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, expected, tol, max_rounds,
+                                        &c->results->tune, &c->results->seq, seq, c->stream));
+        if ((rc = wait_result(c, seq))) return rc;
+        *tau_out = (float)c->results->tune.norm;
+        if (achieved_out) *achieved_out = c->results->tune.rate;
+        return SPAMM_OK;
+    }
+    // four rounds a launch; the reference's 20 rounds are one wait, beyond that the host looks every 20
+    // whether they have ended
+    c->tauws_clean = false;
     int left = (max_rounds - 1 + 3) / 4;
     bool first = true;
     do {
         const int passes = left < 5 ? left : 5;
         HIPCHK(c, launch_tau_tune((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, expected, tol,
-                                  max_rounds, first, passes, c->tauws.p, &c->results->counts, &c->results->tune, c->stream));
+                                  max_rounds, first, passes, c->tauws.p, &c->results->tune, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         left -= passes;
         first = false;
     } while (left > 0 && !c->results->tune.done);
+    c->tauws_clean = true;
     *tau_out = (float)c->results->tune.norm;
     if (achieved_out) *achieved_out = c->results->tune.rate;
     return SPAMM_OK;

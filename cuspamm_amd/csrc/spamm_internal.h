@@ -91,15 +91,20 @@ hipError_t launch_normmap_ab(const void *X, bool in16, int64_t n, int tile, void
 bool normmap_pair_fits(bool in16, bool tau_aware, int64_t M, int64_t K, int64_t N, int tile);
 hipError_t launch_normmap_pair(const void *A, const void *Bm, bool in16, int64_t M, int64_t K, int64_t N, int tile, void *packedA,
                                float *nmA, void *packedB, float *nmB, float *nmBt, float tau_skip, int64_t *kept, hipStream_t s);
-// error report tooling (kernels_tools.hip).  Results go to host_out, pinned host memory: valid once the stream has been
-// waited for.  The workspace's ticket is zero between launches (launch_clear_report once after allocation).
+// error report tooling (kernels_tools.hip).  Results go to host_out, pinned host memory: valid once *host_seq == seq
+// (per_tile: once the stream has been waited for).  The workspace's ticket is zero between launches (launch_clear_report once after allocation).
+struct ReportSums {
+    double v[3];
+};
 size_t report_workspace_bytes(int64_t rows, int64_t N, int n_cu);      // rows = 0: the bound only
 hipError_t launch_clear_report(void *workspace, hipStream_t s);
 hipError_t launch_error_vs_dense(const void *packedA, const void *packedB, int64_t K, int64_t N, int tile, const float *C,
-                                 int64_t row0, int64_t row1, int n_cu, void *workspace, double *host_out3, hipStream_t s);
-// *host_out (optional) = sum over tiles of s_ij^2, s_ij = sum_{k dropped} nA[i,k]*nB[k,j]; per_tile (optional): s_ij
+                                 int64_t row0, int64_t row1, int n_cu, void *workspace, ReportSums *host_out,
+                                 unsigned long long *host_seq, unsigned long long seq, hipStream_t s);
+// host_out->v[0] (optional) = sum over tiles of s_ij^2, s_ij = sum_{k dropped} nA[i,k]*nB[k,j]; per_tile (optional): s_ij
 hipError_t launch_dropped_bound(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, float tau,
-                                void *workspace, double *host_out, double *per_tile, hipStream_t s);
+                                void *workspace, ReportSums *host_out, unsigned long long *host_seq, unsigned long long seq,
+                                double *per_tile, hipStream_t s);
 hipError_t launch_unpack(const void *packed, int64_t rows, int64_t cols, int tile, int role,
                          uint16_t *out, hipStream_t s);
 hipError_t launch_transpose_normmap(const float *nB, int64_t nbK, int64_t nbN, float *nBt,
@@ -149,18 +154,24 @@ struct TauCounts {
 };
 struct TauResult {                // of the bisection so far
     double norm, rate;
-    int done;
+    int64_t done;
 };
 size_t tau_workspace_bytes();
-// Results go to *host_out, pinned host memory: valid once the stream has been waited for.
+// Results go to *host_out, pinned host memory: valid once *host_seq == seq (the kernel that writes it is the
+// call's last), or, of launch_tau_tune, once the stream has been waited for.
+hipError_t launch_tau_clear(void *workspace, hipStream_t s);          // once after allocation, and after a failed call
 hipError_t launch_tau_select(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN,
-                             unsigned long long want, void *workspace, TauState *host_out, hipStream_t s);
-hipError_t launch_tau_count(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN,
-                            double thr, void *workspace, TauCounts *host_out, hipStream_t s);
+                             unsigned long long want, void *workspace, TauState *host_out, unsigned long long *host_seq,
+                             unsigned long long seq, hipStream_t s);
+hipError_t launch_tau_count(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double thr,
+                            void *workspace, TauCounts *host_out, unsigned long long *host_seq, unsigned long long seq, hipStream_t s);
+// the whole bisection in one launch, for few products
+bool tau_tune_small(int64_t nbM, int64_t nbK, int64_t nbN);
+hipError_t launch_tau_tune_small(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double expected, double tol,
+                                 int max_rounds, TauResult *host_out, unsigned long long *host_seq, unsigned long long seq, hipStream_t s);
 // the bisection: `first` starts it (its round 0), then 4 rounds per pass until done
 hipError_t launch_tau_tune(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double expected,
-                           double tol, int max_rounds, bool first, int passes, void *workspace, TauCounts *host_counts,
-                           TauResult *host_out, hipStream_t s);
+                           double tol, int max_rounds, bool first, int passes, void *workspace, TauResult *host_out, hipStream_t s);
 
 hipError_t gemm_init();   // one-time kernel attribute set-up
 hipError_t launch_gemm(const void *packedA, const void *packedB, const GateBuffers &g, int64_t M,

@@ -125,3 +125,30 @@ def test_bisection_stops_at_any_round(orc, ctx, rounds):
     ctx.set_normmaps(nA, nB, 32)
     got, want = ctx.tune_bisect(0.4, 0.01, rounds), orc.tune_bisect(nA, nB, 0.4, 0.01, rounds)
     assert np.float32(got[0]) == np.float32(want[0]) and got[1] == want[1]
+
+
+@pytest.mark.parametrize("shape", [(1, 8192, 1), (1, 8193, 1), (3, 1024, 8), (7, 3511, 1), (1, 24577, 1)])
+def test_selection_at_the_edges_of_what_one_workgroup_holds(orc, ctx, shape):
+    # 8 and 24 products per thread of 1024, and one more than each: exact, as above
+    rng = np.random.default_rng(sum(shape))
+    nA, nB = _maps(rng, *shape, zero_frac=0.3)
+    nA[0, 0] = np.nan                                          # (a NaN product is never kept, and counts as zero)
+    total = shape[0] * shape[1] * shape[2]
+    clean = np.where(np.isnan(nA), 0, nA).astype(np.float32)
+    for a, b, oa in ((nA, nB, clean), (np.round(clean * 4), np.round(nB * 4), np.round(clean * 4))):
+        ctx.set_normmaps(a, b, 32)
+        for ratio in (1.0 / total, 0.37, 0.6, 1.0):
+            got, want = ctx.tau_for_ratio(ratio), orc.tau_for_ratio(oa, b, ratio)
+            assert np.float32(got[0]) == np.float32(want[0]) and got[1] == want[1], (ratio, got, want)
+
+
+@pytest.mark.parametrize("repeat", [1, 1365, 1366, 4096, 4097])
+@pytest.mark.parametrize("rounds", [1, 5, 6, 20, 22])
+def test_bisection_stops_at_any_round_with_many_products(orc, ctx, repeat, rounds):
+    # the six products above, `repeat` times: 8190, 8196, 24576 products of one workgroup, 24582 of many.
+    # Sums of these values are exact in any order
+    nA = np.tile(np.array([[1.0, 2.0, 4.0], [0.5, 8.0, 16.0]], np.float32), (1, repeat))
+    nB = np.ones((3 * repeat, 1), np.float32)
+    ctx.set_normmaps(nA, nB, 32)
+    got, want = ctx.tune_bisect(0.4, 0.01, rounds), orc.tune_bisect(nA, nB, 0.4, 0.01, rounds)
+    assert np.float32(got[0]) == np.float32(want[0]) and got[1] == want[1]
