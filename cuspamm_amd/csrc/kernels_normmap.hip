@@ -40,12 +40,11 @@ __device__ __forceinline__ float butterfly64(float v) {
     return v;
 }
 
-// One workgroup per strip of B rows x SW columns (SW/B tiles; SW = 256 for fp32 input,
-// 512 for fp16 input: a strip row is 1 KiB either way and is read by one wave-wide load; tiles of 128
-// mostly SW = 128, one tile per strip, two or four rows per load).  The
+// One workgroup per strip of B rows x SW columns (SW/B tiles).  A wave-wide load is one strip row of
+// 1 KiB (fp32, SW = 256) or a row each of two or four 8-row groups.  The
 // tiles of a strip pass through LDS in PH phases of SW/B/PH tiles each, sized so that at most
 // ~42 KiB are resident and three workgroups fit a CU; all loads are issued before the first phase.
-//   load    a lane takes whole 8-row groups (wave w: groups w, w + 4, ...); all loads of a lane
+//   load    a lane takes whole 8-row groups; all loads of a lane
 //           are in flight together.
 //   convert fp32 input, A role: a lane holds half a chunk (4 of 8 elements along k); the odd lane
 //           continues the even lane's running sum (DPP) so that the chunk is summed left to
@@ -78,9 +77,8 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
     constexpr int TPS = SW / B;           // tiles per strip
     constexpr int TPP = TPS / PH;         // tiles per phase (resident in LDS together)
     static_assert(TPP * PH == TPS && TPP >= 1, "phases must divide the strip's tiles");
-    // Lane -> element mapping: every wave-wide load is one whole strip row (1 KiB): 64 lanes x EPL
-    // columns (4 floats, or 8 halves for fp16 input: the strip is then 512 columns wide); wave w
-    // takes the 8-row groups w, w + 4, ...  A lane's columns lie in one tile; with PH > 1 the tiles
+    // Lane -> element mapping: LPR lanes of EPL columns (4 floats or 8 halves, 16 bytes) are a strip row; a
+    // wave-wide load is a row of each of GPW 8-row groups.  A lane's columns lie in one tile; with PH > 1 the tiles
     // pass through LDS PH phases one after the other and in phase ph only the lanes of that
     // phase's tiles stage their data.  Tiles of 128 as strips of several in as many phases put up to
     // 128 KiB in registers per workgroup, staged, copied and reduced in turns with little else on the CU
@@ -443,43 +441,56 @@ __global__ __launch_bounds__(256) void k_fill_decay(float *__restrict__ X, int64
 }
 
 // ---------------------------------------------------------------- launchers
+constexpr unsigned NARROW_STRIPS = 512;     // of 256 columns, in a launch: two per CU
+
 template <int ROLE, bool IN16>
 static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int tile, void *packed, float *nm,
                                  float *nmT, int64_t *kept, hipStream_t s, void *packed2 = nullptr, float *nm2 = nullptr,
                                  const float *rowmax = nullptr, float tau_skip = 0.0f) {
     const int64_t nbr = rows / tile, nbc = cols / tile;
-    constexpr int SW = IN16 ? 512 : 256;              // strip width: a wave-wide load is 1 KiB of one row
-    const int64_t nstrip = (cols + SW - 1) / SW;
-    const unsigned grid = (unsigned)(nbr * nstrip);
-    // phases: tiles of a strip resident in LDS together take ~42 KiB at most (three workgroups per CU)
+    const auto strips = [&](int64_t sw) { return (unsigned)(nbr * ((cols + sw - 1) / sw)); };
+#define SPAMM_NORMMAP(T, SW, PH, NWV)                                                                                           \
+    k_normmap<T, ROLE, SW, IN16, PH, NWV><<<strips(SW), 64 * NWV, 0, s>>>(X, cols, cols, nbr, nbc, (cols + SW - 1) / SW, (uint4 *)packed, \
+                                                                          nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept)
+    // strip widths and waves: one 8-row group per lane, at most ~42 KiB of LDS and so three workgroups or more per CU.
+    // fp16 input: 256 columns, two rows per load (512 in phases before: tile 64 1024^2, both passes, 6.2 -> 4.1 us, 4096^2
+    // 28.4 -> 26.3, 16384^2 A = B 303 -> 291; tile 32 2048^2 8.0 -> 7.3, 8192^2 tau-aware 93 -> 87).
     switch (tile) {
-        case 32: k_normmap<32, ROLE, SW, IN16, 1><<<grid, 256, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept); break;
+        case 32:
+            if constexpr (IN16) SPAMM_NORMMAP(32, 256, 1, 2);
+            else SPAMM_NORMMAP(32, 256, 1, 4);
+            break;
         case 64:
-            // tile 64: eight waves per workgroup on fp16 input (tau-aware passes at N = 16384: 0.156 / 0.138 ->
-            // 0.152 / 0.129 ms) and, on fp32 input, for small grids (N = 8192: 0.066 / 0.058 -> 0.063 / 0.056 ms;
-            // at N = 16384 four waves are as fast or 1 % faster)
-            if (IN16 || grid <= 8192u) {
-                k_normmap<64, ROLE, SW, IN16, IN16 ? 2 : 1, 8><<<grid, 512, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept);
-                break;
-            }
-            k_normmap<64, ROLE, SW, IN16, IN16 ? 2 : 1><<<grid, 256, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept); break;
+            // fp32 input: strips of 128 columns where there are few (1024^2, both passes: 5.4 -> 4.4 us; 4096^2 36.1 ->
+            // 36.7), of 256 by eight waves on middling grids (N = 8192: 0.066 / 0.058 -> 0.063 / 0.056 ms), by four waves,
+            // two groups per lane, on large ones (N = 16384: as fast or 1 % faster)
+            // fp16 input, 3 to 4 strips of 256 columns per CU, of which three run at once: strips of 512 in two phases by eight
+            // waves are one turn instead of two (4096^2, A = B: 19.8 against 21.4 us)
+            if constexpr (IN16) {
+                if (strips(256) > 768u && strips(256) <= 1024u) SPAMM_NORMMAP(64, 512, 2, 8);
+                else SPAMM_NORMMAP(64, 256, 1, 4);
+            } else if (strips(256) <= NARROW_STRIPS) SPAMM_NORMMAP(64, 128, 1, 4);
+            else if (strips(256) <= 8192u) SPAMM_NORMMAP(64, 256, 1, 8);
+            else SPAMM_NORMMAP(64, 256, 1, 4);
+            break;
         // tile 128: strips of one tile.  Only the fp32 B role of a large matrix keeps strips of two tiles in two phases by
         // four waves: N = 32768 830 against 867 us, 16384 225 / 231, 12800 159 / 158, 8192 72 / 67.
         case 128:
             if constexpr (IN16) {
                 if constexpr (ROLE == 2) return hipErrorInvalidValue;      // (two passes, or the pair, are faster)
-                else k_normmap<128, ROLE, 128, true, 1, 4><<<(unsigned)(nbr * nbc), 256, 0, s>>>(X, cols, cols, nbr, nbc, nbc, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept);
+                else SPAMM_NORMMAP(128, 128, 1, 4);
             } else {
                 if constexpr (ROLE == 1)
-                    if (grid > 6000u) {
-                        k_normmap<128, ROLE, SW, false, 2, 4><<<grid, 256, 0, s>>>(X, cols, cols, nbr, nbc, nstrip, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept);
+                    if (strips(256) > 6000u) {
+                        SPAMM_NORMMAP(128, 256, 2, 4);
                         break;
                     }
-                k_normmap<128, ROLE, 128, false, 1, 8><<<(unsigned)(nbr * nbc), 512, 0, s>>>(X, cols, cols, nbr, nbc, nbc, (uint4 *)packed, nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept);
+                SPAMM_NORMMAP(128, 128, 1, 8);
             }
             break;
         default: return hipErrorInvalidValue;
     }
+#undef SPAMM_NORMMAP
     return hipGetLastError();
 }
 
@@ -511,15 +522,22 @@ bool normmap_pair_fits(bool in16, bool tau_aware, int64_t M, int64_t K, int64_t 
 hipError_t launch_normmap_pair(const void *A, const void *Bm, bool in16, int64_t M, int64_t K, int64_t N, int tile, void *packedA,
                                float *nmA, void *packedB, float *nmB, float *nmBt, float tau_skip, int64_t *kept, hipStream_t s) {
     const int64_t nbM = M / tile, nbK = K / tile, nbN = N / tile;
-#define SPAMM_PAIR(T, PH16, NWV, SW32)                                                                                          \
-    if (in16) launch_pair<T, 512, PH16, NWV, true>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, kept, s);        \
-    else launch_pair<T, SW32, 1, NWV, false>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, kept, s)
+#define SPAMM_PAIR(T, SW, NWV, IN16) \
+    launch_pair<T, SW, 1, NWV, IN16>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, kept, s)
+    // (strips as the passes of their own have them)
     switch (tile) {
-        case 32: SPAMM_PAIR(32, 1, 4, 256); break;
-        case 64: SPAMM_PAIR(64, 2, 8, 256); break;
+        case 32:
+            if (in16) SPAMM_PAIR(32, 256, 2, true);
+            else SPAMM_PAIR(32, 256, 4, false);
+            break;
+        case 64:
+            if (in16) SPAMM_PAIR(64, 256, 4, true);
+            else if (nbM * ((K + 255) / 256) + nbK * ((N + 255) / 256) <= NARROW_STRIPS) SPAMM_PAIR(64, 128, 4, false);
+            else SPAMM_PAIR(64, 256, 8, false);
+            break;
         case 128:
-            if (in16) launch_pair<128, 128, 1, 4, true>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, kept, s);
-            else launch_pair<128, 128, 1, 8, false>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, kept, s);
+            if (in16) SPAMM_PAIR(128, 128, 4, true);
+            else SPAMM_PAIR(128, 128, 8, false);
             break;
         default: return hipErrorInvalidValue;
     }
