@@ -251,8 +251,11 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_count(const float *__restrict__
     }
 }
 
-// One step of the bisection away from a measured rate (tool.cu:469-486).
-__device__ __forceinline__ void bisect_step(TauTune &t, bool above) {
+// One step of the bisection away from a measured rate (tool.cu:469-486).  False where it leaves everything as it
+// was, bit for bit: every later round then measures the same threshold and ends here again.  (Doubles run out of
+// thresholds within some 5e4 rounds of any target, so no kernel runs longer whatever the caller's limit.)
+__device__ __forceinline__ bool bisect_step(TauTune &t, bool above) {
+    const TauTune was = t;
     if (above) {
         if (t.up == t.norm) t.up *= 2;
         t.down = t.norm;
@@ -261,6 +264,8 @@ __device__ __forceinline__ void bisect_step(TauTune &t, bool above) {
         t.up = t.norm;
         t.norm = (t.norm + t.down) / 2;
     }
+    const auto same = [](double a, double b) { return __builtin_bit_cast(unsigned long long, a) == __builtin_bit_cast(unsigned long long, b); };
+    return !(same(t.norm, was.norm) && same(t.up, was.up) && same(t.down, was.down));
 }
 
 // Four rounds of the bisection.  Node n of the tree (heap order, node 1 = the round to come) is the
@@ -332,9 +337,9 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_tree(const float *__restrict__ 
             break;
         }
         const bool above = t.rate > expected;
-        bisect_step(t, above);
+        const bool moved = bisect_step(t, above);
         n = 2 * n + (above ? 1 : 0);
-        if (++t.rounds >= max_rounds) t.done = 1;
+        if (++t.rounds >= max_rounds || !moved) t.done = 1;
     }
     ws->tune = t;
     TauResult r = {t.norm, t.rate, t.done};
@@ -490,8 +495,8 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_small_tune(const float *__restr
     while (!t.done) {
         t.rate = (double)((float)count(t.norm) / (float)total);
         if (fabs(t.rate - expected) < tol) break;
-        bisect_step(t, t.rate > expected);
-        if (++t.rounds >= max_rounds) break;
+        const bool moved = bisect_step(t, t.rate > expected);
+        if (++t.rounds >= max_rounds || !moved) break;
     }
     if (threadIdx.x == 0) {
         const TauResult res = {t.norm, t.rate, 1};

@@ -911,7 +911,7 @@ int spamm_tune_bisect(spamm_ctx *c, double expected, double tol, int max_rounds,
     // four rounds a launch; the reference's 20 rounds are one wait, beyond that the host looks every 20
     // whether they have ended
     c->tauws_clean = false;
-    int left = (max_rounds - 1 + 3) / 4;
+    int left = (max_rounds - 1) / 4 + ((max_rounds - 1) % 4 != 0);
     bool first = true;
     do {
         const int passes = left < 5 ? left : 5;

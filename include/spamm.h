@@ -42,8 +42,8 @@ extern "C" {
 
 /* spamm_params.flags */
 #define SPAMM_FLAG_A_EQ_B 1u     /* dA == dB, M == K == N (else SPAMM_EINVAL): the matrix is read once for both
-                                  * operand roles (the single pass is reported as ms_normmap_b); at tile 128 on fp16
-                                  * input, and with SPAMM_FLAG_PRUNE, the ordinary passes run */
+                                  * operand roles (the single pass is reported as ms_normmap_b); at tile 128 the ordinary
+                                  * passes run instead on fp16 input and with SPAMM_FLAG_PRUNE */
 #define SPAMM_FLAG_TIMING 2u     /* record per-stage HIP events (spamm_get_stats) */
 #define SPAMM_FLAG_REUSE_A 4u    /* A's fp16 copy and norm map from an earlier call are reused (dA ignored) */
 #define SPAMM_FLAG_REUSE_B 8u    /* same for B: e.g. one B against many A, or matrix powers */

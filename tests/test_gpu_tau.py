@@ -152,3 +152,15 @@ def test_bisection_stops_at_any_round_with_many_products(orc, ctx, repeat, round
     ctx.set_normmaps(nA, nB, 32)
     got, want = ctx.tune_bisect(0.4, 0.01, rounds), orc.tune_bisect(nA, nB, 0.4, 0.01, rounds)
     assert np.float32(got[0]) == np.float32(want[0]) and got[1] == want[1]
+
+
+@pytest.mark.parametrize("repeat", [1, 4097])
+@pytest.mark.parametrize("expected", [0.4, 2.0])
+def test_bisection_without_a_limit_ends_where_its_thresholds_do(orc, ctx, repeat, expected):
+    # a target that is never met and no limit worth the name: doubles have no threshold left between two kept
+    # fractions after some 60 rounds, or below the smallest product after 1100, and further rounds change nothing
+    nA = np.tile(np.array([[1.0, 2.0, 4.0], [0.5, 8.0, 16.0]], np.float32), (1, repeat))
+    nB = np.ones((3 * repeat, 1), np.float32)
+    ctx.set_normmaps(nA, nB, 32)
+    got, want = ctx.tune_bisect(expected, 0.01, 2 ** 31 - 1), orc.tune_bisect(nA, nB, expected, 0.01, 1200)
+    assert np.float32(got[0]) == np.float32(want[0]) and got[1] == want[1]
