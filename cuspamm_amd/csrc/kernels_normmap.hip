@@ -265,16 +265,17 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
         }
     };
     // norms: one wave per tile, canonical order.  With `prune` (tau known and positive) the wave
-    // also decides whether any product can keep the tile: fl(n * n') <= fl(n * bound) for every
-    // partner norm n' <= bound because rounding is monotone, so a tile whose product with the
-    // bound is below tau is never read by the GEMM and its fp16 copy need not be written.  The
-    // bound is max_j nB[k,j] for the A pass (B's norm map is complete by then) and the largest
-    // finite float for the B pass, which runs first: there only tiles of norm zero are left out.
+    // also decides whether any product can keep the tile.  The A pass of its own has the row maxima
+    // (B's norm map is complete by then): fl(n * n') <= fl(n * max_j nB[k,j]) for every partner norm
+    // n' because rounding is monotone, so a tile whose product with the maximum is below tau is never
+    // read by the GEMM and its fp16 copy need not be written.  The other passes know no partner, and
+    // their copies serve any tau > 0 afterwards: they leave out tiles of norm zero (0 * n' is 0 or NaN).
     auto norms = [&](int ph, bool as_b, float *__restrict__ nmo, float *__restrict__ nmTo, bool prune) {
         for (int tt = wave; tt < TPP; tt += NWV) {
             const int64_t Jt = sc * TPS + ph * TPP + tt;
             if (Jt >= nbc) break;
-            const float rmax = prune ? (rowmax != nullptr ? rowmax[Jt] : 3.402823466e+38f) : 0.0f;
+            const bool bounded = prune && rowmax != nullptr;
+            const float rmax = bounded ? rowmax[Jt] : 0.0f;
             float partial = 0.0f;
 #pragma unroll
             for (int it = 0; it < STEPS; it++) {
@@ -286,7 +287,7 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
                 const float nv = sqrtf(partial);
                 nmo[I * nbc + Jt] = nv;
                 if (as_b) nmTo[Jt * nbr + I] = nv;
-                if (prune) s_skip[tt] = nv * rmax < tau_skip;
+                if (prune) s_skip[tt] = bounded ? nv * rmax < tau_skip : nv == 0.0f;
             }
         }
     };

@@ -207,3 +207,46 @@ def test_tau_aware_passes_give_the_same_product(orc, ctx, tile):
     assert torch.equal(ctx.multiply(A, B, tile, 0.0, prune=True), ctx.multiply(A, B, tile, 0.0))
     assert np.array_equal(ctx.get_fp16(1), orc.f32_to_f16_bits(B.cpu().numpy()))
     assert float(ctx.multiply(A, B, tile, float("inf"), prune=True).abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("tile", [32, 64, 128])
+@pytest.mark.parametrize("route", ["pair", "b_alone", "a_eq_b"])
+def test_passes_without_row_maxima_leave_out_tiles_of_norm_zero_only(orc, ctx, route, tile, half):
+    """A tau-aware copy of B (and A's where both are made without row maxima) may lack the tiles of norm zero and no
+    others, however large the call's own tau: it serves every tau > 0 afterwards.  The copies are loud before, so
+    that a tile that was left out shows in the product that reuses it."""
+    import torch
+    n = 768
+    tab = orc.decay_table("exp", n, 0.05)                     # exactly zero in fp16 beyond |i - j| ~ 333
+    A, B = _dev(orc.fill_decay(n, n, tab, 1)), _dev(orc.fill_decay(n, n, tab, 2))
+    if half:
+        A, B = A.half(), B.half()
+    if route == "a_eq_b":
+        B = A
+    loud = torch.full_like(A, 1000.0)
+
+    def pruned(A, B, tau):
+        ctx.multiply(loud, loud, tile, 0.0)
+        if route == "b_alone":                                # A resident and whole: B's pass runs by itself
+            (ctx.normmap_f16 if half else ctx.normmap_f32)(0, A, tile)
+        return ctx.multiply(A, B, tile, tau, prune=True, a_eq_b=route == "a_eq_b", reuse_a=route == "b_alone")
+
+    want = ctx.multiply(A, B, tile, 1e-3).clone()
+    assert 0 < np.count_nonzero(ctx.get_normmap(1) == 0) < (n // tile) ** 2
+    for tau in (float("inf"), 1e35):
+        assert float(pruned(A, B, tau).abs().max()) == 0.0
+        one_pass = route == "a_eq_b" and tile != 128          # (its copy of A is B's equal; the pair's serves no smaller tau)
+        got = ctx.multiply(A, B, tile, 1e-3, reuse_a=route == "b_alone" or one_pass, reuse_b=True)
+        assert torch.equal(got, want), tau
+    # an infinite norm keeps every partner of positive norm, also at tau = inf and in the call itself
+    A = A.clone()
+    A[5, 70] = float("inf")
+    if route == "a_eq_b":
+        B = A
+    want = ctx.multiply(A, B, tile, float("inf")).clone()
+    kept = ctx.get_stats().kept_products
+    assert 0 < kept < (n // tile) ** 3
+    got = pruned(A, B, float("inf"))
+    assert ctx.get_stats().kept_products == kept
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
