@@ -268,10 +268,20 @@ __device__ __forceinline__ bool bisect_step(TauTune &t, bool above) {
     return !(same(t.norm, was.norm) && same(t.up, was.up) && same(t.down, was.down));
 }
 
+// (double)p >= thr over fp32 p is p >= the smallest fp32 value that is not below thr.  (Mean and thresholds are
+// negative where uploaded norm maps hold negative values.)
+__device__ __forceinline__ float fp32_threshold(double thr) {
+    const float f = (float)thr;
+    if (!((double)f < thr)) return f;
+    return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, f) + (f < 0.0f ? -1 : 1));
+}
+
+// What a lane without a product holds: no threshold keeps it.
+constexpr float NO_PRODUCT = __builtin_nanf("");
+
 // Four rounds of the bisection.  Node n of the tree (heap order, node 1 = the round to come) is the
 // threshold after the answers that n's bits below the leading one spell, most significant first:
-// 1 = the kept rate was above the target.  (double)p >= thr over fp32 p is p >= the smallest fp32
-// value that is not below thr.
+// 1 = the kept rate was above the target.
 __global__ __launch_bounds__(TAU_NTH) void k_tau_tree(const float *__restrict__ nA, const float *__restrict__ nBt, int nbM,
                                                       int nbK, int nbN, unsigned long long total, double expected, double tol,
                                                       int max_rounds, TauWorkspace *__restrict__ ws,
@@ -285,8 +295,7 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_tree(const float *__restrict__ 
         TauTune t = ws->tune;
         const int n = (lane & 15) == 0 ? 1 : (lane & 15);
         for (int bit = 30 - __builtin_clz(n); bit >= 0; bit--) bisect_step(t, (n >> bit) & 1);
-        node_thr = (float)t.norm;
-        if ((double)node_thr < t.norm) node_thr = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, node_thr) + 1u);   // thresholds are >= 0
+        node_thr = fp32_threshold(t.norm);
     }
     float thr[TAU_NODES];
     unsigned long long cnt[TAU_NODES];
@@ -296,7 +305,7 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_tree(const float *__restrict__ 
         cnt[n] = 0;
     }
     for_products<TAU_JB_TREE>(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
-        const float q = live ? p : -1.0f;
+        const float q = live ? p : NO_PRODUCT;
 #pragma unroll
         for (int n = 0; n < TAU_NODES; n++) cnt[n] += __builtin_popcountll(__ballot(q >= thr[n]));
     });
@@ -361,7 +370,7 @@ __device__ __forceinline__ void load_products(const float *__restrict__ nA, cons
     for (int e = 0; e < E; e++) {
         const bool live = idx < total;
         const float a = nA[live ? i * nbK + k : 0], b = nBt[live ? j * nbK + k : 0];
-        p[e] = live ? a * b : -1.0f;
+        p[e] = live ? a * b : NO_PRODUCT;
         idx += TAU_NTH;
         k += dk;
         if (k >= nbK) { k -= nbK; j++; }
@@ -471,10 +480,9 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_small_tune(const float *__restr
     for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off, 64);
     if (lane == 0) s_sum[wave] = sum;
     int turn = 0;
-    // products >= thr, of all waves; (double)p >= thr over fp32 p is p >= the smallest fp32 value not below thr
+    // products >= thr, of all waves
     auto count = [&](double thr) -> unsigned int {
-        float f = (float)thr;
-        if ((double)f < thr) f = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, f) + 1u);        // thresholds are >= 0
+        const float f = fp32_threshold(thr);
         unsigned int c = 0;
 #pragma unroll
         for (int e = 0; e < E; e++) c += (unsigned int)__builtin_popcountll(__ballot(p[e] >= f));

@@ -164,3 +164,16 @@ def test_bisection_without_a_limit_ends_where_its_thresholds_do(orc, ctx, repeat
     ctx.set_normmaps(nA, nB, 32)
     got, want = ctx.tune_bisect(expected, 0.01, 2 ** 31 - 1), orc.tune_bisect(nA, nB, expected, 0.01, 1200)
     assert np.float32(got[0]) == np.float32(want[0]) and got[1] == want[1]
+
+
+@pytest.mark.parametrize("repeat", [1, 1366, 4097])
+@pytest.mark.parametrize("rounds", [2, 5, 20])
+def test_bisection_over_uploaded_maps_with_negative_values(orc, ctx, repeat, rounds):
+    # hand-built maps may hold any value: the mean product and with it the thresholds are negative here, and the
+    # lanes without a product must count for none of them.  Sums of these values are exact in any order
+    nA = np.tile(np.array([[-1.0, -2.0, 4.0], [-0.5, -8.0, -16.0]], np.float32), (1, repeat))
+    nB = np.ones((3 * repeat, 1), np.float32)
+    ctx.set_normmaps(nA, nB, 32)
+    for expected in (0.4, 0.9):
+        got, want = ctx.tune_bisect(expected, 0.01, rounds), orc.tune_bisect(nA, nB, expected, 0.01, rounds)
+        assert np.float32(got[0]) == np.float32(want[0]) and got[1] == want[1], (expected, got, want)
