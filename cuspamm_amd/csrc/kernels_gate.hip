@@ -525,7 +525,8 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
             // lanes 0..7 (and again 8..15, so that a rotation by row of 16 is one by 8): the group's i-th
             // super tile and XCD i's length so far.  Ranks are counts over seven rotations of keys that
             // carry the index; XCD x takes the super tile whose rank (heaviest first) is its own (shortest
-            // first).
+            // first).  (One XCD may be dealt all super tiles: its key needs the 32nd bit.)
+            static_assert((uint64_t)BAND_DEAL_MAX * SUPER_M * SUPER_N * 65535 * 8 + MAX_XCD < 0xfffffff0u, "an XCD's key stays below the absent ones'");
             const int x = lane & 7;
             int load = 0, cnt = 0;
             const int ngroups = (n_ne + n_xcd - 1) / n_xcd;
@@ -533,12 +534,13 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
             int w = weight(0);
             for (int g2 = 0; g2 < ngroups; g2++) {
                 const int wn = weight(g2 + 1);
-                const int wkey = (w + 1) * 8 + 7 - x, lkey = x < n_xcd ? load * 8 + x : 0x7ffffff0 + x;
+                const int wkey = (w + 1) * 8 + 7 - x;
+                const uint32_t lkey = x < n_xcd ? (uint32_t)load * 8u + (uint32_t)x : 0xfffffff0u + (uint32_t)x;
                 int wrank = 0, xrank = 0;
                 static_for<7>([&](auto i) {
                     constexpr int ROR = 0x121 + decltype(i)::value;
                     wrank += dpp<ROR>(wkey) > wkey;
-                    xrank += dpp<ROR>(lkey) < lkey;
+                    xrank += (uint32_t)dpp<ROR>((int)lkey) < lkey;
                 });
                 const int pk = (w + 1) << 6 | x << 3 | wrank;
                 int sel = wrank == xrank ? pk : 0;

@@ -270,3 +270,29 @@ def test_small_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N, ti
         assert torch.equal(ctx.gemm_gated(got), want)
     finally:
         apart.close()
+
+
+def test_schedule_of_the_longest_lists_on_one_xcd(ctx):
+    """One XCD takes every super tile of a band, and the lengths dealt to it so far are part of the key it is chosen by:
+    lists of 65535 k tiles bring that sum to 2^28 - 1 before the last super tile is dealt (times 8, plus the XCD's number:
+    more than 31 bits).  Every macro tile must be in the sequence."""
+    import cuspamm_amd as sp
+    nbM, nbK, nbN, tile = 14 * 8, 65535, 16 * 16, 128            # 14 x 16 super tiles of 8 x 16 output tiles
+    nA = np.zeros((nbM, nbK), np.float32)
+    nB = np.ones((nbK, nbN), np.float32)
+    nA[:64] = 1.0                                                # 128 super tiles whose 32 lists hold every k: 268431360 in all,
+    nA[64:66] = 0.5
+    nB[:4095, 0] = 2.0                                           # one with a single list of 4095,
+    nB[:5, 16] = 2.0                                             # and one with a single list of 5
+    other = sp.SpammContext(0)
+    try:
+        other.set_option(sp.OPT_NUM_XCD, 1)
+        other.set_normmaps(nA, nB, tile)
+        other.gate(1.0)
+        counts, sched = other.get_macro_counts()
+        work = counts[..., 0]
+        assert work[:32].min() == 65535 and work[32:].sum() == 4095 + 5
+        assert sched[0] == np.count_nonzero(work) == 32 * 128 + 2
+        assert sched[8] == work.size
+    finally:
+        other.close()
