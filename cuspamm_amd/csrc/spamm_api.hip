@@ -543,6 +543,7 @@ static int multiply_any(spamm_ctx *c, const spamm_params *p, const void *dA, con
     if (reuse_b && !(c->have_b && c->tile == p->tile && c->K == p->K && c->N == p->N)) return SPAMM_ESTATE;
     bool a_eq_b = (p->flags & SPAMM_FLAG_A_EQ_B) != 0;
     if (a_eq_b && (reuse_a || reuse_b || dA != dB || p->M != p->K || p->K != p->N)) return SPAMM_EINVAL;
+    if ((rc = set_device(c))) return rc;        // (with both operands resident no stage below does it)
     const bool prune = (p->flags & SPAMM_FLAG_PRUNE) != 0 && p->tau > 0.0f;
     // tile 128 on fp16 input, and tau-aware: the flag only asserts dA == dB, and the ordinary passes (with
     // their full tau-aware pruning) run
@@ -553,7 +554,6 @@ static int multiply_any(spamm_ctx *c, const spamm_params *p, const void *dA, con
         // convert and norm the same data twice), else both operands' strips side by side
         if (c->tile != p->tile) reset_shape(c, p->tile);
         if (p->M / p->tile > 65535 || p->K / p->tile > 65535 || p->N / p->tile > 65535) return SPAMM_EINVAL;
-        if ((rc = set_device(c))) return rc;
         const size_t ta = (size_t)(p->M / p->tile) * (size_t)(p->K / p->tile), tb = (size_t)(p->K / p->tile) * (size_t)(p->N / p->tile);
         // nothing of the old contents is valid until the pass has been launched
         c->have_a = c->have_b = c->have_gate = false;
