@@ -152,6 +152,9 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_hist(const float *__restrict__ 
         if (lane >= off) incl += o;
     }
     if (lane == 63) s_sum[wave] = incl;
+    // The host goes on when it sees the last pass's result, on another stream if it likes: by then nothing of this
+    // launch is still on its way to the workspace (and the state in it, which no launch after this reads, stays as it is)
+    if constexpr (PASS == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     unsigned long long above = incl - mine;
     for (int w = 0; w < wave; w++) above += s_sum[w];
@@ -180,8 +183,8 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_hist(const float *__restrict__ 
                 st.prefix = (prefix << (PASS ? BITS : 0)) | (uint32_t)(NB - 1 - (int)threadIdx.x * PER - e);
                 st.tau_bits = st.prefix;
                 st.kept = st.greater + h[e];
-                ws->st = st;
                 if (PASS == 2) publish_result(host_out, st, host_seq, seq);
+                else ws->st = st;
             }
             above += h[e];
         }

@@ -690,7 +690,8 @@ static int ensure_results(spamm_ctx *c) {
     return SPAMM_OK;
 }
 
-// Waits for result `seq`, which the last kernel of the call writes when it has done all else: a few microseconds
+// Waits for result `seq`, which the last kernel of the call writes when it has done all else -- its writes to the
+// context's workspaces have arrived, so that the next call may use them from another stream -- a few microseconds
 // sooner than the stream is reported idle.  If the stream ends, or fails, without it, the call has failed.  (A
 // bisection in several launches waits for the stream: what has ended it may have launches behind it that still
 // look at the workspace.)

@@ -177,3 +177,30 @@ def test_bisection_over_uploaded_maps_with_negative_values(orc, ctx, repeat, rou
     for expected in (0.4, 0.9):
         got, want = ctx.tune_bisect(expected, 0.01, rounds), orc.tune_bisect(nA, nB, expected, 0.01, rounds)
         assert np.float32(got[0]) == np.float32(want[0]) and got[1] == want[1], (expected, got, want)
+
+
+def test_results_on_one_stream_after_another(orc):
+    # a result is handed out before its stream is idle: the next call, on another stream, finds the workspace at rest
+    import torch
+    import cuspamm_amd as sp
+    rng = np.random.default_rng(5)
+    nA, nB = _maps(rng, 48, 70, 40, zero_frac=0.2)
+    ratios = (0.02, 0.3, 0.7)
+    want = [orc.tau_for_ratio(nA, nB, r) for r in ratios]
+    prods = nA[:, None, :].astype(np.float64) * nB.T[None].astype(np.float64)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    c = sp.SpammContext(0)
+    try:
+        c.set_normmaps(nA, nB, 32)
+        for rep in range(24):
+            c.set_stream(streams[rep % 2].cuda_stream)
+            r = rep % 3
+            got = c.tau_for_ratio(ratios[r])
+            assert np.float32(got[0]) == np.float32(want[r][0]) and got[1] == want[r][1], rep
+            if rep % 4 == 3:
+                c.set_stream(streams[(rep + 1) % 2].cuda_stream)
+                assert c.count_kept(0.0)[0] == nA.shape[0] * nA.shape[1] * nB.shape[1]
+                # sums of 134400 fp64 terms in another order: below 134400 * 2^-53 = 1.5e-11 of the sum of squares
+                assert c.dropped_bound(float("inf")) == pytest.approx(np.sqrt((prods.sum(axis=2) ** 2).sum()), rel=1.5e-11)
+    finally:
+        c.close()

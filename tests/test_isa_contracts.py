@@ -269,3 +269,29 @@ def test_small_output_kernel_keeps_the_same_contracts(tmp_path):
                  if mn.startswith(("global_", "flat_", "buffer_", "scratch_")) and mn != "global_load_lds_dwordx4"]
         assert not other, "%s: %s between the first and the last global->LDS load" % (name, sorted(set(other)))
         assert not any(mn.startswith("scratch_") for mn in mns), name
+
+
+def test_results_are_published_when_the_workspace_is_at_rest(tmp_path):
+    """The host goes on when it sees a result's sequence number and may use the workspace at once, from another stream:
+    behind a publishing kernel's last barrier no wave stores anything but the result itself (to host memory, in system
+    scope: sc0 sc1), and in the kernel whose waves all clear counters, every wave has waited for its stores before it."""
+    publishing = [("kernels_tau.hip", r"_ZN5spamm10k_tau_histILi2E\w+", 1), ("kernels_tools.hip", r"_ZN5spamm13k_error_denseILi\w+", 3),
+                  ("kernels_tools.hip", r"_ZN5spamm15k_dropped_bound\w+", 1)]
+    for src, name, count in publishing:
+        kernels = re.findall(r"^(%s):[^\n]*\n(.*?)^\.Lfunc_end" % name, _isa(src, tmp_path), flags=re.S | re.M)
+        assert len(kernels) == count, src
+        for kernel, body in kernels:
+            lines = [ln.strip() for ln in body.splitlines()]
+            last = max(i for i, ln in enumerate(lines) if ln.startswith("s_barrier"))
+            stores = [ln for ln in lines[last:] if re.match(r"(global|flat|buffer|scratch)_(store|atomic)", ln)]
+            assert stores and all(ln.endswith("sc0 sc1") for ln in stores), (kernel, stores)
+            if "k_tau_hist" in kernel:
+                block = []
+                for ln in reversed(lines[:last]):
+                    if ln.startswith("s_barrier"):
+                        break
+                    block.append(ln)
+                waits = [i for i, ln in enumerate(block) if re.match(r"s_waitcnt.*vmcnt\(0\)", ln)]
+                clears = [i for i, ln in enumerate(block) if ln.startswith("global_store")]
+                assert clears and waits and waits[0] < clears[0], kernel        # (reversed: the last wait comes after the last store)
+                assert not any(ln.startswith((".LBB", "s_cbranch", "s_branch")) for ln in block[:waits[0]]), kernel
