@@ -43,3 +43,13 @@ def ctx():
     c = sp.SpammContext(0)
     yield c
     c.close()
+
+
+@pytest.fixture(params=[0, 1], ids=["default_unit", "macro_tiles"])
+def work_unit(ctx, request):
+    """The session context as it is (small outputs: gate and multiply in one kernel) and with the GEMM's work unit
+    fixed to whole macro tiles, so that gate, schedule and GEMM run on small outputs too."""
+    import cuspamm_amd as sp
+    ctx.set_option(sp.OPT_GEMM_SHAPE, request.param)
+    yield request.param
+    ctx.set_option(sp.OPT_GEMM_SHAPE, 0)

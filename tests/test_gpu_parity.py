@@ -73,6 +73,7 @@ CASES = [
 ]
 
 
+@pytest.mark.usefixtures("work_unit")
 @pytest.mark.parametrize("M,K,N,tile,kind,lam,tau", CASES)
 def test_multiply_matches_checker(orc, ctx, M, K, N, tile, kind, lam, tau):
     tab = orc.decay_table(kind, max(M, K, N), lam)

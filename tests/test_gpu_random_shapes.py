@@ -6,6 +6,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.usefixtures("work_unit")
 @pytest.mark.parametrize("seed", [11, 12, 13])
 def test_random_cases_against_the_checker(orc, ctx, seed):
     import torch

@@ -26,6 +26,7 @@ def _check(orc, ctx, A, B, tile, tau):
     return ref
 
 
+@pytest.mark.usefixtures("work_unit")
 def test_random_shapes(orc, ctx):
     rng = np.random.default_rng(2024)
     for trial in range(40):
@@ -49,7 +50,7 @@ def test_random_shapes(orc, ctx):
                                         (32, 288000, 32, 32),      # 9000 k tiles: bitmaps beyond 64 KiB of LDS
                                         (64, 65535 * 64, 64, 64),  # the most k tiles the ABI takes
                                         (32, 65535 * 32, 32, 32)])  # ... at tile 32: the gate walks k in four chunks
-def test_extreme_aspect_ratios(orc, ctx, M, K, N, tile):
+def test_extreme_aspect_ratios(orc, ctx, work_unit, M, K, N, tile):
     tab = orc.decay_table("exp", max(M, K, N), 0.002)
     A = orc.fill_decay(M, K, tab, 1)
     B = orc.fill_decay(K, N, tab, 2)
@@ -160,6 +161,7 @@ def test_other_gemm_work_units_give_the_same_product(orc, ctx, shape):
         other.close()
 
 
+@pytest.mark.usefixtures("work_unit")
 def test_scattered_sparsity_pattern(orc, ctx):
     # no band structure at all: random tiles zeroed, so k lists are ragged and macro tiles mixed
     rng = np.random.default_rng(7)
@@ -176,6 +178,7 @@ def test_scattered_sparsity_pattern(orc, ctx):
     assert 0 < ref["kept"] < (n // tile) ** 3 // 2
 
 
+@pytest.mark.usefixtures("work_unit")
 def test_non_finite_inputs_follow_ieee_compare(orc, ctx):
     # inf tile norm: kept against any non-zero tile; NaN product (inf*0, NaN norm) is dropped
     n, tile = 256, 64
@@ -200,7 +203,7 @@ def test_non_finite_inputs_follow_ieee_compare(orc, ctx):
 
 
 @pytest.mark.parametrize("n_xcd", [1, 2, 4])
-def test_schedule_for_other_xcd_counts_gives_the_same_product(orc, ctx, n_xcd):
+def test_schedule_for_other_xcd_counts_gives_the_same_product(orc, ctx, work_unit, n_xcd):
     """The GEMM schedule is built for the device's XCD count (8 on a whole MI355X); a partitioned
     device, or one that is not whole XCDs of 32 CUs, gets 4 / 2 / 1 sequences.  The schedule only
     decides where and when a macro tile runs: mask and C must not change by a bit."""
@@ -208,6 +211,7 @@ def test_schedule_for_other_xcd_counts_gives_the_same_product(orc, ctx, n_xcd):
     import cuspamm_amd as sp
     other = sp.SpammContext(0)
     other.set_option(sp.OPT_NUM_XCD, n_xcd)
+    other.set_option(sp.OPT_GEMM_SHAPE, work_unit)
     try:
         # (the last case is a narrow band over 128 super tiles: the grouped row-major deal)
         for (M, K, N), tile, lam, ratio in [((2304, 1024, 4352), 64, 0.004, 0.3), ((1280, 512, 768), 32, 0.01, 0.5),
@@ -295,4 +299,36 @@ def test_schedule_of_the_longest_lists_on_one_xcd(ctx):
         assert sched[0] == np.count_nonzero(work) == 32 * 128 + 2
         assert sched[8] == work.size
     finally:
+        other.close()
+
+
+@pytest.mark.parametrize("ring", [3, 5])
+def test_other_staging_rings_give_the_same_product(orc, ctx, ring):
+    """The GEMM's ring of LDS stages is four deep by default; three and five walk the same lists.  Lists shorter than
+    the ring, empty ones, an odd number of entries kept by all tiles (tile 32: one stage each), ragged edges of C."""
+    import torch
+    import cuspamm_amd as sp
+    other = sp.SpammContext(0)
+    other.set_option(sp.OPT_GEMM_RING, ring)
+    other.set_option(sp.OPT_GEMM_SHAPE, 1)
+    ctx.set_option(sp.OPT_GEMM_SHAPE, 1)
+    try:
+        for (M, K, N), tile, lam, ratio in [((256, 32, 256), 32, 0.0, 1.0), ((256, 96, 512), 32, 0.0, 1.0), ((512, 224, 256), 32, 0.0, 1.0),
+                                            ((1280, 512, 768), 32, 0.01, 0.5), ((96, 64, 160), 32, 0.0, 1.0),
+                                            ((2304, 1024, 4352), 64, 0.004, 0.3), ((320, 64, 448), 64, 0.0, 1.0),
+                                            ((640, 4096, 896), 128, 0.001, 0.1), ((128, 128, 128), 128, 0.0, 1.0)]:
+            tab = orc.decay_table("exp", max(M, K, N), lam)
+            dA, dB = _dev(orc.fill_decay(M, K, tab, 1)), _dev(orc.fill_decay(K, N, tab, 2))
+            ctx.normmap_f32(1, dB, tile)
+            ctx.normmap_f32(0, dA, tile)
+            tau = 0.0 if ratio == 1.0 else ctx.tau_for_ratio(ratio)[0]
+            want = ctx.multiply(dA, dB, tile, tau)
+            got = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+            other.multiply(dA, dB, tile, tau, C=got)
+            assert torch.equal(got, want), (M, K, N, tile)
+            assert np.array_equal(other.get_mask(), ctx.get_mask())
+        tab = orc.decay_table("exp", 2048, 0.003)
+        _check(orc, other, orc.fill_decay(384, 2048, tab, 3), orc.fill_decay(2048, 320, tab, 4), 32, 0.05)
+    finally:
+        ctx.set_option(sp.OPT_GEMM_SHAPE, 0)
         other.close()

@@ -157,7 +157,8 @@ def test_a_equals_b_single_pass(orc, ctx, tile):
 
 @pytest.mark.parametrize("tile", [32, 64, 128])
 def test_tau_aware_passes_give_the_same_product(orc, ctx, tile):
-    """SPAMM_FLAG_PRUNE: A tiles that no product can keep and B tiles of norm zero are not copied;
+    """SPAMM_FLAG_PRUNE: tiles that no product can keep are not copied -- at this size, where one launch converts
+    both operands, those of norm zero in either (the A pass of its own, which knows B's norms, has a test below);
     C, mask, counts and norm maps must not change.  The workspace is first filled with loud
     operands so that a GEMM reading a skipped tile would show."""
     import torch
@@ -173,11 +174,11 @@ def test_tau_aware_passes_give_the_same_product(orc, ctx, tile):
     Cref = ctx.multiply(A, B, tile, tau).clone()
     mask, counts, nA, nB = ctx.get_mask(), ctx.get_counts(), ctx.get_normmap(0), ctx.get_normmap(1)
     kept = ctx.get_stats().kept_products
-    # the checker's kept set says which A tiles are needed at all: some must be skippable here,
-    # and some B tiles must be exactly zero
+    # the checker's kept set says which A tiles are needed at all: some are not (which matters to a
+    # pass that knows it), and some tiles of either operand must be exactly zero
     needed = np.unpackbits(mask.view(np.uint8), axis=-1, bitorder="little")[..., :K // tile].any(axis=1)
     assert 0 < needed.sum() < needed.size
-    assert 0 < np.count_nonzero(nB == 0) < nB.size
+    assert 0 < np.count_nonzero(nB == 0) < nB.size and 0 < np.count_nonzero(nA == 0) < nA.size
     loud = ctx.multiply(torch.full_like(A, 1000.0), torch.full_like(B, 1000.0), tile, 0.0)   # both workspace copies are now loud
     assert float(loud.min()) > 0
     C = ctx.multiply(A, B, tile, tau, prune=True)
@@ -250,3 +251,95 @@ def test_passes_without_row_maxima_leave_out_tiles_of_norm_zero_only(orc, ctx, r
     got = pruned(A, B, float("inf"))
     assert ctx.get_stats().kept_products == kept
     assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("tile", [32, 64, 128])
+def test_tau_aware_a_pass_by_row_maxima_gives_the_same_product(orc, ctx, tile, half):
+    """A's pass of its own knows B's norms and leaves out every tile that no product keeps (k_rowmax and the bounded
+    test): against a resident B, and in a call of more strips than the paired passes take (4096), where B's pass of
+    its own runs before it.  Both copies are loud before."""
+    import torch
+    M, K, N = 1024, 768, 512 + tile
+    tab = orc.decay_table("exp", 1024, 0.05)
+    A, B = _dev(orc.fill_decay(M, K, tab, 1)), _dev(orc.fill_decay(K, N, tab, 2))
+    # the long one: rows of the first, at scales of their own, over 2045 tile rows
+    scale = torch.exp2(torch.randint(-6, 1, (2045, 1), generator=torch.Generator().manual_seed(3)).float()).cuda()
+    long = (A[:tile].repeat(2045, 1).view(2045, -1) * scale).view(2045 * tile, K)
+    for X, resident in ((A, True), (long, False)):
+        Y = B
+        if half:
+            X, Y = X.half(), B.half()
+        normmap = ctx.normmap_f16 if half else ctx.normmap_f32
+        normmap(1, Y, tile)
+        normmap(0, X, tile)
+        nA, nB = ctx.get_normmap(0), ctx.get_normmap(1)
+        tau = ctx.tau_for_ratio(0.05)[0]
+        skipped = np.count_nonzero(nA * nB.max(axis=1)[None, :] < np.float32(tau))
+        assert np.count_nonzero(nA == 0) < skipped < nA.size
+        want = ctx.multiply(X, Y, tile, tau).clone()
+        mask, counts, kept = ctx.get_mask(), ctx.get_counts(), ctx.get_stats().kept_products
+        ctx.multiply(torch.full_like(X, 1000.0), torch.full_like(Y, 1000.0), tile, 0.0)
+        if resident:
+            normmap(1, Y, tile)
+        got = ctx.multiply(X, Y, tile, tau, prune=True, reuse_b=resident)
+        assert torch.equal(got, want)
+        assert np.array_equal(ctx.get_mask(), mask) and np.array_equal(ctx.get_counts(), counts)
+        assert ctx.get_stats().kept_products == kept > 0
+        assert np.array_equal(ctx.get_normmap(0).view(np.uint32), nA.view(np.uint32))
+        want = ctx.multiply(X, Y, tile, tau * 2).clone()
+        ctx.multiply(torch.full_like(X, 1000.0), torch.full_like(Y, 1000.0), tile, 0.0)
+        ctx.multiply(X, Y, tile, tau, prune=True)
+        assert torch.equal(ctx.multiply(X, Y, tile, tau * 2, reuse_a=True, reuse_b=True), want)
+
+
+def test_fp16_passes_of_three_to_four_strips_per_cu(orc, ctx):
+    # fp16 at tile 64, 769 to 1024 strips of 256 columns: strips of 512 in two phases, here ragged (7 1/8 of them), for
+    # either role and for both at once, against the paired passes (strips of 256) of the same operands
+    import torch
+    n, tile = 57 * 64, 64
+    tab = orc.decay_table("exp", n, 0.01)
+    X = torch.empty((n, n), dtype=torch.float32, device="cuda")
+    ctx.fill_decay(X, tab, 1)
+    X = X.half()
+    bits = X.cpu().numpy().view(np.uint16)
+    ctx.multiply(X, X, tile, 1.0)                             # the paired passes
+    nA, nB = ctx.get_normmap(0), ctx.get_normmap(1)
+    tau = ctx.tau_for_ratio(0.1)[0]
+    want = ctx.multiply(X, X, tile, tau).clone()
+    ctx.multiply(torch.full_like(X, 1000.0), torch.full_like(X, 1000.0), tile, 0.0)
+    for both in (False, True):
+        if both:
+            got = ctx.multiply(X, X, tile, tau, a_eq_b=True)
+        else:
+            ctx.normmap_f16(1, X, tile)
+            ctx.normmap_f16(0, X, tile)
+            ctx.gate(tau)
+            got = ctx.gemm_gated(torch.empty_like(want))
+        assert np.array_equal(ctx.get_fp16(0), bits) and np.array_equal(ctx.get_fp16(1), bits)
+        assert np.array_equal(ctx.get_normmap(0).view(np.uint32), nA.view(np.uint32))
+        assert np.array_equal(ctx.get_normmap(1).view(np.uint32), nB.view(np.uint32))
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("rows,N,row0", [(2048, 1024, 64), (512, 512, 0), (4096, 2048, 0), (2112, 960, 0)])
+def test_error_report_by_any_block_shape(ctx, rows, N, row0):
+    """A wave of the exact product owns 64 x 32 of C (the first case, on 256 CUs), 32 x 32, 64 x 64, or what the grid
+    makes best: against a product in fp64 on the host.  Norms of sums of squares in another order: K + rows * N terms
+    of 2^-53 each, below 1e-9; the difference's norm is as large as C's (half of the products are dropped)."""
+    import torch
+    K, tile = 320, 64
+    M = row0 + rows
+    g = torch.Generator(device="cuda")
+    g.manual_seed(rows + N)
+    A = torch.rand((M, K), generator=g, device="cuda") * torch.exp2(-torch.arange(K, device="cuda") / 40.0) - 0.3
+    B = torch.rand((K, N), generator=g, device="cuda") - 0.5
+    ctx.normmap_f32(1, B, tile)
+    ctx.normmap_f32(0, A, tile)
+    C = ctx.multiply(A, B, tile, ctx.tau_for_ratio(0.5)[0])
+    dense = A.half().double().cpu().numpy()[row0:] @ B.half().double().cpu().numpy()
+    c = C.cpu().numpy().astype(np.float64)[row0:]
+    want = [np.linalg.norm(c - dense), np.linalg.norm(dense), np.linalg.norm(c)]
+    assert want[0] > 0.01 * want[1]
+    for got, ref in zip(ctx.error_vs_dense(C, row0, M), want):
+        assert abs(got - ref) <= 1e-9 * ref

@@ -116,6 +116,7 @@ def test_noalloc_a_equals_b(orc, ctx):
     _check_against(ctx, orc, got, orc.spamm(A, A, 32, 1e-2), "noalloc A = B")
 
 
+@pytest.mark.usefixtures("work_unit")
 def test_noalloc_at_the_workspace_limit(orc, ctx):
     # 3072^3 needs 36 MiB of fp16 copies plus lists: the largest cube that fits the 40 MiB array
     import torch
@@ -167,7 +168,7 @@ def test_noalloc_limits_and_flags(ctx):
 # The callers this entry point is for: a HIP graph captures the multiply once and replays it on
 # changing inputs (mask and schedule are rebuilt on the device at every replay); eager multiplies
 # run between the replays and every replay is compared with one.
-def test_noalloc_multiply_replays_in_a_hip_graph(orc, ctx):
+def test_noalloc_multiply_replays_in_a_hip_graph(orc, ctx, work_unit):
     import torch
     import cuspamm_amd as sp
     M, K, N, tile, tau = 1024, 768, 1280, 64, 0.3
@@ -179,6 +180,7 @@ def test_noalloc_multiply_replays_in_a_hip_graph(orc, ctx):
     side = torch.cuda.Stream()
     with torch.cuda.stream(side):
         gctx = sp.SpammContext(0)                     # bound to the side stream
+        gctx.set_option(sp.OPT_GEMM_SHAPE, work_unit)
         gctx.multiply_noalloc(dA, dB, tile, tau, C)   # warm-up: kernels loaded before the capture
         side.synchronize()
         graph = torch.cuda.CUDAGraph()
