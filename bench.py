@@ -53,6 +53,14 @@ WORKLOADS = {
 FP16_INPUT_WORKLOADS = ("ref_default",)
 
 
+def paired_passes(N, tile, in_bytes, tau_aware):
+    """Whether the library converts both operands of an N^3 multiply in one launch (normmap_pair_fits in
+    kernels_normmap.hip): by tile rows of 1 KiB, at most 16384 of both together, 4096 if tau-aware.  The launch is
+    reported as ms_normmap_b; tau-aware, it leaves out tiles of norm zero only, in both copies."""
+    strips = 2 * (N // tile) * -(-N * int(in_bytes) // 1024)
+    return strips <= (4096 if tau_aware else 16384)
+
+
 def measured_traffic(workload, profile_dir=PROFILE_DIR):
     """HBM-side bytes per launch of each kernel of `workload`, read from the committed rocprofv3
     summaries: every profiles/*.txt carries lines `traffic <workload> <kernel key> <bytes>`
@@ -283,19 +291,28 @@ def main():
     # re-run the same steps reading the events after each one (reading needs a sync, so it is
     # kept out of the wall-clock loop above)
     stage, st = event_ms(lambda: ctx.multiply(tA, tB, tile, tau, C=dC, timing=True, prune=prune), args.steps)
-    # bytes the A pass writes: tile (i, k) is copied iff fl32(nA[i,k] * max_j nB[k,j]) >= tau
+    # bytes the A pass writes: tile (i, k) is copied iff fl32(nA[i,k] * max_j nB[k,j]) >= tau; converted together
+    # with B, every tile of non-zero norm
     nA_h, nB_h = ctx.get_normmap(sp.ROLE_A), ctx.get_normmap(sp.ROLE_B)
     # and the B pass every tile of non-zero norm
     a_tiles = nb * nb
     pruned = prune and tau > 0
-    a_written = int(np.count_nonzero(nA_h * nB_h.max(axis=1)[None, :] >= np.float32(tau))) if pruned else a_tiles
+    paired = paired_passes(N, tile, 2 if in16 else 4, pruned)
+
+    def a_tiles_written(in_bytes):
+        if not pruned:
+            return a_tiles
+        if paired_passes(N, tile, in_bytes, True):
+            return int(np.count_nonzero(nA_h))
+        return int(np.count_nonzero(nA_h * nB_h.max(axis=1)[None, :] >= np.float32(tau)))
+    a_written = a_tiles_written(2 if in16 else 4)
     b_written = int(np.count_nonzero(nB_h)) if pruned else a_tiles
     kept, total = int(st.kept_products), int(st.total_products)
     flops = kept * 2.0 * tile ** 3
     value = flops / (ms_step * 1e-3) / 1e12
     gemm_tflops = flops / (stage[3] * 1e-3) / 1e12
     in_b = 2.0 if in16 else 4.0                                         # bytes per input element
-    nm_bytes = in_b * N * N + 2.0 * N * N + 4.0 * nb * nb               # per matrix, every tile written
+    nm_bytes_all = in_b * N * N + 2.0 * N * N + 4.0 * nb * nb           # per matrix, every tile written
     nm_bytes_a = in_b * N * N + 2.0 * tile * tile * a_written + 4.0 * nb * nb
     nm_bytes_b = in_b * N * N + 2.0 * tile * tile * b_written + 8.0 * nb * nb
     # operand bytes the GEMM must read at least once: the distinct fp16 tiles A(i,k) / B(k,j) that some
@@ -309,7 +326,10 @@ def main():
     gemm_alg_bytes = 4.0 * N * N + 2.0 * tile * tile * (a_tiles_read + b_tiles_read)
     structure = gemm_structure(ctx, N, tile, kept)
     trace_us = measured_trace_us(args.workload)
-    nm_gbs = nm_bytes_b / (stage[0] * 1e-3) / 1e9                      # the B pass
+    # the B pass; paired, the one launch, which also covers A's bytes
+    nm_bytes = nm_bytes_b + (nm_bytes_a if paired else 0.0)
+    nm_gbs = nm_bytes / (stage[0] * 1e-3) / 1e9
+    nm_trace_us = trace_us.get("k_normmap_b", 0.0) + (trace_us.get("k_normmap_a", 0.0) if paired else 0.0)
 
     out = {
         "metric": "spamm_effective_tflops_kept_tiles",
@@ -354,17 +374,20 @@ def main():
             "traffic_over_algorithmic": (round(traffic["k_gemm"] / gemm_alg_bytes, 3) if "k_gemm" in traffic else None),
         },
         "roofline_normmap": {
-            "kernel": "k_normmap<%d, B role> (fp32->fp16 + tile norms)" % tile, "bound": "hbm",
+            "kernel": ("k_normmap_pair<%d> (both operands: fp16 copies + tile norms)" if paired
+                       else "k_normmap<%d, B role> (fp32->fp16 + tile norms)") % tile, "bound": "hbm",
             "achieved": round(nm_gbs, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
             "frac": round(nm_gbs / PEAK_HBM_GBS, 4),
-            "traffic": traffic.get("k_normmap_b" if pruned else "k_normmap_b_unpruned"),
-            "bytes_per_launch": nm_bytes_b, "avg_launch_ms": round(stage[0], 4),
+            "traffic": ((traffic["k_normmap_a"] + traffic["k_normmap_b"] if "k_normmap_a" in traffic else None) if paired
+                        else traffic.get("k_normmap_b" if pruned else "k_normmap_b_unpruned")),
+            "bytes_per_launch": nm_bytes, "avg_launch_ms": round(stage[0], 4),
             "frac_basis": "HIP events: the first stage's interval includes the gap before its kernel starts",
-            "frac_by_kernel_trace": (round(nm_bytes_b / (trace_us["k_normmap_b"] * 1e-6) / 1e9 / PEAK_HBM_GBS, 4)
-                                     if "k_normmap_b" in trace_us and pruned else None),
-            "kernel_trace_avg_launch_ms": round(trace_us["k_normmap_b"] * 1e-3, 4) if "k_normmap_b" in trace_us else None,
-            "tiles_written": b_written, "tiles": a_tiles, "bytes_per_launch_all_tiles": nm_bytes,
+            "frac_by_kernel_trace": (round(nm_bytes / (nm_trace_us * 1e-6) / 1e9 / PEAK_HBM_GBS, 4)
+                                     if nm_trace_us and pruned else None),
+            "kernel_trace_avg_launch_ms": round(nm_trace_us * 1e-3, 4) if nm_trace_us else None,
+            "tiles_written": b_written, "tiles": a_tiles, "bytes_per_launch_all_tiles": nm_bytes_all * (2 if paired else 1),
             "a_pass": {"tiles_written": a_written, "tiles": a_tiles, "bytes_per_launch": nm_bytes_a,
+                       "in_the_launch_above": True} if paired else {"tiles_written": a_written, "tiles": a_tiles, "bytes_per_launch": nm_bytes_a,
                        "avg_launch_ms": round(stage[1], 4),
                        "achieved": round(nm_bytes_a / (stage[1] * 1e-3) / 1e9, 1),
                        "frac": round(nm_bytes_a / (stage[1] * 1e-3) / 1e9 / PEAK_HBM_GBS, 4),
@@ -393,10 +416,13 @@ def main():
                 bw, aw = written
                 bb = in_bytes_elem * N * N + 2.0 * tile * tile * bw + 8.0 * nb * nb
                 ba = in_bytes_elem * N * N + 2.0 * tile * tile * aw + 4.0 * nb * nb
-                v["normmap_b_pass"] = {"bytes_per_launch": bb, "GBps": round(bb / (sg[0] * 1e-3) / 1e9, 1),
-                                       "frac_of_hbm_peak": round(bb / (sg[0] * 1e-3) / 1e9 / PEAK_HBM_GBS, 4)}
-                v["normmap_a_pass"] = {"bytes_per_launch": ba, "GBps": round(ba / (sg[1] * 1e-3) / 1e9, 1),
-                                       "frac_of_hbm_peak": round(ba / (sg[1] * 1e-3) / 1e9 / PEAK_HBM_GBS, 4)}
+                def rate(nbytes, ms_):
+                    gbs = nbytes / (ms_ * 1e-3) / 1e9
+                    return {"bytes_per_launch": nbytes, "GBps": round(gbs, 1), "frac_of_hbm_peak": round(gbs / PEAK_HBM_GBS, 4)}
+                if paired_passes(N, tile, in_bytes_elem, pruned and name != "no_prune"):
+                    v["normmap_both_passes"] = rate(bb + ba, sg[0])
+                else:
+                    v["normmap_b_pass"], v["normmap_a_pass"] = rate(bb, sg[0]), rate(ba, sg[1])
             variants[name] = v
 
         if prune:
@@ -408,7 +434,7 @@ def main():
             variant("fp16_inputs", "spamm_multiply_f16 on fp16 copies made before the timed region (the reference's "
                     "own timed region: para.h:1, cuSpAMM.cu:461-541); passes read 2 bytes per element",
                     lambda: ctx.multiply(hA, hB, tile, tau, C=dC, prune=prune),
-                    lambda: ctx.multiply(hA, hB, tile, tau, C=dC, timing=True, prune=prune), 2.0, (b_written, a_written))
+                    lambda: ctx.multiply(hA, hB, tile, tau, C=dC, timing=True, prune=prune), 2.0, (b_written, a_tiles_written(2)))
             del hA, hB
         # one B against many A: B's fp16 copy and norm map stay resident (A's pass, gate, GEMM remain)
         ctx.multiply(tA, tB, tile, tau, C=dC, prune=prune)

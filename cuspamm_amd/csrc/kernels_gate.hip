@@ -216,7 +216,7 @@ __global__ __launch_bounds__(NTH) void k_gate(GateBuffers g, int nbM, int nbK, i
                 // ---- phase 2c: union list with per-tile bits.  Entries whose k is kept by every
                 // tile of the macro tile ("full") come first, then the partial ones, each group
                 // in ascending k rotated to the anchor: the GEMM runs a branch-free loop over the
-                // first group.
+                // first group.  (k_small lists its units' k in the same order; C's bits depend on it.)
                 const int k1 = (w0 + cwn) * 64 < nbK ? (w0 + cwn) * 64 : nbK;
                 for (int k = w0 * 64 + threadIdx.x; k < k1; k += NTH) {
                     const int w = k >> 6, b = k & 63;

@@ -465,8 +465,10 @@ static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int 
             // fp32 input: strips of 128 columns where there are few (1024^2, both passes: 5.4 -> 4.4 us; 4096^2 36.1 ->
             // 36.7), of 256 by eight waves on middling grids (N = 8192: 0.066 / 0.058 -> 0.063 / 0.056 ms), by four waves,
             // two groups per lane, on large ones (N = 16384: as fast or 1 % faster)
-            // fp16 input, 3 to 4 strips of 256 columns per CU, of which three run at once: strips of 512 in two phases by eight
-            // waves are one turn instead of two (4096^2, A = B: 19.8 against 21.4 us)
+            // fp16 input, 3 to 4 strips of 256 columns per CU (of a whole chip), of which three run at once: strips of 512 in
+            // two phases by eight waves are one turn instead of two.  256 -> 512, A and B pass alone, A = B with the fill of C
+            // behind it: 4096^2 12.5 -> 11.1 us, 12.8 -> 11.6, 42.1 -> 39.1; 3840^2 11.2 -> 10.5, 11.1 -> 10.9, 39.7 -> 37.5;
+            // 3648^2 10.5 -> 10.1, 10.3 -> 10.5, 38.4 -> 36.4; 3584^2 8.9 -> 9.1, 9.5 -> 9.9, 37.0 -> 35.8
             if constexpr (IN16) {
                 if (strips(256) > 768u && strips(256) <= 1024u) SPAMM_NORMMAP(64, 512, 2, 8);
                 else SPAMM_NORMMAP(64, 256, 1, 4);
@@ -510,7 +512,8 @@ static void launch_pair(const void *A, const void *Bm, int64_t nbM, int64_t nbK,
                                                                         (uint4 *)packedB, nmA, nmB, nmBt, tau_skip, kept);
 }
 
-// Where the two passes are worth running as one (strips of both operands).  Whole multiplies, two passes -> one:
+// Where the two passes are worth running as one, by the strips of both operands, counted as tile rows of 1 KiB (256
+// columns of floats, 512 of halves, whatever width the passes take).  Whole multiplies, two passes -> one:
 // 256^3 14.6 -> 10.7 us, 2048^3 28.3 -> 23.9, 4096^3 87.2 -> 83.9, 6144^3 184 -> 182, 8192^3 912.5 -> 909.5; tile 64
 // beyond that runs four waves per workgroup in passes of their own.  A tau-aware A pass of its own (behind k_rowmax)
 // writes less: 3 us less at 4096^3, where the second launch and k_rowmax cost 8, and 13 us less at 8192^3.

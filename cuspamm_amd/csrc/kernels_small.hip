@@ -18,9 +18,9 @@
 // results out -- of which units of 128 (16 KiB a stage, two workgroups per CU) make
 // the k loop shortest and units of 64 spread a small C over more CUs.  Gate, schedule
 // and GEMM as launches of their own -> this kernel, whole multiplies: 256^3 24.6 -> 14.7 us
-// (10.7 with one launch for both norm-map passes), 1056 x 1568 x 1312 38.2 -> 22.8 (18.4),
-// 2048^3 at tile 32, 5 % kept, 38.5 -> 26.3 (24.8), 2048^3 dense 63 -> 38, 1024 rows
-// against a resident 8192^2 50.3 -> 36.5.
+// (today, with one launch for both norm-map passes too: 10.7), 1056 x 1568 x 1312 38.2 -> 22.8
+// (18.5), fp16 2048^3 at tile 32, 5 % kept, 38.5 -> 26.3 (22.5), 2048^3 dense 63 -> 38, 1024 rows
+// against a resident 8192^2 50.3 -> 36.5 (35.8).
 #include "gemm_device.h"
 
 namespace spamm {
@@ -360,9 +360,13 @@ hipError_t launch_clear_kept(int64_t *kept, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Unit by units of 128 in C: with half a unit per CU or more the wide one is faster (256 units: 10 % kept 26.4 -> 24.0 us,
-// dense 51.7 -> 37.6; 144 units: dense 34.8 -> 29.4, 10 % 19.2 -> 20.5), below it the narrow one (99 units: 20.1 -> 18.4,
-// 64 units: 15.4 -> 13.1 and, dense, 21.7 -> 20.6).
+// Unit by units of 128 in C: the wide one from half a unit per CU on.  Resident operands, K = 2048 at tile 32 (64 within
+// 10 %), 2 %, 10 %, 30 % kept and dense, narrow -> wide: 256 units 13.7 -> 12.4, 17.9 -> 15.3, 27.2 -> 20.0, 37.1 -> 24.9 us;
+// 196 units 12.3 -> 12.4, 15.7 -> 15.2, 20.7 -> 19.4, 36.1 -> 23.7; 144 units 10.0 -> 12.2, 13.4 -> 14.5, 17.8 -> 18.5,
+// 28.0 -> 22.9; 128 units 9.9 -> 12.4, 12.8 -> 15.0, 16.0 -> 19.8, 23.8 -> 22.9.  So between 128 and 196 units the line is a
+// choice: a sparse product pays some 2 us there for the 5 to 12 that a dense one, or one of more k, saves (144 units,
+// K = 6144: 30 % kept 28.7 -> 24.7, dense 62.8 -> 47.8).  Below it the narrow one (whole calls, wide -> narrow: 99 units
+// 20.1 -> 18.4, 64 units 15.4 -> 13.1 and, dense, 21.7 -> 20.6).
 static int small_unit(int64_t M, int64_t N) {
     const int64_t units128 = ((M + 127) / 128) * ((N + 127) / 128);
     return units128 >= 128 ? 128 : 64;

@@ -56,10 +56,10 @@ struct TauWorkspace {
 
 size_t tau_workspace_bytes() { return sizeof(TauWorkspace); }
 
-// Every product once: a wave takes one tile row i, 16 tile columns and 64 k, lane = k.  f(product,
+// Every product once: a wave takes one tile row i, TAU_JB tile columns and 64 k, lane = k.  f(product,
 // live) runs in all lanes; `live` is false in lanes beyond the last k.  A wave's step is one round trip
-// of 17 loads and some hundred instructions, so the steps are kept small and spread over as many waves
-// as there are (whole rows of k per wave: 22 us instead of 15 for the last pass over 1.7e7 products).
+// of TAU_JB + 1 loads and some hundred instructions, so the steps are kept small and spread over as many
+// waves as there are (whole rows of k per wave: 22 us instead of 15 for the last pass over 1.7e7 products).
 template <int TAU_JB, typename F>
 __device__ __forceinline__ void for_products(const float *__restrict__ nA, const float *__restrict__ nBt, int nbM, int nbK,
                                              int nbN, F &&f) {
@@ -68,7 +68,7 @@ __device__ __forceinline__ void for_products(const float *__restrict__ nA, const
     const int jb = (nbN + TAU_JB - 1) / TAU_JB, kb = (nbK + 63) / 64;
     const int64_t units = (int64_t)nbM * jb * kb;
     for (int64_t u = (int64_t)blockIdx.x * TAU_NW + wave; u < units; u += (int64_t)gridDim.x * TAU_NW) {
-        // (nbM * jb <= 65535 * 4096; the 64-bit division is a long routine that small problems need not run)
+        // (nbM * jb <= 65535 * 16384 < 2^31; the 64-bit division is a long routine that small problems need not run)
         const int ij = units <= 0x7fffffff ? (int)u / kb : (int)(u / kb);
         const int k0 = (int)(u - (int64_t)ij * kb) * 64;
         const int i = ij / jb, j0 = (ij % jb) * TAU_JB;

@@ -166,9 +166,10 @@ GateBuffers gate_buffers(spamm_ctx *c) {
 }
 
 // Work unit of the gated GEMM when the caller has not fixed it: with at most half a macro tile per CU
-// halves double the workgroups that run at once (2048^3 at tile 32, 64 macro tiles: -6 %); from one
+// halves double the workgroups that run at once (64 macro tiles: -6 %); from one
 // macro tile per CU on, whole macro tiles by four waves are as fast or faster (4096^3 dense, 256 macro
-// tiles: halves +7 %; 128 flop per staged byte against 85).  Between one and three COMPUTING macro
+// tiles: halves +7 %; 128 flop per staged byte against 85).  So small a C comes here only with K / tile beyond
+// what k_small lists, or with the gate's chunk fixed (is_small).  Between one and three COMPUTING macro
 // tiles per CU halves can win up to 10 % by finer rounds (270 on 256 CUs), but that count is known
 // only on the device after the gate, and the host chooses the launch.
 int gemm_shape_for(const spamm_ctx *c) {

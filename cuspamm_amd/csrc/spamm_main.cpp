@@ -157,7 +157,8 @@ int main(int argc, char **argv) {
     printf("SpAMM time=%fs\n", sum / (testtime - warmup - 1));
     printf("valid products=%lld of %lld (ratio %f)\n", (long long)st.kept_products, (long long)st.total_products,
            st.total_products ? (double)st.kept_products / (double)st.total_products : 0.0);
-    printf("stages: normmap B %.4f ms, normmap A %.4f ms, gate %.4f ms, multiply %.4f ms\n", st.ms_normmap_b,
+    printf("stages: normmap B %.4f ms, normmap A %.4f ms, gate %.4f ms, multiply %.4f ms"
+           " (one launch for both norm maps counts as B's, one for gate and multiply as the multiply's)\n", st.ms_normmap_b,
            st.ms_normmap_a, st.ms_gate, st.ms_gemm);
     if (check) {
         double e3[3] = {0, 0, 0}, bound = 0.0;

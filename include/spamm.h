@@ -48,16 +48,17 @@ extern "C" {
 #define SPAMM_FLAG_REUSE_A 4u    /* A's fp16 copy and norm map from an earlier call are reused (dA ignored) */
 #define SPAMM_FLAG_REUSE_B 8u    /* same for B: e.g. one B against many A, or matrix powers */
 #define SPAMM_FLAG_PRUNE 16u     /* tau-aware conversion passes (tau > 0): the fp16 copy of a tile is written only if some
-                                  * product can keep it.  A tile A_ik: fl(|A_ik| * max_j |B_kj|) >= tau (B's norms are
-                                  * complete when A's pass runs).  B tile B_kj: |B_kj| > 0 (B's pass runs first; a
-                                  * tile of norm zero fails the gate against any A).  Exact: fp32 rounding is
-                                  * monotone, so every product of a skipped tile fails the gate.  C, mask and counts
-                                  * are identical to a call without the flag; the passes write less.  Afterwards the
+                                  * product can keep it.  A tile A_ik: fl(|A_ik| * max_j |B_kj|) >= tau where A is
+                                  * converted by a pass of its own, behind B's (a large call, or a resident B).
+                                  * B tile B_kj: |B_kj| > 0 (a tile of norm zero fails the gate against any A).
+                                  * Where one launch converts both operands (a small call, or SPAMM_FLAG_A_EQ_B at
+                                  * tile 32 and 64) no other norms are known, and A's rule is B's.  Exact: fp32
+                                  * rounding is monotone, so every product of a skipped tile fails the gate.  C, mask
+                                  * and counts are identical to a call without the flag; the passes write less.  Afterwards the
                                   * copies are incomplete: SPAMM_FLAG_REUSE_A is accepted only together with
                                   * SPAMM_FLAG_REUSE_B and tau' >= tau, SPAMM_FLAG_REUSE_B only with tau' > 0, and
                                   * spamm_get_fp16 and spamm_error_vs_dense_f64 return SPAMM_ESTATE until the
-                                  * operand is converted again without the flag.  With SPAMM_FLAG_A_EQ_B (one pass, no
-                                  * row maxima yet) only tiles of norm zero are left out, in both copies.  Ignored
+                                  * operand is converted again without the flag.  Ignored
                                   * for tau <= 0.  No counterpart in the reference, which converts on the host
                                   * outside its timed region (tool.cu:418,432). */
 
@@ -106,8 +107,8 @@ SPAMM_API int spamm_destroy(spamm_ctx *ctx);
  *     macro tile of C (one workgroup per CU), 2 = four waves per 128 x 256 half (two workgroups per
  *     CU), 3 = eight waves per macro tile, 4 = shape 1 by workgroups that stay on their CU and draw
  *     macro tiles from a ticket counter per XCD; 0 = chosen per call (a small C -- at most 640
- *     blocks of 128 x 128, 512 for tau <= 0 -- is gated and multiplied by one kernel in units of 128
- *     or 64; otherwise 1, or halves when C has at most half a macro tile per CU).  All add in the same
+ *     blocks of 128 x 128, 512 for tau <= 0, and K / tile <= 2048 -- is gated and multiplied by one
+ *     kernel in units of 128 or 64; otherwise 1, or halves when C has at most half a macro tile per CU).  All add in the same
  *     order: C is bit-identical.
  * SPAMM_EINVAL for an unknown option or a value outside its range.  The reference has no such
  * knobs: its launch shapes are compile-time constants (main.h:32-73). */
