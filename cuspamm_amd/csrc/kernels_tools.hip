@@ -3,19 +3,24 @@
 // The reference compares SpAMM against a dense cuBLAS product and prints
 // ||C_dense - C_spamm||_F, ||C_dense||_F, ||C_spamm||_F (check_simple_gpu,
 // tool.cu:227-280; COUNTERRTRANS, tool.cu:6-24).  Here the dense product is
-// an exact fp64 product of the same fp16 operands, formed on the fp64 matrix
-// pipeline (v_mfma_f64_16x16x4_f64) block by block and reduced on the fly (it is
-// never stored), next to the tau-derived bound
+// the product of the same fp16 operands, formed block by block and reduced on the
+// fly (it is never stored): exactly, in whole numbers on the 8-bit integer matrix
+// pipeline (k_limbs, k_error_limbs), or on the fp64 one (k_error_dense,
+// v_mfma_f64_16x16x4_f64) where values are too large for that, K is too long, the
+// planes too big or the product too small.  Next to it the tau-derived bound
 // sqrt(sum_ij (sum_{k dropped} nA[i,k]*nB[k,j])^2).
 //
-// What bounds it: the fp64 matrix pipeline (128 operations per clock and CU) and the VALU's
+// What bounds k_error_dense: the fp64 matrix pipeline (128 operations per clock and CU) and the VALU's
 // conversions beside it -- fp16 to fp64 is two instructions per value, one of them at a
 // quarter of the rate, and they take the place of MFMAs.  So a wave's block of C is as large as
 // the number of blocks allows: each converted value serves NBR or NBC MFMAs.  4096^3:
 // 2229 us with 32 x 32 per wave and 4-byte loads, 2109 now (65 TFLOP/s; the pipeline's 128 operations at the clock
-// that the chip holds under them, about 2 GHz); 1984 x 2176 x 768: 196 -> 158.  The scalar bound of 64 x 64 x 64
-// tiles 52 -> 7 us, the per-tile one 51 -> 4; results go straight to host memory (a clearing launch before and a copy
-// after each were 25 us a call): the whole report 2429 -> 2174 us at 4096^3, 380 -> 244 at 1984 x 2176 x 768.
+// that the chip holds under them, about 2 GHz); 1984 x 2176 x 768: 196 -> 158.  In whole numbers instead (one call, its
+// host wait included): 4096^3 2107 -> 867 us on uniform values in [-1, 1) (4 bytes each, 16 products, 2.6 Pop/s: power),
+// 620 where 3 bytes do, 272 on exp(-d / 100); 1984 x 2176 x 768 165 -> 82, 67, 49; 64 rows of 4096^3 173 -> 109, 91, 50.
+// The scalar bound of 64 x 64 x 64 tiles 52 -> 7 us, the per-tile one 51 -> 4; results go straight to host memory (a
+// clearing launch before and a copy after each were 25 us a call).
+#include "gemm_device.h"
 #include "reduce_device.h"
 
 namespace spamm {
@@ -25,7 +30,7 @@ typedef _Float16 half8t __attribute__((ext_vector_type(8)));
 
 struct ReportWorkspace {
     unsigned int ticket;                // workgroups of the running launch that have finished; zero between launches
-    unsigned int pad_;
+    unsigned int out_of_range;          // k_limbs: an operand holds values without limbs; zero between calls
     double part[1];                     // per workgroup: its sums (report_workspace_bytes says how many)
 };
 
@@ -38,10 +43,12 @@ __device__ __forceinline__ void finish_sums(ReportWorkspace *ws, double own, Rep
     if (threadIdx.x < N)
         agent_store(reinterpret_cast<unsigned long long *>(&ws->part[(size_t)blockIdx.x * N + threadIdx.x]), __builtin_bit_cast(unsigned long long, own));
     if (!last_workgroup(&ws->ticket)) return;
+    if (threadIdx.x == 0) agent_store(&ws->out_of_range, 0u);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     double v[N];
 #pragma unroll
     for (int i = 0; i < N; i++) v[i] = 0.0;
+#pragma unroll 4
     for (unsigned b = threadIdx.x; b < gridDim.x; b += 256)
 #pragma unroll
         for (int i = 0; i < N; i++)
@@ -162,6 +169,222 @@ __global__ __launch_bounds__(256, NBR * NBC > 8 ? 2 : 3) void k_error_dense(cons
     finish_sums<3>(ws, own, host_out, host_seq, seq);
 }
 
+// ---- the dense product in whole numbers ----
+//
+// Every finite fp16 value is a whole number of 2^-24, so values below 127 in magnitude are four signed bytes
+// ("limbs", balanced digits to the base 256) and a product of fp16 matrices is a sum of 8-bit integer products, at
+// some thirty times the fp64 pipeline's rate each and exact in 32-bit accumulators: limb i of A times limb j of B
+// adds to order i + j.  A block needs only the limbs its largest value reaches (the values of a matrix that decays
+// need fewer with every factor of 256, and a block of zeros none), so 0 to 16 products take the place of one.  What the
+// fp64 pipeline rounds at every step is exact here up to the last addition.
+//
+// k_limbs splits the packed copies: per block of 64 rows (columns of B) x 64 k the number of limbs it needs, and that
+// many planes of 4 KiB: [limb][16 rows][lane][16 bytes], a lane's 16 bytes an operand of v_mfma_i32_16x16x64_i8
+// (lane l: row l % 16, 16 k from l / 16; which k goes where is the same for A and B).
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+constexpr int LIMB_BLOCK = 64, LIMB_PLANE = LIMB_BLOCK * LIMB_BLOCK, LIMBS = 4;
+constexpr float LIMB_MAX = 127.0f;
+
+struct LimbOperand {
+    const _Float16 *packed;     // the whole operand's packed copy
+    int8_t *planes;             // [block rows][nkb][LIMBS][LIMB_PLANE]
+    uint8_t *cls;               // [block rows][nkb]: limbs of the block
+    int64_t row0;               // first row (column of B) to be split, a multiple of 64
+    int64_t n_blocks;           // blocks of 64 rows, times nkb
+};
+
+__global__ __launch_bounds__(256) void k_limbs(LimbOperand a, LimbOperand b, int64_t K, int tile, int nkb, ReportWorkspace *__restrict__ ws) {
+    __shared__ unsigned int s_used[4];
+    const bool is_a = (int64_t)blockIdx.x < a.n_blocks;
+    const LimbOperand op = is_a ? a : b;
+    const int64_t blk = is_a ? blockIdx.x : blockIdx.x - a.n_blocks;
+    const int kb = (int)(blk % nkb);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t r = op.row0 + (blk / nkb) * LIMB_BLOCK + wave * 16 + (lane & 15);
+    const int64_t k = (int64_t)kb * LIMB_BLOCK + (lane >> 4) * 16;
+    half8t h0 = {}, h1 = {};
+    if (k < K) {                // (K is a multiple of 32: the last block may end halfway)
+        const _Float16 *src = op.packed + ((r / tile) * (K / tile) + k / tile) * ((int64_t)tile * tile) + (k % tile) * tile + (r % tile) * 8;
+        h0 = *reinterpret_cast<const half8t *>(src);
+        h1 = *reinterpret_cast<const half8t *>(src + (int64_t)tile * 8);
+    }
+    unsigned int w[16], used = 0;
+    bool fits = true;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+        const float x = (float)(e < 8 ? h0[e & 7] : h1[e & 7]);
+        fits = fits && __builtin_fabsf(x) < LIMB_MAX;                   // (false for a NaN)
+        const int v = (int)((__builtin_fabsf(x) < LIMB_MAX ? x : 0.0f) * 16777216.0f);       // exact
+        w[e] = ((unsigned int)v + 0x00808080u) ^ 0x00808080u;           // byte i is digit i
+        used |= w[e];
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) used |= __shfl_xor(used, off, 64);
+    if (__ballot(!fits) != 0ull && lane == 0) agent_store(&ws->out_of_range, 1u);
+    if (lane == 0) s_used[wave] = used;
+    __syncthreads();
+    used = s_used[0] | s_used[1] | s_used[2] | s_used[3];
+    const int limbs = used == 0 ? 0 : (31 - __builtin_clz(used)) / 8 + 1;
+    if (threadIdx.x == 0) op.cls[blk] = (uint8_t)limbs;
+    int8_t *out = op.planes + blk * (LIMBS * LIMB_PLANE) + threadIdx.x * 16;
+#pragma unroll
+    for (int l = 0; l < LIMBS; l++) {
+        if (l >= limbs) break;
+        i32x4 v;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            // bytes l of four words
+            const unsigned int lo = __builtin_amdgcn_perm(w[4 * g + 1], w[4 * g], 0x0c0c0400u + 0x0101u * l);
+            const unsigned int hi = __builtin_amdgcn_perm(w[4 * g + 3], w[4 * g + 2], 0x0c0c0400u + 0x0101u * l);
+            v[g] = (int)(lo | hi << 16);
+        }
+        *reinterpret_cast<i32x4 *>(out + l * LIMB_PLANE) = v;
+    }
+}
+
+// One workgroup owns 64 x 64 of C, a wave 32 x 32 of it: 4 accumulator registers x 4 MFMA blocks x 7 orders, so that two
+// waves share a SIMD.  The k blocks are sorted by the limbs they need on both sides (whole numbers: the sum does not
+// care), and each kind has a loop of its own without branches, the next block's operands on their way while one is
+// multiplied.  Groups of GB x GB workgroups that share operands in an L2 run on one XCD; the groups of a diagonal, which
+// have much the same work, are spread over the XCDs.
+constexpr int ORDERS = 2 * LIMBS - 1;
+constexpr int64_t LIMB_MAX_K = 32768 - 64;      // an order adds up to 4 products of at most 2^14 per k in 31 bits
+constexpr int LIMB_MAX_KB = 32768 / LIMB_BLOCK;
+
+__global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict__ plA, const uint8_t *__restrict__ clsA,
+                                                        const int8_t *__restrict__ plB, const uint8_t *__restrict__ clsB, int nkb,
+                                                        int nbi, int nbj, int gb, int gj_rounds, int n_xcd, int64_t N,
+                                                        const float *__restrict__ C, ReportWorkspace *__restrict__ ws,
+                                                        ReportSums *__restrict__ host_out, unsigned long long *__restrict__ host_seq,
+                                                        unsigned long long seq) {
+    __shared__ double red[4][3];
+    __shared__ int s_count[17], s_place[16];
+    __shared__ uint16_t s_list[LIMB_MAX_KB];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wr = wave >> 1, wc = wave & 1;
+    const int l16 = lane & 15, q = lane >> 4;
+    const int x = (int)blockIdx.x % n_xcd, at = (int)blockIdx.x / n_xcd, in_group = at % (gb * gb), group = at / (gb * gb);
+    const int gi = group / gj_rounds, gj = (group % gj_rounds) * n_xcd + (x + n_xcd * 2 * gi - 2 * gi) % n_xcd;
+    const int bi = gi * gb + in_group / gb, bj = gj * gb + in_group % gb;
+    const bool bad = ws->out_of_range != 0u;
+    double e2 = 0, d2 = 0, c2 = 0;
+    if (bi < nbi && bj < nbj && !bad) {
+        // ---- k blocks by kind
+        if (threadIdx.x < 17) s_count[threadIdx.x] = 0;
+        __syncthreads();
+        const uint8_t *ca = clsA + (int64_t)bi * nkb, *cb = clsB + (int64_t)bj * nkb;
+        int kind[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int kb = h * 256 + (int)threadIdx.x;
+            const int la = kb < nkb ? ca[kb] : 0, lb = kb < nkb ? cb[kb] : 0;
+            kind[h] = la && lb ? (la - 1) * LIMBS + lb - 1 : -1;
+            if (kind[h] >= 0) atomicAdd(&s_count[kind[h] + 1], 1);
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            int sum = 0;
+            for (int i = 0; i < 16; i++) {
+                s_place[i] = sum;
+                sum += s_count[i + 1];
+                s_count[i + 1] = sum;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            if (kind[h] >= 0) s_list[atomicAdd(&s_place[kind[h]], 1)] = (uint16_t)(h * 256 + threadIdx.x);
+        __syncthreads();
+
+        const int8_t *srcA = plA + (int64_t)bi * nkb * (LIMBS * LIMB_PLANE) + wr * 2048 + lane * 16;
+        const int8_t *srcB = plB + (int64_t)bj * nkb * (LIMBS * LIMB_PLANE) + wc * 2048 + lane * 16;
+        i32x4 acc[ORDERS][2][2];
+#pragma unroll
+        for (int o = 0; o < ORDERS; o++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) acc[o][t >> 1][t & 1] = i32x4{0, 0, 0, 0};
+        static_for<LIMBS * LIMBS>([&](auto kind_) {
+            constexpr int LA = decltype(kind_)::value / LIMBS + 1, LB = decltype(kind_)::value % LIMBS + 1;
+            const int s = __builtin_amdgcn_readfirstlane(s_count[decltype(kind_)::value]);
+            const int e = __builtin_amdgcn_readfirstlane(s_count[decltype(kind_)::value + 1]);
+            if (s == e) return;
+            struct Frags {
+                i32x4 a[LA][2], b[LB][2];
+            };
+            auto load = [&](Frags &f, int i) {
+                const int64_t off = (int64_t)__builtin_amdgcn_readfirstlane((int)s_list[i < e ? i : e - 1]) * (LIMBS * LIMB_PLANE);
+#pragma unroll
+                for (int l = 0; l < LA; l++)
+#pragma unroll
+                    for (int t = 0; t < 2; t++) f.a[l][t] = *reinterpret_cast<const i32x4 *>(srcA + off + l * LIMB_PLANE + t * 1024);
+#pragma unroll
+                for (int l = 0; l < LB; l++)
+#pragma unroll
+                    for (int t = 0; t < 2; t++) f.b[l][t] = *reinterpret_cast<const i32x4 *>(srcB + off + l * LIMB_PLANE + t * 1024);
+            };
+            auto multiply = [&](const Frags &f) {
+#pragma unroll
+                for (int i = 0; i < LA; i++)
+#pragma unroll
+                    for (int j = 0; j < LB; j++)
+#pragma unroll
+                        for (int t = 0; t < 4; t++)
+                            acc[i + j][t >> 1][t & 1] =
+                                __builtin_amdgcn_mfma_i32_16x16x64_i8(f.a[i][t >> 1], f.b[j][t & 1], acc[i + j][t >> 1][t & 1], 0, 0, 0);
+            };
+            if constexpr (LA + LB <= 6) {
+                Frags f0, f1;
+                load(f0, s);
+                int i = s;
+                for (; i + 1 < e; i += 2) {
+                    load(f1, i + 1);
+                    multiply(f0);
+                    load(f0, i + 2);
+                    multiply(f1);
+                }
+                if (i < e) multiply(f0);
+            } else {            // (two sets of operands would not fit the registers; the other wave of the SIMD multiplies meanwhile)
+                for (int i = s; i < e; i++) {
+                    Frags f;
+                    load(f, i);
+                    multiply(f);
+                }
+            }
+        });
+        // accumulator i of lane l in block t: row 4 (l / 16) + i, column l % 16; orders 0 to 3 and 4 to 6 are added in
+        // 64-bit integers, so the one rounding is the last
+        const float *src = C + ((int64_t)bi * LIMB_BLOCK + wr * 32 + 4 * q) * N + (int64_t)bj * LIMB_BLOCK + wc * 32 + l16;
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const double c = (double)src[((t >> 1) * 16 + i) * N + (t & 1) * 16];
+                const long long lo = (long long)acc[0][t >> 1][t & 1][i] + ((long long)acc[1][t >> 1][t & 1][i] << 8) +
+                                     ((long long)acc[2][t >> 1][t & 1][i] << 16) + ((long long)acc[3][t >> 1][t & 1][i] << 24);
+                const long long hi = (long long)acc[4][t >> 1][t & 1][i] + ((long long)acc[5][t >> 1][t & 1][i] << 8) +
+                                     ((long long)acc[6][t >> 1][t & 1][i] << 16);
+                const double d = fma((double)hi, 4294967296.0, (double)lo) * (1.0 / 281474976710656.0);
+                e2 += (c - d) * (c - d);
+                d2 += d * d;
+                c2 += c * c;
+            }
+        for (int off = 32; off > 0; off >>= 1) {
+            e2 += __shfl_down(e2, off, 64);
+            d2 += __shfl_down(d2, off, 64);
+            c2 += __shfl_down(c2, off, 64);
+        }
+    }
+    if (lane == 0) {
+        red[wave][0] = bad ? -1.0 : e2;         // (a sum below zero: the host takes the fp64 product)
+        red[wave][1] = d2;
+        red[wave][2] = c2;
+    }
+    __syncthreads();
+    double own = 0.0;
+    if (threadIdx.x < 3) own = red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
+    finish_sums<3>(ws, own, host_out, host_seq, seq);
+}
+
 // Dropped norm products of every output tile: a wave takes one tile row and BOUND_JB tile columns, lane = k, so that a
 // step's loads go out together.  `per_tile` gets the tiles' sums, host_out (unless null) the sum of their squares, each
 // workgroup's share of it through the workspace: a 64-bit float add on one address by every wave was 50 us of the
@@ -212,7 +435,10 @@ __global__ __launch_bounds__(256) void k_dropped_bound(const float *__restrict__
     finish_sums<1>(ws, threadIdx.x == 0 ? red[0] + red[1] + red[2] + red[3] : 0.0, host_out, host_seq, seq);
 }
 
-__global__ void k_clear_report(ReportWorkspace *ws) { ws->ticket = 0; }
+__global__ void k_clear_report(ReportWorkspace *ws) {
+    ws->ticket = 0;
+    ws->out_of_range = 0;
+}
 
 hipError_t launch_clear_report(void *workspace, hipStream_t s) {
     k_clear_report<<<1, 1, 0, s>>>((ReportWorkspace *)workspace);
@@ -243,9 +469,41 @@ static int error_shape(int64_t rows, int64_t N, int n_cu, int64_t *n_wg) {
     return best;
 }
 
-size_t report_workspace_bytes(int64_t rows, int64_t N, int n_cu) {
+// Workgroups of k_error_limbs: groups of gb x gb, and how many of a group row an XCD has.
+struct LimbGrid {
+    int nbi, nbj, gb, gj_rounds;
+    int64_t n_wg;
+};
+static LimbGrid limb_grid(int64_t rows, int64_t N, int n_xcd) {
+    LimbGrid g;
+    g.nbi = (int)(rows / LIMB_BLOCK);
+    g.nbj = (int)(N / LIMB_BLOCK);
+    const int64_t blocks = (int64_t)g.nbi * g.nbj;
+    g.gb = blocks >= 2048 ? 8 : blocks >= 512 ? 4 : 1;
+    g.gj_rounds = ((g.nbj + g.gb - 1) / g.gb + n_xcd - 1) / n_xcd;
+    g.n_wg = (int64_t)((g.nbi + g.gb - 1) / g.gb) * g.gj_rounds * n_xcd * g.gb * g.gb;
+    return g;
+}
+
+static int64_t limb_kb(int64_t K) { return (K + LIMB_BLOCK - 1) / LIMB_BLOCK; }
+
+// Bytes of the planes and the blocks' numbers of limbs of both operands; 0: the fp64 pipeline is to be used -- beyond
+// what 32 bits add up, beyond 4 GiB of planes, and for so small a product that the second launch costs more than the
+// sums (256^3 26.5 us in fp64, 27 to 29 in whole numbers; 512^3 35.6 against 30 to 34).
+size_t limb_bytes(int64_t rows, int64_t K, int64_t N) {
+    if (K > LIMB_MAX_K || (double)rows * (double)K * (double)N < 64.0e6) return 0;
+    const size_t blocks = (size_t)(rows / LIMB_BLOCK + N / LIMB_BLOCK) * (size_t)limb_kb(K);
+    if (blocks >= (1u << 31) / (LIMBS * LIMB_PLANE / 2)) return 0;       // 4 GiB
+    return blocks * (LIMBS * LIMB_PLANE) + blocks;
+}
+
+size_t report_workspace_bytes(int64_t rows, int64_t N, int n_cu, int n_xcd) {
     int64_t n_wg = 0;
-    if (rows > 0) (void)error_shape(rows, N, n_cu, &n_wg);
+    if (rows > 0) {
+        (void)error_shape(rows, N, n_cu, &n_wg);
+        const int64_t n_limb = limb_grid(rows, N, n_xcd).n_wg;
+        if (n_limb > n_wg) n_wg = n_limb;
+    }
     const size_t doubles = 3 * (size_t)n_wg > BOUND_MAX_WG ? 3 * (size_t)n_wg : BOUND_MAX_WG;
     return sizeof(ReportWorkspace) + doubles * sizeof(double);
 }
@@ -261,6 +519,25 @@ hipError_t launch_error_vs_dense(const void *packedA, const void *packedB, int64
     if (shape == 0) k_error_dense<4, 4><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out, host_seq, seq);
     else if (shape == 1) k_error_dense<4, 2><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out, host_seq, seq);
     else k_error_dense<2, 2><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out, host_seq, seq);
+    return hipGetLastError();
+}
+
+hipError_t launch_error_limbs(const void *packedA, const void *packedB, int64_t K, int64_t N, int tile, const float *C,
+                              int64_t row0, int64_t row1, int n_xcd, void *limbs, void *workspace, ReportSums *host_out,
+                              unsigned long long *host_seq, unsigned long long seq, hipStream_t s) {
+    const LimbGrid g = limb_grid(row1 - row0, N, n_xcd);
+    const int nkb = (int)limb_kb(K);
+    const int64_t blocksA = (int64_t)g.nbi * nkb, blocksB = (int64_t)g.nbj * nkb;
+    ReportWorkspace *ws = (ReportWorkspace *)workspace;
+    int8_t *planes = (int8_t *)limbs;
+    uint8_t *cls = (uint8_t *)limbs + (blocksA + blocksB) * (LIMBS * LIMB_PLANE);
+    const LimbOperand a = {(const _Float16 *)packedA, planes, cls, row0, blocksA};
+    const LimbOperand b = {(const _Float16 *)packedB, planes + blocksA * (LIMBS * LIMB_PLANE), cls + blocksA, 0, blocksB};
+    k_limbs<<<(unsigned)(blocksA + blocksB), 256, 0, s>>>(a, b, K, tile, nkb, ws);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    k_error_limbs<<<(unsigned)g.n_wg, 256, 0, s>>>(a.planes, a.cls, b.planes, b.cls, nkb, g.nbi, g.nbj, g.gb, g.gj_rounds, n_xcd, N,
+                                                   C + row0 * N, ws, host_out, host_seq, seq);
     return hipGetLastError();
 }
 

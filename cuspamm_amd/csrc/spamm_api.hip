@@ -94,6 +94,7 @@ struct spamm_ctx : Workspace {
     DevBuf staging;   // read-back staging / decay table
     DevBuf tauws;     // tau selection workspace
     DevBuf reportws;  // error report workspace
+    DevBuf limbs;     // operands split for the error report's integer product
     double *tile_results = nullptr;   // pinned, TILE_RESULTS_MAX doubles at most: per-tile results of small outputs
     size_t tile_results_cap = 0;
     HostResults *results = nullptr;   // pinned: small results that a kernel writes and the host waits for
@@ -292,6 +293,7 @@ int spamm_destroy(spamm_ctx *c) {
     if (c->staging.p) (void)hipFree(c->staging.p);
     if (c->tauws.p) (void)hipFree(c->tauws.p);
     if (c->reportws.p) (void)hipFree(c->reportws.p);
+    if (c->limbs.p) (void)hipFree(c->limbs.p);
     if (c->tile_results) (void)hipHostFree(c->tile_results);
     if (c->results) (void)hipHostFree(c->results);
     for (int i = 0; i < 5; i++)
@@ -706,7 +708,7 @@ static int wait_result(spamm_ctx *c, unsigned long long seq) {
 static int report_prepare(spamm_ctx *c, int64_t rows) {
     int rc = ensure_results(c);
     if (rc) return rc;
-    const size_t bytes = report_workspace_bytes(rows, c->N, c->n_cu);
+    const size_t bytes = report_workspace_bytes(rows, c->N, c->n_cu, c->n_xcd);
     if (c->reportws.cap >= bytes) return SPAMM_OK;
     if ((rc = ensure(c, c->reportws, bytes))) return rc;
     HIPCHK(c, launch_clear_report(c->reportws.p, c->stream));
@@ -722,6 +724,19 @@ int spamm_error_vs_dense_f64(spamm_ctx *c, const float *dC, int64_t row0, int64_
     int rc = set_device(c);
     if (rc) return rc;
     if ((rc = report_prepare(c, row1 - row0))) return rc;
+    // exact in whole numbers where the operands' values allow it and their planes fit (else, and without memory for
+    // them, in fp64)
+    const size_t limbs = limb_bytes(row1 - row0, c->K, c->N);
+    if (limbs && ensure(c, c->limbs, limbs) == SPAMM_OK) {
+        const unsigned long long first = ++c->seq;
+        HIPCHK(c, launch_error_limbs(c->packedA.p, c->packedB.p, c->K, c->N, c->tile, dC, row0, row1, c->n_xcd, c->limbs.p, c->reportws.p,
+                                     &c->results->report, &c->results->seq, first, c->stream));
+        if ((rc = wait_result(c, first))) return rc;
+        if (!(c->results->report.v[0] < 0.0)) {
+            for (int i = 0; i < 3; i++) out3[i] = sqrt(c->results->report.v[i]);
+            return SPAMM_OK;
+        }
+    }
     const unsigned long long seq = ++c->seq;
     HIPCHK(c, launch_error_vs_dense(c->packedA.p, c->packedB.p, c->K, c->N, c->tile, dC, row0, row1, c->n_cu, c->reportws.p,
                                     &c->results->report, &c->results->seq, seq, c->stream));

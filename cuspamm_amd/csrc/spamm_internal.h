@@ -96,11 +96,17 @@ hipError_t launch_normmap_pair(const void *A, const void *Bm, bool in16, int64_t
 struct ReportSums {
     double v[3];
 };
-size_t report_workspace_bytes(int64_t rows, int64_t N, int n_cu);      // rows = 0: the bound only
+size_t report_workspace_bytes(int64_t rows, int64_t N, int n_cu, int n_xcd);      // rows = 0: the bound only
 hipError_t launch_clear_report(void *workspace, hipStream_t s);
 hipError_t launch_error_vs_dense(const void *packedA, const void *packedB, int64_t K, int64_t N, int tile, const float *C,
                                  int64_t row0, int64_t row1, int n_cu, void *workspace, ReportSums *host_out,
                                  unsigned long long *host_seq, unsigned long long seq, hipStream_t s);
+// the same on the integer matrix pipeline; limbs: limb_bytes() of scratch (0: not for this shape).  A first sum below
+// zero: an operand holds values it cannot take (beyond +-127, inf, NaN), the sums are not valid
+size_t limb_bytes(int64_t rows, int64_t K, int64_t N);
+hipError_t launch_error_limbs(const void *packedA, const void *packedB, int64_t K, int64_t N, int tile, const float *C,
+                              int64_t row0, int64_t row1, int n_xcd, void *limbs, void *workspace, ReportSums *host_out,
+                              unsigned long long *host_seq, unsigned long long seq, hipStream_t s);
 // host_out->v[0] (optional) = sum over tiles of s_ij^2, s_ij = sum_{k dropped} nA[i,k]*nB[k,j]; per_tile (optional): s_ij
 hipError_t launch_dropped_bound(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, float tau,
                                 void *workspace, ReportSums *host_out, unsigned long long *host_seq, unsigned long long seq,

@@ -343,3 +343,51 @@ def test_error_report_by_any_block_shape(ctx, rows, N, row0):
     assert want[0] > 0.01 * want[1]
     for got, ref in zip(ctx.error_vs_dense(C, row0, M), want):
         assert abs(got - ref) <= 1e-9 * ref
+
+
+@pytest.mark.parametrize("tile,M,K,N,row0,rows,kind", [
+    (32, 64, 32, 64, 0, 64, "unit"), (32, 192, 416, 320, 64, 128, "unit"), (64, 576, 1088, 640, 0, 576, "limbs"),
+    (32, 1024, 608, 2304, 128, 832, "limbs"), (128, 4096, 256, 2176, 0, 4096, "limbs"), (64, 512, 32704, 512, 0, 512, "edge"),
+    (64, 256, 32768, 256, 0, 256, "edge"), (64, 2048, 320, 1024, 0, 2048, "large"), (128, 512, 512, 512, 0, 512, "large"),
+    (64, 320, 192, 320, 0, 320, "inf"), (32, 256, 256, 256, 0, 256, "zero")])
+def test_error_report_over_the_range_of_fp16(ctx, tile, M, K, N, row0, rows, kind):
+    """Whatever the magnitudes: 0 to 4 bytes a value by blocks, just inside and outside of what bytes hold, subnormals,
+    infinities, sums at the length where 32 bits end.  Against fp64 on the host (K terms a sum, rows * N in a norm, 2^-53
+    each, below 1e-9); the exact product of whole multiples of 2^-24 is what both sides form."""
+    import torch
+    rng = np.random.default_rng(M + K + N)
+
+    def operand(r, c):
+        X = rng.uniform(-1.0, 1.0, (r, c))
+        if kind == "limbs":       # 64 x 64 blocks of every magnitude that needs 0 to 4 bytes, and what lies below fp16
+            X *= np.kron(np.exp2(rng.choice([-40, -22, -16, -15, -9, -8, -1, 0, 6], (-(-r // 64), -(-c // 64)))), np.ones((64, 64)))[:r, :c]
+        elif kind == "edge":      # the largest digits everywhere: 4 products a k and order, all of one sign
+            X = np.where(X < 0, -126.5, 126.5)
+            X[:, ::2] = np.where(X[:, ::2] < 0, -0.50196, 0.50196)
+        elif kind == "large":
+            X *= 60000.0
+        return X.astype(np.float32)
+
+    A, B = operand(M, K), operand(K, N)
+    if kind == "edge":
+        A, B = np.abs(A), np.abs(B)
+    if kind == "zero":
+        A[:] = 0
+    if kind == "inf":
+        A[70, 100] = np.inf
+    hA, hB = A.astype(np.float16).astype(np.float64), B.astype(np.float16).astype(np.float64)
+    ctx.normmap_f32(1, torch.from_numpy(B).cuda(), tile)
+    ctx.normmap_f32(0, torch.from_numpy(A).cuda(), tile)
+    with np.errstate(invalid="ignore"):
+        dense = hA[row0:row0 + rows] @ hB
+    C = np.zeros((M, N), dtype=np.float32)
+    C[row0:row0 + rows] = (0.75 * np.nan_to_num(dense, nan=1.0, posinf=1.0, neginf=1.0)).astype(np.float32)
+    c = C[row0:row0 + rows].astype(np.float64)
+    for _ in range(2):            # (the second call finds the workspace as the first left it)
+        got = ctx.error_vs_dense(torch.from_numpy(C).cuda(), row0, row0 + rows)
+        if kind == "inf":
+            assert not np.isfinite(got[0]) and not np.isfinite(got[1])
+            assert abs(got[2] - np.linalg.norm(c)) <= 1e-9 * np.linalg.norm(c)
+            continue
+        for g, ref in zip(got, (np.linalg.norm(c - dense), np.linalg.norm(dense), np.linalg.norm(c))):
+            assert abs(g - ref) <= 1e-9 * ref

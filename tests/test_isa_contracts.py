@@ -276,7 +276,7 @@ def test_results_are_published_when_the_workspace_is_at_rest(tmp_path):
     behind a publishing kernel's last barrier no wave stores anything but the result itself (to host memory, in system
     scope: sc0 sc1), and in the kernel whose waves all clear counters, every wave has waited for its stores before it."""
     publishing = [("kernels_tau.hip", r"_ZN5spamm10k_tau_histILi2E\w+", 1), ("kernels_tools.hip", r"_ZN5spamm13k_error_denseILi\w+", 3),
-                  ("kernels_tools.hip", r"_ZN5spamm15k_dropped_bound\w+", 1)]
+                  ("kernels_tools.hip", r"_ZN5spamm15k_dropped_bound\w+", 1), ("kernels_tools.hip", r"_ZN5spamm13k_error_limbs\w+", 1)]
     for src, name, count in publishing:
         kernels = re.findall(r"^(%s):[^\n]*\n(.*?)^\.Lfunc_end" % name, _isa(src, tmp_path), flags=re.S | re.M)
         assert len(kernels) == count, src
