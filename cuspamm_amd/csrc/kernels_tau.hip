@@ -6,8 +6,8 @@
 //    (11 + 11 + 10 bits, most significant first) over the nbM*nbN*nbK products,
 //    recomputed from the norm maps in every pass, finds the want-th largest.
 //  - count:  number of products >= a threshold and their sum.
-//  - bisect: the reference's bisection, four of its rounds per launch: the
-//    thresholds that four rounds can visit form a binary tree of 15 nodes, one
+//  - bisect: the reference's bisection, ten of its rounds per launch: the
+//    thresholds that ten rounds can visit form a binary tree of 1023 nodes, one
 //    walk over the products counts all of them, and the path actually taken is
 //    followed afterwards.
 //
@@ -24,7 +24,7 @@
 // are one launch.
 // Whole calls, norm maps and the multiply behind them included: 5024 x 4128 x 3168 at
 // tile 32 to a kept fraction 667 -> 138 us, the reference's tuned 2048^3 (8 of at most
-// 20 rounds) 381 -> 93 us.
+// 20 rounds) 381 -> 85 us.
 #include "gemm_device.h"
 #include "reduce_device.h"
 
@@ -36,12 +36,15 @@ constexpr int TAU_MAXB = 256;               // one workgroup per CU at most: eve
 constexpr int TAU_JB_COUNT = 16;            // output columns whose products share one load of nA
 constexpr int TAU_JB_TREE = 4;              // (where a product is much work: more waves, and code that is fetched sooner)
 constexpr int TAU_COPIES = 2;               // global copies of a histogram: workgroups that add to one copy queue on its busy bins
-constexpr int TAU_NODES = 15;               // thresholds of four rounds
+constexpr int TREE_LEAVES = 1 << TREE_ROUNDS;
+constexpr int TREE_COPIES = 4;              // global copies of the leaves' counts
 constexpr int64_t TAU_SMALL_MAX = 24 * TAU_NTH;   // products that one workgroup holds
 
 struct TauTune {
     double norm, up, down, rate;
-    int rounds, done;
+    int done;
+    unsigned int call;                      // whose bisection this is
+    int rounds, pad_;
 };
 
 struct TauWorkspace {
@@ -51,7 +54,8 @@ struct TauWorkspace {
     unsigned int pad_;
     unsigned long long zeros;               // products that are not positive
     unsigned long long hist[3][TAU_COPIES][2048];   // one per pass: cleared together, beforehand
-    unsigned long long part[TAU_MAXB][16];  // per workgroup: counts of a pass, or {count, bits of the sum}
+    unsigned long long leaf[TREE_COPIES][TREE_LEAVES];
+    unsigned long long part[TAU_MAXB][2];   // per workgroup: {count, bits of the sum}
 };
 
 size_t tau_workspace_bytes() { return sizeof(TauWorkspace); }
@@ -194,7 +198,7 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_hist(const float *__restrict__ 
 // Round 0 of the bisection measures at tau = 0 and moves to the mean product (tool.cu:445-468).
 __device__ __forceinline__ TauTune first_round(unsigned long long cnt, double sum, unsigned long long total, double expected, double tol,
                                                int max_rounds) {
-    TauTune t;
+    TauTune t = {};
     t.rate = (double)((float)cnt / (float)total);
     t.norm = t.up = t.down = 0.0;
     t.done = fabs(t.rate - expected) < tol;
@@ -204,12 +208,24 @@ __device__ __forceinline__ TauTune first_round(unsigned long long cnt, double su
     return t;
 }
 
+// The state of the bisection passes from launch to launch, and from call to call on whatever stream: stored where every
+// XCD sees it, so that nothing of it is written back after the result has been published.
+__device__ __forceinline__ void store_tune(TauWorkspace *ws, const TauTune &t) {
+    static_assert(sizeof(TauTune) % 8 == 0, "the state is whole 64-bit words");
+    struct Words {
+        unsigned long long w[sizeof(TauTune) / 8];
+    };
+    const Words words = __builtin_bit_cast(Words, t);
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(TauTune) / 8; i++) agent_store(reinterpret_cast<unsigned long long *>(&ws->tune) + i, words.w[i]);
+}
+
 // The two numbers that a round of the bisection starts from (tool.cu:448-463), and with `tune` its
 // first round: products with (double)p >= thr and the double sum of all products.  Sums of a
 // workgroup and of the whole are added in a fixed order: the same norm maps give the same sum.
 __global__ __launch_bounds__(TAU_NTH) void k_tau_count(const float *__restrict__ nA, const float *__restrict__ nBt, int nbM,
                                                        int nbK, int nbN, double thr, unsigned long long total, int tune,
-                                                       double expected, double tol, int max_rounds,
+                                                       double expected, double tol, int max_rounds, unsigned int call, int last,
                                                        TauWorkspace *__restrict__ ws, TauCounts *__restrict__ host_out,
                                                        TauResult *__restrict__ host_tune, unsigned long long *__restrict__ host_seq,
                                                        unsigned long long seq) {
@@ -247,10 +263,11 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_count(const float *__restrict__
     tc.sum = sum;
     if (!tune) publish_result(host_out, tc, host_seq, seq);
     if (tune) {
-        const TauTune t = first_round(cnt, sum, total, expected, tol, max_rounds);
-        ws->tune = t;
-        TauResult r = {t.norm, t.rate, t.done};
-        *host_tune = r;
+        TauTune t = first_round(cnt, sum, total, expected, tol, max_rounds);
+        t.call = call;
+        store_tune(ws, t);
+        const TauResult r = {t.norm, t.rate, t.done};
+        if (t.done || last) publish_result(host_tune, r, host_seq, seq);
     }
 }
 
@@ -282,80 +299,126 @@ __device__ __forceinline__ float fp32_threshold(double thr) {
 // What a lane without a product holds: no threshold keeps it.
 constexpr float NO_PRODUCT = __builtin_nanf("");
 
-// Four rounds of the bisection.  Node n of the tree (heap order, node 1 = the round to come) is the
+// TREE_ROUNDS rounds of the bisection.  Node n of the tree (heap order, node 1 = the round to come) is the
 // threshold after the answers that n's bits below the leading one spell, most significant first:
-// 1 = the kept rate was above the target.
+// 1 = the kept rate was above the target.  A product is looked up among the thresholds as in a search tree, one
+// level per round, and counted in the leaf where it ends: node by node the products that it keeps are then those of
+// the leaves from its rank up.  The thresholds of a tree are in order by themselves unless the mean is negative or
+// no number (uploaded norm maps), and are ranked one by one then.
+// What bounds it: round trips past the L2 -- the state, the norms, the counts, the ticket, the counts again -- and, from
+// 1e7 products on, the look-up's ten LDS reads.  Whole calls, four rounds a launch, each product compared with all of 15
+// thresholds, and a wait for the stream -> this (rounds 9 | 20): 64000 products 40 | 60 -> 32 | 42, 2.6e5 41 | 63 -> 32 | 43,
+// 2.0e6 57 | 100 -> 40 | 56, 1.7e7 (10 rounds) 165 | 252 -> 71 | 113.
 __global__ __launch_bounds__(TAU_NTH) void k_tau_tree(const float *__restrict__ nA, const float *__restrict__ nBt, int nbM,
                                                       int nbK, int nbN, unsigned long long total, double expected, double tol,
-                                                      int max_rounds, TauWorkspace *__restrict__ ws,
-                                                      TauResult *__restrict__ host_tune) {
-    if (ws->tune.done) return;
-    __shared__ unsigned long long s_tot[TAU_NW][16];
+                                                      int max_rounds, unsigned int call, int last, TauWorkspace *__restrict__ ws,
+                                                      TauResult *__restrict__ host_tune, unsigned long long *__restrict__ host_seq,
+                                                      unsigned long long seq) {
+    // a launch behind the one that ended the bisection has nothing to do, and by now the workspace may be another
+    // call's, on another stream: what tells is one word
+    const unsigned long long state = agent_load(reinterpret_cast<const unsigned long long *>(&ws->tune.done));
+    if ((unsigned int)state != 0u || (unsigned int)(state >> 32) != call) return;
+    constexpr int COPIES = 4;
+    __shared__ float s_heap[TREE_LEAVES];
+    __shared__ float s_sorted[TREE_LEAVES];
+    __shared__ unsigned int s_leaf[TREE_LEAVES * COPIES];
+    __shared__ unsigned long long s_kept[TREE_LEAVES];
+    __shared__ unsigned long long s_sum[TAU_NW];
+    __shared__ int s_unsorted;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    float node_thr;
+    // thread n: node n and its rank among the thresholds, 1 to TREE_LEAVES - 1
+    static_assert(TREE_LEAVES == TAU_NTH, "a thread per node");
+    const int n = threadIdx.x;
+    const TauTune start = ws->tune;
+    float own;
     {
-        TauTune t = ws->tune;
-        const int n = (lane & 15) == 0 ? 1 : (lane & 15);
-        for (int bit = 30 - __builtin_clz(n); bit >= 0; bit--) bisect_step(t, (n >> bit) & 1);
-        node_thr = fp32_threshold(t.norm);
+        TauTune t = start;
+        for (int bit = 30 - __builtin_clz(n ? n : 1); bit >= 0; bit--) bisect_step(t, (n >> bit) & 1);
+        own = fp32_threshold(t.norm);
     }
-    float thr[TAU_NODES];
-    unsigned long long cnt[TAU_NODES];
-#pragma unroll
-    for (int n = 0; n < TAU_NODES; n++) {
-        thr[n] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, node_thr), n + 1));
-        cnt[n] = 0;
+    const int depth = 31 - __builtin_clz(n ? n : 1);
+    int rank = n ? (2 * (n - (1 << depth)) + 1) << (TREE_ROUNDS - 1 - depth) : 0;
+    if (n == 0) {
+        own = -__builtin_inff();
+        s_unsorted = 0;
     }
-    for_products<TAU_JB_TREE>(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
-        const float q = live ? p : NO_PRODUCT;
+    s_sorted[rank] = own;
 #pragma unroll
-        for (int n = 0; n < TAU_NODES; n++) cnt[n] += __builtin_popcountll(__ballot(q >= thr[n]));
-    });
-    // workgroup totals: a wave's counts (uniform) by lane 0, then one thread per node
-#pragma unroll
-    for (int n = 0; n < TAU_NODES; n++)
-        if (lane == 0) s_tot[wave][n + 1] = cnt[n];
+    for (int c = 0; c < COPIES; c++) s_leaf[n * COPIES + c] = 0;
     __syncthreads();
-    if (threadIdx.x >= 1 && threadIdx.x < 16) {
+    if (n && !(s_sorted[n - 1] <= s_sorted[n])) s_unsorted = 1;
+    __syncthreads();
+    if (s_unsorted) {                                             // (a threshold that is no number keeps nothing: last)
+        const bool nan = own != own;
+        int r = 0;
+        for (int m = 1; m < TREE_LEAVES; m++) {
+            const int at = 31 - __builtin_clz(m);
+            const float o = s_sorted[(2 * (m - (1 << at)) + 1) << (TREE_ROUNDS - 1 - at)];
+            r += nan ? (o == o || m <= n) : (o < own || (o == own && m <= n));
+        }
+        if (n) rank = r;
+        __syncthreads();
+        s_sorted[rank] = own;
+        __syncthreads();
+    }
+    s_heap[n] = n ? s_sorted[(2 * (n - (1 << depth)) + 1) << (TREE_ROUNDS - 1 - depth)] : 0.0f;
+    __syncthreads();
+    for_products<TAU_JB_TREE>(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
+        int at = 1;
+#pragma unroll
+        for (int level = 0; level < TREE_ROUNDS; level++) at = 2 * at + (p >= s_heap[at] ? 1 : 0);
+        if (live && at != TREE_LEAVES) atomicAdd(&s_leaf[(at - TREE_LEAVES) * COPIES + (lane & (COPIES - 1))], 1u);
+    });
+    __syncthreads();
+    {
         unsigned long long c = 0;
-        for (int w = 0; w < TAU_NW; w++) c += s_tot[w][threadIdx.x];
-        agent_store(&ws->part[blockIdx.x][threadIdx.x], c);
+#pragma unroll
+        for (int r = 0; r < COPIES; r++) c += s_leaf[n * COPIES + r];
+        if (c) atomicAdd(&ws->leaf[blockIdx.x % TREE_COPIES][n], c);
     }
     if (!last_workgroup(&ws->ticket)) return;
-    {
-        const int n = threadIdx.x & 15;
-        unsigned long long c = 0;
-        if (n)
-            for (unsigned b = threadIdx.x >> 4; b < gridDim.x; b += TAU_NTH / 16) c += agent_load(&ws->part[b][n]);
-        c += __shfl_xor(c, 16, 64);
-        c += __shfl_xor(c, 32, 64);
-        if (lane < 16) s_tot[wave][n] = c;
-    }
-    __syncthreads();
-    if (threadIdx.x >= 64) return;
-    unsigned long long node_cnt = 0;                              // lane n: node n
+    // products in the leaves from each thread's own up
+    unsigned long long part[TREE_COPIES], incl = 0;
 #pragma unroll
-    for (int r = 0; r < TAU_NW; r++) node_cnt += s_tot[r][lane & 15];
-    if (lane < 16) s_tot[0][lane] = node_cnt;
-    __builtin_amdgcn_wave_barrier();
+    for (int r = 0; r < TREE_COPIES; r++) part[r] = agent_load(&ws->leaf[r][TREE_LEAVES - 1 - n]);
+#pragma unroll
+    for (int r = 0; r < TREE_COPIES; r++) {
+        if (part[r]) agent_store(&ws->leaf[r][TREE_LEAVES - 1 - n], 0ull);
+        incl += part[r];
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const unsigned long long o = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += o;
+    }
+    if (lane == 63) s_sum[wave] = incl;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // (the leaves are zero again before the result is published)
+    __syncthreads();
+    for (int w = 0; w < wave; w++) incl += s_sum[w];
+    s_kept[TREE_LEAVES - 1 - n] = incl;
+    __syncthreads();
+    const unsigned long long kept = n ? s_kept[rank] : 0ull;
+    __syncthreads();
+    s_kept[n] = kept;                                             // now by node
+    __syncthreads();
     if (threadIdx.x != 0) return;
-    TauTune t = ws->tune;
-    int n = 1;
-    for (int level = 0; level < 4 && !t.done; level++) {
-        t.rate = (double)((float)s_tot[0][n] / (float)total);
+    TauTune t = start;
+    int node = 1;
+    for (int level = 0; level < TREE_ROUNDS && !t.done; level++) {
+        t.rate = (double)((float)s_kept[node] / (float)total);
         if (fabs(t.rate - expected) < tol) {
             t.done = 1;
             break;
         }
         const bool above = t.rate > expected;
         const bool moved = bisect_step(t, above);
-        n = 2 * n + (above ? 1 : 0);
+        node = 2 * node + (above ? 1 : 0);
         if (++t.rounds >= max_rounds || !moved) t.done = 1;
     }
-    ws->tune = t;
-    TauResult r = {t.norm, t.rate, t.done};
-    *host_tune = r;
+    store_tune(ws, t);
+    const TauResult res = {t.norm, t.rate, t.done};
+    if (t.done || last) publish_result(host_tune, res, host_seq, seq);
 }
 
 // Small problems by one workgroup that holds every product in registers: E per thread, 1024 threads.  All
@@ -519,6 +582,7 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_small_tune(const float *__restr
 __global__ __launch_bounds__(256) void k_tau_clear(TauWorkspace *ws) {
     const int b = blockIdx.x * 256 + threadIdx.x;                 // 8 workgroups per histogram copy
     (&ws->hist[0][0][0])[b] = 0;
+    if (b < TREE_COPIES * TREE_LEAVES) (&ws->leaf[0][0])[b] = 0;
     if (b == 0) {
         ws->ticket = 0;
         ws->zeros = 0;
@@ -566,7 +630,7 @@ hipError_t launch_tau_count(const float *nA, const float *nBt, int64_t nbM, int6
                             void *workspace, TauCounts *host_out, unsigned long long *host_seq, unsigned long long seq, hipStream_t s) {
     TauWorkspace *ws = (TauWorkspace *)workspace;
     k_tau_count<<<tau_grid(nbM, nbK, nbN), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, thr,
-                                                       (unsigned long long)nbM * nbK * nbN, 0, 0.0, 0.0, 0, ws, host_out, nullptr,
+                                                       (unsigned long long)nbM * nbK * nbN, 0, 0.0, 0.0, 0, 0u, 0, ws, host_out, nullptr,
                                                        host_seq, seq);
     return hipGetLastError();
 }
@@ -581,16 +645,17 @@ hipError_t launch_tau_tune_small(const float *nA, const float *nBt, int64_t nbM,
     return hipGetLastError();
 }
 
-hipError_t launch_tau_tune(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double expected,
-                           double tol, int max_rounds, bool first, int passes, void *workspace, TauResult *host_out, hipStream_t s) {
+hipError_t launch_tau_tune(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double expected, double tol,
+                           int max_rounds, bool first, int passes, unsigned int call, void *workspace, TauResult *host_out,
+                           unsigned long long *host_seq, unsigned long long seq, hipStream_t s) {
     TauWorkspace *ws = (TauWorkspace *)workspace;
     const unsigned long long total = (unsigned long long)nbM * nbK * nbN;
     if (first)
         k_tau_count<<<tau_grid(nbM, nbK, nbN), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, 0.0, total, 1, expected, tol,
-                                                           max_rounds, ws, nullptr, host_out, nullptr, 0);
+                                                           max_rounds, call, passes == 0, ws, nullptr, host_out, host_seq, seq);
     for (int p = 0; p < passes; p++)
         k_tau_tree<<<tau_grid(nbM, nbK, nbN, TAU_JB_TREE), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, expected, tol,
-                                                                       max_rounds, ws, host_out);
+                                                                       max_rounds, call, p == passes - 1, ws, host_out, host_seq, seq);
     return hipGetLastError();
 }
 

@@ -696,8 +696,7 @@ static int ensure_results(spamm_ctx *c) {
 // Waits for result `seq`, which the last kernel of the call writes when it has done all else -- its writes to the
 // context's workspaces have arrived, so that the next call may use them from another stream -- a few microseconds
 // sooner than the stream is reported idle.  If the stream ends, or fails, without it, the call has failed.  (A
-// bisection in several launches waits for the stream: what has ended it may have launches behind it that still
-// look at the workspace.)
+// bisection may have a launch behind the one that ended it, which only looks whether it has anything to do.)
 static int wait_result(spamm_ctx *c, unsigned long long seq) {
     for (int i = 0; i < 50000; i++)           // (some 100 us)
         if (__atomic_load_n(&c->results->seq, __ATOMIC_ACQUIRE) == seq) return SPAMM_OK;
@@ -925,16 +924,18 @@ int spamm_tune_bisect(spamm_ctx *c, double expected, double tol, int max_rounds,
         if (achieved_out) *achieved_out = c->results->tune.rate;
         return SPAMM_OK;
     }
-    // four rounds a launch; the reference's 20 rounds are one wait, beyond that the host looks every 20
+    // the reference's 20 rounds are a count and two passes, and one wait; beyond that the host looks every other pass
     // whether they have ended
     c->tauws_clean = false;
-    int left = (max_rounds - 1) / 4 + ((max_rounds - 1) % 4 != 0);
+    const unsigned int call = (unsigned int)(c->seq + 1);
+    int left = (max_rounds - 1) / TREE_ROUNDS + ((max_rounds - 1) % TREE_ROUNDS != 0);
     bool first = true;
     do {
-        const int passes = left < 5 ? left : 5;
-        HIPCHK(c, launch_tau_tune((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, expected, tol,
-                                  max_rounds, first, passes, c->tauws.p, &c->results->tune, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
+        const int passes = left < 2 ? left : 2;
+        const unsigned long long seq = ++c->seq;
+        HIPCHK(c, launch_tau_tune((const float *)c->nA.p, (const float *)c->nBt.p, s.nbM, s.nbK, s.nbN, expected, tol, max_rounds,
+                                  first, passes, call, c->tauws.p, &c->results->tune, &c->results->seq, seq, c->stream));
+        if ((rc = wait_result(c, seq))) return rc;
         left -= passes;
         first = false;
     } while (left > 0 && !c->results->tune.done);

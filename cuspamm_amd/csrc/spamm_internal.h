@@ -164,7 +164,7 @@ struct TauResult {                // of the bisection so far
 };
 size_t tau_workspace_bytes();
 // Results go to *host_out, pinned host memory: valid once *host_seq == seq (the kernel that writes it is the
-// call's last), or, of launch_tau_tune, once the stream has been waited for.
+// last of the call that does anything).
 hipError_t launch_tau_clear(void *workspace, hipStream_t s);          // once after allocation, and after a failed call
 hipError_t launch_tau_select(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN,
                              unsigned long long want, void *workspace, TauState *host_out, unsigned long long *host_seq,
@@ -175,9 +175,12 @@ hipError_t launch_tau_count(const float *nA, const float *nBt, int64_t nbM, int6
 bool tau_tune_small(int64_t nbM, int64_t nbK, int64_t nbN);
 hipError_t launch_tau_tune_small(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double expected, double tol,
                                  int max_rounds, TauResult *host_out, unsigned long long *host_seq, unsigned long long seq, hipStream_t s);
-// the bisection: `first` starts it (its round 0), then 4 rounds per pass until done
-hipError_t launch_tau_tune(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double expected,
-                           double tol, int max_rounds, bool first, int passes, void *workspace, TauResult *host_out, hipStream_t s);
+// the bisection: `first` starts it (its round 0), then TREE_ROUNDS rounds per pass until done.  *host_seq == seq: it is done
+// or the passes are; `call` tells the bisection's launches from those of a later one
+constexpr int TREE_ROUNDS = 10;
+hipError_t launch_tau_tune(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double expected, double tol,
+                           int max_rounds, bool first, int passes, unsigned int call, void *workspace, TauResult *host_out,
+                           unsigned long long *host_seq, unsigned long long seq, hipStream_t s);
 
 hipError_t gemm_init();   // one-time kernel attribute set-up
 hipError_t launch_gemm(const void *packedA, const void *packedB, const GateBuffers &g, int64_t M,

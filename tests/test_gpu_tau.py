@@ -119,7 +119,7 @@ def test_selection_at_the_edges_of_its_work_units(orc, ctx, shape):
 
 @pytest.mark.parametrize("rounds", [1, 2, 4, 5, 6, 9, 20, 21, 22, 45])
 def test_bisection_stops_at_any_round(orc, ctx, rounds):
-    # four rounds per launch, twenty per wait: every remainder of both, on a target that is never met (the kept
+    # several rounds per launch, twenty per wait: remainders of both, on a target that is never met (the kept
     # fractions of 6 products are sixths), so that exactly `rounds` rounds run; sums of these values are exact
     nA, nB = np.array([[1.0, 2.0, 4.0], [0.5, 8.0, 16.0]], np.float32), np.ones((3, 1), np.float32)
     ctx.set_normmaps(nA, nB, 32)
@@ -204,3 +204,23 @@ def test_results_on_one_stream_after_another(orc):
                 assert c.dropped_bound(float("inf")) == pytest.approx(np.sqrt((prods.sum(axis=2) ** 2).sum()), rel=1.5e-11)
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("shape", [(40, 130, 23), (64, 64, 64), (1, 40000, 1), (300, 1, 301)])
+@pytest.mark.parametrize("rounds", [2, 11, 12, 21, 22, 32])
+def test_bisection_by_a_search_tree(orc, ctx, shape, rounds):
+    # ten rounds per launch, twenty per wait, on one stream and then another: remainders of the work units, ties,
+    # zeros, many octaves, and kept fractions at the ends.  Products of small whole numbers (times a power of two): their
+    # sums are exact in any order, so thresholds and fractions are those of the checker bit for bit
+    import torch
+    rng = np.random.default_rng(sum(shape) + rounds)
+    nA = rng.integers(0, 64, size=shape[:2]).astype(np.float32)
+    nB = (2.0 ** rng.integers(-6, 7, size=shape[1:])).astype(np.float32)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for at, expected in enumerate((0.75, 0.2, 0.003, 0.999, 2.0)):
+        ctx.set_stream(streams[at % 2].cuda_stream)
+        ctx.set_normmaps(nA, nB, 32)
+        for tol in (0.01, 1e-7):
+            got, want = ctx.tune_bisect(expected, tol, rounds), orc.tune_bisect(nA, nB, expected, tol, rounds)
+            assert np.float32(got[0]) == np.float32(want[0]) and got[1] == want[1], (expected, tol, got, want)
+    ctx.set_stream(None)

@@ -295,3 +295,14 @@ def test_results_are_published_when_the_workspace_is_at_rest(tmp_path):
                 clears = [i for i, ln in enumerate(block) if ln.startswith("global_store")]
                 assert clears and waits and waits[0] < clears[0], kernel        # (reversed: the last wait comes after the last store)
                 assert not any(ln.startswith((".LBB", "s_cbranch", "s_branch")) for ln in block[:waits[0]]), kernel
+
+
+def test_bisection_state_is_stored_past_the_cache(tmp_path):
+    """The bisection's state is read by the next call, on whatever stream, as soon as the host has seen a result: no
+    kernel of it stores to global memory but past its XCD's cache (sc1)."""
+    text = _isa("kernels_tau.hip", tmp_path)
+    for name in ("k_tau_count", "k_tau_tree"):
+        kernels = re.findall(r"^(_ZN5spamm\d+%s\w+):[^\n]*\n(.*?)^\.Lfunc_end" % name, text, flags=re.S | re.M)
+        assert len(kernels) == 1
+        stores = [ln.strip() for ln in kernels[0][1].splitlines() if re.match(r"\s*(global|flat|buffer|scratch)_store", ln)]
+        assert stores and all("sc1" in ln for ln in stores), (name, stores)
