@@ -1,6 +1,6 @@
-// Stages 2 and 3 in one launch, for outputs that leave the chip half empty.
+// Stages 2 and 3 in one launch, for small and middling outputs.
 //
-// Where C has few macro tiles the gate (k_gate), the schedule (k_order) and the
+// Where C has few macro tiles (up to some 1.5 per CU) the gate (k_gate), the schedule (k_order) and the
 // gated GEMM are each a few microseconds of latency on a mostly idle chip, and the
 // GEMM's 256-wide work units leave most CUs without any.  Here one workgroup owns a
 // unit of U x U elements of C (U = 128 or 64) and does all three for it: it forms the
@@ -15,7 +15,7 @@
 // the same bit for bit whichever kernel runs.
 //
 // What bounds it: a chain of latencies -- norms in, first stages in, one sync per 32 k,
-// results out -- of which units of 128 (16 KiB a stage, two workgroups per CU) make
+// results out -- of which units of 128 (16 KiB a stage, two workgroups per CU, or three) make
 // the k loop shortest and units of 64 spread a small C over more CUs.  Gate, schedule
 // and GEMM as launches of their own -> this kernel, whole multiplies: 256^3 24.6 -> 14.7 us
 // (today, with one launch for both norm-map passes too: 10.7), 1056 x 1568 x 1312 38.2 -> 22.8
@@ -25,7 +25,7 @@
 
 namespace spamm {
 
-template <int B, int U>
+template <int B, int U, int RING>
 struct SmallCfg {
     static constexpr int MT = 256 / B;                       // tiles per macro tile per dimension
     static constexpr int PD = 256 / U;                       // units per macro tile per dimension
@@ -36,7 +36,7 @@ struct SmallCfg {
     static constexpr int TILE_BYTES = B * B * 2;
     static constexpr int OP_BYTES = U * 64;                  // one operand's part of a stage
     static constexpr int STAGE_BYTES = 2 * OP_BYTES;         // 16 or 8 KiB
-    static constexpr int NBUF = U == 128 ? 4 : 6;
+    static constexpr int NBUF = RING;
     static constexpr int CPS = RS / 16;                      // 1 KiB chunks per slot
     static constexpr int CHW = U / 64;                       // chunks per wave per operand per stage (in one slot)
     static constexpr int LPW = 2 * CHW;
@@ -54,11 +54,11 @@ size_t small_lds_bytes_(int stage_bytes, int nbuf, int tt, int64_t nbK) {
     return (size_t)stage_bytes * nbuf + words * 64 * 4 + words * tt * 8 + words * 16 + words * 64 * 2;
 }
 
-template <int B, int U>
-__global__ __launch_bounds__(256, 2) void k_small(const unsigned char *__restrict__ pA, const unsigned char *__restrict__ pB,
-                                                  GateBuffers g, int nbM, int nbK, int nbN, int nMacN, int n_units, int n_xcd,
-                                                  int mode, float tau, int64_t M, int64_t N, float *__restrict__ C) {
-    using H = SmallCfg<B, U>;
+template <int B, int U, int RING>
+__device__ __forceinline__ void small_unit_body(const unsigned char *__restrict__ pA, const unsigned char *__restrict__ pB, const GateBuffers &g,
+                                                int nbM, int nbK, int nbN, int nMacN, int n_units, int n_xcd, int mode, float tau,
+                                                int64_t M, int64_t N, float *__restrict__ C) {
+    using H = SmallCfg<B, U, RING>;
     constexpr int NBUF = H::NBUF, MT = H::MT, TU = H::TU, TT = H::TT, NB = H::NB;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int words = (nbK + 63) >> 6;
@@ -353,6 +353,21 @@ __global__ __launch_bounds__(256, 2) void k_small(const unsigned char *__restric
     store_gate();
 }
 
+template <int B, int U>
+__global__ __launch_bounds__(256, 2) void k_small(const unsigned char *__restrict__ pA, const unsigned char *__restrict__ pB,
+                                                  GateBuffers g, int nbM, int nbK, int nbN, int nMacN, int n_units, int n_xcd,
+                                                  int mode, float tau, int64_t M, int64_t N, float *__restrict__ C) {
+    small_unit_body<B, U, (U == 128 ? 4 : 6)>(pA, pB, g, nbM, nbK, nbN, nMacN, n_units, n_xcd, mode, tau, M, N, C);
+}
+
+// Units of 128 by three workgroups per CU (small_three).
+template <int B>
+__global__ __launch_bounds__(256, 3) void k_small_three(const unsigned char *__restrict__ pA, const unsigned char *__restrict__ pB,
+                                                        GateBuffers g, int nbM, int nbK, int nbN, int nMacN, int n_units, int n_xcd,
+                                                        int mode, float tau, int64_t M, int64_t N, float *__restrict__ C) {
+    small_unit_body<B, 128, 3>(pA, pB, g, nbM, nbK, nbN, nMacN, n_units, n_xcd, mode, tau, M, N, C);
+}
+
 __global__ void k_clear_kept(int64_t *kept) { *kept = 0; }
 
 hipError_t launch_clear_kept(int64_t *kept, hipStream_t s) {
@@ -372,54 +387,102 @@ static int small_unit(int64_t M, int64_t N) {
     return units128 >= 128 ? 128 : 64;
 }
 
-template <int B, int U>
+// More than two units of 128 per CU: a ring of three stages leaves room for a third workgroup on the CU, whose loads and
+// syncs fill the others' waits.  Ring of four, two workgroups -> this, whole multiplies, fp16: 576 units, K = 2048 at tile
+// 32, 10 % kept 42.0 -> 37.4 us, 40 % 54.3 -> 48.5, dense 70.6 -> 63.5; 640 units 45.8 -> 41.0, 60.2 -> 54.5, 75.6 -> 69;
+// 768 units 48.5 -> 44.7, 65.4 -> 58.7, 79.6 -> 75.7; 1024 units, 5 % 47.4 -> 45.2, 40 % 75.7 -> 78.7; 484 units (two per
+// CU hold them all) 29.3 -> 30.0, 34.3 -> 34.3, 45.2 -> 44.3.  A list too long for three in a CU's LDS keeps the ring of four.
+static bool small_three(int64_t units128, int64_t nbK, int tile) {
+    const int tt = tile >= 128 ? 1 : (128 / tile) * (128 / tile);
+    return units128 > 512 && 3 * (small_lds_bytes_(16384, 3, tt, nbK) + 2048) <= 160 * 1024;
+}
+
+template <int B, int U, bool THREE>
+static constexpr auto small_kernel() {
+    if constexpr (THREE) return &k_small_three<B>;
+    else return &k_small<B, U>;
+}
+
+template <int B, int U, bool THREE>
+static size_t small_lds(int64_t nbK) {
+    using H = SmallCfg<B, U, (THREE ? 3 : (U == 128 ? 4 : 6))>;
+    return small_lds_bytes_(H::STAGE_BYTES, H::NBUF, H::TT, nbK);
+}
+
+template <int B, int U, bool THREE>
 static hipError_t launch_small_(const void *pA, const void *pB, const GateBuffers &g, int64_t M, int64_t K, int64_t N,
                                 int mode, float tau, float *C, int n_xcd, hipStream_t s) {
-    using H = SmallCfg<B, U>;
+    using H = SmallCfg<B, U, 4>;
     const int nbM = (int)(M / B), nbK = (int)(K / B), nbN = (int)(N / B);
     const int nMacM = (nbM + H::MT - 1) / H::MT, nMacN = (nbN + H::MT - 1) / H::MT;
     const int n_units = nMacM * nMacN * H::PD * H::PD;
     const unsigned grid = (unsigned)((n_units + n_xcd - 1) / n_xcd * n_xcd);
-    k_small<B, U><<<grid, 256, small_lds_bytes_(H::STAGE_BYTES, H::NBUF, H::TT, nbK), s>>>(
+    small_kernel<B, U, THREE>()<<<grid, 256, small_lds<B, U, THREE>(nbK), s>>>(
         (const unsigned char *)pA, (const unsigned char *)pB, g, nbM, nbK, nbN, nMacN, n_units, n_xcd, mode, tau, M, N, C);
     return hipGetLastError();
 }
 
-template <int B, int U>
+template <int B, int U, bool THREE>
 static hipError_t small_attr() {
-    using H = SmallCfg<B, U>;
-    return hipFuncSetAttribute(reinterpret_cast<const void *>(&k_small<B, U>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)small_lds_bytes_(H::STAGE_BYTES, H::NBUF, H::TT, SMALL_MAX_NBK));
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(small_kernel<B, U, THREE>()), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)small_lds<B, U, THREE>(SMALL_MAX_NBK));
+}
+
+template <int B>
+static hipError_t small_attrs() {
+    hipError_t e;
+    if ((e = small_attr<B, 128, true>()) != hipSuccess || (e = small_attr<B, 128, false>()) != hipSuccess) return e;
+    return small_attr<B, 64, false>();
 }
 
 hipError_t small_init() {
     hipError_t e;
-    if ((e = small_attr<32, 128>()) != hipSuccess || (e = small_attr<32, 64>()) != hipSuccess) return e;
-    if ((e = small_attr<64, 128>()) != hipSuccess || (e = small_attr<64, 64>()) != hipSuccess) return e;
-    if ((e = small_attr<128, 128>()) != hipSuccess) return e;
-    return small_attr<128, 64>();
+    if ((e = small_attrs<32>()) != hipSuccess || (e = small_attrs<64>()) != hipSuccess) return e;
+    return small_attrs<128>();
 }
 
-// Whole multiplies, gate and GEMM apart -> this kernel, by units of 128 in C (tile 64 unless said): 484 units, dense
-// 88.3 -> 71.2 us, 10 % kept 59.2 -> 44.1; 512 units, dense 118 -> 101; 576 units, dense 94.4 -> 95.1, 10 % at tile 32
-// 63.9 -> 50.1; 1024 units, dense 156 -> 180, 40 % 115 -> 121, 10 % 84.4 -> 77.8.  Up to 512 units run at once; beyond
-// that the 256-wide units' thriftier staging wins the more is kept, and how much that is the host does not know, but
-// for tau <= 0 (everything).
-bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau) {
-    const int64_t units128 = ((M + 127) / 128) * ((N + 127) / 128);
-    return units128 <= (tau > 0.0f ? 640 : 512) && K / tile <= SMALL_MAX_NBK;
+// Whole multiplies on fp16 operands, gate, schedule and GEMM apart -> this kernel, by units of 128 in C; "m" is the number of
+// macro tiles (four units each), of which k_gemm runs 256 at a time.
+//
+// tau > 0, at most 6 units per CU.  K = 4096 at tile 64, 5 % | 40 % kept: 768 units 66 -> 51 | 94 -> 82 us; 1000 units
+// 69 -> 61 | 115 -> 113; 1296 units 78 -> 69 | 145 -> 135.  K = 2048 at tile 32: 54.6 -> 40.2 | 77 -> 58.7, 62 -> 51.5 |
+// 84.8 -> 80.5, 68.6 -> 57.6 | 93.5 -> 92.4.  K = 8192 at tile 128, 25 % | 50 %: 1088 units 171 -> 144 | 246 -> 221, 1444
+// units 191 -> 174 | 287 -> 266.  Beyond: 1600 units, K = 5120, 10 % of a band 107.8 -> 112, 25 % 160 -> 146; 1936 units, K =
+// 2048, 25 % 99 -> 119; 4096 units 243 -> 265.  What decides is how many macro tiles compute, which the host does not know:
+// the fewer, the more CUs k_gemm leaves idle.  Where its one round is all but full (833 to 1024 units) and much is kept, its
+// thriftier staging wins with long K: 1024 units, 5 % | 40 %, K = 2048 62 -> 45 | 83 -> 79, K = 4096 73 -> 61 | 105 -> 109,
+// K = 8192 (2 % | 25 %) 91 -> 80 | 141 -> 137, K = 16384 151 -> 133 | 224 -> 250.
+//
+// tau <= 0, everything is kept and the rounds are known.  Up to 512 units 88.3 -> 71.2 us (484), 118 -> 101 (512).  With m =
+// 160 to 192 a round is a third empty: 640 units, K = 2048 | 4096 82 -> 69 | 139 -> 123; 704 units 80 -> 70 | 133 -> 123; 768
+// units 82.6 -> 75.7 | 140 -> 132; but 600 units 70 -> 67 | 108 -> 119 and 841 units 81 -> 90 | 135 -> 161.  With m = 257 to
+// 324 a second round is mostly empty: 1088 units 129 -> 104 | 220 -> 184, 1296 units 136 -> 120 | 233 -> 220; 1444 units
+// 132 -> 126 | 228 -> 227 and, K = 8192, 412 -> 436.
+// Gate and multiply called apart (`stages`) form mask and list twice, which k_gate's list spares: 5024 x 4128 x 3168 at tile
+// 32, 10 % kept, 58 us of k_gate, k_order and k_gemm against 68 by two of these launches.
+bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau, bool stages) {
+    const int64_t units128 = ((M + 127) / 128) * ((N + 127) / 128), m = ((M + 255) / 256) * ((N + 255) / 256);
+    if (K / tile > SMALL_MAX_NBK) return false;
+    if (units128 <= 512) return true;
+    if (stages) return tau > 0.0f && units128 <= 640;
+    if (tau > 0.0f) return units128 <= 1536 && (units128 <= 832 || units128 > 1024 || K <= 8192);
+    return (m >= 160 && m <= 192) || (m >= 257 && m <= 324);
+}
+
+template <int B>
+static hipError_t launch_small_(const void *pA, const void *pB, const GateBuffers &g, int64_t M, int64_t K, int64_t N,
+                                int mode, float tau, float *C, int n_xcd, hipStream_t s) {
+    if (small_unit(M, N) != 128) return launch_small_<B, 64, false>(pA, pB, g, M, K, N, mode, tau, C, n_xcd, s);
+    if (small_three(((M + 127) / 128) * ((N + 127) / 128), K / B, B)) return launch_small_<B, 128, true>(pA, pB, g, M, K, N, mode, tau, C, n_xcd, s);
+    return launch_small_<B, 128, false>(pA, pB, g, M, K, N, mode, tau, C, n_xcd, s);
 }
 
 hipError_t launch_small(const void *packedA, const void *packedB, const GateBuffers &g, int64_t M, int64_t K, int64_t N,
                         int tile, int mode, float tau, float *C, int n_xcd, hipStream_t s) {
-    const bool wide = small_unit(M, N) == 128;
     switch (tile) {
-        case 32: return wide ? launch_small_<32, 128>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s)
-                             : launch_small_<32, 64>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s);
-        case 64: return wide ? launch_small_<64, 128>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s)
-                             : launch_small_<64, 64>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s);
-        case 128: return wide ? launch_small_<128, 128>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s)
-                              : launch_small_<128, 64>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s);
+        case 32: return launch_small_<32>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s);
+        case 64: return launch_small_<64>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s);
+        case 128: return launch_small_<128>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s);
         default: return hipErrorInvalidValue;
     }
 }

@@ -463,9 +463,9 @@ static int build_lists(spamm_ctx *c, float tau) {
 }
 
 // Small outputs are gated and multiplied by a kernel of their own (kernels_small.hip); a caller who fixes
-// the work unit or the gate's chunks gets the gate and the GEMM.
-static bool is_small(const spamm_ctx *c, float tau) {
-    return c->gemm_shape == 0 && c->gate_chunk_cap == 0 && small_fits(c->M, c->K, c->N, c->tile, tau);
+// the work unit or the gate's chunks gets the gate and the GEMM.  `stages`: called apart.
+static bool is_small(const spamm_ctx *c, float tau, bool stages) {
+    return c->gemm_shape == 0 && c->gate_chunk_cap == 0 && small_fits(c->M, c->K, c->N, c->tile, tau, stages);
 }
 
 // Its gate, its multiply (dC), or both.  kept_clear: a norm-map pass of this call has cleared the kept total.
@@ -494,7 +494,7 @@ int spamm_gate(spamm_ctx *c, float tau) {
     int rc = set_device(c);
     if (rc) return rc;
     if (c->timing && !c->ev_a) HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
-    if (is_small(c, tau)) rc = run_small(c, SMALL_GATE, tau, false, nullptr);
+    if (is_small(c, tau, true)) rc = run_small(c, SMALL_GATE, tau, false, nullptr);
     else rc = build_lists(c, tau);
     if (rc) return rc;
     if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[3], c->stream)); c->ev_gate = true; }
@@ -511,7 +511,7 @@ int spamm_gemm_gated(spamm_ctx *c, float *dC) {
     if (c->b_pruned && !(c->tau > 0.0f)) return SPAMM_ESTATE;               // B's copy lacks its zero tiles
     int rc = set_device(c);
     if (rc) return rc;
-    const bool small = is_small(c, c->tau);
+    const bool small = is_small(c, c->tau, true);
     if (!small && !c->have_lists && (rc = build_lists(c, c->tau))) return rc;    // (the work unit was fixed after a small gate)
     if (c->timing && !c->ev_gate) HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
     if (small) {
@@ -605,7 +605,7 @@ static int multiply_any(spamm_ctx *c, const spamm_params *p, const void *dA, con
         HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
         c->ev_a = true;
     }
-    if (is_small(c, p->tau)) {
+    if (is_small(c, p->tau, false)) {
         // one launch for both stages (the gate's interval is empty)
         if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[3], c->stream)); c->ev_gate = true; }
         if ((rc = run_small(c, SMALL_GATE | SMALL_MULTIPLY, p->tau, !(reuse_a && reuse_b), dC))) return rc;

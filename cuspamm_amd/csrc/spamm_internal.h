@@ -193,7 +193,7 @@ hipError_t launch_gemm(const void *packedA, const void *packedB, const GateBuffe
 hipError_t launch_clear_kept(int64_t *kept, hipStream_t s);
 constexpr int64_t SMALL_MAX_NBK = 2048;      // its k list lives in LDS
 hipError_t small_init();
-bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau);
+bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau, bool stages);
 constexpr int SMALL_GATE = 1, SMALL_MULTIPLY = 2;    // what launch_small does: either or both
 hipError_t launch_small(const void *packedA, const void *packedB, const GateBuffers &g, int64_t M, int64_t K, int64_t N,
                         int tile, int mode, float tau, float *C, int n_xcd, hipStream_t s);

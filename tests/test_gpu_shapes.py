@@ -276,6 +276,15 @@ def test_small_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N, ti
         apart.close()
 
 
+@pytest.mark.parametrize("M,K,N,tile", [(2944, 256, 2912, 32),      # 529 units: the first that no longer fit two to a CU
+                                        (2944, 12320, 2912, 32),    # a list too long for three to a CU
+                                        (4096, 512, 2560, 64), (4352, 320, 4160, 64),               # dense too: 160 and 289 macro tiles
+                                        (4096, 96, 4096, 32), (3968, 384, 4224, 128), (4096, 64, 6144, 64),
+                                        (192, 640, 98304, 64)])     # 1536 units, the most
+def test_middling_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N, tile):
+    test_small_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N, tile)
+
+
 def test_schedule_of_the_longest_lists_on_one_xcd(ctx):
     """One XCD takes every super tile of a band, and the lengths dealt to it so far are part of the key it is chosen by:
     lists of 65535 k tiles bring that sum to 2^28 - 1 before the last super tile is dealt (times 8, plus the XCD's number:

@@ -271,6 +271,19 @@ def test_small_output_kernel_keeps_the_same_contracts(tmp_path):
         assert not any(mn.startswith("scratch_") for mn in mns), name
 
 
+def test_three_small_units_per_cu_keep_the_same_contracts(tmp_path):
+    # the ring of three: no other vector-memory instruction between its loads, no scratch
+    text = _isa("kernels_small.hip", tmp_path)
+    kernels = re.findall(r"^(_ZN5spamm13k_small_threeILi\d+EEE\w+):[^\n]*\n(.*?)s_endpgm", text, flags=re.S | re.M)
+    assert len(kernels) == 3
+    for name, body in kernels:
+        mns = [mn for mn, _, _ in _instructions(body)]
+        dma = [i for i, mn in enumerate(mns) if mn == "global_load_lds_dwordx4"]
+        assert len(dma) >= 12, name
+        memory = {mn for mn in mns[dma[0]:dma[-1] + 1] if mn.startswith(("global_", "flat_", "buffer_", "scratch_"))}
+        assert memory == {"global_load_lds_dwordx4"} and not any(mn.startswith("scratch_") for mn in mns), name
+
+
 def test_results_are_published_when_the_workspace_is_at_rest(tmp_path):
     """The host goes on when it sees a result's sequence number and may use the workspace at once, from another stream:
     behind a publishing kernel's last barrier no wave stores anything but the result itself (to host memory, in system
