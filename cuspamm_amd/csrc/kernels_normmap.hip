@@ -326,13 +326,11 @@ template <int B, int ROLE, int SW, bool IN16, int PH = 1, int NWV = 4>
 __global__ __launch_bounds__(64 * NWV, 1) void k_normmap(
     const void *__restrict__ Xv, int64_t ld, int64_t cols, int64_t nbr, int64_t nbc, int64_t nstrip, uint4 *__restrict__ packed,
     float *__restrict__ nm, float *__restrict__ nmT, uint4 *__restrict__ packed2, float *__restrict__ nm2,
-    const float *__restrict__ rowmax, float tau_skip, int64_t *__restrict__ kept) {
+    const float *__restrict__ rowmax, float tau_skip) {
     using L = NormCfg<B, SW, PH>;
     __shared__ __attribute__((aligned(16))) unsigned char s_pack[L::TPP * L::TS];
     __shared__ float s_chunk[L::TPP * L::CH];
     __shared__ int s_skip[L::TPP];
-    // (the multiply's kept-product total, which k_small adds to: cleared by the passes that run before it)
-    if (blockIdx.x == 0 && threadIdx.x == 0) *kept = 0;
     normmap_strip<B, ROLE, SW, IN16, PH, NWV>(Xv, ld, cols, nbr, nbc, nstrip, packed, nm, nmT, packed2, nm2, rowmax, tau_skip,
                                               blockIdx.x, s_pack, s_chunk, s_skip);
 }
@@ -345,12 +343,11 @@ __global__ __launch_bounds__(64 * NWV) void k_normmap_pair(const void *__restric
                                                            int64_t nbK, int64_t nbN, unsigned n_b, int64_t strips_a, int64_t strips_b,
                                                            uint4 *__restrict__ packedA, uint4 *__restrict__ packedB,
                                                            float *__restrict__ nmA, float *__restrict__ nmB,
-                                                           float *__restrict__ nmBt, float tau_skip, int64_t *__restrict__ kept) {
+                                                           float *__restrict__ nmBt, float tau_skip) {
     using L = NormCfg<B, SW, PH>;
     __shared__ __attribute__((aligned(16))) unsigned char s_pack[L::TPP * L::TS];
     __shared__ float s_chunk[L::TPP * L::CH];
     __shared__ int s_skip[L::TPP];
-    if (blockIdx.x == 0 && threadIdx.x == 0) *kept = 0;
     if (blockIdx.x < n_b)
         normmap_strip<B, 1, SW, IN16, PH, NWV>(Bm, nbN * B, nbN * B, nbK, nbN, strips_b, packedB, nmB, nmBt, nullptr, nullptr,
                                                nullptr, tau_skip, blockIdx.x, s_pack, s_chunk, s_skip);
@@ -446,13 +443,13 @@ constexpr unsigned NARROW_STRIPS = 512;     // of 256 columns, in a launch: two 
 
 template <int ROLE, bool IN16>
 static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int tile, void *packed, float *nm,
-                                 float *nmT, int64_t *kept, hipStream_t s, void *packed2 = nullptr, float *nm2 = nullptr,
+                                 float *nmT, hipStream_t s, void *packed2 = nullptr, float *nm2 = nullptr,
                                  const float *rowmax = nullptr, float tau_skip = 0.0f) {
     const int64_t nbr = rows / tile, nbc = cols / tile;
     const auto strips = [&](int64_t sw) { return (unsigned)(nbr * ((cols + sw - 1) / sw)); };
 #define SPAMM_NORMMAP(T, SW, PH, NWV)                                                                                           \
     k_normmap<T, ROLE, SW, IN16, PH, NWV><<<strips(SW), 64 * NWV, 0, s>>>(X, cols, cols, nbr, nbc, (cols + SW - 1) / SW, (uint4 *)packed, \
-                                                                          nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip, kept)
+                                                                          nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip)
     // strip widths and waves: one 8-row group per lane, at most ~42 KiB of LDS and so three workgroups or more per CU.
     // fp16 input: 256 columns, two rows per load (512 in phases before: tile 64 1024^2, both passes, 6.2 -> 4.1 us, 4096^2
     // 28.4 -> 26.3, 16384^2 A = B 303 -> 291; tile 32 2048^2 8.0 -> 7.3, 8192^2 tau-aware 93 -> 87).
@@ -498,18 +495,18 @@ static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int 
 }
 
 hipError_t launch_normmap_a(const void *X, bool in16, int64_t rows, int64_t cols, int tile, void *packed,
-                            float *nm, const float *rowmax, float tau_skip, int64_t *kept, hipStream_t s) {
-    return in16 ? launch_normmap<0, true>(X, rows, cols, tile, packed, nm, nullptr, kept, s, nullptr, nullptr, rowmax, tau_skip)
-                : launch_normmap<0, false>(X, rows, cols, tile, packed, nm, nullptr, kept, s, nullptr, nullptr, rowmax, tau_skip);
+                            float *nm, const float *rowmax, float tau_skip, hipStream_t s) {
+    return in16 ? launch_normmap<0, true>(X, rows, cols, tile, packed, nm, nullptr, s, nullptr, nullptr, rowmax, tau_skip)
+                : launch_normmap<0, false>(X, rows, cols, tile, packed, nm, nullptr, s, nullptr, nullptr, rowmax, tau_skip);
 }
 
 template <int B, int SW, int PH, int NWV, bool IN16>
 static void launch_pair(const void *A, const void *Bm, int64_t nbM, int64_t nbK, int64_t nbN, void *packedA, void *packedB,
-                        float *nmA, float *nmB, float *nmBt, float tau_skip, int64_t *kept, hipStream_t s) {
+                        float *nmA, float *nmB, float *nmBt, float tau_skip, hipStream_t s) {
     const int64_t strips_a = (nbK * B + SW - 1) / SW, strips_b = (nbN * B + SW - 1) / SW;
     const unsigned n_b = (unsigned)(nbK * strips_b), n_a = (unsigned)(nbM * strips_a);
     k_normmap_pair<B, SW, IN16, PH, NWV><<<n_a + n_b, 64 * NWV, 0, s>>>(A, Bm, nbM, nbK, nbN, n_b, strips_a, strips_b, (uint4 *)packedA,
-                                                                        (uint4 *)packedB, nmA, nmB, nmBt, tau_skip, kept);
+                                                                        (uint4 *)packedB, nmA, nmB, nmBt, tau_skip);
 }
 
 // Where the two passes are worth running as one, by the strips of both operands, counted as tile rows of 1 KiB (256
@@ -524,10 +521,10 @@ bool normmap_pair_fits(bool in16, bool tau_aware, int64_t M, int64_t K, int64_t 
 }
 
 hipError_t launch_normmap_pair(const void *A, const void *Bm, bool in16, int64_t M, int64_t K, int64_t N, int tile, void *packedA,
-                               float *nmA, void *packedB, float *nmB, float *nmBt, float tau_skip, int64_t *kept, hipStream_t s) {
+                               float *nmA, void *packedB, float *nmB, float *nmBt, float tau_skip, hipStream_t s) {
     const int64_t nbM = M / tile, nbK = K / tile, nbN = N / tile;
 #define SPAMM_PAIR(T, SW, NWV, IN16) \
-    launch_pair<T, SW, 1, NWV, IN16>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, kept, s)
+    launch_pair<T, SW, 1, NWV, IN16>(A, Bm, nbM, nbK, nbN, packedA, packedB, nmA, nmB, nmBt, tau_skip, s)
     // (strips as the passes of their own have them)
     switch (tile) {
         case 32:
@@ -555,15 +552,15 @@ hipError_t launch_rowmax(const float *nB, int64_t nbK, int64_t nbN, float *rowma
 }
 
 hipError_t launch_normmap_ab(const void *X, bool in16, int64_t n, int tile, void *packedA, float *nmA,
-                             void *packedB, float *nmB, float *nmBt, float tau_skip, int64_t *kept, hipStream_t s) {
-    return in16 ? launch_normmap<2, true>(X, n, n, tile, packedA, nmA, nmBt, kept, s, packedB, nmB, nullptr, tau_skip)
-                : launch_normmap<2, false>(X, n, n, tile, packedA, nmA, nmBt, kept, s, packedB, nmB, nullptr, tau_skip);
+                             void *packedB, float *nmB, float *nmBt, float tau_skip, hipStream_t s) {
+    return in16 ? launch_normmap<2, true>(X, n, n, tile, packedA, nmA, nmBt, s, packedB, nmB, nullptr, tau_skip)
+                : launch_normmap<2, false>(X, n, n, tile, packedA, nmA, nmBt, s, packedB, nmB, nullptr, tau_skip);
 }
 
 hipError_t launch_normmap_b(const void *X, bool in16, int64_t rows, int64_t cols, int tile, void *packed,
-                            float *nm, float *nmT, float tau_skip, int64_t *kept, hipStream_t s) {
-    return in16 ? launch_normmap<1, true>(X, rows, cols, tile, packed, nm, nmT, kept, s, nullptr, nullptr, nullptr, tau_skip)
-                : launch_normmap<1, false>(X, rows, cols, tile, packed, nm, nmT, kept, s, nullptr, nullptr, nullptr, tau_skip);
+                            float *nm, float *nmT, float tau_skip, hipStream_t s) {
+    return in16 ? launch_normmap<1, true>(X, rows, cols, tile, packed, nm, nmT, s, nullptr, nullptr, nullptr, tau_skip)
+                : launch_normmap<1, false>(X, rows, cols, tile, packed, nm, nmT, s, nullptr, nullptr, nullptr, tau_skip);
 }
 
 hipError_t launch_unpack(const void *packed, int64_t rows, int64_t cols, int tile, int role,

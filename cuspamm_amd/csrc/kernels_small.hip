@@ -82,21 +82,24 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
 
     // ---- gate: a wave takes 64 k at a time, lane = k, and holds the norms of the macro tile's rows and
     // columns (loads unconditional, from clamped addresses)
+    const bool multiply = (mode & SMALL_MULTIPLY) != 0;        // (the gate alone needs no list, and the unit's norms only)
     const bool interior = (mi + 1) * MT <= nbM && (mj + 1) * MT <= nbN;
     for (int w = wave; w < words; w += 4) {
         const int k = w * 64 + lane, kc = k < nbK ? k : nbK - 1;
         const bool live = k < nbK;
-        float a[MT], b[MT], au[TU], bu[TU];
-#pragma unroll
-        for (int x = 0; x < MT; x++) {
-            const int i = mi * MT + x, j = mj * MT + x;
-            a[x] = g.nA[(int64_t)(i < nbM ? i : nbM - 1) * nbK + kc];
-            b[x] = g.nBt[(int64_t)(j < nbN ? j : nbN - 1) * nbK + kc];
-        }
+        float a[MT] = {}, b[MT] = {}, au[TU], bu[TU];
 #pragma unroll
         for (int x = 0; x < TU; x++) {
             au[x] = g.nA[(int64_t)(ti0 + x < nbM ? ti0 + x : nbM - 1) * nbK + kc];
             bu[x] = g.nBt[(int64_t)(tj0 + x < nbN ? tj0 + x : nbN - 1) * nbK + kc];
+        }
+        if (multiply) {
+#pragma unroll
+            for (int x = 0; x < MT; x++) {
+                const int i = mi * MT + x, j = mj * MT + x;
+                a[x] = g.nA[(int64_t)(i < nbM ? i : nbM - 1) * nbK + kc];
+                b[x] = g.nBt[(int64_t)(j < nbN ? j : nbN - 1) * nbK + kc];
+            }
         }
         uint32_t ub = 0;
 #pragma unroll
@@ -140,6 +143,33 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
         s_bits[k] = (uint16_t)ub;
     }
     __syncthreads();
+    // What the gate leaves behind (a tile shared by several units is written by the first).  A unit's kept products are
+    // a word of its own: added to one total by atomics they queued up at the kernel's end, where 200 to 1000 units finish
+    // together (1024^3 10 % 15.4 -> 13.7 us whole, 2048^3 dense 33.8 -> 31.5, 1056 x 1568 x 1312 18.6 -> 17.7).
+    auto store_gate = [&]() {
+        if (!(mode & SMALL_GATE)) return;
+        const bool first = (ui * U) % B == 0 && (uj * U) % B == 0;
+        for (int e = first ? threadIdx.x : TT * words; e < TT * words; e += 256) {
+            const int t = e / words, w = e - t * words, i = ti0 + t / TU, j = tj0 + t % TU;
+            if (i < nbM && j < nbN) g.mask[((int64_t)i * nbN + j) * words + w] = s_word[w * TT + t];
+        }
+        if (wave == 0) {
+            int cnt = 0;
+            if (first && lane < TT) {
+                for (int w = 0; w < words; w++) cnt += __builtin_popcountll(s_word[w * TT + lane]);
+                const int i = ti0 + lane / TU, j = tj0 + lane % TU;
+                if (i < nbM && j < nbN) g.counts[(int64_t)i * nbN + j] = cnt;
+            }
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
+            if (lane == 0) g.kept_units[(urow / U) * ((N + U - 1) / U) + ucol / U] = (uint32_t)cnt;
+        }
+    };
+
+    if (!multiply) {
+        store_gate();
+        return;
+    }
     // ---- list: every wave scans the words' counts (at most 64 words), then places its own words' entries
     const uint64_t Fl = lane < words ? s_fp[2 * lane] : 0ull, Pl = lane < words ? s_fp[2 * lane + 1] : 0ull;
     int bf = __builtin_popcountll(Fl), bp = __builtin_popcountll(Pl);
@@ -173,30 +203,6 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
     __syncthreads();
     const int S = (n_full + n_part) * H::NSPE, Sfull = n_full * H::NSPE;
 
-    // what the gate leaves behind (a tile shared by several units is written by the first)
-    auto store_gate = [&]() {
-        if (!(mode & SMALL_GATE) || (ui * U) % B != 0 || (uj * U) % B != 0) return;
-        for (int e = threadIdx.x; e < TT * words; e += 256) {
-            const int t = e / words, w = e - t * words, i = ti0 + t / TU, j = tj0 + t % TU;
-            if (i < nbM && j < nbN) g.mask[((int64_t)i * nbN + j) * words + w] = s_word[w * TT + t];
-        }
-        if (wave == 0) {
-            int cnt = 0;
-            if (lane < TT) {
-                for (int w = 0; w < words; w++) cnt += __builtin_popcountll(s_word[w * TT + lane]);
-                const int i = ti0 + lane / TU, j = tj0 + lane % TU;
-                if (i < nbM && j < nbN) g.counts[(int64_t)i * nbN + j] = cnt;
-            }
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
-            if (lane == 0 && cnt) atomicAdd(reinterpret_cast<unsigned long long *>(g.kept_total), (unsigned long long)cnt);
-        }
-    };
-
-    if (!(mode & SMALL_MULTIPLY)) {
-        store_gate();
-        return;
-    }
     if (S == 0) {
         constexpr int LPR = U / 4;                                     // lanes per row
         const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -368,13 +374,6 @@ __global__ __launch_bounds__(256, 3) void k_small_three(const unsigned char *__r
     small_unit_body<B, 128, 3>(pA, pB, g, nbM, nbK, nbN, nMacN, n_units, n_xcd, mode, tau, M, N, C);
 }
 
-__global__ void k_clear_kept(int64_t *kept) { *kept = 0; }
-
-hipError_t launch_clear_kept(int64_t *kept, hipStream_t s) {
-    k_clear_kept<<<1, 1, 0, s>>>(kept);
-    return hipGetLastError();
-}
-
 // Unit by units of 128 in C: the wide one from half a unit per CU on.  Resident operands, K = 2048 at tile 32 (64 within
 // 10 %), 2 %, 10 %, 30 % kept and dense, narrow -> wide: 256 units 13.7 -> 12.4, 17.9 -> 15.3, 27.2 -> 20.0, 37.1 -> 24.9 us;
 // 196 units 12.3 -> 12.4, 15.7 -> 15.2, 20.7 -> 19.4, 36.1 -> 23.7; 144 units 10.0 -> 12.2, 13.4 -> 14.5, 17.8 -> 18.5,
@@ -385,6 +384,11 @@ hipError_t launch_clear_kept(int64_t *kept, hipStream_t s) {
 static int small_unit(int64_t M, int64_t N) {
     const int64_t units128 = ((M + 127) / 128) * ((N + 127) / 128);
     return units128 >= 128 ? 128 : 64;
+}
+
+int64_t small_units(int64_t M, int64_t N) {
+    const int64_t u = small_unit(M, N);
+    return ((M + u - 1) / u) * ((N + u - 1) / u);
 }
 
 // More than two units of 128 per CU: a ring of three stages leaves room for a third workgroup on the CU, whose loads and
@@ -458,14 +462,16 @@ hipError_t small_init() {
 // units 82.6 -> 75.7 | 140 -> 132; but 600 units 70 -> 67 | 108 -> 119 and 841 units 81 -> 90 | 135 -> 161.  With m = 257 to
 // 324 a second round is mostly empty: 1088 units 129 -> 104 | 220 -> 184, 1296 units 136 -> 120 | 233 -> 220; 1444 units
 // 132 -> 126 | 228 -> 227 and, K = 8192, 412 -> 436.
-// Gate and multiply called apart (`stages`) form mask and list twice, which k_gate's list spares: 5024 x 4128 x 3168 at tile
-// 32, 10 % kept, 58 us of k_gate, k_order and k_gemm against 68 by two of these launches.
+// Gate and multiply called apart (`stages`) form mask and list twice, which costs what the schedule does: the lines are
+// drawn closer (tau to a fraction and both stages, apart -> this: 625 units 114.7 -> 98 us; 768 units 122 -> 105, 127 -> 110;
+// 900 units 157 -> 160; 1000 units at tile 32 137.5 -> 139; 1120 units 162.5 -> 149.6, 126 -> 116; 1444 units 139 -> 147).
 bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau, bool stages) {
     const int64_t units128 = ((M + 127) / 128) * ((N + 127) / 128), m = ((M + 255) / 256) * ((N + 255) / 256);
     if (K / tile > SMALL_MAX_NBK) return false;
+    static_assert(SMALL_MAX_UNITS >= 6 * 256 && SMALL_MAX_UNITS >= 4 * 127, "units of either size");
     if (units128 <= 512) return true;
-    if (stages) return tau > 0.0f && units128 <= 640;
-    if (tau > 0.0f) return units128 <= 1536 && (units128 <= 832 || units128 > 1024 || K <= 8192);
+    if (stages) return tau > 0.0f && (units128 <= 832 || (units128 > 1024 && units128 <= 1200));
+    if (tau > 0.0f) return units128 <= SMALL_MAX_UNITS && (units128 <= 832 || units128 > 1024 || K <= 8192);
     return (m >= 160 && m <= 192) || (m >= 257 && m <= 324);
 }
 

@@ -20,7 +20,7 @@ using namespace spamm;
 // the moment the library is loaded until the process ends.  In host code this name is only a
 // handle for hipGetSymbolAddress: the device address is looked up once per context (= per device)
 // in spamm_create and everything below uses that pointer.
-static __device__ __align__(256) unsigned char scratch[SPAMM_NOALLOC_WORKSPACE_BYTES];
+static __device__ __align__(256) unsigned char scratch[SPAMM_NOALLOC_WORKSPACE_BYTES + SMALL_MAX_UNITS * 4];
 
 // Every spamm_multiply_noalloc on a device overwrites that device's array, whichever context makes
 // the call: a per-device generation number, bumped by each such call, tells a context whether what
@@ -71,7 +71,8 @@ struct Workspace {
     bool b_pruned = false;
 
     DevBuf packedA, packedB, nA, nB, nBt, rowmaxB;
-    DevBuf counts, klist, mask, macro_list, macro_count, macro_work, order, sched, kept_total;
+    DevBuf counts, klist, mask, macro_list, macro_count, macro_work, order, sched, kept_total, kept_units;
+    int64_t n_kept_units = 0;   // words of kept_units that add up to the last gate's kept products (0: kept_total has them)
 };
 
 struct spamm_ctx : Workspace {
@@ -163,6 +164,7 @@ GateBuffers gate_buffers(spamm_ctx *c) {
     g.order = (int32_t *)c->order.p;
     g.sched = (int32_t *)c->sched.p;
     g.kept_total = (int64_t *)c->kept_total.p;
+    g.kept_units = (uint32_t *)c->kept_units.p;
     return g;
 }
 
@@ -197,7 +199,7 @@ void reset_shape(spamm_ctx *c, int tile) {
 // The buffers of a workspace that the library allocated (carve-outs of the fixed array are not freed).
 void free_workspace(Workspace &w) {
     DevBuf *bufs[] = {&w.packedA, &w.packedB, &w.nA, &w.nB, &w.nBt, &w.rowmaxB, &w.counts, &w.klist,
-                      &w.mask, &w.macro_list, &w.macro_count, &w.macro_work, &w.order, &w.sched, &w.kept_total};
+                      &w.mask, &w.macro_list, &w.macro_count, &w.macro_work, &w.order, &w.sched, &w.kept_total, &w.kept_units};
     for (DevBuf *b : bufs) {
         if (b->p && !b->borrowed) (void)hipFree(b->p);
         *b = DevBuf();
@@ -360,8 +362,6 @@ static int normmap_any(spamm_ctx *c, int role, const void *dX, bool in16, int64_
     if (c->tile != tile) reset_shape(c, tile);
     const size_t nt = (size_t)(rows / tile) * (size_t)(cols / tile);
     c->have_gate = false;
-    if ((rc = ensure(c, c->kept_total, 16))) return rc;
-    int64_t *kept = (int64_t *)c->kept_total.p;
     if (role == SPAMM_ROLE_A) {
         // a new A invalidates B (fp16 copy and norm map alike) only if the shared dimension K
         // changes; A itself is invalid until its pass has been launched
@@ -380,7 +380,7 @@ static int normmap_any(spamm_ctx *c, int role, const void *dX, bool in16, int64_
         }
         if (c->timing) HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
         HIPCHK(c, launch_normmap_a(dX, in16, rows, cols, tile, c->packedA.p, (float *)c->nA.p,
-                                   prune ? (const float *)c->rowmaxB.p : nullptr, prune ? *prune_tau : 0.0f, kept, c->stream));
+                                   prune ? (const float *)c->rowmaxB.p : nullptr, prune ? *prune_tau : 0.0f, c->stream));
         if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[2], c->stream)); c->ev_a = true; }
         c->have_a = c->nm_a = true;
         c->a_pruned = prune;
@@ -398,7 +398,7 @@ static int normmap_any(spamm_ctx *c, int role, const void *dX, bool in16, int64_
         if (c->timing) HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
         const bool prune = prune_tau != nullptr && *prune_tau > 0.0f;
         HIPCHK(c, launch_normmap_b(dX, in16, rows, cols, tile, c->packedB.p, (float *)c->nB.p,
-                                   (float *)c->nBt.p, prune ? *prune_tau : 0.0f, kept, c->stream));
+                                   (float *)c->nBt.p, prune ? *prune_tau : 0.0f, c->stream));
         if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[1], c->stream)); c->ev_b = true; }
         c->have_b = c->nm_b = true;
         c->b_pruned = prune;
@@ -459,6 +459,7 @@ static int build_lists(spamm_ctx *c, float tau) {
     if ((rc = ensure(c, c->kept_total, 16))) return rc;
     HIPCHK(c, launch_gate(gate_buffers(c), s.nbM, s.nbK, s.nbN, c->tile, tau, c->n_xcd, c->gate_chunk_cap, c->stream));
     c->have_lists = true;
+    c->n_kept_units = 0;
     return SPAMM_OK;
 }
 
@@ -468,20 +469,20 @@ static bool is_small(const spamm_ctx *c, float tau, bool stages) {
     return c->gemm_shape == 0 && c->gate_chunk_cap == 0 && small_fits(c->M, c->K, c->N, c->tile, tau, stages);
 }
 
-// Its gate, its multiply (dC), or both.  kept_clear: a norm-map pass of this call has cleared the kept total.
-static int run_small(spamm_ctx *c, int mode, float tau, bool kept_clear, float *dC) {
+// Its gate, its multiply (dC), or both.
+static int run_small(spamm_ctx *c, int mode, float tau, float *dC) {
     int rc;
     const Shape s = shape_of(c);
     const size_t nt = (size_t)s.nbM * s.nbN;
     if ((rc = ensure(c, c->counts, nt * 4))) return rc;
     if ((rc = ensure(c, c->mask, nt * s.words * 8))) return rc;
-    if ((rc = ensure(c, c->kept_total, 16))) return rc;
-    if ((mode & SMALL_GATE) && !kept_clear) HIPCHK(c, launch_clear_kept((int64_t *)c->kept_total.p, c->stream));
+    if ((rc = ensure(c, c->kept_units, SMALL_MAX_UNITS * 4))) return rc;
     HIPCHK(c, launch_small(c->packedA.p, c->packedB.p, gate_buffers(c), c->M, c->K, c->N, c->tile, mode, tau, dC, c->n_xcd, c->stream));
     if (mode & SMALL_GATE) {
         c->tau = tau;
         c->have_gate = true;
         c->have_lists = false;
+        c->n_kept_units = small_units(c->M, c->N);
     }
     return SPAMM_OK;
 }
@@ -494,7 +495,7 @@ int spamm_gate(spamm_ctx *c, float tau) {
     int rc = set_device(c);
     if (rc) return rc;
     if (c->timing && !c->ev_a) HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
-    if (is_small(c, tau, true)) rc = run_small(c, SMALL_GATE, tau, false, nullptr);
+    if (is_small(c, tau, true)) rc = run_small(c, SMALL_GATE, tau, nullptr);
     else rc = build_lists(c, tau);
     if (rc) return rc;
     if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[3], c->stream)); c->ev_gate = true; }
@@ -515,7 +516,7 @@ int spamm_gemm_gated(spamm_ctx *c, float *dC) {
     if (!small && !c->have_lists && (rc = build_lists(c, c->tau))) return rc;    // (the work unit was fixed after a small gate)
     if (c->timing && !c->ev_gate) HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
     if (small) {
-        if ((rc = run_small(c, SMALL_MULTIPLY, c->tau, true, dC))) return rc;
+        if ((rc = run_small(c, SMALL_MULTIPLY, c->tau, dC))) return rc;
     } else {
         HIPCHK(c, launch_gemm(c->packedA.p, c->packedB.p, gate_buffers(c), c->M, c->K, c->N, c->tile, dC,
                               c->n_xcd, c->n_cu, c->gemm_ring, gemm_shape_for(c), c->stream));
@@ -567,19 +568,17 @@ static int multiply_any(spamm_ctx *c, const spamm_params *p, const void *dA, con
         if ((rc = ensure(c, c->nA, ta * 4))) return rc;
         if ((rc = ensure(c, c->nB, tb * 4))) return rc;
         if ((rc = ensure(c, c->nBt, tb * 4))) return rc;
-        if ((rc = ensure(c, c->kept_total, 16))) return rc;
         c->M = p->M;
         c->K = p->K;
         c->N = p->N;
         if (c->timing) HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
         const float tau_skip = prune ? p->tau : 0.0f;
-        int64_t *kept = (int64_t *)c->kept_total.p;
         if (a_eq_b)
             HIPCHK(c, launch_normmap_ab(dA, in16, p->M, p->tile, c->packedA.p, (float *)c->nA.p, c->packedB.p,
-                                        (float *)c->nB.p, (float *)c->nBt.p, tau_skip, kept, c->stream));
+                                        (float *)c->nB.p, (float *)c->nBt.p, tau_skip, c->stream));
         else
             HIPCHK(c, launch_normmap_pair(dA, dB, in16, p->M, p->K, p->N, p->tile, c->packedA.p, (float *)c->nA.p, c->packedB.p,
-                                          (float *)c->nB.p, (float *)c->nBt.p, tau_skip, kept, c->stream));
+                                          (float *)c->nB.p, (float *)c->nBt.p, tau_skip, c->stream));
         if (c->timing) {
             HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
             HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
@@ -608,7 +607,7 @@ static int multiply_any(spamm_ctx *c, const spamm_params *p, const void *dA, con
     if (is_small(c, p->tau, false)) {
         // one launch for both stages (the gate's interval is empty)
         if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[3], c->stream)); c->ev_gate = true; }
-        if ((rc = run_small(c, SMALL_GATE | SMALL_MULTIPLY, p->tau, !(reuse_a && reuse_b), dC))) return rc;
+        if ((rc = run_small(c, SMALL_GATE | SMALL_MULTIPLY, p->tau, dC))) return rc;
         if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[4], c->stream)); c->ev_gemm = true; }
         return SPAMM_OK;
     }
@@ -650,6 +649,11 @@ static size_t carve_static(Workspace &w, const spamm_params *p, unsigned char *b
     take(w.order, (size_t)sched_rounds(p->tile, (int64_t)nbM, (int64_t)nbN) * MAX_XCD * SUPER_M * SUPER_N * 4);
     take(w.sched, SCHED_WORDS * 4);
     take(w.kept_total, 16);
+    if (base) {                        // (behind the bytes that the limit speaks of)
+        w.kept_units.p = base + SPAMM_NOALLOC_WORKSPACE_BYTES;
+        w.kept_units.cap = SMALL_MAX_UNITS * 4;
+        w.kept_units.borrowed = true;
+    }
     return off;
 }
 
@@ -955,7 +959,13 @@ int spamm_get_stats(spamm_ctx *c, spamm_stats *out) {
     const Shape s = shape_of(c);
     out->total_products = s.nbM * s.nbK * s.nbN;
     int64_t kept = 0;
-    if ((rc = copy_out(c, c->kept_total.p, &kept, 8))) return rc;
+    if (c->n_kept_units) {
+        std::vector<uint32_t> units((size_t)c->n_kept_units);
+        if ((rc = copy_out(c, c->kept_units.p, units.data(), units.size() * 4))) return rc;
+        for (uint32_t u : units) kept += u;
+    } else if ((rc = copy_out(c, c->kept_total.p, &kept, 8))) {
+        return rc;
+    }
     out->kept_products = kept;
     if (c->timing && c->ev_a && c->ev_b && c->ev_gate && c->ev_gemm) {
         HIPCHK(c, hipEventElapsedTime(&out->ms_normmap_b, c->ev[0], c->ev[1]));

@@ -72,25 +72,25 @@ struct GateBuffers {
     int32_t *order;         // [n_xcd * P]     macro tile of XCD x's q-th workgroup (P = rounds * 32), valid for q < sched[8 + x]
     int32_t *sched;         // [24]            per XCD x: [x] computing items, [8 + x] all items, [16 + x] ticket
                             //                 counter of the persistent GEMM (zero between launches)
-    int64_t *kept_total;    // [1]  kept products
+    int64_t *kept_total;    // [1]  kept products (k_gate and k_order)
+    uint32_t *kept_units;   // [units of C, row by row]  kept products of each (k_small)
 };
 
-// The norm-map passes also clear *kept, the kept-product total that launch_small adds to.
 // tau_skip > 0: tau-aware pass, the fp16 copy of tile (i, k) is written only if
 // fl(nA[i,k] * rowmax[k]) >= tau_skip (rowmax[k] = max_j nB[k,j], launch_rowmax)
 hipError_t launch_normmap_a(const void *X, bool in16, int64_t rows, int64_t cols, int tile, void *packed,
-                            float *nm, const float *rowmax, float tau_skip, int64_t *kept, hipStream_t s);
+                            float *nm, const float *rowmax, float tau_skip, hipStream_t s);
 hipError_t launch_rowmax(const float *nB, int64_t nbK, int64_t nbN, float *rowmax, hipStream_t s);
 // tau_skip > 0: the fp16 copy of tiles of norm zero is not written (no product with them reaches tau)
 hipError_t launch_normmap_b(const void *X, bool in16, int64_t rows, int64_t cols, int tile, void *packed,
-                            float *nm, float *nmT, float tau_skip, int64_t *kept, hipStream_t s);
+                            float *nm, float *nmT, float tau_skip, hipStream_t s);
 // A = B (square): one pass over X for both operand roles
 hipError_t launch_normmap_ab(const void *X, bool in16, int64_t n, int tile, void *packedA, float *nmA,
-                             void *packedB, float *nmB, float *nmBt, float tau_skip, int64_t *kept, hipStream_t s);
+                             void *packedB, float *nmB, float *nmBt, float tau_skip, hipStream_t s);
 // both operands in one launch, for small ones (normmap_pair_fits); tau_skip > 0: tiles of norm zero are not written
 bool normmap_pair_fits(bool in16, bool tau_aware, int64_t M, int64_t K, int64_t N, int tile);
 hipError_t launch_normmap_pair(const void *A, const void *Bm, bool in16, int64_t M, int64_t K, int64_t N, int tile, void *packedA,
-                               float *nmA, void *packedB, float *nmB, float *nmBt, float tau_skip, int64_t *kept, hipStream_t s);
+                               float *nmA, void *packedB, float *nmB, float *nmBt, float tau_skip, hipStream_t s);
 // error report tooling (kernels_tools.hip).  Results go to host_out, pinned host memory: valid once *host_seq == seq
 // (per_tile: once the stream has been waited for).  The workspace's ticket is zero between launches (launch_clear_report once after allocation).
 struct ReportSums {
@@ -188,11 +188,11 @@ hipError_t launch_gemm(const void *packedA, const void *packedB, const GateBuffe
 // work unit of the gated GEMM: a whole macro tile (256 x 256 of C, one workgroup per CU), half of
 // one (128 x 256, two workgroups per CU), a whole one by eight waves, or whole ones by workgroups
 // that stay on their CU and draw items from a ticket counter per XCD
-// gate and multiply in one launch (kernels_small.hip); kept_total must be zero before it (launch_clear_kept where no
-// norm-map pass has run)
-hipError_t launch_clear_kept(int64_t *kept, hipStream_t s);
+// gate and multiply in one launch (kernels_small.hip)
 constexpr int64_t SMALL_MAX_NBK = 2048;      // its k list lives in LDS
 hipError_t small_init();
+int64_t small_units(int64_t M, int64_t N);   // its units of C
+constexpr int64_t SMALL_MAX_UNITS = 1536;
 bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau, bool stages);
 constexpr int SMALL_GATE = 1, SMALL_MULTIPLY = 2;    // what launch_small does: either or both
 hipError_t launch_small(const void *packedA, const void *packedB, const GateBuffers &g, int64_t M, int64_t K, int64_t N,
