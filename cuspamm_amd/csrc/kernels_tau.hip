@@ -50,8 +50,7 @@ struct TauTune {
 struct TauWorkspace {
     TauState st;
     TauTune tune;
-    unsigned int ticket;                    // workgroups of the running pass that have finished
-    unsigned int pad_;
+    Tickets tickets;                        // workgroups of the running pass that have finished
     unsigned long long zeros;               // products that are not positive
     unsigned long long hist[3][TAU_COPIES][2048];   // one per pass: cleared together, beforehand
     unsigned long long leaf[TREE_COPIES][TREE_LEAVES];
@@ -125,7 +124,7 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_hist(const float *__restrict__ 
         if (c) atomicAdd(&ws->hist[PASS][blockIdx.x % TAU_COPIES][b], c);
     }
     if (PASS == 0 && lane == 0 && zeros) atomicAdd(&ws->zeros, zeros);
-    if (!last_workgroup(&ws->ticket)) return;
+    if (!last_workgroup(&ws->tickets)) return;
 
     // thread t takes bins NB - 1 - t * PER downwards; `above` = products in the bins over its own.
     // (The loads of this step are independent and go out together: a round trip that bypasses the L2
@@ -251,7 +250,7 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_count(const float *__restrict__
         agent_store(&ws->part[blockIdx.x][0], cnt);
         agent_store(&ws->part[blockIdx.x][1], __builtin_bit_cast(unsigned long long, sum));
     }
-    if (!last_workgroup(&ws->ticket)) return;
+    if (!last_workgroup(&ws->tickets)) return;
     const bool have = threadIdx.x < gridDim.x;                    // gridDim.x <= TAU_MAXB <= TAU_NTH
     cnt = have ? agent_load(&ws->part[threadIdx.x][0]) : 0ull;
     sum = have ? __builtin_bit_cast(double, agent_load(&ws->part[threadIdx.x][1])) : 0.0;
@@ -377,7 +376,7 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_tree(const float *__restrict__ 
         for (int r = 0; r < COPIES; r++) c += s_leaf[n * COPIES + r];
         if (c) atomicAdd(&ws->leaf[blockIdx.x % TREE_COPIES][n], c);
     }
-    if (!last_workgroup(&ws->ticket)) return;
+    if (!last_workgroup(&ws->tickets)) return;
     // products in the leaves from each thread's own up
     unsigned long long part[TREE_COPIES], incl = 0;
 #pragma unroll
@@ -578,15 +577,15 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_small_tune(const float *__restr
     }
 }
 
-// once after allocation: every launch leaves the ticket and the histograms as it found them
+// once after allocation: every launch leaves the tickets and the histograms as it found them
 __global__ __launch_bounds__(256) void k_tau_clear(TauWorkspace *ws) {
     const int b = blockIdx.x * 256 + threadIdx.x;                 // 8 workgroups per histogram copy
     (&ws->hist[0][0][0])[b] = 0;
     if (b < TREE_COPIES * TREE_LEAVES) (&ws->leaf[0][0])[b] = 0;
     if (b == 0) {
-        ws->ticket = 0;
         ws->zeros = 0;
     }
+    if (b <= (int)TICKET_GROUPS) ws->tickets.t[b].n = 0;
 }
 
 hipError_t launch_tau_clear(void *workspace, hipStream_t s) {

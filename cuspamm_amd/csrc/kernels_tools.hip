@@ -29,7 +29,7 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half8t __attribute__((ext_vector_type(8)));
 
 struct ReportWorkspace {
-    unsigned int ticket;                // workgroups of the running launch that have finished; zero between launches
+    Tickets tickets;                    // workgroups of the running launch that have finished; zero between launches
     unsigned int out_of_range;          // k_limbs: an operand holds values without limbs; zero between calls
     double part[1];                     // per workgroup: its sums (report_workspace_bytes says how many)
 };
@@ -42,7 +42,7 @@ __device__ __forceinline__ void finish_sums(ReportWorkspace *ws, double own, Rep
     __shared__ double s_fin[4][N];
     if (threadIdx.x < N)
         agent_store(reinterpret_cast<unsigned long long *>(&ws->part[(size_t)blockIdx.x * N + threadIdx.x]), __builtin_bit_cast(unsigned long long, own));
-    if (!last_workgroup(&ws->ticket)) return;
+    if (!last_workgroup(&ws->tickets)) return;
     if (threadIdx.x == 0) agent_store(&ws->out_of_range, 0u);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     double v[N];
@@ -436,12 +436,12 @@ __global__ __launch_bounds__(256) void k_dropped_bound(const float *__restrict__
 }
 
 __global__ void k_clear_report(ReportWorkspace *ws) {
-    ws->ticket = 0;
-    ws->out_of_range = 0;
+    if (threadIdx.x <= TICKET_GROUPS) ws->tickets.t[threadIdx.x].n = 0;
+    if (threadIdx.x == 0) ws->out_of_range = 0;
 }
 
 hipError_t launch_clear_report(void *workspace, hipStream_t s) {
-    k_clear_report<<<1, 1, 0, s>>>((ReportWorkspace *)workspace);
+    k_clear_report<<<1, 64, 0, s>>>((ReportWorkspace *)workspace);
     return hipGetLastError();
 }
 

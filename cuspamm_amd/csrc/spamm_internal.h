@@ -92,7 +92,7 @@ bool normmap_pair_fits(bool in16, bool tau_aware, int64_t M, int64_t K, int64_t 
 hipError_t launch_normmap_pair(const void *A, const void *Bm, bool in16, int64_t M, int64_t K, int64_t N, int tile, void *packedA,
                                float *nmA, void *packedB, float *nmB, float *nmBt, float tau_skip, hipStream_t s);
 // error report tooling (kernels_tools.hip).  Results go to host_out, pinned host memory: valid once *host_seq == seq
-// (per_tile: once the stream has been waited for).  The workspace's ticket is zero between launches (launch_clear_report once after allocation).
+// (per_tile: once the stream has been waited for).  The workspace's tickets are zero between launches (launch_clear_report once after allocation).
 struct ReportSums {
     double v[3];
 };

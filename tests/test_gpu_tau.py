@@ -224,3 +224,24 @@ def test_bisection_by_a_search_tree(orc, ctx, shape, rounds):
             got, want = ctx.tune_bisect(expected, tol, rounds), orc.tune_bisect(nA, nB, expected, tol, rounds)
             assert np.float32(got[0]) == np.float32(want[0]) and got[1] == want[1], (expected, tol, got, want)
     ctx.set_stream(None)
+
+
+@pytest.mark.parametrize("workgroups", [47, 48, 49, 63, 65, 256])
+def test_counts_of_few_and_many_workgroups(ctx, workgroups):
+    """Workgroups of a pass hand their part to the one that ends last, found by one ticket (up to 48) or by groups' tickets:
+    every product is counted once, and again in the next call (16 products of a norm map row in 64 k each per wave)."""
+    rng = np.random.default_rng(workgroups)
+    nA = rng.random((16 * workgroups, 64), dtype=np.float32)
+    nB = rng.random((64, 16), dtype=np.float32)
+    p = nA[:, None, :] * np.ascontiguousarray(nB.T)[None]
+    ordered = np.sort(p.ravel())
+    ctx.set_normmaps(nA, nB, 32)
+    for _ in range(2):
+        for thr in (0.0, 0.25, 0.9):
+            assert ctx.count_kept(thr)[0] == np.count_nonzero(p.astype(np.float64) >= thr)
+        tau, achieved = ctx.tau_for_ratio(0.3)
+        assert np.float32(tau) == ordered[p.size - int(np.ceil(0.3 * p.size))]
+        assert achieved == np.count_nonzero(p >= np.float32(tau)) / p.size
+        tau, achieved = ctx.tune_bisect(0.5, 0.01, 20)
+        assert abs(achieved - 0.5) < 0.01 and abs(np.count_nonzero(p >= np.float32(tau)) / p.size - achieved) < 1e-6
+        assert ctx.dropped_bound(0.5) == pytest.approx(np.sqrt((np.where(p < 0.5, p.astype(np.float64), 0.0).sum(axis=2) ** 2).sum()), rel=1e-6)
