@@ -9,6 +9,10 @@
 // counts, kept total -- is written on the way out; the macro tiles' work lists, which
 // nothing reads after this kernel, are built by k_gate if somebody asks for them.
 //
+// Of the k loop's 0.285 us per stage on 256 CUs (2048^3 dense) the loads alone take 0.2 (a bare copy of the same panels into
+// LDS, 21 TB/s over the chip), all else without them 0.18; without the MFMAs 0.27, without the LDS reads 0.285.  Two stages
+// per sync, rings of 6 and 8 and square blocks of units per XCD changed it by 1 % or cost workgroups per CU.
+//
 // The order of the sum is k_gemm's: entries that every tile of the unit's MACRO tile
 // keeps come first, then the others, each group in ascending k rotated to the
 // macro tile's anchor.  So a unit looks at the norms of its whole macro tile, and C is
@@ -18,8 +22,8 @@
 // results out -- of which units of 128 (16 KiB a stage, two workgroups per CU, or three) make
 // the k loop shortest and units of 64 spread a small C over more CUs.  Gate, schedule
 // and GEMM as launches of their own -> this kernel, whole multiplies: 256^3 24.6 -> 14.7 us
-// (today, with one launch for both norm-map passes too: 10.7), 1056 x 1568 x 1312 38.2 -> 22.8
-// (18.5), fp16 2048^3 at tile 32, 5 % kept, 38.5 -> 26.3 (22.5), 2048^3 dense 63 -> 38, 1024 rows
+// (today, with one launch for both norm-map passes too: 10.3), 1056 x 1568 x 1312 38.2 -> 22.8
+// (17.4), fp16 2048^3 at tile 32, 5 % kept, 38.5 -> 26.3 (21.8), 2048^3 dense 63 -> 38 (36), 1024 rows
 // against a resident 8192^2 50.3 -> 36.5 (35.8).
 #include "gemm_device.h"
 
