@@ -245,3 +245,18 @@ def test_counts_of_few_and_many_workgroups(ctx, workgroups):
         tau, achieved = ctx.tune_bisect(0.5, 0.01, 20)
         assert abs(achieved - 0.5) < 0.01 and abs(np.count_nonzero(p >= np.float32(tau)) / p.size - achieved) < 1e-6
         assert ctx.dropped_bound(0.5) == pytest.approx(np.sqrt((np.where(p < 0.5, p.astype(np.float64), 0.0).sum(axis=2) ** 2).sum()), rel=1e-6)
+
+
+@pytest.mark.parametrize("nbK", [1023, 1025])
+def test_selection_of_products_that_fit_32_bits_and_more(ctx, nbK):
+    """Below 2^32 products two bins share a word of the histogram.  Products of row i are all i + 1: what a kept fraction
+    selects is known."""
+    nbM = nbN = 2048
+    nA = np.repeat(np.arange(1, nbM + 1, dtype=np.float32)[:, None], nbK, axis=1)
+    ctx.set_normmaps(nA, np.ones((nbK, nbN), np.float32), 32)
+    per_row, total = nbK * nbN, nbM * nbK * nbN
+    for ratio in (0.0, 1e-4, 0.3, 0.999, 1.0):
+        want = min(max(1, int(np.ceil(ratio * float(total)))), total)
+        row = nbM - (want - 1) // per_row
+        tau, achieved = ctx.tau_for_ratio(ratio)
+        assert tau == row and achieved == (nbM - row + 1) * per_row / total
