@@ -276,8 +276,9 @@ def test_small_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N, ti
         apart.close()
 
 
-@pytest.mark.parametrize("M,K,N,tile", [(2944, 256, 2912, 32),      # 529 units: the first that no longer fit two to a CU
-                                        (2944, 12320, 2912, 32),    # a list too long for three to a CU
+@pytest.mark.parametrize("M,K,N,tile", [(2944, 256, 2912, 32),      # 529 units: no longer two to a CU at once
+                                        (3200, 160, 3072, 32), (3200, 256, 3200, 64),               # 600 and 625: two and three to a CU
+                                        (3200, 12320, 3136, 32),    # a list too long for three to a CU
                                         (4096, 512, 2560, 64), (4352, 320, 4160, 64),               # dense too: 160 and 289 macro tiles
                                         (4096, 96, 4096, 32), (3968, 384, 4224, 128), (4096, 64, 6144, 64),
                                         (192, 640, 98304, 64)])     # 1536 units, the most
