@@ -23,7 +23,7 @@
 // at zero.  Few products (k_tau_small_*) are held by one workgroup, and all passes
 // are one launch.
 // Whole calls, norm maps and the multiply behind them included: 5024 x 4128 x 3168 at
-// tile 32 to a kept fraction 667 -> 135 us, the reference's tuned 2048^3 (8 of at most
+// tile 32 to a kept fraction 667 -> 133 us, the reference's tuned 2048^3 (8 of at most
 // 20 rounds) 381 -> 75 us.
 #include "gemm_device.h"
 #include "reduce_device.h"
