@@ -621,6 +621,15 @@ static unsigned tau_grid(int64_t nbM, int64_t nbK, int64_t nbN, int jb = TAU_JB_
     return (unsigned)(blocks < TAU_MAXB ? blocks : TAU_MAXB);
 }
 
+// For passes whose workgroups count in 32 bits and leave no part of their own (k_tau_hist, k_tau_tree): as many workgroups
+// that none has much over 2^30 products.  (A multiply that fits the card's memory stays below it; norm maps alone,
+// 65535 tiles a side, hold up to 2^48 products.)
+static unsigned tau_count_grid(int64_t nbM, int64_t nbK, int64_t nbN, int jb) {
+    const unsigned grid = tau_grid(nbM, nbK, nbN, jb);
+    const int64_t total = tau_products(nbM, nbK, nbN);
+    return total >> 31 > grid / 2 ? (unsigned)(total >> 30) : grid;
+}
+
 hipError_t launch_tau_select(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN,
                              unsigned long long want, void *workspace, TauState *host_out, unsigned long long *host_seq,
                              unsigned long long seq, hipStream_t s) {
@@ -633,10 +642,8 @@ hipError_t launch_tau_select(const float *nA, const float *nBt, int64_t nbM, int
 #undef SPAMM_SELECT
         return hipGetLastError();
     }
-    unsigned grid = tau_grid(nbM, nbK, nbN);
+    const unsigned grid = tau_count_grid(nbM, nbK, nbN, TAU_JB_COUNT);
     const unsigned long long total = (unsigned long long)n;
-    // a workgroup counts in 32 bits (2e9 products each is N = 262144 at tile 32)
-    if (total >> 31 > grid / 2) grid = (unsigned)(total >> 30);
     k_tau_hist<0><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out, host_seq, seq);
     k_tau_hist<1><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out, host_seq, seq);
     k_tau_hist<2><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out, host_seq, seq);
@@ -671,8 +678,8 @@ hipError_t launch_tau_tune(const float *nA, const float *nBt, int64_t nbM, int64
         k_tau_count<<<tau_grid(nbM, nbK, nbN), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, 0.0, total, 1, expected, tol,
                                                            max_rounds, call, passes == 0, ws, nullptr, host_out, host_seq, seq);
     for (int p = 0; p < passes; p++)
-        k_tau_tree<<<tau_grid(nbM, nbK, nbN, TAU_JB_TREE), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, expected, tol,
-                                                                       max_rounds, call, p == passes - 1, ws, host_out, host_seq, seq);
+        k_tau_tree<<<tau_count_grid(nbM, nbK, nbN, TAU_JB_TREE), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, expected, tol,
+                                                                             max_rounds, call, p == passes - 1, ws, host_out, host_seq, seq);
     return hipGetLastError();
 }
 

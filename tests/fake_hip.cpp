@@ -5,6 +5,8 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <map>
+#include <string>
 
 namespace {
 
@@ -30,6 +32,9 @@ struct Config {
 };
 thread_local Config pushed;
 
+std::map<const void *, std::string> kernel_names;
+std::string launched;       // "name grid;" of every launch since fake_launches was last asked
+
 }  // namespace
 
 extern "C" {
@@ -39,6 +44,12 @@ void fake_thread_device(int device) { current = device; }
 void fake_expect(int device) { expected = device; n_checked = n_wrong = 0; first_wrong[0] = 0; }
 int fake_checked() { return n_checked; }
 const char *fake_wrong() { return n_wrong ? first_wrong : nullptr; }
+const char *fake_launches() {
+    static std::string out;
+    out.swap(launched);
+    launched.clear();
+    return out.c_str();
+}
 
 // --- the runtime
 hipError_t hipGetDeviceCount(int *n) { *n = 2; return hipSuccess; }
@@ -84,12 +95,13 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hi
     *stream = pushed.stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t s) {
+hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **, size_t, hipStream_t s) {
+    launched += kernel_names[f] + " " + std::to_string(grid.x) + ";";
     check("hipLaunchKernel", current == expected && (!s || ((Owned *)s)->device == current));
     return hipSuccess;
 }
 void **__hipRegisterFatBinary(const void *) { static void *handle; return &handle; }
-void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, void *, void *, dim3 *, dim3 *, int *) {}
+void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, void *, void *, dim3 *, dim3 *, int *) { kernel_names[f] = name; }
 void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
 void __hipUnregisterFatBinary(void **) {}
 

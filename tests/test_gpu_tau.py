@@ -260,3 +260,14 @@ def test_selection_of_products_that_fit_32_bits_and_more(ctx, nbK):
         row = nbM - (want - 1) // per_row
         tau, achieved = ctx.tau_for_ratio(ratio)
         assert tau == row and achieved == (nbM - row + 1) * per_row / total
+
+
+def test_bisection_of_more_products_than_workgroups_count(orc, ctx):
+    """Beyond 2^38 products a pass has more workgroups than the chip runs at once.  Products of row i are all i + 1, 2^24 of
+    each: kept fractions and the mean are those of one product a row, whose bisection the checker has."""
+    nbM, nbK, nbN = 16640, 1024, 16384
+    rows = np.arange(1, nbM + 1, dtype=np.float32)[:, None]
+    ctx.set_normmaps(np.repeat(rows, nbK, axis=1), np.ones((nbK, nbN), np.float32), 32)
+    for expected in (0.5, 0.003):
+        got, want = ctx.tune_bisect(expected, 1e-4, 20), orc.tune_bisect(rows, np.ones((1, 1), np.float32), expected, 1e-4, 20)
+        assert np.float32(got[0]) == np.float32(want[0]) and got[1] == want[1]

@@ -1,0 +1,82 @@
+"""What the engine's host side launches and allocates, on a runtime of imaginary GPUs (fake_hip.cpp): kernels do nothing
+there, so a call that waits for a kernel's result reports a runtime error.  Each check runs in a process of its own."""
+import ctypes
+import os
+import re
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+i64, f64, p = ctypes.c_int64, ctypes.c_double, ctypes.byref
+
+
+class Engine:
+    def __init__(self, fake_path, lib_path):
+        self.fake = ctypes.CDLL(fake_path, mode=ctypes.RTLD_GLOBAL)
+        self.fake.fake_launches.restype = ctypes.c_char_p
+        self.L = ctypes.CDLL(lib_path)
+
+    def context(self):
+        h = ctypes.c_void_p()
+        assert self.L.spamm_create(p(h), 0) == 0
+        return h
+
+    def launches(self):
+        """(kernel, workgroups) of each launch since the last look."""
+        out = []
+        for item in self.fake.fake_launches().decode().split(";")[:-1]:
+            name, grid = item.rsplit(" ", 1)
+            length, rest = re.match(r"_ZN5spamm(\d+)(\w+)", name).groups()
+            out.append((rest[:int(length)], int(grid)))
+        return out
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    lib = os.path.join(ROOT, "cuspamm_amd", "libspamm_gfx950.so")
+    if not os.path.exists(lib):
+        pytest.fail("the engine has not been built")
+    fake = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(HERE, "fake_hip.cpp"), "-o", fake], check=True)
+
+    def run(check, *args):
+        done = subprocess.run([sys.executable, os.path.abspath(__file__), fake, lib, check] + [str(a) for a in args], text=True,
+                              stdout=subprocess.PIPE, stderr=subprocess.STDOUT, timeout=120)
+        assert done.returncode == 0 and done.stdout.strip().endswith("ok"), done.stdout[-3000:]
+    return run
+
+
+def counters_of_the_tau_passes(e, nbM, nbK, nbN):
+    h = e.context()
+    maps = ctypes.create_string_buffer(4 * max(nbM, nbN) * nbK)
+    assert e.L.spamm_set_normmaps(h, maps, maps, i64(nbM), i64(nbK), i64(nbN), 32) == 0
+    out = ctypes.c_float()
+    e.launches()
+    assert e.L.spamm_tau_for_ratio(h, f64(0.5), p(out), None) == -3
+    assert e.L.spamm_tune_bisect(h, f64(0.5), f64(0.01), 20, p(out), None) == -3
+    seen = set()
+    for name, grid in e.launches():
+        jb = {"k_tau_hist": 16, "k_tau_tree": 4}.get(name)
+        if jb:
+            seen.add(name)
+            units = nbM * -(-nbN // jb) * -(-nbK // 64)                     # of jb columns and 64 k, dealt to waves in turn
+            share = -(-units // (16 * grid)) * 16 * jb * 64
+            assert share < 2 ** 32, "%s: %d workgroups of up to %d products" % (name, grid, share)
+            assert nbM * nbK * nbN > 2 ** 38 or grid <= 256
+    assert seen == {"k_tau_hist", "k_tau_tree"}
+
+
+# the most products of two norm maps of half a gigabyte or less, and sizes that a multiply has
+@pytest.mark.parametrize("shape", [(65535, 1025, 65535), (65535, 1, 65535), (1024, 512, 1024), (64, 33, 64)])
+def test_a_workgroup_counts_less_than_32_bits_hold(run, shape):
+    """Products that fall into one bin or leaf together -- equal norms -- must not pass its 32-bit counter."""
+    run("counters_of_the_tau_passes", *shape)
+
+
+if __name__ == "__main__":
+    globals()[sys.argv[3]](Engine(*sys.argv[1:3]), *map(int, sys.argv[4:]))
+    print("ok")
