@@ -438,7 +438,7 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
                 g.sched[2 * MAX_XCD + wave] = 0;
             }
         }
-        if (threadIdx.x == 0) g.kept_total[0] = (int64_t)total;
+        if (threadIdx.x == 0) g.kept->total = (int64_t)total;
         return;
     }
     int n_ne = 0;                               // super tiles with work
@@ -655,7 +655,7 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
             g.sched[2 * MAX_XCD + x] = 0;      // ticket counter of the persistent GEMM
         }
     }
-    if (threadIdx.x == 0) g.kept_total[0] = (int64_t)total;
+    if (threadIdx.x == 0) g.kept->total = (int64_t)total;
     __syncthreads();
     // the sequences, all waves: XCD x by 16 / n_xcd of them, half a wave per super tile, lane = macro tile
     {

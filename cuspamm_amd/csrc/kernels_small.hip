@@ -149,7 +149,8 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
     __syncthreads();
     // What the gate leaves behind (a tile shared by several units is written by the first).  A unit's kept products are
     // a word of its own: added to one total by atomics they queued up at the kernel's end, where 200 to 1000 units finish
-    // together (1024^3 10 % 15.4 -> 13.7 us whole, 2048^3 dense 33.8 -> 31.5, 1056 x 1568 x 1312 18.6 -> 17.7).
+    // together (1024^3 10 % 15.4 -> 13.7 us whole, 2048^3 dense 33.8 -> 31.5, 1056 x 1568 x 1312 18.6 -> 17.7).  The total is
+    // minus their number then: what the last gate was is known on the device, also behind a replayed graph.
     auto store_gate = [&]() {
         if (!(mode & SMALL_GATE)) return;
         const bool first = (ui * U) % B == 0 && (uj * U) % B == 0;
@@ -166,7 +167,9 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
             }
 #pragma unroll
             for (int off = 32; off >= 1; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
-            if (lane == 0) g.kept_units[(urow / U) * ((N + U - 1) / U) + ucol / U] = (uint32_t)cnt;
+            const int64_t per_row = (N + U - 1) / U;
+            if (lane == 0) g.kept->units[(urow / U) * per_row + ucol / U] = (uint32_t)cnt;
+            if (lane == 0 && urow == 0 && ucol == 0) g.kept->total = -((M + U - 1) / U * per_row);
         }
     };
 
@@ -388,11 +391,6 @@ __global__ __launch_bounds__(256, 3) void k_small_three(const unsigned char *__r
 static int small_unit(int64_t M, int64_t N) {
     const int64_t units128 = ((M + 127) / 128) * ((N + 127) / 128);
     return units128 >= 128 ? 128 : 64;
-}
-
-int64_t small_units(int64_t M, int64_t N) {
-    const int64_t u = small_unit(M, N);
-    return ((M + u - 1) / u) * ((N + u - 1) / u);
 }
 
 // Clearly more than two units of 128 per CU: a ring of three stages leaves room for a third workgroup on the CU, whose loads

@@ -20,7 +20,7 @@ using namespace spamm;
 // the moment the library is loaded until the process ends.  In host code this name is only a
 // handle for hipGetSymbolAddress: the device address is looked up once per context (= per device)
 // in spamm_create and everything below uses that pointer.
-static __device__ __align__(256) unsigned char scratch[SPAMM_NOALLOC_WORKSPACE_BYTES + SMALL_MAX_UNITS * 4];
+static __device__ __align__(256) unsigned char scratch[SPAMM_NOALLOC_WORKSPACE_BYTES + sizeof(KeptProducts)];
 
 // Every spamm_multiply_noalloc on a device overwrites that device's array, whichever context makes
 // the call: a per-device generation number, bumped by each such call, tells a context whether what
@@ -71,8 +71,7 @@ struct Workspace {
     bool b_pruned = false;
 
     DevBuf packedA, packedB, nA, nB, nBt, rowmaxB;
-    DevBuf counts, klist, mask, macro_list, macro_count, macro_work, order, sched, kept_total, kept_units;
-    int64_t n_kept_units = 0;   // words of kept_units that add up to the last gate's kept products (0: kept_total has them)
+    DevBuf counts, klist, mask, macro_list, macro_count, macro_work, order, sched, kept;
 };
 
 struct spamm_ctx : Workspace {
@@ -163,8 +162,7 @@ GateBuffers gate_buffers(spamm_ctx *c) {
     g.macro_work = (int32_t *)c->macro_work.p;
     g.order = (int32_t *)c->order.p;
     g.sched = (int32_t *)c->sched.p;
-    g.kept_total = (int64_t *)c->kept_total.p;
-    g.kept_units = (uint32_t *)c->kept_units.p;
+    g.kept = (KeptProducts *)c->kept.p;
     return g;
 }
 
@@ -199,7 +197,7 @@ void reset_shape(spamm_ctx *c, int tile) {
 // The buffers of a workspace that the library allocated (carve-outs of the fixed array are not freed).
 void free_workspace(Workspace &w) {
     DevBuf *bufs[] = {&w.packedA, &w.packedB, &w.nA, &w.nB, &w.nBt, &w.rowmaxB, &w.counts, &w.klist,
-                      &w.mask, &w.macro_list, &w.macro_count, &w.macro_work, &w.order, &w.sched, &w.kept_total, &w.kept_units};
+                      &w.mask, &w.macro_list, &w.macro_count, &w.macro_work, &w.order, &w.sched, &w.kept};
     for (DevBuf *b : bufs) {
         if (b->p && !b->borrowed) (void)hipFree(b->p);
         *b = DevBuf();
@@ -456,10 +454,9 @@ static int build_lists(spamm_ctx *c, float tau) {
     if ((rc = ensure(c, c->macro_work, (size_t)s.n_macro * 4))) return rc;
     if ((rc = ensure(c, c->order, (size_t)sched_rounds(c->tile, s.nbM, s.nbN) * MAX_XCD * SUPER_M * SUPER_N * 4))) return rc;
     if ((rc = ensure(c, c->sched, SCHED_WORDS * 4))) return rc;
-    if ((rc = ensure(c, c->kept_total, 16))) return rc;
+    if ((rc = ensure(c, c->kept, sizeof(KeptProducts)))) return rc;
     HIPCHK(c, launch_gate(gate_buffers(c), s.nbM, s.nbK, s.nbN, c->tile, tau, c->n_xcd, c->gate_chunk_cap, c->stream));
     c->have_lists = true;
-    c->n_kept_units = 0;
     return SPAMM_OK;
 }
 
@@ -476,13 +473,12 @@ static int run_small(spamm_ctx *c, int mode, float tau, float *dC) {
     const size_t nt = (size_t)s.nbM * s.nbN;
     if ((rc = ensure(c, c->counts, nt * 4))) return rc;
     if ((rc = ensure(c, c->mask, nt * s.words * 8))) return rc;
-    if ((rc = ensure(c, c->kept_units, SMALL_MAX_UNITS * 4))) return rc;
+    if ((rc = ensure(c, c->kept, sizeof(KeptProducts)))) return rc;
     HIPCHK(c, launch_small(c->packedA.p, c->packedB.p, gate_buffers(c), c->M, c->K, c->N, c->tile, mode, tau, dC, c->n_xcd, c->stream));
     if (mode & SMALL_GATE) {
         c->tau = tau;
         c->have_gate = true;
         c->have_lists = false;
-        c->n_kept_units = small_units(c->M, c->N);
     }
     return SPAMM_OK;
 }
@@ -648,11 +644,10 @@ static size_t carve_static(Workspace &w, const spamm_params *p, unsigned char *b
     take(w.macro_work, n_macro * 4);
     take(w.order, (size_t)sched_rounds(p->tile, (int64_t)nbM, (int64_t)nbN) * MAX_XCD * SUPER_M * SUPER_N * 4);
     take(w.sched, SCHED_WORDS * 4);
-    take(w.kept_total, 16);
-    if (base) {                        // (behind the bytes that the limit speaks of)
-        w.kept_units.p = base + SPAMM_NOALLOC_WORKSPACE_BYTES;
-        w.kept_units.cap = SMALL_MAX_UNITS * 4;
-        w.kept_units.borrowed = true;
+    take(w.kept, 16);
+    if (base) {                        // (it lies behind the bytes that the limit speaks of, of which it has always counted so many)
+        w.kept.p = base + SPAMM_NOALLOC_WORKSPACE_BYTES;
+        w.kept.cap = sizeof(KeptProducts);
     }
     return off;
 }
@@ -958,15 +953,14 @@ int spamm_get_stats(spamm_ctx *c, spamm_stats *out) {
     if (rc) return rc;
     const Shape s = shape_of(c);
     out->total_products = s.nbM * s.nbK * s.nbN;
-    int64_t kept = 0;
-    if (c->n_kept_units) {
-        std::vector<uint32_t> units((size_t)c->n_kept_units);
-        if ((rc = copy_out(c, c->kept_units.p, units.data(), units.size() * 4))) return rc;
-        for (uint32_t u : units) kept += u;
-    } else if ((rc = copy_out(c, c->kept_total.p, &kept, 8))) {
-        return rc;
+    KeptProducts kept;
+    if ((rc = copy_out(c, c->kept.p, &kept, sizeof(kept)))) return rc;
+    if (kept.total < 0) {              // a gate by units, each with a word of its own
+        const int64_t n = -kept.total < SMALL_MAX_UNITS ? -kept.total : SMALL_MAX_UNITS;
+        kept.total = 0;
+        for (int64_t i = 0; i < n; i++) kept.total += kept.units[i];
     }
-    out->kept_products = kept;
+    out->kept_products = kept.total;
     if (c->timing && c->ev_a && c->ev_b && c->ev_gate && c->ev_gemm) {
         HIPCHK(c, hipEventElapsedTime(&out->ms_normmap_b, c->ev[0], c->ev[1]));
         HIPCHK(c, hipEventElapsedTime(&out->ms_normmap_a, c->ev[1], c->ev[2]));

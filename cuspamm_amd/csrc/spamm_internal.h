@@ -61,6 +61,14 @@ struct __attribute__((aligned(16))) MacroEntry {
     uint32_t mask_hi;
 };
 
+// Kept products of a gate: their total (k_gate, k_order), or below zero minus the number of units that C has, and each
+// unit's (k_small, row by row).
+constexpr int64_t SMALL_MAX_UNITS = 1536;
+struct KeptProducts {
+    int64_t total;
+    uint32_t units[SMALL_MAX_UNITS];
+};
+
 struct GateBuffers {
     const float *nA;        // [nbM x nbK]
     const float *nBt;       // [nbN x nbK]  (transposed B norm map)
@@ -72,8 +80,7 @@ struct GateBuffers {
     int32_t *order;         // [n_xcd * P]     macro tile of XCD x's q-th workgroup (P = rounds * 32), valid for q < sched[8 + x]
     int32_t *sched;         // [24]            per XCD x: [x] computing items, [8 + x] all items, [16 + x] ticket
                             //                 counter of the persistent GEMM (zero between launches)
-    int64_t *kept_total;    // [1]  kept products (k_gate and k_order)
-    uint32_t *kept_units;   // [units of C, row by row]  kept products of each (k_small)
+    KeptProducts *kept;
 };
 
 // tau_skip > 0: tau-aware pass, the fp16 copy of tile (i, k) is written only if
@@ -191,8 +198,6 @@ hipError_t launch_gemm(const void *packedA, const void *packedB, const GateBuffe
 // gate and multiply in one launch (kernels_small.hip)
 constexpr int64_t SMALL_MAX_NBK = 2048;      // its k list lives in LDS
 hipError_t small_init();
-int64_t small_units(int64_t M, int64_t N);   // its units of C
-constexpr int64_t SMALL_MAX_UNITS = 1536;
 bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau, bool stages);
 constexpr int SMALL_GATE = 1, SMALL_MULTIPLY = 2;    // what launch_small does: either or both
 hipError_t launch_small(const void *packedA, const void *packedB, const GateBuffers &g, int64_t M, int64_t K, int64_t N,

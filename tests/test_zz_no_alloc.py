@@ -201,3 +201,41 @@ def test_noalloc_multiply_replays_in_a_hip_graph(orc, ctx, work_unit):
         err, nrm, _ = orc.frob_diff(C.cpu().numpy(), ref["C"])
         assert err <= 1e-3 * nrm
     gctx.close()
+
+
+@pytest.mark.parametrize("units", [(0, 1), (1, 0)], ids=["one_launch_replayed", "gate_and_gemm_replayed"])
+def test_kept_products_are_those_of_the_last_gate_that_ran(ctx, units):
+    """A replay of one form of the multiply behind an eager call of the other: both leave their kept products where
+    get_stats looks, whichever ran last."""
+    import torch
+    import cuspamm_amd as sp
+    M, K, N, tile = 640, 768, 512, 64
+    g = torch.Generator(device="cuda").manual_seed(7)
+    dA = torch.rand((M, K), generator=g, device="cuda") - 0.5
+    dB = torch.rand((K, N), generator=g, device="cuda") - 0.5
+    ctx.multiply(dA, dB, tile, 0.0)
+    taus = [ctx.tau_for_ratio(r)[0] for r in (0.25, 0.75)]
+    want = []
+    for tau in taus:
+        ctx.gate(tau)
+        want.append(int(ctx.get_counts().sum()))
+    C = torch.zeros((M, N), dtype=torch.float32, device="cuda")
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        gctx = sp.SpammContext(0)
+        for unit, tau in zip(units, taus):
+            gctx.set_option(sp.OPT_GEMM_SHAPE, unit)
+            gctx.multiply_noalloc(dA, dB, tile, tau, C)
+        gctx.set_option(sp.OPT_GEMM_SHAPE, units[0])
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            gctx.multiply_noalloc(dA, dB, tile, taus[0], C)
+        gctx.set_option(sp.OPT_GEMM_SHAPE, units[1])
+        for _ in range(2):
+            gctx.multiply_noalloc(dA, dB, tile, taus[1], C)
+            assert gctx.get_stats().kept_products == want[1]
+            graph.replay()
+            side.synchronize()
+            assert gctx.get_stats().kept_products == want[0]
+        gctx.close()
