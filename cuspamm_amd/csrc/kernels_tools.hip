@@ -245,15 +245,16 @@ __global__ __launch_bounds__(256) void k_limbs(LimbOperand a, LimbOperand b, int
 // One workgroup owns 64 x 64 of C, a wave 32 x 32 of it: 4 accumulator registers x 4 MFMA blocks x 7 orders, so that two
 // waves share a SIMD.  The k blocks are sorted by the limbs they need on both sides (whole numbers: the sum does not
 // care), and each kind has a loop of its own without branches, the next block's operands on their way while one is
-// multiplied.  Groups of GB x GB workgroups that share operands in an L2 run on one XCD; the groups of a diagonal, which
-// have much the same work, are spread over the XCDs.
+// multiplied.  Groups of GB x GB workgroups that share operands in an L2 run on one XCD; the groups, row by row, go round
+// the XCDs, each row turned by two against the one above, so that those of a diagonal, which have much the same work, are
+// spread over them.
 constexpr int ORDERS = 2 * LIMBS - 1;
 constexpr int64_t LIMB_MAX_K = 32768 - 64;      // an order adds up to 4 products of at most 2^14 per k in 31 bits
 constexpr int LIMB_MAX_KB = 32768 / LIMB_BLOCK;
 
 __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict__ plA, const uint8_t *__restrict__ clsA,
                                                         const int8_t *__restrict__ plB, const uint8_t *__restrict__ clsB, int nkb,
-                                                        int nbi, int nbj, int gb, int gj_rounds, int n_xcd, int64_t N,
+                                                        int nbi, int nbj, int gb, int ngj, int n_xcd, int64_t N,
                                                         const float *__restrict__ C, ReportWorkspace *__restrict__ ws,
                                                         ReportSums *__restrict__ host_out, unsigned long long *__restrict__ host_seq,
                                                         unsigned long long seq) {
@@ -264,7 +265,7 @@ __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict
     const int wr = wave >> 1, wc = wave & 1;
     const int l16 = lane & 15, q = lane >> 4;
     const int x = (int)blockIdx.x % n_xcd, at = (int)blockIdx.x / n_xcd, in_group = at % (gb * gb), group = at / (gb * gb);
-    const int gi = group / gj_rounds, gj = (group % gj_rounds) * n_xcd + (x + n_xcd * 2 * gi - 2 * gi) % n_xcd;
+    const int gi = (group * n_xcd + x) / ngj, gj = ((group * n_xcd + x) % ngj + 2 * (ngj - gi % ngj)) % ngj;
     const int bi = gi * gb + in_group / gb, bj = gj * gb + in_group % gb;
     const bool bad = ws->out_of_range != 0u;
     double e2 = 0, d2 = 0, c2 = 0;
@@ -469,9 +470,11 @@ static int error_shape(int64_t rows, int64_t N, int n_cu, int64_t *n_wg) {
     return best;
 }
 
-// Workgroups of k_error_limbs: groups of gb x gb, and how many of a group row an XCD has.
+// Workgroups of k_error_limbs: groups of gb x gb, ngj of them side by side.  A group is no wider than C in either direction
+// and there is one for every gb x gb blocks that C has, but for what rounds up to whole groups and XCDs: workgroups
+// without a block are launched, waited for and added up all the same (1048576 x 64 with 64 of them to a block 6050 us).
 struct LimbGrid {
-    int nbi, nbj, gb, gj_rounds;
+    int nbi, nbj, gb, ngj;
     int64_t n_wg;
 };
 static LimbGrid limb_grid(int64_t rows, int64_t N, int n_xcd) {
@@ -480,8 +483,10 @@ static LimbGrid limb_grid(int64_t rows, int64_t N, int n_xcd) {
     g.nbj = (int)(N / LIMB_BLOCK);
     const int64_t blocks = (int64_t)g.nbi * g.nbj;
     g.gb = blocks >= 2048 ? 8 : blocks >= 512 ? 4 : 1;
-    g.gj_rounds = ((g.nbj + g.gb - 1) / g.gb + n_xcd - 1) / n_xcd;
-    g.n_wg = (int64_t)((g.nbi + g.gb - 1) / g.gb) * g.gj_rounds * n_xcd * g.gb * g.gb;
+    while (g.gb > g.nbi || g.gb > g.nbj) g.gb /= 2;
+    g.ngj = (g.nbj + g.gb - 1) / g.gb;
+    const int64_t groups = (int64_t)((g.nbi + g.gb - 1) / g.gb) * g.ngj;
+    g.n_wg = (groups + n_xcd - 1) / n_xcd * n_xcd * g.gb * g.gb;
     return g;
 }
 
@@ -536,7 +541,7 @@ hipError_t launch_error_limbs(const void *packedA, const void *packedB, int64_t 
     k_limbs<<<(unsigned)(blocksA + blocksB), 256, 0, s>>>(a, b, K, tile, nkb, ws);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    k_error_limbs<<<(unsigned)g.n_wg, 256, 0, s>>>(a.planes, a.cls, b.planes, b.cls, nkb, g.nbi, g.nbj, g.gb, g.gj_rounds, n_xcd, N,
+    k_error_limbs<<<(unsigned)g.n_wg, 256, 0, s>>>(a.planes, a.cls, b.planes, b.cls, nkb, g.nbi, g.nbj, g.gb, g.ngj, n_xcd, N,
                                                    C + row0 * N, ws, host_out, host_seq, seq);
     return hipGetLastError();
 }

@@ -77,6 +77,32 @@ def test_a_workgroup_counts_less_than_32_bits_hold(run, shape):
     run("counters_of_the_tau_passes", *shape)
 
 
+def resident_operands(e, h, M, K, N, tile):
+    X = ctypes.create_string_buffer(16)                                     # (nothing reads them)
+    assert e.L.spamm_normmap_f32(h, 1, X, i64(K), i64(N), tile) == 0
+    assert e.L.spamm_normmap_f32(h, 0, X, i64(M), i64(K), tile) == 0
+
+
+def workgroups_of_the_report(e, M, K, N):
+    h = e.context()
+    resident_operands(e, h, M, K, N, 64)
+    out = (ctypes.c_double * 3)()
+    e.launches()
+    e.L.spamm_error_vs_dense_f64(h, ctypes.create_string_buffer(16), i64(0), i64(M), out)
+    grid = dict(e.launches())["k_error_limbs"]
+    blocks = (M // 64) * (N // 64)
+    # whole groups of at most 8 x 8, no wider than C: less than twice the blocks in the narrower direction's last
+    # group, and one round of groups over the XCDs
+    assert blocks <= grid <= 2 * blocks + 8 * 64, "%d workgroups for %d blocks" % (grid, blocks)
+
+
+@pytest.mark.parametrize("shape", [(262144, 512, 64), (64, 512, 262144), (16384, 512, 512), (512, 512, 16384), (4096, 512, 512),
+                                   (4096, 4096, 4096), (576, 1024, 14592), (1088, 512, 4160), (640, 640, 640)])
+def test_the_report_has_a_workgroup_per_block_of_c(run, shape):
+    """Of 64 x 64: also where C is narrow, which takes no more of them than the same C the other way round."""
+    run("workgroups_of_the_report", *shape)
+
+
 if __name__ == "__main__":
     globals()[sys.argv[3]](Engine(*sys.argv[1:3]), *map(int, sys.argv[4:]))
     print("ok")
