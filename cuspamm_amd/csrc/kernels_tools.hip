@@ -18,6 +18,8 @@
 // that the chip holds under them, about 2 GHz); 1984 x 2176 x 768: 196 -> 158.  In whole numbers instead (one call, its
 // host wait included): 4096^3 2107 -> 867 us on uniform values in [-1, 1) (4 bytes each, 16 products, 2.6 Pop/s: power),
 // 620 where 3 bytes do, 272 on exp(-d / 100); 1984 x 2176 x 768 165 -> 82, 67, 49; 64 rows of 4096^3 173 -> 109, 91, 50.
+// An operand with a value of 127 or more costs both launches for nothing (flags of their own per 16 blocks, no planes
+// behind them, and no host between): 4096^3 2115 -> 2144, 2048^3 316 -> 327, 1280^3 106 -> 111, 1024^3 56 -> 61.6.
 // The scalar bound of 64 x 64 x 64 tiles 52 -> 7 us, the per-tile one 51 -> 4; results go straight to host memory (a
 // clearing launch before and a copy after each were 25 us a call).
 #include "gemm_device.h"
@@ -28,11 +30,22 @@ namespace spamm {
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half8t __attribute__((ext_vector_type(8)));
 
+constexpr int RANGE_FLAGS = 16;         // (stores to one address queue: 32768 waves that all found such values took 0.6 ms)
+struct alignas(128) RangeFlag {
+    unsigned long long call;
+};
+
 struct ReportWorkspace {
     Tickets tickets;                    // workgroups of the running launch that have finished; zero between launches
-    unsigned int out_of_range;          // k_limbs: an operand holds values without limbs; zero between calls
+    RangeFlag range[RANGE_FLAGS];       // k_limbs: the last call of which an operand held values without limbs
     double part[1];                     // per workgroup: its sums (report_workspace_bytes says how many)
 };
+
+// Whether an operand of this call held values that k_limbs has no limbs for.  (By the call's number: the flags are never
+// put back, so a launch that finds its call done may look at them while a later call, on another stream, sets its own.)
+__device__ __forceinline__ bool out_of_range(const ReportWorkspace *ws, unsigned long long call) {
+    return __ballot(agent_load(&ws->range[threadIdx.x % RANGE_FLAGS].call) == call) != 0ull;
+}
 
 // Sums of all workgroups' N values, by the workgroup that finishes last, to host_out (pinned host memory): in a
 // fixed order, so that a repeated call gives the same number.  `own`: the workgroup's values, in thread i the i-th.
@@ -43,7 +56,6 @@ __device__ __forceinline__ void finish_sums(ReportWorkspace *ws, double own, Rep
     if (threadIdx.x < N)
         agent_store(reinterpret_cast<unsigned long long *>(&ws->part[(size_t)blockIdx.x * N + threadIdx.x]), __builtin_bit_cast(unsigned long long, own));
     if (!last_workgroup(&ws->tickets)) return;
-    if (threadIdx.x == 0) agent_store(&ws->out_of_range, 0u);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     double v[N];
 #pragma unroll
@@ -76,7 +88,10 @@ __global__ __launch_bounds__(256, NBR * NBC > 8 ? 2 : 3) void k_error_dense(cons
                                                                         int64_t K, int64_t N, int tile, const float *__restrict__ C,
                                                                         int64_t row0, int64_t row1, int nwg_n,
                                                                         ReportWorkspace *__restrict__ ws, ReportSums *__restrict__ host_out,
-                                                                        unsigned long long *__restrict__ host_seq, unsigned long long seq) {
+                                                                        unsigned long long *__restrict__ host_seq, unsigned long long seq,
+                                                                        bool behind_limbs) {
+    // behind k_error_limbs, which has already published the result unless the operands' values were too large for it
+    if (behind_limbs && !out_of_range(ws, seq)) return;
     __shared__ double red[4][3];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wr = wave >> 1, wc = wave & 1;
@@ -193,8 +208,10 @@ struct LimbOperand {
     int64_t n_blocks;           // blocks of 64 rows, times nkb
 };
 
-__global__ __launch_bounds__(256) void k_limbs(LimbOperand a, LimbOperand b, int64_t K, int tile, int nkb, ReportWorkspace *__restrict__ ws) {
+__global__ __launch_bounds__(256) void k_limbs(LimbOperand a, LimbOperand b, int64_t K, int tile, int nkb, unsigned long long call,
+                                               ReportWorkspace *__restrict__ ws) {
     __shared__ unsigned int s_used[4];
+    __shared__ bool s_fits[4];
     const bool is_a = (int64_t)blockIdx.x < a.n_blocks;
     const LimbOperand op = is_a ? a : b;
     const int64_t blk = is_a ? blockIdx.x : blockIdx.x - a.n_blocks;
@@ -220,9 +237,17 @@ __global__ __launch_bounds__(256) void k_limbs(LimbOperand a, LimbOperand b, int
     }
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) used |= __shfl_xor(used, off, 64);
-    if (__ballot(!fits) != 0ull && lane == 0) agent_store(&ws->out_of_range, 1u);
-    if (lane == 0) s_used[wave] = used;
+    fits = __ballot(!fits) == 0ull;
+    if (lane == 0) {
+        s_used[wave] = used;
+        s_fits[wave] = fits;
+    }
     __syncthreads();
+    if (!(s_fits[0] && s_fits[1] && s_fits[2] && s_fits[3])) {          // nothing will read the planes
+        unsigned long long *flag = &ws->range[blockIdx.x % RANGE_FLAGS].call;
+        if (threadIdx.x == 0 && agent_load(flag) != call) agent_store(flag, call);
+        return;
+    }
     used = s_used[0] | s_used[1] | s_used[2] | s_used[3];
     const int limbs = used == 0 ? 0 : (31 - __builtin_clz(used)) / 8 + 1;
     if (threadIdx.x == 0) op.cls[blk] = (uint8_t)limbs;
@@ -258,6 +283,7 @@ __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict
                                                         const float *__restrict__ C, ReportWorkspace *__restrict__ ws,
                                                         ReportSums *__restrict__ host_out, unsigned long long *__restrict__ host_seq,
                                                         unsigned long long seq) {
+    if (out_of_range(ws, seq)) return;          // (k_error_dense comes behind this launch)
     __shared__ double red[4][3];
     __shared__ int s_count[17], s_place[16];
     __shared__ uint16_t s_list[LIMB_MAX_KB];
@@ -267,9 +293,8 @@ __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict
     const int x = (int)blockIdx.x % n_xcd, at = (int)blockIdx.x / n_xcd, in_group = at % (gb * gb), group = at / (gb * gb);
     const int gi = (group * n_xcd + x) / ngj, gj = ((group * n_xcd + x) % ngj + 2 * (ngj - gi % ngj)) % ngj;
     const int bi = gi * gb + in_group / gb, bj = gj * gb + in_group % gb;
-    const bool bad = ws->out_of_range != 0u;
     double e2 = 0, d2 = 0, c2 = 0;
-    if (bi < nbi && bj < nbj && !bad) {
+    if (bi < nbi && bj < nbj) {
         // ---- k blocks by kind
         if (threadIdx.x < 17) s_count[threadIdx.x] = 0;
         __syncthreads();
@@ -376,7 +401,7 @@ __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict
         }
     }
     if (lane == 0) {
-        red[wave][0] = bad ? -1.0 : e2;         // (a sum below zero: the host takes the fp64 product)
+        red[wave][0] = e2;
         red[wave][1] = d2;
         red[wave][2] = c2;
     }
@@ -438,7 +463,7 @@ __global__ __launch_bounds__(256) void k_dropped_bound(const float *__restrict__
 
 __global__ void k_clear_report(ReportWorkspace *ws) {
     if (threadIdx.x <= TICKET_GROUPS) ws->tickets.t[threadIdx.x].n = 0;
-    if (threadIdx.x == 0) ws->out_of_range = 0;
+    if (threadIdx.x < RANGE_FLAGS) ws->range[threadIdx.x].call = 0;
 }
 
 hipError_t launch_clear_report(void *workspace, hipStream_t s) {
@@ -515,15 +540,18 @@ size_t report_workspace_bytes(int64_t rows, int64_t N, int n_cu, int n_xcd) {
 
 hipError_t launch_error_vs_dense(const void *packedA, const void *packedB, int64_t K, int64_t N, int tile, const float *C,
                                  int64_t row0, int64_t row1, int n_cu, void *workspace, ReportSums *host_out,
-                                 unsigned long long *host_seq, unsigned long long seq, hipStream_t s) {
+                                 unsigned long long *host_seq, unsigned long long seq, bool behind_limbs, hipStream_t s) {
     int64_t n_wg = 0;
     const int shape = error_shape(row1 - row0, N, n_cu, &n_wg);
     const _Float16 *pA = (const _Float16 *)packedA, *pB = (const _Float16 *)packedB;
     ReportWorkspace *ws = (ReportWorkspace *)workspace;
     const int nwg_n = (int)((N + 32 * ERROR_SHAPES[shape].nbc - 1) / (32 * ERROR_SHAPES[shape].nbc));
-    if (shape == 0) k_error_dense<4, 4><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out, host_seq, seq);
-    else if (shape == 1) k_error_dense<4, 2><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out, host_seq, seq);
-    else k_error_dense<2, 2><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out, host_seq, seq);
+#define SPAMM_DENSE(NBR, NBC) \
+    k_error_dense<NBR, NBC><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out, host_seq, seq, behind_limbs)
+    if (shape == 0) SPAMM_DENSE(4, 4);
+    else if (shape == 1) SPAMM_DENSE(4, 2);
+    else SPAMM_DENSE(2, 2);
+#undef SPAMM_DENSE
     return hipGetLastError();
 }
 
@@ -538,7 +566,7 @@ hipError_t launch_error_limbs(const void *packedA, const void *packedB, int64_t 
     uint8_t *cls = (uint8_t *)limbs + (blocksA + blocksB) * (LIMBS * LIMB_PLANE);
     const LimbOperand a = {(const _Float16 *)packedA, planes, cls, row0, blocksA};
     const LimbOperand b = {(const _Float16 *)packedB, planes + blocksA * (LIMBS * LIMB_PLANE), cls + blocksA, 0, blocksB};
-    k_limbs<<<(unsigned)(blocksA + blocksB), 256, 0, s>>>(a, b, K, tile, nkb, ws);
+    k_limbs<<<(unsigned)(blocksA + blocksB), 256, 0, s>>>(a, b, K, tile, nkb, seq, ws);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     k_error_limbs<<<(unsigned)g.n_wg, 256, 0, s>>>(a.planes, a.cls, b.planes, b.cls, nkb, g.nbi, g.nbj, g.gb, g.ngj, n_xcd, N,

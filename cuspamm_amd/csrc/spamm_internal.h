@@ -107,9 +107,10 @@ size_t report_workspace_bytes(int64_t rows, int64_t N, int n_cu, int n_xcd);    
 hipError_t launch_clear_report(void *workspace, hipStream_t s);
 hipError_t launch_error_vs_dense(const void *packedA, const void *packedB, int64_t K, int64_t N, int tile, const float *C,
                                  int64_t row0, int64_t row1, int n_cu, void *workspace, ReportSums *host_out,
-                                 unsigned long long *host_seq, unsigned long long seq, hipStream_t s);
-// the same on the integer matrix pipeline; limbs: limb_bytes() of scratch (0: not for this shape).  A first sum below
-// zero: an operand holds values it cannot take (beyond +-127, inf, NaN), the sums are not valid
+                                 unsigned long long *host_seq, unsigned long long seq, bool behind_limbs, hipStream_t s);
+// the same on the integer matrix pipeline; limbs: limb_bytes() of scratch (0: not for this shape).  It publishes nothing if an
+// operand holds values that it cannot take (beyond +-127, inf, NaN): launch_error_vs_dense with the same seq and behind_limbs
+// follows it, and does nothing otherwise
 size_t limb_bytes(int64_t rows, int64_t K, int64_t N);
 hipError_t launch_error_limbs(const void *packedA, const void *packedB, int64_t K, int64_t N, int tile, const float *C,
                               int64_t row0, int64_t row1, int n_xcd, void *limbs, void *workspace, ReportSums *host_out,

@@ -350,7 +350,9 @@ def test_error_report_by_any_block_shape(ctx, rows, N, row0):
     (32, 1024, 608, 2304, 128, 832, "limbs"), (128, 4096, 256, 2176, 0, 4096, "limbs"), (64, 512, 32704, 512, 0, 512, "edge"),
     (64, 256, 32768, 256, 0, 256, "edge"), (64, 2048, 320, 1024, 0, 2048, "large"), (128, 512, 512, 512, 0, 512, "large"),
     (64, 8256, 512, 128, 64, 8192, "limbs"), (64, 576, 1024, 14592, 0, 576, "unit"),        # blocks of C one or few across, or high
-    (64, 320, 192, 320, 0, 320, "inf"), (32, 256, 256, 256, 0, 256, "zero")])
+    (64, 320, 192, 320, 0, 320, "inf"), (32, 256, 256, 256, 0, 256, "zero"),
+    (64, 1280, 1024, 1088, 0, 1280, "inf"), (32, 1184, 1056, 1280, 64, 1088, "nan"), (128, 1280, 1024, 1280, 0, 1280, "zero"),
+    (32, 1344, 1056, 1280, 64, 1280, "unit")])
 def test_error_report_over_the_range_of_fp16(ctx, tile, M, K, N, row0, rows, kind):
     """Whatever the magnitudes: 0 to 4 bytes a value by blocks, just inside and outside of what bytes hold, subnormals,
     infinities, sums at the length where 32 bits end.  Against fp64 on the host (K terms a sum, rows * N in a norm, 2^-53
@@ -374,8 +376,8 @@ def test_error_report_over_the_range_of_fp16(ctx, tile, M, K, N, row0, rows, kin
         A, B = np.abs(A), np.abs(B)
     if kind == "zero":
         A[:] = 0
-    if kind == "inf":
-        A[70, 100] = np.inf
+    if kind in ("inf", "nan"):
+        A[70, 100] = np.inf if kind == "inf" else np.nan
     hA, hB = A.astype(np.float16).astype(np.float64), B.astype(np.float16).astype(np.float64)
     ctx.normmap_f32(1, torch.from_numpy(B).cuda(), tile)
     ctx.normmap_f32(0, torch.from_numpy(A).cuda(), tile)
@@ -386,9 +388,35 @@ def test_error_report_over_the_range_of_fp16(ctx, tile, M, K, N, row0, rows, kin
     c = C[row0:row0 + rows].astype(np.float64)
     for _ in range(2):            # (the second call finds the workspace as the first left it)
         got = ctx.error_vs_dense(torch.from_numpy(C).cuda(), row0, row0 + rows)
-        if kind == "inf":
+        if kind in ("inf", "nan"):
             assert not np.isfinite(got[0]) and not np.isfinite(got[1])
             assert abs(got[2] - np.linalg.norm(c)) <= 1e-9 * np.linalg.norm(c)
             continue
         for g, ref in zip(got, (np.linalg.norm(c - dense), np.linalg.norm(dense), np.linalg.norm(c))):
             assert abs(g - ref) <= 1e-9 * ref
+
+
+def test_error_reports_of_small_and_large_values_by_turns(ctx):
+    """The integer product has the fp64 one behind it, which does nothing unless values were too large: report after
+    report, of one kind and the other, each on another stream than the last and none waited for."""
+    import torch
+    M, K, N, tile = 1280, 1024, 1088, 64
+    rng = np.random.default_rng(5)
+    A, B = rng.uniform(-1.0, 1.0, (M, K)).astype(np.float16), rng.uniform(-1.0, 1.0, (K, N)).astype(np.float16)
+    C = rng.uniform(-1.0, 1.0, (M, N)).astype(np.float32)
+    dB, dC = torch.from_numpy(B).cuda(), torch.from_numpy(C).cuda()
+    kinds = []
+    for scale in (1, 1024):                       # (a power of two: fp16 holds the scaled values too)
+        X = A * np.float16(scale)
+        dense = X.astype(np.float64) @ B.astype(np.float64)
+        kinds.append((torch.from_numpy(X).cuda(), [np.linalg.norm(v) for v in (C - dense, dense, C.astype(np.float64))]))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for at, kind in enumerate((0, 1, 0, 0, 1, 1, 0, 1)):
+        ctx.set_stream(streams[at % 2].cuda_stream)
+        ctx.normmap_f16(1, dB, tile)
+        ctx.normmap_f16(0, kinds[kind][0], tile)
+        for got, want in zip(ctx.error_vs_dense(dC), kinds[kind][1]):
+            assert abs(got - want) <= 1e-9 * want, at
+    torch.cuda.synchronize()
+    ctx.set_stream(None)

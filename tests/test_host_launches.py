@@ -103,6 +103,20 @@ def test_the_report_has_a_workgroup_per_block_of_c(run, shape):
     run("workgroups_of_the_report", *shape)
 
 
+def launches_of_the_report(e):
+    h = e.context()
+    resident_operands(e, h, 2048, 2048, 2048, 64)
+    out = (ctypes.c_double * 3)()
+    e.launches()
+    assert e.L.spamm_error_vs_dense_f64(h, ctypes.create_string_buffer(16), i64(0), i64(2048), out) == -3
+    assert [name for name, _ in e.launches()][-3:] == ["k_limbs", "k_error_limbs", "k_error_dense"]
+
+
+def test_the_report_launches_its_fp64_product_before_it_waits(run):
+    """Which of the two products does the work is known on the device alone: the host does not come back for it."""
+    run("launches_of_the_report")
+
+
 if __name__ == "__main__":
     globals()[sys.argv[3]](Engine(*sys.argv[1:3]), *map(int, sys.argv[4:]))
     print("ok")
