@@ -472,14 +472,14 @@ hipError_t launch_clear_report(void *workspace, hipStream_t s) {
 }
 
 // Blocks per wave of the dense product: 16-wide blocks, rows x columns.  Every SIMD works through the same number of
-// waves, so a wave's time (in MFMAs, and the share that the conversions add) times the fullest SIMD's number of waves decides.
+// waves, so a wave's time (in MFMAs a step, and the share that the conversions add) times the fullest SIMD's number of waves decides.
 struct ErrorShape {
     int nbr, nbc;
     double cost;        // per MFMA, relative
 };
 static const ErrorShape ERROR_SHAPES[3] = {{4, 4, 1.00}, {4, 2, 1.06}, {2, 2, 1.12}};
 
-static int error_shape(int64_t rows, int64_t N, int n_cu, int64_t *n_wg) {
+static int error_shape(int64_t rows, int64_t N, int n_cu, int64_t *n_wg, double *mfmas = nullptr) {
     int best = 0;
     double best_time = 0.0;
     for (int i = 0; i < 3; i++) {
@@ -492,6 +492,7 @@ static int error_shape(int64_t rows, int64_t N, int n_cu, int64_t *n_wg) {
             *n_wg = wg;
         }
     }
+    if (mfmas) *mfmas = best_time;
     return best;
 }
 
@@ -518,10 +519,21 @@ static LimbGrid limb_grid(int64_t rows, int64_t N, int n_xcd) {
 static int64_t limb_kb(int64_t K) { return (K + LIMB_BLOCK - 1) / LIMB_BLOCK; }
 
 // Bytes of the planes and the blocks' numbers of limbs of both operands; 0: the fp64 pipeline is to be used -- beyond
-// what 32 bits add up, beyond 4 GiB of planes, and for so small a product that the second launch costs more than the
-// sums (256^3 26.5 us in fp64, 27 to 29 in whole numbers; 512^3 35.6 against 30 to 34).
-size_t limb_bytes(int64_t rows, int64_t K, int64_t N) {
-    if (K > LIMB_MAX_K || (double)rows * (double)K * (double)N < 64.0e6) return 0;
+// what 32 bits add up, beyond 4 GiB of planes, and where the split of the operands, which no block of C shares, is more than
+// a quarter of the fp64 product's time.  Both are estimated in us: of the split its launches and 3 TB/s of operands, of the product
+// 0.033 per MFMA of its fullest SIMD (4096^3 2112, 1280^3 94, 64 rows of 4096^2 151).  fp64 -> whole numbers, whole calls, on
+// uniform values | exp(-d / 100) | values too large for limbs, by the estimates' ratio: 2.8, 1024 x 512 x 1024 39.0 -> 39.2 | 36.2
+// | 43.1 and 64 x 1024 x 65536 160 -> 173 | 66 | 224; 3.6, 640^3 41 -> 39.7 | 37.9 | 47.0; 4.2, 256 x 1024 x 4096 57 -> 53 | 45 | 66.5
+// and 768^3 46 -> 44.1 | 41.2 | 51.6; 5.1, 1024^3 57 -> 50 | 45.5 | 61.7; 10, 65536 x 512 x 256 289 -> 186 | 87 | 311.  With K
+// below 256 a block's fixed costs outweigh its few products: 4096 x 64 x 4096 61 -> 82 | 73 | 68, K = 128 94 -> 94 | 74 | 102,
+// K = 256 159 -> 119 | 79 | 168.
+size_t limb_bytes(int64_t rows, int64_t K, int64_t N, int n_cu) {
+    if (K > LIMB_MAX_K || K < 256) return 0;
+    int64_t n_wg = 0;
+    double mfmas = 0.0;
+    (void)error_shape(rows, N, n_cu, &n_wg, &mfmas);
+    const double dense = 0.033 * mfmas * (double)(K / 4), split = 6.0 + (double)(rows + N) * (double)K * 2.0 / 3.0e6;
+    if (dense < 4.0 * split) return 0;
     const size_t blocks = (size_t)(rows / LIMB_BLOCK + N / LIMB_BLOCK) * (size_t)limb_kb(K);
     if (blocks >= (1u << 31) / (LIMBS * LIMB_PLANE / 2)) return 0;       // 4 GiB
     return blocks * (LIMBS * LIMB_PLANE) + blocks;

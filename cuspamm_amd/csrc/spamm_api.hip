@@ -725,7 +725,7 @@ int spamm_error_vs_dense_f64(spamm_ctx *c, const float *dC, int64_t row0, int64_
     // exact in whole numbers where the operands' values allow it and their planes fit (else, and without memory for
     // them, in fp64: behind the integer product's launch, which alone knows the values)
     const unsigned long long seq = ++c->seq;
-    const size_t limbs = limb_bytes(row1 - row0, c->K, c->N);
+    const size_t limbs = limb_bytes(row1 - row0, c->K, c->N, c->n_cu);
     const bool whole = limbs && ensure(c, c->limbs, limbs) == SPAMM_OK;
     if (whole)
         HIPCHK(c, launch_error_limbs(c->packedA.p, c->packedB.p, c->K, c->N, c->tile, dC, row0, row1, c->n_xcd, c->limbs.p, c->reportws.p,

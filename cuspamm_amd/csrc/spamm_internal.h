@@ -111,7 +111,7 @@ hipError_t launch_error_vs_dense(const void *packedA, const void *packedB, int64
 // the same on the integer matrix pipeline; limbs: limb_bytes() of scratch (0: not for this shape).  It publishes nothing if an
 // operand holds values that it cannot take (beyond +-127, inf, NaN): launch_error_vs_dense with the same seq and behind_limbs
 // follows it, and does nothing otherwise
-size_t limb_bytes(int64_t rows, int64_t K, int64_t N);
+size_t limb_bytes(int64_t rows, int64_t K, int64_t N, int n_cu);
 hipError_t launch_error_limbs(const void *packedA, const void *packedB, int64_t K, int64_t N, int tile, const float *C,
                               int64_t row0, int64_t row1, int n_xcd, void *limbs, void *workspace, ReportSums *host_out,
                               unsigned long long *host_seq, unsigned long long seq, hipStream_t s);

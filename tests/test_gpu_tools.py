@@ -349,10 +349,10 @@ def test_error_report_by_any_block_shape(ctx, rows, N, row0):
     (32, 64, 32, 64, 0, 64, "unit"), (32, 192, 416, 320, 64, 128, "unit"), (64, 576, 1088, 640, 0, 576, "limbs"),
     (32, 1024, 608, 2304, 128, 832, "limbs"), (128, 4096, 256, 2176, 0, 4096, "limbs"), (64, 512, 32704, 512, 0, 512, "edge"),
     (64, 256, 32768, 256, 0, 256, "edge"), (64, 2048, 320, 1024, 0, 2048, "large"), (128, 512, 512, 512, 0, 512, "large"),
-    (64, 8256, 512, 128, 64, 8192, "limbs"), (64, 576, 1024, 14592, 0, 576, "unit"),        # blocks of C one or few across, or high
+    (64, 8256, 2048, 128, 64, 8192, "limbs"), (64, 576, 1024, 14592, 0, 576, "unit"),        # blocks of C one or few across, or high
     (64, 320, 192, 320, 0, 320, "inf"), (32, 256, 256, 256, 0, 256, "zero"),
     (64, 1280, 1024, 1088, 0, 1280, "inf"), (32, 1184, 1056, 1280, 64, 1088, "nan"), (128, 1280, 1024, 1280, 0, 1280, "zero"),
-    (32, 1344, 1056, 1280, 64, 1280, "unit")])
+    (32, 1344, 1056, 1280, 64, 1280, "unit"), (64, 1280, 1024, 1088, 0, 1280, "large")])
 def test_error_report_over_the_range_of_fp16(ctx, tile, M, K, N, row0, rows, kind):
     """Whatever the magnitudes: 0 to 4 bytes a value by blocks, just inside and outside of what bytes hold, subnormals,
     infinities, sums at the length where 32 bits end.  Against fp64 on the host (K terms a sum, rows * N in a norm, 2^-53

@@ -96,11 +96,29 @@ def workgroups_of_the_report(e, M, K, N):
     assert blocks <= grid <= 2 * blocks + 8 * 64, "%d workgroups for %d blocks" % (grid, blocks)
 
 
-@pytest.mark.parametrize("shape", [(262144, 512, 64), (64, 512, 262144), (16384, 512, 512), (512, 512, 16384), (4096, 512, 512),
-                                   (4096, 4096, 4096), (576, 1024, 14592), (1088, 512, 4160), (640, 640, 640)])
+@pytest.mark.parametrize("shape", [(65536, 4096, 128), (128, 4096, 65536), (16384, 512, 512), (512, 512, 16384), (4096, 512, 512),
+                                   (4096, 4096, 4096), (576, 1024, 14592), (1088, 512, 4160), (832, 832, 832)])
 def test_the_report_has_a_workgroup_per_block_of_c(run, shape):
     """Of 64 x 64: also where C is narrow, which takes no more of them than the same C the other way round."""
     run("workgroups_of_the_report", *shape)
+
+
+def product_of_the_report(e, M, K, N, whole):
+    h = e.context()
+    resident_operands(e, h, M, K, N, 64)
+    e.launches()
+    e.L.spamm_error_vs_dense_f64(h, ctypes.create_string_buffer(16), i64(0), i64(M), (ctypes.c_double * 3)())
+    assert ("k_limbs" in dict(e.launches())) == bool(whole)
+
+
+@pytest.mark.parametrize("shape", [(1048576, 64, 64), (4096, 64, 4096), (4096, 192, 4096), (65536, 1024, 64), (64, 4096, 131072), (512, 512, 512)])
+def test_reports_that_the_split_would_make_longer_are_left_in_fp64(run, shape):
+    run("product_of_the_report", *shape, 0)
+
+
+@pytest.mark.parametrize("shape", [(4096, 256, 4096), (1024, 1024, 1024), (64, 4096, 4096), (16384, 512, 512), (4096, 4096, 4096)])
+def test_reports_in_whole_numbers(run, shape):
+    run("product_of_the_report", *shape, 1)
 
 
 def launches_of_the_report(e):
