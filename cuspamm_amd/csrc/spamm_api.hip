@@ -74,6 +74,11 @@ struct Workspace {
     DevBuf counts, klist, mask, macro_list, macro_count, macro_work, order, sched, kept;
 };
 
+// Scratch of a report that a context keeps for the next one: that of 8192^3.  A larger one is given back -- to allocate and
+// free it takes 0.3 to 0.7 ms, beside 1.3 to 67 ms of reports of 12288^3 and 16384^3 -- and what is kept goes when another
+// buffer of the context finds no memory.
+constexpr size_t LIMBS_KEPT = ((size_t)512 << 20) + ((size_t)512 << 10);
+
 struct spamm_ctx : Workspace {
     int device = 0;
     hipStream_t own_stream = nullptr;
@@ -94,7 +99,7 @@ struct spamm_ctx : Workspace {
     DevBuf staging;   // read-back staging / decay table
     DevBuf tauws;     // tau selection workspace
     DevBuf reportws;  // error report workspace
-    DevBuf limbs;     // operands split for the error report's integer product
+    DevBuf limbs;     // operands split for the error report's integer product; at most LIMBS_KEPT between calls
     double *tile_results = nullptr;   // pinned, TILE_RESULTS_MAX doubles at most: per-tile results of small outputs
     size_t tile_results_cap = 0;
     HostResults *results = nullptr;   // pinned: small results that a kernel writes and the host waits for
@@ -118,18 +123,30 @@ namespace {
         }                                         \
     } while (0)
 
-int ensure(spamm_ctx *c, DevBuf &b, size_t bytes) {
-    if (bytes == 0) bytes = 16;
-    if (b.cap >= bytes) return SPAMM_OK;
-    if (c->no_alloc) return SPAMM_ELIMIT;       // the carve-out was sized by the same formulas: not reached
+int release(spamm_ctx *c, DevBuf &b) {
     if (b.p && !b.borrowed) {
         HIPCHK(c, hipStreamSynchronize(c->stream));
         HIPCHK(c, hipFree(b.p));
     }
-    b.p = nullptr;
-    b.cap = 0;
-    b.borrowed = false;
-    HIPCHK(c, hipMalloc(&b.p, bytes));
+    b = DevBuf();
+    return SPAMM_OK;
+}
+
+int ensure(spamm_ctx *c, DevBuf &b, size_t bytes) {
+    if (bytes == 0) bytes = 16;
+    if (b.cap >= bytes) return SPAMM_OK;
+    if (c->no_alloc) return SPAMM_ELIMIT;       // the carve-out was sized by the same formulas: not reached
+    int rc = release(c, b);
+    if (rc) return rc;
+    hipError_t e = hipMalloc(&b.p, bytes);
+    if (e == hipErrorOutOfMemory && c->limbs.p && &b != &c->limbs) {        // what a report may need again goes first
+        b.p = nullptr;
+        (void)hipGetLastError();
+        if ((rc = release(c, c->limbs))) return rc;
+        e = hipMalloc(&b.p, bytes);
+    }
+    if (e != hipSuccess) b.p = nullptr;
+    HIPCHK(c, e);
     b.cap = bytes;
     return SPAMM_OK;
 }
@@ -726,7 +743,9 @@ int spamm_error_vs_dense_f64(spamm_ctx *c, const float *dC, int64_t row0, int64_
     // them, in fp64: behind the integer product's launch, which alone knows the values)
     const unsigned long long seq = ++c->seq;
     const size_t limbs = limb_bytes(row1 - row0, c->K, c->N, c->n_cu);
+    const int last_hip = c->last_hip;
     const bool whole = limbs && ensure(c, c->limbs, limbs) == SPAMM_OK;
+    if (!whole) c->last_hip = last_hip;
     if (whole)
         HIPCHK(c, launch_error_limbs(c->packedA.p, c->packedB.p, c->K, c->N, c->tile, dC, row0, row1, c->n_xcd, c->limbs.p, c->reportws.p,
                                      &c->results->report, &c->results->seq, seq, c->stream));
@@ -734,6 +753,7 @@ int spamm_error_vs_dense_f64(spamm_ctx *c, const float *dC, int64_t row0, int64_
                                     &c->results->report, &c->results->seq, seq, whole, c->stream));
     if ((rc = wait_result(c, seq))) return rc;
     for (int i = 0; i < 3; i++) out3[i] = sqrt(c->results->report.v[i]);
+    if (c->limbs.cap > LIMBS_KEPT && (rc = release(c, c->limbs))) return rc;
     return SPAMM_OK;
 }
 

@@ -238,7 +238,10 @@ SPAMM_API int spamm_fill_decay_f32(spamm_ctx *ctx, float *dX, int64_t rows, int6
 /* Error report (check_simple_gpu / COUNTERRTRANS, tool.cu:227-280, 6-24, with an
  * exact fp64 product of the resident fp16 operands instead of cuBLAS):
  * out3 = { ||C - C_dense||_F, ||C_dense||_F, ||C||_F } over rows [row0, row1)
- * (multiples of 64; N a multiple of 64).  The dense product is never stored. */
+ * (multiples of 64; N a multiple of 64).  The dense product is never stored.  Where that is faster it is formed in whole
+ * numbers, from copies of the operands in device memory: 4 bytes for each of (row1 - row0 + N) * K values, 4 GiB at most.
+ * Up to 512 MiB of them stay with the context for the next report, until another of its buffers finds no memory;
+ * without memory for them the product is formed in fp64. */
 SPAMM_API int spamm_error_vs_dense_f64(spamm_ctx *ctx, const float *dC, int64_t row0, int64_t row1,
                                        double *out3);
 /* tau-derived bound on that error: sqrt(sum_ij s_ij^2) with s_ij = sum_{k dropped} nA[i,k]*nB[k,j],

@@ -11,6 +11,7 @@
 namespace {
 
 thread_local int current = 0;
+thread_local hipError_t last_error = hipSuccess;      // until it is asked for
 int expected = 0;
 int n_checked = 0, n_wrong = 0;
 char first_wrong[128];
@@ -33,6 +34,9 @@ struct Config {
 thread_local Config pushed;
 
 std::map<const void *, std::string> kernel_names;
+std::map<std::string, std::pair<int, int>> answers;     // by part of a kernel's name
+std::map<void *, size_t> sizes;                         // of the device's allocations
+size_t held = 0, limit = ~(size_t)0 / 2;
 std::string launched;       // "name grid;" of every launch since fake_launches was last asked
 
 }  // namespace
@@ -51,6 +55,11 @@ const char *fake_launches() {
     return out.c_str();
 }
 
+size_t fake_held() { return held; }
+void fake_limit(size_t bytes) { limit = bytes; }
+// kernels of this name publish a result: their arguments (by number) are where its sequence number goes, and the number
+void fake_answer(const char *name, int host_seq, int seq) { answers[name] = {host_seq, seq}; }
+
 // --- the runtime
 hipError_t hipGetDeviceCount(int *n) { *n = 2; return hipSuccess; }
 hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int) {       // (the header's name for the versioned symbol)
@@ -60,12 +69,27 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int) {       // (the heade
     return hipSuccess;
 }
 hipError_t hipSetDevice(int d) { current = d; return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+    const hipError_t e = last_error;
+    last_error = hipSuccess;
+    return e;
+}
 hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { check("hipFuncSetAttribute", current == expected); return hipSuccess; }
 
-hipError_t hipMalloc(void **p, size_t n) { check("hipMalloc", current == expected); *p = calloc(1, n); return *p ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipMalloc(void **p, size_t n) {
+    check("hipMalloc", current == expected);
+    *p = held + n <= limit ? calloc(1, n) : nullptr;
+    if (!*p) return last_error = hipErrorOutOfMemory;
+    held += sizes[*p] = n;
+    return hipSuccess;
+}
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) { *p = calloc(1, n); return *p ? hipSuccess : hipErrorOutOfMemory; }
-hipError_t hipFree(void *p) { free(p); return hipSuccess; }
+hipError_t hipFree(void *p) {
+    const auto it = sizes.find(p);
+    if (it != sizes.end()) held -= it->second, sizes.erase(it);
+    free(p);
+    return hipSuccess;
+}
 hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) { memcpy(d, s, n); return hipSuccess; }
 hipError_t hipGetSymbolAddress(void **p, const void *) {
@@ -95,7 +119,10 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hi
     *stream = pushed.stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **, size_t, hipStream_t s) {
+hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **args, size_t, hipStream_t s) {
+    for (const auto &a : answers)
+        if (kernel_names[f].find(a.first) != std::string::npos)
+            **(unsigned long long **)args[a.second.first] = *(unsigned long long *)args[a.second.second];
     launched += kernel_names[f] + " " + std::to_string(grid.x) + ";";
     check("hipLaunchKernel", current == expected && (!s || ((Owned *)s)->device == current));
     return hipSuccess;

@@ -1,5 +1,5 @@
 """What the engine's host side launches and allocates, on a runtime of imaginary GPUs (fake_hip.cpp): kernels do nothing
-there, so a call that waits for a kernel's result reports a runtime error.  Each check runs in a process of its own."""
+there, so a call that waits for a kernel's result reports a runtime error, unless the runtime is told to answer for it.  Each check runs in a process of its own."""
 import ctypes
 import os
 import re
@@ -17,6 +17,8 @@ class Engine:
     def __init__(self, fake_path, lib_path):
         self.fake = ctypes.CDLL(fake_path, mode=ctypes.RTLD_GLOBAL)
         self.fake.fake_launches.restype = ctypes.c_char_p
+        self.fake.fake_held.restype = ctypes.c_size_t
+        self.fake.fake_limit.argtypes = [ctypes.c_size_t]
         self.L = ctypes.CDLL(lib_path)
 
     def context(self):
@@ -133,6 +135,56 @@ def launches_of_the_report(e):
 def test_the_report_launches_its_fp64_product_before_it_waits(run):
     """Which of the two products does the work is known on the device alone: the host does not come back for it."""
     run("launches_of_the_report")
+
+
+MIB = 1 << 20
+
+
+def report(e, h, M):
+    e.fake.fake_answer(b"k_error_limbs", 14, 15)
+    e.fake.fake_answer(b"k_error_dense", 11, 12)
+    e.launches()
+    assert e.L.spamm_error_vs_dense_f64(h, ctypes.create_string_buffer(16), i64(0), i64(M), (ctypes.c_double * 3)()) == 0
+    return [name for name, _ in e.launches()]
+
+
+def memory_after_a_report(e, n):
+    h = e.context()
+    resident_operands(e, h, n, n, n, 64)
+    before = e.fake.fake_held()
+    assert "k_limbs" in report(e, h, n)
+    assert e.fake.fake_held() - before <= 513 * MIB, "%d MiB more than before" % ((e.fake.fake_held() - before) // MIB)
+
+
+@pytest.mark.parametrize("n", [2048, 8192, 8256, 16384])
+def test_a_report_gives_its_scratch_back(run, n):
+    run("memory_after_a_report", n)
+
+
+def multiply_on_a_full_card(e):
+    h = e.context()
+    resident_operands(e, h, 4096, 4096, 4096, 64)
+    e.fake.fake_limit(e.fake.fake_held() + 130 * MIB)
+    assert "k_limbs" in report(e, h, 4096)                                  # 128 MiB of scratch, which stay
+    X = ctypes.create_string_buffer(16)
+    assert e.L.spamm_normmap_f32(h, 1, X, i64(4096), i64(8192), 64) == 0    # needs 64 MiB in the place of 32
+    assert e.L.spamm_last_hip_error(h) == 0
+
+
+def test_scratch_of_a_report_goes_when_a_multiply_finds_no_memory(run):
+    run("multiply_on_a_full_card")
+
+
+def report_on_a_full_card(e):
+    h = e.context()
+    resident_operands(e, h, 4096, 4096, 4096, 64)
+    e.fake.fake_limit(e.fake.fake_held() + MIB)
+    assert report(e, h, 4096)[-1] == "k_error_dense"
+    assert e.L.spamm_last_hip_error(h) == 0
+
+
+def test_a_report_without_memory_for_its_scratch_leaves_no_error(run):
+    run("report_on_a_full_card")
 
 
 if __name__ == "__main__":
