@@ -18,8 +18,8 @@
 // that the chip holds under them, about 2 GHz); 1984 x 2176 x 768: 196 -> 158.  In whole numbers instead (one call, its
 // host wait included): 4096^3 2107 -> 867 us on uniform values in [-1, 1) (4 bytes each, 16 products, 2.6 Pop/s: power),
 // 620 where 3 bytes do, 272 on exp(-d / 100); 1984 x 2176 x 768 165 -> 82, 67, 49; 64 rows of 4096^3 173 -> 109, 91, 50.
-// An operand with a value of 127 or more costs both launches for nothing (flags of their own per 16 blocks, no planes
-// behind them, and no host between): 4096^3 2115 -> 2144, 2048^3 316 -> 327, 1280^3 106 -> 111, 1024^3 56 -> 61.6.
+// An operand with a value of 127 or more has been read by k_limbs for nothing, which writes no planes then, and blocks of 64 x 64
+// of C are formed in fp64 by k_error_limbs itself: 1024^3 56 -> 59.5 us, 1280^3 106 -> 111, 4096^3 2121 -> 2106.
 // The scalar bound of 64 x 64 x 64 tiles 52 -> 7 us, the per-tile one 51 -> 4; results go straight to host memory (a
 // clearing launch before and a copy after each were 25 us a call).
 #include "gemm_device.h"
@@ -30,21 +30,23 @@ namespace spamm {
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half8t __attribute__((ext_vector_type(8)));
 
-constexpr int RANGE_FLAGS = 16;         // (stores to one address queue: 32768 waves that all found such values took 0.6 ms)
+// Stores to one address queue (32768 waves that all found such values took 0.6 ms): a workgroup sets one of 16 flags, unless
+// it finds it set, and who set that first the one that is read.
+constexpr int RANGE_FLAGS = 16;
 struct alignas(128) RangeFlag {
     unsigned long long call;
 };
 
 struct ReportWorkspace {
     Tickets tickets;                    // workgroups of the running launch that have finished; zero between launches
-    RangeFlag range[RANGE_FLAGS];       // k_limbs: the last call of which an operand held values without limbs
+    RangeFlag range[1 + RANGE_FLAGS];   // k_limbs: the last call of which an operand held values without limbs
     double part[1];                     // per workgroup: its sums (report_workspace_bytes says how many)
 };
 
-// Whether an operand of this call held values that k_limbs has no limbs for.  (By the call's number: the flags are never
-// put back, so a launch that finds its call done may look at them while a later call, on another stream, sets its own.)
+// Whether an operand of this call held values that k_limbs has no limbs for.  (By the call's number: the flags need not be
+// put back.)
 __device__ __forceinline__ bool out_of_range(const ReportWorkspace *ws, unsigned long long call) {
-    return __ballot(agent_load(&ws->range[threadIdx.x % RANGE_FLAGS].call) == call) != 0ull;
+    return ws->range[0].call == call;
 }
 
 // Sums of all workgroups' N values, by the workgroup that finishes last, to host_out (pinned host memory): in a
@@ -84,89 +86,92 @@ __device__ __forceinline__ void finish_sums(ReportWorkspace *ws, double own, Rep
 // operand block for 32 k, and element e of the vectors makes MFMA step e.  Which k goes to which step is the same for A
 // and B, and the sum over k does not care.  fp16 -> fp64 is exact.
 template <int NBR, int NBC>
+__device__ __forceinline__ void dense_block(const _Float16 *__restrict__ pA, const _Float16 *__restrict__ pB, int64_t K, int64_t N, int tile,
+                                            const float *__restrict__ C, int64_t br, int64_t bc, double &e2, double &d2, double &c2) {
+    const int lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
+    const int64_t nbK = K / tile, tile_halves = (int64_t)tile * tile;
+    const _Float16 *srcA[NBR], *srcB[NBC];
+#pragma unroll
+    for (int t = 0; t < NBR; t++) {
+        const int64_t r = br + t * 16 + l16;
+        srcA[t] = pA + (r / tile) * nbK * tile_halves + (r % tile) * 8 + (int64_t)q * tile * 8;
+    }
+#pragma unroll
+    for (int t = 0; t < NBC; t++) {
+        const int64_t c = bc + t * 16 + l16;
+        srcB[t] = pB + (c / tile) * nbK * tile_halves + (c % tile) * 8 + (int64_t)q * tile * 8;
+    }
+    f64x4 acc[NBR][NBC];
+#pragma unroll
+    for (int a = 0; a < NBR; a++)
+#pragma unroll
+        for (int b = 0; b < NBC; b++) acc[a][b] = f64x4{0.0, 0.0, 0.0, 0.0};
+    struct Vecs {
+        half8t a[NBR], b[NBC];
+    };
+    // four k-groups are 32 * tile halves, and a tile's are followed by the next k tile's
+    const int64_t steps = K / 32, stride = (int64_t)32 * tile;
+    auto load = [&](Vecs &v, int64_t s) {
+        const int64_t off = (s < steps ? s : steps - 1) * stride;
+#pragma unroll
+        for (int t = 0; t < NBR; t++) v.a[t] = *reinterpret_cast<const half8t *>(srcA[t] + off);
+#pragma unroll
+        for (int t = 0; t < NBC; t++) v.b[t] = *reinterpret_cast<const half8t *>(srcB[t] + off);
+    };
+    auto multiply = [&](const Vecs &v) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            double a[NBR], b[NBC];
+#pragma unroll
+            for (int t = 0; t < NBR; t++) a[t] = (double)(float)v.a[t][e];
+#pragma unroll
+            for (int t = 0; t < NBC; t++) b[t] = (double)(float)v.b[t][e];
+#pragma unroll
+            for (int ta = 0; ta < NBR; ta++)
+#pragma unroll
+                for (int tb = 0; tb < NBC; tb++)
+                    acc[ta][tb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ta], b[tb], acc[ta][tb], 0, 0, 0);
+        }
+    };
+    Vecs v0, v1;
+    load(v0, 0);
+    int64_t s = 0;
+    for (; s + 1 < steps; s += 2) {
+        load(v1, s + 1);
+        multiply(v0);
+        load(v0, s + 2);
+        multiply(v1);
+    }
+    if (s < steps) multiply(v0);
+    // accumulator i of lane l in block (ta, tb): row 4 i + l / 16, column l % 16
+#pragma unroll
+    for (int ta = 0; ta < NBR; ta++)
+#pragma unroll
+        for (int tb = 0; tb < NBC; tb++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const double c = (double)C[(br + ta * 16 + 4 * i + q) * N + bc + tb * 16 + l16];
+                const double d = acc[ta][tb][i];
+                e2 += (c - d) * (c - d);
+                d2 += d * d;
+                c2 += c * c;
+            }
+}
+
+template <int NBR, int NBC>
 __global__ __launch_bounds__(256, NBR * NBC > 8 ? 2 : 3) void k_error_dense(const _Float16 *__restrict__ pA, const _Float16 *__restrict__ pB,
                                                                         int64_t K, int64_t N, int tile, const float *__restrict__ C,
                                                                         int64_t row0, int64_t row1, int nwg_n,
                                                                         ReportWorkspace *__restrict__ ws, ReportSums *__restrict__ host_out,
-                                                                        unsigned long long *__restrict__ host_seq, unsigned long long seq,
-                                                                        bool behind_limbs) {
-    // behind k_error_limbs, which has already published the result unless the operands' values were too large for it
-    if (behind_limbs && !out_of_range(ws, seq)) return;
+                                                                        unsigned long long *__restrict__ host_seq, unsigned long long seq) {
     __shared__ double red[4][3];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wr = wave >> 1, wc = wave & 1;
     const int64_t br = row0 + (int64_t)(blockIdx.x / nwg_n) * (NBR * 32) + wr * (NBR * 16);
     const int64_t bc = (int64_t)(blockIdx.x % nwg_n) * (NBC * 32) + wc * (NBC * 16);
-    const int l16 = lane & 15, q = lane >> 4;
     double e2 = 0, d2 = 0, c2 = 0;
     if (br < row1 && bc < N) {              // (whole blocks: rows and columns come in multiples of 64)
-        const int64_t nbK = K / tile, tile_halves = (int64_t)tile * tile;
-        const _Float16 *srcA[NBR], *srcB[NBC];
-#pragma unroll
-        for (int t = 0; t < NBR; t++) {
-            const int64_t r = br + t * 16 + l16;
-            srcA[t] = pA + (r / tile) * nbK * tile_halves + (r % tile) * 8 + (int64_t)q * tile * 8;
-        }
-#pragma unroll
-        for (int t = 0; t < NBC; t++) {
-            const int64_t c = bc + t * 16 + l16;
-            srcB[t] = pB + (c / tile) * nbK * tile_halves + (c % tile) * 8 + (int64_t)q * tile * 8;
-        }
-        f64x4 acc[NBR][NBC];
-#pragma unroll
-        for (int a = 0; a < NBR; a++)
-#pragma unroll
-            for (int b = 0; b < NBC; b++) acc[a][b] = f64x4{0.0, 0.0, 0.0, 0.0};
-        struct Vecs {
-            half8t a[NBR], b[NBC];
-        };
-        // four k-groups are 32 * tile halves, and a tile's are followed by the next k tile's
-        const int64_t steps = K / 32, stride = (int64_t)32 * tile;
-        auto load = [&](Vecs &v, int64_t s) {
-            const int64_t off = (s < steps ? s : steps - 1) * stride;
-#pragma unroll
-            for (int t = 0; t < NBR; t++) v.a[t] = *reinterpret_cast<const half8t *>(srcA[t] + off);
-#pragma unroll
-            for (int t = 0; t < NBC; t++) v.b[t] = *reinterpret_cast<const half8t *>(srcB[t] + off);
-        };
-        auto multiply = [&](const Vecs &v) {
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                double a[NBR], b[NBC];
-#pragma unroll
-                for (int t = 0; t < NBR; t++) a[t] = (double)(float)v.a[t][e];
-#pragma unroll
-                for (int t = 0; t < NBC; t++) b[t] = (double)(float)v.b[t][e];
-#pragma unroll
-                for (int ta = 0; ta < NBR; ta++)
-#pragma unroll
-                    for (int tb = 0; tb < NBC; tb++)
-                        acc[ta][tb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ta], b[tb], acc[ta][tb], 0, 0, 0);
-            }
-        };
-        Vecs v0, v1;
-        load(v0, 0);
-        int64_t s = 0;
-        for (; s + 1 < steps; s += 2) {
-            load(v1, s + 1);
-            multiply(v0);
-            load(v0, s + 2);
-            multiply(v1);
-        }
-        if (s < steps) multiply(v0);
-        // accumulator i of lane l in block (ta, tb): row 4 i + l / 16, column l % 16
-#pragma unroll
-        for (int ta = 0; ta < NBR; ta++)
-#pragma unroll
-            for (int tb = 0; tb < NBC; tb++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const double c = (double)C[(br + ta * 16 + 4 * i + q) * N + bc + tb * 16 + l16];
-                    const double d = acc[ta][tb][i];
-                    e2 += (c - d) * (c - d);
-                    d2 += d * d;
-                    c2 += c * c;
-                }
+        dense_block<NBR, NBC>(pA, pB, K, N, tile, C, br, bc, e2, d2, c2);
         for (int off = 32; off > 0; off >>= 1) {
             e2 += __shfl_down(e2, off, 64);
             d2 += __shfl_down(d2, off, 64);
@@ -244,8 +249,10 @@ __global__ __launch_bounds__(256) void k_limbs(LimbOperand a, LimbOperand b, int
     }
     __syncthreads();
     if (!(s_fits[0] && s_fits[1] && s_fits[2] && s_fits[3])) {          // nothing will read the planes
-        unsigned long long *flag = &ws->range[blockIdx.x % RANGE_FLAGS].call;
-        if (threadIdx.x == 0 && agent_load(flag) != call) agent_store(flag, call);
+        unsigned long long *flag = &ws->range[1 + blockIdx.x % RANGE_FLAGS].call;
+        if (threadIdx.x == 0 && agent_load(flag) != call &&
+            __hip_atomic_exchange(flag, call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != call)
+            agent_store(&ws->range[0].call, call);
         return;
     }
     used = s_used[0] | s_used[1] | s_used[2] | s_used[3];
@@ -279,11 +286,16 @@ constexpr int LIMB_MAX_KB = 32768 / LIMB_BLOCK;
 
 __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict__ plA, const uint8_t *__restrict__ clsA,
                                                         const int8_t *__restrict__ plB, const uint8_t *__restrict__ clsB, int nkb,
-                                                        int nbi, int nbj, int gb, int ngj, int n_xcd, int64_t N,
-                                                        const float *__restrict__ C, ReportWorkspace *__restrict__ ws,
+                                                        int nbi, int nbj, int gb, int ngj, int n_xcd, const _Float16 *__restrict__ pA,
+                                                        const _Float16 *__restrict__ pB, int64_t K, int64_t N, int tile,
+                                                        const float *__restrict__ C, int64_t row0, ReportWorkspace *__restrict__ ws,
                                                         ReportSums *__restrict__ host_out, unsigned long long *__restrict__ host_seq,
-                                                        unsigned long long seq) {
-    if (out_of_range(ws, seq)) return;          // (k_error_dense comes behind this launch)
+                                                        unsigned long long seq, bool dense_here) {
+    const bool fp64 = out_of_range(ws, seq);
+    if (fp64 && !dense_here) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) publish_result(host_out, ReportSums{{-1.0, 0.0, 0.0}}, host_seq, seq);
+        return;
+    }
     __shared__ double red[4][3];
     __shared__ int s_count[17], s_place[16];
     __shared__ uint16_t s_list[LIMB_MAX_KB];
@@ -294,7 +306,9 @@ __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict
     const int gi = (group * n_xcd + x) / ngj, gj = ((group * n_xcd + x) % ngj + 2 * (ngj - gi % ngj)) % ngj;
     const int bi = gi * gb + in_group / gb, bj = gj * gb + in_group % gb;
     double e2 = 0, d2 = 0, c2 = 0;
-    if (bi < nbi && bj < nbj) {
+    if (bi < nbi && bj < nbj && fp64) {
+        dense_block<2, 2>(pA, pB, K, N, tile, C, row0 + (int64_t)bi * LIMB_BLOCK + wr * 32, (int64_t)bj * LIMB_BLOCK + wc * 32, e2, d2, c2);
+    } else if (bi < nbi && bj < nbj) {
         // ---- k blocks by kind
         if (threadIdx.x < 17) s_count[threadIdx.x] = 0;
         __syncthreads();
@@ -379,7 +393,7 @@ __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict
         });
         // accumulator i of lane l in block t: row 4 (l / 16) + i, column l % 16; orders 0 to 3 and 4 to 6 are added in
         // 64-bit integers, so the one rounding is the last
-        const float *src = C + ((int64_t)bi * LIMB_BLOCK + wr * 32 + 4 * q) * N + (int64_t)bj * LIMB_BLOCK + wc * 32 + l16;
+        const float *src = C + (row0 + (int64_t)bi * LIMB_BLOCK + wr * 32 + 4 * q) * N + (int64_t)bj * LIMB_BLOCK + wc * 32 + l16;
 #pragma unroll
         for (int t = 0; t < 4; t++)
 #pragma unroll
@@ -394,11 +408,11 @@ __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict
                 d2 += d * d;
                 c2 += c * c;
             }
-        for (int off = 32; off > 0; off >>= 1) {
-            e2 += __shfl_down(e2, off, 64);
-            d2 += __shfl_down(d2, off, 64);
-            c2 += __shfl_down(c2, off, 64);
-        }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        e2 += __shfl_down(e2, off, 64);
+        d2 += __shfl_down(d2, off, 64);
+        c2 += __shfl_down(c2, off, 64);
     }
     if (lane == 0) {
         red[wave][0] = e2;
@@ -463,7 +477,7 @@ __global__ __launch_bounds__(256) void k_dropped_bound(const float *__restrict__
 
 __global__ void k_clear_report(ReportWorkspace *ws) {
     if (threadIdx.x <= TICKET_GROUPS) ws->tickets.t[threadIdx.x].n = 0;
-    if (threadIdx.x < RANGE_FLAGS) ws->range[threadIdx.x].call = 0;
+    if (threadIdx.x <= RANGE_FLAGS) ws->range[threadIdx.x].call = 0;
 }
 
 hipError_t launch_clear_report(void *workspace, hipStream_t s) {
@@ -519,24 +533,26 @@ static LimbGrid limb_grid(int64_t rows, int64_t N, int n_xcd) {
 static int64_t limb_kb(int64_t K) { return (K + LIMB_BLOCK - 1) / LIMB_BLOCK; }
 
 // Bytes of the planes and the blocks' numbers of limbs of both operands; 0: the fp64 pipeline is to be used -- beyond
-// what 32 bits add up, beyond 4 GiB of planes, and where the split of the operands, which no block of C shares, is more than
-// a quarter of the fp64 product's time.  Both are estimated in us: of the split its launches and 3 TB/s of operands, of the product
-// 0.033 per MFMA of its fullest SIMD (4096^3 2112, 1280^3 94, 64 rows of 4096^2 151).  fp64 -> whole numbers, whole calls, on
-// uniform values | exp(-d / 100) | values too large for limbs, by the estimates' ratio: 2.8, 1024 x 512 x 1024 39.0 -> 39.2 | 36.2
-// | 43.1 and 64 x 1024 x 65536 160 -> 173 | 66 | 224; 3.6, 640^3 41 -> 39.7 | 37.9 | 47.0; 4.2, 256 x 1024 x 4096 57 -> 53 | 45 | 66.5
-// and 768^3 46 -> 44.1 | 41.2 | 51.6; 5.1, 1024^3 57 -> 50 | 45.5 | 61.7; 10, 65536 x 512 x 256 289 -> 186 | 87 | 311.  With K
-// below 256 a block's fixed costs outweigh its few products: 4096 x 64 x 4096 61 -> 82 | 73 | 68, K = 128 94 -> 94 | 74 | 102,
-// K = 256 159 -> 119 | 79 | 168.
+// what 32 bits add up, beyond 4 GiB of planes, and where the split of the operands, which no block of C shares, takes more than
+// 1 / 2.4 of the fp64 product's time.  Both are estimated, in us: of the product 0.033 per MFMA of its fullest SIMD (4096^3 2112,
+// 1280^3 94, 64 rows of 4096^2 151), of the split 6 for its launches, two passes over 2 bytes a value at 3 TB/s, and the
+// scratch's allocation where the context does not keep it.  fp64 -> whole numbers, whole calls, on uniform values | exp(-d / 100) |
+// values too large for limbs, by the estimates' ratio: 1.5, 65536 x 1024 x 64 155 -> 178 | 69 | 185; 2.2, 512 x 384 x 512
+// 31.2 -> 32.2 | 31.8 | 35.8; 2.5, 4096 x 256 x 512 38 -> 35.8 | 31.0 | 43.2 and 1024 x 512 x 1024 39.2 -> 38.5 | 35.8 | 41.2;
+// 2.8, 512^3 35.9 -> 34.9 | 33.9 | 40.1 and 65536 x 512 x 128 158 -> 120 | 62 | 172; 3.9, 1024^3 57 -> 49.4 | 44.4 | 59.5; 7.6,
+// 65536 x 512 x 256 289 -> 186 | 87 | 311; 10, 1280^3 106 -> 64 | 55 | 111.  With K below 256 a block's fixed costs outweigh its
+// few products: 4096 x 64 x 4096 61 -> 82 | 73 | 68, K = 128 94 -> 94 | 74 | 102, K = 256 158 -> 118 | 79 | 164.
 size_t limb_bytes(int64_t rows, int64_t K, int64_t N, int n_cu) {
     if (K > LIMB_MAX_K || K < 256) return 0;
+    const size_t blocks = (size_t)(rows / LIMB_BLOCK + N / LIMB_BLOCK) * (size_t)limb_kb(K);
+    if (blocks >= (1u << 31) / (LIMBS * LIMB_PLANE / 2)) return 0;       // 4 GiB
+    const size_t bytes = blocks * (LIMBS * LIMB_PLANE) + blocks;
     int64_t n_wg = 0;
     double mfmas = 0.0;
     (void)error_shape(rows, N, n_cu, &n_wg, &mfmas);
-    const double dense = 0.033 * mfmas * (double)(K / 4), split = 6.0 + (double)(rows + N) * (double)K * 2.0 / 3.0e6;
-    if (dense < 4.0 * split) return 0;
-    const size_t blocks = (size_t)(rows / LIMB_BLOCK + N / LIMB_BLOCK) * (size_t)limb_kb(K);
-    if (blocks >= (1u << 31) / (LIMBS * LIMB_PLANE / 2)) return 0;       // 4 GiB
-    return blocks * (LIMBS * LIMB_PLANE) + blocks;
+    const double dense = 0.033 * mfmas * (double)(K / 4);
+    const double split = 6.0 + (double)(rows + N) * (double)K * 4.0 / 3.0e6 + (bytes > LIMBS_KEPT ? 500.0 : 0.0);
+    return dense < 2.4 * split ? 0 : bytes;
 }
 
 size_t report_workspace_bytes(int64_t rows, int64_t N, int n_cu, int n_xcd) {
@@ -552,14 +568,14 @@ size_t report_workspace_bytes(int64_t rows, int64_t N, int n_cu, int n_xcd) {
 
 hipError_t launch_error_vs_dense(const void *packedA, const void *packedB, int64_t K, int64_t N, int tile, const float *C,
                                  int64_t row0, int64_t row1, int n_cu, void *workspace, ReportSums *host_out,
-                                 unsigned long long *host_seq, unsigned long long seq, bool behind_limbs, hipStream_t s) {
+                                 unsigned long long *host_seq, unsigned long long seq, hipStream_t s) {
     int64_t n_wg = 0;
     const int shape = error_shape(row1 - row0, N, n_cu, &n_wg);
     const _Float16 *pA = (const _Float16 *)packedA, *pB = (const _Float16 *)packedB;
     ReportWorkspace *ws = (ReportWorkspace *)workspace;
     const int nwg_n = (int)((N + 32 * ERROR_SHAPES[shape].nbc - 1) / (32 * ERROR_SHAPES[shape].nbc));
 #define SPAMM_DENSE(NBR, NBC) \
-    k_error_dense<NBR, NBC><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out, host_seq, seq, behind_limbs)
+    k_error_dense<NBR, NBC><<<(unsigned)n_wg, 256, 0, s>>>(pA, pB, K, N, tile, C, row0, row1, nwg_n, ws, host_out, host_seq, seq)
     if (shape == 0) SPAMM_DENSE(4, 4);
     else if (shape == 1) SPAMM_DENSE(4, 2);
     else SPAMM_DENSE(2, 2);
@@ -568,21 +584,26 @@ hipError_t launch_error_vs_dense(const void *packedA, const void *packedB, int64
 }
 
 hipError_t launch_error_limbs(const void *packedA, const void *packedB, int64_t K, int64_t N, int tile, const float *C,
-                              int64_t row0, int64_t row1, int n_xcd, void *limbs, void *workspace, ReportSums *host_out,
+                              int64_t row0, int64_t row1, int n_cu, int n_xcd, void *limbs, void *workspace, ReportSums *host_out,
                               unsigned long long *host_seq, unsigned long long seq, hipStream_t s) {
     const LimbGrid g = limb_grid(row1 - row0, N, n_xcd);
     const int nkb = (int)limb_kb(K);
     const int64_t blocksA = (int64_t)g.nbi * nkb, blocksB = (int64_t)g.nbj * nkb;
+    const _Float16 *pA = (const _Float16 *)packedA, *pB = (const _Float16 *)packedB;
     ReportWorkspace *ws = (ReportWorkspace *)workspace;
     int8_t *planes = (int8_t *)limbs;
     uint8_t *cls = (uint8_t *)limbs + (blocksA + blocksB) * (LIMBS * LIMB_PLANE);
-    const LimbOperand a = {(const _Float16 *)packedA, planes, cls, row0, blocksA};
-    const LimbOperand b = {(const _Float16 *)packedB, planes + blocksA * (LIMBS * LIMB_PLANE), cls + blocksA, 0, blocksB};
+    const LimbOperand a = {pA, planes, cls, row0, blocksA};
+    const LimbOperand b = {pB, planes + blocksA * (LIMBS * LIMB_PLANE), cls + blocksA, 0, blocksB};
     k_limbs<<<(unsigned)(blocksA + blocksB), 256, 0, s>>>(a, b, K, tile, nkb, seq, ws);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    k_error_limbs<<<(unsigned)g.n_wg, 256, 0, s>>>(a.planes, a.cls, b.planes, b.cls, nkb, g.nbi, g.nbj, g.gb, g.ngj, n_xcd, N,
-                                                   C + row0 * N, ws, host_out, host_seq, seq);
+    // Where fp64 takes larger blocks of C than 64 x 64 the host launches it when it is told to: some 10 us beside the 300
+    // and more of such a product.  (Launched behind every call of these sizes it was 4 us on the next one.)
+    int64_t n_wg = 0;
+    const bool dense_here = error_shape(row1 - row0, N, n_cu, &n_wg) == 2;
+    k_error_limbs<<<(unsigned)g.n_wg, 256, 0, s>>>(a.planes, a.cls, b.planes, b.cls, nkb, g.nbi, g.nbj, g.gb, g.ngj, n_xcd, pA, pB, K, N,
+                                                   tile, C, row0, ws, host_out, host_seq, seq, dense_here);
     return hipGetLastError();
 }
 

@@ -74,11 +74,6 @@ struct Workspace {
     DevBuf counts, klist, mask, macro_list, macro_count, macro_work, order, sched, kept;
 };
 
-// Scratch of a report that a context keeps for the next one: that of 8192^3.  A larger one is given back -- to allocate and
-// free it takes 0.3 to 0.7 ms, beside 1.3 to 67 ms of reports of 12288^3 and 16384^3 -- and what is kept goes when another
-// buffer of the context finds no memory.
-constexpr size_t LIMBS_KEPT = ((size_t)512 << 20) + ((size_t)512 << 10);
-
 struct spamm_ctx : Workspace {
     int device = 0;
     hipStream_t own_stream = nullptr;
@@ -712,7 +707,7 @@ static int ensure_results(spamm_ctx *c) {
 // Waits for result `seq`, which the last kernel of the call writes when it has done all else -- its writes to the
 // context's workspaces have arrived, so that the next call may use them from another stream -- a few microseconds
 // sooner than the stream is reported idle.  If the stream ends, or fails, without it, the call has failed.  (A
-// bisection and an error report may have a launch behind the one that ended them, which only looks whether it has anything to do.)
+// bisection may have a launch behind the one that ended it, which only looks whether it has anything to do.)
 static int wait_result(spamm_ctx *c, unsigned long long seq) {
     for (int i = 0; i < 50000; i++)           // (some 100 us)
         if (__atomic_load_n(&c->results->seq, __ATOMIC_ACQUIRE) == seq) return SPAMM_OK;
@@ -740,18 +735,25 @@ int spamm_error_vs_dense_f64(spamm_ctx *c, const float *dC, int64_t row0, int64_
     if (rc) return rc;
     if ((rc = report_prepare(c, row1 - row0))) return rc;
     // exact in whole numbers where the operands' values allow it and their planes fit (else, and without memory for
-    // them, in fp64: behind the integer product's launch, which alone knows the values)
-    const unsigned long long seq = ++c->seq;
+    // them, in fp64)
     const size_t limbs = limb_bytes(row1 - row0, c->K, c->N, c->n_cu);
     const int last_hip = c->last_hip;
-    const bool whole = limbs && ensure(c, c->limbs, limbs) == SPAMM_OK;
-    if (!whole) c->last_hip = last_hip;
-    if (whole)
-        HIPCHK(c, launch_error_limbs(c->packedA.p, c->packedB.p, c->K, c->N, c->tile, dC, row0, row1, c->n_xcd, c->limbs.p, c->reportws.p,
-                                     &c->results->report, &c->results->seq, seq, c->stream));
-    HIPCHK(c, launch_error_vs_dense(c->packedA.p, c->packedB.p, c->K, c->N, c->tile, dC, row0, row1, c->n_cu, c->reportws.p,
-                                    &c->results->report, &c->results->seq, seq, whole, c->stream));
-    if ((rc = wait_result(c, seq))) return rc;
+    bool whole = limbs && ensure(c, c->limbs, limbs) == SPAMM_OK;
+    if (whole) {
+        const unsigned long long seq = ++c->seq;
+        HIPCHK(c, launch_error_limbs(c->packedA.p, c->packedB.p, c->K, c->N, c->tile, dC, row0, row1, c->n_cu, c->n_xcd, c->limbs.p,
+                                     c->reportws.p, &c->results->report, &c->results->seq, seq, c->stream));
+        if ((rc = wait_result(c, seq))) return rc;
+        whole = !(c->results->report.v[0] < 0.0);
+    } else {
+        c->last_hip = last_hip;
+    }
+    if (!whole) {
+        const unsigned long long seq = ++c->seq;
+        HIPCHK(c, launch_error_vs_dense(c->packedA.p, c->packedB.p, c->K, c->N, c->tile, dC, row0, row1, c->n_cu, c->reportws.p,
+                                        &c->results->report, &c->results->seq, seq, c->stream));
+        if ((rc = wait_result(c, seq))) return rc;
+    }
     for (int i = 0; i < 3; i++) out3[i] = sqrt(c->results->report.v[i]);
     if (c->limbs.cap > LIMBS_KEPT && (rc = release(c, c->limbs))) return rc;
     return SPAMM_OK;

@@ -107,13 +107,17 @@ size_t report_workspace_bytes(int64_t rows, int64_t N, int n_cu, int n_xcd);    
 hipError_t launch_clear_report(void *workspace, hipStream_t s);
 hipError_t launch_error_vs_dense(const void *packedA, const void *packedB, int64_t K, int64_t N, int tile, const float *C,
                                  int64_t row0, int64_t row1, int n_cu, void *workspace, ReportSums *host_out,
-                                 unsigned long long *host_seq, unsigned long long seq, bool behind_limbs, hipStream_t s);
-// the same on the integer matrix pipeline; limbs: limb_bytes() of scratch (0: not for this shape).  It publishes nothing if an
-// operand holds values that it cannot take (beyond +-127, inf, NaN): launch_error_vs_dense with the same seq and behind_limbs
-// follows it, and does nothing otherwise
+                                 unsigned long long *host_seq, unsigned long long seq, hipStream_t s);
+// the same on the integer matrix pipeline; limbs: limb_bytes() of scratch (0: not for this shape).  Where an operand holds
+// values that it cannot take (beyond +-127, inf, NaN) it forms small blocks of C in fp64 itself; a first sum below zero asks
+// for launch_error_vs_dense, whose blocks are larger
 size_t limb_bytes(int64_t rows, int64_t K, int64_t N, int n_cu);
+// Scratch of a report that a context keeps for the next one: that of 8192^3.  A larger one is given back -- to allocate and
+// free it takes 0.3 to 0.7 ms, beside 1.3 to 67 ms of reports of 12288^3 and 16384^3 -- and what is kept goes when another
+// buffer of the context finds no memory.
+constexpr size_t LIMBS_KEPT = ((size_t)512 << 20) + ((size_t)512 << 10);
 hipError_t launch_error_limbs(const void *packedA, const void *packedB, int64_t K, int64_t N, int tile, const float *C,
-                              int64_t row0, int64_t row1, int n_xcd, void *limbs, void *workspace, ReportSums *host_out,
+                              int64_t row0, int64_t row1, int n_cu, int n_xcd, void *limbs, void *workspace, ReportSums *host_out,
                               unsigned long long *host_seq, unsigned long long seq, hipStream_t s);
 // host_out->v[0] (optional) = sum over tiles of s_ij^2, s_ij = sum_{k dropped} nA[i,k]*nB[k,j]; per_tile (optional): s_ij
 hipError_t launch_dropped_bound(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, float tau,

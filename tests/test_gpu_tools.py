@@ -352,7 +352,8 @@ def test_error_report_by_any_block_shape(ctx, rows, N, row0):
     (64, 8256, 2048, 128, 64, 8192, "limbs"), (64, 576, 1024, 14592, 0, 576, "unit"),        # blocks of C one or few across, or high
     (64, 320, 192, 320, 0, 320, "inf"), (32, 256, 256, 256, 0, 256, "zero"),
     (64, 1280, 1024, 1088, 0, 1280, "inf"), (32, 1184, 1056, 1280, 64, 1088, "nan"), (128, 1280, 1024, 1280, 0, 1280, "zero"),
-    (32, 1344, 1056, 1280, 64, 1280, "unit"), (64, 1280, 1024, 1088, 0, 1280, "large")])
+    (32, 1344, 1056, 1280, 64, 1280, "unit"), (64, 1280, 1024, 1088, 0, 1280, "large"),
+    (128, 2048, 512, 2048, 0, 2048, "large"), (32, 2048, 544, 2112, 64, 1984, "inf")])
 def test_error_report_over_the_range_of_fp16(ctx, tile, M, K, N, row0, rows, kind):
     """Whatever the magnitudes: 0 to 4 bytes a value by blocks, just inside and outside of what bytes hold, subnormals,
     infinities, sums at the length where 32 bits end.  Against fp64 on the host (K terms a sum, rows * N in a norm, 2^-53
@@ -396,11 +397,11 @@ def test_error_report_over_the_range_of_fp16(ctx, tile, M, K, N, row0, rows, kin
             assert abs(g - ref) <= 1e-9 * ref
 
 
-def test_error_reports_of_small_and_large_values_by_turns(ctx):
-    """The integer product has the fp64 one behind it, which does nothing unless values were too large: report after
+@pytest.mark.parametrize("M,K,N,tile", [(1280, 1024, 1088, 64), (2048, 512, 2048, 128)])
+def test_error_reports_of_small_and_large_values_by_turns(ctx, M, K, N, tile):
+    """Values that are too large are taken by the integer product's launch, or by another when it has said so: report after
     report, of one kind and the other, each on another stream than the last and none waited for."""
     import torch
-    M, K, N, tile = 1280, 1024, 1088, 64
     rng = np.random.default_rng(5)
     A, B = rng.uniform(-1.0, 1.0, (M, K)).astype(np.float16), rng.uniform(-1.0, 1.0, (K, N)).astype(np.float16)
     C = rng.uniform(-1.0, 1.0, (M, N)).astype(np.float32)

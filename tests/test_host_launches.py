@@ -98,7 +98,7 @@ def workgroups_of_the_report(e, M, K, N):
     assert blocks <= grid <= 2 * blocks + 8 * 64, "%d workgroups for %d blocks" % (grid, blocks)
 
 
-@pytest.mark.parametrize("shape", [(65536, 4096, 128), (128, 4096, 65536), (16384, 512, 512), (512, 512, 16384), (4096, 512, 512),
+@pytest.mark.parametrize("shape", [(65536, 1024, 128), (128, 1024, 65536), (16384, 512, 512), (512, 512, 16384), (4096, 512, 512),
                                    (4096, 4096, 4096), (576, 1024, 14592), (1088, 512, 4160), (832, 832, 832)])
 def test_the_report_has_a_workgroup_per_block_of_c(run, shape):
     """Of 64 x 64: also where C is narrow, which takes no more of them than the same C the other way round."""
@@ -113,35 +113,21 @@ def product_of_the_report(e, M, K, N, whole):
     assert ("k_limbs" in dict(e.launches())) == bool(whole)
 
 
-@pytest.mark.parametrize("shape", [(1048576, 64, 64), (4096, 64, 4096), (4096, 192, 4096), (65536, 1024, 64), (64, 4096, 131072), (512, 512, 512)])
+@pytest.mark.parametrize("shape", [(1048576, 64, 64), (4096, 64, 4096), (4096, 192, 4096), (65536, 1024, 64), (64, 4096, 131072), (65536, 2048, 128), (512, 256, 512)])
 def test_reports_that_the_split_would_make_longer_are_left_in_fp64(run, shape):
     run("product_of_the_report", *shape, 0)
 
 
-@pytest.mark.parametrize("shape", [(4096, 256, 4096), (1024, 1024, 1024), (64, 4096, 4096), (16384, 512, 512), (4096, 4096, 4096)])
+@pytest.mark.parametrize("shape", [(4096, 256, 4096), (512, 512, 512), (1024, 1024, 1024), (64, 4096, 4096), (16384, 512, 512), (4096, 4096, 4096)])
 def test_reports_in_whole_numbers(run, shape):
     run("product_of_the_report", *shape, 1)
-
-
-def launches_of_the_report(e):
-    h = e.context()
-    resident_operands(e, h, 2048, 2048, 2048, 64)
-    out = (ctypes.c_double * 3)()
-    e.launches()
-    assert e.L.spamm_error_vs_dense_f64(h, ctypes.create_string_buffer(16), i64(0), i64(2048), out) == -3
-    assert [name for name, _ in e.launches()][-3:] == ["k_limbs", "k_error_limbs", "k_error_dense"]
-
-
-def test_the_report_launches_its_fp64_product_before_it_waits(run):
-    """Which of the two products does the work is known on the device alone: the host does not come back for it."""
-    run("launches_of_the_report")
 
 
 MIB = 1 << 20
 
 
 def report(e, h, M):
-    e.fake.fake_answer(b"k_error_limbs", 14, 15)
+    e.fake.fake_answer(b"k_error_limbs", 19, 20)
     e.fake.fake_answer(b"k_error_dense", 11, 12)
     e.launches()
     assert e.L.spamm_error_vs_dense_f64(h, ctypes.create_string_buffer(16), i64(0), i64(M), (ctypes.c_double * 3)()) == 0
