@@ -72,6 +72,7 @@ struct KeptProducts {
 struct GateBuffers {
     const float *nA;        // [nbM x nbK]
     const float *nBt;       // [nbN x nbK]  (transposed B norm map)
+    KeptProducts *kept;
     int32_t *counts;        // [nbM*nbN]
     uint64_t *mask;         // [nbM*nbN*words]
     MacroEntry *macro_list; // [n_macro*nbK]   union list of k per macro tile
@@ -80,7 +81,6 @@ struct GateBuffers {
     int32_t *order;         // [n_xcd * P]     macro tile of XCD x's q-th workgroup (P = rounds * 32), valid for q < sched[8 + x]
     int32_t *sched;         // [24]            per XCD x: [x] computing items, [8 + x] all items, [16 + x] ticket
                             //                 counter of the persistent GEMM (zero between launches)
-    KeptProducts *kept;
 };
 
 // tau_skip > 0: tau-aware pass, the fp16 copy of tile (i, k) is written only if

@@ -284,6 +284,16 @@ def test_three_small_units_per_cu_keep_the_same_contracts(tmp_path):
         assert memory == {"global_load_lds_dwordx4"} and not any(mn.startswith("scratch_") for mn in mns), name
 
 
+def test_small_output_kernels_read_their_arguments_from_two_lines(tmp_path):
+    # a later line of arguments would be fetched when M, N and C are needed, in the middle of the kernel's chain
+    text = _isa("kernels_small.hip", tmp_path)
+    kernels = re.findall(r"^(_ZN5spamm(?:7k_small|13k_small_three)I\w+):[^\n]*\n(.*?)s_endpgm", text, flags=re.S | re.M)
+    assert len(kernels) == 9
+    for name, body in kernels:
+        loads = re.findall(r"s_load_dword(?:x(\d+))?\s+\S+, s\[\d+:\d+\], (0x[0-9a-f]+)", body)
+        assert loads and max(int(at, 16) + 4 * int(n or 1) for n, at in loads) <= 128, (name, loads)
+
+
 def test_results_are_published_when_the_workspace_is_at_rest(tmp_path):
     """The host goes on when it sees a result's sequence number and may use the workspace at once, from another stream:
     behind a publishing kernel's last barrier no wave stores anything but the result itself (to host memory, in system
