@@ -384,6 +384,11 @@ __global__ __launch_bounds__(256, 3) void k_small_three(const unsigned char *__r
     small_unit_body<B, 128, 3>(pA, pB, g, nbM, nbK, nbN, nMacN, n_units, n_xcd, mode, tau, M, N, C);
 }
 
+// Units of 128 in C, as many as 256 CUs would have for the same share of a CU: what the lines below balance is workgroups per
+// CU and k_gemm's rounds of a macro tile per CU, so on a partition of fewer CUs they lie at as many units less.
+static int64_t per_256_cus(int64_t units, int n_cu) { return (units * 256 + n_cu - 1) / n_cu; }
+static int64_t units_of_128(int64_t M, int64_t N, int n_cu) { return per_256_cus(((M + 127) / 128) * ((N + 127) / 128), n_cu); }
+
 // Unit by units of 128 in C: the wide one from half a unit per CU on.  Resident operands, K = 2048 at tile 32 (64 within
 // 10 %), 2 %, 10 %, 30 % kept and dense, narrow -> wide: 256 units 13.7 -> 12.4, 17.9 -> 15.3, 27.2 -> 20.0, 37.1 -> 24.9 us;
 // 196 units 12.3 -> 12.4, 15.7 -> 15.2, 20.7 -> 19.4, 36.1 -> 23.7; 144 units 10.0 -> 12.2, 13.4 -> 14.5, 17.8 -> 18.5,
@@ -391,10 +396,7 @@ __global__ __launch_bounds__(256, 3) void k_small_three(const unsigned char *__r
 // choice: a sparse product pays some 2 us there for the 5 to 12 that a dense one, or one of more k, saves (144 units,
 // K = 6144: 30 % kept 28.7 -> 24.7, dense 62.8 -> 47.8).  Below it the narrow one (whole calls, wide -> narrow: 99 units
 // 20.1 -> 18.4, 64 units 15.4 -> 13.1 and, dense, 21.7 -> 20.6).
-static int small_unit(int64_t M, int64_t N) {
-    const int64_t units128 = ((M + 127) / 128) * ((N + 127) / 128);
-    return units128 >= 128 ? 128 : 64;
-}
+static int small_unit(int64_t units128) { return units128 >= 128 ? 128 : 64; }
 
 // Clearly more than two units of 128 per CU: a ring of three stages leaves room for a third workgroup on the CU, whose loads
 // and syncs fill the others' waits.  Ring of four, two workgroups -> this, whole multiplies, fp16: 640 units, K = 2048 at tile
@@ -471,9 +473,9 @@ hipError_t small_init() {
 // Gate and multiply called apart (`stages`) form mask and list twice, which costs what the schedule does: the lines are
 // drawn closer (tau to a fraction and both stages, apart -> this: 625 units 114.7 -> 98 us; 768 units 122 -> 105, 127 -> 110;
 // 900 units 157 -> 160; 1000 units at tile 32 137.5 -> 139; 1120 units 162.5 -> 149.6, 126 -> 116; 1444 units 139 -> 147).
-bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau, bool stages) {
-    const int64_t units128 = ((M + 127) / 128) * ((N + 127) / 128), m = ((M + 255) / 256) * ((N + 255) / 256);
-    if (K / tile > SMALL_MAX_NBK) return false;
+bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau, bool stages, int n_cu) {
+    const int64_t units128 = units_of_128(M, N, n_cu), m = per_256_cus(((M + 255) / 256) * ((N + 255) / 256), n_cu);
+    if (K / tile > SMALL_MAX_NBK || n_cu > 256) return false;
     static_assert(SMALL_MAX_UNITS >= 6 * 256 && SMALL_MAX_UNITS >= 4 * 127, "units of either size");
     if (units128 <= 512) return true;
     if (stages) return tau > 0.0f && (units128 <= 832 || (units128 > 1024 && units128 <= 1200));
@@ -483,18 +485,19 @@ bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau, bool stage
 
 template <int B>
 static hipError_t launch_small_(const void *pA, const void *pB, const GateBuffers &g, int64_t M, int64_t K, int64_t N,
-                                int mode, float tau, float *C, int n_xcd, hipStream_t s) {
-    if (small_unit(M, N) != 128) return launch_small_<B, 64, false>(pA, pB, g, M, K, N, mode, tau, C, n_xcd, s);
-    if (small_three(((M + 127) / 128) * ((N + 127) / 128), K / B, B)) return launch_small_<B, 128, true>(pA, pB, g, M, K, N, mode, tau, C, n_xcd, s);
+                                int mode, float tau, float *C, int n_cu, int n_xcd, hipStream_t s) {
+    const int64_t units128 = units_of_128(M, N, n_cu);
+    if (small_unit(units128) != 128) return launch_small_<B, 64, false>(pA, pB, g, M, K, N, mode, tau, C, n_xcd, s);
+    if (small_three(units128, K / B, B)) return launch_small_<B, 128, true>(pA, pB, g, M, K, N, mode, tau, C, n_xcd, s);
     return launch_small_<B, 128, false>(pA, pB, g, M, K, N, mode, tau, C, n_xcd, s);
 }
 
 hipError_t launch_small(const void *packedA, const void *packedB, const GateBuffers &g, int64_t M, int64_t K, int64_t N,
-                        int tile, int mode, float tau, float *C, int n_xcd, hipStream_t s) {
+                        int tile, int mode, float tau, float *C, int n_cu, int n_xcd, hipStream_t s) {
     switch (tile) {
-        case 32: return launch_small_<32>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s);
-        case 64: return launch_small_<64>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s);
-        case 128: return launch_small_<128>(packedA, packedB, g, M, K, N, mode, tau, C, n_xcd, s);
+        case 32: return launch_small_<32>(packedA, packedB, g, M, K, N, mode, tau, C, n_cu, n_xcd, s);
+        case 64: return launch_small_<64>(packedA, packedB, g, M, K, N, mode, tau, C, n_cu, n_xcd, s);
+        case 128: return launch_small_<128>(packedA, packedB, g, M, K, N, mode, tau, C, n_cu, n_xcd, s);
         default: return hipErrorInvalidValue;
     }
 }

@@ -475,7 +475,7 @@ static int build_lists(spamm_ctx *c, float tau) {
 // Small outputs are gated and multiplied by a kernel of their own (kernels_small.hip); a caller who fixes
 // the work unit or the gate's chunks gets the gate and the GEMM.  `stages`: called apart.
 static bool is_small(const spamm_ctx *c, float tau, bool stages) {
-    return c->gemm_shape == 0 && c->gate_chunk_cap == 0 && small_fits(c->M, c->K, c->N, c->tile, tau, stages);
+    return c->gemm_shape == 0 && c->gate_chunk_cap == 0 && small_fits(c->M, c->K, c->N, c->tile, tau, stages, c->n_cu);
 }
 
 // Its gate, its multiply (dC), or both.
@@ -486,7 +486,7 @@ static int run_small(spamm_ctx *c, int mode, float tau, float *dC) {
     if ((rc = ensure(c, c->counts, nt * 4))) return rc;
     if ((rc = ensure(c, c->mask, nt * s.words * 8))) return rc;
     if ((rc = ensure(c, c->kept, sizeof(KeptProducts)))) return rc;
-    HIPCHK(c, launch_small(c->packedA.p, c->packedB.p, gate_buffers(c), c->M, c->K, c->N, c->tile, mode, tau, dC, c->n_xcd, c->stream));
+    HIPCHK(c, launch_small(c->packedA.p, c->packedB.p, gate_buffers(c), c->M, c->K, c->N, c->tile, mode, tau, dC, c->n_cu, c->n_xcd, c->stream));
     if (mode & SMALL_GATE) {
         c->tau = tau;
         c->have_gate = true;

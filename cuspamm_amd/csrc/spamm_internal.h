@@ -203,10 +203,10 @@ hipError_t launch_gemm(const void *packedA, const void *packedB, const GateBuffe
 // gate and multiply in one launch (kernels_small.hip)
 constexpr int64_t SMALL_MAX_NBK = 2048;      // its k list lives in LDS
 hipError_t small_init();
-bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau, bool stages);
+bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau, bool stages, int n_cu);
 constexpr int SMALL_GATE = 1, SMALL_MULTIPLY = 2;    // what launch_small does: either or both
 hipError_t launch_small(const void *packedA, const void *packedB, const GateBuffers &g, int64_t M, int64_t K, int64_t N,
-                        int tile, int mode, float tau, float *C, int n_xcd, hipStream_t s);
+                        int tile, int mode, float tau, float *C, int n_cu, int n_xcd, hipStream_t s);
 constexpr int GEMM_SHAPE_FULL = 1, GEMM_SHAPE_HALF = 2, GEMM_SHAPE_W8 = 3, GEMM_SHAPE_PERSIST = 4;
 constexpr int SCHED_WORDS = 3 * MAX_XCD;     // GateBuffers::sched
 

@@ -107,7 +107,8 @@ SPAMM_API int spamm_destroy(spamm_ctx *ctx);
  *     macro tile of C (one workgroup per CU), 2 = four waves per 128 x 256 half (two workgroups per
  *     CU), 3 = eight waves per macro tile, 4 = shape 1 by workgroups that stay on their CU and draw
  *     macro tiles from a ticket counter per XCD; 0 = chosen per call (a C of at most 1536
- *     blocks of 128 x 128 at tau > 0, 512 and some sizes up to 1296 at tau <= 0, with K / tile <= 2048, is
+ *     blocks of 128 x 128 at tau > 0, 512 and some sizes up to 1296 at tau <= 0 (by 256 CUs; as many
+ *     less on a partition of fewer), with K / tile <= 2048, is
  *     gated and multiplied by one kernel in units of 128 or 64; otherwise 1, or halves when C has at most half a macro tile per CU).  All add in the same
  *     order: C is bit-identical.
  * SPAMM_EINVAL for an unknown option or a value outside its range.  The reference has no such

@@ -37,6 +37,7 @@ std::map<const void *, std::string> kernel_names;
 std::map<std::string, std::pair<int, int>> answers;     // by part of a kernel's name
 std::map<void *, size_t> sizes;                         // of the device's allocations
 size_t held = 0, limit = ~(size_t)0 / 2;
+int cus = 256;
 std::string launched;       // "name grid;" of every launch since fake_launches was last asked
 
 }  // namespace
@@ -57,6 +58,7 @@ const char *fake_launches() {
 
 size_t fake_held() { return held; }
 void fake_limit(size_t bytes) { limit = bytes; }
+void fake_cus(int n) { cus = n; }
 // kernels of this name publish a result: their arguments (by number) are where its sequence number goes, and the number
 void fake_answer(const char *name, int host_seq, int seq) { answers[name] = {host_seq, seq}; }
 
@@ -65,7 +67,7 @@ hipError_t hipGetDeviceCount(int *n) { *n = 2; return hipSuccess; }
 hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int) {       // (the header's name for the versioned symbol)
     memset(p, 0, sizeof *p);
     strcpy(p->gcnArchName, "gfx950");
-    p->multiProcessorCount = 256;
+    p->multiProcessorCount = cus;
     return hipSuccess;
 }
 hipError_t hipSetDevice(int d) { current = d; return hipSuccess; }

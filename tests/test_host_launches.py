@@ -173,6 +173,38 @@ def test_a_report_without_memory_for_its_scratch_leaves_no_error(run):
     run("report_on_a_full_card")
 
 
+class Params(ctypes.Structure):
+    _fields_ = [("M", i64), ("K", i64), ("N", i64), ("tile", ctypes.c_int32), ("tau", ctypes.c_float), ("flags", ctypes.c_uint32),
+                ("reserved", ctypes.c_uint32)]
+
+
+def multiply_on_a_partition(e, cus):
+    e.fake.fake_cus(cus)
+    h = e.context()
+    X = ctypes.create_string_buffer(16)
+
+    def kernels(eighths, K, tau):
+        """Of a C with so many eighths of a unit of 128 x 128 per CU."""
+        M, N = 128 * eighths, 128 * (cus // 8)
+        e.launches()
+        assert e.L.spamm_multiply(h, p(Params(M, K, N, 64, tau, 0, 0)), X, X, X) == 0
+        return [name for name, _ in e.launches() if name in ("k_small", "k_small_three", "k_gate", "k_gemm")]
+
+    for tau, most in ((0.5, 48), (0.0, 16)):
+        assert kernels(2, 2048, tau) == ["k_small"] and kernels(16, 2048, tau) == ["k_small"]
+        if tau:
+            assert kernels(20, 2048, tau) == ["k_small_three"] and kernels(24, 16384, tau) == ["k_small_three"]
+            assert "k_gate" in kernels(32, 16384, tau) and "k_gate" in kernels(60, 2048, tau)
+        assert "k_gate" in kernels(most + 2, 2048, tau)
+        assert ("k_gate" in kernels(most, 2048, tau)) is False
+
+
+@pytest.mark.parametrize("cus", [256, 128, 64, 32])
+def test_lines_of_the_small_kernel_are_by_work_per_cu(run, cus):
+    """A partition of an XCD or a few has its lines where a CU has as much to do as on the whole chip."""
+    run("multiply_on_a_partition", cus)
+
+
 if __name__ == "__main__":
     globals()[sys.argv[3]](Engine(*sys.argv[1:3]), *map(int, sys.argv[4:]))
     print("ok")
