@@ -392,7 +392,7 @@ __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict
             }
         });
         // accumulator i of lane l in block t: row 4 (l / 16) + i, column l % 16; orders 0 to 3 and 4 to 6 are added in
-        // 64-bit integers, so the one rounding is the last
+        // 64-bit integers, of which the upper one takes the carry and stays below 2^53: the one rounding is the last
         const float *src = C + (row0 + (int64_t)bi * LIMB_BLOCK + wr * 32 + 4 * q) * N + (int64_t)bj * LIMB_BLOCK + wc * 32 + l16;
 #pragma unroll
         for (int t = 0; t < 4; t++)
@@ -403,7 +403,7 @@ __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict
                                      ((long long)acc[2][t >> 1][t & 1][i] << 16) + ((long long)acc[3][t >> 1][t & 1][i] << 24);
                 const long long hi = (long long)acc[4][t >> 1][t & 1][i] + ((long long)acc[5][t >> 1][t & 1][i] << 8) +
                                      ((long long)acc[6][t >> 1][t & 1][i] << 16);
-                const double d = fma((double)hi, 4294967296.0, (double)lo) * (1.0 / 281474976710656.0);
+                const double d = fma((double)(hi + (lo >> 32)), 4294967296.0, (double)(unsigned int)lo) * (1.0 / 281474976710656.0);
                 e2 += (c - d) * (c - d);
                 d2 += d * d;
                 c2 += c * c;

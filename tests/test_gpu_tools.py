@@ -397,6 +397,21 @@ def test_error_report_over_the_range_of_fp16(ctx, tile, M, K, N, row0, rows, kin
             assert abs(g - ref) <= 1e-9 * ref
 
 
+def test_error_report_rounds_once(ctx):
+    """21800 products of 257 / 512 with itself, 10900 of minus twice that by values with other digits, and one of 2^-24 with
+    itself: the upper and the lower orders of a sum pass 2^53 and cancel, and what is left is the last product."""
+    import torch
+    K = 32704
+    a, b = np.zeros(K), np.zeros(K)
+    a[:21800] = b[:21800] = 257 / 512
+    a[21800:32700], b[21800:32700] = -64.25, 257 * 2.0 ** -15
+    a[32700] = b[32700] = 2.0 ** -24
+    ctx.normmap_f16(1, torch.from_numpy(np.repeat(b[:, None], 64, axis=1).astype(np.float16)).cuda(), 32)
+    ctx.normmap_f16(0, torch.from_numpy(np.repeat(a[None], 64, axis=0).astype(np.float16)).cuda(), 32)
+    C = torch.full((64, 64), 2.0 ** -48, dtype=torch.float32, device="cuda")
+    assert ctx.error_vs_dense(C) == (0.0, 64 * 2.0 ** -48, 64 * 2.0 ** -48)
+
+
 @pytest.mark.parametrize("M,K,N,tile", [(1280, 1024, 1088, 64), (2048, 512, 2048, 128)])
 def test_error_reports_of_small_and_large_values_by_turns(ctx, M, K, N, tile):
     """Values that are too large are taken by the integer product's launch, or by another when it has said so: report after
