@@ -356,8 +356,9 @@ def test_error_report_by_any_block_shape(ctx, rows, N, row0):
     (128, 2048, 512, 2048, 0, 2048, "large"), (32, 2048, 544, 2112, 64, 1984, "inf")])
 def test_error_report_over_the_range_of_fp16(ctx, tile, M, K, N, row0, rows, kind):
     """Whatever the magnitudes: 0 to 4 bytes a value by blocks, just inside and outside of what bytes hold, subnormals,
-    infinities, sums at the length where 32 bits end.  Against fp64 on the host (K terms a sum, rows * N in a norm, 2^-53
-    each, below 1e-9); the exact product of whole multiples of 2^-24 is what both sides form."""
+    infinities and NaN, the largest sums that 11 bits a value make at the longest K.  Against fp64 on the host (K terms a sum,
+    rows * N in a norm, 2^-53 each, below 1e-9); the exact product of whole multiples of 2^-24 is what both sides form.
+    Whole numbers from K = 256 on where the split is worth it, and one shape or two of every kind on the other side of that."""
     import torch
     rng = np.random.default_rng(M + K + N)
 
@@ -365,7 +366,7 @@ def test_error_report_over_the_range_of_fp16(ctx, tile, M, K, N, row0, rows, kin
         X = rng.uniform(-1.0, 1.0, (r, c))
         if kind == "limbs":       # 64 x 64 blocks of every magnitude that needs 0 to 4 bytes, and what lies below fp16
             X *= np.kron(np.exp2(rng.choice([-40, -22, -16, -15, -9, -8, -1, 0, 6], (-(-r // 64), -(-c // 64)))), np.ones((64, 64)))[:r, :c]
-        elif kind == "edge":      # the largest digits everywhere: 4 products a k and order, all of one sign
+        elif kind == "edge":      # digits (0, 0, -128, 127) and (0, -128, -127, 1), of one sign: an order's sum reaches 8e8, 0.37 of 2^31
             X = np.where(X < 0, -126.5, 126.5)
             X[:, ::2] = np.where(X[:, ::2] < 0, -0.50196, 0.50196)
         elif kind == "large":

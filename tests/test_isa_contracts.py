@@ -329,3 +329,27 @@ def test_bisection_state_is_stored_past_the_cache(tmp_path):
         assert len(kernels) == 1
         stores = [ln.strip() for ln in kernels[0][1].splitlines() if re.match(r"\s*(global|flat|buffer|scratch)_store", ln)]
         assert stores and all("sc1" in ln for ln in stores), (name, stores)
+
+
+def test_bisection_publishes_when_its_workspace_is_at_rest(tmp_path):
+    """The same for the bisection, which publishes from the launch that ends it: behind the last barrier one thread stores the
+    state, then the result, waits, and stores the sequence number; and every wave of the tree, all of which clear leaves, has
+    waited for its stores before a barrier in between."""
+    text = _isa("kernels_tau.hip", tmp_path)
+    for name, waits in (("k_tau_count", 1 + 2), ("k_tau_tree", 1 + 1 + 1)):     # last_workgroup, the leaves, publish_result (two calls)
+        (body,) = re.findall(r"^_ZN5spamm\d+%s\w+:[^\n]*\n(.*?)^\.Lfunc_end" % name, text, flags=re.S | re.M)
+        lines = [ln.strip() for ln in body.splitlines()]
+        asm = [i for i, ln in enumerate(lines) if re.match(r"s_waitcnt vmcnt\(0\)$", ln) and lines[i - 1].startswith(";;#ASMSTART")]
+        assert len(asm) == waits, (name, asm)
+        last = max(i for i, ln in enumerate(lines) if ln.startswith("s_barrier"))
+        assert asm[-1] > last
+        end = [i for i in range(last, len(lines)) if re.match(r"(global|flat|buffer|scratch)_(store|atomic)", lines[i])]
+        results = [i for i in end if "sc0 sc1" in lines[i]]
+        assert all("sc1" in lines[i] for i in end) and results[-1] == end[-1] and asm[-1] == max(i for i in asm if i < end[-1])
+        assert not [i for i in end[:-1] if i > asm[-1]], name                   # the sequence number alone comes behind the wait
+        if name == "k_tau_tree":
+            rest = lines[asm[1] + 1:]
+            barrier = next(i for i, ln in enumerate(rest) if ln.startswith("s_barrier"))
+            assert not any(re.match(r"\.LBB|s_cbranch|s_branch|global_|flat_", ln) for ln in rest[:barrier]) and asm[1] + 1 + barrier < last
+            clears = [i for i, ln in enumerate(lines) if ln.startswith("global_store") and asm[0] < i < last]
+            assert len(clears) >= 4, clears
