@@ -243,10 +243,9 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
 
         // entry of a stage (stages beyond the last repeat the last entry: loaded, never multiplied)
         auto entry_at = [&](int t) -> uint32_t { return s_list[(t < S ? t : S - 1) / H::NSPE]; };
-        auto issue = [&](int t, uint32_t ent, auto idx) {
+        auto issue = [&](int t, uint32_t ent, uint32_t boff, auto idx) {
             constexpr int i = decltype(idx)::value, j = i % H::CHW;
             const int64_t koff = (int64_t)(ent & 0xffffu) * H::TILE_BYTES + ((t < S ? t : S - 1) % H::NSPE) * (B * 64);
-            const uint32_t boff = (uint32_t)(t % NBUF) * H::STAGE_BYTES;
             // a slot that no tile pair of the entry reads is not fetched: its load goes to one place that is
             // cache resident, so that the number of loads in flight stays fixed
             if constexpr (i < H::CHW) {
@@ -269,9 +268,9 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
         struct Frags {
             half8 a[NB], b[NB];
         };
-        auto load_frag = [&](Frags &f, int t, auto idx) {
+        auto load_frag = [&](Frags &f, uint32_t boff, auto idx) {
             constexpr int i = decltype(idx)::value;
-            const unsigned char *bufA = smem + (t % NBUF) * H::STAGE_BYTES;
+            const unsigned char *bufA = smem + boff;
             if constexpr (i == 0) f.a[0] = *reinterpret_cast<const half8 *>(bufA + frag_off(wr, 0));
             else if constexpr (i <= NB) f.b[i - 1] = *reinterpret_cast<const half8 *>(bufA + H::OP_BYTES + frag_off(wc, i - 1));
             else f.a[i - NB] = *reinterpret_cast<const half8 *>(bufA + frag_off(wr, i - NB));
@@ -280,9 +279,19 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
 #pragma unroll
         for (int t = 0; t < NBUF; t++) {
             const uint32_t e = __builtin_amdgcn_readfirstlane(entry_at(t));
-            static_for<H::LPW>([&](auto i) { issue(t, e, i); });
+            static_for<H::LPW>([&](auto i) { issue(t, e, t * H::STAGE_BYTES, i); });
         }
+        // The buffer of stage t -- once that is in registers, of stage t + NBUF -- and the next one's, which is formed before the
+        // sync: behind it a wave's first reads of LDS wait for their address.  (By t % NBUF where they are used the compiler
+        // put up to 13 scalar instructions there, which depended on the order of the kernel's arguments: 384 x 4736 x 416 at
+        // tile 32 33.4 or 34.3 us, 32.75 now; 1056 x 1568 x 1312 17.34 or 17.5, 17.07 now.)
         int t = 0;
+        uint32_t buf = 0;
+        auto next_buf = [&]() {
+            uint32_t next = buf + H::STAGE_BYTES == NBUF * H::STAGE_BYTES ? 0u : buf + H::STAGE_BYTES;
+            asm volatile("" : "+s"(next));
+            return next;
+        };
         uint32_t e_cur = entry_at(0), e_new = entry_at(NBUF);
         __builtin_amdgcn_s_waitcnt(waitcnt_imm(H::LPW * (NBUF - 1), 0));
         __syncthreads();
@@ -290,6 +299,7 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
         static_for<2 * NB>([&](auto i) { load_frag(f0, 0, i); });
 #define SPAMM_FENCE() __builtin_amdgcn_sched_barrier(0)
         auto full_stage = [&](const Frags &cur, Frags &nxt) {
+            const uint32_t next = next_buf();
             sync_next();
             const uint32_t en = __builtin_amdgcn_readfirstlane(e_new);
             e_cur = entry_at(t + 1);
@@ -298,17 +308,19 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
             static_for<NB * NB>([&](auto idx) {
                 constexpr int i = decltype(idx)::value, r = i / NB, c = i % NB;
                 acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cur.a[r], cur.b[c], acc[r][c], 0, 0, 0);
-                if constexpr (i < 2 * NB) load_frag(nxt, t + 1, idx);
-                if constexpr (NB == 4 ? (i >= 8 && i % 2 == 0) : i >= 2) issue(t + NBUF, en, std::integral_constant<int, NB == 4 ? (i >= 8 ? (i - 8) / 2 : 0) : (i >= 2 ? i - 2 : 0)>{});
+                if constexpr (i < 2 * NB) load_frag(nxt, next, idx);
+                if constexpr (NB == 4 ? (i >= 8 && i % 2 == 0) : i >= 2) issue(t + NBUF, en, buf, std::integral_constant<int, NB == 4 ? (i >= 8 ? (i - 8) / 2 : 0) : (i >= 2 ? i - 2 : 0)>{});
                 SPAMM_FENCE();
             });
             t++;
+            buf = next;
         };
         while (__builtin_expect(t + 1 < Sfull, 1)) {
             full_stage(f0, f1);
             full_stage(f1, f0);
         }
         auto partial_stage = [&](const Frags &cur, Frags &nxt) {
+            const uint32_t next = next_buf();
             sync_next();
             const uint32_t en = t + NBUF < S ? __builtin_amdgcn_readfirstlane(e_new) : (__builtin_amdgcn_readfirstlane(e_new) & 0xffffu);
             const uint32_t ec = t < S ? (__builtin_amdgcn_readfirstlane(e_cur) >> 16) >> (TU > 1 ? wr * TU + wc : 0) : 0u;
@@ -327,13 +339,14 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
                 }
                 if constexpr (p == 0) {
                     SPAMM_FENCE();
-                    static_for<2 * NB>([&](auto i) { load_frag(nxt, t + 1, i); });
-                    static_for<H::LPW>([&](auto i) { issue(t + NBUF, en, i); });
+                    static_for<2 * NB>([&](auto i) { load_frag(nxt, next, i); });
+                    static_for<H::LPW>([&](auto i) { issue(t + NBUF, en, buf, i); });
                     SPAMM_FENCE();
                 }
             });
             SPAMM_FENCE();
             t++;
+            buf = next;
         };
         while (__builtin_expect(t < S, 1)) {
             partial_stage(f0, f1);

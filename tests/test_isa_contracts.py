@@ -294,6 +294,21 @@ def test_small_output_kernels_read_their_arguments_from_two_lines(tmp_path):
         assert loads and max(int(at, 16) + 4 * int(n or 1) for n, at in loads) <= 128, (name, loads)
 
 
+def test_small_output_kernels_read_lds_soon_behind_a_sync(tmp_path):
+    # gate, list, prologue, then two full and two partial stages a turn: a full stage has an entry's read, its address and
+    # its own reads' in front of them
+    text = _isa("kernels_small.hip", tmp_path)
+    kernels = re.findall(r"^(_ZN5spamm(?:7k_small|13k_small_three)I\w+):[^\n]*\n(.*?)^\.Lfunc_end", text, flags=re.S | re.M)
+    assert len(kernels) == 9
+    for name, body in kernels:
+        lines = [ln for ln in (re.sub(r";.*", "", ln).strip() for ln in body.splitlines()) if ln and not ln.startswith(".")]
+        syncs = [i for i, ln in enumerate(lines) if ln.startswith("s_barrier")]
+        assert len(syncs) == 7, name
+        for at in syncs[3:5]:
+            reads = next(i for i in range(at, len(lines)) if lines[i].startswith("ds_read_b128"))
+            assert reads - at <= 8, (name, reads - at)
+
+
 def test_results_are_published_when_the_workspace_is_at_rest(tmp_path):
     """The host goes on when it sees a result's sequence number and may use the workspace at once, from another stream:
     behind a publishing kernel's last barrier no wave stores anything but the result itself (to host memory, in system
