@@ -414,9 +414,12 @@ static int small_unit(int64_t units128) { return units128 >= 128 ? 128 : 64; }
 // Clearly more than two units of 128 per CU: a ring of three stages leaves room for a third workgroup on the CU, whose loads
 // and syncs fill the others' waits.  Ring of four, two workgroups -> this, whole multiplies, fp16: 640 units, K = 2048 at tile
 // 32, 10 % kept 45.8 -> 41.0 us, 40 % 60.2 -> 54.5, dense 75.6 -> 69; 768 units 48.5 -> 44.7, 65.4 -> 58.7, 79.6 -> 75.7; 1024
-// units, 5 % 47.4 -> 45.2, 40 % 75.7 -> 78.7.  Up to 600 units, where a second turn of two per CU is short, it is the worse
-// of the two for narrow bands, whose few long lists want the longer ring (576 units, 3.5 % kept 39.2 -> 40.9, 594 units at tile
-// 128 43.2 -> 45.4; but 576 units, 10 % algebraic 42.0 -> 37.4).  A list too long for three in a CU's LDS keeps the ring of four.
+// units, 5 % 47.4 -> 45.2, 40 % 75.7 -> 78.7.  From 513 to 600 units, where a second turn of two per CU is short, neither is the
+// better one: over 120 calls (K of 1024 to 4096, all tiles, 3.5 % kept to dense) this takes 0.99 of the time in the geometric
+// mean, 0.85 to 1.16 of it.  Bands, whose few long lists want the longer ring, lose (576 units, K = 2048 at tile 64, 10 %
+// 32.9 -> 38.1 us; 600 units at tile 32, 3.5 % 31.3 -> 34.3), slow decay gains (576 units, 30 % algebraic 50.8 -> 45.0, 550 units,
+// 10 % 42.4 -> 38.9): the host cannot tell them apart, and bands are the usual operands.  A list too long for three in a CU's LDS
+// keeps the ring of four.
 static bool small_three(int64_t units128, int64_t nbK, int tile) {
     const int tt = tile >= 128 ? 1 : (128 / tile) * (128 / tile);
     return units128 > 600 && 3 * (small_lds_bytes_(16384, 3, tt, nbK) + 2048) <= 160 * 1024;
