@@ -38,6 +38,9 @@ CFLAGS = [
 # drawn by one lane with a returning atomic that is asked for early and looked at late; the compiler's
 # rewrite of atomics in divergent code (one lane adds for all, then a broadcast) would wait for it at once.
 GEMM_FLAGS = ["-Wno-inline-asm", "-mllvm", "-amdgpu-atomic-optimizer-strategy=None"]
+# by source, beside CFLAGS: the kernels with global->LDS loads, of which the multiply's must not spill (_check_no_scratch)
+NO_SPILL = ("kernels_gemm.hip", "kernels_small.hip")
+EXTRA_FLAGS = {"kernels_gemm.hip": GEMM_FLAGS, "kernels_small.hip": GEMM_FLAGS, "kernels_tools.hip": ["-Wno-inline-asm"]}
 
 
 def _run(cmd):
@@ -73,9 +76,9 @@ def build_library(verbose=False):
 
     def compile_one(pair):
         src, obj = pair
-        extra = ["-Rpass-analysis=kernel-resource-usage"] + GEMM_FLAGS if src in ("kernels_gemm.hip", "kernels_small.hip") else []
-        log = _run([HIPCC] + CFLAGS + extra + ["-c", os.path.join(CSRC, src), "-o", obj])
-        if extra:
+        remarks = ["-Rpass-analysis=kernel-resource-usage"] if src in NO_SPILL else []
+        log = _run([HIPCC] + CFLAGS + remarks + EXTRA_FLAGS.get(src, []) + ["-c", os.path.join(CSRC, src), "-o", obj])
+        if remarks:
             _check_no_scratch(log, src)
             keep, skip = [], 0
             for line in log.splitlines():          # drop the remarks and the source excerpts printed under them

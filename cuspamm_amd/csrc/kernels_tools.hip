@@ -16,10 +16,11 @@
 // the number of blocks allows: each converted value serves NBR or NBC MFMAs.  4096^3:
 // 2229 us with 32 x 32 per wave and 4-byte loads, 2109 now (65 TFLOP/s; the pipeline's 128 operations at the clock
 // that the chip holds under them, about 2 GHz); 1984 x 2176 x 768: 196 -> 158.  In whole numbers instead (one call, its
-// host wait included): 4096^3 2107 -> 867 us on uniform values in [-1, 1) (4 bytes each, 16 products, 2.6 Pop/s: power),
-// 620 where 3 bytes do, 272 on exp(-d / 100); 1984 x 2176 x 768 165 -> 82, 67, 49; 64 rows of 4096^3 173 -> 109, 91, 50.
+// host wait included): 4096^3 2107 -> 742 us on uniform values in [-1, 1) (4 bytes each, 16 products, 3.1 Pop/s),
+// 469 where 3 bytes do, 232 on exp(-d / 100); 1984 x 2176 x 768 165 -> 76, 63, 45; 64 rows of 4096^3 173 -> 87, 68, 45.
 // An operand with a value of 127 or more has been read by k_limbs for nothing, which writes no planes then, and blocks of 64 x 64
-// of C are formed in fp64 by k_error_limbs itself: 1024^3 56 -> 59.5 us, 1280^3 106 -> 111, 4096^3 2121 -> 2106.
+// of C are formed in fp64 by k_error_limbs itself, two workgroups per CU where k_error_dense has three, so its loads go out
+// three steps ahead instead of one (1280^3 122.7 -> 115): 1024^3 56 -> 59.5 us, 1280^3 106 -> 111, 4096^3 2121 -> 2106.
 // The scalar bound of 64 x 64 x 64 tiles 52 -> 7 us, the per-tile one 51 -> 4; results go straight to host memory (a
 // clearing launch before and a copy after each were 25 us a call).
 #include "gemm_device.h"
@@ -85,7 +86,7 @@ __device__ __forceinline__ void finish_sums(ReportWorkspace *ws, double own, Rep
 // row (A) / column (B); of every four k-groups lane group q = lane / 16 takes the q-th, one 16-byte load per lane and
 // operand block for 32 k, and element e of the vectors makes MFMA step e.  Which k goes to which step is the same for A
 // and B, and the sum over k does not care.  fp16 -> fp64 is exact.
-template <int NBR, int NBC>
+template <int NBR, int NBC, int DEPTH = 2>
 __device__ __forceinline__ void dense_block(const _Float16 *__restrict__ pA, const _Float16 *__restrict__ pB, int64_t K, int64_t N, int tile,
                                             const float *__restrict__ C, int64_t br, int64_t bc, double &e2, double &d2, double &c2) {
     const int lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
@@ -133,16 +134,19 @@ __device__ __forceinline__ void dense_block(const _Float16 *__restrict__ pA, con
                     acc[ta][tb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ta], b[tb], acc[ta][tb], 0, 0, 0);
         }
     };
-    Vecs v0, v1;
-    load(v0, 0);
+    Vecs v[DEPTH];                          // steps whose loads are under way or done
+#pragma unroll
+    for (int i = 0; i < DEPTH - 1; i++) load(v[i], i);
     int64_t s = 0;
-    for (; s + 1 < steps; s += 2) {
-        load(v1, s + 1);
-        multiply(v0);
-        load(v0, s + 2);
-        multiply(v1);
-    }
-    if (s < steps) multiply(v0);
+    for (; s + DEPTH <= steps; s += DEPTH)
+#pragma unroll
+        for (int i = 0; i < DEPTH; i++) {
+            load(v[(i + DEPTH - 1) % DEPTH], s + i + DEPTH - 1);
+            multiply(v[i]);
+        }
+#pragma unroll
+    for (int i = 0; i < DEPTH - 1; i++)
+        if (s + i < steps) multiply(v[i]);
     // accumulator i of lane l in block (ta, tb): row 4 i + l / 16, column l % 16
 #pragma unroll
     for (int ta = 0; ta < NBR; ta++)
@@ -276,13 +280,46 @@ __global__ __launch_bounds__(256) void k_limbs(LimbOperand a, LimbOperand b, int
 
 // One workgroup owns 64 x 64 of C, a wave 32 x 32 of it: 4 accumulator registers x 4 MFMA blocks x 7 orders, so that two
 // waves share a SIMD.  The k blocks are sorted by the limbs they need on both sides (whole numbers: the sum does not
-// care), and each kind has a loop of its own without branches, the next block's operands on their way while one is
-// multiplied.  Groups of GB x GB workgroups that share operands in an L2 run on one XCD; the groups, row by row, go round
+// care) and taken in steps of as many blocks of a kind as have LIMB_STEP planes or fewer; each kind has a loop of its own.  A
+// step's planes are multiplied from LDS, which two waves share each, while direct global->LDS loads bring the next step's, whatever
+// its kind.  (Where a wave loaded its operands to registers, kind by kind, every plane passed the L1 twice and
+// a kind, of two or three blocks on the average, began with a wait: kernel alone, 4096^3 exp(-d / 100) 241 -> 201 us, uniform 780 ->
+// 670, 4096^3 algebraic 252 -> 187.)  What bounds it: a step of 0.69 us, of which the MFMAs of both
+// workgroups take 0.25 to 0.9 and LDS 0.5 (4 KiB written and 8 read per plane); without the reads the calls are 10 % shorter,
+// without the loads 12 %.  Planes in a ring of 16 with loads up to two steps ahead: 6 % longer (addresses); steps of 6 planes by three
+// workgroups per CU: decaying values 5 to 10 % shorter, uniform ones 50 % longer (4 + 4 limbs take two steps, and
+// 168 registers are too few).
+// Groups of GB x GB workgroups that share operands in an L2 run on one XCD; the groups, row by row, go round
 // the XCDs, each row turned by two against the one above, so that those of a diagonal, which have much the same work, are
 // spread over them.
 constexpr int ORDERS = 2 * LIMBS - 1;
 constexpr int64_t LIMB_MAX_K = 32768 - 64;      // an order adds up to 4 products of at most 2^14 per k in 31 bits
 constexpr int LIMB_MAX_KB = 32768 / LIMB_BLOCK;
+constexpr int LIMB_STEP = 2 * LIMBS;            // planes
+constexpr int LIMB_MAX_STEPS = LIMB_MAX_KB + LIMBS * LIMBS;
+
+// log2 of the blocks of a kind, (limbs of A - 1) * LIMBS + limbs of B - 1, that a step takes
+__host__ __device__ constexpr int limb_per_step(int kind) {
+    const int planes = kind / LIMBS + kind % LIMBS + 2;
+    return planes == 2 ? 2 : (planes <= 4 ? 1 : 0);
+}
+
+// Sum over the wave, in lane 63.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double add_dpp(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, ROWS, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, ROWS, 0xf, false);
+    return v + __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+    v = add_dpp<0xB1, 0xf>(v);          // lane ^ 1, lane ^ 2, the other half and the other quarter of 16 lanes
+    v = add_dpp<0x4E, 0xf>(v);
+    v = add_dpp<0x141, 0xf>(v);
+    v = add_dpp<0x140, 0xf>(v);
+    v = add_dpp<0x142, 0xa>(v);         // the last lane of 16 to the next 16, of 32 to the next 32
+    return add_dpp<0x143, 0xc>(v);
+}
 
 __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict__ plA, const uint8_t *__restrict__ clsA,
                                                         const int8_t *__restrict__ plB, const uint8_t *__restrict__ clsB, int nkb,
@@ -291,103 +328,141 @@ __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict
                                                         const float *__restrict__ C, int64_t row0, ReportWorkspace *__restrict__ ws,
                                                         ReportSums *__restrict__ host_out, unsigned long long *__restrict__ host_seq,
                                                         unsigned long long seq, bool dense_here) {
-    const bool fp64 = out_of_range(ws, seq);
-    if (fp64 && !dense_here) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) publish_result(host_out, ReportSums{{-1.0, 0.0, 0.0}}, host_seq, seq);
-        return;
-    }
+    __shared__ __attribute__((aligned(16))) unsigned char s_planes[2][LIMB_STEP][LIMB_PLANE];     // of this step and the next
+    __shared__ uint16_t s_desc[LIMB_MAX_STEPS][LIMB_STEP];        // plane of A or (bit 15) of B, or none
     __shared__ double red[4][3];
-    __shared__ int s_count[17], s_place[16];
-    __shared__ uint16_t s_list[LIMB_MAX_KB];
+    __shared__ int s_count[LIMBS * LIMBS];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wr = wave >> 1, wc = wave & 1;
     const int l16 = lane & 15, q = lane >> 4;
     const int x = (int)blockIdx.x % n_xcd, at = (int)blockIdx.x / n_xcd, in_group = at % (gb * gb), group = at / (gb * gb);
     const int gi = (group * n_xcd + x) / ngj, gj = ((group * n_xcd + x) % ngj + 2 * (ngj - gi % ngj)) % ngj;
     const int bi = gi * gb + in_group / gb, bj = gj * gb + in_group % gb;
+    const bool inside = bi < nbi && bj < nbj;
+    // (asked for before anything is waited for: the blocks' limbs, which mean nothing in fp64)
+    int la[2], lb[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int kb = h * 256 + (int)threadIdx.x, at = kb < nkb ? kb : 0;
+        la[h] = clsA[inside ? (int64_t)bi * nkb + at : 0];
+        lb[h] = clsB[inside ? (int64_t)bj * nkb + at : 0];
+        if (kb >= nkb) la[h] = 0;
+    }
+    const bool fp64 = out_of_range(ws, seq);
+    if (fp64 && !dense_here) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) publish_result(host_out, ReportSums{{-1.0, 0.0, 0.0}}, host_seq, seq);
+        return;
+    }
     double e2 = 0, d2 = 0, c2 = 0;
-    if (bi < nbi && bj < nbj && fp64) {
-        dense_block<2, 2>(pA, pB, K, N, tile, C, row0 + (int64_t)bi * LIMB_BLOCK + wr * 32, (int64_t)bj * LIMB_BLOCK + wc * 32, e2, d2, c2);
-    } else if (bi < nbi && bj < nbj) {
+    if (inside && fp64) {
+        dense_block<2, 2, 4>(pA, pB, K, N, tile, C, row0 + (int64_t)bi * LIMB_BLOCK + wr * 32, (int64_t)bj * LIMB_BLOCK + wc * 32, e2, d2, c2);
+    } else if (inside) {
         // ---- k blocks by kind
-        if (threadIdx.x < 17) s_count[threadIdx.x] = 0;
+        constexpr int KINDS = LIMBS * LIMBS;
+        constexpr uint32_t NO_PLANE = 0xffffu;
+        if (threadIdx.x < KINDS) s_count[threadIdx.x] = 0;
+        for (int i = threadIdx.x; i < nkb + KINDS; i += 256) reinterpret_cast<u32x4 *>(s_desc)[i] = u32x4{~0u, ~0u, ~0u, ~0u};
         __syncthreads();
-        const uint8_t *ca = clsA + (int64_t)bi * nkb, *cb = clsB + (int64_t)bj * nkb;
-        int kind[2];
+        int kind[2], nth[2];
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            const int kb = h * 256 + (int)threadIdx.x;
-            const int la = kb < nkb ? ca[kb] : 0, lb = kb < nkb ? cb[kb] : 0;
-            kind[h] = la && lb ? (la - 1) * LIMBS + lb - 1 : -1;
-            if (kind[h] >= 0) atomicAdd(&s_count[kind[h] + 1], 1);
+            kind[h] = la[h] && lb[h] ? (la[h] - 1) * LIMBS + lb[h] - 1 : -1;
+            nth[h] = kind[h] >= 0 ? atomicAdd(&s_count[kind[h]], 1) : 0;
         }
         __syncthreads();
-        if (threadIdx.x == 0) {
-            int sum = 0;
-            for (int i = 0; i < 16; i++) {
-                s_place[i] = sum;
-                sum += s_count[i + 1];
-                s_count[i + 1] = sum;
+        // lane i of every wave: blocks of kind i, and the first step of the kind behind it
+        const int blocks = lane < KINDS ? s_count[lane] : 0, per = limb_per_step(lane % KINDS);
+        int behind = (blocks + (1 << per) - 1) >> per;
+        const int own_steps = behind;
+#pragma unroll
+        for (int off = 1; off < KINDS; off <<= 1) {
+            const int o = __shfl_up(behind, off, 64);
+            if (lane >= off) behind += o;
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int at = kind[h] < 0 ? 0 : kind[h], each = limb_per_step(at);
+            const int first = __shfl(behind - own_steps, at, 64);
+            if (kind[h] < 0) continue;
+            uint16_t *d = &s_desc[first + (nth[h] >> each)][(nth[h] & ((1 << each) - 1)) * (la[h] + lb[h])];
+            const int plane = (h * 256 + (int)threadIdx.x) * LIMBS;
+#pragma unroll
+            for (int l = 0; l < LIMBS; l++) {
+                if (l < la[h]) d[l] = (uint16_t)(plane + l);
+                if (l < lb[h]) d[la[h] + l] = (uint16_t)(0x8000 + plane + l);
             }
         }
         __syncthreads();
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-            if (kind[h] >= 0) s_list[atomicAdd(&s_place[kind[h]], 1)] = (uint16_t)(h * 256 + threadIdx.x);
-        __syncthreads();
 
-        const int8_t *srcA = plA + (int64_t)bi * nkb * (LIMBS * LIMB_PLANE) + wr * 2048 + lane * 16;
-        const int8_t *srcB = plB + (int64_t)bj * nkb * (LIMBS * LIMB_PLANE) + wc * 2048 + lane * 16;
+        // ---- loads: wave w brings planes w and w + 4 of a step; lane i holds what they are in step 64 n + i
+        const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)&s_planes[0][0][0] + wave * LIMB_PLANE;
+        const unsigned char *baseA = reinterpret_cast<const unsigned char *>(plA) + (int64_t)bi * nkb * (LIMBS * LIMB_PLANE);
+        const unsigned char *baseB = reinterpret_cast<const unsigned char *>(plB) + (int64_t)bj * nkb * (LIMBS * LIMB_PLANE);
+        const uint32_t voff = lane * 16;
+        uint32_t desc[2] = {NO_PLANE, NO_PLANE};
+        int step = 0;                                           // the one whose loads are issued next
+        auto issue = [&]() {
+            if ((step & 63) == 0) {
+                const int s = step + lane;
+#pragma unroll
+                for (int h = 0; h < 2; h++) desc[h] = s < nkb + KINDS ? s_desc[s][wave + 4 * h] : NO_PLANE;
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const uint32_t d = __builtin_amdgcn_readlane(desc[h], step & 63);
+                if (d != NO_PLANE) {
+                    const unsigned char *from = (d & 0x8000u ? baseB : baseA) + (int64_t)(d & 0x7fffu) * LIMB_PLANE;
+                    const uint32_t to = lds_base + ((step & 1) * LIMB_STEP + 4 * h) * LIMB_PLANE;
+                    dma_load<0>(from, voff, to);
+                    dma_load<1024>(from, voff, to);
+                    dma_load<2048>(from, voff, to);
+                    dma_load<3072>(from, voff, to);
+                }
+            }
+            step++;
+        };
+        issue();
         i32x4 acc[ORDERS][2][2];
 #pragma unroll
         for (int o = 0; o < ORDERS; o++)
 #pragma unroll
             for (int t = 0; t < 4; t++) acc[o][t >> 1][t & 1] = i32x4{0, 0, 0, 0};
-        static_for<LIMBS * LIMBS>([&](auto kind_) {
+        const unsigned char *vecs = &s_planes[0][0][0] + lane * 16;
+        static_for<KINDS>([&](auto kind_) {
             constexpr int LA = decltype(kind_)::value / LIMBS + 1, LB = decltype(kind_)::value % LIMBS + 1;
-            const int s = __builtin_amdgcn_readfirstlane(s_count[decltype(kind_)::value]);
-            const int e = __builtin_amdgcn_readfirstlane(s_count[decltype(kind_)::value + 1]);
-            if (s == e) return;
-            struct Frags {
-                i32x4 a[LA][2], b[LB][2];
-            };
-            auto load = [&](Frags &f, int i) {
-                const int64_t off = (int64_t)__builtin_amdgcn_readfirstlane((int)s_list[i < e ? i : e - 1]) * (LIMBS * LIMB_PLANE);
+            constexpr int PER = 1 << limb_per_step(decltype(kind_)::value);
+            for (int left = __builtin_amdgcn_readlane(blocks, decltype(kind_)::value); left > 0; left -= PER) {
+                __builtin_amdgcn_s_setprio(0);
+                __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
+                __syncthreads();       // the step's planes are there for all waves, and all have read the step before
+                const unsigned char *half = vecs + (step - 1 & 1) * (LIMB_STEP * LIMB_PLANE);
+                issue();
+                i32x4 a[PER][LA][2], b[PER][LB][2];
 #pragma unroll
-                for (int l = 0; l < LA; l++)
+                for (int e = 0; e < PER; e++) {
 #pragma unroll
-                    for (int t = 0; t < 2; t++) f.a[l][t] = *reinterpret_cast<const i32x4 *>(srcA + off + l * LIMB_PLANE + t * 1024);
+                    for (int l = 0; l < LA; l++)
 #pragma unroll
-                for (int l = 0; l < LB; l++)
+                        for (int t = 0; t < 2; t++)
+                            a[e][l][t] = *reinterpret_cast<const i32x4 *>(half + (e * (LA + LB) + l) * LIMB_PLANE + (2 * wr + t) * 1024);
 #pragma unroll
-                    for (int t = 0; t < 2; t++) f.b[l][t] = *reinterpret_cast<const i32x4 *>(srcB + off + l * LIMB_PLANE + t * 1024);
-            };
-            auto multiply = [&](const Frags &f) {
+                    for (int l = 0; l < LB; l++)
 #pragma unroll
-                for (int i = 0; i < LA; i++)
-#pragma unroll
-                    for (int j = 0; j < LB; j++)
-#pragma unroll
-                        for (int t = 0; t < 4; t++)
-                            acc[i + j][t >> 1][t & 1] =
-                                __builtin_amdgcn_mfma_i32_16x16x64_i8(f.a[i][t >> 1], f.b[j][t & 1], acc[i + j][t >> 1][t & 1], 0, 0, 0);
-            };
-            if constexpr (LA + LB <= 6) {
-                Frags f0, f1;
-                load(f0, s);
-                int i = s;
-                for (; i + 1 < e; i += 2) {
-                    load(f1, i + 1);
-                    multiply(f0);
-                    load(f0, i + 2);
-                    multiply(f1);
+                        for (int t = 0; t < 2; t++)
+                            b[e][l][t] = *reinterpret_cast<const i32x4 *>(half + (e * (LA + LB) + LA + l) * LIMB_PLANE + (2 * wc + t) * 1024);
                 }
-                if (i < e) multiply(f0);
-            } else {            // (two sets of operands would not fit the registers; the other wave of the SIMD multiplies meanwhile)
-                for (int i = s; i < e; i++) {
-                    Frags f;
-                    load(f, i);
-                    multiply(f);
+                __builtin_amdgcn_s_setprio(1);         // (the SIMD's other wave is another workgroup's: 1 %)
+#pragma unroll
+                for (int e = 0; e < PER; e++) {
+                    if (e && left <= e) break;
+#pragma unroll
+                    for (int i = 0; i < LA; i++)
+#pragma unroll
+                        for (int j = 0; j < LB; j++)
+#pragma unroll
+                            for (int t = 0; t < 4; t++)
+                                acc[i + j][t >> 1][t & 1] =
+                                    __builtin_amdgcn_mfma_i32_16x16x64_i8(a[e][i][t >> 1], b[e][j][t & 1], acc[i + j][t >> 1][t & 1], 0, 0, 0);
                 }
             }
         });
@@ -398,23 +473,21 @@ __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict
         for (int t = 0; t < 4; t++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const double c = (double)src[((t >> 1) * 16 + i) * N + (t & 1) * 16];
+                const double cd = (double)src[((t >> 1) * 16 + i) * N + (t & 1) * 16];
                 const long long lo = (long long)acc[0][t >> 1][t & 1][i] + ((long long)acc[1][t >> 1][t & 1][i] << 8) +
                                      ((long long)acc[2][t >> 1][t & 1][i] << 16) + ((long long)acc[3][t >> 1][t & 1][i] << 24);
                 const long long hi = (long long)acc[4][t >> 1][t & 1][i] + ((long long)acc[5][t >> 1][t & 1][i] << 8) +
                                      ((long long)acc[6][t >> 1][t & 1][i] << 16);
                 const double d = fma((double)(hi + (lo >> 32)), 4294967296.0, (double)(unsigned int)lo) * (1.0 / 281474976710656.0);
-                e2 += (c - d) * (c - d);
+                e2 += (cd - d) * (cd - d);
                 d2 += d * d;
-                c2 += c * c;
+                c2 += cd * cd;
             }
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        e2 += __shfl_down(e2, off, 64);
-        d2 += __shfl_down(d2, off, 64);
-        c2 += __shfl_down(c2, off, 64);
-    }
-    if (lane == 0) {
+    e2 = wave_sum(e2);
+    d2 = wave_sum(d2);
+    c2 = wave_sum(c2);
+    if (lane == 63) {
         red[wave][0] = e2;
         red[wave][1] = d2;
         red[wave][2] = c2;
@@ -540,7 +613,8 @@ static int64_t limb_kb(int64_t K) { return (K + LIMB_BLOCK - 1) / LIMB_BLOCK; }
 // values too large for limbs, by the estimates' ratio: 1.5, 65536 x 1024 x 64 155 -> 178 | 69 | 185; 2.2, 512 x 384 x 512
 // 31.2 -> 32.2 | 31.8 | 35.8; 2.5, 4096 x 256 x 512 38 -> 35.8 | 31.0 | 43.2 and 1024 x 512 x 1024 39.2 -> 38.5 | 35.8 | 41.2;
 // 2.8, 512^3 35.9 -> 34.9 | 33.9 | 40.1 and 65536 x 512 x 128 158 -> 120 | 62 | 172; 3.9, 1024^3 57 -> 49.4 | 44.4 | 59.5; 7.6,
-// 65536 x 512 x 256 289 -> 186 | 87 | 311; 10, 1280^3 106 -> 64 | 55 | 111.  With K below 256 a block's fixed costs outweigh its
+// 65536 x 512 x 256 289 -> 186 | 87 | 311; 10, 1280^3 106 -> 64 | 55 | 111.  (Whole numbers as they were with operands loaded to
+// registers; the product takes less since: 512^3 31 | 30, 65536 x 512 x 128 107 | 58, 1024^3 43.4 | 39.6, 1280^3 58 | 48.)  With K below 256 a block's fixed costs outweigh its
 // few products: 4096 x 64 x 4096 61 -> 82 | 73 | 68, K = 128 94 -> 94 | 74 | 102, K = 256 158 -> 118 | 79 | 164.
 size_t limb_bytes(int64_t rows, int64_t K, int64_t N, int n_cu) {
     if (K > LIMB_MAX_K || K < 256) return 0;

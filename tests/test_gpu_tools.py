@@ -398,6 +398,30 @@ def test_error_report_over_the_range_of_fp16(ctx, tile, M, K, N, row0, rows, kin
             assert abs(g - ref) <= 1e-9 * ref
 
 
+@pytest.mark.parametrize("K", [4096 - 32, 4096, 64 * 66, 16384 + 64])
+def test_error_report_by_steps_of_every_kind(ctx, K):
+    """Blocks of 64 k that need 0 to 4 bytes on either side, drawn so that every pair of them occurs an odd number of times here and
+    an even one there: steps with one block, some and all they can hold, 64 steps and more of one block of C, a last
+    block of 32 k.  The exact product of whole multiples of 2^-24 on both sides; sums of squares in another order, 1e-9."""
+    import torch
+    rng = np.random.default_rng(K)
+    M = N = 512
+    nkb = -(-K // 64)
+
+    def scales(n):
+        s = np.exp2(rng.choice([-40.0, -20.0, -12.0, -4.0, 5.0], (8, n), p=[0.1, 0.25, 0.25, 0.25, 0.15]))
+        return np.kron(s, np.ones((64, 64)))[:, :K]
+    A = (rng.uniform(-1.0, 1.0, (M, K)) * scales(nkb)).astype(np.float16)
+    B = (rng.uniform(-1.0, 1.0, (K, N)) * scales(nkb).T).astype(np.float16)
+    dense = A.astype(np.float64) @ B.astype(np.float64)
+    C = (0.75 * dense).astype(np.float32)
+    ctx.normmap_f16(1, torch.from_numpy(B).cuda(), 32)
+    ctx.normmap_f16(0, torch.from_numpy(A).cuda(), 32)
+    got = ctx.error_vs_dense(torch.from_numpy(C).cuda())
+    for g, ref in zip(got, (np.linalg.norm(C - dense), np.linalg.norm(dense), np.linalg.norm(C.astype(np.float64)))):
+        assert abs(g - ref) <= 1e-9 * ref
+
+
 def test_error_report_rounds_once(ctx):
     """21800 products of 257 / 512 with itself, 10900 of minus twice that by values with other digits, and one of 2^-24 with
     itself: the upper and the lower orders of a sum pass 2^53 and cancel, and what is left is the last product."""

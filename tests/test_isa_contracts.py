@@ -368,3 +368,13 @@ def test_bisection_publishes_when_its_workspace_is_at_rest(tmp_path):
             assert not any(re.match(r"\.LBB|s_cbranch|s_branch|global_|flat_", ln) for ln in rest[:barrier]) and asm[1] + 1 + barrier < last
             clears = [i for i, ln in enumerate(lines) if ln.startswith("global_store") and asm[0] < i < last]
             assert len(clears) >= 4, clears
+
+
+def test_integer_product_keeps_the_same_distance(tmp_path):
+    """kernels_tools.hip: the planes' addresses come through v_readlane, and the global->LDS loads take what scalar instructions
+    make of it; the accumulators of seven orders stay in registers."""
+    text = _isa("kernels_tools.hip", tmp_path)
+    found, checked = _hazards(_instructions(text), "global_load_lds_dwordx4", 5)
+    assert not found and checked > 20, found
+    ((_, body),) = re.findall(r"^(_ZN5spamm13k_error_limbs\w+):[^\n]*\n(.*?)^\.Lfunc_end", text, flags=re.S | re.M)
+    assert not any(mn.startswith("scratch_") for mn, _, _ in _instructions(body))
