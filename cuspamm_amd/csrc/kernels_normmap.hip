@@ -12,6 +12,8 @@
 //   exact in fp32); chunk index c = r*(b/8)+q; lane L = c%64 accumulates
 //   chunks c = L, 64+L, 128+L, ... in ascending order; then a 6-step xor
 //   butterfly (1,2,4,8,16,32) across the 64 lanes; norm = sqrtf(sum).
+#include <type_traits>
+
 #include "spamm_internal.h"
 
 namespace spamm {
@@ -56,6 +58,13 @@ __device__ __forceinline__ float butterfly64(float v) {
 //   store   after one barrier: the tiles are copied out with contiguous 1 KiB wave stores (a
 //           packed tile is one contiguous block in memory), and one wave per tile applies the
 //           canonical reduction.
+// KEEP: the input's lines stay in the caches (keep_input).
+template <bool KEEP, typename T>
+__device__ __forceinline__ T load_strip(const T *from) {
+    if constexpr (KEEP) return *from;
+    else return __builtin_nontemporal_load(from);
+}
+
 template <int B, int SW, int PH>
 struct NormCfg {
     static constexpr int TPP = SW / B / PH;          // tiles resident in LDS together
@@ -66,13 +75,14 @@ struct NormCfg {
     static constexpr int CH = B * PITCH;             // floats per tile in the chunk-sum table
 };
 
-// `strip`: which strip of the operand; s_pack / s_chunk / s_skip: NormCfg's TPP * TS bytes, TPP * CH floats, TPP ints of LDS
-template <int B, int ROLE, int SW, bool IN16, int PH, int NWV>
+// `strip`: which strip of the operand; s_pack / s_chunk / s_skip / s_seen: NormCfg's TPP * TS bytes, TPP * CH floats, TPP and NWV
+// ints of LDS
+template <int B, int ROLE, int SW, bool IN16, int PH, int NWV, bool KEEP>
 __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64_t ld, int64_t cols, int64_t nbr, int64_t nbc,
                                               int64_t nstrip, uint4 *__restrict__ packed, float *__restrict__ nm,
                                               float *__restrict__ nmT, uint4 *__restrict__ packed2, float *__restrict__ nm2,
-                                              const float *__restrict__ rowmax, float tau_skip, unsigned strip,
-                                              unsigned char *s_pack, float *s_chunk, int *s_skip) {
+                                              const float *__restrict__ rowmax, float tau_skip, bool keep_copy, unsigned strip,
+                                              unsigned char *s_pack, float *s_chunk, int *s_skip, int *s_seen) {
     using L = NormCfg<B, SW, PH>;
     constexpr int TPS = SW / B;           // tiles per strip
     constexpr int TPP = TPS / PH;         // tiles per phase (resident in LDS together)
@@ -121,7 +131,7 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
         for (int i = 0; i < NGW; i++)
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                h16[i][j] = __builtin_nontemporal_load(
+                h16[i][j] = load_strip<KEEP>(
                     reinterpret_cast<const u32x4n *>(src + (int64_t)(8 * (g0 + GSTEP * i) + j) * ld));
             }
         if (!valid) {
@@ -139,7 +149,7 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
                 if (!valid)
                     v[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                 else
-                    v[i][j] = __builtin_nontemporal_load(
+                    v[i][j] = load_strip<KEEP>(
                         reinterpret_cast<const f32x4 *>(static_cast<const float *>(Xv) + eoff + (int64_t)r * ld));
             }
     }
@@ -147,6 +157,8 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
     // B role writes 8 neighbouring x per lane, lanes 128 bytes apart: the low three bits of x are
     // xor-ed with the next three so that the lanes of one store spread over the banks.
     auto vpos = [](int x, bool swz) -> int { return swz ? (x ^ ((x >> 3) & 7)) : x; };
+
+    float seen = 0.0f;                                // sum of the chunk sums that the lane has staged
 
     // ROLE 2 = the same matrix is both operands (A = B): one read of X, both packed layouts and
     // both norm maps (A role first -> packed/nm, then B role -> packed2/nm2/nmT), LDS reused.
@@ -167,6 +179,7 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
                     for (int e = 0; e < 8; e++) { const float f = (float)hv[e]; s8 = s8 + f * f; }
                     *reinterpret_cast<u32x4n *>(s_pack + t * TS + q * QS + r * 16) = h16[i][j];
                     s_chunk[t * CH + r * PITCH + q] = s8;
+                    seen += s8;
                 }
         } else {
 #pragma unroll
@@ -190,6 +203,7 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
                 o.y = __builtin_bit_cast(uint32_t, p1);
                 *reinterpret_cast<uint2 *>(s_pack + t * TS + q * QS + r * 16 + h * 8) = o;
                 if (h) s_chunk[t * CH + r * PITCH + q] = s8;
+                seen += s8;
             }
         }
     };
@@ -218,6 +232,7 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
                     *reinterpret_cast<u32x4n *>(s_pack + t * TS + kg * QS + vpos(cin + c, true) * 16) =
                         __builtin_bit_cast(u32x4n, o);
                     s_chunk[t * CH + (cin + c) * PITCH + kg] = sc_;
+                    seen += sc_;
                 }
             }
         } else {
@@ -246,12 +261,13 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
             for (int c = 0; c < 4; c++) {
                 *reinterpret_cast<uint4 *>(s_pack + t * TS + kg * QS + (cin + c) * 16) = o[c];
                 s_chunk[t * CH + (cin + c) * PITCH + kg] = s[c];
+                seen += s[c];
             }
         }
         }
     };
     // packed tiles out (256 threads x 16 bytes = 4 KiB per step, contiguous per tile)
-    auto copy_out = [&](int ph, bool as_b, uint4 *__restrict__ pk, bool prune) {
+    auto copy_out_as = [&](int ph, bool as_b, uint4 *__restrict__ pk, bool prune, auto keep) {
 #pragma unroll
         for (int i = 0; i < TPP * VPT / (64 * NWV); i++) {
             const int vi = threadIdx.x + 64 * NWV * i;
@@ -260,9 +276,20 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
             if (Jt < nbc && !(prune && s_skip[tt])) {
                 const uint4 d = *reinterpret_cast<const uint4 *>(s_pack + tt * TS + (iv / B) * QS + vpos(iv % B, IN16 && as_b) * 16);
                 const int64_t tile = as_b ? Jt * nbr + I : I * nbc + Jt;
-                __builtin_nontemporal_store(*reinterpret_cast<const u32x4n *>(&d), reinterpret_cast<u32x4n *>(pk + tile * VPT + iv));
+                const u32x4n dv = *reinterpret_cast<const u32x4n *>(&d);
+                u32x4n *to = reinterpret_cast<u32x4n *>(pk + tile * VPT + iv);
+                if constexpr (decltype(keep)::value) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" :: "v"(to), "v"(dv) : "memory");
+                else __builtin_nontemporal_store(dv, to);
             }
         }
+    };
+    // (a strip of nothing but zeros, which no threshold above zero keeps, is not left in the cache)
+    auto copy_out = [&](int ph, bool as_b, uint4 *__restrict__ pk, bool prune) {
+        int any = 0;
+#pragma unroll
+        for (int w = 0; w < NWV; w++) any |= s_seen[w];
+        if (keep_copy && __builtin_amdgcn_readfirstlane(any)) copy_out_as(ph, as_b, pk, prune, std::true_type{});
+        else copy_out_as(ph, as_b, pk, prune, std::false_type{});
     };
     // norms: one wave per tile, canonical order.  With `prune` (tau known and positive) the wave
     // also decides whether any product can keep the tile.  The A pass of its own has the row maxima
@@ -297,7 +324,10 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
 #pragma unroll
         for (int ph = 0; ph < PH; ph++) {
             if (ph) __syncthreads();           // the previous phase's tiles have been copied out
+            seen = 0.0f;
             if (as_b) stage_b(ph); else stage_a(ph);
+            const bool used = __ballot(seen != 0.0f) != 0ull;
+            if (lane == 0) s_seen[wave] = used;
             __syncthreads();
             if (prune) {
                 norms(ph, as_b, nmo, nmTo, true);
@@ -322,38 +352,38 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
     }
 }
 
-template <int B, int ROLE, int SW, bool IN16, int PH = 1, int NWV = 4>
+template <int B, int ROLE, int SW, bool IN16, int PH = 1, int NWV = 4, bool KEEP = false>
 __global__ __launch_bounds__(64 * NWV, 1) void k_normmap(
     const void *__restrict__ Xv, int64_t ld, int64_t cols, int64_t nbr, int64_t nbc, int64_t nstrip, uint4 *__restrict__ packed,
     float *__restrict__ nm, float *__restrict__ nmT, uint4 *__restrict__ packed2, float *__restrict__ nm2,
-    const float *__restrict__ rowmax, float tau_skip) {
+    const float *__restrict__ rowmax, float tau_skip, bool keep_copy) {
     using L = NormCfg<B, SW, PH>;
     __shared__ __attribute__((aligned(16))) unsigned char s_pack[L::TPP * L::TS];
     __shared__ float s_chunk[L::TPP * L::CH];
-    __shared__ int s_skip[L::TPP];
-    normmap_strip<B, ROLE, SW, IN16, PH, NWV>(Xv, ld, cols, nbr, nbc, nstrip, packed, nm, nmT, packed2, nm2, rowmax, tau_skip,
-                                              blockIdx.x, s_pack, s_chunk, s_skip);
+    __shared__ int s_skip[L::TPP], s_seen[NWV];
+    normmap_strip<B, ROLE, SW, IN16, PH, NWV, KEEP>(Xv, ld, cols, nbr, nbc, nstrip, packed, nm, nmT, packed2, nm2, rowmax, tau_skip,
+                                              keep_copy, blockIdx.x, s_pack, s_chunk, s_skip, s_seen);
 }
 
 // Both operands in one launch: the first n_b workgroups are B's strips, the others A's.  One after the other,
 // small passes are a few microseconds of memory latency each; together they share it (and neither sees the
 // other's norms: a tau-aware call then leaves out tiles of norm zero only, in both copies).
-template <int B, int SW, bool IN16, int PH, int NWV>
+template <int B, int SW, bool IN16, int PH, int NWV, bool KEEP = false>
 __global__ __launch_bounds__(64 * NWV) void k_normmap_pair(const void *__restrict__ A, const void *__restrict__ Bm, int64_t nbM,
                                                            int64_t nbK, int64_t nbN, unsigned n_b, int64_t strips_a, int64_t strips_b,
                                                            uint4 *__restrict__ packedA, uint4 *__restrict__ packedB,
                                                            float *__restrict__ nmA, float *__restrict__ nmB,
-                                                           float *__restrict__ nmBt, float tau_skip) {
+                                                           float *__restrict__ nmBt, float tau_skip, bool keep_copy) {
     using L = NormCfg<B, SW, PH>;
     __shared__ __attribute__((aligned(16))) unsigned char s_pack[L::TPP * L::TS];
     __shared__ float s_chunk[L::TPP * L::CH];
-    __shared__ int s_skip[L::TPP];
+    __shared__ int s_skip[L::TPP], s_seen[NWV];
     if (blockIdx.x < n_b)
-        normmap_strip<B, 1, SW, IN16, PH, NWV>(Bm, nbN * B, nbN * B, nbK, nbN, strips_b, packedB, nmB, nmBt, nullptr, nullptr,
-                                               nullptr, tau_skip, blockIdx.x, s_pack, s_chunk, s_skip);
+        normmap_strip<B, 1, SW, IN16, PH, NWV, KEEP>(Bm, nbN * B, nbN * B, nbK, nbN, strips_b, packedB, nmB, nmBt, nullptr, nullptr,
+                                               nullptr, tau_skip, keep_copy, blockIdx.x, s_pack, s_chunk, s_skip, s_seen);
     else
-        normmap_strip<B, 0, SW, IN16, PH, NWV>(A, nbK * B, nbK * B, nbM, nbK, strips_a, packedA, nmA, nullptr, nullptr, nullptr,
-                                               nullptr, tau_skip, blockIdx.x - n_b, s_pack, s_chunk, s_skip);
+        normmap_strip<B, 0, SW, IN16, PH, NWV, KEEP>(A, nbK * B, nbK * B, nbM, nbK, strips_a, packedA, nmA, nullptr, nullptr, nullptr,
+                                               nullptr, tau_skip, keep_copy, blockIdx.x - n_b, s_pack, s_chunk, s_skip, s_seen);
 }
 
 // rowmax[k] = max_j nB[k, j] (nB row-major [nbK x nbN]); one wave per row.  NaNs are ignored:
@@ -441,22 +471,47 @@ __global__ __launch_bounds__(256) void k_fill_decay(float *__restrict__ X, int64
 // ---------------------------------------------------------------- launchers
 constexpr unsigned NARROW_STRIPS = 512;     // of 256 columns, in a launch: two per CU
 
+// Which of a pass's accesses leave their lines in the 256 MB memory-side cache.  Whole calls on three sets of operands and
+// workspaces in turn, so that nothing of a call is there when the set comes round again.
+// Copies, written through (sc1) instead of non-temporally up to 448 MiB an operand: the multiply reads them, or what of them
+// still lies there, from that cache.  1056 x 1568 x 1312 17.4 -> 17.0 us, 2048^3 24.7 -> 23.0, 3072^3 47.0 -> 41.7, 4096^3 76 -> 64,
+// 6144^3 179 -> 169, 7168^3 238 -> 219, dense 8192^3 911 -> 888, 10240^3 513 -> 480, 12288^3 728 -> 706; fp16 4096^3 69.4 -> 56.8,
+// 8192^3 270 -> 257, 10048^3 425 -> 418, 14336^3 912 -> 890; A = B 4096^2 66 -> 57, 7168^2 202 -> 182, 9216^2 332 -> 312.  Beyond, the
+// copies drive each other out: 16384^3 1205 on both sides, tau-aware 1252 -> 1274; 20032^3 2052 -> 2067, tau-aware 1929 -> 1966.
+// Strips of nothing but zeros, most of a narrow band's operands, are written past it all the same: left out of that rule, and
+// then with it, 8192^3 of a band 278 -> 276 -> 261, A = B 235 -> 237 to 246 -> 224, 9216^2 332 -> 317 -> 309.
+// Input, by ordinary loads up to 32 MiB a launch: a producer's output of that size may be there.  2048^3 23.0 -> 21.8, fp16
+// 20.9 -> 19.6, 1056 x 1568 x 1312 17.0 -> 16.3, 1024 rows against a resident 8192^2 34.6 -> 33.1; beyond it takes the copies'
+// place (3072^3 41.8 -> 45.0, 4096^3 63.9 -> 69.3).
+constexpr int64_t KEEP_INPUT_MAX = 32ll << 20, KEEP_COPY_MAX = 448ll << 20;
+static bool keep_input(int64_t bytes) { return bytes <= KEEP_INPUT_MAX; }
+static bool keep_copy(int64_t bytes) { return bytes <= KEEP_COPY_MAX; }
+
 template <int ROLE, bool IN16>
 static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int tile, void *packed, float *nm,
                                  float *nmT, hipStream_t s, void *packed2 = nullptr, float *nm2 = nullptr,
                                  const float *rowmax = nullptr, float tau_skip = 0.0f) {
     const int64_t nbr = rows / tile, nbc = cols / tile;
+    const bool keep = keep_input(rows * cols * (IN16 ? 2 : 4));
     const auto strips = [&](int64_t sw) { return (unsigned)(nbr * ((cols + sw - 1) / sw)); };
-#define SPAMM_NORMMAP(T, SW, PH, NWV)                                                                                           \
-    k_normmap<T, ROLE, SW, IN16, PH, NWV><<<strips(SW), 64 * NWV, 0, s>>>(X, cols, cols, nbr, nbc, (cols + SW - 1) / SW, (uint4 *)packed, \
-                                                                          nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip)
+#define SPAMM_NORMMAP_(T, SW, PH, NWV, KEEP)                                                                                        \
+    k_normmap<T, ROLE, SW, IN16, PH, NWV, KEEP><<<strips(SW), 64 * NWV, 0, s>>>(X, cols, cols, nbr, nbc, (cols + SW - 1) / SW, (uint4 *)packed, \
+                                                                                nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip,   \
+                                                                                keep_copy(rows * cols * 2))
+#define SPAMM_NORMMAP(T, SW, PH, NWV) SPAMM_NORMMAP_(T, SW, PH, NWV, false)
+// (the shapes that inputs of up to KEEP_INPUT_MAX take, but for a few fp16 ones)
+#define SPAMM_NORMMAP_KEEP(T, SW, PH, NWV)                                                     \
+    do {                                                                                       \
+        if (keep) SPAMM_NORMMAP_(T, SW, PH, NWV, true);                                        \
+        else SPAMM_NORMMAP_(T, SW, PH, NWV, false);                                            \
+    } while (0)
     // strip widths and waves: one 8-row group per lane, at most ~42 KiB of LDS and so three workgroups or more per CU.
     // fp16 input: 256 columns, two rows per load (512 in phases before: tile 64 1024^2, both passes, 6.2 -> 4.1 us, 4096^2
     // 28.4 -> 26.3, 16384^2 A = B 303 -> 291; tile 32 2048^2 8.0 -> 7.3, 8192^2 tau-aware 93 -> 87).
     switch (tile) {
         case 32:
-            if constexpr (IN16) SPAMM_NORMMAP(32, 256, 1, 2);
-            else SPAMM_NORMMAP(32, 256, 1, 4);
+            if constexpr (IN16) SPAMM_NORMMAP_KEEP(32, 256, 1, 2);
+            else SPAMM_NORMMAP_KEEP(32, 256, 1, 4);
             break;
         case 64:
             // fp32 input: strips of 128 columns where there are few (1024^2, both passes: 5.4 -> 4.4 us; 4096^2 36.1 ->
@@ -468,8 +523,8 @@ static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int 
             // 3648^2 10.5 -> 10.1, 10.3 -> 10.5, 38.4 -> 36.4; 3584^2 8.9 -> 9.1, 9.5 -> 9.9, 37.0 -> 35.8
             if constexpr (IN16) {
                 if (strips(256) > 768u && strips(256) <= 1024u) SPAMM_NORMMAP(64, 512, 2, 8);
-                else SPAMM_NORMMAP(64, 256, 1, 4);
-            } else if (strips(256) <= NARROW_STRIPS) SPAMM_NORMMAP(64, 128, 1, 4);
+                else SPAMM_NORMMAP_KEEP(64, 256, 1, 4);
+            } else if (strips(256) <= NARROW_STRIPS) SPAMM_NORMMAP_KEEP(64, 128, 1, 4);
             else if (strips(256) <= 8192u) SPAMM_NORMMAP(64, 256, 1, 8);
             else SPAMM_NORMMAP(64, 256, 1, 4);
             break;
@@ -478,19 +533,21 @@ static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int 
         case 128:
             if constexpr (IN16) {
                 if constexpr (ROLE == 2) return hipErrorInvalidValue;      // (two passes, or the pair, are faster)
-                else SPAMM_NORMMAP(128, 128, 1, 4);
+                else SPAMM_NORMMAP_KEEP(128, 128, 1, 4);
             } else {
                 if constexpr (ROLE == 1)
                     if (strips(256) > 6000u) {
                         SPAMM_NORMMAP(128, 256, 2, 4);
                         break;
                     }
-                SPAMM_NORMMAP(128, 128, 1, 8);
+                SPAMM_NORMMAP_KEEP(128, 128, 1, 8);
             }
             break;
         default: return hipErrorInvalidValue;
     }
+#undef SPAMM_NORMMAP_KEEP
 #undef SPAMM_NORMMAP
+#undef SPAMM_NORMMAP_
     return hipGetLastError();
 }
 
@@ -505,8 +562,11 @@ static void launch_pair(const void *A, const void *Bm, int64_t nbM, int64_t nbK,
                         float *nmA, float *nmB, float *nmBt, float tau_skip, hipStream_t s) {
     const int64_t strips_a = (nbK * B + SW - 1) / SW, strips_b = (nbN * B + SW - 1) / SW;
     const unsigned n_b = (unsigned)(nbK * strips_b), n_a = (unsigned)(nbM * strips_a);
-    k_normmap_pair<B, SW, IN16, PH, NWV><<<n_a + n_b, 64 * NWV, 0, s>>>(A, Bm, nbM, nbK, nbN, n_b, strips_a, strips_b, (uint4 *)packedA,
-                                                                        (uint4 *)packedB, nmA, nmB, nmBt, tau_skip);
+    const int64_t a = nbM * nbK * B * B, b = nbK * nbN * B * B;
+    const bool keep = keep_input((a + b) * (IN16 ? 2 : 4));
+    (keep ? &k_normmap_pair<B, SW, IN16, PH, NWV, true> : &k_normmap_pair<B, SW, IN16, PH, NWV, false>)<<<n_a + n_b, 64 * NWV, 0, s>>>(
+        A, Bm, nbM, nbK, nbN, n_b, strips_a, strips_b, (uint4 *)packedA, (uint4 *)packedB, nmA, nmB, nmBt, tau_skip,
+        keep_copy(2 * (a > b ? a : b)));
 }
 
 // Where the two passes are worth running as one, by the strips of both operands, counted as tile rows of 1 KiB (256

@@ -322,6 +322,38 @@ def test_fp16_passes_of_three_to_four_strips_per_cu(orc, ctx):
         assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("tile", [32, 64, 128])
+@pytest.mark.parametrize("half", [False, True])
+def test_conversion_on_either_side_of_what_the_caches_keep(ctx, tile, half):
+    """Input of more than 32 MiB is read past the caches, less through them, by launches of their own: the halves of a matrix that
+    lies just beyond, one by one and as one, in both roles and with norms and values bit for bit; A = B by one read below."""
+    import torch
+    rows, cols = 512, (33280 if half else 16640) if tile < 128 else (33024 if half else 16640)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(tile)
+    X = torch.rand((rows, cols), generator=g, device="cuda") * 2.0 - 1.0
+    X = X.half() if half else X
+    assert X.numel() * X.element_size() > 32 << 20
+    convert = ctx.normmap_f16 if half else ctx.normmap_f32
+    bits = X.half().cpu().numpy().view(np.uint16)
+    for role in (1, 0):
+        for M in ((X, X[: rows // 2]) if role == 0 else (X, X[: rows // 2])):
+            other = torch.zeros((tile, M.shape[0]) if role == 1 else (M.shape[1], tile), dtype=X.dtype, device="cuda")
+            convert(1 - role, other, tile)
+            convert(role, M, tile)
+            assert np.array_equal(ctx.get_fp16(role), bits[: M.shape[0]])
+            nm = ctx.get_normmap(role)
+            if M is X:
+                whole = nm
+            else:
+                assert np.array_equal(nm.view(np.uint32), whole[: nm.shape[0]].view(np.uint32))
+    n = 1024
+    Y = X[:, :n].contiguous().repeat(2, 1)
+    two = ctx.multiply(Y, Y.clone(), tile, 0.0)
+    assert torch.equal(ctx.multiply(Y, Y, tile, 0.0, a_eq_b=True), two)
+    assert np.array_equal(ctx.get_fp16(0), Y.half().cpu().numpy().view(np.uint16)) and np.array_equal(ctx.get_fp16(1), ctx.get_fp16(0))
+
+
 @pytest.mark.parametrize("rows,N,row0", [(2048, 1024, 64), (512, 512, 0), (4096, 2048, 0), (2112, 960, 0)])
 def test_error_report_by_any_block_shape(ctx, rows, N, row0):
     """A wave of the exact product owns 64 x 32 of C (the first case, on 256 CUs), 32 x 32, 64 x 64, or what the grid
