@@ -9,6 +9,11 @@
 // counts, kept total -- is written on the way out; the macro tiles' work lists, which
 // nothing reads after this kernel, are built by k_gate if somebody asks for them.
 //
+// A unit's life, fp16 2048^3 at tile 32, 5 % kept, us: gate 2.0 (most of it the norms' round trip), list 0.3, first stages 0.8, 9 to
+// 14 stages 3.4 to 6, C 1.5.  With 64-bit places, divisions by the grid's sizes, a scan for the one word of 64 k that most lists
+// are, and counts formed behind C's stores it was 1 us longer (whole calls: 256^3 10.5 -> 9.8 us, 1024^3 11.6 -> 10.6, 1056 x 1568 x
+// 1312 16.3 -> 15.5, this one 19.5 -> 18.4, 4096^2 of a band 57.9 -> 56.2).
+//
 // Of the k loop's 0.285 us per stage on 256 CUs (2048^3 dense) the loads alone take 0.2 (a bare copy of the same panels into
 // LDS, 21 TB/s over the chip), all else without them 0.18; without the MFMAs 0.27, without the LDS reads 0.285.  Two stages
 // per sync, rings of 6 and 8 and square blocks of units per XCD changed it by 1 % or cost workgroups per CU.
@@ -58,14 +63,22 @@ size_t small_lds_bytes_(int stage_bytes, int nbuf, int tt, int64_t nbK) {
     return (size_t)stage_bytes * nbuf + words * 64 * 4 + words * tt * 8 + words * 16 + words * 64 * 2;
 }
 
+// Offsets are 32-bit: C has SMALL_MAX_UNITS units of 128 x 128 at most and K / B is at most SMALL_MAX_NBK, so that C, the norm
+// maps and the masks stay below 2^31 bytes (the packed operands need not).
+struct SmallGrid {
+    int nMacN;
+    uint32_t mac_rec;        // floor((2^32 - 1) / nMacN): the macro row of macro tile m is the upper half of (m + 1) * mac_rec
+    int n_units, chunk;      // units, and per XCD
+    int xcd_shift, mode;     // log2 of the XCDs
+};
+
 template <int B, int U, int RING>
 __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict__ pA, const unsigned char *__restrict__ pB, const GateBuffers &g,
-                                                int nbM, int nbK, int nbN, int nMacN, int n_units, int n_xcd, int mode, float tau,
-                                                int64_t M, int64_t N, float *__restrict__ C) {
+                                                int nbM, int nbK, int nbN, const SmallGrid &sg, float tau, float *__restrict__ C) {
     using H = SmallCfg<B, U, RING>;
     constexpr int NBUF = H::NBUF, MT = H::MT, TU = H::TU, TT = H::TT, NB = H::NB;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    const int words = (nbK + 63) >> 6;
+    const int words = (nbK + 63) >> 6, mode = sg.mode;
     uint32_t *s_list = reinterpret_cast<uint32_t *>(smem + NBUF * H::STAGE_BYTES);   // k | tile bits << 16
     uint64_t *s_word = reinterpret_cast<uint64_t *>(s_list + words * 64);            // [words][TT]
     uint64_t *s_fp = s_word + words * TT;                                            // [words][2]
@@ -75,44 +88,68 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wr = wave >> 1, wc = wave & 1;
     // consecutive units (neighbours share operand panels) in equal chunks, one per XCD
-    const int chunk = (n_units + n_xcd - 1) / n_xcd;
-    const int unit = ((int)blockIdx.x % n_xcd) * chunk + (int)blockIdx.x / n_xcd;
-    if (unit >= n_units) return;
-    const int macro = unit / (H::PD * H::PD), part = unit % (H::PD * H::PD);
-    const int mi = macro / nMacN, mj = macro % nMacN, ui = part / H::PD, uj = part % H::PD;
-    const int64_t urow = (int64_t)mi * 256 + ui * U, ucol = (int64_t)mj * 256 + uj * U;
+    const uint32_t unit = (blockIdx.x & ((1u << sg.xcd_shift) - 1u)) * (uint32_t)sg.chunk + (blockIdx.x >> sg.xcd_shift);
+    if (unit >= (uint32_t)sg.n_units) return;
+    const uint32_t macro = unit / (H::PD * H::PD), part = unit % (H::PD * H::PD), ui = part / H::PD, uj = part % H::PD;
+    const int mi = (int)__umulhi(macro + 1u, sg.mac_rec), mj = (int)macro - mi * sg.nMacN;
+    const int M = nbM * B, N = nbN * B;
+    const int urow = mi * 256 + (int)ui * U, ucol = mj * 256 + (int)uj * U;
     if (urow >= M || ucol >= N) return;
-    const int ti0 = (int)(urow / B), tj0 = (int)(ucol / B);            // first tile of the unit
+    const int ti0 = urow / B, tj0 = ucol / B;                          // first tile of the unit
 
     // ---- gate: a wave takes 64 k at a time, lane = k, and holds the norms of the macro tile's rows and
-    // columns (loads unconditional, from clamped addresses)
+    // columns (loads unconditional, from clamped addresses), the next 64's on their way
     const bool multiply = (mode & SMALL_MULTIPLY) != 0;        // (the gate alone needs no list, and the unit's norms only)
     const bool interior = (mi + 1) * MT <= nbM && (mj + 1) * MT <= nbN;
-    for (int w = wave; w < words; w += 4) {
-        const int k = w * 64 + lane, kc = k < nbK ? k : nbK - 1;
-        const bool live = k < nbK;
-        float a[MT] = {}, b[MT] = {}, au[TU], bu[TU];
+    const int rows_in = nbM - ti0 < TU ? nbM - ti0 : TU, cols_in = nbN - tj0 < TU ? nbN - tj0 : TU;
+    uint32_t inside = (1u << cols_in) - 1u;                            // the unit's tiles that exist
 #pragma unroll
-        for (int x = 0; x < TU; x++) {
-            au[x] = g.nA[(int64_t)(ti0 + x < nbM ? ti0 + x : nbM - 1) * nbK + kc];
-            bu[x] = g.nBt[(int64_t)(tj0 + x < nbN ? tj0 + x : nbN - 1) * nbK + kc];
-        }
+    for (int x = 1; x < TU; x++) inside |= x < rows_in ? ((1u << cols_in) - 1u) << (x * TU) : 0u;
+    float a[MT] = {}, b[MT] = {}, au[TU], bu[TU];
+    auto load_norms = [&](int w) {
+        const int k = w * 64 + lane;
+        const uint32_t kb = (uint32_t)(k < nbK ? k : nbK - 1) * 4u;
+        auto norm = [&](const float *map, int row, int n) {
+            const uint32_t at = (uint32_t)((row < n ? row : n - 1) * nbK) * 4u + kb;
+            return *reinterpret_cast<const float *>(reinterpret_cast<const unsigned char *>(map) + at);
+        };
         if (multiply) {
 #pragma unroll
             for (int x = 0; x < MT; x++) {
-                const int i = mi * MT + x, j = mj * MT + x;
-                a[x] = g.nA[(int64_t)(i < nbM ? i : nbM - 1) * nbK + kc];
-                b[x] = g.nBt[(int64_t)(j < nbN ? j : nbN - 1) * nbK + kc];
+                a[x] = norm(g.nA, mi * MT + x, nbM);
+                b[x] = norm(g.nBt, mj * MT + x, nbN);
+            }
+        } else {
+#pragma unroll
+            for (int x = 0; x < TU; x++) {
+                au[x] = norm(g.nA, ti0 + x, nbM);
+                bu[x] = norm(g.nBt, tj0 + x, nbN);
+            }
+        }
+    };
+    if (wave < words) load_norms(wave);
+    const int anchor = multiply ? list_anchor(mi, mj, MT, nbM, nbK, nbN) : 0;
+    for (int w = wave; w < words; w += 4) {
+        const int k = w * 64 + lane;
+        const bool live = k < nbK;
+        if (multiply) {                                                // the unit's among the macro tile's
+#pragma unroll
+            for (int x = 0; x < TU; x++) {
+                au[x] = a[x];
+                bu[x] = b[x];
+#pragma unroll
+                for (int o = TU; o < MT; o += TU) {
+                    au[x] = ti0 - mi * MT == o ? a[o + x] : au[x];
+                    bu[x] = tj0 - mj * MT == o ? b[o + x] : bu[x];
+                }
             }
         }
         uint32_t ub = 0;
 #pragma unroll
         for (int x = 0; x < TU; x++)
 #pragma unroll
-            for (int y = 0; y < TU; y++) {
-                const bool inside = ti0 + x < nbM && tj0 + y < nbN;
-                if (inside && live && au[x] * bu[y] >= tau) ub |= 1u << (x * TU + y);
-            }
+            for (int y = 0; y < TU; y++) ub |= au[x] * bu[y] >= tau ? 1u << (x * TU + y) : 0u;
+        ub = live ? ub & inside : 0u;
         // kept by every tile of the macro tile: rounding is monotone, so the product of the smallest norms
         // decides -- unless one is not finite (inf * 0 and NaN are never kept): then all products are looked at
         float amin = a[0], bmin = b[0];
@@ -133,6 +170,7 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
         }
         full = full && live && interior;
         const uint64_t F = __ballot(full), P = __ballot(ub != 0u && !full);
+        if (w + 4 < words) load_norms(w + 4);
         uint64_t mine = 0;                                             // lane t: bitmap word of tile t
 #pragma unroll
         for (int t = 0; t < TT; t++) {
@@ -152,81 +190,101 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
     // together (1024^3 10 % 15.4 -> 13.7 us whole, 2048^3 dense 33.8 -> 31.5, 1056 x 1568 x 1312 18.6 -> 17.7).  The total is
     // minus their number then: what the last gate was is known on the device, also behind a replayed graph.  (By a wave that has
     // nothing else to store: behind unit 0's own word it was 0.13 us.)
-    auto store_gate = [&]() {
-        if (!(mode & SMALL_GATE)) return;
-        const bool first = (ui * U) % B == 0 && (uj * U) % B == 0;
-        for (int e = first ? threadIdx.x : TT * words; e < TT * words; e += 256) {
-            const int t = e / words, w = e - t * words, i = ti0 + t / TU, j = tj0 + t % TU;
-            if (i < nbM && j < nbN) g.mask[((int64_t)i * nbN + j) * words + w] = s_word[w * TT + t];
-        }
-        if (unit == 0 && wave == 3 && lane == 0) g.kept->total = -((M + U - 1) / U * ((N + U - 1) / U));
+    // Counts and places are worked out while the first stages' loads are under way; what is left for the end is a store or two
+    // (0.8 us with all of it at the end).
+    struct Left {
+        int tile, count, total;      // lane t < TT: the tile's number (-1: not this unit's) and kept k; lane 0: the unit's
+    };
+    auto count_gate = [&]() -> Left {
+        Left l = {-1, 0, 0};
+        if (!(mode & SMALL_GATE)) return l;
+        const int i = ti0 + lane / TU, j = tj0 + lane % TU;
+        if ((ui * U) % B == 0 && (uj * U) % B == 0 && lane < TT && i < nbM && j < nbN) l.tile = i * nbN + j;
         if (wave == 0) {
-            int cnt = 0;
-            if (first && lane < TT) {
-                for (int w = 0; w < words; w++) cnt += __builtin_popcountll(s_word[w * TT + lane]);
-                const int i = ti0 + lane / TU, j = tj0 + lane % TU;
-                if (i < nbM && j < nbN) g.counts[(int64_t)i * nbN + j] = cnt;
-            }
+            if (l.tile >= 0)
+                for (int w = 0; w < words; w++) l.count += __builtin_popcountll(s_word[w * TT + lane]);
+            l.total = l.count;
 #pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
-            if (lane == 0) g.kept->units[(urow / U) * ((N + U - 1) / U) + ucol / U] = (uint32_t)cnt;
+            for (int off = 1; off < TT; off <<= 1) l.total += __shfl_xor(l.total, off, 64);
+        }
+        return l;
+    };
+    auto store_gate = [&](const Left &l) {
+        if (!(mode & SMALL_GATE)) return;
+        const int units_n = (N + U - 1) / U;
+        if (unit == 0 && wave == 3 && lane == 0) g.kept->total = -((M + U - 1) / U * units_n);
+        if (l.tile >= 0)
+            for (int w = wave; w < words; w += 4) g.mask[(uint32_t)(l.tile * words + w)] = s_word[w * TT + lane];
+        if (wave == 0) {
+            if (l.tile >= 0) g.counts[(uint32_t)l.tile] = l.count;
+            if (lane == 0) g.kept->units[urow / U * units_n + ucol / U] = (uint32_t)l.total;
         }
     };
 
-    if (!multiply) {
-        store_gate();
-        return;
-    }
-    // ---- list: every wave scans the words' counts (at most 64 words), then places its own words' entries
-    const uint64_t Fl = lane < words ? s_fp[2 * lane] : 0ull, Pl = lane < words ? s_fp[2 * lane + 1] : 0ull;
-    int bf = __builtin_popcountll(Fl), bp = __builtin_popcountll(Pl);
-    const int own_f = bf, own_p = bp;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int tf = __shfl_up(bf, off, 64), tp = __shfl_up(bp, off, 64);
-        if (lane >= off) { bf += tf; bp += tp; }
-    }
-    const int n_full = __builtin_amdgcn_readlane(bf, 63), n_part = __builtin_amdgcn_readlane(bp, 63);
-    bf -= own_f;
-    bp -= own_p;
-    const int anchor = list_anchor(mi, mj, MT, nbM, nbK, nbN);
-    const uint64_t below_a = (1ull << (anchor & 63)) - 1ull;
-    const int rot_f = __builtin_amdgcn_readlane(bf + __builtin_popcountll(Fl & below_a), anchor >> 6);
-    const int rot_p = __builtin_amdgcn_readlane(bp + __builtin_popcountll(Pl & below_a), anchor >> 6);
-    for (int w = wave; w < words; w += 4) {
-        const uint64_t F = s_fp[2 * w], P = s_fp[2 * w + 1], below = (1ull << lane) - 1ull;
-        const int base_f = __builtin_amdgcn_readlane(bf, w), base_p = __builtin_amdgcn_readlane(bp, w);
-        int pos = -1;
-        if ((F >> lane) & 1ull) {
-            pos = base_f + __builtin_popcountll(F & below) - rot_f;
-            if (pos < 0) pos += n_full;
-        } else if ((P >> lane) & 1ull) {
-            pos = base_p + __builtin_popcountll(P & below) - rot_p;
-            if (pos < 0) pos += n_part;
-            pos += n_full;
+    Left left;
+    int S = 0, Sfull = 0;
+    if (multiply) {
+        // ---- list: every wave scans the words' counts (at most 64 words), then places its own words' entries
+        const uint64_t below_a = (1ull << (anchor & 63)) - 1ull;
+        int n_full, n_part;
+        auto place = [&](int w, uint64_t F, uint64_t P, int base_f, int base_p, int rot_f, int rot_p) {
+            const uint64_t below = (1ull << lane) - 1ull;
+            int pos = -1;
+            if ((F >> lane) & 1ull) {
+                pos = base_f + __builtin_popcountll(F & below) - rot_f;
+                if (pos < 0) pos += n_full;
+            } else if ((P >> lane) & 1ull) {
+                pos = base_p + __builtin_popcountll(P & below) - rot_p;
+                if (pos < 0) pos += n_part;
+                pos += n_full;
+            }
+            if (pos >= 0) s_list[pos] = (uint32_t)(w * 64 + lane) | (uint32_t)s_bits[w * 64 + lane] << 16;
+        };
+        if (words == 1) {                                                  // (nothing to scan)
+            auto uniform = [](uint64_t v) {
+                return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+            };
+            const uint64_t F = uniform(s_fp[0]), P = uniform(s_fp[1]);
+            n_full = __builtin_popcountll(F);
+            n_part = __builtin_popcountll(P);
+            if (wave == 0) place(0, F, P, 0, 0, __builtin_popcountll(F & below_a), __builtin_popcountll(P & below_a));
+        } else {
+            const uint64_t Fl = lane < words ? s_fp[2 * lane] : 0ull, Pl = lane < words ? s_fp[2 * lane + 1] : 0ull;
+            int bf = __builtin_popcountll(Fl), bp = __builtin_popcountll(Pl);
+            const int own_f = bf, own_p = bp;
+            for (int off = 1; off < words; off <<= 1) {
+                const int tf = __shfl_up(bf, off, 64), tp = __shfl_up(bp, off, 64);
+                if (lane >= off) { bf += tf; bp += tp; }
+            }
+            n_full = __builtin_amdgcn_readlane(bf, words - 1);
+            n_part = __builtin_amdgcn_readlane(bp, words - 1);
+            bf -= own_f;
+            bp -= own_p;
+            const int rot_f = __builtin_amdgcn_readlane(bf + __builtin_popcountll(Fl & below_a), anchor >> 6);
+            const int rot_p = __builtin_amdgcn_readlane(bp + __builtin_popcountll(Pl & below_a), anchor >> 6);
+            for (int w = wave; w < words; w += 4)
+                place(w, s_fp[2 * w], s_fp[2 * w + 1], __builtin_amdgcn_readlane(bf, w), __builtin_amdgcn_readlane(bp, w), rot_f, rot_p);
         }
-        if (pos >= 0) s_list[pos] = (uint32_t)(w * 64 + lane) | (uint32_t)s_bits[w * 64 + lane] << 16;
+        __syncthreads();
+        S = (n_full + n_part) * H::NSPE;
+        Sfull = n_full * H::NSPE;
     }
-    __syncthreads();
-    const int S = (n_full + n_part) * H::NSPE, Sfull = n_full * H::NSPE;
 
-    if (S == 0) {
+    if (multiply && S == 0) {
         constexpr int LPR = U / 4;                                     // lanes per row
         const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-        const int64_t c0 = ucol + (lane % LPR) * 4;
+        const int c0 = ucol + (lane % LPR) * 4;
         if (c0 < N)
             for (int r = wave * (64 / LPR) + lane / LPR; r < U && urow + r < M; r += 4 * (64 / LPR))
-                __builtin_nontemporal_store(zero, reinterpret_cast<f32x4 *>(C + (urow + r) * N + c0));
-        store_gate();
-        return;
+                __builtin_nontemporal_store(zero, reinterpret_cast<f32x4 *>(C + (uint32_t)((urow + r) * N + c0)));
     }
-
+    if (S == 0) left = count_gate();
     f32x4 acc[NB][NB];
 #pragma unroll
     for (int r = 0; r < NB; r++)
 #pragma unroll
         for (int c = 0; c < NB; c++) acc[r][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    {
+    if (S > 0) {
         // ---- staging: a wave copies CHW consecutive 1 KiB chunks of the A part and of the B part of a stage
         // (the ring protocol and its hand-counted waits are k_gemm's)
         const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
@@ -235,8 +293,8 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
         ti = ti < nbM ? ti : nbM - 1;
         tj = tj < nbN ? tj : nbN - 1;
         const int within = (vec / H::RS) * B + vec % H::RS;            // 16-byte vector inside the tile's 4 k-groups
-        const unsigned char *rowA = pA + (int64_t)ti * nbK * H::TILE_BYTES + (within + (ui * U) % B) * 16;
-        const unsigned char *rowB = pB + (int64_t)tj * nbK * H::TILE_BYTES + (within + (uj * U) % B) * 16;
+        const unsigned char *rowA = pA + (int64_t)ti * nbK * H::TILE_BYTES + (within + (int)(ui * U) % B) * 16;
+        const unsigned char *rowB = pB + (int64_t)tj * nbK * H::TILE_BYTES + (within + (int)(uj * U) % B) * 16;
         const uint32_t ldsA = lds_base + chunk0 * 1024, ldsB = ldsA + H::OP_BYTES;
         const uint32_t needA = (H::ROW_BITS << (slot * TU)) << 16, needB = (H::COL_BITS << slot) << 16;   // entry bits that read this slot
         const uint32_t voff = lane * 16;
@@ -293,6 +351,7 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
             return next;
         };
         uint32_t e_cur = entry_at(0), e_new = entry_at(NBUF);
+        left = count_gate();
         __builtin_amdgcn_s_waitcnt(waitcnt_imm(H::LPW * (NBUF - 1), 0));
         __syncthreads();
         Frags f0, f1;
@@ -357,26 +416,28 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
     }
 
     // ---- epilogue: as k_gemm's
-    const uint32_t lane_off = (uint32_t)(32 * (lane >> 5)) * (uint32_t)N + 4 * (lane & 31);     // bytes
+    if (S > 0) {
+        const uint32_t lane_off = (uint32_t)(32 * (lane >> 5)) * (uint32_t)N + 4 * (lane & 31);     // bytes
 #pragma unroll
-    for (int r = 0; r < NB; r++) {
-        const int64_t row0 = urow + (TU > 1 ? (wr + 2 * (r * 16 / B)) * B + (r * 16) % B : wr * (U / 2) + r * 16);
-        if (row0 >= M) continue;
+        for (int r = 0; r < NB; r++) {
+            const int row0 = urow + (TU > 1 ? (wr + 2 * (r * 16 / B)) * B + (r * 16) % B : wr * (U / 2) + r * 16);
+            if (row0 >= M) continue;
 #pragma unroll
-        for (int c = 0; c < NB; c += 2) {
-            const int64_t col0 = ucol + (TU > 1 ? (wc + 2 * (c * 16 / B)) * B + (c * 16) % B : wc * (U / 2) + c * 16);
-            if (col0 >= N) continue;
+            for (int c = 0; c < NB; c += 2) {
+                const int col0 = ucol + (TU > 1 ? (wc + 2 * (c * 16 / B)) * B + (c * 16) % B : wc * (U / 2) + c * 16);
+                if (col0 >= N) continue;
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float x = acc[r][c][i], y = acc[r][c + 1][i];
-                const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
-                float *out = C + (row0 + i) * N + col0;
-                asm volatile("global_store_dword %0, %1, %2 nt" :: "v"(lane_off), "v"(sw[0]), "s"(out) : "memory");
-                asm volatile("global_store_dword %0, %1, %2 nt" :: "v"(lane_off), "v"(sw[1]), "s"(out + 4 * N) : "memory");
+                for (int i = 0; i < 4; i++) {
+                    const float x = acc[r][c][i], y = acc[r][c + 1][i];
+                    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+                    float *out = C + (uint32_t)((row0 + i) * N + col0);
+                    asm volatile("global_store_dword %0, %1, %2 nt" :: "v"(lane_off), "v"(sw[0]), "s"(out) : "memory");
+                    asm volatile("global_store_dword %0, %1, %2 nt" :: "v"(lane_off), "v"(sw[1]), "s"(out + 4 * N) : "memory");
+                }
             }
         }
     }
-    store_gate();
+    store_gate(left);
 }
 
 // The arguments come in the order of their use, and all that are read lie in the first 128 bytes: a line of them that nothing
@@ -384,17 +445,15 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
 // 24.74 against M, N and C in a third line).
 template <int B, int U>
 __global__ __launch_bounds__(256, 2) void k_small(const unsigned char *__restrict__ pA, const unsigned char *__restrict__ pB, int nbM, int nbK,
-                                                  int nbN, int nMacN, int n_units, int n_xcd, int mode, float tau, int64_t M, int64_t N,
-                                                  float *__restrict__ C, GateBuffers g) {
-    small_unit_body<B, U, (U == 128 ? 4 : 6)>(pA, pB, g, nbM, nbK, nbN, nMacN, n_units, n_xcd, mode, tau, M, N, C);
+                                                  int nbN, SmallGrid sg, float tau, float *__restrict__ C, GateBuffers g) {
+    small_unit_body<B, U, (U == 128 ? 4 : 6)>(pA, pB, g, nbM, nbK, nbN, sg, tau, C);
 }
 
 // Units of 128 by three workgroups per CU (small_three).
 template <int B>
 __global__ __launch_bounds__(256, 3) void k_small_three(const unsigned char *__restrict__ pA, const unsigned char *__restrict__ pB, int nbM,
-                                                        int nbK, int nbN, int nMacN, int n_units, int n_xcd, int mode, float tau, int64_t M,
-                                                        int64_t N, float *__restrict__ C, GateBuffers g) {
-    small_unit_body<B, 128, 3>(pA, pB, g, nbM, nbK, nbN, nMacN, n_units, n_xcd, mode, tau, M, N, C);
+                                                        int nbK, int nbN, SmallGrid sg, float tau, float *__restrict__ C, GateBuffers g) {
+    small_unit_body<B, 128, 3>(pA, pB, g, nbM, nbK, nbN, sg, tau, C);
 }
 
 // Units of 128 in C, as many as 256 CUs would have for the same share of a CU: what the lines below balance is workgroups per
@@ -445,8 +504,9 @@ static hipError_t launch_small_(const void *pA, const void *pB, const GateBuffer
     const int nMacM = (nbM + H::MT - 1) / H::MT, nMacN = (nbN + H::MT - 1) / H::MT;
     const int n_units = nMacM * nMacN * H::PD * H::PD;
     const unsigned grid = (unsigned)((n_units + n_xcd - 1) / n_xcd * n_xcd);
+    const SmallGrid sg = {nMacN, 0xffffffffu / (uint32_t)nMacN, n_units, (n_units + n_xcd - 1) / n_xcd, __builtin_ctz((unsigned)n_xcd), mode};
     small_kernel<B, U, THREE>()<<<grid, 256, small_lds<B, U, THREE>(nbK), s>>>(
-        (const unsigned char *)pA, (const unsigned char *)pB, nbM, nbK, nbN, nMacN, n_units, n_xcd, mode, tau, M, N, C, g);
+        (const unsigned char *)pA, (const unsigned char *)pB, nbM, nbK, nbN, sg, tau, C, g);
     return hipGetLastError();
 }
 

@@ -276,6 +276,14 @@ def test_small_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N, ti
         apart.close()
 
 
+@pytest.mark.parametrize("words_k", [31, 32, 33, 63, 64, 65, 127, 128, 129, 256, 257])
+@pytest.mark.parametrize("M,N", [(96, 160), (2080, 1952)])
+def test_small_outputs_list_every_place_of_a_word(orc, ctx, M, N, words_k):
+    """Units of 64 and of 128: a word of 64 k that is the list's only one, or the first or last of several, with its places up to
+    the 32nd and the 64th kept, all of them and every other one."""
+    test_small_outputs_in_one_launch_give_the_same_product(orc, ctx, M, 32 * words_k, N, 32)
+
+
 @pytest.mark.parametrize("M,K,N,tile", [(2944, 256, 2912, 32),      # 529 units: no longer two to a CU at once
                                         (3200, 160, 3072, 32), (3200, 256, 3200, 64),               # 600 and 625: two and three to a CU
                                         (3200, 12320, 3136, 32),    # a list too long for three to a CU
