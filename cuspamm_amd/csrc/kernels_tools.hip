@@ -274,7 +274,8 @@ __global__ __launch_bounds__(256) void k_limbs(LimbOperand a, LimbOperand b, int
             const unsigned int hi = __builtin_amdgcn_perm(w[4 * g + 3], w[4 * g + 2], 0x0c0c0400u + 0x0101u * l);
             v[g] = (int)(lo | hi << 16);
         }
-        *reinterpret_cast<i32x4 *>(out + l * LIMB_PLANE) = v;
+        // (written through: the planes are read by every XCD; 1984 x 768 x 2176 46.3 -> 44.9 us, 4096^3 algebraic 219 -> 214)
+        asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" :: "v"(out + l * LIMB_PLANE), "v"(v) : "memory");
     }
 }
 
