@@ -535,27 +535,30 @@ hipError_t small_init() {
 // tau > 0, at most 6 units per CU.  K = 4096 at tile 64, 5 % | 40 % kept: 768 units 66 -> 51 | 94 -> 82 us; 1000 units
 // 69 -> 61 | 115 -> 113; 1296 units 78 -> 69 | 145 -> 135.  K = 2048 at tile 32: 54.6 -> 40.2 | 77 -> 58.7, 62 -> 51.5 |
 // 84.8 -> 80.5, 68.6 -> 57.6 | 93.5 -> 92.4.  K = 8192 at tile 128, 25 % | 50 %: 1088 units 171 -> 144 | 246 -> 221, 1444
-// units 191 -> 174 | 287 -> 266.  Beyond: 1600 units, K = 5120, 10 % of a band 107.8 -> 112, 25 % 160 -> 146; 1936 units, K =
-// 2048, 25 % 99 -> 119; 4096 units 243 -> 265.  What decides is how many macro tiles compute, which the host does not know:
-// the fewer, the more CUs k_gemm leaves idle.  Where its one round is all but full (833 to 1024 units) and much is kept, its
-// thriftier staging wins with long K: 1024 units, 5 % | 40 %, K = 2048 62 -> 45 | 83 -> 79, K = 4096 73 -> 61 | 105 -> 109,
-// K = 8192 (2 % | 25 %) 91 -> 80 | 141 -> 137, K = 16384 151 -> 133 | 224 -> 250.
+// units 191 -> 174 | 287 -> 266.  K beyond 8192 in the one round that k_gemm fills (833 to 1024 units), 10 % | 40 %: 960
+// units, K = 12288 156.9 -> 151 | 271 -> 265.5; 1024 units, K = 16384 159.9 -> 156.3 | 313 -> 309.7 (passes and all: the packed
+// copies stay in the memory-side cache; from HBM the second took 224 -> 250).  Beyond 6 units, 10 % | 40 %, also with the
+// passes: 1600 units, K = 3072 88.6 -> 76.1 | 131 -> 150; 1936 units, K = 5120 114 -> 102 | 203 -> 218; 2304 units, K = 5120
+// 130 -> 113 | 228 -> 231, and 30 % at K = 8192 268 -> 284.  What decides is how many macro tiles compute, which the host does
+// not know: the fewer, the more CUs k_gemm leaves idle.
 //
 // tau <= 0, everything is kept and the rounds are known.  Up to 512 units 88.3 -> 71.2 us (484), 118 -> 101 (512).  With m =
 // 160 to 192 a round is a third empty: 640 units, K = 2048 | 4096 82 -> 69 | 139 -> 123; 704 units 80 -> 70 | 133 -> 123; 768
 // units 82.6 -> 75.7 | 140 -> 132; but 600 units 70 -> 67 | 108 -> 119 and 841 units 81 -> 90 | 135 -> 161.  With m = 257 to
 // 324 a second round is mostly empty: 1088 units 129 -> 104 | 220 -> 184, 1296 units 136 -> 120 | 233 -> 220; 1444 units
 // 132 -> 126 | 228 -> 227 and, K = 8192, 412 -> 436.
-// Gate and multiply called apart (`stages`) form mask and list twice, which costs what the schedule does: the lines are
-// drawn closer (tau to a fraction and both stages, apart -> this: 625 units 114.7 -> 98 us; 768 units 122 -> 105, 127 -> 110;
-// 900 units 157 -> 160; 1000 units at tile 32 137.5 -> 139; 1120 units 162.5 -> 149.6, 126 -> 116; 1444 units 139 -> 147).
+// Gate and multiply called apart (`stages`) form mask and list twice, which still is less than what the schedule costs (tau
+// to a fraction and both stages, 6 % | 40 % kept, apart -> this: 840 units 108.7 -> 91.7 | 143 -> 135 us; fp16 900 units, K =
+// 2048 95.1 -> 77.3 | 118 -> 107; 1000 units at tile 32 121.9 -> 110.4 | 183 -> 174.9; 1024 units, K = 4096 114.9 -> 101.8 |
+// 161.6 -> 161.4; but 1444 units 112.8 -> 102 | 159.6 -> 162.4, hence the line at 1200).
+
 bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau, bool stages, int n_cu) {
     const int64_t units128 = units_of_128(M, N, n_cu), m = per_256_cus(((M + 255) / 256) * ((N + 255) / 256), n_cu);
     if (K / tile > SMALL_MAX_NBK || n_cu > 256) return false;
     static_assert(SMALL_MAX_UNITS >= 6 * 256 && SMALL_MAX_UNITS >= 4 * 127, "units of either size");
     if (units128 <= 512) return true;
-    if (stages) return tau > 0.0f && (units128 <= 832 || (units128 > 1024 && units128 <= 1200));
-    if (tau > 0.0f) return units128 <= SMALL_MAX_UNITS && (units128 <= 832 || units128 > 1024 || K <= 8192);
+    if (stages) return tau > 0.0f && units128 <= 1200;
+    if (tau > 0.0f) return units128 <= SMALL_MAX_UNITS && (units128 <= 832 || units128 > 1024 || K <= 16384);   // longer: not measured
     return (m >= 160 && m <= 192) || (m >= 257 && m <= 324);
 }
 
