@@ -532,15 +532,21 @@ hipError_t small_init() {
 // Whole multiplies on fp16 operands, gate, schedule and GEMM apart -> this kernel, by units of 128 in C; "m" is the number of
 // macro tiles (four units each), of which k_gemm runs 256 at a time.
 //
-// tau > 0, at most 6 units per CU.  K = 4096 at tile 64, 5 % | 40 % kept: 768 units 66 -> 51 | 94 -> 82 us; 1000 units
-// 69 -> 61 | 115 -> 113; 1296 units 78 -> 69 | 145 -> 135.  K = 2048 at tile 32: 54.6 -> 40.2 | 77 -> 58.7, 62 -> 51.5 |
-// 84.8 -> 80.5, 68.6 -> 57.6 | 93.5 -> 92.4.  K = 8192 at tile 128, 25 % | 50 %: 1088 units 171 -> 144 | 246 -> 221, 1444
-// units 191 -> 174 | 287 -> 266.  K beyond 8192 in the one round that k_gemm fills (833 to 1024 units), 10 % | 40 %: 960
-// units, K = 12288 156.9 -> 151 | 271 -> 265.5; 1024 units, K = 16384 159.9 -> 156.3 | 313 -> 309.7 (passes and all: the packed
-// copies stay in the memory-side cache; from HBM the second took 224 -> 250).  Beyond 6 units, 10 % | 40 %, also with the
-// passes: 1600 units, K = 3072 88.6 -> 76.1 | 131 -> 150; 1936 units, K = 5120 114 -> 102 | 203 -> 218; 2304 units, K = 5120
-// 130 -> 113 | 228 -> 231, and 30 % at K = 8192 268 -> 284.  What decides is how many macro tiles compute, which the host does
-// not know: the fewer, the more CUs k_gemm leaves idle.
+// tau > 0, at most 6 units per CU; 1 / (1 + d)^2, 10 % | 40 % kept, passes and all (their copies lie in the memory-side cache).  K =
+// 2048 at tile 32: 768 units 33.1 -> 28.4 | 44.4 -> 41.5 us; 840 units 37.4 -> 30.3 | 47.3 -> 44.2; 1024 units 40.3 -> 32.9 | 50.7 ->
+// 52.8; 1296 units 46.5 -> 41.3 | 58.9 -> 66.1; 1444 units 48.7 -> 43.5 | 64.0 -> 74.4.  K = 4096 at tile 64: 768 units 46.0 -> 41.7 |
+// 67.3 -> 72.4; 840 units 52.3 -> 44.8 | 76.0 -> 79.6; 1024 units 55.0 -> 50.1 | 81.9 -> 91.6; 1296 units 63.1 -> 61.7 | 98.1 ->
+// 117.2; 1444 units 70.1 -> 66.7 | 108.6 -> 129.3.  K = 8192 at tile 128: 840 units 76.0 -> 74.9 | 120.6 -> 146.6; 1024 units 84.3 ->
+// 86.5 | 131.1 -> 173.5; 1296 units 100.9 -> 103.5 | 163.8 -> 221.1.  What decides is how many macro tiles compute, which the host
+// does not know: the fewer, the more CUs k_gemm leaves idle.  Operands that lie there already and come from HBM (converted before,
+// other work since), where three workgroups per CU hide more of the latency: 1024 units, K = 4096 94.8 -> 76.7 | 124.3 -> 112.3,
+// K = 8192 102.7 -> 84.4 | 156.8 -> 157.5; 1296 units, K = 8192 136.4 -> 94.7 | 227.1 -> 188.3.
+// In the one round that k_gemm fills (833 to 1024 units) K ends at 8192, where neither gains any more, few kept with the
+// passes or many from HBM.  Beyond it, 5 % | 40 %: 840 units, K = 16384 112.4 -> 110.5 | 214.3 -> 309.4 and, from HBM, 100.7 -> 78.0 |
+// 237.7 -> 263.9; 1024 units, K = 12288 100.6 -> 102.3 | 186.5 -> 290.3 and 101.3 -> 83.7 | 198.5 -> 225.3, K = 16384 129.7 -> 134.6 |
+// 237.8 -> 353.1 and 114.0 -> 94.3 | 251.9 -> 287.6.
+// Beyond 6 units, 10 % | 40 %, with the passes: 1600 units, K = 3072 88.6 -> 76.1 | 131 -> 150; 1936 units, K = 5120 114 -> 102 |
+// 203 -> 218; 2304 units, K = 5120 130 -> 113 | 228 -> 231, and 30 % at K = 8192 268 -> 284.
 //
 // tau <= 0, everything is kept and the rounds are known.  Up to 512 units 88.3 -> 71.2 us (484), 118 -> 101 (512).  With m =
 // 160 to 192 a round is a third empty: 640 units, K = 2048 | 4096 82 -> 69 | 139 -> 123; 704 units 80 -> 70 | 133 -> 123; 768
@@ -551,14 +557,13 @@ hipError_t small_init() {
 // to a fraction and both stages, 6 % | 40 % kept, apart -> this: 840 units 108.7 -> 91.7 | 143 -> 135 us; fp16 900 units, K =
 // 2048 95.1 -> 77.3 | 118 -> 107; 1000 units at tile 32 121.9 -> 110.4 | 183 -> 174.9; 1024 units, K = 4096 114.9 -> 101.8 |
 // 161.6 -> 161.4; but 1444 units 112.8 -> 102 | 159.6 -> 162.4, hence the line at 1200).
-
 bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau, bool stages, int n_cu) {
     const int64_t units128 = units_of_128(M, N, n_cu), m = per_256_cus(((M + 255) / 256) * ((N + 255) / 256), n_cu);
     if (K / tile > SMALL_MAX_NBK || n_cu > 256) return false;
     static_assert(SMALL_MAX_UNITS >= 6 * 256 && SMALL_MAX_UNITS >= 4 * 127, "units of either size");
     if (units128 <= 512) return true;
     if (stages) return tau > 0.0f && units128 <= 1200;
-    if (tau > 0.0f) return units128 <= SMALL_MAX_UNITS && (units128 <= 832 || units128 > 1024 || K <= 16384);   // longer: not measured
+    if (tau > 0.0f) return units128 <= SMALL_MAX_UNITS && (units128 <= 832 || units128 > 1024 || K <= 8192);
     return (m >= 160 && m <= 192) || (m >= 257 && m <= 324);
 }
 

@@ -495,7 +495,9 @@ static int run_small(spamm_ctx *c, int mode, float tau, float *dC) {
     return SPAMM_OK;
 }
 
-int spamm_gate(spamm_ctx *c, float tau) {
+// The stages, `apart` from each other or as what a multiply does that is not small: its own line has been asked then, and the
+// stages', which lies elsewhere, would have it gate and multiply by two launches of k_small.
+static int gate_stage(spamm_ctx *c, float tau, bool apart) {
     if (!c) return SPAMM_EINVAL;
     if (static_stale(c)) return SPAMM_ESTATE;
     if (!c->tile || !c->M || !c->K || !c->N || !c->nm_a || !c->nm_b) return SPAMM_ESTATE;   // both norm maps, same K and tile
@@ -503,7 +505,7 @@ int spamm_gate(spamm_ctx *c, float tau) {
     int rc = set_device(c);
     if (rc) return rc;
     if (c->timing && !c->ev_a) HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
-    if (is_small(c, tau, true)) rc = run_small(c, SMALL_GATE, tau, nullptr);
+    if (apart && is_small(c, tau, true)) rc = run_small(c, SMALL_GATE, tau, nullptr);
     else rc = build_lists(c, tau);
     if (rc) return rc;
     if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[3], c->stream)); c->ev_gate = true; }
@@ -512,7 +514,7 @@ int spamm_gate(spamm_ctx *c, float tau) {
     return SPAMM_OK;
 }
 
-int spamm_gemm_gated(spamm_ctx *c, float *dC) {
+static int gemm_stage(spamm_ctx *c, float *dC, bool apart) {
     if (!c || !dC) return SPAMM_EINVAL;
     if (static_stale(c)) return SPAMM_ESTATE;
     if (!c->have_a || !c->have_b || !c->have_gate) return SPAMM_ESTATE;
@@ -520,7 +522,7 @@ int spamm_gemm_gated(spamm_ctx *c, float *dC) {
     if (c->b_pruned && !(c->tau > 0.0f)) return SPAMM_ESTATE;               // B's copy lacks its zero tiles
     int rc = set_device(c);
     if (rc) return rc;
-    const bool small = is_small(c, c->tau, true);
+    const bool small = apart && is_small(c, c->tau, true);
     if (!small && !c->have_lists && (rc = build_lists(c, c->tau))) return rc;    // (the work unit was fixed after a small gate)
     if (c->timing && !c->ev_gate) HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
     if (small) {
@@ -532,6 +534,10 @@ int spamm_gemm_gated(spamm_ctx *c, float *dC) {
     if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[4], c->stream)); c->ev_gemm = true; }
     return SPAMM_OK;
 }
+
+int spamm_gate(spamm_ctx *c, float tau) { return gate_stage(c, tau, true); }
+
+int spamm_gemm_gated(spamm_ctx *c, float *dC) { return gemm_stage(c, dC, true); }
 
 static int multiply_any(spamm_ctx *c, const spamm_params *p, const void *dA, const void *dB, bool in16,
                         float *dC) {
@@ -619,8 +625,8 @@ static int multiply_any(spamm_ctx *c, const spamm_params *p, const void *dA, con
         if (c->timing) { HIPCHK(c, hipEventRecord(c->ev[4], c->stream)); c->ev_gemm = true; }
         return SPAMM_OK;
     }
-    if ((rc = spamm_gate(c, p->tau))) return rc;
-    return spamm_gemm_gated(c, dC);
+    if ((rc = gate_stage(c, p->tau, false))) return rc;
+    return gemm_stage(c, dC, false);
 }
 
 // Gives every buffer a multiply of this shape needs its place in the fixed array (base != null) and

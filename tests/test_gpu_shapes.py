@@ -289,6 +289,8 @@ def test_small_outputs_list_every_place_of_a_word(orc, ctx, M, N, words_k):
                                         (3200, 12320, 3136, 32),    # a list too long for three to a CU
                                         (4096, 512, 2560, 64), (4352, 320, 4160, 64),               # dense too: 160 and 289 macro tiles
                                         (4096, 96, 4096, 32), (3968, 384, 4224, 128), (4096, 64, 6144, 64),
+                                        (3712, 8192, 3712, 64), (4096, 8192, 4096, 128),            # 841 and 1024 units at their longest
+                                        (3712, 8256, 3712, 64), (4096, 12288, 3584, 128),           # beyond it: gate and GEMM
                                         (192, 640, 98304, 64)])     # 1536 units, the most
 def test_middling_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N, tile):
     test_small_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N, tile)

@@ -195,6 +195,10 @@ def multiply_on_a_partition(e, cus):
         if tau:
             assert kernels(20, 2048, tau) == ["k_small_three"] and kernels(24, 16384, tau) == ["k_small_three"]
             assert "k_gate" in kernels(32, 16384, tau) and "k_gate" in kernels(60, 2048, tau)
+            for eighths in (27, 32):                # the one round that macro tiles fill: K up to 8192, on either side of it any
+                assert kernels(eighths, 8192, tau) == ["k_small_three"]
+                assert kernels(eighths, 8256, tau) == ["k_gate", "k_gemm"] and kernels(eighths, 65536, tau) == ["k_gate", "k_gemm"]
+            assert kernels(26, 8256, tau) == ["k_small_three"] and kernels(33, 8256, tau) == ["k_small_three"]
         assert "k_gate" in kernels(most + 2, 2048, tau)
         assert ("k_gate" in kernels(most, 2048, tau)) is False
 
