@@ -553,16 +553,21 @@ hipError_t small_init() {
 // units 82.6 -> 75.7 | 140 -> 132; but 600 units 70 -> 67 | 108 -> 119 and 841 units 81 -> 90 | 135 -> 161.  With m = 257 to
 // 324 a second round is mostly empty: 1088 units 129 -> 104 | 220 -> 184, 1296 units 136 -> 120 | 233 -> 220; 1444 units
 // 132 -> 126 | 228 -> 227 and, K = 8192, 412 -> 436.
-// Gate and multiply called apart (`stages`) form mask and list twice, which still is less than what the schedule costs (tau
-// to a fraction and both stages, 6 % | 40 % kept, apart -> this: 840 units 108.7 -> 91.7 | 143 -> 135 us; fp16 900 units, K =
-// 2048 95.1 -> 77.3 | 118 -> 107; 1000 units at tile 32 121.9 -> 110.4 | 183 -> 174.9; 1024 units, K = 4096 114.9 -> 101.8 |
-// 161.6 -> 161.4; but 1444 units 112.8 -> 102 | 159.6 -> 162.4, hence the line at 1200).
+// Gate and multiply called apart (`stages`) form mask and list twice, which costs less than the schedule does up to 1200 units
+// (fp32 passes, tau to a fraction, both stages, 10 % | 40 % kept: 1120 units, K = 2048 at tile 32 98.3 -> 89.8 | 109.4 -> 109.7 us, K =
+// 4096 at tile 64 122.0 -> 110.6 | 150.5 -> 149.3; 1200 units 97.2 -> 92.4 | 105.9 -> 113.8, 118.7 -> 114.2 | 150.8 -> 156.9; but 1444
+// units 125.6 -> 123.8 | 159.8 -> 175.9).  In the round that k_gemm fills (833 to 1024 units) it pays for one word of 64 k and up to
+// K = 4096 (10 % | 40 % | 75 %: 840 units, K = 2048 at tile 32 98.0 -> 87.4 | 105.6 -> 100.5 | 107.5 -> 112.2; 1024 units 101.7 -> 91.6 |
+// 110.2 -> 108.4 | 112.7 -> 121.9, K = 4096 at tile 64 118.8 -> 106.5 | 138.9 -> 138.5 | 161.0 -> 167.5, at tile 128 116.1 -> 103.7 |
+// 137.7 -> 133.8 | 160.7 -> 163.4); beyond that few kept still gain, a quarter is even, and more lose more (10 % | 25 % | 50 %: 1000
+// units at tile 32, K = 4128 120.5 -> 112.7 | 131.1 -> 132.5 | 147.1 -> 165.2; 10 % | 50 % at tile 128, 1024 units, K = 8192 157.1 -> 146.8 |
+// 209.0 -> 224.3; passes and stages alone, 1024 units at tile 64, K = 8192, 10 % | 40 % 86.0 -> 91.9 | 129.7 -> 169.6).
 bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau, bool stages, int n_cu) {
     const int64_t units128 = units_of_128(M, N, n_cu), m = per_256_cus(((M + 255) / 256) * ((N + 255) / 256), n_cu);
     if (K / tile > SMALL_MAX_NBK || n_cu > 256) return false;
     static_assert(SMALL_MAX_UNITS >= 6 * 256 && SMALL_MAX_UNITS >= 4 * 127, "units of either size");
     if (units128 <= 512) return true;
-    if (stages) return tau > 0.0f && units128 <= 1200;
+    if (stages) return tau > 0.0f && units128 <= 1200 && (units128 <= 832 || units128 > 1024 || (K <= 4096 && K / tile <= 64));
     if (tau > 0.0f) return units128 <= SMALL_MAX_UNITS && (units128 <= 832 || units128 > 1024 || K <= 8192);
     return (m >= 160 && m <= 192) || (m >= 257 && m <= 324);
 }

@@ -296,6 +296,38 @@ def test_middling_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N,
     test_small_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N, tile)
 
 
+@pytest.mark.parametrize("M,K,N,tile", [(3712, 2048, 3712, 32), (3712, 2080, 3712, 32), (4096, 4096, 3584, 64), (4096, 4160, 3584, 64),
+                                        (4096, 4096, 4096, 128), (4096, 4224, 4096, 128)])
+def test_stages_on_either_side_of_their_line(orc, ctx, M, K, N, tile):
+    """Gate, then multiply, by the one-launch kernel's two halves up to one word of 64 k and K = 4096, by the gate and the GEMM
+    beyond: mask, counts and, bit for bit, C as by the latter."""
+    import torch
+    import cuspamm_amd as sp
+    apart = sp.SpammContext(0)
+    apart.set_option(sp.OPT_GEMM_SHAPE, 1)
+    try:
+        tab = orc.decay_table("exp", max(M, K, N), 12.0 / max(M, K, N))
+        dA = torch.empty((M, K), dtype=torch.float32, device="cuda")
+        dB = torch.empty((K, N), dtype=torch.float32, device="cuda")
+        ctx.fill_decay(dA, tab, 1)
+        ctx.fill_decay(dB, tab, 2)
+        for c in (ctx, apart):
+            c.normmap_f32(1, dB, tile)
+            c.normmap_f32(0, dA, tile)
+        for tau in (ctx.tau_for_ratio(0.03)[0], ctx.tau_for_ratio(0.4)[0], float("inf")):
+            out = []
+            for c in (ctx, apart):
+                C = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+                c.gate(tau)
+                before = c.get_mask(), c.get_counts()
+                out.append((c.gemm_gated(C), before, c.get_stats().kept_products))
+            (C, maps, kept), (C2, maps2, kept2) = out
+            assert torch.equal(C, C2) and kept == kept2
+            assert all(np.array_equal(x, y) for x, y in zip(maps, maps2))
+    finally:
+        apart.close()
+
+
 def test_schedule_of_the_longest_lists_on_one_xcd(ctx):
     """One XCD takes every super tile of a band, and the lengths dealt to it so far are part of the key it is chosen by:
     lists of 65535 k tiles bring that sum to 2^28 - 1 before the last super tile is dealt (times 8, plus the XCD's number:

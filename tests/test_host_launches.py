@@ -203,6 +203,34 @@ def multiply_on_a_partition(e, cus):
         assert ("k_gate" in kernels(most, 2048, tau)) is False
 
 
+def stages_on_a_partition(e, cus):
+    e.fake.fake_cus(cus)
+    h = e.context()
+    X = ctypes.create_string_buffer(16)
+
+    def kernels(eighths, K, tile, tau=0.5):
+        resident_operands(e, h, 128 * eighths, K, 128 * (cus // 8), tile)
+        e.launches()
+        assert e.L.spamm_gate(h, ctypes.c_float(tau)) == 0 and e.L.spamm_gemm_gated(h, X) == 0
+        return [name for name, _ in e.launches() if name in ("k_small", "k_small_three", "k_gate", "k_gemm")]
+
+    apart = ["k_gate", "k_gemm"]
+    assert kernels(16, 65536, 64) == ["k_small"] * 2 and kernels(16, 2048, 32, 0.0) == ["k_small"] * 2 and kernels(17, 2048, 32, 0.0) == apart
+    for eighths, K, tile in ((26, 8256, 64), (33, 8256, 64), (37, 2048, 32)):          # up to 832 and from 1025 to 1200 units: any K
+        assert kernels(eighths, K, tile) == ["k_small_three"] * 2
+    assert kernels(38, 2048, 32) == apart
+    for eighths in (27, 32):                                                           # the round that macro tiles fill: 64 k tiles, K = 4096
+        for K, tile in ((2048, 32), (4096, 64), (4096, 128)):
+            assert kernels(eighths, K, tile) == ["k_small_three"] * 2 and kernels(eighths, K + tile, tile) == apart
+        assert kernels(eighths, 8192, 128) == apart and kernels(eighths, 65536, 128) == apart
+
+
+@pytest.mark.parametrize("cus", [256, 128, 64, 32])
+def test_lines_of_the_stages_by_the_small_kernel(run, cus):
+    """Gate and multiply called apart: the one-launch kernel runs twice, so its lines lie elsewhere than a multiply's."""
+    run("stages_on_a_partition", cus)
+
+
 @pytest.mark.parametrize("cus", [256, 128, 64, 32])
 def test_lines_of_the_small_kernel_are_by_work_per_cu(run, cus):
     """A partition of an XCD or a few has its lines where a CU has as much to do as on the whole chip."""
