@@ -330,7 +330,7 @@ __global__ __launch_bounds__(256, 2) void k_error_limbs(const int8_t *__restrict
                                                         ReportSums *__restrict__ host_out, unsigned long long *__restrict__ host_seq,
                                                         unsigned long long seq, bool dense_here) {
     __shared__ __attribute__((aligned(16))) unsigned char s_planes[2][LIMB_STEP][LIMB_PLANE];     // of this step and the next
-    __shared__ uint16_t s_desc[LIMB_MAX_STEPS][LIMB_STEP];        // plane of A or (bit 15) of B, or none
+    __shared__ __attribute__((aligned(16))) uint16_t s_desc[LIMB_MAX_STEPS][LIMB_STEP];           // plane of A or (bit 15) of B, or none
     __shared__ double red[4][3];
     __shared__ int s_count[LIMBS * LIMBS];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

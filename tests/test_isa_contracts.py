@@ -380,6 +380,22 @@ def test_integer_product_keeps_the_same_distance(tmp_path):
     assert not any(mn.startswith("scratch_") for mn, _, _ in _instructions(body))
 
 
+def test_lds_written_16_bytes_at_a_time_is_declared_for_it():
+    """The compiler gives larger arrays 16 bytes by itself, which nothing promises: what is written or read by vectors of 16 bytes
+    says so where it is declared."""
+    seen = 0
+    for src in sorted(os.listdir(CSRC)):
+        if not src.endswith((".hip", ".h")):
+            continue
+        text = open(os.path.join(CSRC, src)).read()
+        wide = set(re.findall(r"reinterpret_cast<(?:const )?(?:u32x4n?|i32x4|f32x4|uint4|half8t) \*>\((s_\w+)", text))
+        for decl in re.findall(r"^\s*__shared__ ([^;]*);", text, flags=re.M):
+            names = set(re.findall(r"(s_\w+)\[", decl)) & wide
+            seen += len(names)
+            assert not names or "aligned(16)" in decl, (src, decl)
+    assert seen >= 3
+
+
 def test_wide_stores_written_out_keep_their_data(tmp_path):
     """A vector instruction may not write the registers of a store of more than 64 bits within two wait states of it, which the
     compiler sees to around stores of its own: the ones written out carry the wait states."""
