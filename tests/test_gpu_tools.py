@@ -325,33 +325,47 @@ def test_fp16_passes_of_three_to_four_strips_per_cu(orc, ctx):
 @pytest.mark.parametrize("tile", [32, 64, 128])
 @pytest.mark.parametrize("half", [False, True])
 def test_conversion_on_either_side_of_what_the_caches_keep(ctx, tile, half):
-    """Input of more than 32 MiB is read past the caches, less through them, by launches of their own: the halves of a matrix that
-    lies just beyond, one by one and as one, in both roles and with norms and values bit for bit; A = B by one read below."""
+    """Input of more than 32 MiB is read past the caches, less through them, by launches of their own, and strips of nothing but
+    zeros are stored past them: a matrix just beyond that line and each of its halves, in both roles, with zero strips, zeros beside
+    the smallest value there is and single values; values against the input's, the halves' norms against the whole's, bit for
+    bit.  A = B by one read on either side of the line."""
     import torch
+
+    def with_zeros(X):
+        X[:tile, 512:1024] = 0.0
+        X[tile:2 * tile, :512] = 0.0
+        X[tile + 5, 131] = 1.0
+        X[-tile:, 1024:1536] = 0.0
+        X[-1, 1535] = 2.0 ** -24
+        X[:, 2048:2112] = 0.0
+        return X.half() if half else X
     rows, cols = 512, (33280 if half else 16640) if tile < 128 else (33024 if half else 16640)
     g = torch.Generator(device="cuda")
     g.manual_seed(tile)
-    X = torch.rand((rows, cols), generator=g, device="cuda") * 2.0 - 1.0
-    X = X.half() if half else X
+    X = with_zeros(torch.rand((rows, cols), generator=g, device="cuda") * 2.0 - 1.0)
     assert X.numel() * X.element_size() > 32 << 20
     convert = ctx.normmap_f16 if half else ctx.normmap_f32
     bits = X.half().cpu().numpy().view(np.uint16)
     for role in (1, 0):
-        for M in ((X, X[: rows // 2]) if role == 0 else (X, X[: rows // 2])):
-            other = torch.zeros((tile, M.shape[0]) if role == 1 else (M.shape[1], tile), dtype=X.dtype, device="cuda")
+        whole = None
+        for first, last in ((0, rows), (0, rows // 2), (rows // 2, rows)):
+            part = X[first:last]
+            other = torch.zeros((tile, last - first) if role == 1 else (cols, tile), dtype=X.dtype, device="cuda")
             convert(1 - role, other, tile)
-            convert(role, M, tile)
-            assert np.array_equal(ctx.get_fp16(role), bits[: M.shape[0]])
+            convert(role, part, tile)
+            assert np.array_equal(ctx.get_fp16(role), bits[first:last])
             nm = ctx.get_normmap(role)
-            if M is X:
-                whole = nm
-            else:
-                assert np.array_equal(nm.view(np.uint32), whole[: nm.shape[0]].view(np.uint32))
-    n = 1024
-    Y = X[:, :n].contiguous().repeat(2, 1)
-    two = ctx.multiply(Y, Y.clone(), tile, 0.0)
-    assert torch.equal(ctx.multiply(Y, Y, tile, 0.0, a_eq_b=True), two)
-    assert np.array_equal(ctx.get_fp16(0), Y.half().cpu().numpy().view(np.uint16)) and np.array_equal(ctx.get_fp16(1), ctx.get_fp16(0))
+            whole = nm if whole is None else whole
+            assert np.array_equal(nm.view(np.uint32), whole[first // tile:last // tile].view(np.uint32))
+            assert nm.min() == 0.0 < nm.max()
+    for n in (2048, 4224 if half else 2944):
+        Y = with_zeros(torch.rand((n, n), generator=g, device="cuda") * 2.0 - 1.0)
+        two = ctx.multiply(Y, Y.clone(), tile, 0.0)
+        maps = ctx.get_normmap(0), ctx.get_normmap(1)
+        assert torch.equal(ctx.multiply(Y, Y, tile, 0.0, a_eq_b=True), two)
+        for role in (0, 1):
+            assert np.array_equal(ctx.get_fp16(role), Y.half().cpu().numpy().view(np.uint16))
+            assert np.array_equal(ctx.get_normmap(role).view(np.uint32), maps[role].view(np.uint32))
 
 
 @pytest.mark.parametrize("rows,N,row0", [(2048, 1024, 64), (512, 512, 0), (4096, 2048, 0), (2112, 960, 0)])

@@ -26,8 +26,8 @@ CSRC = os.path.join(ROOT, "cuspamm_amd", "csrc")
 def _isa(src, tmp_path):
     from cuspamm_amd import build
     out = os.path.join(str(tmp_path), src.replace(".hip", ".s"))
-    cmd = [build.HIPCC] + [f for f in build.CFLAGS if f != "-Wall"] + build.GEMM_FLAGS + ["-S", "--cuda-device-only",
-                                                                                      os.path.join(CSRC, src), "-o", out]
+    cmd = [build.HIPCC] + [f for f in build.CFLAGS if f != "-Wall"] + build.EXTRA_FLAGS.get(src, []) + ["-S", "--cuda-device-only",
+                                                                                                     os.path.join(CSRC, src), "-o", out]
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     assert proc.returncode == 0, proc.stdout[-2000:]
     return open(out).read()
