@@ -347,6 +347,15 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
     } else {
         // one pass for both roles: no row maxima yet, so only tiles of norm zero are left out
         emit_role(false, packed, nm, nullptr, prune);
+        // (With two groups per lane the second role converts again: kept from the first, values and squares were 174 registers a
+        // lane, of which 168 leave room for the third workgroup that a CU's LDS holds.  Tau-aware squares of 16384: 472 -> 417 us for 0.07 %
+        // of a narrow band, 1188 -> 1133 for 10 % of a wide one.)
+        if constexpr (!IN16 && NGW > 1) {
+#pragma unroll
+            for (int i = 0; i < NGW; i++)
+#pragma unroll
+                for (int j = 0; j < 8; j++) asm volatile("" : "+v"(v[i][j]));
+        }
         __syncthreads();
         emit_role(true, packed2, nm2, nmT, prune);
     }

@@ -380,6 +380,14 @@ def test_integer_product_keeps_the_same_distance(tmp_path):
     assert not any(mn.startswith("scratch_") for mn, _, _ in _instructions(body))
 
 
+def test_single_pass_of_two_groups_leaves_room_for_a_third_workgroup(tmp_path):
+    """kernels_normmap.hip: the fp32 pass of A = B with two 8-row groups per lane lives from three workgroups per CU, which 42 KiB of
+    LDS and up to 168 registers allow; nothing is spilled for it."""
+    text = _isa("kernels_normmap.hip", tmp_path)
+    found = re.findall(r"\.name:\s+_ZN5spamm9k_normmapILi64ELi2ELi256ELb0ELi1ELi4E\w*.*?\.vgpr_count:\s+(\d+)\s+\.vgpr_spill_count:\s+(\d+)", text, flags=re.S)
+    assert found and all(int(n) <= 168 and int(spilled) == 0 for n, spilled in found), found
+
+
 def test_lds_written_16_bytes_at_a_time_is_declared_for_it():
     """The compiler gives larger arrays 16 bytes by itself, which nothing promises: what is written or read by vectors of 16 bytes
     says so where it is declared."""
