@@ -548,11 +548,14 @@ hipError_t small_init() {
 // Beyond 6 units, 10 % | 40 %, with the passes: 1600 units, K = 3072 88.6 -> 76.1 | 131 -> 150; 1936 units, K = 5120 114 -> 102 |
 // 203 -> 218; 2304 units, K = 5120 130 -> 113 | 228 -> 231, and 30 % at K = 8192 268 -> 284.
 //
-// tau <= 0, everything is kept and the rounds are known.  Up to 512 units 88.3 -> 71.2 us (484), 118 -> 101 (512).  With m =
-// 160 to 192 a round is a third empty: 640 units, K = 2048 | 4096 82 -> 69 | 139 -> 123; 704 units 80 -> 70 | 133 -> 123; 768
-// units 82.6 -> 75.7 | 140 -> 132; but 600 units 70 -> 67 | 108 -> 119 and 841 units 81 -> 90 | 135 -> 161.  With m = 257 to
-// 324 a second round is mostly empty: 1088 units 129 -> 104 | 220 -> 184, 1296 units 136 -> 120 | 233 -> 220; 1444 units
-// 132 -> 126 | 228 -> 227 and, K = 8192, 412 -> 436.
+// tau <= 0, everything is kept and the rounds are known.  Tile 64, whole multiplies | operands from HBM, K = 2048 and 4096.  With m = 160
+// to 192 a round is a third empty: 640 units 64.5 -> 53.8 | 108.1 -> 79.4 and 111.8 -> 112.1 | 152.3 -> 124.8; 704 units 64.9 -> 59.7 |
+// 108.9 -> 81.7 and 116.7 -> 119.6 | 153.4 -> 130.3; 768 units 62.0 -> 64.5 | 108.4 -> 86.7 and 115.2 -> 124.8 | 153.5 -> 134.7; but 600
+// units 101.9 -> 107.7 | 152.6 -> 130.6 and 841 units 63.4 -> 74.8 | 109.0 -> 99.1 and 117.8 -> 157.3 | 153.4 -> 156.8.  With m = 257 to 324
+// a second round is mostly empty, which pays from HBM only: 1088 units, K = 1024 56.6 -> 47.7 | 113.6 -> 76.4, K = 2048 80.4 -> 91.2 |
+// 154.1 -> 113.2, K = 4096 145.4 -> 175.7 | 231.3 -> 182.7, K = 8192 268.4 -> 397.2 | 383.2 -> 332.7; 1296 units 91.4 -> 108.0 | 154.7 ->
+// 121.7 and 165.5 -> 236.7 | 230.9 -> 205.7; 1444 units 104.3 -> 121.8 | 157.6 -> 133.3 and 184.3 -> 257.9 | 236.9 -> 220.9.  (The lines were
+// drawn when every multiply read its operands from HBM; whether the passes have just run is not asked here.)
 // Gate and multiply called apart (`stages`) form mask and list twice, which costs less than the schedule does up to 1200 units
 // (fp32 passes, tau to a fraction, both stages, 10 % | 40 % kept: 1120 units, K = 2048 at tile 32 98.3 -> 89.8 | 109.4 -> 109.7 us, K =
 // 4096 at tile 64 122.0 -> 110.6 | 150.5 -> 149.3; 1200 units 97.2 -> 92.4 | 105.9 -> 113.8, 118.7 -> 114.2 | 150.8 -> 156.9; but 1444

@@ -16,11 +16,12 @@
 // the number of blocks allows: each converted value serves NBR or NBC MFMAs.  4096^3:
 // 2229 us with 32 x 32 per wave and 4-byte loads, 2109 now (65 TFLOP/s; the pipeline's 128 operations at the clock
 // that the chip holds under them, about 2 GHz); 1984 x 2176 x 768: 196 -> 158.  In whole numbers instead (one call, its
-// host wait included): 4096^3 2107 -> 742 us on uniform values in [-1, 1) (4 bytes each, 16 products, 3.1 Pop/s),
-// 469 where 3 bytes do, 232 on exp(-d / 100); 1984 x 2176 x 768 165 -> 76, 63, 45; 64 rows of 4096^3 173 -> 87, 68, 45.
+// host wait included): 4096^3 2046 -> 661 us on uniform values in [-1, 1) (4 bytes each, 16 products, 3.3 Pop/s),
+// 444 where 3 bytes do, 203 on exp(-d / 100); 1984 x 768 x 2176 151 -> 72, 60, 54; 64 rows of 4096^3 186 -> 86, 68, 45.
 // An operand with a value of 127 or more has been read by k_limbs for nothing, which writes no planes then, and blocks of 64 x 64
 // of C are formed in fp64 by k_error_limbs itself, two workgroups per CU where k_error_dense has three, so its loads go out
-// three steps ahead instead of one (1280^3 122.7 -> 115): 1024^3 56 -> 59.5 us, 1280^3 106 -> 111, 4096^3 2121 -> 2106.
+// three steps ahead instead of one (1088^3 107 -> 98 us, 1536 x 1024 x 1024 107 -> 97, 1280^3 123 -> 117 to 122).  Against a report that
+// is never split: 1024^3 55 -> 58, 1280^3 102 -> 117 to 122, 4096^3, by k_error_dense behind it, 2046 -> 2092.
 // The scalar bound of 64 x 64 x 64 tiles 52 -> 7 us, the per-tile one 51 -> 4; results go straight to host memory (a
 // clearing launch before and a copy after each were 25 us a call).
 #include "gemm_device.h"
@@ -285,9 +286,10 @@ __global__ __launch_bounds__(256) void k_limbs(LimbOperand a, LimbOperand b, int
 // step's planes are multiplied from LDS, which two waves share each, while direct global->LDS loads bring the next step's, whatever
 // its kind.  (Where a wave loaded its operands to registers, kind by kind, every plane passed the L1 twice and
 // a kind, of two or three blocks on the average, began with a wait: kernel alone, 4096^3 exp(-d / 100) 241 -> 201 us, uniform 780 ->
-// 670, 4096^3 algebraic 252 -> 187.)  What bounds it: a step of 0.69 us, of which the MFMAs of both
-// workgroups take 0.25 to 0.9 and LDS 0.5 (4 KiB written and 8 read per plane); without the reads the calls are 10 % shorter,
-// without the loads 12 %.  Planes in a ring of 16 with loads up to two steps ahead: 6 % longer (addresses); steps of 6 planes by three
+// 670, 4096^3 algebraic 252 -> 187.)  What bounds it, per step of the two
+// workgroups of a CU, 4096^3: 0.99 us on exp(-d / 100) (24 steps a workgroup, its fixed costs included), where their MFMAs take 0.4
+// and LDS 0.5 (4 KiB written and 8 read per plane), 1.3 us on uniform values (64 steps), where they take 0.9 and 0.7; without the
+// reads the calls were 10 % shorter, without the loads 12 %.  Planes in a ring of 16 with loads up to two steps ahead: 6 % longer (addresses); steps of 6 planes by three
 // workgroups per CU: decaying values 5 to 10 % shorter, uniform ones 50 % longer (4 + 4 limbs take two steps, and
 // 168 registers are too few).
 // Groups of GB x GB workgroups that share operands in an L2 run on one XCD; the groups, row by row, go round
@@ -611,12 +613,13 @@ static int64_t limb_kb(int64_t K) { return (K + LIMB_BLOCK - 1) / LIMB_BLOCK; }
 // 1 / 2.4 of the fp64 product's time.  Both are estimated, in us: of the product 0.033 per MFMA of its fullest SIMD (4096^3 2112,
 // 1280^3 94, 64 rows of 4096^2 151), of the split 6 for its launches, two passes over 2 bytes a value at 3 TB/s, and the
 // scratch's allocation where the context does not keep it.  fp64 -> whole numbers, whole calls, on uniform values | exp(-d / 100) |
-// values too large for limbs, by the estimates' ratio: 1.5, 65536 x 1024 x 64 155 -> 178 | 69 | 185; 2.2, 512 x 384 x 512
-// 31.2 -> 32.2 | 31.8 | 35.8; 2.5, 4096 x 256 x 512 38 -> 35.8 | 31.0 | 43.2 and 1024 x 512 x 1024 39.2 -> 38.5 | 35.8 | 41.2;
-// 2.8, 512^3 35.9 -> 34.9 | 33.9 | 40.1 and 65536 x 512 x 128 158 -> 120 | 62 | 172; 3.9, 1024^3 57 -> 49.4 | 44.4 | 59.5; 7.6,
-// 65536 x 512 x 256 289 -> 186 | 87 | 311; 10, 1280^3 106 -> 64 | 55 | 111.  (Whole numbers as they were with operands loaded to
-// registers; the product takes less since: 512^3 31 | 30, 65536 x 512 x 128 107 | 58, 1024^3 43.4 | 39.6, 1280^3 58 | 48.)  With K below 256 a block's fixed costs outweigh its
-// few products: 4096 x 64 x 4096 61 -> 82 | 73 | 68, K = 128 94 -> 94 | 74 | 102, K = 256 158 -> 118 | 79 | 164.
+// values too large for limbs, by the estimates' ratio: 1.5, 512 x 256 x 512 27.4 -> 27.1 | 26.4 | 31.0 and 65536 x 1024 x 64 151 ->
+// 147 | 61 | 226; 2.2, 512 x 384 x 512 32.2 -> 29.4 | 28.1 | 35.7; 2.4, 4096 x 256 x 512 35.6 -> 31.7 | 27.8 | 46.9 and 32768 x 512 x 128
+// 88 -> 62 | 41 | 118; 2.6, 1024 x 512 x 1024 37.1 -> 34.0 | 32.1 | 40.1; 2.7, 65536 x 512 x 128 150 -> 102 | 58 | 193; 2.8, 512^3 36.9 ->
+// 31.4 | 30.1 | 40.1; 4.3, 1024^3 55.2 -> 41.4 | 38.5 | 58.4; 5.3, 65536 x 512 x 256 281 -> 157 | 80 | 326; 8.6, 1280^3 102 -> 54 | 45 |
+// 122.  What the line weighs is the tenth to half that large values lose against what the others gain, 5 to 20 % just below it.  With
+// K below 256 a block's fixed costs outweigh its few products: 4096 x 64 x 4096 59 -> 75 | 66 | 70, K = 128 92 -> 83 | 67 | 103, K = 192 122 ->
+// 92 | 68 | 134.  (Both lines were drawn when the product loaded its operands to registers and took longer.)
 size_t limb_bytes(int64_t rows, int64_t K, int64_t N, int n_cu) {
     if (K > LIMB_MAX_K || K < 256) return 0;
     const size_t blocks = (size_t)(rows / LIMB_BLOCK + N / LIMB_BLOCK) * (size_t)limb_kb(K);
