@@ -9,8 +9,10 @@
 // counts, kept total -- is written on the way out; the macro tiles' work lists, which
 // nothing reads after this kernel, are built by k_gate if somebody asks for them.
 //
-// A unit's life, fp16 2048^3 at tile 32, 5 % kept, us: gate 2.0 (most of it the norms' round trip), list 0.3, first stages 0.8, 9 to
-// 14 stages 3.4 to 6, C 1.5.  With 64-bit places, divisions by the grid's sizes, a scan for the one word of 64 k that most lists
+// Two forms: K / tile up to 64 (k_small_word, the list in a register) and beyond (k_small, the list in LDS).
+//
+// A unit's life in k_small, measured on fp16 2048^3 at tile 32, 5 % kept, us: gate 2.0 (most of it the norms' round trip), list 0.3, first
+// stages 0.8, 9 to 14 stages 3.4 to 6, C 1.5.  With 64-bit places, divisions by the grid's sizes, a scan for the one word of 64 k that most lists
 // are, and counts formed behind C's stores it was 1 us longer (whole calls: 256^3 10.5 -> 9.8 us, 1024^3 11.6 -> 10.6, 1056 x 1568 x
 // 1312 16.3 -> 15.5, this one 19.5 -> 18.4, 4096^2 of a band 57.9 -> 56.2).
 //
@@ -240,15 +242,7 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
             }
             if (pos >= 0) s_list[pos] = (uint32_t)(w * 64 + lane) | (uint32_t)s_bits[w * 64 + lane] << 16;
         };
-        if (words == 1) {                                                  // (nothing to scan)
-            auto uniform = [](uint64_t v) {
-                return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-            };
-            const uint64_t F = uniform(s_fp[0]), P = uniform(s_fp[1]);
-            n_full = __builtin_popcountll(F);
-            n_part = __builtin_popcountll(P);
-            if (wave == 0) place(0, F, P, 0, 0, __builtin_popcountll(F & below_a), __builtin_popcountll(P & below_a));
-        } else {
+        {
             const uint64_t Fl = lane < words ? s_fp[2 * lane] : 0ull, Pl = lane < words ? s_fp[2 * lane + 1] : 0ull;
             int bf = __builtin_popcountll(Fl), bp = __builtin_popcountll(Pl);
             const int own_f = bf, own_p = bp;
@@ -456,6 +450,361 @@ __global__ __launch_bounds__(256, 3) void k_small_three(const unsigned char *__r
     small_unit_body<B, 128, 3>(pA, pB, g, nbM, nbK, nbN, sg, tau, C);
 }
 
+// ---------------------------------------------------------------- one word of k tiles (K / tile <= 64), the usual small problem
+// The same unit, with the list in a register.  A wave of such a kernel is alone on its SIMD and issues one instruction in some
+// five clocks, so the time to its first stage is a number of instructions: 7900 clocks in the kernel above (fp16 2048^3, 5 % kept: gate 1500
+// behind the norms' arrival, list 900, the ring's first loads 1600, which wait for each entry in turn), 4600 here.  Every wave forms the whole
+// list for itself -- lane = k, a lane's place by counting bits, one permutation of the lanes -- without LDS, without a sync, and takes a
+// stage's entry out of it by v_readlane.  Norms, operands and C are addressed by a buffer's scalar offset, one scalar instruction a load, and
+// all arguments are asked for at once.  A slot that no tile pair of an entry reads, and stages beyond the last, are loads from a
+// buffer of no bytes: they keep the number of loads in flight fixed and fetch nothing (their offset is one of the operand's all the same).
+// Kernels alone, k_small -> this: 256^3 5.35 -> 3.45 us (its gate alone 3.2 -> 1.9), 1056 x 1568 x 1312 9.0 -> 6.4, 1024^3 at tile 64 6.1 ->
+// 4.5, fp16 2048^3 at tile 32 5 % kept 11.6 -> 9.4, 75 % 26.5 -> 23, 4096^3 at tile 64 10 % 33.7 -> 31.
+// What bounds it now: launch and arguments 700 clocks, norms 1200, gate and list 1000, the ring's first loads at 64 bytes a clock 1100, a stage
+// of 128 x 128 x 32 some 600 (of which its loads alone take 440), C at 64 bytes a clock.
+typedef int i32x4s __attribute__((ext_vector_type(4)));
+
+// Raw buffer of `bytes` from p on (gfx950: 32-bit data, no swizzle, no stride)
+__device__ __forceinline__ i32x4s raw_buffer(const void *p, int bytes) {
+    const uint64_t a = (uint64_t)(uintptr_t)p;
+    return i32x4s{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), bytes, 0x00020000};
+}
+
+// As dma_load, from a buffer: lane l's 16 bytes from soff + voff(l) + IMM land at lds_addr + IMM + 16 * l.
+template <int N>
+__device__ __forceinline__ void dma_buffer(const i32x4s &rsrc, uint32_t voff, uint32_t soff, uint32_t lds_addr) {
+    if constexpr (N == 2)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\tbuffer_load_dwordx4 %1, %2, %3 offen offset:1024 lds"
+                     :
+                     : "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)
+                     : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                     :
+                     : "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)
+                     : "memory", "m0");
+}
+
+// What a unit needs of GateBuffers, within the second line of arguments
+struct WordGate {
+    const float *nA, *nBt;
+    KeptProducts *kept;
+    int32_t *counts;
+    uint64_t *mask;
+};
+
+template <int B, int U, int RING>
+__device__ __forceinline__ void small_word_body(const unsigned char *pA, const unsigned char *pB, int nbM, int nbK, int nbN, SmallGrid sg,
+                                                float tau, float *C, WordGate g) {
+    using H = SmallCfg<B, U, RING>;
+    constexpr int NBUF = H::NBUF, MT = H::MT, TU = H::TU, TT = H::TT, NB = H::NB, BLK = MT / TU;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    // all arguments at once: a line of them asked for later is another 0.3 us
+    asm volatile("" : "+s"(pA), "+s"(pB), "+s"(nbM), "+s"(nbK), "+s"(nbN), "+s"(tau), "+s"(C), "+s"(g.nA), "+s"(g.nBt), "+s"(g.kept),
+                 "+s"(g.counts), "+s"(g.mask));
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wr = wave >> 1, wc = wave & 1, mode = sg.mode;
+    const uint32_t unit = (blockIdx.x & ((1u << sg.xcd_shift) - 1u)) * (uint32_t)sg.chunk + (blockIdx.x >> sg.xcd_shift);
+    if (unit >= (uint32_t)sg.n_units) return;
+    const uint32_t macro = unit / (H::PD * H::PD), part = unit % (H::PD * H::PD), ui = part / H::PD, uj = part % H::PD;
+    const int mi = (int)__umulhi(macro + 1u, sg.mac_rec), mj = (int)macro - mi * sg.nMacN;
+    const int M = nbM * B, N = nbN * B;
+    const int urow = mi * 256 + (int)ui * U, ucol = mj * 256 + (int)uj * U;
+    if (urow >= M || ucol >= N) return;
+    const int ti0 = urow / B, tj0 = ucol / B;                          // first tile of the unit
+
+    // ---- gate: lane = k, norms of the macro tile's rows and columns, the unit's own first (rows clamped; a lane beyond the last k
+    // reads what follows, or nothing behind the map's end)
+    const bool multiply = (mode & SMALL_MULTIPLY) != 0;
+    const int rows_in = nbM - ti0, cols_in = nbN - tj0;                // of the unit's tile rows and columns, those below exist
+    uint32_t a[MT], b[MT];
+    {
+        const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)g.nA, 0, nbM * nbK * 4, 0x00020000);
+        const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)g.nBt, 0, nbN * nbK * 4, 0x00020000);
+        const int stride = nbK * 4;
+        auto load = [&](int blk) {
+            const int i0 = mi * MT + ((ti0 + blk * TU) & (MT - 1)), j0 = mj * MT + ((tj0 + blk * TU) & (MT - 1));
+#pragma unroll
+            for (int x = 0; x < TU; x++) {
+                const int i = i0 + x < nbM ? i0 + x : nbM - 1, j = j0 + x < nbN ? j0 + x : nbN - 1;
+                a[blk * TU + x] = __builtin_amdgcn_raw_buffer_load_b32(ra, lane * 4, i * stride, 0);
+                b[blk * TU + x] = __builtin_amdgcn_raw_buffer_load_b32(rb, lane * 4, j * stride, 0);
+            }
+        };
+        load(0);
+        if (multiply) {
+#pragma unroll
+            for (int blk = 1; blk < BLK; blk++) load(blk);
+        }
+    }
+    const int anchor = multiply ? list_anchor(mi, mj, MT, nbM, nbK, nbN) : 0;
+    const uint64_t live = nbK >= 64 ? ~0ull : (1ull << nbK) - 1ull;
+    const bool mine = (live >> lane) & 1ull;
+    float au[TU], bu[TU];
+#pragma unroll
+    for (int x = 0; x < TU; x++) {                                     // (what does not exist is kept at no threshold: NaN)
+        au[x] = mine && x < rows_in ? __uint_as_float(a[x]) : __builtin_nanf("");
+        bu[x] = x < cols_in ? __uint_as_float(b[x]) : __builtin_nanf("");
+    }
+    uint32_t ub = 0;                                                   // the unit's tiles that keep this lane's k
+#pragma unroll
+    for (int t = TT - 1; t >= 0; t--) ub = ub + ub + (au[t / TU] * bu[t % TU] >= tau ? 1u : 0u);
+
+    // What the gate leaves behind: wave x has row x of the unit's tiles (a tile shared by several units is written by the first)
+    auto store_gate = [&]() {
+        if (!(mode & SMALL_GATE)) return;
+        const int units_n = (N + U - 1) / U;
+        if (wave < TU) {
+            uint64_t word = 0;
+#pragma unroll
+            for (int y = 0; y < TU; y++) {
+                const uint64_t m = __ballot((ub >> (wave * TU + y)) & 1u);
+                word = lane == y ? m : word;
+            }
+            if ((ui * U) % B == 0 && (uj * U) % B == 0 && lane < TU && wave < rows_in && lane < cols_in) {
+                const uint32_t tile = (uint32_t)((ti0 + wave) * nbN + tj0 + lane);
+                g.mask[tile] = word;
+                g.counts[tile] = __builtin_popcountll(word);
+            }
+        }
+        // the unit's kept products, a word of its own; their total is minus the number of units (see k_small)
+        if (wave == 3) {
+            int total = 0;
+#pragma unroll
+            for (int t = 0; t < TT; t++) total += __builtin_popcountll(__ballot((ub >> t) & 1u));
+            if (lane == 0) {
+                g.kept->units[urow / U * units_n + ucol / U] = (uint32_t)(((ui * U) % B == 0 && (uj * U) % B == 0) ? total : 0);
+                if (unit == 0) g.kept->total = -((M + U - 1) / U * units_n);
+            }
+        }
+    };
+    if (!multiply) {
+        store_gate();
+        return;
+    }
+
+    // ---- list: kept by every tile of the macro tile (rounding is monotone, so the product of the smallest norms decides, unless one is
+    // not finite, or below zero), then the others, each group rotated to the anchor
+    uint32_t amin = a[0], bmin = b[0], big = a[0] > b[0] ? a[0] : b[0];
+#pragma unroll
+    for (int x = 1; x < MT; x++) {
+        amin = a[x] < amin ? a[x] : amin;
+        bmin = b[x] < bmin ? b[x] : bmin;
+        const uint32_t m = a[x] > b[x] ? a[x] : b[x];
+        big = m > big ? m : big;
+    }
+    bool full = __uint_as_float(amin) * __uint_as_float(bmin) >= tau;
+    if (__ballot(big >= 0x7f800000u) != 0ull) {
+        full = true;
+#pragma unroll 1
+        for (int x = 0; x < MT; x++) {
+#pragma unroll
+            for (int y = 0; y < MT; y++) {
+                float ax = __uint_as_float(a[0]);
+#pragma unroll
+                for (int z = 1; z < MT; z++) ax = x == z ? __uint_as_float(a[z]) : ax;
+                full = full && ax * __uint_as_float(b[y]) >= tau;
+            }
+        }
+    }
+    const bool interior = (mi + 1) * MT <= nbM && (mj + 1) * MT <= nbN;
+    const uint64_t F = interior ? __ballot(full) & live : 0ull, P = __ballot(ub != 0u) & ~F;
+    const int n_full = __builtin_popcountll(F), n = n_full + __builtin_popcountll(P), S = n * H::NSPE, Sfull = n_full * H::NSPE;
+    f32x4 acc[NB][NB];
+#pragma unroll
+    for (int r = 0; r < NB; r++)
+#pragma unroll
+        for (int c = 0; c < NB; c++) acc[r][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc((void *)C, 0, M * N * 4, 0x00020000);
+    constexpr int NT = 2;                                              // cache policy of the stores of C: non-temporal
+    if (S == 0) {
+        constexpr int LPR = U / 4;                                     // lanes per row
+        const i32x4s zero = {0, 0, 0, 0};
+        const int c0 = ucol + (lane % LPR) * 4;
+        if (c0 < N)
+            for (int r = wave * (64 / LPR) + lane / LPR; r < U && urow + r < M; r += 4 * (64 / LPR))
+                __builtin_amdgcn_raw_buffer_store_b128(zero, rc, ((urow + r) * N + c0) * 4, 0, NT);
+    } else {
+        // every lane goes to its place: full entries, partial ones, and what is not kept behind them
+        auto below = [](uint64_t m) { return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)); };
+        const uint64_t below_a = (1ull << anchor) - 1ull;
+        int pf = below(F) - __builtin_popcountll(F & below_a), pp = below(P) - __builtin_popcountll(P & below_a);
+        pf = pf < 0 ? pf + n_full : pf;
+        pp = (pp < 0 ? pp + n : pp + n_full);
+        int place = n + below(~(F | P));
+        place = (F >> lane) & 1ull ? pf : ((P >> lane) & 1ull ? pp : place);
+        const uint32_t list = (uint32_t)__builtin_amdgcn_ds_permute(place * 4, (int)(ub | (uint32_t)lane << 16));      // lane i: entry i
+
+        // ---- staging, as k_small's: a wave copies CHW consecutive 1 KiB chunks of the A part and of the B part of a stage
+        const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
+        const int chunk0 = wave * H::CHW, slot = chunk0 / H::CPS, vec = (chunk0 % H::CPS) * 64;
+        int ti = ti0 + slot, tj = tj0 + slot;
+        ti = ti < nbM ? ti : nbM - 1;
+        tj = tj < nbN ? tj : nbN - 1;
+        const int within = (vec / H::RS) * B + vec % H::RS;            // 16-byte vector inside the tile's 4 k-groups
+        const int row_bytes = nbK * H::TILE_BYTES;
+        i32x4s rA = raw_buffer(pA + (int64_t)ti * row_bytes, row_bytes), rB = raw_buffer(pB + (int64_t)tj * row_bytes, row_bytes);
+        const uint32_t voffA = (uint32_t)(lane + within + (int)(ui * U) % B) * 16, voffB = (uint32_t)(lane + within + (int)(uj * U) % B) * 16;
+        const uint32_t ldsA = lds_base + chunk0 * 1024, ldsB = ldsA + H::OP_BYTES;
+        const uint32_t needA = H::ROW_BITS << (slot * TU), needB = H::COL_BITS << slot;   // entry bits that read this slot
+
+        // stage t's entry (of the last one's k, and with no tile, beyond it) and what its loads start from
+        auto entry_at = [&](int t) -> uint32_t { return (uint32_t)__builtin_amdgcn_readlane((int)list, (t < S ? t : S - 1) / H::NSPE); };
+        auto offset = [&](int t, uint32_t ent) -> uint32_t {
+            const uint32_t k = (ent >> 16) * H::TILE_BYTES;
+            if constexpr (H::NSPE == 1) return k;
+            else return k + (uint32_t)(t % H::NSPE) * (B * 64);
+        };
+        auto issue_a = [&](uint32_t koff, uint32_t boff) { dma_buffer<H::CHW>(rA, voffA, koff, ldsA + boff); };
+        auto issue_b = [&](uint32_t koff, uint32_t boff) { dma_buffer<H::CHW>(rB, voffB, koff, ldsB + boff); };
+        auto sync_next = [&]() {
+            __builtin_amdgcn_s_waitcnt(waitcnt_imm(H::LPW * (NBUF - 2), 0));
+            __syncthreads();
+        };
+        auto frag_off = [&](int wsel, int blk) -> int {
+            const int s = TU > 1 ? wsel + 2 * (blk * 16 / H::RS) : 0;
+            const int ro = TU > 1 ? (blk * 16) % H::RS : wsel * (U / 2) + blk * 16;
+            return s * H::RS * 64 + ((lane >> 4) * H::RS + ro + (lane & 15)) * 16;
+        };
+        struct Frags {
+            half8 a[NB], b[NB];
+        };
+        auto load_frag = [&](Frags &f, uint32_t boff, auto idx) {
+            constexpr int i = decltype(idx)::value;
+            const unsigned char *bufA = smem + boff;
+            if constexpr (i == 0) f.a[0] = *reinterpret_cast<const half8 *>(bufA + frag_off(wr, 0));
+            else if constexpr (i <= NB) f.b[i - 1] = *reinterpret_cast<const half8 *>(bufA + H::OP_BYTES + frag_off(wc, i - 1));
+            else f.a[i - NB] = *reinterpret_cast<const half8 *>(bufA + frag_off(wr, i - NB));
+        };
+        // ---- prologue
+        const int all = row_bytes;
+#pragma unroll
+        for (int t = 0; t < NBUF; t++) {
+            const uint32_t e = entry_at(t), koff = offset(t, e), bits = t < S ? e : 0u;
+            rA.z = (bits & needA) ? all : 0;
+            rB.z = (bits & needB) ? all : 0;
+            issue_a(koff, t * H::STAGE_BYTES);
+            issue_b(koff, t * H::STAGE_BYTES);
+        }
+        int t = 0;
+        uint32_t buf = 0;
+        auto next_buf = [&]() {
+            uint32_t next = buf + H::STAGE_BYTES == NBUF * H::STAGE_BYTES ? 0u : buf + H::STAGE_BYTES;
+            asm volatile("" : "+s"(next));
+            return next;
+        };
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm(H::LPW * (NBUF - 1), 0));
+        __syncthreads();
+        Frags f0, f1;
+        static_for<2 * NB>([&](auto i) { load_frag(f0, 0, i); });
+#define SPAMM_FENCE() __builtin_amdgcn_sched_barrier(0)
+        // (every slot of a full stage is fetched, and of the partial ones that follow the last of them what the list's bits ask for or not)
+        auto full_stage = [&](const Frags &cur, Frags &nxt) {
+            const uint32_t next = next_buf();
+            sync_next();
+            SPAMM_FENCE();
+            uint32_t en = 0, koff = 0;
+            static_for<NB * NB>([&](auto idx) {
+                constexpr int i = decltype(idx)::value, r = i / NB, c = i % NB, A_AT = NB == 4 ? 8 : 2, B_AT = NB == 4 ? 12 : 3;
+                acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cur.a[r], cur.b[c], acc[r][c], 0, 0, 0);
+                if constexpr (i < 2 * NB) load_frag(nxt, next, idx);
+                if constexpr (i == A_AT - 2) {
+                    en = entry_at(t + NBUF);
+                    rA.z = rB.z = t + NBUF < S ? all : 0;
+                }
+                if constexpr (i == A_AT - 1) koff = offset(t + NBUF, en);
+                if constexpr (i == A_AT) issue_a(koff, buf);
+                if constexpr (i == B_AT) issue_b(koff, buf);
+                SPAMM_FENCE();
+            });
+            t++;
+            buf = next;
+        };
+        while (__builtin_expect(t + 1 < Sfull, 1)) {
+            full_stage(f0, f1);
+            full_stage(f1, f0);
+        }
+        auto partial_stage = [&](const Frags &cur, Frags &nxt) {
+            const uint32_t next = next_buf();
+            const uint32_t ec = (entry_at(t) & 0xffffu) >> (TU > 1 ? wr * TU + wc : 0);
+            const uint32_t en = entry_at(t + NBUF), koff = offset(t + NBUF, en), bits = t + NBUF < S ? en : 0u;
+            rA.z = (bits & needA) ? all : 0;
+            rB.z = (bits & needB) ? all : 0;
+            sync_next();
+            SPAMM_FENCE();
+            static_for<H::NP * H::NP>([&](auto pair) {
+                constexpr int p = decltype(pair)::value, px = p / H::NP, py = p % H::NP, bit = 2 * px * TU + 2 * py;
+                if ((ec >> bit) & 1u) {
+#pragma unroll
+                    for (int r = 0; r < H::RB; r++)
+#pragma unroll
+                        for (int c = 0; c < H::RB; c++)
+                            acc[px * H::RB + r][py * H::RB + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                cur.a[px * H::RB + r], cur.b[py * H::RB + c], acc[px * H::RB + r][py * H::RB + c], 0, 0, 0);
+                }
+                if constexpr (p == 0) {
+                    SPAMM_FENCE();
+                    static_for<2 * NB>([&](auto i) { load_frag(nxt, next, i); });
+                    issue_a(koff, buf);
+                    issue_b(koff, buf);
+                    SPAMM_FENCE();
+                }
+            });
+            SPAMM_FENCE();
+            t++;
+            buf = next;
+        };
+        while (t < S) {
+            partial_stage(f0, f1);
+            if (t >= S) break;
+            partial_stage(f1, f0);
+        }
+#undef SPAMM_FENCE
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));                 // the ring still holds loads of nothing
+
+        // ---- C, as k_gemm's epilogue: a store is 32 lanes of each of two rows
+        const int lane_off = 32 * (lane >> 5) * N + 4 * (lane & 31);     // bytes
+        const int col00 = ucol + (TU > 1 ? wc * B : wc * (U / 2));
+#pragma unroll
+        for (int r = 0; r < NB; r++) {
+            const int row0 = urow + (TU > 1 ? (wr + 2 * (r * 16 / B)) * B + (r * 16) % B : wr * (U / 2) + r * 16);
+            if (row0 >= M) continue;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int soff = ((row0 + i) * N + col00) * 4;
+#pragma unroll
+                for (int c = 0; c < NB; c += 2) {
+                    constexpr auto delta = [](int c) { return TU > 1 ? 2 * (c * 16 / B) * B + (c * 16) % B : c * 16; };
+                    if (col00 + delta(c) >= N) continue;
+                    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[r][c][i]), __float_as_uint(acc[r][c + 1][i]), false, false);
+                    __builtin_amdgcn_raw_buffer_store_b32(sw[0], rc, lane_off + delta(c) * 4, soff, NT);
+                    __builtin_amdgcn_raw_buffer_store_b32(sw[1], rc, lane_off + delta(c) * 4, soff + 16 * N, NT);
+                }
+            }
+        }
+    }
+    store_gate();
+}
+
+// Stages in the ring.  Units of 64, ring of 4 | 5 | 6: short lists lose by a stage more (256^3 3.40 | 3.44 | 3.52 us, 1056 x 1568 x 1312
+// 6.35 | 6.38 | 6.56), long ones by one less (1024 x 8192 x 1024 at tile 128, 30 % kept 15.2 | 13.2 | 13.0, 1024 x 2048 x 1024 dense 11.7 | 10.55 |
+// 10.47).  Units of 128: 4, 6 and 8 are even alone, and behind the passes 6 and 8 lose 3 % (fp16 2048^3, 5 %: 18.6 | 19.2 | 19.6).
+template <int U>
+static constexpr int WORD_RING = U == 128 ? 4 : 5;
+
+template <int B, int U>
+__global__ __launch_bounds__(256, 2) void k_small_word(const unsigned char *pA, const unsigned char *pB, int nbM, int nbK, int nbN,
+                                                       SmallGrid sg, float tau, float *C, WordGate g) {
+    small_word_body<B, U, WORD_RING<U>>(pA, pB, nbM, nbK, nbN, sg, tau, C, g);
+}
+
+template <int B>
+__global__ __launch_bounds__(256, 3) void k_small_word_three(const unsigned char *pA, const unsigned char *pB, int nbM, int nbK, int nbN,
+                                                             SmallGrid sg, float tau, float *C, WordGate g) {
+    small_word_body<B, 128, 3>(pA, pB, nbM, nbK, nbN, sg, tau, C, g);
+}
+
 // Units of 128 in C, as many as 256 CUs would have for the same share of a CU: what the lines below balance is workgroups per
 // CU and k_gemm's rounds of a macro tile per CU, so on a partition of fewer CUs they lie at as many units less.
 static int64_t per_256_cus(int64_t units, int n_cu) { return (units * 256 + n_cu - 1) / n_cu; }
@@ -484,16 +833,19 @@ static bool small_three(int64_t units128, int64_t nbK, int tile) {
     return units128 > 600 && 3 * (small_lds_bytes_(16384, 3, tt, nbK) + 2048) <= 160 * 1024;
 }
 
-template <int B, int U, bool THREE>
+// (WORD: one word of k tiles)
+template <int B, int U, bool THREE, bool WORD>
 static constexpr auto small_kernel() {
-    if constexpr (THREE) return &k_small_three<B>;
+    if constexpr (THREE && WORD) return &k_small_word_three<B>;
+    else if constexpr (THREE) return &k_small_three<B>;
+    else if constexpr (WORD) return &k_small_word<B, U>;
     else return &k_small<B, U>;
 }
 
-template <int B, int U, bool THREE>
+template <int B, int U, bool THREE, bool WORD>
 static size_t small_lds(int64_t nbK) {
-    using H = SmallCfg<B, U, (THREE ? 3 : (U == 128 ? 4 : 6))>;
-    return small_lds_bytes_(H::STAGE_BYTES, H::NBUF, H::TT, nbK);
+    using H = SmallCfg<B, U, (THREE ? 3 : (WORD ? WORD_RING<U> : (U == 128 ? 4 : 6)))>;
+    return WORD ? (size_t)H::STAGE_BYTES * H::NBUF : small_lds_bytes_(H::STAGE_BYTES, H::NBUF, H::TT, nbK);
 }
 
 template <int B, int U, bool THREE>
@@ -505,15 +857,22 @@ static hipError_t launch_small_(const void *pA, const void *pB, const GateBuffer
     const int n_units = nMacM * nMacN * H::PD * H::PD;
     const unsigned grid = (unsigned)((n_units + n_xcd - 1) / n_xcd * n_xcd);
     const SmallGrid sg = {nMacN, 0xffffffffu / (uint32_t)nMacN, n_units, (n_units + n_xcd - 1) / n_xcd, __builtin_ctz((unsigned)n_xcd), mode};
-    small_kernel<B, U, THREE>()<<<grid, 256, small_lds<B, U, THREE>(nbK), s>>>(
-        (const unsigned char *)pA, (const unsigned char *)pB, nbM, nbK, nbN, sg, tau, C, g);
+    const unsigned char *a = (const unsigned char *)pA, *b = (const unsigned char *)pB;
+    if (nbK <= 64)
+        small_kernel<B, U, THREE, true>()<<<grid, 256, small_lds<B, U, THREE, true>(nbK), s>>>(a, b, nbM, nbK, nbN, sg, tau, C,
+                                                                                          WordGate{g.nA, g.nBt, g.kept, g.counts, g.mask});
+    else
+        small_kernel<B, U, THREE, false>()<<<grid, 256, small_lds<B, U, THREE, false>(nbK), s>>>(a, b, nbM, nbK, nbN, sg, tau, C, g);
     return hipGetLastError();
 }
 
 template <int B, int U, bool THREE>
 static hipError_t small_attr() {
-    return hipFuncSetAttribute(reinterpret_cast<const void *>(small_kernel<B, U, THREE>()), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)small_lds<B, U, THREE>(SMALL_MAX_NBK));
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(small_kernel<B, U, THREE, true>()),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)small_lds<B, U, THREE, true>(64));
+    if (e != hipSuccess) return e;
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(small_kernel<B, U, THREE, false>()), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)small_lds<B, U, THREE, false>(SMALL_MAX_NBK));
 }
 
 template <int B>

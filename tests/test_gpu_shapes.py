@@ -296,6 +296,31 @@ def test_middling_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N,
     test_small_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N, tile)
 
 
+@pytest.mark.parametrize("M,K,N,tile", [(192, 64, 320, 64), (1088, 4032, 832, 64), (1152, 4096, 2112, 64), (2048, 4160, 1088, 64),
+                                        (256, 128, 384, 128), (640, 8064, 1152, 128), (1920, 8192, 2176, 128), (1920, 8320, 2176, 128),
+                                        (3200, 64, 3264, 64), (3264, 2048, 3136, 64), (3200, 128, 3200, 128)])
+def test_one_word_of_k_tiles_at_its_ends(orc, ctx, M, K, N, tile):
+    """The kernel whose list is a register, at one k tile, at 63 and 64 and the other one at 65, by every size of unit and two and
+    three units to a CU; stages of its own here (a gate that forms no list), too."""
+    import torch
+    test_small_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N, tile)
+    tab = orc.decay_table("exp", max(M, K, N), 12.0 / max(M, K, N))
+    dA = torch.empty((M, K), dtype=torch.float32, device="cuda")
+    dB = torch.empty((K, N), dtype=torch.float32, device="cuda")
+    ctx.fill_decay(dA, tab, 1)
+    ctx.fill_decay(dB, tab, 2)
+    ctx.normmap_f32(1, dB, tile)
+    ctx.normmap_f32(0, dA, tile)
+    tau = ctx.tau_for_ratio(0.2)[0]
+    want = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    ctx.multiply(dA, dB, tile, tau, C=want)
+    mask, counts, kept = ctx.get_mask(), ctx.get_counts(), ctx.get_stats().kept_products
+    ctx.gate(float("inf"))
+    ctx.gate(tau)
+    assert np.array_equal(ctx.get_mask(), mask) and np.array_equal(ctx.get_counts(), counts) and ctx.get_stats().kept_products == kept
+    assert torch.equal(ctx.gemm_gated(torch.full_like(want, float("nan"))), want)
+
+
 @pytest.mark.parametrize("M,K,N,tile", [(3712, 2048, 3712, 32), (3712, 2080, 3712, 32), (4096, 4096, 3584, 64), (4096, 4160, 3584, 64),
                                         (4096, 4096, 4096, 128), (4096, 4224, 4096, 128)])
 def test_stages_on_either_side_of_their_line(orc, ctx, M, K, N, tile):

@@ -414,3 +414,21 @@ def test_wide_stores_written_out_keep_their_data(tmp_path):
         for i in wide:
             mn, ops, _ = ins[i + 1]
             assert mn == "s_nop" and int(ops[0], 0) >= 1, ins[i:i + 2]
+
+
+def test_one_word_kernels_keep_the_same_contracts(tmp_path):
+    """k_small_word and k_small_word_three: their buffer->LDS loads keep their distance from VALU-written SGPRs and are the only
+    vector-memory instructions between the first and the last of them, nothing is spilled, and the arguments lie in two lines."""
+    text = _isa("kernels_small.hip", tmp_path)
+    found, checked = _hazards(_instructions(text), "buffer_load_dwordx4", 5)
+    assert not found and checked > 60, found
+    kernels = re.findall(r"^(_ZN5spamm(?:12k_small_word|18k_small_word_three)I\w+):[^\n]*\n(.*?)^\.Lfunc_end", text, flags=re.S | re.M)
+    assert len(kernels) == 9
+    for name, body in kernels:
+        ins = _instructions(body)
+        dma = [i for i, (mn, _, in_asm) in enumerate(ins) if in_asm and mn == "buffer_load_dwordx4"]
+        assert len(dma) >= 12, name
+        other = [mn for i, (mn, _, _) in enumerate(ins) if dma[0] <= i <= dma[-1] and i not in dma and mn.startswith(("global_", "flat_", "buffer_", "scratch_"))]
+        assert not other and not any(mn.startswith("scratch_") for mn, _, _ in ins), (name, other)
+        loads = re.findall(r"s_load_dword(?:x(\d+))?\s+\S+, s\[\d+:\d+\], (0x[0-9a-f]+)", body)
+        assert loads and max(int(at, 16) + 4 * int(n or 1) for n, at in loads) <= 128, (name, loads)
