@@ -58,13 +58,6 @@ __device__ __forceinline__ float butterfly64(float v) {
 //   store   after one barrier: the tiles are copied out with contiguous 1 KiB wave stores (a
 //           packed tile is one contiguous block in memory), and one wave per tile applies the
 //           canonical reduction.
-// KEEP: the input's lines stay in the caches (keep_input).
-template <bool KEEP, typename T>
-__device__ __forceinline__ T load_strip(const T *from) {
-    if constexpr (KEEP) return *from;
-    else return __builtin_nontemporal_load(from);
-}
-
 template <int B, int SW, int PH>
 struct NormCfg {
     static constexpr int TPP = SW / B / PH;          // tiles resident in LDS together
@@ -77,7 +70,7 @@ struct NormCfg {
 
 // `strip`: which strip of the operand; s_pack / s_chunk / s_skip / s_seen: NormCfg's TPP * TS bytes, TPP * CH floats, TPP and NWV
 // ints of LDS
-template <int B, int ROLE, int SW, bool IN16, int PH, int NWV, bool KEEP>
+template <int B, int ROLE, int SW, bool IN16, int PH, int NWV>
 __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64_t ld, int64_t cols, int64_t nbr, int64_t nbc,
                                               int64_t nstrip, uint4 *__restrict__ packed, float *__restrict__ nm,
                                               float *__restrict__ nmT, uint4 *__restrict__ packed2, float *__restrict__ nm2,
@@ -131,7 +124,7 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
         for (int i = 0; i < NGW; i++)
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                h16[i][j] = load_strip<KEEP>(
+                h16[i][j] = __builtin_nontemporal_load(
                     reinterpret_cast<const u32x4n *>(src + (int64_t)(8 * (g0 + GSTEP * i) + j) * ld));
             }
         if (!valid) {
@@ -149,7 +142,7 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
                 if (!valid)
                     v[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                 else
-                    v[i][j] = load_strip<KEEP>(
+                    v[i][j] = __builtin_nontemporal_load(
                         reinterpret_cast<const f32x4 *>(static_cast<const float *>(Xv) + eoff + (int64_t)r * ld));
             }
     }
@@ -361,7 +354,7 @@ __device__ __forceinline__ void normmap_strip(const void *__restrict__ Xv, int64
     }
 }
 
-template <int B, int ROLE, int SW, bool IN16, int PH = 1, int NWV = 4, bool KEEP = false>
+template <int B, int ROLE, int SW, bool IN16, int PH = 1, int NWV = 4>
 __global__ __launch_bounds__(64 * NWV, 1) void k_normmap(
     const void *__restrict__ Xv, int64_t ld, int64_t cols, int64_t nbr, int64_t nbc, int64_t nstrip, uint4 *__restrict__ packed,
     float *__restrict__ nm, float *__restrict__ nmT, uint4 *__restrict__ packed2, float *__restrict__ nm2,
@@ -370,14 +363,14 @@ __global__ __launch_bounds__(64 * NWV, 1) void k_normmap(
     __shared__ __attribute__((aligned(16))) unsigned char s_pack[L::TPP * L::TS];
     __shared__ float s_chunk[L::TPP * L::CH];
     __shared__ int s_skip[L::TPP], s_seen[NWV];
-    normmap_strip<B, ROLE, SW, IN16, PH, NWV, KEEP>(Xv, ld, cols, nbr, nbc, nstrip, packed, nm, nmT, packed2, nm2, rowmax, tau_skip,
+    normmap_strip<B, ROLE, SW, IN16, PH, NWV>(Xv, ld, cols, nbr, nbc, nstrip, packed, nm, nmT, packed2, nm2, rowmax, tau_skip,
                                               keep_copy, blockIdx.x, s_pack, s_chunk, s_skip, s_seen);
 }
 
 // Both operands in one launch: the first n_b workgroups are B's strips, the others A's.  One after the other,
 // small passes are a few microseconds of memory latency each; together they share it (and neither sees the
 // other's norms: a tau-aware call then leaves out tiles of norm zero only, in both copies).
-template <int B, int SW, bool IN16, int PH, int NWV, bool KEEP = false>
+template <int B, int SW, bool IN16, int PH, int NWV>
 __global__ __launch_bounds__(64 * NWV) void k_normmap_pair(const void *__restrict__ A, const void *__restrict__ Bm, int64_t nbM,
                                                            int64_t nbK, int64_t nbN, unsigned n_b, int64_t strips_a, int64_t strips_b,
                                                            uint4 *__restrict__ packedA, uint4 *__restrict__ packedB,
@@ -388,11 +381,225 @@ __global__ __launch_bounds__(64 * NWV) void k_normmap_pair(const void *__restric
     __shared__ float s_chunk[L::TPP * L::CH];
     __shared__ int s_skip[L::TPP], s_seen[NWV];
     if (blockIdx.x < n_b)
-        normmap_strip<B, 1, SW, IN16, PH, NWV, KEEP>(Bm, nbN * B, nbN * B, nbK, nbN, strips_b, packedB, nmB, nmBt, nullptr, nullptr,
+        normmap_strip<B, 1, SW, IN16, PH, NWV>(Bm, nbN * B, nbN * B, nbK, nbN, strips_b, packedB, nmB, nmBt, nullptr, nullptr,
                                                nullptr, tau_skip, keep_copy, blockIdx.x, s_pack, s_chunk, s_skip, s_seen);
     else
-        normmap_strip<B, 0, SW, IN16, PH, NWV, KEEP>(A, nbK * B, nbK * B, nbM, nbK, strips_a, packedA, nmA, nullptr, nullptr, nullptr,
+        normmap_strip<B, 0, SW, IN16, PH, NWV>(A, nbK * B, nbK * B, nbM, nbK, strips_a, packedA, nmA, nullptr, nullptr, nullptr,
                                                nullptr, tau_skip, keep_copy, blockIdx.x - n_b, s_pack, s_chunk, s_skip, s_seen);
+}
+
+// ---- small inputs (at most KEEP_INPUT_MAX bytes a launch).  There is little to stream: a workgroup's waves are almost alone on their
+// SIMDs, issue an instruction in some five clocks, and the pass takes as long as its chain of instructions.  So everything is
+// addressed by 32-bit offsets into buffers that begin at the strip -- rows by the scalar offset, a lane beyond the last column or a tile
+// beyond the last one by an offset that the buffer does not hold, without a branch --, the strip's place comes from a reciprocal
+// instead of a 64-bit division, and a wave reduces all its tiles' norms together, by lane exchanges that are not LDS operations.
+// Both operands in one launch, alone, inputs from HBM, the streaming kernel -> this: 256^3 3.83 -> 3.01 us (of which 1.55 are an empty
+// launch), 1024^3 at tile 64 4.48 -> 4.14, 1056 x 1568 x 1312 8.2 -> 7.4, fp16 1024 x 2048 x 1024 5.93 -> 4.82, 2048^3 at tile 32 10.3 -> 8.1,
+// 512^3 at tile 128 3.50 -> 3.39 (one wave adds a lane's 32 chunks in their order).
+//
+// Sum over the 64 lanes, in every lane: the same additions as butterfly64.  (Behind the steps of 1 and 2 all lanes of a quad hold one sum, so
+// that a mirrored quad is the neighbour; likewise for 8.)
+__device__ __forceinline__ float butterfly64_dpp(float v) {
+    auto dpp = [](float x, auto ctrl) {
+        const int i = __builtin_bit_cast(int, x);
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, decltype(ctrl)::value, 0xF, 0xF, false));
+    };
+    v = v + dpp(v, std::integral_constant<int, 0xB1>{});       // lanes 1, 0, 3, 2 of a quad
+    v = v + dpp(v, std::integral_constant<int, 0x4E>{});       // lanes 2, 3, 0, 1
+    v = v + dpp(v, std::integral_constant<int, 0x141>{});      // half a row mirrored: the other quad
+    v = v + dpp(v, std::integral_constant<int, 0x140>{});      // a row mirrored: the other half
+    const auto r16 = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+    v = __builtin_bit_cast(float, (uint32_t)r16[0]) + __builtin_bit_cast(float, (uint32_t)r16[1]);
+    const auto r32 = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+    return __builtin_bit_cast(float, (uint32_t)r32[0]) + __builtin_bit_cast(float, (uint32_t)r32[1]);
+}
+
+// A strip's place: row and column of strips, `rec` = strip_reciprocal(nstrip).  Exact while strips * nstrip < 2^32: an input of KEEP_INPUT_MAX bytes
+// is at most 2^14 strips of 2 KiB or more.
+inline uint32_t strip_reciprocal(uint32_t nstrip) { return 0xffffffffu / nstrip; }
+
+template <int B, int ROLE, int SW, bool IN16, int NWV>
+__device__ __forceinline__ void normmap_strip_small(const void *X, uint32_t cols, uint32_t nbr, uint32_t nbc, uint32_t nstrip, uint32_t rec,
+                                                    void *packed, float *nm, float *nmT, void *packed2, float *nm2, const float *rowmax,
+                                                    float tau_skip, bool keep_copy, uint32_t strip, unsigned char *s_pack, float *s_chunk,
+                                                    int *s_skip, int *s_seen) {
+    using L = NormCfg<B, SW, 1>;
+    constexpr int TPP = L::TPP, QN = L::QN, QS = L::QS, TS = L::TS, PITCH = L::PITCH, CH = L::CH;
+    constexpr int E = IN16 ? 2 : 4, EPL = 16 / E;      // bytes per element, elements per lane
+    constexpr int LPR = SW / EPL, GPW = 64 / LPR;      // lanes per strip row, 8-row groups of a wave
+    static_assert(B == 8 * NWV * GPW, "a lane has one 8-row group");
+    constexpr int VPT = B * B / 8, STEPS = VPT / 64;   // 16-byte vectors per tile; chunks per lane of its norm
+    constexpr int NT = TPP > NWV ? TPP / NWV : 1;      // tiles per wave of the norms
+    constexpr uint32_t NOWHERE = 0x80000000u;          // an offset no buffer here holds
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t I = __umulhi(strip + 1u, rec), sc = strip - I * nstrip, col0 = sc * SW, J0 = sc * TPP;
+    const uint32_t ld = cols * E;                      // bytes per row
+    const int cl = EPL * (lane % LPR);                 // first column of this lane inside the strip
+    const int t = cl / B, cin = cl % B;                // tile of the strip, column inside the tile
+    const int g = wave * GPW + lane / LPR;             // 8-row group of this lane
+    const __amdgpu_buffer_rsrc_t in = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char *>(static_cast<const unsigned char *>(X)) + (size_t)I * B * ld + col0 * E, 0,
+                                                                        (int)((B - 1) * ld + (cols - col0) * E), 0x00020000);
+    u32x4n x[8];
+    {
+        const uint32_t voff = col0 + cl < cols ? (uint32_t)(lane / LPR) * 8u * ld + (uint32_t)cl * E : NOWHERE;
+        uint32_t soff = (uint32_t)(wave * GPW * 8) * ld;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            x[j] = __builtin_bit_cast(u32x4n, __builtin_amdgcn_raw_buffer_load_b128(in, (int)voff, (int)soff, 0));
+            soff += ld;
+        }
+    }
+    auto vpos = [](int f, bool swz) -> int { return swz ? (f ^ ((f >> 3) & 7)) : f; };     // (as in normmap_strip)
+    float seen = 0.0f;
+    auto stage_a = [&]() {
+        const int q = cin / 8, h = (cin % 8) / 4;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int r = 8 * g + j;
+            if constexpr (IN16) {
+                const half8n hv = __builtin_bit_cast(half8n, x[j]);
+                float s8 = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; e++) { const float f = (float)hv[e]; s8 = s8 + f * f; }
+                *reinterpret_cast<u32x4n *>(s_pack + t * TS + q * QS + r * 16) = x[j];
+                s_chunk[t * CH + r * PITCH + q] = s8;
+                seen += s8;
+            } else {
+                const f32x4 v = __builtin_bit_cast(f32x4, x[j]);
+                const _Float16 h0 = (_Float16)v.x, h1 = (_Float16)v.y, h2 = (_Float16)v.z, h3 = (_Float16)v.w;
+                const float f0 = (float)h0, f1 = (float)h1, f2 = (float)h2, f3 = (float)h3;
+                float s = 0.0f;
+                s = s + f0 * f0; s = s + f1 * f1; s = s + f2 * f2; s = s + f3 * f3;
+                float s8 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0xA0, 0xF, 0xF, false));
+                s8 = s8 + f0 * f0; s8 = s8 + f1 * f1; s8 = s8 + f2 * f2; s8 = s8 + f3 * f3;
+                const half2v p0 = {h0, h1}, p1 = {h2, h3};
+                uint2 o;
+                o.x = __builtin_bit_cast(uint32_t, p0);
+                o.y = __builtin_bit_cast(uint32_t, p1);
+                *reinterpret_cast<uint2 *>(s_pack + t * TS + q * QS + r * 16 + h * 8) = o;
+                if (h) s_chunk[t * CH + r * PITCH + q] = s8;
+                seen += s8;
+            }
+        }
+    };
+    auto stage_b = [&]() {
+#pragma unroll
+        for (int c = 0; c < EPL; c++) {
+            u32x4n o;
+            float s = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                if constexpr (IN16) {
+                    const _Float16 h0 = __builtin_bit_cast(half8n, x[j])[c], h1 = __builtin_bit_cast(half8n, x[j + 1])[c];
+                    const float f0 = (float)h0, f1 = (float)h1;
+                    s = s + f0 * f0;
+                    s = s + f1 * f1;
+                    const half2v p = {h0, h1};
+                    o[j / 2] = __builtin_bit_cast(uint32_t, p);
+                } else {
+                    o[j / 2] = cvt_pack2(__builtin_bit_cast(f32x4, x[j])[c], __builtin_bit_cast(f32x4, x[j + 1])[c], s);
+                }
+            }
+            *reinterpret_cast<u32x4n *>(s_pack + t * TS + g * QS + vpos(cin + c, IN16) * 16) = o;
+            s_chunk[t * CH + (cin + c) * PITCH + g] = s;
+            seen += s;
+        }
+    };
+    // one operand role
+    auto emit = [&](bool as_b, void *pk, float *nmo, float *nmTo) {
+        const bool prune = tau_skip > 0.0f;
+        seen = 0.0f;
+        if (as_b) stage_b(); else stage_a();
+        const bool used = __ballot(seen != 0.0f) != 0ull;
+        if (lane == 0) s_seen[wave] = used;
+        __syncthreads();
+        // norms in the canonical order: lane n of a wave ends up with its n-th tile's
+        const int t0 = wave * NT;
+        auto norms = [&]() {
+            if (t0 >= TPP) return;
+            float nv = 0.0f;
+#pragma unroll
+            for (int n = 0; n < NT; n++) {
+                float partial = 0.0f;
+#pragma unroll
+                for (int it = 0; it < STEPS; it++) {
+                    const int c = it * 64 + lane;
+                    partial = partial + s_chunk[(t0 + n) * CH + (c / QN) * PITCH + (c % QN)];
+                }
+                partial = butterfly64_dpp(partial);
+                nv = lane == n ? partial : nv;
+            }
+            nv = sqrtf(nv);
+            const uint32_t Jt = J0 + t0 + lane;
+            if (lane < NT && Jt < nbc) {
+                nmo[I * nbc + Jt] = nv;
+                if (as_b) nmTo[Jt * nbr + I] = nv;
+                if (prune) s_skip[t0 + lane] = rowmax != nullptr ? nv * rowmax[Jt] < tau_skip : nv == 0.0f;
+            }
+        };
+        // (what is stored where, and for a tau-aware pass what is left out: as in normmap_strip)
+        if (prune) {
+            norms();
+            __syncthreads();
+        }
+        int any = 0;
+#pragma unroll
+        for (int w = 0; w < NWV; w++) any |= s_seen[w];
+        const uint32_t step = as_b ? nbr * (uint32_t)(B * B * 2) : (uint32_t)(B * B * 2);      // bytes from a tile to the next of the strip
+        const uint32_t first = as_b ? (J0 * nbr + I) * (uint32_t)(B * B * 2) : (I * nbc + J0) * (uint32_t)(B * B * 2);
+        const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(static_cast<unsigned char *>(pk) + first, 0, 0x7fffffff, 0x00020000);
+        auto copy = [&](auto cached) {
+#pragma unroll
+            for (int i = 0; i < TPP * VPT / (64 * NWV); i++) {
+                const int vi = threadIdx.x + 64 * NWV * i, tt = vi / VPT, iv = vi % VPT;
+                const u32x4n d = *reinterpret_cast<const u32x4n *>(s_pack + tt * TS + (iv / B) * QS + vpos(iv % B, IN16 && as_b) * 16);
+                uint32_t at = (uint32_t)tt * step + (uint32_t)iv * 16u;
+                at = J0 + tt < nbc && !(prune && s_skip[tt]) ? at : NOWHERE;
+                __builtin_amdgcn_raw_buffer_store_b128(d, out, (int)at, 0, decltype(cached)::value ? 16 : 2);      // sc1, or non-temporal
+            }
+        };
+        if (keep_copy && __builtin_amdgcn_readfirstlane(any)) copy(std::true_type{});
+        else copy(std::false_type{});
+        if (!prune) norms();
+    };
+    if constexpr (ROLE != 1) emit(false, packed, nm, nullptr);
+    if constexpr (ROLE == 1) emit(true, packed, nm, nmT);
+    if constexpr (ROLE == 2) {
+        __syncthreads();
+        emit(true, packed2, nm2, nmT);
+    }
+}
+
+template <int B, int ROLE, int SW, bool IN16, int NWV>
+__global__ __launch_bounds__(64 * NWV) void k_normmap_small(const void *X, uint32_t cols, uint32_t nbr, uint32_t nbc, uint32_t nstrip,
+                                                            uint32_t rec, void *packed, float *nm, float *nmT, void *packed2, float *nm2,
+                                                            const float *rowmax, float tau_skip, bool keep_copy) {
+    using L = NormCfg<B, SW, 1>;
+    __shared__ __attribute__((aligned(16))) unsigned char s_pack[L::TPP * L::TS];
+    __shared__ float s_chunk[L::TPP * L::CH];
+    __shared__ int s_skip[L::TPP], s_seen[NWV];
+    asm volatile("" : "+s"(X), "+s"(packed), "+s"(nm), "+s"(nmT), "+s"(tau_skip));        // (all arguments at once)
+    normmap_strip_small<B, ROLE, SW, IN16, NWV>(X, cols, nbr, nbc, nstrip, rec, packed, nm, nmT, packed2, nm2, rowmax, tau_skip, keep_copy,
+                                                blockIdx.x, s_pack, s_chunk, s_skip, s_seen);
+}
+
+template <int B, int SW, bool IN16, int NWV>
+__global__ __launch_bounds__(64 * NWV) void k_normmap_pair_small(const void *A, const void *Bm, uint32_t nbM, uint32_t nbK, uint32_t nbN,
+                                                                 uint32_t n_b, uint32_t strips_a, uint32_t rec_a, uint32_t strips_b,
+                                                                 uint32_t rec_b, void *packedA, void *packedB, float *nmA, float *nmB,
+                                                                 float *nmBt, float tau_skip, bool keep_copy) {
+    using L = NormCfg<B, SW, 1>;
+    __shared__ __attribute__((aligned(16))) unsigned char s_pack[L::TPP * L::TS];
+    __shared__ float s_chunk[L::TPP * L::CH];
+    __shared__ int s_skip[L::TPP], s_seen[NWV];
+    asm volatile("" : "+s"(A), "+s"(Bm), "+s"(packedA), "+s"(packedB), "+s"(nmA), "+s"(nmB), "+s"(nmBt), "+s"(tau_skip));
+    if (blockIdx.x < n_b)
+        normmap_strip_small<B, 1, SW, IN16, NWV>(Bm, nbN * B, nbK, nbN, strips_b, rec_b, packedB, nmB, nmBt, nullptr, nullptr, nullptr, tau_skip,
+                                                 keep_copy, blockIdx.x, s_pack, s_chunk, s_skip, s_seen);
+    else
+        normmap_strip_small<B, 0, SW, IN16, NWV>(A, nbK * B, nbM, nbK, strips_a, rec_a, packedA, nmA, nullptr, nullptr, nullptr, nullptr, tau_skip,
+                                                 keep_copy, blockIdx.x - n_b, s_pack, s_chunk, s_skip, s_seen);
 }
 
 // rowmax[k] = max_j nB[k, j] (nB row-major [nbK x nbN]); one wave per row.  NaNs are ignored:
@@ -503,24 +710,27 @@ static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int 
     const int64_t nbr = rows / tile, nbc = cols / tile;
     const bool keep = keep_input(rows * cols * (IN16 ? 2 : 4));
     const auto strips = [&](int64_t sw) { return (unsigned)(nbr * ((cols + sw - 1) / sw)); };
-#define SPAMM_NORMMAP_(T, SW, PH, NWV, KEEP)                                                                                        \
-    k_normmap<T, ROLE, SW, IN16, PH, NWV, KEEP><<<strips(SW), 64 * NWV, 0, s>>>(X, cols, cols, nbr, nbc, (cols + SW - 1) / SW, (uint4 *)packed, \
-                                                                                nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip,   \
-                                                                                keep_copy(rows * cols * 2))
-#define SPAMM_NORMMAP(T, SW, PH, NWV) SPAMM_NORMMAP_(T, SW, PH, NWV, false)
+#define SPAMM_NORMMAP(T, SW, PH, NWV)                                                                                              \
+    k_normmap<T, ROLE, SW, IN16, PH, NWV><<<strips(SW), 64 * NWV, 0, s>>>(X, cols, cols, nbr, nbc, (cols + SW - 1) / SW, (uint4 *)packed, \
+                                                                          nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip,        \
+                                                                          keep_copy(rows * cols * 2))
 // (the shapes that inputs of up to KEEP_INPUT_MAX take, but for a few fp16 ones)
-#define SPAMM_NORMMAP_KEEP(T, SW, PH, NWV)                                                     \
-    do {                                                                                       \
-        if (keep) SPAMM_NORMMAP_(T, SW, PH, NWV, true);                                        \
-        else SPAMM_NORMMAP_(T, SW, PH, NWV, false);                                            \
+#define SPAMM_NORMMAP_KEEP(T, SW, NWV)                                                                                             \
+    do {                                                                                                                           \
+        const uint32_t ns = (uint32_t)((cols + SW - 1) / SW);                                                                      \
+        if (keep)                                                                                                                  \
+            k_normmap_small<T, ROLE, SW, IN16, NWV><<<strips(SW), 64 * NWV, 0, s>>>(X, (uint32_t)cols, (uint32_t)nbr, (uint32_t)nbc, ns, \
+                                                                                    strip_reciprocal(ns), packed, nm, nmT, packed2, nm2, \
+                                                                                    rowmax, tau_skip, keep_copy(rows * cols * 2)); \
+        else SPAMM_NORMMAP(T, SW, 1, NWV);                                                                                         \
     } while (0)
     // strip widths and waves: one 8-row group per lane, at most ~42 KiB of LDS and so three workgroups or more per CU.
     // fp16 input: 256 columns, two rows per load (512 in phases before: tile 64 1024^2, both passes, 6.2 -> 4.1 us, 4096^2
     // 28.4 -> 26.3, 16384^2 A = B 303 -> 291; tile 32 2048^2 8.0 -> 7.3, 8192^2 tau-aware 93 -> 87).
     switch (tile) {
         case 32:
-            if constexpr (IN16) SPAMM_NORMMAP_KEEP(32, 256, 1, 2);
-            else SPAMM_NORMMAP_KEEP(32, 256, 1, 4);
+            if constexpr (IN16) SPAMM_NORMMAP_KEEP(32, 256, 2);
+            else SPAMM_NORMMAP_KEEP(32, 256, 4);
             break;
         case 64:
             // fp32 input: strips of 128 columns where there are few (1024^2, both passes: 5.4 -> 4.4 us; 4096^2 36.1 ->
@@ -532,8 +742,8 @@ static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int 
             // 3648^2 10.5 -> 10.1, 10.3 -> 10.5, 38.4 -> 36.4; 3584^2 8.9 -> 9.1, 9.5 -> 9.9, 37.0 -> 35.8
             if constexpr (IN16) {
                 if (strips(256) > 768u && strips(256) <= 1024u) SPAMM_NORMMAP(64, 512, 2, 8);
-                else SPAMM_NORMMAP_KEEP(64, 256, 1, 4);
-            } else if (strips(256) <= NARROW_STRIPS) SPAMM_NORMMAP_KEEP(64, 128, 1, 4);
+                else SPAMM_NORMMAP_KEEP(64, 256, 4);
+            } else if (strips(256) <= NARROW_STRIPS) SPAMM_NORMMAP_KEEP(64, 128, 4);
             else if (strips(256) <= 8192u) SPAMM_NORMMAP(64, 256, 1, 8);
             else SPAMM_NORMMAP(64, 256, 1, 4);
             break;
@@ -542,21 +752,20 @@ static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int 
         case 128:
             if constexpr (IN16) {
                 if constexpr (ROLE == 2) return hipErrorInvalidValue;      // (two passes, or the pair, are faster)
-                else SPAMM_NORMMAP_KEEP(128, 128, 1, 4);
+                else SPAMM_NORMMAP_KEEP(128, 128, 4);
             } else {
                 if constexpr (ROLE == 1)
                     if (strips(256) > 6000u) {
                         SPAMM_NORMMAP(128, 256, 2, 4);
                         break;
                     }
-                SPAMM_NORMMAP_KEEP(128, 128, 1, 8);
+                SPAMM_NORMMAP_KEEP(128, 128, 8);
             }
             break;
         default: return hipErrorInvalidValue;
     }
 #undef SPAMM_NORMMAP_KEEP
 #undef SPAMM_NORMMAP
-#undef SPAMM_NORMMAP_
     return hipGetLastError();
 }
 
@@ -573,9 +782,14 @@ static void launch_pair(const void *A, const void *Bm, int64_t nbM, int64_t nbK,
     const unsigned n_b = (unsigned)(nbK * strips_b), n_a = (unsigned)(nbM * strips_a);
     const int64_t a = nbM * nbK * B * B, b = nbK * nbN * B * B;
     const bool keep = keep_input((a + b) * (IN16 ? 2 : 4));
-    (keep ? &k_normmap_pair<B, SW, IN16, PH, NWV, true> : &k_normmap_pair<B, SW, IN16, PH, NWV, false>)<<<n_a + n_b, 64 * NWV, 0, s>>>(
-        A, Bm, nbM, nbK, nbN, n_b, strips_a, strips_b, (uint4 *)packedA, (uint4 *)packedB, nmA, nmB, nmBt, tau_skip,
-        keep_copy(2 * (a > b ? a : b)));
+    const bool cached = keep_copy(2 * (a > b ? a : b));
+    if (keep)
+        k_normmap_pair_small<B, SW, IN16, NWV><<<n_a + n_b, 64 * NWV, 0, s>>>(
+            A, Bm, (uint32_t)nbM, (uint32_t)nbK, (uint32_t)nbN, n_b, (uint32_t)strips_a, strip_reciprocal((uint32_t)strips_a),
+            (uint32_t)strips_b, strip_reciprocal((uint32_t)strips_b), packedA, packedB, nmA, nmB, nmBt, tau_skip, cached);
+    else
+        k_normmap_pair<B, SW, IN16, PH, NWV><<<n_a + n_b, 64 * NWV, 0, s>>>(A, Bm, nbM, nbK, nbN, n_b, strips_a, strips_b, (uint4 *)packedA,
+                                                                            (uint4 *)packedB, nmA, nmB, nmBt, tau_skip, cached);
 }
 
 // Where the two passes are worth running as one, by the strips of both operands, counted as tile rows of 1 KiB (256

@@ -409,3 +409,43 @@ def test_other_staging_rings_give_the_same_product(orc, ctx, ring):
     finally:
         ctx.set_option(sp.OPT_GEMM_SHAPE, 0)
         other.close()
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("tile", [32, 64, 128])
+def test_passes_over_small_inputs_end_strips_anywhere(orc, ctx, tile, half):
+    """The passes of small inputs, whose strips of up to eight tiles end at the last column or before it: each operand by itself, both in
+    one launch and A = B, copies and norm maps bit for bit, with tiles of zeros, subnormals and values from 2^-24 to 2^15; and a tau-aware
+    call beside a plain one."""
+    import torch
+    rng = np.random.default_rng(tile + half)
+    kind = torch.float16 if half else torch.float32
+
+    def operand(rows, cols):
+        x = (rng.uniform(-1.0, 1.0, (rows, cols)) * 2.0 ** rng.integers(-24, 16, (rows, cols))).astype(np.float32)
+        x[:tile, cols - tile:] = 0.0
+        x[rows - tile:, :tile] *= rng.random((tile, tile)) < 0.01
+        return torch.from_numpy(x).cuda().to(kind)
+
+    def same(role, X):
+        bits = X.half().cpu().numpy().view(np.uint16)
+        assert np.array_equal(ctx.get_fp16(role), bits)
+        assert np.array_equal(ctx.get_normmap(role).view(np.uint32), orc.normmap(bits, tile, role).view(np.uint32))
+
+    alone = ctx.normmap_f16 if half else ctx.normmap_f32
+    for m, k, n in ((1, 1, 1), (1, 2, 3), (3, 5, 7), (2, 8, 9), (9, 16, 4), (5, 17, 15)):
+        A, B = operand(m * tile, k * tile), operand(k * tile, n * tile)
+        alone(1, B, tile)
+        alone(0, A, tile)
+        same(0, A)
+        same(1, B)
+        want = ctx.multiply(A, B, tile, 0.5)
+        same(0, A)
+        same(1, B)
+        got = ctx.multiply(A, B, tile, 0.5, prune=True)
+        assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(want)) and torch.equal(got.isnan(), want.isnan())
+    for n in (1, 3, 8, 9):
+        A = operand(n * tile, n * tile)
+        ctx.multiply(A, A, tile, 0.5, a_eq_b=True)
+        same(0, A)
+        same(1, A)
