@@ -59,10 +59,10 @@ struct SmallCfg {
     static_assert(CHW == 1 || CPS >= 2, "a wave's two chunks lie in one slot, one after the other");
 };
 
-// LDS behind the ring: list entries, bitmap words of the unit's tiles, {full, partial} words, tile bits per k
-size_t small_lds_bytes_(int stage_bytes, int nbuf, int tt, int64_t nbK) {
+// LDS behind the ring: list entries, {full, partial} words, tile bits per k
+size_t small_lds_bytes_(int stage_bytes, int nbuf, int64_t nbK) {
     const size_t words = (size_t)((nbK + 63) / 64);
-    return (size_t)stage_bytes * nbuf + words * 64 * 4 + words * tt * 8 + words * 16 + words * 64 * 2;
+    return (size_t)stage_bytes * nbuf + words * 64 * 4 + words * 16 + words * 64 * 2;
 }
 
 // Offsets are 32-bit: C has SMALL_MAX_UNITS units of 128 x 128 at most and K / B is at most SMALL_MAX_NBK, so that C, the norm
@@ -74,16 +74,41 @@ struct SmallGrid {
     int xcd_shift, mode;     // log2 of the XCDs
 };
 
+// What a unit needs of GateBuffers, within the second line of arguments
+struct UnitGate {
+    const float *nA, *nBt;
+    KeptProducts *kept;
+    int32_t *counts;
+    uint64_t *mask;
+};
+
+// Two (or one) dma_loads of neighbouring chunks
+template <int N>
+__device__ __forceinline__ void dma_chunks(const unsigned char *sbase, uint32_t voff, uint32_t lds_addr) {
+    if constexpr (N == 2)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024"
+                     :
+                     : "s"(lds_addr), "v"(voff), "s"(sbase)
+                     : "memory", "m0");
+    else
+        dma_load<0>(sbase, voff, lds_addr);
+}
+
+// (Norms by buffers' scalar offsets, smallest and largest norm as integers, the first entries by one read of LDS, loads of full stages without a
+// look at the entry's bits, masks and counts formed at the end: 1024 rows against a resident 8192^2 23.6 -> 22.4 us alone, its gate 3.3 -> 2.8,
+// 5024 x 4128 x 3168 at tile 32, 10 % kept 41.3 -> 39.8, its gate 7.2 -> 6.0.)
 template <int B, int U, int RING>
-__device__ __forceinline__ void small_unit_body(const unsigned char *__restrict__ pA, const unsigned char *__restrict__ pB, const GateBuffers &g,
-                                                int nbM, int nbK, int nbN, const SmallGrid &sg, float tau, float *__restrict__ C) {
+__device__ __forceinline__ void small_unit_body(const unsigned char *pA, const unsigned char *pB, int nbM, int nbK, int nbN, SmallGrid sg,
+                                                float tau, float *C, UnitGate g) {
     using H = SmallCfg<B, U, RING>;
-    constexpr int NBUF = H::NBUF, MT = H::MT, TU = H::TU, TT = H::TT, NB = H::NB;
+    constexpr int NBUF = H::NBUF, MT = H::MT, TU = H::TU, TT = H::TT, NB = H::NB, BLK = MT / TU;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    // all arguments at once: a line of them asked for later is another 0.3 us
+    asm volatile("" : "+s"(pA), "+s"(pB), "+s"(nbM), "+s"(nbK), "+s"(nbN), "+s"(tau), "+s"(C), "+s"(g.nA), "+s"(g.nBt), "+s"(g.kept),
+                 "+s"(g.counts), "+s"(g.mask));
     const int words = (nbK + 63) >> 6, mode = sg.mode;
     uint32_t *s_list = reinterpret_cast<uint32_t *>(smem + NBUF * H::STAGE_BYTES);   // k | tile bits << 16
-    uint64_t *s_word = reinterpret_cast<uint64_t *>(s_list + words * 64);            // [words][TT]
-    uint64_t *s_fp = s_word + words * TT;                                            // [words][2]
+    uint64_t *s_fp = reinterpret_cast<uint64_t *>(s_list + words * 64);              // [words][2]
     uint16_t *s_bits = reinterpret_cast<uint16_t *>(s_fp + 2 * words);               // [words * 64]
 
     const int lane = threadIdx.x & 63;
@@ -99,34 +124,29 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
     if (urow >= M || ucol >= N) return;
     const int ti0 = urow / B, tj0 = ucol / B;                          // first tile of the unit
 
-    // ---- gate: a wave takes 64 k at a time, lane = k, and holds the norms of the macro tile's rows and
-    // columns (loads unconditional, from clamped addresses), the next 64's on their way
+    // ---- gate: a wave takes 64 k at a time, lane = k, and holds the norms of the macro tile's rows and columns, the unit's own first (rows
+    // clamped; a lane beyond the last k reads what follows, or nothing behind the map's end), the next 64's on their way
     const bool multiply = (mode & SMALL_MULTIPLY) != 0;        // (the gate alone needs no list, and the unit's norms only)
     const bool interior = (mi + 1) * MT <= nbM && (mj + 1) * MT <= nbN;
-    const int rows_in = nbM - ti0 < TU ? nbM - ti0 : TU, cols_in = nbN - tj0 < TU ? nbN - tj0 : TU;
-    uint32_t inside = (1u << cols_in) - 1u;                            // the unit's tiles that exist
-#pragma unroll
-    for (int x = 1; x < TU; x++) inside |= x < rows_in ? ((1u << cols_in) - 1u) << (x * TU) : 0u;
-    float a[MT] = {}, b[MT] = {}, au[TU], bu[TU];
+    const int rows_in = nbM - ti0, cols_in = nbN - tj0;                // of the unit's tile rows and columns, those below exist
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)g.nA, 0, nbM * nbK * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)g.nBt, 0, nbN * nbK * 4, 0x00020000);
+    uint32_t a[MT] = {}, b[MT] = {};
     auto load_norms = [&](int w) {
-        const int k = w * 64 + lane;
-        const uint32_t kb = (uint32_t)(k < nbK ? k : nbK - 1) * 4u;
-        auto norm = [&](const float *map, int row, int n) {
-            const uint32_t at = (uint32_t)((row < n ? row : n - 1) * nbK) * 4u + kb;
-            return *reinterpret_cast<const float *>(reinterpret_cast<const unsigned char *>(map) + at);
-        };
-        if (multiply) {
-#pragma unroll
-            for (int x = 0; x < MT; x++) {
-                a[x] = norm(g.nA, mi * MT + x, nbM);
-                b[x] = norm(g.nBt, mj * MT + x, nbN);
-            }
-        } else {
+        const int voff = (w * 64 + lane) * 4, stride = nbK * 4;
+        auto load = [&](int blk) {
+            const int i0 = mi * MT + ((ti0 + blk * TU) & (MT - 1)), j0 = mj * MT + ((tj0 + blk * TU) & (MT - 1));
 #pragma unroll
             for (int x = 0; x < TU; x++) {
-                au[x] = norm(g.nA, ti0 + x, nbM);
-                bu[x] = norm(g.nBt, tj0 + x, nbN);
+                const int i = i0 + x < nbM ? i0 + x : nbM - 1, j = j0 + x < nbN ? j0 + x : nbN - 1;
+                a[blk * TU + x] = __builtin_amdgcn_raw_buffer_load_b32(ra, voff, i * stride, 0);
+                b[blk * TU + x] = __builtin_amdgcn_raw_buffer_load_b32(rb, voff, j * stride, 0);
             }
+        };
+        load(0);
+        if (multiply) {
+#pragma unroll
+            for (int blk = 1; blk < BLK; blk++) load(blk);
         }
     };
     if (wave < words) load_norms(wave);
@@ -134,52 +154,36 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
     for (int w = wave; w < words; w += 4) {
         const int k = w * 64 + lane;
         const bool live = k < nbK;
-        if (multiply) {                                                // the unit's among the macro tile's
+        float au[TU], bu[TU];
 #pragma unroll
-            for (int x = 0; x < TU; x++) {
-                au[x] = a[x];
-                bu[x] = b[x];
-#pragma unroll
-                for (int o = TU; o < MT; o += TU) {
-                    au[x] = ti0 - mi * MT == o ? a[o + x] : au[x];
-                    bu[x] = tj0 - mj * MT == o ? b[o + x] : bu[x];
-                }
-            }
+        for (int x = 0; x < TU; x++) {                                 // (what does not exist is kept at no threshold: NaN)
+            au[x] = live && x < rows_in ? __uint_as_float(a[x]) : __builtin_nanf("");
+            bu[x] = x < cols_in ? __uint_as_float(b[x]) : __builtin_nanf("");
         }
-        uint32_t ub = 0;
+        uint32_t ub = 0;                                               // the unit's tiles that keep this lane's k
 #pragma unroll
-        for (int x = 0; x < TU; x++)
+        for (int t = TT - 1; t >= 0; t--) ub = ub + ub + (au[t / TU] * bu[t % TU] >= tau ? 1u : 0u);
+        // kept by every tile of the macro tile: rounding is monotone, so the product of the smallest norms decides -- unless one
+        // is not finite (inf * 0 and NaN are never kept), or below zero: then all products are looked at
+        uint32_t amin = a[0], bmin = b[0], big = a[0] > b[0] ? a[0] : b[0];
 #pragma unroll
-            for (int y = 0; y < TU; y++) ub |= au[x] * bu[y] >= tau ? 1u << (x * TU + y) : 0u;
-        ub = live ? ub & inside : 0u;
-        // kept by every tile of the macro tile: rounding is monotone, so the product of the smallest norms
-        // decides -- unless one is not finite (inf * 0 and NaN are never kept): then all products are looked at
-        float amin = a[0], bmin = b[0];
-        bool finite = true;
-#pragma unroll
-        for (int x = 0; x < MT; x++) {
-            finite = finite && __builtin_isfinite(a[x]) && __builtin_isfinite(b[x]);
-            amin = fminf(amin, a[x]);
-            bmin = fminf(bmin, b[x]);
+        for (int x = 1; x < MT; x++) {
+            amin = a[x] < amin ? a[x] : amin;
+            bmin = b[x] < bmin ? b[x] : bmin;
+            const uint32_t m = a[x] > b[x] ? a[x] : b[x];
+            big = m > big ? m : big;
         }
-        bool full = amin * bmin >= tau;
-        if (__ballot(!finite) != 0ull) {
+        bool full = __uint_as_float(amin) * __uint_as_float(bmin) >= tau;
+        if (__ballot(big >= 0x7f800000u) != 0ull) {
             full = true;
 #pragma unroll
             for (int x = 0; x < MT; x++)
 #pragma unroll
-                for (int y = 0; y < MT; y++) full = full && a[x] * b[y] >= tau;
+                for (int y = 0; y < MT; y++) full = full && __uint_as_float(a[x]) * __uint_as_float(b[y]) >= tau;
         }
         full = full && live && interior;
         const uint64_t F = __ballot(full), P = __ballot(ub != 0u && !full);
         if (w + 4 < words) load_norms(w + 4);
-        uint64_t mine = 0;                                             // lane t: bitmap word of tile t
-#pragma unroll
-        for (int t = 0; t < TT; t++) {
-            const uint64_t m = __ballot((ub >> t) & 1u);
-            mine = lane == t ? m : mine;
-        }
-        if (lane < TT) s_word[w * TT + lane] = mine;
         if (lane == 0) {
             s_fp[2 * w] = F;
             s_fp[2 * w + 1] = P;
@@ -187,43 +191,44 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
         s_bits[k] = (uint16_t)ub;
     }
     __syncthreads();
-    // What the gate leaves behind (a tile shared by several units is written by the first).  A unit's kept products are
-    // a word of its own: added to one total by atomics they queued up at the kernel's end, where 200 to 1000 units finish
-    // together (1024^3 10 % 15.4 -> 13.7 us whole, 2048^3 dense 33.8 -> 31.5, 1056 x 1568 x 1312 18.6 -> 17.7).  The total is
-    // minus their number then: what the last gate was is known on the device, also behind a replayed graph.  (By a wave that has
-    // nothing else to store: behind unit 0's own word it was 0.13 us.)
-    // Counts and places are worked out while the first stages' loads are under way; what is left for the end is a store or two
-    // (0.8 us with all of it at the end).
-    struct Left {
-        int tile, count, total;      // lane t < TT: the tile's number (-1: not this unit's) and kept k; lane 0: the unit's
-    };
-    auto count_gate = [&]() -> Left {
-        Left l = {-1, 0, 0};
-        if (!(mode & SMALL_GATE)) return l;
-        const int i = ti0 + lane / TU, j = tj0 + lane % TU;
-        if ((ui * U) % B == 0 && (uj * U) % B == 0 && lane < TT && i < nbM && j < nbN) l.tile = i * nbN + j;
-        if (wave == 0) {
-            if (l.tile >= 0)
-                for (int w = 0; w < words; w++) l.count += __builtin_popcountll(s_word[w * TT + lane]);
-            l.total = l.count;
-#pragma unroll
-            for (int off = 1; off < TT; off <<= 1) l.total += __shfl_xor(l.total, off, 64);
-        }
-        return l;
-    };
-    auto store_gate = [&](const Left &l) {
+    // What the gate leaves behind, out of s_bits: wave x has row x of the unit's tiles (a tile shared by several units is written by the
+    // first).  A unit's kept products are a word of its own: added to one total by atomics they queued up at the kernel's end, where 200
+    // to 1000 units finish together (1024^3 10 % 15.4 -> 13.7 us whole, 2048^3 dense 33.8 -> 31.5, 1056 x 1568 x 1312 18.6 -> 17.7).  The total is
+    // minus their number then: what the last gate was is known on the device, also behind a replayed graph.
+    auto store_gate = [&]() {
         if (!(mode & SMALL_GATE)) return;
-        const int units_n = (N + U - 1) / U;
-        if (unit == 0 && wave == 3 && lane == 0) g.kept->total = -((M + U - 1) / U * units_n);
-        if (l.tile >= 0)
-            for (int w = wave; w < words; w += 4) g.mask[(uint32_t)(l.tile * words + w)] = s_word[w * TT + lane];
-        if (wave == 0) {
-            if (l.tile >= 0) g.counts[(uint32_t)l.tile] = l.count;
-            if (lane == 0) g.kept->units[urow / U * units_n + ucol / U] = (uint32_t)l.total;
+        const bool owner = (ui * U) % B == 0 && (uj * U) % B == 0;
+        if (wave < TU && wave < rows_in && owner) {
+            const bool mine = lane < TU && lane < cols_in;
+            const uint32_t tile = (uint32_t)((ti0 + wave) * nbN + tj0 + lane);
+            int count = 0;
+            for (int w = 0; w < words; w++) {
+                const uint32_t ub = (uint32_t)s_bits[w * 64 + lane] >> (wave * TU);
+                uint64_t word = 0;
+#pragma unroll
+                for (int y = 0; y < TU; y++) {
+                    const uint64_t m = __ballot((ub >> y) & 1u);
+                    word = lane == y ? m : word;
+                }
+                if (mine) g.mask[tile * (uint32_t)words + w] = word;
+                count += __builtin_popcountll(word);
+            }
+            if (mine) g.counts[tile] = count;
+        }
+        if (wave == 3) {
+            const int units_n = (N + U - 1) / U;
+            int total = 0;
+            if (owner)
+                for (int w = 0; w < words; w++) total += __builtin_popcount((uint32_t)s_bits[w * 64 + lane]);
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) total += __shfl_xor(total, off, 64);
+            if (lane == 0) {
+                g.kept->units[urow / U * units_n + ucol / U] = (uint32_t)total;
+                if (unit == 0) g.kept->total = -((M + U - 1) / U * units_n);
+            }
         }
     };
 
-    Left left;
     int S = 0, Sfull = 0;
     if (multiply) {
         // ---- list: every wave scans the words' counts (at most 64 words), then places its own words' entries
@@ -272,7 +277,6 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
             for (int r = wave * (64 / LPR) + lane / LPR; r < U && urow + r < M; r += 4 * (64 / LPR))
                 __builtin_nontemporal_store(zero, reinterpret_cast<f32x4 *>(C + (uint32_t)((urow + r) * N + c0)));
     }
-    if (S == 0) left = count_gate();
     f32x4 acc[NB][NB];
 #pragma unroll
     for (int r = 0; r < NB; r++)
@@ -295,19 +299,13 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
 
         // entry of a stage (stages beyond the last repeat the last entry: loaded, never multiplied)
         auto entry_at = [&](int t) -> uint32_t { return s_list[(t < S ? t : S - 1) / H::NSPE]; };
-        auto issue = [&](int t, uint32_t ent, uint32_t boff, auto idx) {
-            constexpr int i = decltype(idx)::value, j = i % H::CHW;
-            const int64_t koff = (int64_t)(ent & 0xffffu) * H::TILE_BYTES + ((t < S ? t : S - 1) % H::NSPE) * (B * 64);
-            // a slot that no tile pair of the entry reads is not fetched: its load goes to one place that is
-            // cache resident, so that the number of loads in flight stays fixed
-            if constexpr (i < H::CHW) {
-                const int64_t on = (ent & needA) ? -1ll : 0ll;
-                dma_load<j * 1024>(pA + (((rowA - pA) + koff) & on), voff, ldsA + boff);
-            } else {
-                const int64_t on = (ent & needB) ? -1ll : 0ll;
-                dma_load<j * 1024>(pB + (((rowB - pB) + koff) & on), voff, ldsB + boff);
-            }
+        auto offset = [&](int t, uint32_t ent) -> uint32_t {           // (a row of tiles is at most SMALL_MAX_NBK tiles: 64 MiB)
+            return (ent & 0xffffu) * H::TILE_BYTES + (uint32_t)(((t < S ? t : S - 1) % H::NSPE) * (B * 64));
         };
+        // a slot that no tile pair of the entry reads is not fetched: its load goes to one place that is cache resident, so that the
+        // number of loads in flight stays fixed
+        auto issue_a = [&](const unsigned char *from, uint32_t boff) { dma_chunks<H::CHW>(from, voff, ldsA + boff); };
+        auto issue_b = [&](const unsigned char *from, uint32_t boff) { dma_chunks<H::CHW>(from, voff, ldsB + boff); };
         auto sync_next = [&]() {
             __builtin_amdgcn_s_waitcnt(waitcnt_imm(H::LPW * (NBUF - 2), 0));
             __syncthreads();
@@ -327,16 +325,18 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
             else if constexpr (i <= NB) f.b[i - 1] = *reinterpret_cast<const half8 *>(bufA + H::OP_BYTES + frag_off(wc, i - 1));
             else f.a[i - NB] = *reinterpret_cast<const half8 *>(bufA + frag_off(wr, i - NB));
         };
-        // ---- prologue
+        // ---- prologue: the first entries by one read (each in turn, their latencies were half of it)
+        const uint32_t firsts = entry_at(lane);
 #pragma unroll
         for (int t = 0; t < NBUF; t++) {
-            const uint32_t e = __builtin_amdgcn_readfirstlane(entry_at(t));
-            static_for<H::LPW>([&](auto i) { issue(t, e, t * H::STAGE_BYTES, i); });
+            const uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)firsts, t), koff = offset(t, e);
+            issue_a((e & needA) ? rowA + koff : pA, t * H::STAGE_BYTES);
+            issue_b((e & needB) ? rowB + koff : pB, t * H::STAGE_BYTES);
         }
         // The buffer of stage t -- once that is in registers, of stage t + NBUF -- and the next one's, which is formed before the
         // sync: behind it a wave's first reads of LDS wait for their address.  (By t % NBUF where they are used the compiler
         // put up to 13 scalar instructions there, which depended on the order of the kernel's arguments: 384 x 4736 x 416 at
-        // tile 32 33.4 or 34.3 us, 32.75 now; 1056 x 1568 x 1312 17.34 or 17.5, 17.07 now.)
+        // tile 32 33.4 or 34.3 us, 32.75 then; 1056 x 1568 x 1312 17.34 or 17.5, 17.07 then.)
         int t = 0;
         uint32_t buf = 0;
         auto next_buf = [&]() {
@@ -345,24 +345,26 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
             return next;
         };
         uint32_t e_cur = entry_at(0), e_new = entry_at(NBUF);
-        left = count_gate();
         __builtin_amdgcn_s_waitcnt(waitcnt_imm(H::LPW * (NBUF - 1), 0));
         __syncthreads();
         Frags f0, f1;
         static_for<2 * NB>([&](auto i) { load_frag(f0, 0, i); });
 #define SPAMM_FENCE() __builtin_amdgcn_sched_barrier(0)
+        // (every slot of the stages that are fetched here is, whether its entry reads it or not: all but the last few are full ones)
         auto full_stage = [&](const Frags &cur, Frags &nxt) {
             const uint32_t next = next_buf();
             sync_next();
             const uint32_t en = __builtin_amdgcn_readfirstlane(e_new);
-            e_cur = entry_at(t + 1);
             e_new = entry_at(t + 1 + NBUF);
             SPAMM_FENCE();
+            uint32_t koff = 0;
             static_for<NB * NB>([&](auto idx) {
-                constexpr int i = decltype(idx)::value, r = i / NB, c = i % NB;
+                constexpr int i = decltype(idx)::value, r = i / NB, c = i % NB, A_AT = NB == 4 ? 8 : 2, B_AT = NB == 4 ? 12 : 3;
                 acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cur.a[r], cur.b[c], acc[r][c], 0, 0, 0);
                 if constexpr (i < 2 * NB) load_frag(nxt, next, idx);
-                if constexpr (NB == 4 ? (i >= 8 && i % 2 == 0) : i >= 2) issue(t + NBUF, en, buf, std::integral_constant<int, NB == 4 ? (i >= 8 ? (i - 8) / 2 : 0) : (i >= 2 ? i - 2 : 0)>{});
+                if constexpr (i == A_AT - 1) koff = offset(t + NBUF, en);
+                if constexpr (i == A_AT) issue_a(rowA + koff, buf);
+                if constexpr (i == B_AT) issue_b(rowB + koff, buf);
                 SPAMM_FENCE();
             });
             t++;
@@ -372,6 +374,7 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
             full_stage(f0, f1);
             full_stage(f1, f0);
         }
+        e_cur = entry_at(t);
         auto partial_stage = [&](const Frags &cur, Frags &nxt) {
             const uint32_t next = next_buf();
             sync_next();
@@ -379,6 +382,7 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
             const uint32_t ec = t < S ? (__builtin_amdgcn_readfirstlane(e_cur) >> 16) >> (TU > 1 ? wr * TU + wc : 0) : 0u;
             e_cur = entry_at(t + 1);
             e_new = entry_at(t + 1 + NBUF);
+            const uint32_t koff = offset(t + NBUF, en);
             SPAMM_FENCE();
             static_for<H::NP * H::NP>([&](auto pair) {
                 constexpr int p = decltype(pair)::value, px = p / H::NP, py = p % H::NP, bit = 2 * px * TU + 2 * py;
@@ -393,7 +397,8 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
                 if constexpr (p == 0) {
                     SPAMM_FENCE();
                     static_for<2 * NB>([&](auto i) { load_frag(nxt, next, i); });
-                    static_for<H::LPW>([&](auto i) { issue(t + NBUF, en, buf, i); });
+                    issue_a((en & needA) ? rowA + koff : pA, buf);
+                    issue_b((en & needB) ? rowB + koff : pB, buf);
                     SPAMM_FENCE();
                 }
             });
@@ -401,8 +406,9 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
             t++;
             buf = next;
         };
-        while (__builtin_expect(t < S, 1)) {
+        while (t < S) {
             partial_stage(f0, f1);
+            if (t >= S) break;
             partial_stage(f1, f0);
         }
 #undef SPAMM_FENCE
@@ -431,23 +437,23 @@ __device__ __forceinline__ void small_unit_body(const unsigned char *__restrict_
             }
         }
     }
-    store_gate(left);
+    store_gate();
 }
 
 // The arguments come in the order of their use, and all that are read lie in the first 128 bytes: a line of them that nothing
 // has asked for yet is 0.2 to 0.4 us away when it is needed (256^3 10.44 -> 10.27 us, fp16 2048^3 at tile 32, 5 % kept 25.15 ->
 // 24.74 against M, N and C in a third line).
 template <int B, int U>
-__global__ __launch_bounds__(256, 2) void k_small(const unsigned char *__restrict__ pA, const unsigned char *__restrict__ pB, int nbM, int nbK,
-                                                  int nbN, SmallGrid sg, float tau, float *__restrict__ C, GateBuffers g) {
-    small_unit_body<B, U, (U == 128 ? 4 : 6)>(pA, pB, g, nbM, nbK, nbN, sg, tau, C);
+__global__ __launch_bounds__(256, 2) void k_small(const unsigned char *pA, const unsigned char *pB, int nbM, int nbK, int nbN, SmallGrid sg,
+                                                  float tau, float *C, UnitGate g) {
+    small_unit_body<B, U, (U == 128 ? 4 : 6)>(pA, pB, nbM, nbK, nbN, sg, tau, C, g);
 }
 
 // Units of 128 by three workgroups per CU (small_three).
 template <int B>
-__global__ __launch_bounds__(256, 3) void k_small_three(const unsigned char *__restrict__ pA, const unsigned char *__restrict__ pB, int nbM,
-                                                        int nbK, int nbN, SmallGrid sg, float tau, float *__restrict__ C, GateBuffers g) {
-    small_unit_body<B, 128, 3>(pA, pB, g, nbM, nbK, nbN, sg, tau, C);
+__global__ __launch_bounds__(256, 3) void k_small_three(const unsigned char *pA, const unsigned char *pB, int nbM, int nbK, int nbN,
+                                                        SmallGrid sg, float tau, float *C, UnitGate g) {
+    small_unit_body<B, 128, 3>(pA, pB, nbM, nbK, nbN, sg, tau, C, g);
 }
 
 // ---------------------------------------------------------------- one word of k tiles (K / tile <= 64), the usual small problem
@@ -485,17 +491,9 @@ __device__ __forceinline__ void dma_buffer(const i32x4s &rsrc, uint32_t voff, ui
                      : "memory", "m0");
 }
 
-// What a unit needs of GateBuffers, within the second line of arguments
-struct WordGate {
-    const float *nA, *nBt;
-    KeptProducts *kept;
-    int32_t *counts;
-    uint64_t *mask;
-};
-
 template <int B, int U, int RING>
 __device__ __forceinline__ void small_word_body(const unsigned char *pA, const unsigned char *pB, int nbM, int nbK, int nbN, SmallGrid sg,
-                                                float tau, float *C, WordGate g) {
+                                                float tau, float *C, UnitGate g) {
     using H = SmallCfg<B, U, RING>;
     constexpr int NBUF = H::NBUF, MT = H::MT, TU = H::TU, TT = H::TT, NB = H::NB, BLK = MT / TU;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -795,13 +793,13 @@ static constexpr int WORD_RING = U == 128 ? 4 : 5;
 
 template <int B, int U>
 __global__ __launch_bounds__(256, 2) void k_small_word(const unsigned char *pA, const unsigned char *pB, int nbM, int nbK, int nbN,
-                                                       SmallGrid sg, float tau, float *C, WordGate g) {
+                                                       SmallGrid sg, float tau, float *C, UnitGate g) {
     small_word_body<B, U, WORD_RING<U>>(pA, pB, nbM, nbK, nbN, sg, tau, C, g);
 }
 
 template <int B>
 __global__ __launch_bounds__(256, 3) void k_small_word_three(const unsigned char *pA, const unsigned char *pB, int nbM, int nbK, int nbN,
-                                                             SmallGrid sg, float tau, float *C, WordGate g) {
+                                                             SmallGrid sg, float tau, float *C, UnitGate g) {
     small_word_body<B, 128, 3>(pA, pB, nbM, nbK, nbN, sg, tau, C, g);
 }
 
@@ -828,9 +826,8 @@ static int small_unit(int64_t units128) { return units128 >= 128 ? 128 : 64; }
 // 32.9 -> 38.1 us; 600 units at tile 32, 3.5 % 31.3 -> 34.3), slow decay gains (576 units, 30 % algebraic 50.8 -> 45.0, 550 units,
 // 10 % 42.4 -> 38.9): the host cannot tell them apart, and bands are the usual operands.  A list too long for three in a CU's LDS
 // keeps the ring of four.
-static bool small_three(int64_t units128, int64_t nbK, int tile) {
-    const int tt = tile >= 128 ? 1 : (128 / tile) * (128 / tile);
-    return units128 > 600 && 3 * (small_lds_bytes_(16384, 3, tt, nbK) + 2048) <= 160 * 1024;
+static bool small_three(int64_t units128, int64_t nbK) {
+    return units128 > 600 && 3 * (small_lds_bytes_(16384, 3, nbK) + 2048) <= 160 * 1024;
 }
 
 // (WORD: one word of k tiles)
@@ -845,7 +842,7 @@ static constexpr auto small_kernel() {
 template <int B, int U, bool THREE, bool WORD>
 static size_t small_lds(int64_t nbK) {
     using H = SmallCfg<B, U, (THREE ? 3 : (WORD ? WORD_RING<U> : (U == 128 ? 4 : 6)))>;
-    return WORD ? (size_t)H::STAGE_BYTES * H::NBUF : small_lds_bytes_(H::STAGE_BYTES, H::NBUF, H::TT, nbK);
+    return WORD ? (size_t)H::STAGE_BYTES * H::NBUF : small_lds_bytes_(H::STAGE_BYTES, H::NBUF, nbK);
 }
 
 template <int B, int U, bool THREE>
@@ -858,11 +855,11 @@ static hipError_t launch_small_(const void *pA, const void *pB, const GateBuffer
     const unsigned grid = (unsigned)((n_units + n_xcd - 1) / n_xcd * n_xcd);
     const SmallGrid sg = {nMacN, 0xffffffffu / (uint32_t)nMacN, n_units, (n_units + n_xcd - 1) / n_xcd, __builtin_ctz((unsigned)n_xcd), mode};
     const unsigned char *a = (const unsigned char *)pA, *b = (const unsigned char *)pB;
+    const UnitGate w = {g.nA, g.nBt, g.kept, g.counts, g.mask};
     if (nbK <= 64)
-        small_kernel<B, U, THREE, true>()<<<grid, 256, small_lds<B, U, THREE, true>(nbK), s>>>(a, b, nbM, nbK, nbN, sg, tau, C,
-                                                                                          WordGate{g.nA, g.nBt, g.kept, g.counts, g.mask});
+        small_kernel<B, U, THREE, true>()<<<grid, 256, small_lds<B, U, THREE, true>(nbK), s>>>(a, b, nbM, nbK, nbN, sg, tau, C, w);
     else
-        small_kernel<B, U, THREE, false>()<<<grid, 256, small_lds<B, U, THREE, false>(nbK), s>>>(a, b, nbM, nbK, nbN, sg, tau, C, g);
+        small_kernel<B, U, THREE, false>()<<<grid, 256, small_lds<B, U, THREE, false>(nbK), s>>>(a, b, nbM, nbK, nbN, sg, tau, C, w);
     return hipGetLastError();
 }
 
@@ -939,7 +936,7 @@ static hipError_t launch_small_(const void *pA, const void *pB, const GateBuffer
                                 int mode, float tau, float *C, int n_cu, int n_xcd, hipStream_t s) {
     const int64_t units128 = units_of_128(M, N, n_cu);
     if (small_unit(units128) != 128) return launch_small_<B, 64, false>(pA, pB, g, M, K, N, mode, tau, C, n_xcd, s);
-    if (small_three(units128, K / B, B)) return launch_small_<B, 128, true>(pA, pB, g, M, K, N, mode, tau, C, n_xcd, s);
+    if (small_three(units128, K / B)) return launch_small_<B, 128, true>(pA, pB, g, M, K, N, mode, tau, C, n_xcd, s);
     return launch_small_<B, 128, false>(pA, pB, g, M, K, N, mode, tau, C, n_xcd, s);
 }
 

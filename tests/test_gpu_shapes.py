@@ -298,7 +298,8 @@ def test_middling_outputs_in_one_launch_give_the_same_product(orc, ctx, M, K, N,
 
 @pytest.mark.parametrize("M,K,N,tile", [(192, 64, 320, 64), (1088, 4032, 832, 64), (1152, 4096, 2112, 64), (2048, 4160, 1088, 64),
                                         (256, 128, 384, 128), (640, 8064, 1152, 128), (1920, 8192, 2176, 128), (1920, 8320, 2176, 128),
-                                        (3200, 64, 3264, 64), (3264, 2048, 3136, 64), (3200, 128, 3200, 128)])
+                                        (3200, 64, 3264, 64), (3264, 2048, 3136, 64), (3200, 128, 3200, 128),
+                                        (3200, 16416, 3136, 32)])   # (a list too long for three units to a CU)
 def test_one_word_of_k_tiles_at_its_ends(orc, ctx, M, K, N, tile):
     """The kernel whose list is a register, at one k tile, at 63 and 64 and the other one at 65, by every size of unit and two and
     three units to a CU; stages of its own here (a gate that forms no list), too."""
