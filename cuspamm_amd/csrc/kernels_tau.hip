@@ -25,6 +25,10 @@
 // Whole calls, norm maps and the multiply behind them included: 5024 x 4128 x 3168 at
 // tile 32 to a kept fraction 667 -> 133 us, the reference's tuned 2048^3 (8 of at most
 // 20 rounds) 381 -> 75 us.
+// What is left in a launch of 2.6e5 products, 6.3 us for a count: five round trips past the L2 (arguments, norms, parts, ticket, parts
+// again), the result's way to the host, and some 500 instructions.  (Divisions of a step's number, 64-bit addresses of its rows, wave sums by
+// LDS shuffles, the tree's state read word by word and its decisions taken one after the other by one thread: count 7.35 -> 6.3 us, a bisection
+// of one tree 18.75 -> 16.4, a selection 22.4 -> 21.7; 2.1e6 products 7.7 -> 6.9, 24.3 -> 21.9, 24.6 -> 23.5.)
 #include "gemm_device.h"
 #include "reduce_device.h"
 
@@ -62,28 +66,116 @@ size_t tau_workspace_bytes() { return sizeof(TauWorkspace); }
 // live) runs in all lanes; `live` is false in lanes beyond the last k.  A wave's step is one round trip
 // of TAU_JB + 1 loads and some hundred instructions, so the steps are kept small and spread over as many
 // waves as there are (whole rows of k per wave: 22 us instead of 15 for the last pass over 1.7e7 products).
-template <int TAU_JB, typename F>
-__device__ __forceinline__ void for_products(const float *__restrict__ nA, const float *__restrict__ nBt, int nbM, int nbK,
-                                             int nbN, F &&f) {
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int jb = (nbN + TAU_JB - 1) / TAU_JB, kb = (nbK + 63) / 64;
-    const int64_t units = (int64_t)nbM * jb * kb;
-    for (int64_t u = (int64_t)blockIdx.x * TAU_NW + wave; u < units; u += (int64_t)gridDim.x * TAU_NW) {
-        // (nbM * jb <= 65535 * 16384 < 2^31; the 64-bit division is a long routine that small problems need not run)
-        const int ij = units <= 0x7fffffff ? (int)u / kb : (int)(u / kb);
-        const int k0 = (int)(u - (int64_t)ij * kb) * 64;
-        const int i = ij / jb, j0 = (ij % jb) * TAU_JB;
-        const bool live = k0 + lane < nbK;
-        const int k = live ? k0 + lane : nbK - 1;
-        const float a = nA[(int64_t)i * nbK + k];
-        float b[TAU_JB];
-#pragma unroll
-        for (int jj = 0; jj < TAU_JB; jj++) b[jj] = nBt[(int64_t)(j0 + jj < nbN ? j0 + jj : nbN - 1) * nbK + k];
+// In two parts, as most waves have one step or a few: the first step's norms are asked for by the constructor, ahead of what a
+// kernel prepares for its products.  Rows lie at a buffer's scalar offset, a step's place comes by reciprocals (TauGrid).
+struct TauGrid {
+    uint32_t kb, jb;             // words of 64 k, groups of TAU_JB columns
+    uint32_t rec_kb, rec_jb;     // floor((2^32 - 1) / kb), (.. / jb); rec_kb = 0: steps * kb or rows * jb * jb leaves 32 bits, divide
+};
+
+template <int TAU_JB>
+struct Products {
+    const float *nA, *nBt;
+    int nbM, nbK, nbN;
+    TauGrid g;
+    int64_t units, u;
+    int lane, rows;              // rows: of TAU_JB, those that exist
+    bool live;
+    float a, b[TAU_JB];
+
+    __device__ __forceinline__ void load() {
+        uint32_t ij, i, j;
+        int k0;
+        if (g.rec_kb) {
+            ij = __umulhi((uint32_t)u + 1u, g.rec_kb);
+            k0 = (int)((uint32_t)u - ij * g.kb) * 64;
+            i = __umulhi(ij + 1u, g.rec_jb);
+            j = ij - i * g.jb;
+        } else {
+            ij = (uint32_t)(u / g.kb);
+            k0 = (int)(u - (int64_t)ij * g.kb) * 64;
+            i = ij / g.jb;
+            j = ij % g.jb;
+        }
+        const int j0 = (int)j * TAU_JB, stride = nbK * 4;
+        rows = nbN - j0 < TAU_JB ? nbN - j0 : TAU_JB;
+        live = k0 + lane < nbK;
+        const int voff = (live ? k0 + lane : nbK - 1) * 4;
+        const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)(nA + (int64_t)i * nbK), 0, stride, 0x00020000);
+        const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)(nBt + (int64_t)j0 * nbK), 0, rows * stride, 0x00020000);
+        a = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ra, voff, 0, 0));
 #pragma unroll
         for (int jj = 0; jj < TAU_JB; jj++)
-            if (j0 + jj < nbN) f(a * b[jj], live);
+            b[jj] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, voff, (jj < rows ? jj : rows - 1) * stride, 0));
     }
+    __device__ __forceinline__ Products(const float *nA_, const float *nBt_, int nbM_, int nbK_, int nbN_, const TauGrid &g_)
+        : nA(nA_), nBt(nBt_), nbM(nbM_), nbK(nbK_), nbN(nbN_), g(g_) {
+        lane = threadIdx.x & 63;
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        units = (int64_t)nbM * g.jb * g.kb;
+        u = (int64_t)blockIdx.x * TAU_NW + wave;
+        if (u < units) load();
+    }
+    template <typename F>
+    __device__ __forceinline__ void each(F &&f) {
+        while (u < units) {
+#pragma unroll
+            for (int jj = 0; jj < TAU_JB; jj++)
+                if (jj < rows) f(a * b[jj], live);
+            u += (int64_t)gridDim.x * TAU_NW;
+            if (u < units) load();
+        }
+    }
+};
+
+// Sum over the 64 lanes in every lane, added as shuffles down by 32, 16, .. 1 add in lane 0, without LDS operations: behind the first
+// two steps a lane's partner is anywhere in its row, which repeats every 8, 4, 2 lanes.
+template <typename T>
+__device__ __forceinline__ T wave_sum(T v) {
+    struct Words {
+        uint32_t w[sizeof(T) / 4];
+    };
+    auto both = [&](auto swap) {
+        Words x = __builtin_bit_cast(Words, v), lo, hi;
+#pragma unroll
+        for (unsigned i = 0; i < sizeof(T) / 4; i++) {
+            const auto r = swap(x.w[i]);
+            lo.w[i] = r[0];
+            hi.w[i] = r[1];
+        }
+        v = __builtin_bit_cast(T, lo) + __builtin_bit_cast(T, hi);
+    };
+    both([](uint32_t x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); });
+    both([](uint32_t x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); });
+    auto turned = [&](auto ctrl) {
+        Words x = __builtin_bit_cast(Words, v);
+#pragma unroll
+        for (unsigned i = 0; i < sizeof(T) / 4; i++)
+            x.w[i] = (uint32_t)__builtin_amdgcn_update_dpp((int)x.w[i], (int)x.w[i], decltype(ctrl)::value, 0xF, 0xF, false);
+        v = v + __builtin_bit_cast(T, x);
+    };
+    turned(std::integral_constant<int, 0x128>{});                // row rotated by 8, 4, 2, 1
+    turned(std::integral_constant<int, 0x124>{});
+    turned(std::integral_constant<int, 0x122>{});
+    turned(std::integral_constant<int, 0x121>{});
+    return v;
+}
+
+// Inclusive sum over the lanes up to each, without LDS operations
+__device__ __forceinline__ unsigned long long wave_scan(unsigned long long v) {
+    auto step = [&](auto ctrl, auto rows) {
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+        v += (unsigned long long)hi << 32 | lo;
+    };
+    constexpr std::integral_constant<int, 0xF> all{};
+    step(std::integral_constant<int, 0x111>{}, all);             // from 1, 2, 4, 8 lanes below in the row
+    step(std::integral_constant<int, 0x112>{}, all);
+    step(std::integral_constant<int, 0x114>{}, all);
+    step(std::integral_constant<int, 0x118>{}, all);
+    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});      // the last lane of rows 0 and 2 to the row above,
+    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});      // of row 1 to the two above it
+    return v;
 }
 
 // One digit of the select: histogram of the PASS-th digit over the products whose higher bits equal
@@ -98,21 +190,22 @@ __device__ __forceinline__ void for_products(const float *__restrict__ nA, const
 // (2.6e5 products 35.3 -> 34.4 us, 1.6e7 84.1 -> 81.7).
 template <int PASS>
 __global__ __launch_bounds__(TAU_NTH) void k_tau_hist(const float *__restrict__ nA, const float *__restrict__ nBt, int nbM,
-                                                      int nbK, int nbN, unsigned long long total, unsigned long long want0,
+                                                      int nbK, int nbN, TauGrid grid, unsigned long long total, unsigned long long want0,
                                                       TauWorkspace *__restrict__ ws, TauState *__restrict__ host_out,
                                                       unsigned long long *__restrict__ host_seq, unsigned long long seq) {
     constexpr int BITS = PASS == 2 ? 10 : 11, SHIFT = PASS == 0 ? 21 : (PASS == 1 ? 10 : 0);
     constexpr int NB = 1 << BITS, COPIES = 4, PER = NB / TAU_NTH;
-    __shared__ unsigned int lh[NB * COPIES];
+    __shared__ __attribute__((aligned(16))) unsigned int lh[NB * COPIES];
     __shared__ unsigned long long s_sum[TAU_NW];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int b = threadIdx.x; b < NB * COPIES; b += TAU_NTH) lh[b] = 0;
-    __syncthreads();
+    Products<TAU_JB_COUNT> products(nA, nBt, nbM, nbK, nbN, grid);
     TauState prev = {};
     if (PASS) prev = ws->st;
+    for (int b = threadIdx.x; b < NB * COPIES / 4; b += TAU_NTH) reinterpret_cast<uint4 *>(lh)[b] = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
     const uint32_t prefix = prev.prefix;
     const bool packed = total >> 32 == 0;                         // no count leaves 32 bits: two bins a word
-    for_products<TAU_JB_COUNT>(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
+    products.each([&](float p, bool live) {
         const bool pos = live && p > 0.0f;                        // NaN counts as 0
         const uint32_t key = __builtin_bit_cast(uint32_t, p);
         bool in = pos;
@@ -169,12 +262,7 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_hist(const float *__restrict__ 
         for (int r = 0; r < TAU_COPIES; r++) h[e] += part[e][r];
         mine += h[e];
     }
-    unsigned long long incl = mine;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const unsigned long long o = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += o;
-    }
+    const unsigned long long incl = wave_scan(mine);
     if (lane == 63) s_sum[wave] = incl;
     // The host goes on when it sees the last pass's result, on another stream if it likes: by then nothing of this
     // launch is still on its way to the workspace (and the state in it, which no launch after this reads, stays as it is)
@@ -240,11 +328,19 @@ __device__ __forceinline__ void store_tune(TauWorkspace *ws, const TauTune &t) {
     for (unsigned i = 0; i < sizeof(TauTune) / 8; i++) agent_store(reinterpret_cast<unsigned long long *>(&ws->tune) + i, words.w[i]);
 }
 
+// (double)p >= thr over fp32 p is p >= the smallest fp32 value that is not below thr.  (Mean and thresholds are
+// negative where uploaded norm maps hold negative values.)
+__device__ __forceinline__ float fp32_threshold(double thr) {
+    const float f = (float)thr;
+    if (!((double)f < thr)) return f;
+    return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, f) + (f < 0.0f ? -1 : 1));
+}
+
 // The two numbers that a round of the bisection starts from (tool.cu:448-463), and with `tune` its
 // first round: products with (double)p >= thr and the double sum of all products.  Sums of a
 // workgroup and of the whole are added in a fixed order: the same norm maps give the same sum.
 __global__ __launch_bounds__(TAU_NTH) void k_tau_count(const float *__restrict__ nA, const float *__restrict__ nBt, int nbM,
-                                                       int nbK, int nbN, double thr, unsigned long long total, int tune,
+                                                       int nbK, int nbN, TauGrid grid, double thr, unsigned long long total, int tune,
                                                        double expected, double tol, int max_rounds, unsigned int call, int last,
                                                        TauWorkspace *__restrict__ ws, TauCounts *__restrict__ host_out,
                                                        TauResult *__restrict__ host_tune, unsigned long long *__restrict__ host_seq,
@@ -252,14 +348,16 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_count(const float *__restrict__
     __shared__ unsigned long long s_cnt[TAU_NW];
     __shared__ double s_sum[TAU_NW];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    Products<TAU_JB_COUNT> products(nA, nBt, nbM, nbK, nbN, grid);
+    const float thr32 = fp32_threshold(thr);
     unsigned long long cnt = 0;
     double sum = 0.0;
-    for_products<TAU_JB_COUNT>(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
-        cnt += __builtin_popcountll(__ballot(live && (double)p >= thr));
+    products.each([&](float p, bool live) {
+        cnt += __builtin_popcountll(__ballot(live && p >= thr32));
         sum += live ? (double)p : 0.0;
     });
     auto block_sum = [&]() {                                      // of sum and the waves' cnt, in thread 0
-        for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off, 64);
+        sum = wave_sum(sum);
         if (lane == 0) { s_cnt[wave] = cnt; s_sum[wave] = sum; }
         __syncthreads();
         cnt = 0;
@@ -275,7 +373,7 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_count(const float *__restrict__
     const bool have = threadIdx.x < gridDim.x;                    // gridDim.x <= TAU_MAXB <= TAU_NTH
     cnt = have ? agent_load(&ws->part[threadIdx.x][0]) : 0ull;
     sum = have ? __builtin_bit_cast(double, agent_load(&ws->part[threadIdx.x][1])) : 0.0;
-    for (int off = 32; off > 0; off >>= 1) cnt += __shfl_down(cnt, off, 64);
+    cnt = wave_sum(cnt);
     block_sum();
     if (threadIdx.x != 0) return;
     TauCounts tc;
@@ -296,24 +394,12 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_count(const float *__restrict__
 // thresholds within some 5e4 rounds of any target, so no kernel runs longer whatever the caller's limit.)
 __device__ __forceinline__ bool bisect_step(TauTune &t, bool above) {
     const TauTune was = t;
-    if (above) {
-        if (t.up == t.norm) t.up *= 2;
-        t.down = t.norm;
-        t.norm = (t.norm + t.up) / 2;
-    } else {
-        t.up = t.norm;
-        t.norm = (t.norm + t.down) / 2;
-    }
+    const double up = was.up == was.norm ? was.up * 2 : was.up;
+    t.norm = (was.norm + (above ? up : was.down)) / 2;
+    t.up = above ? up : was.norm;
+    t.down = above ? was.norm : was.down;
     const auto same = [](double a, double b) { return __builtin_bit_cast(unsigned long long, a) == __builtin_bit_cast(unsigned long long, b); };
     return !(same(t.norm, was.norm) && same(t.up, was.up) && same(t.down, was.down));
-}
-
-// (double)p >= thr over fp32 p is p >= the smallest fp32 value that is not below thr.  (Mean and thresholds are
-// negative where uploaded norm maps hold negative values.)
-__device__ __forceinline__ float fp32_threshold(double thr) {
-    const float f = (float)thr;
-    if (!((double)f < thr)) return f;
-    return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, f) + (f < 0.0f ? -1 : 1));
 }
 
 // What a lane without a product holds: no threshold keeps it.
@@ -330,40 +416,44 @@ constexpr float NO_PRODUCT = __builtin_nanf("");
 // thresholds, and a wait for the stream -> this (rounds 9 | 20): 64000 products 40 | 60 -> 32 | 42, 2.6e5 41 | 63 -> 32 | 43,
 // 2.0e6 57 | 100 -> 40 | 56, 1.7e7 (10 rounds) 165 | 252 -> 71 | 113.
 __global__ __launch_bounds__(TAU_NTH) void k_tau_tree(const float *__restrict__ nA, const float *__restrict__ nBt, int nbM,
-                                                      int nbK, int nbN, unsigned long long total, double expected, double tol,
+                                                      int nbK, int nbN, TauGrid grid, unsigned long long total, double expected, double tol,
                                                       int max_rounds, unsigned int call, int last, TauWorkspace *__restrict__ ws,
                                                       TauResult *__restrict__ host_tune, unsigned long long *__restrict__ host_seq,
                                                       unsigned long long seq) {
     // a launch behind the one that ended the bisection has nothing to do, and by now the workspace may be another
-    // call's, on another stream: what tells is one word
-    const unsigned long long state = agent_load(reinterpret_cast<const unsigned long long *>(&ws->tune.done));
-    if ((unsigned int)state != 0u || (unsigned int)(state >> 32) != call) return;
+    // call's, on another stream: what tells is one word, read with the others, which are used only if it says so
+    TauTune start;
+    {
+        struct Words {
+            unsigned long long w[sizeof(TauTune) / 8];
+        } words;
+#pragma unroll
+        for (unsigned i = 0; i < sizeof(TauTune) / 8; i++) words.w[i] = agent_load(reinterpret_cast<const unsigned long long *>(&ws->tune) + i);
+        start = __builtin_bit_cast(TauTune, words);
+    }
+    if (start.done != 0 || start.call != call) return;
     constexpr int COPIES = 4;
     __shared__ float s_heap[TREE_LEAVES];
     __shared__ float s_sorted[TREE_LEAVES];
     __shared__ unsigned int s_leaf[TREE_LEAVES * COPIES];
     __shared__ unsigned long long s_kept[TREE_LEAVES];
     __shared__ unsigned long long s_sum[TAU_NW];
+    __shared__ uint16_t s_next[TREE_LEAVES];
     __shared__ int s_unsorted;
+    Products<TAU_JB_TREE> products(nA, nBt, nbM, nbK, nbN, grid);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // thread n: node n and its rank among the thresholds, 1 to TREE_LEAVES - 1
     static_assert(TREE_LEAVES == TAU_NTH, "a thread per node");
     const int n = threadIdx.x;
-    const TauTune start = ws->tune;
-    float own;
-    {
-        TauTune t = start;
-        for (int bit = 30 - __builtin_clz(n ? n : 1); bit >= 0; bit--) bisect_step(t, (n >> bit) & 1);
-        own = fp32_threshold(t.norm);
-    }
+    TauTune at_node = start;
+    for (int bit = 30 - __builtin_clz(n ? n : 1); bit >= 0; bit--) bisect_step(at_node, (n >> bit) & 1);
+    const float own = n ? fp32_threshold(at_node.norm) : -__builtin_inff();
     const int depth = 31 - __builtin_clz(n ? n : 1);
     int rank = n ? (2 * (n - (1 << depth)) + 1) << (TREE_ROUNDS - 1 - depth) : 0;
-    if (n == 0) {
-        own = -__builtin_inff();
-        s_unsorted = 0;
-    }
+    if (n == 0) s_unsorted = 0;
     s_sorted[rank] = own;
+    s_heap[n] = own;
 #pragma unroll
     for (int c = 0; c < COPIES; c++) s_leaf[n * COPIES + c] = 0;
     __syncthreads();
@@ -377,14 +467,15 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_tree(const float *__restrict__ 
             const float o = s_sorted[(2 * (m - (1 << at)) + 1) << (TREE_ROUNDS - 1 - at)];
             r += nan ? (o == o || m <= n) : (o < own || (o == own && m <= n));
         }
+        const int place = rank;
         if (n) rank = r;
         __syncthreads();
         s_sorted[rank] = own;
         __syncthreads();
+        if (n) s_heap[n] = s_sorted[place];
+        __syncthreads();
     }
-    s_heap[n] = n ? s_sorted[(2 * (n - (1 << depth)) + 1) << (TREE_ROUNDS - 1 - depth)] : 0.0f;
-    __syncthreads();
-    for_products<TAU_JB_TREE>(nA, nBt, nbM, nbK, nbN, [&](float p, bool live) {
+    products.each([&](float p, bool live) {
         int at = 1;
 #pragma unroll
         for (int level = 0; level < TREE_ROUNDS; level++) at = 2 * at + (p >= s_heap[at] ? 1 : 0);
@@ -407,35 +498,30 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_tree(const float *__restrict__ 
         if (part[r]) agent_store(&ws->leaf[r][TREE_LEAVES - 1 - n], 0ull);
         incl += part[r];
     }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const unsigned long long o = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += o;
-    }
+    incl = wave_scan(incl);
     if (lane == 63) s_sum[wave] = incl;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // (the leaves are zero again before the result is published)
     __syncthreads();
     for (int w = 0; w < wave; w++) incl += s_sum[w];
     s_kept[TREE_LEAVES - 1 - n] = incl;
     __syncthreads();
-    const unsigned long long kept = n ? s_kept[rank] : 0ull;
-    __syncthreads();
-    s_kept[n] = kept;                                             // now by node
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    TauTune t = start;
-    int node = 1;
-    for (int level = 0; level < TREE_ROUNDS && !t.done; level++) {
-        t.rate = (double)((float)s_kept[node] / (float)total);
-        if (fabs(t.rate - expected) < tol) {
-            t.done = 1;
-            break;
-        }
-        const bool above = t.rate > expected;
+    // every thread takes its node's decision; the path from the root then is a look-up per round, and the thread of the node where it
+    // ends has the result (one thread that took the decisions in turn: 2 us)
+    TauTune t = at_node;
+    t.rate = (double)((float)s_kept[rank] / (float)total);
+    t.rounds = start.rounds + depth;
+    t.done = fabs(t.rate - expected) < tol;
+    const bool above = t.rate > expected;
+    if (!t.done) {
         const bool moved = bisect_step(t, above);
-        node = 2 * node + (above ? 1 : 0);
-        if (++t.rounds >= max_rounds || !moved) t.done = 1;
+        t.done = ++t.rounds >= max_rounds || !moved;
     }
+    s_next[n] = (uint16_t)(t.done || depth == TREE_ROUNDS - 1 ? n : 2 * n + (above ? 1 : 0));
+    __syncthreads();
+    int node = 1;
+#pragma unroll
+    for (int level = 0; level < TREE_ROUNDS - 1; level++) node = s_next[node];
+    if (n != node) return;
     store_tune(ws, t);
     const TauResult res = {t.norm, t.rate, t.done};
     if (t.done || last) publish_result(host_tune, res, host_seq, seq);
@@ -615,6 +701,12 @@ static int64_t tau_products(int64_t nbM, int64_t nbK, int64_t nbN) { return nbM 
 
 bool tau_tune_small(int64_t nbM, int64_t nbK, int64_t nbN) { return tau_products(nbM, nbK, nbN) <= TAU_SMALL_MAX; }
 
+static TauGrid tau_steps(int64_t nbM, int64_t nbK, int64_t nbN, int jb) {
+    const uint64_t kb = (uint64_t)(nbK + 63) / 64, groups = (uint64_t)(nbN + jb - 1) / jb, rows = (uint64_t)nbM * groups;
+    const bool short_ = rows * kb * kb < 0xffffffffull && rows * groups < 0xffffffffull;
+    return {(uint32_t)kb, (uint32_t)groups, short_ ? 0xffffffffu / (uint32_t)kb : 0u, short_ ? 0xffffffffu / (uint32_t)groups : 0u};
+}
+
 static unsigned tau_grid(int64_t nbM, int64_t nbK, int64_t nbN, int jb = TAU_JB_COUNT) {
     const int64_t units = nbM * ((nbN + jb - 1) / jb) * ((nbK + 63) / 64);
     const int64_t blocks = (units + TAU_NW - 1) / TAU_NW;
@@ -644,16 +736,17 @@ hipError_t launch_tau_select(const float *nA, const float *nBt, int64_t nbM, int
     }
     const unsigned grid = tau_count_grid(nbM, nbK, nbN, TAU_JB_COUNT);
     const unsigned long long total = (unsigned long long)n;
-    k_tau_hist<0><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out, host_seq, seq);
-    k_tau_hist<1><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out, host_seq, seq);
-    k_tau_hist<2><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, want, ws, host_out, host_seq, seq);
+    const TauGrid steps = tau_steps(nbM, nbK, nbN, TAU_JB_COUNT);
+    k_tau_hist<0><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, steps, total, want, ws, host_out, host_seq, seq);
+    k_tau_hist<1><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, steps, total, want, ws, host_out, host_seq, seq);
+    k_tau_hist<2><<<grid, TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, steps, total, want, ws, host_out, host_seq, seq);
     return hipGetLastError();
 }
 
 hipError_t launch_tau_count(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double thr,
                             void *workspace, TauCounts *host_out, unsigned long long *host_seq, unsigned long long seq, hipStream_t s) {
     TauWorkspace *ws = (TauWorkspace *)workspace;
-    k_tau_count<<<tau_grid(nbM, nbK, nbN), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, thr,
+    k_tau_count<<<tau_grid(nbM, nbK, nbN), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, tau_steps(nbM, nbK, nbN, TAU_JB_COUNT), thr,
                                                        (unsigned long long)nbM * nbK * nbN, 0, 0.0, 0.0, 0, 0u, 0, ws, host_out, nullptr,
                                                        host_seq, seq);
     return hipGetLastError();
@@ -675,10 +768,10 @@ hipError_t launch_tau_tune(const float *nA, const float *nBt, int64_t nbM, int64
     TauWorkspace *ws = (TauWorkspace *)workspace;
     const unsigned long long total = (unsigned long long)nbM * nbK * nbN;
     if (first)
-        k_tau_count<<<tau_grid(nbM, nbK, nbN), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, 0.0, total, 1, expected, tol,
+        k_tau_count<<<tau_grid(nbM, nbK, nbN), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, tau_steps(nbM, nbK, nbN, TAU_JB_COUNT), 0.0, total, 1, expected, tol,
                                                            max_rounds, call, passes == 0, ws, nullptr, host_out, host_seq, seq);
     for (int p = 0; p < passes; p++)
-        k_tau_tree<<<tau_count_grid(nbM, nbK, nbN, TAU_JB_TREE), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, total, expected, tol,
+        k_tau_tree<<<tau_count_grid(nbM, nbK, nbN, TAU_JB_TREE), TAU_NTH, 0, s>>>(nA, nBt, (int)nbM, (int)nbK, (int)nbN, tau_steps(nbM, nbK, nbN, TAU_JB_TREE), total, expected, tol,
                                                                              max_rounds, call, p == passes - 1, ws, host_out, host_seq, seq);
     return hipGetLastError();
 }

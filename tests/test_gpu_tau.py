@@ -271,3 +271,29 @@ def test_bisection_of_more_products_than_workgroups_count(orc, ctx):
     for expected in (0.5, 0.003):
         got, want = ctx.tune_bisect(expected, 1e-4, 20), orc.tune_bisect(rows, np.ones((1, 1), np.float32), expected, 1e-4, 20)
         assert np.float32(got[0]) == np.float32(want[0]) and got[1] == want[1]
+
+
+@pytest.mark.parametrize("shape", [(65535, 1, 4096), (65535, 1, 4112), (3, 200, 33), (2, 64 * 130 + 1, 5)])
+def test_steps_by_reciprocals_and_by_divisions_visit_every_product(ctx, shape):
+    """Where a step's number times the divisor leaves 32 bits (65535 x 257 groups of columns) the steps are divided for; the shapes beside
+    it go by reciprocals.  Norms are powers of two, so products are too, and their distribution is the sum of the exponents'."""
+    nbM, nbK, nbN = shape
+    rng = np.random.default_rng(nbM + nbN)
+    ea, eb = rng.integers(0, 8, (nbM, nbK)), rng.integers(0, 8, (nbK, nbN))
+    ctx.set_normmaps((2.0 ** -ea).astype(np.float32), (2.0 ** -eb).astype(np.float32), 32)
+    having = np.zeros(15, dtype=np.int64)                        # products of 2^-e
+    for x in range(8):
+        for y in range(8):
+            having[x + y] += int(((ea == x).sum(axis=0) * (eb == y).sum(axis=1)).sum())
+    upto = np.cumsum(having)
+    assert upto[-1] == nbM * nbK * nbN
+    for e in (0, 3, 7, 14):
+        cnt, sm = ctx.count_kept(2.0 ** -e)
+        assert cnt == upto[e]
+        assert abs(sm - (having * 2.0 ** -np.arange(15.0)).sum()) <= 1e-9 * sm
+    for ratio in (0.01, 0.3, 0.9):
+        e = int(np.searchsorted(upto, np.ceil(ratio * upto[-1])))
+        tau, achieved = ctx.tau_for_ratio(ratio)
+        assert tau == 2.0 ** -e and achieved == upto[e] / upto[-1]
+    tau, achieved = ctx.tune_bisect(0.5, 0.2, 20)
+    assert achieved == np.float32(upto[int(np.floor(-np.log2(tau)))]) / np.float32(upto[-1])
