@@ -388,14 +388,18 @@ __global__ __launch_bounds__(64 * NWV) void k_normmap_pair(const void *__restric
                                                nullptr, tau_skip, keep_copy, blockIdx.x - n_b, s_pack, s_chunk, s_skip, s_seen);
 }
 
-// ---- small inputs (at most KEEP_INPUT_MAX bytes a launch).  There is little to stream: a workgroup's waves are almost alone on their
-// SIMDs, issue an instruction in some five clocks, and the pass takes as long as its chain of instructions.  So everything is
+// ---- the same strip in fewer instructions, with one 8-row group per lane and one phase.  In a small launch (at most KEEP_INPUT_MAX bytes
+// of input) there is little to stream: a workgroup's waves are almost alone on their SIMDs, issue an instruction in some five clocks, and the pass takes as long as its chain of instructions.  So everything is
 // addressed by 32-bit offsets into buffers that begin at the strip -- rows by the scalar offset, a lane beyond the last column or a tile
 // beyond the last one by an offset that the buffer does not hold, without a branch --, the strip's place comes from a reciprocal
 // instead of a 64-bit division, and a wave reduces all its tiles' norms together, by lane exchanges that are not LDS operations.
 // Both operands in one launch, alone, inputs from HBM, the streaming kernel -> this: 256^3 3.83 -> 3.01 us (of which 1.55 are an empty
 // launch), 1024^3 at tile 64 4.48 -> 4.14, 1056 x 1568 x 1312 8.2 -> 7.4, fp16 1024 x 2048 x 1024 5.93 -> 4.82, 2048^3 at tile 32 10.3 -> 8.1,
 // 512^3 at tile 128 3.50 -> 3.39 (one wave adds a lane's 32 chunks in their order).
+// Large inputs are bound by the HBM, and take it where it is not slower (launch_normmap); passes alone: tile 32 5024 x 4128 fp32 22.2 -> 21.0 us,
+// tau-aware 23.0 -> 20.6, fp16 5024^2 20.5 -> 19.3, tau-aware 17.8 -> 16.2, 12032^2 155 -> 153.5; fp32 tile 64 4096^2 A = B 25.9 -> 24.2, both operands in
+// one launch 33.6 -> 32.4, 8192^2 61.7 -> 61.0.  Reads alone reach 6.8 to 7.2 TB/s there; as soon as one workgroup in sixteen writes its
+// tile the whole comes to 5.5 to 5.8, in whatever order or policy (4 GiB read, 1/16, 3/16, all of the copies written: 624 -> 770, 870, 1090 us).
 //
 // Sum over the 64 lanes, in every lane: the same additions as butterfly64.  (Behind the steps of 1 and 2 all lanes of a quad hold one sum, so
 // that a mirrored quad is the neighbour; likewise for 8.)
@@ -414,12 +418,12 @@ __device__ __forceinline__ float butterfly64_dpp(float v) {
     return __builtin_bit_cast(float, (uint32_t)r32[0]) + __builtin_bit_cast(float, (uint32_t)r32[1]);
 }
 
-// A strip's place: row and column of strips, `rec` = strip_reciprocal(nstrip).  Exact while strips * nstrip < 2^32: an input of KEEP_INPUT_MAX bytes
-// is at most 2^14 strips of 2 KiB or more.
-inline uint32_t strip_reciprocal(uint32_t nstrip) { return 0xffffffffu / nstrip; }
+// A strip's place: row and column of strips by a reciprocal, exact while strips * nstrip <= 2^32; else (0) by a division.
+inline uint32_t strip_reciprocal(uint32_t strips, uint32_t nstrip) { return (uint64_t)strips * nstrip < 0xffffffffull ? 0xffffffffu / nstrip : 0u; }
 
-template <int B, int ROLE, int SW, bool IN16, int NWV>
-__device__ __forceinline__ void normmap_strip_small(const void *X, uint32_t cols, uint32_t nbr, uint32_t nbc, uint32_t nstrip, uint32_t rec,
+// KEEP: the input's lines stay in the caches (keep_input).
+template <int B, int ROLE, int SW, bool IN16, int NWV, bool KEEP>
+__device__ __forceinline__ void normmap_strip_lean(const void *X, uint32_t cols, uint32_t nbr, uint32_t nbc, uint32_t nstrip, uint32_t rec,
                                                     void *packed, float *nm, float *nmT, void *packed2, float *nm2, const float *rowmax,
                                                     float tau_skip, bool keep_copy, uint32_t strip, unsigned char *s_pack, float *s_chunk,
                                                     int *s_skip, int *s_seen) {
@@ -430,23 +434,23 @@ __device__ __forceinline__ void normmap_strip_small(const void *X, uint32_t cols
     static_assert(B == 8 * NWV * GPW, "a lane has one 8-row group");
     constexpr int VPT = B * B / 8, STEPS = VPT / 64;   // 16-byte vectors per tile; chunks per lane of its norm
     constexpr int NT = TPP > NWV ? TPP / NWV : 1;      // tiles per wave of the norms
-    constexpr uint32_t NOWHERE = 0x80000000u;          // an offset no buffer here holds
+    constexpr uint32_t NOWHERE = 0x80000000u, TB = B * B * 2;          // an offset no output buffer here holds; bytes of a tile
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t I = __umulhi(strip + 1u, rec), sc = strip - I * nstrip, col0 = sc * SW, J0 = sc * TPP;
-    const uint32_t ld = cols * E;                      // bytes per row
+    const uint32_t I = rec ? __umulhi(strip + 1u, rec) : strip / nstrip, sc = strip - I * nstrip, col0 = sc * SW, J0 = sc * TPP;
+    const uint32_t ld = cols * E;                      // bytes per row (of which B are less than 4 GiB)
     const int cl = EPL * (lane % LPR);                 // first column of this lane inside the strip
     const int t = cl / B, cin = cl % B;                // tile of the strip, column inside the tile
     const int g = wave * GPW + lane / LPR;             // 8-row group of this lane
-    const __amdgpu_buffer_rsrc_t in = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char *>(static_cast<const unsigned char *>(X)) + (size_t)I * B * ld + col0 * E, 0,
+    const __amdgpu_buffer_rsrc_t in = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char *>(static_cast<const unsigned char *>(X)) + (uint64_t)I * B * ld + (uint64_t)col0 * E, 0,
                                                                         (int)((B - 1) * ld + (cols - col0) * E), 0x00020000);
     u32x4n x[8];
     {
-        const uint32_t voff = col0 + cl < cols ? (uint32_t)(lane / LPR) * 8u * ld + (uint32_t)cl * E : NOWHERE;
+        const uint32_t voff = col0 + cl < cols ? (uint32_t)(lane / LPR) * 8u * ld + (uint32_t)cl * E : 0xffffff00u;
         uint32_t soff = (uint32_t)(wave * GPW * 8) * ld;
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            x[j] = __builtin_bit_cast(u32x4n, __builtin_amdgcn_raw_buffer_load_b128(in, (int)voff, (int)soff, 0));
+            x[j] = __builtin_bit_cast(u32x4n, __builtin_amdgcn_raw_buffer_load_b128(in, (int)voff, (int)soff, KEEP ? 0 : 2));
             soff += ld;
         }
     }
@@ -533,8 +537,8 @@ __device__ __forceinline__ void normmap_strip_small(const void *X, uint32_t cols
             nv = sqrtf(nv);
             const uint32_t Jt = J0 + t0 + lane;
             if (lane < NT && Jt < nbc) {
-                nmo[I * nbc + Jt] = nv;
-                if (as_b) nmTo[Jt * nbr + I] = nv;
+                nmo[(uint64_t)I * nbc + Jt] = nv;
+                if (as_b) nmTo[(uint64_t)Jt * nbr + I] = nv;
                 if (prune) s_skip[t0 + lane] = rowmax != nullptr ? nv * rowmax[Jt] < tau_skip : nv == 0.0f;
             }
         };
@@ -546,9 +550,9 @@ __device__ __forceinline__ void normmap_strip_small(const void *X, uint32_t cols
         int any = 0;
 #pragma unroll
         for (int w = 0; w < NWV; w++) any |= s_seen[w];
-        const uint32_t step = as_b ? nbr * (uint32_t)(B * B * 2) : (uint32_t)(B * B * 2);      // bytes from a tile to the next of the strip
-        const uint32_t first = as_b ? (J0 * nbr + I) * (uint32_t)(B * B * 2) : (I * nbc + J0) * (uint32_t)(B * B * 2);
-        const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(static_cast<unsigned char *>(pk) + first, 0, 0x7fffffff, 0x00020000);
+        const uint32_t step = as_b ? nbr * TB : TB;    // bytes from a tile to the next of the strip (all of them: less than 2 GiB)
+        const uint64_t first = as_b ? (uint64_t)J0 * nbr + I : (uint64_t)I * nbc + J0;
+        const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(static_cast<unsigned char *>(pk) + first * TB, 0, 0x7fffffff, 0x00020000);
         auto copy = [&](auto cached) {
 #pragma unroll
             for (int i = 0; i < TPP * VPT / (64 * NWV); i++) {
@@ -571,8 +575,8 @@ __device__ __forceinline__ void normmap_strip_small(const void *X, uint32_t cols
     }
 }
 
-template <int B, int ROLE, int SW, bool IN16, int NWV>
-__global__ __launch_bounds__(64 * NWV) void k_normmap_small(const void *X, uint32_t cols, uint32_t nbr, uint32_t nbc, uint32_t nstrip,
+template <int B, int ROLE, int SW, bool IN16, int NWV, bool KEEP>
+__global__ __launch_bounds__(64 * NWV) void k_normmap_lean(const void *X, uint32_t cols, uint32_t nbr, uint32_t nbc, uint32_t nstrip,
                                                             uint32_t rec, void *packed, float *nm, float *nmT, void *packed2, float *nm2,
                                                             const float *rowmax, float tau_skip, bool keep_copy) {
     using L = NormCfg<B, SW, 1>;
@@ -580,12 +584,12 @@ __global__ __launch_bounds__(64 * NWV) void k_normmap_small(const void *X, uint3
     __shared__ float s_chunk[L::TPP * L::CH];
     __shared__ int s_skip[L::TPP], s_seen[NWV];
     asm volatile("" : "+s"(X), "+s"(packed), "+s"(nm), "+s"(nmT), "+s"(tau_skip));        // (all arguments at once)
-    normmap_strip_small<B, ROLE, SW, IN16, NWV>(X, cols, nbr, nbc, nstrip, rec, packed, nm, nmT, packed2, nm2, rowmax, tau_skip, keep_copy,
+    normmap_strip_lean<B, ROLE, SW, IN16, NWV, KEEP>(X, cols, nbr, nbc, nstrip, rec, packed, nm, nmT, packed2, nm2, rowmax, tau_skip, keep_copy,
                                                 blockIdx.x, s_pack, s_chunk, s_skip, s_seen);
 }
 
-template <int B, int SW, bool IN16, int NWV>
-__global__ __launch_bounds__(64 * NWV) void k_normmap_pair_small(const void *A, const void *Bm, uint32_t nbM, uint32_t nbK, uint32_t nbN,
+template <int B, int SW, bool IN16, int NWV, bool KEEP>
+__global__ __launch_bounds__(64 * NWV) void k_normmap_pair_lean(const void *A, const void *Bm, uint32_t nbM, uint32_t nbK, uint32_t nbN,
                                                                  uint32_t n_b, uint32_t strips_a, uint32_t rec_a, uint32_t strips_b,
                                                                  uint32_t rec_b, void *packedA, void *packedB, float *nmA, float *nmB,
                                                                  float *nmBt, float tau_skip, bool keep_copy) {
@@ -595,10 +599,10 @@ __global__ __launch_bounds__(64 * NWV) void k_normmap_pair_small(const void *A, 
     __shared__ int s_skip[L::TPP], s_seen[NWV];
     asm volatile("" : "+s"(A), "+s"(Bm), "+s"(packedA), "+s"(packedB), "+s"(nmA), "+s"(nmB), "+s"(nmBt), "+s"(tau_skip));
     if (blockIdx.x < n_b)
-        normmap_strip_small<B, 1, SW, IN16, NWV>(Bm, nbN * B, nbK, nbN, strips_b, rec_b, packedB, nmB, nmBt, nullptr, nullptr, nullptr, tau_skip,
+        normmap_strip_lean<B, 1, SW, IN16, NWV, KEEP>(Bm, nbN * B, nbK, nbN, strips_b, rec_b, packedB, nmB, nmBt, nullptr, nullptr, nullptr, tau_skip,
                                                  keep_copy, blockIdx.x, s_pack, s_chunk, s_skip, s_seen);
     else
-        normmap_strip_small<B, 0, SW, IN16, NWV>(A, nbK * B, nbM, nbK, strips_a, rec_a, packedA, nmA, nullptr, nullptr, nullptr, nullptr, tau_skip,
+        normmap_strip_lean<B, 0, SW, IN16, NWV, KEEP>(A, nbK * B, nbM, nbK, strips_a, rec_a, packedA, nmA, nullptr, nullptr, nullptr, nullptr, tau_skip,
                                                  keep_copy, blockIdx.x - n_b, s_pack, s_chunk, s_skip, s_seen);
 }
 
@@ -714,37 +718,45 @@ static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int 
     k_normmap<T, ROLE, SW, IN16, PH, NWV><<<strips(SW), 64 * NWV, 0, s>>>(X, cols, cols, nbr, nbc, (cols + SW - 1) / SW, (uint4 *)packed, \
                                                                           nm, nmT, (uint4 *)packed2, nm2, rowmax, tau_skip,        \
                                                                           keep_copy(rows * cols * 2))
-// (the shapes that inputs of up to KEEP_INPUT_MAX take, but for a few fp16 ones)
-#define SPAMM_NORMMAP_KEEP(T, SW, NWV)                                                                                             \
-    do {                                                                                                                           \
-        const uint32_t ns = (uint32_t)((cols + SW - 1) / SW);                                                                      \
-        if (keep)                                                                                                                  \
-            k_normmap_small<T, ROLE, SW, IN16, NWV><<<strips(SW), 64 * NWV, 0, s>>>(X, (uint32_t)cols, (uint32_t)nbr, (uint32_t)nbc, ns, \
-                                                                                    strip_reciprocal(ns), packed, nm, nmT, packed2, nm2, \
-                                                                                    rowmax, tau_skip, keep_copy(rows * cols * 2)); \
-        else SPAMM_NORMMAP(T, SW, 1, NWV);                                                                                         \
+#define SPAMM_LEAN_(T, SW, NWV, KEEP)                                                                                                     \
+    do {                                                                                                                                  \
+        const uint32_t ns = (uint32_t)((cols + SW - 1) / SW);                                                                             \
+        k_normmap_lean<T, ROLE, SW, IN16, NWV, KEEP><<<strips(SW), 64 * NWV, 0, s>>>(                                                     \
+            X, (uint32_t)cols, (uint32_t)nbr, (uint32_t)nbc, ns, strip_reciprocal(strips(SW), ns), packed, nm, nmT, packed2, nm2, rowmax, \
+            tau_skip, keep_copy(rows * cols * 2));                                                                                        \
+    } while (0)
+#define SPAMM_LEAN(T, SW, NWV)                    \
+    do {                                          \
+        if (keep) SPAMM_LEAN_(T, SW, NWV, true);  \
+        else SPAMM_LEAN_(T, SW, NWV, false);      \
+    } while (0)
+#define SPAMM_LEAN_IF_KEPT(T, SW, NWV)            \
+    do {                                          \
+        if (keep) SPAMM_LEAN_(T, SW, NWV, true);  \
+        else SPAMM_NORMMAP(T, SW, 1, NWV);        \
     } while (0)
     // strip widths and waves: one 8-row group per lane, at most ~42 KiB of LDS and so three workgroups or more per CU.
     // fp16 input: 256 columns, two rows per load (512 in phases before: tile 64 1024^2, both passes, 6.2 -> 4.1 us, 4096^2
     // 28.4 -> 26.3, 16384^2 A = B 303 -> 291; tile 32 2048^2 8.0 -> 7.3, 8192^2 tau-aware 93 -> 87).
     switch (tile) {
         case 32:
-            if constexpr (IN16) SPAMM_NORMMAP_KEEP(32, 256, 2);
-            else SPAMM_NORMMAP_KEEP(32, 256, 4);
+            if constexpr (IN16) SPAMM_LEAN(32, 256, 2);
+            else SPAMM_LEAN(32, 256, 4);
             break;
         case 64:
             // fp32 input: strips of 128 columns where there are few (1024^2, both passes: 5.4 -> 4.4 us; 4096^2 36.1 ->
             // 36.7), of 256 by eight waves on middling grids (N = 8192: 0.066 / 0.058 -> 0.063 / 0.056 ms), by four waves,
-            // two groups per lane, on large ones (N = 16384: as fast or 1 % faster)
+            // two groups per lane, on large ones (N = 16384: as fast or 1 % faster; against the lean strip by eight waves both 2 to 4 % slower
+            // in plain passes of 16384^2, even at 12032^2, 2 % faster at 20032^2 and 5 % in tau-aware squares of a narrow band)
             // fp16 input, 3 to 4 strips of 256 columns per CU (of a whole chip), of which three run at once: strips of 512 in
             // two phases by eight waves are one turn instead of two.  256 -> 512, A and B pass alone, A = B with the fill of C
             // behind it: 4096^2 12.5 -> 11.1 us, 12.8 -> 11.6, 42.1 -> 39.1; 3840^2 11.2 -> 10.5, 11.1 -> 10.9, 39.7 -> 37.5;
             // 3648^2 10.5 -> 10.1, 10.3 -> 10.5, 38.4 -> 36.4; 3584^2 8.9 -> 9.1, 9.5 -> 9.9, 37.0 -> 35.8
             if constexpr (IN16) {
                 if (strips(256) > 768u && strips(256) <= 1024u) SPAMM_NORMMAP(64, 512, 2, 8);
-                else SPAMM_NORMMAP_KEEP(64, 256, 4);
-            } else if (strips(256) <= NARROW_STRIPS) SPAMM_NORMMAP_KEEP(64, 128, 4);
-            else if (strips(256) <= 8192u) SPAMM_NORMMAP(64, 256, 1, 8);
+                else SPAMM_LEAN_IF_KEPT(64, 256, 4);
+            } else if (strips(256) <= NARROW_STRIPS) SPAMM_LEAN(64, 128, 4);
+            else if (strips(256) <= 8192u) SPAMM_LEAN(64, 256, 8);
             else SPAMM_NORMMAP(64, 256, 1, 4);
             break;
         // tile 128: strips of one tile.  Only the fp32 B role of a large matrix keeps strips of two tiles in two phases by
@@ -752,19 +764,21 @@ static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int 
         case 128:
             if constexpr (IN16) {
                 if constexpr (ROLE == 2) return hipErrorInvalidValue;      // (two passes, or the pair, are faster)
-                else SPAMM_NORMMAP_KEEP(128, 128, 4);
+                else SPAMM_LEAN_IF_KEPT(128, 128, 4);
             } else {
                 if constexpr (ROLE == 1)
                     if (strips(256) > 6000u) {
                         SPAMM_NORMMAP(128, 256, 2, 4);
                         break;
                     }
-                SPAMM_NORMMAP_KEEP(128, 128, 8);
+                SPAMM_LEAN_IF_KEPT(128, 128, 8);
             }
             break;
         default: return hipErrorInvalidValue;
     }
-#undef SPAMM_NORMMAP_KEEP
+#undef SPAMM_LEAN_IF_KEPT
+#undef SPAMM_LEAN
+#undef SPAMM_LEAN_
 #undef SPAMM_NORMMAP
     return hipGetLastError();
 }
@@ -783,10 +797,13 @@ static void launch_pair(const void *A, const void *Bm, int64_t nbM, int64_t nbK,
     const int64_t a = nbM * nbK * B * B, b = nbK * nbN * B * B;
     const bool keep = keep_input((a + b) * (IN16 ? 2 : 4));
     const bool cached = keep_copy(2 * (a > b ? a : b));
-    if (keep)
-        k_normmap_pair_small<B, SW, IN16, NWV><<<n_a + n_b, 64 * NWV, 0, s>>>(
-            A, Bm, (uint32_t)nbM, (uint32_t)nbK, (uint32_t)nbN, n_b, (uint32_t)strips_a, strip_reciprocal((uint32_t)strips_a),
-            (uint32_t)strips_b, strip_reciprocal((uint32_t)strips_b), packedA, packedB, nmA, nmB, nmBt, tau_skip, cached);
+    auto lean = [&](auto kept) {
+        k_normmap_pair_lean<B, SW, IN16, NWV, decltype(kept)::value><<<n_a + n_b, 64 * NWV, 0, s>>>(
+            A, Bm, (uint32_t)nbM, (uint32_t)nbK, (uint32_t)nbN, n_b, (uint32_t)strips_a, strip_reciprocal(n_a, (uint32_t)strips_a),
+            (uint32_t)strips_b, strip_reciprocal(n_b, (uint32_t)strips_b), packedA, packedB, nmA, nmB, nmBt, tau_skip, cached);
+    };
+    if (keep) lean(std::true_type{});
+    else if constexpr (B == 32 || (B == 64 && !IN16)) lean(std::false_type{});          // (as launch_normmap)
     else
         k_normmap_pair<B, SW, IN16, PH, NWV><<<n_a + n_b, 64 * NWV, 0, s>>>(A, Bm, nbM, nbK, nbN, n_b, strips_a, strips_b, (uint4 *)packedA,
                                                                             (uint4 *)packedB, nmA, nmB, nmBt, tau_skip, cached);

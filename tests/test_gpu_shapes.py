@@ -450,3 +450,38 @@ def test_passes_over_small_inputs_end_strips_anywhere(orc, ctx, tile, half):
         ctx.multiply(A, A, tile, 0.5, a_eq_b=True)
         same(0, A)
         same(1, A)
+
+
+@pytest.mark.parametrize("tile,half,n", [(32, False, 2912), (32, True, 4128), (64, False, 2944), (64, False, 4160), (64, True, 4160)])
+def test_passes_over_inputs_beyond_the_cache_line(orc, ctx, tile, half, n):
+    """The same beyond 32 MiB an operand, where rows are streamed past the caches: ragged strips, each operand by itself, both in one
+    launch, A = B, and a tau-aware call beside a plain one."""
+    import torch
+    kind = torch.float16 if half else torch.float32
+    m = n + tile
+    tab = orc.decay_table("exp", m, 0.01)
+    A = torch.empty((m, n), dtype=torch.float32, device="cuda")
+    B = torch.empty((n, m), dtype=torch.float32, device="cuda")
+    ctx.fill_decay(A, tab, 1)
+    ctx.fill_decay(B, tab, 2)
+    A, B = A.to(kind), B.to(kind)
+
+    def same(role, X):
+        bits = X.half().cpu().numpy().view(np.uint16)
+        assert np.array_equal(ctx.get_fp16(role), bits)
+        assert np.array_equal(ctx.get_normmap(role).view(np.uint32), orc.normmap(bits, tile, role).view(np.uint32))
+
+    alone = ctx.normmap_f16 if half else ctx.normmap_f32
+    alone(1, B, tile)
+    alone(0, A, tile)
+    same(0, A)
+    same(1, B)
+    tau = ctx.tau_for_ratio(0.05)[0]
+    want = ctx.multiply(A, B, tile, tau)
+    same(0, A)
+    same(1, B)
+    assert torch.equal(ctx.multiply(A, B, tile, tau, prune=True), want)
+    X = A[:n].contiguous()
+    ctx.multiply(X, X, tile, tau, a_eq_b=True)
+    same(0, X)
+    same(1, X)
