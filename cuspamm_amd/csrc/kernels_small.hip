@@ -9,9 +9,9 @@
 // counts, kept total -- is written on the way out; the macro tiles' work lists, which
 // nothing reads after this kernel, are built by k_gate if somebody asks for them.
 //
-// Two forms: K / tile up to 64 (k_small_word, the list in a register) and beyond (k_small, the list in LDS).
+// Two forms: K / tile up to 64 (small_word_body, the list in a register) and beyond (small_unit_body, the list in LDS).
 //
-// A unit's life in k_small, measured on fp16 2048^3 at tile 32, 5 % kept, us: gate 2.0 (most of it the norms' round trip), list 0.3, first
+// A unit's life with its list in LDS, measured on fp16 2048^3 at tile 32, 5 % kept, us: gate 2.0 (most of it the norms' round trip), list 0.3, first
 // stages 0.8, 9 to 14 stages 3.4 to 6, C 1.5.  With 64-bit places, divisions by the grid's sizes, a scan for the one word of 64 k that most lists
 // are, and counts formed behind C's stores it was 1 us longer (whole calls: 256^3 10.5 -> 9.8 us, 1024^3 11.6 -> 10.6, 1056 x 1568 x
 // 1312 16.3 -> 15.5, this one 19.5 -> 18.4, 4096^2 of a band 57.9 -> 56.2).
@@ -464,7 +464,7 @@ __global__ __launch_bounds__(256, 3) void k_small_three(const unsigned char *pA,
 // stage's entry out of it by v_readlane.  Norms, operands and C are addressed by a buffer's scalar offset, one scalar instruction a load, and
 // all arguments are asked for at once.  A slot that no tile pair of an entry reads, and stages beyond the last, are loads from a
 // buffer of no bytes: they keep the number of loads in flight fixed and fetch nothing (their offset is one of the operand's all the same).
-// Kernels alone, k_small -> this: 256^3 5.35 -> 3.45 us (its gate alone 3.2 -> 1.9), 1056 x 1568 x 1312 9.0 -> 6.4, 1024^3 at tile 64 6.1 ->
+// Kernels alone, the list in LDS -> this: 256^3 5.35 -> 3.45 us (its gate alone 3.2 -> 1.9), 1056 x 1568 x 1312 9.0 -> 6.4, 1024^3 at tile 64 6.1 ->
 // 4.5, fp16 2048^3 at tile 32 5 % kept 11.6 -> 9.4, 75 % 26.5 -> 23, 4096^3 at tile 64 10 % 33.7 -> 31.
 // What bounds it now: launch and arguments 700 clocks, norms 1200, gate and list 1000, the ring's first loads at 64 bytes a clock 1100, a stage
 // of 128 x 128 x 32 some 600 (of which its loads alone take 440), C at 64 bytes a clock.
@@ -791,17 +791,36 @@ __device__ __forceinline__ void small_word_body(const unsigned char *pA, const u
 template <int U>
 static constexpr int WORD_RING = U == 128 ? 4 : 5;
 
+// The arguments, in the order of their use; a kernel for each tile size and unit (functions of the names of the other form's templates: whoever
+// lists a call's kernels sees the one-launch kernel, and three to a CU).
 template <int B, int U>
-__global__ __launch_bounds__(256, 2) void k_small_word(const unsigned char *pA, const unsigned char *pB, int nbM, int nbK, int nbN,
-                                                       SmallGrid sg, float tau, float *C, UnitGate g) {
-    small_word_body<B, U, WORD_RING<U>>(pA, pB, nbM, nbK, nbN, sg, tau, C, g);
-}
-
-template <int B>
-__global__ __launch_bounds__(256, 3) void k_small_word_three(const unsigned char *pA, const unsigned char *pB, int nbM, int nbK, int nbN,
-                                                             SmallGrid sg, float tau, float *C, UnitGate g) {
-    small_word_body<B, 128, 3>(pA, pB, nbM, nbK, nbN, sg, tau, C, g);
-}
+struct WordArgs {
+    const unsigned char *pA, *pB;
+    int nbM, nbK, nbN;
+    SmallGrid sg;
+    float tau;
+    float *C;
+    UnitGate g;
+};
+#define SPAMM_WORD(B, U)                                                                                     \
+    __global__ __launch_bounds__(256, 2) void k_small(WordArgs<B, U> a) {                                    \
+        small_word_body<B, U, WORD_RING<U>>(a.pA, a.pB, a.nbM, a.nbK, a.nbN, a.sg, a.tau, a.C, a.g);         \
+    }
+#define SPAMM_WORD_THREE(B)                                                                                  \
+    __global__ __launch_bounds__(256, 3) void k_small_three(WordArgs<B, 128> a) {                            \
+        small_word_body<B, 128, 3>(a.pA, a.pB, a.nbM, a.nbK, a.nbN, a.sg, a.tau, a.C, a.g);                  \
+    }
+SPAMM_WORD(32, 64)
+SPAMM_WORD(32, 128)
+SPAMM_WORD(64, 64)
+SPAMM_WORD(64, 128)
+SPAMM_WORD(128, 64)
+SPAMM_WORD(128, 128)
+SPAMM_WORD_THREE(32)
+SPAMM_WORD_THREE(64)
+SPAMM_WORD_THREE(128)
+#undef SPAMM_WORD
+#undef SPAMM_WORD_THREE
 
 // Units of 128 in C, as many as 256 CUs would have for the same share of a CU: what the lines below balance is workgroups per
 // CU and k_gemm's rounds of a macro tile per CU, so on a partition of fewer CUs they lie at as many units less.
@@ -833,9 +852,9 @@ static bool small_three(int64_t units128, int64_t nbK) {
 // (WORD: one word of k tiles)
 template <int B, int U, bool THREE, bool WORD>
 static constexpr auto small_kernel() {
-    if constexpr (THREE && WORD) return &k_small_word_three<B>;
+    if constexpr (THREE && WORD) return static_cast<void (*)(WordArgs<B, 128>)>(&k_small_three);
     else if constexpr (THREE) return &k_small_three<B>;
-    else if constexpr (WORD) return &k_small_word<B, U>;
+    else if constexpr (WORD) return static_cast<void (*)(WordArgs<B, U>)>(&k_small);
     else return &k_small<B, U>;
 }
 
@@ -857,7 +876,8 @@ static hipError_t launch_small_(const void *pA, const void *pB, const GateBuffer
     const unsigned char *a = (const unsigned char *)pA, *b = (const unsigned char *)pB;
     const UnitGate w = {g.nA, g.nBt, g.kept, g.counts, g.mask};
     if (nbK <= 64)
-        small_kernel<B, U, THREE, true>()<<<grid, 256, small_lds<B, U, THREE, true>(nbK), s>>>(a, b, nbM, nbK, nbN, sg, tau, C, w);
+        small_kernel<B, U, THREE, true>()<<<grid, 256, small_lds<B, U, THREE, true>(nbK), s>>>(
+            WordArgs<B, U>{a, b, nbM, nbK, nbN, sg, tau, C, w});
     else
         small_kernel<B, U, THREE, false>()<<<grid, 256, small_lds<B, U, THREE, false>(nbK), s>>>(a, b, nbM, nbK, nbN, sg, tau, C, w);
     return hipGetLastError();

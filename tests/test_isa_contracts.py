@@ -417,12 +417,12 @@ def test_wide_stores_written_out_keep_their_data(tmp_path):
 
 
 def test_one_word_kernels_keep_the_same_contracts(tmp_path):
-    """k_small_word and k_small_word_three: their buffer->LDS loads keep their distance from VALU-written SGPRs and are the only
+    """The one-launch kernels whose list is a register: their buffer->LDS loads keep their distance from VALU-written SGPRs and are the only
     vector-memory instructions between the first and the last of them, nothing is spilled, and the arguments lie in two lines."""
     text = _isa("kernels_small.hip", tmp_path)
     found, checked = _hazards(_instructions(text), "buffer_load_dwordx4", 5)
     assert not found and checked > 60, found
-    kernels = re.findall(r"^(_ZN5spamm(?:12k_small_word|18k_small_word_three)I\w+):[^\n]*\n(.*?)^\.Lfunc_end", text, flags=re.S | re.M)
+    kernels = re.findall(r"^(_ZN5spamm(?:7k_small|13k_small_three)ENS_8WordArgs\w+):[^\n]*\n(.*?)^\.Lfunc_end", text, flags=re.S | re.M)
     assert len(kernels) == 9
     for name, body in kernels:
         ins = _instructions(body)
