@@ -48,6 +48,7 @@ class SpammError(RuntimeError):
 _lib = None
 _torch = None       # the module, and its types by name, once the library is loaded
 _dtypes = {}
+_call = None        # _spamm_call (csrc/spamm_pycall.cpp): the multiply calls for the usual arguments
 
 
 def library_path():
@@ -57,7 +58,7 @@ def library_path():
 
 def load_library():
     """Loads libspamm_gfx950.so; raises if it has not been built (no fallback)."""
-    global _lib, _torch
+    global _lib, _torch, _call
     if _lib is not None:
         return _lib
     path = library_path()
@@ -105,6 +106,12 @@ def load_library():
     L.spamm_strerror.restype = ctypes.c_char_p
     L.spamm_last_hip_error.argtypes = [vp]
     L.spamm_version.restype = ctypes.c_int
+    try:
+        from . import _spamm_call
+        _spamm_call.bind(*(ctypes.cast(f, vp).value for f in (L.spamm_multiply, L.spamm_multiply_f16, L.spamm_multiply_noalloc)))
+        _call = _spamm_call
+    except ImportError as e:
+        raise ImportError("%s: build it with `python -m cuspamm_amd.build`" % e) from e
     _torch = torch
     _dtypes.update(float16=torch.float16, float32=torch.float32)
     _lib = L
@@ -123,8 +130,9 @@ def _check(code, what):
         raise SpammError(code, what)
 
 
-# What a call costs on the host bounds the smallest ones (256 x 256 x 256: 9.4 us a call beside 9.0 of the GPU's): the checks
-# below are made with as few objects as they can be, types by identity and addresses as plain integers (8.4 us a call).
+# What a call costs on the host bounds the smallest ones (256 x 256 x 256: 6.8 us of the GPU): the multiply calls take the usual
+# arguments through native code (spamm_pycall.cpp), and the checks below, which are made for all others, are made with as few objects as they can
+# be, types by identity and addresses as plain integers.
 def _devptr(t, dtype_name):
     if not (type(t) is _torch.Tensor or isinstance(t, _torch.Tensor)) or not t.is_cuda:
         raise TypeError("expected a CUDA tensor")
@@ -196,6 +204,12 @@ class SpammContext:
         operand's fp16 copy and norm map from the previous call are kept (pass the same tensor, it
         only supplies the shape).  prune: tau-aware conversion passes (same C, mask and counts; the
         fp16 copies are then incomplete, see SPAMM_FLAG_PRUNE)."""
+        done = _call.multiply(self._h.value, A, B, C, tile, tau, timing, reuse_a, reuse_b, a_eq_b, prune)
+        if done is not None:
+            if type(done) is int:
+                _check(done, "spamm_multiply" if A.dtype is _dtypes["float32"] else "spamm_multiply_f16")
+            self._shape = done
+            return C
         if A.dim() != 2 or B.dim() != 2:
             raise ValueError("A and B must be matrices")
         M, K = A.shape
@@ -226,6 +240,12 @@ class SpammContext:
     def multiply_noalloc(self, A, B, tile, tau, C, timing=False, a_eq_b=False, prune=False):
         """spamm_multiply_noalloc: the same multiply in the library's fixed device workspace (fp32 inputs,
         caller-provided C, no device allocation inside the call; SpammError ELIMIT beyond the workspace)."""
+        done = _call.multiply_noalloc(self._h.value, A, B, C, tile, tau, timing, a_eq_b, prune)
+        if done is not None:
+            if type(done) is int:
+                _check(done, "spamm_multiply_noalloc")
+            self._shape = done
+            return C
         if getattr(A, "dim", lambda: 0)() != 2 or getattr(B, "dim", lambda: 0)() != 2:
             raise ValueError("A and B must be matrices")
         M, K = A.shape

@@ -12,6 +12,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_PATH = os.path.join(HERE, "libspamm_gfx950.so")
 DEV_LIB_PATH = os.path.join(HERE, "libspamm_dev_gfx950.so")   # measurement aids (csrc/dev_probe.hip), not the engine
+CALL_PATH = os.path.join(HERE, "_spamm_call.so")                # the Python mirror's multiply calls (csrc/spamm_pycall.cpp)
 MAIN_PATH = os.path.join(HERE, "spamm_main")     # the reference's main() on top of the C ABI (csrc/spamm_main.cpp)
 
 SOURCES = ["kernels_normmap.hip", "kernels_gate.hip", "kernels_gemm.hip", "kernels_small.hip", "kernels_tau.hip", "kernels_tools.hip",
@@ -92,8 +93,20 @@ def build_library(verbose=False):
             log = "\n".join(keep)
         return log
 
+    def compile_call():
+        import sysconfig
+        import torch
+        from torch.utils import cpp_extension
+        dirs = cpp_extension.include_paths() + [sysconfig.get_paths()["include"]]
+        lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+        return _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+                     "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi()] + ["-I" + d for d in dirs] +
+                    [os.path.join(CSRC, "spamm_pycall.cpp"), "-o", CALL_PATH, "-L" + lib, "-ltorch_python", "-ltorch_cpu", "-lc10"])
+
     with ThreadPoolExecutor(max_workers=4) as ex:
+        call = ex.submit(compile_call)
         logs = list(ex.map(compile_one, zip(SOURCES, objs)))
+        logs.append(call.result())
     logs.append(_run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH] + objs))
     logs.append(_run([HIPCC] + CFLAGS + ["-shared", os.path.join(CSRC, "dev_probe.hip"), "-o", DEV_LIB_PATH]))
     logs.append(_run([HIPCC, "--offload-arch=gfx950", "-O2", "-std=c++17", "-Wall", os.path.join(CSRC, "spamm_main.cpp"), "-o", MAIN_PATH,

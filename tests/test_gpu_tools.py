@@ -507,3 +507,56 @@ def test_error_reports_of_small_and_large_values_by_turns(ctx, M, K, N, tile):
             assert abs(got - want) <= 1e-9 * want, at
     torch.cuda.synchronize()
     ctx.set_stream(None)
+
+
+def test_native_multiply_call_answers_as_the_checks_in_python(ctx):
+    """The multiply calls take usual arguments through native code and leave all others to the checks in Python: with and without it the
+    same results and the same errors, and nothing of a refused call remains."""
+    import types
+    import torch
+    from cuspamm_amd import api
+    N, tile = 256, 32
+    g = torch.Generator(device="cuda").manual_seed(5)
+    A = torch.randn((N, N), generator=g, device="cuda")
+    B = torch.randn((N, 2 * N), generator=g, device="cuda")
+    h = A.half()
+    C = torch.empty((N, 2 * N), device="cuda")
+    none = types.SimpleNamespace(multiply=lambda *a: None, multiply_noalloc=lambda *a: None)
+    calls = [lambda: ctx.multiply(A, B, tile, 4.0, C), lambda: ctx.multiply(A, B, tile, 4.0, C=C, prune=True), lambda: ctx.multiply(A, B, tile, 4),
+             lambda: ctx.multiply(A, B, np.int64(tile), np.float32(4.0), C), lambda: ctx.multiply(h, B.half(), tile, 4.0, C),
+             lambda: ctx.multiply(A, B, tile, 4.0, C, reuse_b=True), lambda: ctx.multiply(A, A, tile, 4.0, a_eq_b=True),
+             lambda: ctx.multiply_noalloc(A, B, tile, 4.0, C), lambda: ctx.multiply_noalloc(A, B, tile, 4.0, C, timing=True),
+             lambda: ctx.multiply(A.requires_grad_(False), torch.nn.Parameter(B), tile, 4.0, C),
+             # refused: by the checks, or by the engine
+             lambda: ctx.multiply(A, B.t(), tile, 4.0, C), lambda: ctx.multiply(A.t(), B, tile, 4.0, C), lambda: ctx.multiply(A, B, tile, 4.0, C[:, :N]),
+             lambda: ctx.multiply(A, B, tile, 4.0, C.cpu()), lambda: ctx.multiply(A.cpu(), B, tile, 4.0, C), lambda: ctx.multiply(A, B.half(), tile, 4.0, C),
+             lambda: ctx.multiply(A.double(), B.double(), tile, 4.0, C), lambda: ctx.multiply(A, B, tile, 4.0, C.half()), lambda: ctx.multiply(A[0], B, tile, 4.0, C),
+             lambda: ctx.multiply(A, B, 48, 4.0, C), lambda: ctx.multiply(A, B, 0, 4.0, C), lambda: ctx.multiply(A, B, "32", "x", C),
+             lambda: ctx.multiply(A, B, tile, float("nan"), C), lambda: ctx.multiply(A, B, tile, None, C), lambda: ctx.multiply(A, B, tile, 4.0, "C"),
+             lambda: ctx.multiply(A, B, tile, 4.0, C, a_eq_b=True), lambda: ctx.multiply_noalloc(h, B.half(), tile, 4.0, C),
+             lambda: ctx.multiply_noalloc(A, B, tile, 4.0, None)]
+
+    def outcome(call):
+        ctx.multiply(A, B, tile, 4.0, C)                          # (what reuse_b refers to)
+        C.fill_(float("nan"))
+        try:
+            out = call().clone()
+            return out, ctx._shape, ctx.get_mask()
+        except Exception as e:
+            return type(e), str(e), ctx._shape
+
+    native, seen = api._call, 0
+    for i, call in enumerate(calls):
+        first = outcome(call)
+        api._call = none
+        try:
+            second = outcome(call)
+        finally:
+            api._call = native
+        if isinstance(first[0], torch.Tensor):
+            seen += 1
+            assert torch.equal(first[0], second[0]) and first[1] == second[1] and np.array_equal(first[2], second[2]), i
+        else:
+            assert first == second, (i, first, second)
+    assert seen == 10
+    assert native.multiply(None, A, B, C, tile, 4.0, False, False, False, False, False) is None and native.multiply(1, A, B) is None
