@@ -352,7 +352,7 @@ __global__ __launch_bounds__(NTH) void k_gate(GateBuffers g, int nbM, int nbK, i
 // moves inside a row (DPP) instead of trips through LDS, and every thread writes its own part of
 // the sequences.  By the kernel trace, before -> now: 8192^2 of C (32 super tiles, 10 % kept, dealt
 // greedily) 12.2 -> 9.2 us, 16384^2 (128, band) 16.6 -> 12.1, 10048^2 (50, greedy) 19.5 -> 12.5, 32768^2 (512,
-// band) 52.9 -> 24.3.
+// band) 52.9 -> 24.3.  (Up to 64 super tiles are k_order_few's now.)
 __device__ __forceinline__ int order_origin(int sid, int nSupN) {     // first macro tile row, column
     return ((sid / nSupN) * SUPER_M) << 16 | ((sid % nSupN) * SUPER_N);
 }
@@ -416,31 +416,7 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
     //               N = 32768, but +1 to +3 % when most super tiles hold work (algebraic decay,
     //               30 % kept), hence the condition;
     //   DEAL_SNAKE  ranked by length, dealt in snake order (no table: any number of super tiles).
-    //   DEAL_FLAT   fewer super tiles than XCDs (C of at most 7 x 32 macro tiles): whole super tiles
-    //               would leave XCDs empty -- 2048^3 at tile 32 is two of them, 64 workgroups on a
-    //               quarter of the chip -- so the macro tiles themselves are dealt, consecutive
-    //               ones in row-major order (neighbours along a row share the A panel) in equal
-    //               chunks, one per XCD; no ranking (the problem is a few microseconds long).
-    enum { DEAL_LPT, DEAL_BAND, DEAL_SNAKE, DEAL_FLAT };
-    if (n_super < n_xcd) {                      // DEAL_FLAT: one round of at most 28 macro tiles per XCD
-        const int chunk = (nMacM * nMacN + n_xcd - 1) / n_xcd;
-        if (wave < n_xcd) {
-            const int m = wave * chunk + lane;
-            const bool in = lane < chunk && m < nMacM * nMacN;
-            const bool comp = in && g.macro_work[in ? m : 0] > 0;
-            const uint64_t bi = __ballot(in), bc = __ballot(comp), be = bi & ~bc;
-            const int nall = __builtin_popcountll(bi);
-            if (comp) g.order[wave * P + __builtin_popcountll(bc & below)] = m;
-            else if (in) g.order[wave * P + nall - 1 - __builtin_popcountll(be & below)] = m;
-            if (lane == 0) {
-                g.sched[wave] = __builtin_popcountll(bc);
-                g.sched[MAX_XCD + wave] = nall;
-                g.sched[2 * MAX_XCD + wave] = 0;
-            }
-        }
-        if (threadIdx.x == 0) g.kept->total = (int64_t)total;
-        return;
-    }
+    enum { DEAL_LPT, DEAL_BAND, DEAL_SNAKE };
     int n_ne = 0;                               // super tiles with work
     for (int sid0 = 0; sid0 < n_super; sid0 += blockDim.x) {
         const int sid = sid0 + threadIdx.x;
@@ -678,6 +654,152 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
     }
 }
 
+// The schedule of at most 64 super tiles, a super tile a lane: every wave ranks and deals all of them for itself, in registers, and
+// then lays out the sequence of one XCD (fewer XCDs: several waves share one).  Dealt as by k_order, which
+// with so few always deals greedily; fewer super tiles than XCDs (C of at most 7 x 32 macro tiles) are not dealt whole, which would
+// leave XCDs empty -- 2048^3 at tile 32 is two of them, 64 workgroups on a quarter of the chip -- but the macro
+// tiles themselves, consecutive ones in row-major order (neighbours along a row share the A panel) in equal chunks, one per XCD,
+// unranked.
+// What bounds it: its chain of instructions, alone on the chip: a load, a barrier, a readlane and a compare per rank, a deal of 14
+// instructions per super tile.  Against k_order, which has ranks and deals go through LDS with some twenty barriers
+// among 16 waves, gate and schedule together: 5120^2 of C (15 super tiles) 12.3 -> 8.0 us, 8192^2 (32, 10 % kept) 13.9 -> 9.6,
+// 10048^2 (50) 21.4 -> 15.7.  The line is the wave's 64 lanes.
+constexpr int ORDER_FEW = 64;
+constexpr int ORDER_FEW_WAVES = 8;
+static_assert(ORDER_FEW <= LPT_GREEDY_MAX && MAX_XCD <= ORDER_FEW_WAVES, "always the greedy deal; a wave for every XCD");
+__global__ __launch_bounds__(ORDER_FEW_WAVES * 64) void k_order_few(const int32_t *macro_work, const int32_t *macro_count, int32_t *order, int32_t *sched,
+                                                                  KeptProducts *kept, int nMacM, int nMacN, int nSupN, uint32_t sup_rec,
+                                                                  int n_super, int rounds, int xcd_shift) {
+    asm volatile("" : "+s"(macro_work), "+s"(macro_count), "+s"(order), "+s"(sched), "+s"(kept), "+s"(nMacM), "+s"(nMacN), "+s"(nSupN),
+                 "+s"(sup_rec), "+s"(n_super), "+s"(rounds), "+s"(xcd_shift));
+    struct Super {
+        uint32_t len, comp, work;       // entries of its macro tiles' lists, computing macro tiles (bit: slot), kept products
+    };
+    __shared__ Super s_super[ORDER_FEW];
+    __shared__ u32x4 s_seq[ORDER_FEW + MAX_XCD];     // [n_xcd][rounds] origin, computing macro tiles, of the XCD's ones before it computing | empty << 16
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n_xcd = 1 << xcd_shift, n_macro = nMacM * nMacN, P = rounds * SUPER_M * SUPER_N;
+    auto below = [](uint64_t m) { return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)); };
+    auto origin_of = [&](int sid) {                  // first macro tile row, column
+        const int si = (int)__umulhi((uint32_t)sid + 1u, sup_rec);
+        return si * SUPER_M << 16 | (sid - si * nSupN) * SUPER_N;
+    };
+    // eight threads a super tile, four macro tiles a thread; what lies outside C reads as zero
+    {
+        static_assert(SUPER_M * SUPER_N == 32, "eight threads of four macro tiles");
+        const int sid = threadIdx.x >> 3, a = threadIdx.x >> 1 & 3, b0 = (threadIdx.x & 1) * 4;
+        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)macro_work, 0, n_macro * 4, 0x00020000);
+        const __amdgpu_buffer_rsrc_t rl = __builtin_amdgcn_make_buffer_rsrc((void *)macro_count, 0, n_macro * 8, 0x00020000);
+        const int origin = origin_of(sid), mi = (origin >> 16) + a, mj = (origin & 0xffff) + b0;
+        const int at = (mi * nMacN + mj) * 4, room = sid < n_super && mi < nMacM ? nMacN - mj : 0;
+        uint32_t w[4], l[4];
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            const int off = b < room ? at + b * 4 : 0x40000000;
+            w[b] = __builtin_amdgcn_raw_buffer_load_b32(rw, off, 0, 0);
+            l[b] = __builtin_amdgcn_raw_buffer_load_b32(rl, off * 2, 0, 0);
+        }
+        uint32_t len = l[0] + l[1] + l[2] + l[3], work = w[0] + w[1] + w[2] + w[3], comp = 0;
+#pragma unroll
+        for (int b = 0; b < 4; b++) comp |= l[b] ? 1u << b : 0u;
+        comp <<= (threadIdx.x & 7) * 4;
+        auto eight = [&](auto ctrl) {
+            len += (uint32_t)dpp<decltype(ctrl)::value>((int)len);
+            work += (uint32_t)dpp<decltype(ctrl)::value>((int)work);
+            comp |= (uint32_t)dpp<decltype(ctrl)::value>((int)comp);
+        };
+        eight(std::integral_constant<int, 0xB1>{});          // lane ^ 1
+        eight(std::integral_constant<int, 0x4E>{});          // lane ^ 2
+        eight(std::integral_constant<int, 0x141>{});         // 7 - lane: the other four
+        if ((threadIdx.x & 7) == 0) s_super[sid] = {len, comp, work};
+    }
+    __syncthreads();
+    if (wave == ORDER_FEW_WAVES - 1) {
+        const unsigned long long total = wave_sum((unsigned long long)s_super[lane].work);
+        if (lane == 0) kept->total = (int64_t)total;
+    }
+    if (n_super < n_xcd) {                      // one round of at most 28 macro tiles per XCD
+        if (wave < n_xcd) {
+            const int chunk = (n_macro + n_xcd - 1) >> xcd_shift, m = wave * chunk + lane;
+            const bool in = lane < chunk && m < n_macro;
+            const bool comp = in && macro_work[in ? m : 0] > 0;
+            const uint64_t bi = __ballot(in), bc = __ballot(comp), be = bi & ~bc;
+            const int nall = __builtin_popcountll(bi);
+            if (comp) order[wave * P + below(bc)] = m;
+            else if (in) order[wave * P + nall - 1 - below(be)] = m;
+            if (lane == 0) {
+                sched[wave] = __builtin_popcountll(bc);
+                sched[MAX_XCD + wave] = nall;
+                sched[2 * MAX_XCD + wave] = 0;
+            }
+        }
+        return;
+    }
+    // Ranked by descending length, equal lengths by index: no two keys are equal, and those of lanes without a super tile are the least
+    static_assert((uint64_t)SUPER_M * SUPER_N * 65535 * 64 < 1ull << 32, "a key's length");
+    const uint32_t key = s_super[lane].len << 6 | (uint32_t)(63 - lane);
+    int rank = 0;
+    for (int j = 0; j < n_super; j += 8)
+#pragma unroll
+        for (int d = 0; d < 8; d++) rank += (uint32_t)__builtin_amdgcn_readlane((int)key, j + d) > key ? 1 : 0;
+    const uint32_t ranked = (uint32_t)__builtin_amdgcn_ds_permute(rank * 4, (int)key);      // (lanes from n_super on: anything)
+    const int len = lane < n_super ? (int)(ranked >> 6) : 0, sid = 63 - (int)(ranked & 63u);
+    const uint32_t comp = lane < n_super ? s_super[sid].comp : 0u;
+    const int n_ne = __builtin_popcountll(__ballot(len > 0));     // super tiles with work: the first ranks
+    // Each to the XCD with the least length so far that has room: the least of (length, XCD) over eight lanes, of which every eight
+    // hold the same.  The first ones go to the XCDs in turn.
+    int dealt = lane;
+    if (n_ne > n_xcd) {
+        const int x = lane & 7;
+        uint32_t load = x < n_xcd ? (uint32_t)__builtin_amdgcn_ds_bpermute(x * 4, len) << 3 | (uint32_t)x : ~0u;
+        int room = rounds - 1;
+        for (int r = n_xcd; r < n_ne; r++) {
+            uint32_t least = load, o;
+            o = (uint32_t)dpp<0xB1>((int)least); least = o < least ? o : least;
+            o = (uint32_t)dpp<0x4E>((int)least); least = o < least ? o : least;
+            o = (uint32_t)dpp<0x141>((int)least); least = o < least ? o : least;
+            const uint32_t more = load + ((uint32_t)__builtin_amdgcn_readlane(len, r) << 3);
+            const bool mine = load == least;
+            room -= mine ? 1 : 0;
+            load = mine ? (room > 0 ? more : ~0u) : load;
+            dealt = lane == r ? (int)least : dealt;
+        }
+    }
+    dealt &= 7;
+    // The XCD's super tiles: those dealt to it, then of the ones without work, which fill the XCDs' remaining slots in order
+    const int x = wave & (n_xcd - 1), part = wave >> xcd_shift, parts = ORDER_FEW_WAVES >> xcd_shift;
+    const bool work = lane < n_ne;
+    const int n_dealt = __builtin_popcountll(__ballot(work && dealt == x)), n_less = __builtin_popcountll(__ballot(work && dealt < x));
+    const int fill = n_ne + x * rounds - n_less, fill_end = fill + rounds - n_dealt;
+    const bool member = work ? dealt == x : lane < n_super && lane >= fill && lane < fill_end;
+    const uint64_t members = __ballot(member);
+    const int origin = origin_of(sid), hm = nMacM - (origin >> 16), wn = nMacN - (origin & 0xffff);
+    const int n_comp = member ? __builtin_popcount(comp) : 0;
+    const int n_empty = member ? (hm < SUPER_M ? hm : SUPER_M) * (wn < SUPER_N ? wn : SUPER_N) - n_comp : 0;
+    const uint32_t own = (uint32_t)n_comp | (uint32_t)n_empty << 16, incl = wave_scan(own);      // (at most 2048 of each)
+    const uint32_t last = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    const int nc = (int)(last & 0xffffu), nall = nc + (int)(last >> 16);
+    if (member) s_seq[x * rounds + below(members)] = u32x4{(uint32_t)origin, comp, incl - own, 0u};    // (where waves share an XCD all write the same)
+    if (lane == 0 && part == 0) {
+        sched[x] = nc;
+        sched[MAX_XCD + x] = nall;
+        sched[2 * MAX_XCD + x] = 0;             // ticket counter of the persistent GEMM
+    }
+    __builtin_amdgcn_wave_barrier();
+    // Half a wave per super tile, lane = macro tile: computing ones to the front of the sequence in order, the others to its back
+    const int slot = lane & 31, n_members = __builtin_popcountll(members);
+    const uint32_t before = (1u << slot) - 1u;
+    for (int r = part * 2 + (lane >> 5); r < n_members; r += parts * 2) {
+        const u32x4 e = s_seq[x * rounds + r];
+        const int oi = (int)(e.x >> 16), oj = (int)(e.x & 0xffffu), mi = oi + slot / SUPER_N, mj = oj + slot % SUPER_N;
+        const int width = nMacN - oj < SUPER_N ? nMacN - oj : SUPER_N;       // (slots before this one that exist, less the computing ones)
+        const int c = __builtin_popcount(e.y & before);
+        const int q = (e.y >> slot) & 1u ? (int)(e.z & 0xffffu) + c
+                                         : nall - 1 - ((int)(e.z >> 16) + (slot / SUPER_N) * width + slot % SUPER_N - c);
+        if (mi < nMacM && mj < nMacN) order[x * P + q] = mi * nMacN + mj;
+    }
+}
+
 // Per-tile ascending list of kept k (the reference's offset[], cuSpAMM.cu:315-325)
 // from the gate's bitmaps: one wave per output tile, popcount below the lane's
 // bit gives every kept k its slot.
@@ -758,7 +880,11 @@ hipError_t launch_gate(const GateBuffers &g, int64_t nbM, int64_t nbK, int64_t n
     const int nSupM = (nMacM + SUPER_M - 1) / SUPER_M, nSupN = (nMacN + SUPER_N - 1) / SUPER_N;
     const int n_super = nSupM * nSupN;
     const int rounds = (n_super + n_xcd - 1) / n_xcd;
-    k_order<<<1, 1024, order_lds_bytes(tile, nbM, nbN), s>>>(g, nMacM, nMacN, nSupN, n_super, rounds, n_xcd);
+    if (n_super <= ORDER_FEW)
+        k_order_few<<<1, ORDER_FEW_WAVES * 64, 0, s>>>(g.macro_work, g.macro_count, g.order, g.sched, g.kept, nMacM, nMacN, nSupN,
+                                                       0xffffffffu / (uint32_t)nSupN, n_super, rounds, __builtin_ctz((unsigned)n_xcd));
+    else
+        k_order<<<1, 1024, order_lds_bytes(tile, nbM, nbN), s>>>(g, nMacM, nMacN, nSupN, n_super, rounds, n_xcd);
     return hipGetLastError();
 }
 

@@ -128,56 +128,6 @@ struct Products {
     }
 };
 
-// Sum over the 64 lanes in every lane, added as shuffles down by 32, 16, .. 1 add in lane 0, without LDS operations: behind the first
-// two steps a lane's partner is anywhere in its row, which repeats every 8, 4, 2 lanes.
-template <typename T>
-__device__ __forceinline__ T wave_sum(T v) {
-    struct Words {
-        uint32_t w[sizeof(T) / 4];
-    };
-    auto both = [&](auto swap) {
-        Words x = __builtin_bit_cast(Words, v), lo, hi;
-#pragma unroll
-        for (unsigned i = 0; i < sizeof(T) / 4; i++) {
-            const auto r = swap(x.w[i]);
-            lo.w[i] = r[0];
-            hi.w[i] = r[1];
-        }
-        v = __builtin_bit_cast(T, lo) + __builtin_bit_cast(T, hi);
-    };
-    both([](uint32_t x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); });
-    both([](uint32_t x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); });
-    auto turned = [&](auto ctrl) {
-        Words x = __builtin_bit_cast(Words, v);
-#pragma unroll
-        for (unsigned i = 0; i < sizeof(T) / 4; i++)
-            x.w[i] = (uint32_t)__builtin_amdgcn_update_dpp((int)x.w[i], (int)x.w[i], decltype(ctrl)::value, 0xF, 0xF, false);
-        v = v + __builtin_bit_cast(T, x);
-    };
-    turned(std::integral_constant<int, 0x128>{});                // row rotated by 8, 4, 2, 1
-    turned(std::integral_constant<int, 0x124>{});
-    turned(std::integral_constant<int, 0x122>{});
-    turned(std::integral_constant<int, 0x121>{});
-    return v;
-}
-
-// Inclusive sum over the lanes up to each, without LDS operations
-__device__ __forceinline__ unsigned long long wave_scan(unsigned long long v) {
-    auto step = [&](auto ctrl, auto rows) {
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
-        v += (unsigned long long)hi << 32 | lo;
-    };
-    constexpr std::integral_constant<int, 0xF> all{};
-    step(std::integral_constant<int, 0x111>{}, all);             // from 1, 2, 4, 8 lanes below in the row
-    step(std::integral_constant<int, 0x112>{}, all);
-    step(std::integral_constant<int, 0x114>{}, all);
-    step(std::integral_constant<int, 0x118>{}, all);
-    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});      // the last lane of rows 0 and 2 to the row above,
-    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});      // of row 1 to the two above it
-    return v;
-}
-
 // One digit of the select: histogram of the PASS-th digit over the products whose higher bits equal
 // the prefix found so far, then (last workgroup) the bin that holds the wanted rank.  Zero products
 // never enter the histogram: sparse data would otherwise queue on one bin.  (What the first pass counted is the

@@ -354,6 +354,47 @@ def test_stages_on_either_side_of_their_line(orc, ctx, M, K, N, tile):
         apart.close()
 
 
+@pytest.mark.parametrize("n_xcd", [1, 4, 8])
+@pytest.mark.parametrize("nMacM,nMacN", [(1, 1), (28, 8), (29, 8), (5, 57), (33, 9), (4, 505), (32, 64), (29, 63), (17, 97)])
+def test_schedule_of_few_super_tiles_deals_every_macro_tile_once(nMacM, nMacN, n_xcd):
+    """At most 64 super tiles of C are scheduled a super tile a lane: below, at and above the number of XCDs, up to
+    64 and one more, ragged in either direction, some of them with nothing kept.  Macro tiles and computing ones per XCD are those of
+    the greedy deal, and C, NaN before, is the product (whole numbers: every sum is exact)."""
+    import torch
+    import cuspamm_amd as sp
+    tile, rng = 128, np.random.default_rng(nMacM * 1000 + nMacN)
+    M, K, N = nMacM * 256 - 128, 16 * tile, nMacN * 256 - 128
+    A = torch.from_numpy(rng.integers(-2, 3, (M, K)).astype(np.float32)).cuda()
+    B = torch.from_numpy(rng.integers(-2, 3, (K, N)).astype(np.float32)).cuda()
+    for i in range(0, M, tile):                          # lists of different lengths, groups of rows without any
+        A[i:i + tile, (0 if i // 1024 % 3 == 1 else rng.integers(0, 17)) * tile:] = 0.0
+    B[:, -N // 4:] = 0.0
+    other = sp.SpammContext(0)
+    try:
+        other.set_option(sp.OPT_NUM_XCD, n_xcd)
+        other.set_option(sp.OPT_GEMM_SHAPE, 1)
+        C = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+        other.multiply(A, B, tile, 1.0, C=C)
+        counts, sched = other.get_macro_counts()
+    finally:
+        other.close()
+    assert torch.equal(C, A @ B)
+    supers = [counts[i:i + 4, j:j + 8, 0] for i in range(0, nMacM, 4) for j in range(0, nMacN, 8)]
+    rounds, want = -(-len(supers) // n_xcd), [[0, 0, 0, 0] for _ in range(n_xcd)]      # length, super tiles, computing, all
+    if len(supers) < n_xcd:
+        chunk = -(-counts[..., 0].size // n_xcd)
+        for x in range(n_xcd):
+            part = counts[..., 0].reshape(-1)[x * chunk:(x + 1) * chunk]
+            want[x][2:] = [np.count_nonzero(part), part.size]
+    else:
+        for s in sorted(supers, key=lambda s: -int(s.sum())):
+            room = [x for x in range(n_xcd) if want[x][1] < rounds]
+            x = min(room, key=lambda x: (want[x][0], x)) if s.any() else room[0]
+            for n, v in enumerate((int(s.sum()), 1, np.count_nonzero(s), s.size)):
+                want[x][n] += v
+    assert [list(v) for v in zip(sched[:n_xcd], sched[8:8 + n_xcd])] == [w[2:] for w in want]
+
+
 def test_schedule_of_the_longest_lists_on_one_xcd(ctx):
     """One XCD takes every super tile of a band, and the lengths dealt to it so far are part of the key it is chosen by:
     lists of 65535 k tiles bring that sum to 2^28 - 1 before the last super tile is dealt (times 8, plus the XCD's number:
