@@ -5,43 +5,21 @@
 // (fp32 multiply, fp32 compare, :305-306), serial O(n^2) compaction
 // (:315-325) and a shared-memory tree count (:328-334).  Here one workgroup
 // owns one macro tile (256 x 256 elements of C = MT x MT output tiles):
-//   phase 1  a wave takes a block of up to 4 x 4 output tiles and 64 k at a
-//            time: it loads the 4 + 4 norms once per lane, forms the 16
-//            products in registers and ballots each comparison into the
-//            tile's 64-bit bitmap word, kept in LDS;
-//   phase 2  per-tile counts and the bitmaps go to memory; then every 64-k
-//            word of the MT*MT bitmaps is transposed across a wave (lane =
-//            k), which gives each k the bit set of tiles that keep it, the
-//            union and the kept-by-all word; an LDS prefix sum over the words
-//            places every kept k of the union in the macro tile's list.  The
-//            union list is what the gated GEMM walks; its length and the
-//            kept-product total are the work counts used to order macro tiles
-//            for load balance.
+//   gate     a wave takes 64 k at a time, lane = k: the comparisons of the macro
+//            tile's norm pairs are the lane's bits, the set of tiles that keep its
+//            k; transposed across the wave they are the tiles' bitmaps, which go
+//            to memory with the per-tile counts;
+//   list     each k with a bit set is an entry of the macro tile's union list,
+//            those kept by every tile first; a scan of the words' entry counts
+//            places them.  The union list is what the gated GEMM walks; its
+//            length and the kept-product total are the work counts used to order
+//            macro tiles for load balance.
 // The reference's compacted per-tile list (offset[], :315-325) is the bitmap's
 // set bits in ascending order; nothing downstream reads it, so it is produced
 // from the bitmap only when asked for (k_klist).
 #include "gemm_device.h"
 
 namespace spamm {
-
-// 64 x 64 bit-matrix transpose across a wave: lane t holds row t; on return
-// lane b holds column b (bit t of the result = bit b of lane t's input).
-// Six butterfly steps, each swapping the off-diagonal j x j blocks of lane
-// pairs (l, l ^ j).
-__device__ __forceinline__ uint64_t transpose64(uint64_t x, int lane) {
-    constexpr uint64_t MASKS[6] = {0x00000000FFFFFFFFull, 0x0000FFFF0000FFFFull, 0x00FF00FF00FF00FFull,
-                                   0x0F0F0F0F0F0F0F0Full, 0x3333333333333333ull, 0x5555555555555555ull};
-#pragma unroll
-    for (int s = 0; s < 6; s++) {
-        const int j = 32 >> s;
-        const uint64_t y = (uint64_t)__shfl_xor((long long)x, j, 64);
-        const bool upper = (lane & j) == 0;              // this lane is the row without bit j
-        const uint64_t ru = upper ? x : y, rl = upper ? y : x;
-        const uint64_t t = ((ru >> j) ^ rl) & MASKS[s];
-        x ^= upper ? (t << j) : t;
-    }
-    return x;
-}
 
 // lo[lane idx] = low word, hi[lane idx] = high word of a wave-uniform 64-bit m; idx must fold to
 // a constant (unrolled loops).  On gfx90a and later a VALU instruction that reads an SGPR needs
@@ -57,6 +35,36 @@ __device__ __forceinline__ void set_lane2(int &lo, int &hi, uint64_t m, int idx)
         : "s"(mlo), "s"(mhi), "n"(idx));
 }
 
+template <int CTRL>
+__device__ __forceinline__ int dpp(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+
+// 64 x 64 bit-matrix transpose across a wave: lane t holds row t; on return lane b holds column b (bit t of the result = bit b
+// of lane t's input).  Six butterfly steps, each swapping the off-diagonal j x j blocks of lane pairs (l, l ^ j), without LDS: the
+// blocks of 32 and of 16 are swapped by instructions of their own, bytes picked by a permute, and what stays is a rotate and a
+// bitwise select.
+__device__ __forceinline__ uint64_t transpose64(uint64_t x, int lane) {
+    const auto h = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)(x >> 32), false, false);
+    uint32_t v[2] = {h[0], h[1]};
+    const uint32_t sel16 = lane & 16 ? 0x07060302u : 0x05040100u, sel8 = lane & 8 ? 0x03070105u : 0x06020400u;
+    const uint32_t keep4 = lane & 4 ? 0xf0f0f0f0u : 0x0f0f0f0fu, keep2 = lane & 2 ? 0xccccccccu : 0x33333333u, keep1 = lane & 1 ? 0xaaaaaaaau : 0x55555555u;
+    const uint32_t turn4 = lane & 4 ? 4u : 28u, turn2 = lane & 2 ? 2u : 30u, turn1 = lane & 1 ? 1u : 31u;
+    auto part = [](uint32_t w, uint32_t other, uint32_t keep, uint32_t turn) {
+        return (w & keep) | (__builtin_amdgcn_alignbit(other, other, turn) & ~keep);
+    };
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v[i], v[i], false, false);       // the pair's even row's, its odd row's
+        uint32_t w = __builtin_amdgcn_perm(r[1], r[0], sel16);
+        w = __builtin_amdgcn_perm((uint32_t)dpp<0x128>((int)w), w, sel8);                // lane ^ 8
+        w = part(w, (uint32_t)dpp<0x1B>(dpp<0x141>((int)w)), keep4, turn4);              // 7 - lane, ^ 3: lane ^ 4
+        w = part(w, (uint32_t)dpp<0x4E>((int)w), keep2, turn2);                          // lane ^ 2
+        v[i] = part(w, (uint32_t)dpp<0xB1>((int)w), keep1, turn1);                       // lane ^ 1
+    }
+    return (uint64_t)v[1] << 32 | v[0];
+}
+
 template <int MT>
 struct GateCfg {
     static constexpr int NT = MT * MT;             // output tiles per macro tile
@@ -67,23 +75,16 @@ struct GateCfg {
     static constexpr uint64_t FULL = NT == 64 ? ~0ull : ((1ull << NT) - 1ull);
 };
 
-// NTH threads per workgroup: 256, or 64 for macro tiles of 2 x 2 output tiles (tile 128), whose
-// four tiles give three of four waves nothing to do: one wave per macro tile lets four times as
-// many macro tiles be in flight on a CU, and this kernel's time is memory latency.
-template <int MT, bool ONE, int NTH = (MT == 2 ? 64 : 256)>
-__global__ __launch_bounds__(NTH) void k_gate(GateBuffers g, int nbM, int nbK, int nbN, int nMacN, float tau, int cw_arg) {
+// A macro tile whose bitmaps exceed a CU's LDS (K / tile beyond ~19 400 at tile 32): the k range is walked in chunks of `cw` 64-k
+// words, twice -- once to count, once to place the list entries -- and the bitmaps of a chunk are recomputed for the second walk;
+// the per-word summaries cover all words.
+template <int MT, int NTH = (MT == 2 ? 64 : 256)>
+__global__ __launch_bounds__(NTH) void k_gate_chunks(GateBuffers g, int nbM, int nbK, int nbN, int nMacN, float tau, int cw) {
     using G = GateCfg<MT>;
     constexpr int NW = NTH / 64;
     constexpr int NT = G::NT, NTP = G::NTP, BT = G::BT;
     extern __shared__ uint64_t smem[];
     const int words = (nbK + 63) >> 6;
-    // LDS holds the tile bitmaps of `cw` 64-k words at a time (cw = words unless K / tile is so
-    // large that a macro tile's bitmaps exceed a CU's LDS: then the k range is walked in chunks,
-    // twice -- once to count, once to place the list entries -- and the bitmaps of a chunk are
-    // recomputed for the second walk); the per-word summaries below cover all words.  ONE: the
-    // instantiation for cw = words, straight-line code without the chunk loop.
-    constexpr bool one_chunk = ONE;
-    const int cw = ONE ? words : cw_arg;
     uint64_t *lmask = smem;                                  // [cw][NTP]: tile bitmaps, later transposed in place
     uint64_t *luf = smem + (size_t)cw * NTP;                 // [words][2]: union word, kept-by-all word
     int *wfull = reinterpret_cast<int *>(luf + 2 * (size_t)words);   // [words + 1] prefix of full entries
@@ -192,10 +193,8 @@ __global__ __launch_bounds__(NTH) void k_gate(GateBuffers g, int nbM, int nbK, i
         int w0 = 0;
         do {
             const int cwn = words - w0 < cw ? words - w0 : cw;
-            if constexpr (pass == 0 || !one_chunk) {
-                build_bitmaps(w0, cwn);
-                __syncthreads();
-            }
+            build_bitmaps(w0, cwn);
+            __syncthreads();
             if constexpr (pass == 0) {
                 // ---- phase 2a: per-tile counts and the bitmaps to memory
                 if (wave == 0 && lane < NT)
@@ -208,10 +207,8 @@ __global__ __launch_bounds__(NTH) void k_gate(GateBuffers g, int nbM, int nbK, i
                 }
                 __syncthreads();
             }
-            if constexpr (pass == 0 || !one_chunk) {
-                transpose_words(w0, cwn, pass == 0);
-                __syncthreads();
-            }
+            transpose_words(w0, cwn, pass == 0);
+            __syncthreads();
             if constexpr (pass == 1) {
                 // ---- phase 2c: union list with per-tile bits.  Entries whose k is kept by every
                 // tile of the macro tile ("full") come first, then the partial ones, each group
@@ -248,10 +245,10 @@ __global__ __launch_bounds__(NTH) void k_gate(GateBuffers g, int nbM, int nbK, i
                         g.macro_list[(int64_t)macro * nbK + pos] = en;
                     }
                 }
-                if constexpr (!one_chunk) __syncthreads();     // the next chunk's bitmaps overwrite these
+                __syncthreads();     // the next chunk's bitmaps overwrite these
             }
             w0 += cw;
-        } while (!ONE && w0 < words);
+        } while (w0 < words);
     };
     walk(std::integral_constant<int, 0>{});
     // ---- between the walks: inclusive scans over the words give each word's offset in its group
@@ -321,6 +318,184 @@ __global__ __launch_bounds__(NTH) void k_gate(GateBuffers g, int nbM, int nbK, i
     }
 }
 
+// The gate of one macro tile.  A wave takes whole 64-k words, lane = k: the MT + MT norms of its k come in at once, and the MT * MT
+// comparisons are the lane's own bits -- the set of tiles that keep its k, which is what the list needs.  Norms are neither negative nor NaN
+// as a rule, so that their products order like their bit patterns: a comparison is a product, a subtraction, and a shift
+// that takes the sign in.  (A word with others in it, or a tau that is NaN, is compared as floats.)  A word in which not even
+// the largest norms' product is kept is done with there.  The tiles' bitmaps are the words' transposes.
+// One barrier: behind it every wave has all words' unions, places them by a scan of its own, and lists the words it gated.
+// NTH threads: 256, or 64 for macro tiles of 2 x 2 output tiles (tile 128), whose few comparisons give three of four waves
+// nothing to do.
+// What bounds it: instructions, and for few macro tiles their chain.  A wave per 4 x 4 tiles with a ballot and two lane writes a
+// comparison, bitmaps in LDS and their transposes by LDS shuffles, against this; gate and schedule together (the schedule's part is 4 to
+// 5 us up to 64 super tiles, 12 at 128, 24 at 512): tile 32 5024^3 10.1 -> 7.1 us, 12032^3 31.6 -> 22.3; tile 64 8192^3 9.6 -> 8.1,
+// 10048^3 15.7 -> 12.3, 16384^3 (band) 26.4 -> 20.0; tile 128 32768^3 (band) 49.5 -> 34.4.
+template <int MT, int NTH = (MT == 2 ? 64 : 256)>
+__global__ __launch_bounds__(NTH) void k_gate(GateBuffers g, int nbM, int nbK, int nbN, float tau) {
+    using G = GateCfg<MT>;
+    constexpr int NW = NTH / 64, NT = G::NT;
+    constexpr int STEP = MT == 8 ? 1 : (MT == 4 ? 2 : 4);     // words whose norms a wave has in flight
+    asm volatile("" : "+s"(g.nA), "+s"(g.nBt), "+s"(g.counts), "+s"(g.mask), "+s"(g.macro_list), "+s"(g.macro_count), "+s"(g.macro_work),
+                 "+s"(nbM), "+s"(nbK), "+s"(nbN), "+s"(tau));
+    extern __shared__ __attribute__((aligned(16))) uint64_t smem[];
+    __shared__ int s_cnt[NW][64];
+    const int words = (nbK + 63) >> 6;
+    ulonglong2 *s_uf = reinterpret_cast<ulonglong2 *>(smem);                   // [words] union, kept by all
+    uint32_t *s_pre = reinterpret_cast<uint32_t *>(s_uf + words);              // [words, even] entries before the word: kept by all | others << 16
+    typedef typename std::conditional<MT == 8, uint64_t, typename std::conditional<MT == 4, uint16_t, uint8_t>::type>::type Bits;
+    Bits *s_bits = reinterpret_cast<Bits *>(s_pre + ((words + 1) & ~1));       // [words][64]
+
+    const int lane = threadIdx.x & 63, wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int mi = blockIdx.y, mj = blockIdx.x;
+    const int64_t macro = (int64_t)mi * gridDim.x + mj;
+    const int rows = nbM - mi * MT < MT ? nbM - mi * MT : MT, cols = nbN - mj * MT < MT ? nbN - mj * MT : MT;
+    const bool interior = rows == MT && cols == MT;
+    uint64_t inside = 0;                                                       // tiles of the macro tile that exist
+#pragma unroll
+    for (int a = 0; a < MT; a++) inside |= a < rows ? ((1ull << cols) - 1ull) << (a * MT) : 0ull;
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)(g.nA + (int64_t)mi * MT * nbK), 0, rows * nbK * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)(g.nBt + (int64_t)mj * MT * nbK), 0, cols * nbK * 4, 0x00020000);
+    const uint32_t tau_bits = tau > 0.0f ? __float_as_uint(tau) : 0u;
+    const int ti = lane / MT, tj = lane % MT;
+    const bool tile_lane = lane < NT && ti < rows && tj < cols;                // lane = tile
+    const int64_t tile = (int64_t)(mi * MT + ti) * nbN + mj * MT + tj;
+    auto below = [](uint64_t m) { return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)); };
+
+    int cnt = 0;                               // lane < NT: kept k of tile `lane` in the wave's words
+    const bool in_regs = words <= NW * STEP;
+    uint64_t bits_[STEP];
+    for (int w0 = wave; w0 < words; w0 += NW * STEP) {
+        uint32_t a[STEP][MT], b[STEP][MT];
+#pragma unroll
+        for (int n = 0; n < STEP; n++) {
+            const int w = w0 + n * NW, k = w * 64 + lane;
+            if (w >= words) break;
+            const int voff = k < nbK ? k * 4 : 0x40000000;
+#pragma unroll
+            for (int x = 0; x < MT; x++) {
+                a[n][x] = __builtin_amdgcn_raw_buffer_load_b32(ra, voff, (x < rows ? x : rows - 1) * (nbK * 4), 0);
+                b[n][x] = __builtin_amdgcn_raw_buffer_load_b32(rb, voff, (x < cols ? x : cols - 1) * (nbK * 4), 0);
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < STEP; n++) {
+            const int w = w0 + n * NW;
+            if (w >= words) break;
+            const bool live = w * 64 + lane < nbK;
+            uint32_t amax = a[n][0], bmax = b[n][0];
+#pragma unroll
+            for (int x = 1; x < MT; x++) {
+                amax = a[n][x] > amax ? a[n][x] : amax;
+                bmax = b[n][x] > bmax ? b[n][x] : bmax;
+            }
+            uint64_t bits = 0, row = 0, u = 0, f = 0;
+            const bool plain = __ballot((amax > bmax ? amax : bmax) >= 0x7f800000u) == 0ull && tau == tau;
+            if (!plain || __ballot(live && __uint_as_float(amax) * __uint_as_float(bmax) >= tau) != 0ull) {
+                if (plain) {
+                    uint32_t half[2] = {0u, 0u};
+#pragma unroll
+                    for (int t = NT - 1; t >= 0; t--) {
+                        const uint32_t p = __float_as_uint(__uint_as_float(a[n][t / MT]) * __uint_as_float(b[n][t % MT]));
+                        half[t / 32] = __builtin_amdgcn_alignbit(half[t / 32], p - tau_bits, 31);
+                    }
+                    bits = ~((uint64_t)half[1] << 32 | half[0]) & G::FULL;
+                } else {
+#pragma unroll
+                    for (int t = 0; t < NT; t++)
+                        bits |= __uint_as_float(a[n][t / MT]) * __uint_as_float(b[n][t % MT]) >= tau ? 1ull << t : 0ull;
+                }
+                if (!interior) bits &= inside;
+                bits = live ? bits : 0ull;
+                u = __ballot(bits != 0ull);
+                f = __ballot(bits == G::FULL);
+                row = transpose64(bits, lane);
+                cnt += __builtin_popcountll(row);
+                if (!in_regs) s_bits[w * 64 + lane] = (Bits)bits;
+            }
+            bits_[n] = bits;
+            if (tile_lane) g.mask[tile * words + w] = row;
+            if (lane == 0) s_uf[w] = ulonglong2{u, f};
+        }
+    }
+    s_cnt[wave][lane] = cnt;
+    __syncthreads();
+
+    // Where each word's entries lie: those kept by every tile of the macro tile ("full") first, then the partial ones.  (Where
+    // several waves are, all write the same.)
+    uint32_t before = 0;
+    for (int v0 = 0; v0 < words; v0 += 64) {
+        const int v = v0 + lane;
+        const ulonglong2 uf = s_uf[v < words ? v : 0];
+        const uint32_t own = v < words ? (uint32_t)__builtin_popcountll(uf.y) | (uint32_t)__builtin_popcountll(uf.x & ~uf.y) << 16 : 0u;
+        const uint32_t incl = wave_scan(own);
+        if (v < words) s_pre[v] = before + incl - own;
+        before += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    }
+    __builtin_amdgcn_wave_barrier();
+    const int n_full = (int)(before & 0xffffu), n_part = (int)(before >> 16);
+    if (wave == 0) {                           // per-tile counts and the macro tile's kept-product total
+        int sum = 0;
+#pragma unroll
+        for (int v = 0; v < NW; v++) sum += s_cnt[v][lane];
+        if (tile_lane) g.counts[tile] = sum;
+        const int work = wave_sum(sum);
+        if (lane == 0) {
+            g.macro_count[2 * macro] = n_full + n_part;
+            g.macro_count[2 * macro + 1] = n_full;
+            g.macro_work[macro] = work;
+        }
+    }
+    if (before == 0u) return;
+    // Each group in ascending k, rotated to start at an anchor k shared by the whole super tile (the k where its diagonal would
+    // sit): the workgroups of a super tile run together on one XCD, and walking k from a common start keeps them on the same A row
+    // panels and B column panels at the same time.  (k_small lists its units' k in the same order; C's bits depend on it.)
+    const int anchor = list_anchor(mi, mj, MT, nbM, nbK, nbN), wa = anchor >> 6;
+    const ulonglong2 anchor_uf = s_uf[wa];
+    const uint64_t below_a = (1ull << (anchor & 63)) - 1ull;
+    const uint32_t at_a = s_pre[wa];
+    const int rot_f = (int)(at_a & 0xffffu) + __builtin_popcountll(anchor_uf.y & below_a);         // entries of each group below the anchor
+    const int rot_p = (int)(at_a >> 16) + __builtin_popcountll(anchor_uf.x & ~anchor_uf.y & below_a);
+    const __amdgpu_buffer_rsrc_t rl = __builtin_amdgcn_make_buffer_rsrc((void *)(g.macro_list + macro * nbK), 0, nbK * (int)sizeof(MacroEntry), 0x00020000);
+    auto list_word = [&](int w, uint64_t bits) {
+        const ulonglong2 uf = s_uf[w];
+        const uint32_t pre = s_pre[w];
+        int pf = (int)(pre & 0xffffu) + below(uf.y) - rot_f, pp = (int)(pre >> 16) + below(uf.x & ~uf.y) - rot_p;
+        pf = pf < 0 ? pf + n_full : pf;
+        pp = pp < 0 ? pp + n_full + n_part : pp + n_full;
+        const int pos = bits == G::FULL ? pf : pp;
+        uint32_t need = 0;                     // rows, columns of the macro tile that keep this k
+        if constexpr (MT == 8) {
+            uint32_t c = (uint32_t)bits | (uint32_t)(bits >> 32);
+            c |= c >> 16;
+            need = ((c | c >> 8) & 0xffu) << 8;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                uint32_t x = (uint32_t)(bits >> (32 * h));
+                x |= x >> 4;
+                x |= x >> 2;
+                x = (x | x >> 1) & 0x01010101u;
+                need |= ((x * 0x10204080u) >> 28) << (4 * h);
+            }
+        } else {
+#pragma unroll
+            for (int x = 0; x < MT; x++) {
+                const uint32_t rowbits = (uint32_t)bits >> (x * MT) & ((1u << MT) - 1u);
+                need |= (rowbits ? 1u << x : 0u) | rowbits << 8;
+            }
+        }
+        const u32x4 en = {(uint32_t)(w * 64 + lane), need, (uint32_t)bits, (uint32_t)(bits >> 32)};
+        __builtin_amdgcn_raw_buffer_store_b128(en, rl, bits != 0ull ? pos * (int)sizeof(MacroEntry) : 0x40000000, 0, 0);
+    };
+    if (in_regs) {
+#pragma unroll
+        for (int n = 0; n < STEP; n++)
+            if (wave + n * NW < words && __ballot(bits_[n] != 0ull) != 0ull) list_word(wave + n * NW, bits_[n]);
+    } else {
+        for (int w = wave; w < words; w += NW)
+            if (__builtin_amdgcn_readfirstlane((int)(s_uf[w].x != 0ull))) list_word(w, (uint64_t)s_bits[w * 64 + lane]);
+    }
+}
+
 // Schedule for the GEMM.  Macro tiles are grouped into super tiles of
 // SUPER_M x SUPER_N (= 32, one per CU of an XCD); workgroups are dispatched
 // round-robin over the n_xcd XCDs of the device, so workgroup b runs on XCD
@@ -355,10 +530,6 @@ __global__ __launch_bounds__(NTH) void k_gate(GateBuffers g, int nbM, int nbK, i
 // band) 52.9 -> 24.3.  (Up to 64 super tiles are k_order_few's now.)
 __device__ __forceinline__ int order_origin(int sid, int nSupN) {     // first macro tile row, column
     return ((sid / nSupN) * SUPER_M) << 16 | ((sid % nSupN) * SUPER_N);
-}
-template <int CTRL>
-__device__ __forceinline__ int dpp(int v) {
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
 }
 
 __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nMacN, int nSupN,
@@ -847,9 +1018,9 @@ size_t gate_lds_bytes(int tile, int64_t nbK, int cap) {
 // k_gate may use all of a CU's LDS for the macro tile's bitmaps (its workgroups are short)
 hipError_t gate_init() {
     hipError_t e;
-    const void *gates[6] = {reinterpret_cast<const void *>(&k_gate<8, true>), reinterpret_cast<const void *>(&k_gate<8, false>),
-                            reinterpret_cast<const void *>(&k_gate<4, true>), reinterpret_cast<const void *>(&k_gate<4, false>),
-                            reinterpret_cast<const void *>(&k_gate<2, true>), reinterpret_cast<const void *>(&k_gate<2, false>)};
+    const void *gates[6] = {reinterpret_cast<const void *>(&k_gate<8>), reinterpret_cast<const void *>(&k_gate_chunks<8>),
+                            reinterpret_cast<const void *>(&k_gate<4>), reinterpret_cast<const void *>(&k_gate_chunks<4>),
+                            reinterpret_cast<const void *>(&k_gate<2>), reinterpret_cast<const void *>(&k_gate_chunks<2>)};
     for (const void *f : gates)
         if ((e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gate_lds_limit())) != hipSuccess) return e;
     // k_order: its tables may take order_lds_limit() on top of a few static bytes
@@ -866,8 +1037,8 @@ hipError_t launch_gate(const GateBuffers &g, int64_t nbM, int64_t nbK, int64_t n
     const int cw = gate_chunk_words(tile, nbK, chunk_cap);
     const bool one = cw >= (int)((nbK + 63) / 64);
 #define SPAMM_GATE(MTV)                                                                                          \
-    if (one) k_gate<MTV, true><<<n_macro, MTV == 2 ? 64 : 256, lds, s>>>(g, (int)nbM, (int)nbK, (int)nbN, nMacN, tau, cw);      \
-    else k_gate<MTV, false><<<n_macro, MTV == 2 ? 64 : 256, lds, s>>>(g, (int)nbM, (int)nbK, (int)nbN, nMacN, tau, cw)
+    if (one) k_gate<MTV><<<dim3((unsigned)nMacN, (unsigned)nMacM), MTV == 2 ? 64 : 256, lds, s>>>(g, (int)nbM, (int)nbK, (int)nbN, tau);      \
+    else k_gate_chunks<MTV><<<n_macro, MTV == 2 ? 64 : 256, lds, s>>>(g, (int)nbM, (int)nbK, (int)nbN, nMacN, tau, cw)
     switch (MT) {
         case 8: SPAMM_GATE(8); break;
         case 4: SPAMM_GATE(4); break;

@@ -131,7 +131,7 @@ hipError_t launch_fill_decay(float *X, int64_t rows, int64_t cols, const float *
                              uint64_t seed, int random, hipStream_t s);
 
 size_t gate_lds_bytes(int tile, int64_t nbK, int chunk_cap = 0);   // chunk_cap > 0: at most that many 64-k words of bitmaps in LDS at a time
-inline size_t gate_lds_limit() { return 160 * 1024 - 64; }   // dynamic LDS of k_gate (a few static bytes aside)
+inline size_t gate_lds_limit() { return 160 * 1024 - 1088; }   // dynamic LDS of k_gate (beside 1 KiB of counts)
 // k_order ranks the super tiles of C (4 x 8 macro tiles of 256 x 256) in one workgroup's LDS
 constexpr int LPT_MAX_SUPER = 2048;     // the greedy deal's table is laid out for at most this many super tiles,
 constexpr int LPT_GREEDY_MAX = 64;      // and it runs while at most this many of them hold any work

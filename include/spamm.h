@@ -101,7 +101,7 @@ SPAMM_API int spamm_destroy(spamm_ctx *ctx);
  *     1, 2, 4 or 8; 0 = derive from the device's CU count (what spamm_create does; a partitioned
  *     device shows fewer).  Invalidates the gate of the last call.
  *   SPAMM_OPT_GATE_CHUNK_WORDS: the gate walks K in chunks of at most this many 64-k-tile bitmap
- *     words; 0 = as many as fit LDS (one chunk unless K / tile exceeds ~19 500 at tile 32).
+ *     words; 0 = as many as fit LDS (one chunk unless K / tile exceeds ~19 400 at tile 32).
  *   SPAMM_OPT_GEMM_RING: LDS stages of the GEMM's operand ring, 3..5; 0 = default (4).
  *   SPAMM_OPT_GEMM_SHAPE: work unit of the gated GEMM: 1 = a workgroup of four waves per 256 x 256
  *     macro tile of C (one workgroup per CU), 2 = four waves per 128 x 256 half (two workgroups per
@@ -174,7 +174,7 @@ SPAMM_API int spamm_normmap_f16(spamm_ctx *ctx, int role, const void *dXh, int64
  * spamm_set_normmaps); SPAMM_ESTATE unless both are present for the same K and tile.
  * Shape limit (SPAMM_EINVAL): at most 8192 super tiles of 1024 x 2048 elements of C.  K is not
  * limited beyond the 65535 tiles per dimension: a macro tile's bitmaps are held in LDS, and where
- * they do not fit (K / tile beyond about 19 500 at tile 32) the gate walks K in chunks. */
+ * they do not fit (K / tile beyond about 19 400 at tile 32) the gate walks K in chunks. */
 SPAMM_API int spamm_gate(spamm_ctx *ctx, float tau);
 
 /* Stage 3 -- replaces the product loop of get_C_FP16_B32 (cuSpAMM.cu:336-391):

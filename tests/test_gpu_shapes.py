@@ -114,6 +114,53 @@ def test_gate_in_small_k_chunks_gives_the_same_lists(orc, ctx, chunk_words):
         other.close()
 
 
+@pytest.mark.parametrize("tile,nbM,nbK,nbN", [(32, 8, 64, 8), (32, 9, 65, 23), (32, 16, 257, 8), (32, 3, 4161, 5), (64, 4, 1, 4), (64, 7, 128, 9),
+                                              (64, 8, 513, 4), (64, 5, 8200, 3), (128, 2, 63, 2), (128, 5, 256, 3), (128, 3, 321, 7)])
+def test_gate_by_bits_of_a_lane_gives_the_same_lists(ctx, tile, nbM, nbK, nbN):
+    """The gate of a macro tile whose bitmaps fit LDS against the one that walks k in chunks, and against numpy: words
+    held in registers and in LDS, one word to more than a wave's lanes, the last one cut, macro tiles cut by the matrix, norms
+    that are zero, infinite, negative or NaN, products that overflow or are denormal, every kind of tau.  Where operands
+    are small enough, C, whose bits depend on the lists, as well."""
+    import torch
+    import cuspamm_amd as sp
+    rng = np.random.default_rng(nbK)
+    nA = rng.random((nbM, nbK), dtype=np.float32) * np.exp(-0.02 * rng.integers(0, 400, (1, nbK))).astype(np.float32)
+    nB = rng.random((nbK, nbN), dtype=np.float32)
+    nA[:, : nbK // 2 // 64 * 64] *= np.float32(1e-30)                 # words with nothing kept, at most of the taus
+    other = sp.SpammContext(0)
+    other.set_option(sp.OPT_GATE_CHUNK_WORDS, 3)
+    plain = sp.SpammContext(0)
+    plain.set_option(sp.OPT_GEMM_SHAPE, 1)
+    try:
+        for special in (False, True):
+            if special:
+                odd = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, -1.0, 3e38, 1e-40], np.float32)
+                for X in (nA, nB):
+                    at = rng.random(X.shape) < 0.02
+                    X[at] = rng.choice(odd, at.sum())
+            at_tau = float(nA[0, -1] * nB[-1, 0])
+            for tau in (0.0, 0.3, 1e-33, 0.1 if at_tau != at_tau else at_tau, -1.0, float("inf")):
+                got = []
+                for c in (plain, other):
+                    c.set_normmaps(nA, nB, tile)
+                    c.gate(tau)
+                    got.append((c.get_mask(), c.get_counts(), c.get_macro_counts()[0], c.get_stats().kept_products))
+                with np.errstate(all="ignore"):
+                    keep = nA[:, None, :] * nB.T[None, :, :] >= np.float32(tau)
+                assert np.array_equal(got[0][1], keep.sum(axis=2)) and got[0][3] == keep.sum()
+                for x, y in zip(*got):
+                    assert np.array_equal(x, y)
+        if nbK <= 600:
+            M, K, N = nbM * tile, nbK * tile, nbN * tile
+            A = torch.randn((M, K), device="cuda") * (torch.rand((nbM, 1, nbK, 1), device="cuda") < 0.6).expand(-1, tile, -1, tile).reshape(M, K)
+            B = torch.randn((K, N), device="cuda") * torch.logspace(0, -4, nbN, device="cuda").repeat_interleave(tile)
+            for tau in (0.0, 0.05 * tile, 1.02 * tile):
+                assert torch.equal(plain.multiply(A, B, tile, tau), other.multiply(A, B, tile, tau))
+    finally:
+        plain.close()
+        other.close()
+
+
 @pytest.mark.parametrize("shape", [2, 3, 4])
 def test_other_gemm_work_units_give_the_same_product(orc, ctx, shape):
     """The GEMM's work unit is a whole 256 x 256 macro tile by four waves (shape 1), a 128 x 256
