@@ -521,18 +521,59 @@ __global__ __launch_bounds__(NTH) void k_gate(GateBuffers g, int nbM, int nbK, i
 // q < sched[8 + x] (entries beyond are not written), sched[x] = number of
 // computing items, sched[8 + x] = number of all items.
 // What bounds it: one workgroup on an idle chip, so its time is latencies one after the other.
-// The macro tiles' results are read once, by all threads; what the later steps need of them
+// The macro tiles' results are read once, by all threads, along C's rows; what the later steps need of them
 // -- a length and a set of computing macro tiles per super tile -- stays in LDS, ranks come from
 // prefix sums where the key is only "holds work", the serial deals run in one wave on lane
 // moves inside a row (DPP) instead of trips through LDS, and every thread writes its own part of
-// the sequences.  By the kernel trace, before -> now: 8192^2 of C (32 super tiles, 10 % kept, dealt
-// greedily) 12.2 -> 9.2 us, 16384^2 (128, band) 16.6 -> 12.1, 10048^2 (50, greedy) 19.5 -> 12.5, 32768^2 (512,
-// band) 52.9 -> 24.3.  (Up to 64 super tiles are k_order_few's now.)
-__device__ __forceinline__ int order_origin(int sid, int nSupN) {     // first macro tile row, column
-    return ((sid / nSupN) * SUPER_M) << 16 | ((sid % nSupN) * SUPER_N);
+// the sequences, the tables of four super tiles in flight.  By the kernel trace, first form -> before: 16384^2 of C (128 super
+// tiles, band) 16.6 -> 12.1 us, 32768^2 (512, band) 52.9 -> 24.3.  Then reads along the rows, the band's groups dealt by two
+// sorts of eight lanes, divisions by reciprocals and sequences four at a time, gate and schedule together: 16384^2 20.0 -> 17.6 us,
+// 32768^2 34.4 -> 27.1.  Up to 64 super tiles are k_order_few's.
+// Super tiles along C's rows, and floor((2^32 - 1) / them): exact quotients, there are at most ORDER_MAX_SUPER super tiles
+struct SuperGrid {
+    int n;
+    uint32_t rec;
+    __device__ __forceinline__ int origin(int sid) const {               // first macro tile row, column
+        const int si = (int)__umulhi((uint32_t)sid + 1u, rec);
+        return si * SUPER_M << 16 | (sid - si * n) * SUPER_N;
+    }
+};
+
+struct Super {
+    uint32_t len, comp, work;       // entries of its macro tiles' lists, computing macro tiles (bit: slot), kept products
+};
+// Sums over every eight lanes, in all of them
+__device__ __forceinline__ Super super_of_eight(Super s) {
+    auto eight = [&](auto ctrl) {
+        s.len += (uint32_t)dpp<decltype(ctrl)::value>((int)s.len);
+        s.work += (uint32_t)dpp<decltype(ctrl)::value>((int)s.work);
+        s.comp |= (uint32_t)dpp<decltype(ctrl)::value>((int)s.comp);
+    };
+    eight(std::integral_constant<int, 0xB1>{});          // lane ^ 1
+    eight(std::integral_constant<int, 0x4E>{});          // lane ^ 2
+    eight(std::integral_constant<int, 0x141>{});         // 7 - lane: the other four
+    return s;
 }
 
-__global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nMacN, int nSupN,
+// Every eight lanes' keys in order, the least (DOWN: the greatest) in the first
+template <bool DOWN>
+__device__ __forceinline__ uint32_t sort8(uint32_t k, int lane) {
+    auto step = [&](auto ctrl, int upper) {
+        const uint32_t o = (uint32_t)dpp<decltype(ctrl)::value>((int)k), lo = k < o ? k : o, hi = k < o ? o : k;
+        k = (upper != 0) != DOWN ? hi : lo;
+    };
+    constexpr std::integral_constant<int, 0xB1> x1{};
+    constexpr std::integral_constant<int, 0x4E> x2{};
+    step(x1, lane & 1);
+    step(std::integral_constant<int, 0x1B>{}, lane & 2);         // 3 - lane of the four
+    step(x1, lane & 1);
+    step(std::integral_constant<int, 0x141>{}, lane & 4);        // 7 - lane of the eight
+    step(x2, lane & 2);
+    step(x1, lane & 1);
+    return k;
+}
+
+__global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nMacN, SuperGrid sup,
                                                 int n_super, int rounds, int n_xcd) {
     extern __shared__ __attribute__((aligned(16))) int swork[];               // [n_super + 8] length; at the end, computing macro tiles before an XCD's r-th super tile
     int *sempty = swork + n_super + MAX_XCD;                                  // [n_super + 8] at the end: empty macro tiles before it
@@ -540,39 +581,51 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
     int *srank_id = reinterpret_cast<int *>(scomp + n_super);                 // [n_super] super tile origin by rank,
     uint16_t *sdeal = reinterpret_cast<uint16_t *>(srank_id + n_super);      // then (dealt by table) [n_xcd][rounds] rank of each XCD's r-th super tile
     __shared__ unsigned long long total;
-    __shared__ int s_count[16], s_len[64], s_orig[64];
+    __shared__ int s_with_work, s_count[16], s_len[64], s_orig[64];
     __shared__ int s_cnt[MAX_XCD], s_before[MAX_XCD], s_nall[MAX_XCD];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wave_u = __builtin_amdgcn_readfirstlane(wave);
     const uint64_t below = (1ull << lane) - 1ull;
     const int P = rounds * SUPER_M * SUPER_N;
-    if (threadIdx.x == 0) total = 0;
-    // every thread takes one macro tile row of one super tile: all loads of a step are in flight at once
-    for (int sid = threadIdx.x; sid < n_super; sid += blockDim.x) { swork[sid] = 0; scomp[sid] = 0u; }
+    if (threadIdx.x == 0) { total = 0; s_with_work = 0; }
     __syncthreads();
-    unsigned long long mine = 0;
-    for (int e = threadIdx.x; e < n_super * SUPER_M; e += blockDim.x) {
-        const int sid = e / SUPER_M, a = e % SUPER_M;
-        const int mi = (sid / nSupN) * SUPER_M + a, mj0 = (sid % nSupN) * SUPER_N;
-        int w[SUPER_N], l[SUPER_N], len = 0;
-        uint32_t bits = 0;
+    {
+        const __amdgpu_buffer_rsrc_t work_of = __builtin_amdgcn_make_buffer_rsrc((void *)g.macro_work, 0, nMacM * nMacN * 4, 0x00020000);
+        const __amdgpu_buffer_rsrc_t count_of = __builtin_amdgcn_make_buffer_rsrc((void *)g.macro_count, 0, nMacM * nMacN * 8, 0x00020000);
+        unsigned long long mine = 0;
+        int with_work = 0;
+        // A wave reads 64 macro tiles of each of a super tile row's rows, a column a lane: eight super tiles.  (By super tiles, four macro
+        // tiles a thread, an instruction touched 32 lines: 512 super tiles 19000 clocks.)
+        static_assert(SUPER_N == 8, "eight lanes a super tile");
+        const int across = (sup.n + 7) / 8, strips = (nMacM + SUPER_M - 1) / SUPER_M * across;
+        const uint32_t across_rec = 0xffffffffu / (uint32_t)across;
+#pragma unroll 2
+        for (int strip = wave_u; strip < strips; strip += 16) {
+            const int si = (int)__umulhi((uint32_t)strip + 1u, across_rec), sj = (strip - si * across) * 8 + (lane >> 3);
+            const int mj = sj * SUPER_N + (lane & 7), mi0 = si * SUPER_M;
+            uint32_t w[SUPER_M], l[SUPER_M];
 #pragma unroll
-        for (int b = 0; b < SUPER_N; b++) {
-            const bool in = mi < nMacM && mj0 + b < nMacN;
-            w[b] = in ? g.macro_work[mi * nMacN + mj0 + b] : 0;
-            l[b] = in ? g.macro_count[2 * (mi * nMacN + mj0 + b)] : 0;
-        }
+            for (int a = 0; a < SUPER_M; a++) {
+                const int off = mi0 + a < nMacM && mj < nMacN ? ((mi0 + a) * nMacN + mj) * 4 : 0x40000000;      // beyond C: zero
+                w[a] = __builtin_amdgcn_raw_buffer_load_b32(work_of, off, 0, 0);
+                l[a] = __builtin_amdgcn_raw_buffer_load_b32(count_of, off * 2, 0, 0);
+            }
+            Super sp = {0, 0, 0};
 #pragma unroll
-        for (int b = 0; b < SUPER_N; b++) {
-            len += l[b];
-            bits |= w[b] > 0 ? 1u << b : 0u;
-            mine += (unsigned long long)w[b];
+            for (int a = 0; a < SUPER_M; a++) {
+                sp.len += l[a];
+                sp.work += w[a];
+                sp.comp |= (l[a] ? 1u << (a * SUPER_N) : 0u);
+            }
+            sp.comp <<= lane & 7;
+            sp = super_of_eight(sp);
+            const bool leads = (lane & 7) == 0 && sj < sup.n;
+            if (leads) { swork[si * sup.n + sj] = (int)sp.len; scomp[si * sup.n + sj] = sp.comp; }
+            mine += leads ? sp.work : 0u;
+            with_work += __builtin_popcountll(__ballot(leads && sp.len > 0));
         }
-        if (len) atomicAdd(&swork[sid], len);
-        if (bits) atomicOr(&scomp[sid], bits << (a * SUPER_N));
+        mine = wave_sum(mine);
+        if (lane == 0 && mine) { atomicAdd(&total, mine); atomicAdd(&s_with_work, with_work); }
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) mine += __shfl_xor(mine, off, 64);
-    if (lane == 0 && mine) atomicAdd(&total, mine);
     __syncthreads();
     // How the super tiles are dealt to the XCDs (sdeal, or the snake formula in dealt):
     //   DEAL_LPT    few super tiles hold work: ranked by length, each goes to the XCD with the
@@ -588,16 +641,7 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
     //               30 % kept), hence the condition;
     //   DEAL_SNAKE  ranked by length, dealt in snake order (no table: any number of super tiles).
     enum { DEAL_LPT, DEAL_BAND, DEAL_SNAKE };
-    int n_ne = 0;                               // super tiles with work
-    for (int sid0 = 0; sid0 < n_super; sid0 += blockDim.x) {
-        const int sid = sid0 + threadIdx.x;
-        const uint64_t m = __ballot(sid < n_super && swork[sid < n_super ? sid : 0] > 0);
-        if (lane == 0) s_count[wave] = __builtin_popcountll(m);
-        __syncthreads();
-#pragma unroll
-        for (int v = 0; v < 16; v++) n_ne += s_count[v];
-        __syncthreads();
-    }
+    const int n_ne = s_with_work;               // super tiles with work
     const int deal = n_super > LPT_MAX_SUPER ? DEAL_SNAKE
                      : (n_ne <= LPT_GREEDY_MAX ? DEAL_LPT
                         : (n_ne <= BAND_DEAL_MAX && 5 * n_ne <= 3 * n_super ? DEAL_BAND : DEAL_SNAKE));
@@ -611,6 +655,7 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
         int len_[STEPS], rank_[STEPS], ne = 0;
 #pragma unroll
         for (int n = 0; n < STEPS; n++) {
+            if (n * 1024 >= n_super) break;
             const int sid = n * 1024 + threadIdx.x;
             const int len = sid < n_super ? swork[sid] : 0;
             const uint64_t m = __ballot(len > 0);
@@ -632,7 +677,7 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
         for (int n = 0; n < STEPS; n++) {
             const int sid = n * 1024 + threadIdx.x;
             if (sid >= n_super) break;
-            const int rank = rank_[n], origin = order_origin(sid, nSupN);
+            const int rank = rank_[n], origin = sup.origin(sid);
             swork[rank] = len_[n];
             srank_id[rank] = origin;
             if (deal == DEAL_LPT && rank < n_ne) { s_len[rank] = len_[n]; s_orig[rank] = origin; }
@@ -669,41 +714,27 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
             if (x < MAX_XCD) s_cnt[x] = cnt;
         }
         if (wave == 0 && deal == DEAL_BAND) {
-            // lanes 0..7 (and again 8..15, so that a rotation by row of 16 is one by 8): the group's i-th
-            // super tile and XCD i's length so far.  Ranks are counts over seven rotations of keys that
-            // carry the index; XCD x takes the super tile whose rank (heaviest first) is its own (shortest
-            // first).  (One XCD may be dealt all super tiles: its key needs the 32nd bit.)
+            // every eight lanes: the XCDs by their length so far and the group's super tiles by theirs, both sorted with
+            // the number in the key; the n-th shortest XCD takes the n-th heaviest super tile.  (One XCD may be dealt all super
+            // tiles: its key needs the 32nd bit.)
             static_assert((uint64_t)BAND_DEAL_MAX * SUPER_M * SUPER_N * 65535 * 8 + MAX_XCD < 0xfffffff0u, "an XCD's key stays below the absent ones'");
             const int x = lane & 7;
-            int load = 0, cnt = 0;
             const int ngroups = (n_ne + n_xcd - 1) / n_xcd;
             auto weight = [&](int g2) -> int { const int r = g2 * n_xcd + x; return x < n_xcd && r < n_ne ? swork[r] : -1; };     // -1: no super tile
+            uint32_t load = x < n_xcd ? (uint32_t)x : 0xfffffff0u + (uint32_t)x;      // length << 3 | XCD; absent ones stay behind all others
             int w = weight(0);
             for (int g2 = 0; g2 < ngroups; g2++) {
                 const int wn = weight(g2 + 1);
-                const int wkey = (w + 1) * 8 + 7 - x;
-                const uint32_t lkey = x < n_xcd ? (uint32_t)load * 8u + (uint32_t)x : 0xfffffff0u + (uint32_t)x;
-                int wrank = 0, xrank = 0;
-                static_for<7>([&](auto i) {
-                    constexpr int ROR = 0x121 + decltype(i)::value;
-                    wrank += dpp<ROR>(wkey) > wkey;
-                    xrank += (uint32_t)dpp<ROR>((int)lkey) < lkey;
-                });
-                const int pk = (w + 1) << 6 | x << 3 | wrank;
-                int sel = wrank == xrank ? pk : 0;
-                static_for<7>([&](auto i) {
-                    const int o = dpp<0x121 + decltype(i)::value>(pk);
-                    sel = (o & 7) == xrank ? o : sel;
-                });
-                const int wm = (sel >> 6) - 1;
-                if (x < n_xcd && wm > 0) {       // (the last group may have fewer super tiles than XCDs)
-                    if (lane < MAX_XCD) sdeal[x * rounds + cnt] = (uint16_t)(g2 * n_xcd + ((sel >> 3) & 7));
-                    cnt++;
-                    load += wm;
+                load = sort8<false>(load, lane);
+                const uint32_t heavy = sort8<true>((uint32_t)(w + 1) << 3 | (uint32_t)(7 - x), lane);
+                const int wm = (int)(heavy >> 3) - 1;
+                if (wm > 0) {                    // (the last group may have fewer super tiles than XCDs)
+                    if (lane < MAX_XCD) sdeal[(load & 7u) * rounds + g2] = (uint16_t)(g2 * n_xcd + 7 - (int)(heavy & 7u));
+                    load += (uint32_t)wm << 3;
                 }
+                if (g2 == ngroups - 1 && lane < n_xcd) s_cnt[load & 7u] = g2 + (wm > 0);
                 w = wn;
             }
-            if (lane < MAX_XCD) s_cnt[x] = cnt;
         }
         __syncthreads();
         // super tiles with nothing kept (ranks n_ne ..) fill the XCDs' remaining slots in order
@@ -735,7 +766,7 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
         const int sid = threadIdx.x;              // n_super <= RANK_SORT_MIN < blockDim.x: one super tile per thread
         const int rank = sid < n_super ? srank_id[sid] : 0;
         __syncthreads();
-        if (sid < n_super) srank_id[rank] = order_origin(sid, nSupN);
+        if (sid < n_super) srank_id[rank] = sup.origin(sid);
     } else {
         // a bitonic sort of the indices in LDS (padded to a power of two with indices >= n_super,
         // which sort last): log^2 steps of one compare-exchange per thread instead of n_super
@@ -757,7 +788,7 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
                 __syncthreads();
             }
         // sidx[rank] = super tile; every thread turns its own slots into origins
-        for (int r = threadIdx.x; r < n_super; r += blockDim.x) srank_id[r] = order_origin(sidx[r], nSupN);
+        for (int r = threadIdx.x; r < n_super; r += blockDim.x) srank_id[r] = sup.origin(sidx[r]);
     }
     __syncthreads();
 
@@ -766,7 +797,7 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
         if (deal == DEAL_SNAKE) return r * n_xcd + ((r & 1) ? n_xcd - 1 - x : x);
         return r < s_cnt[x] ? (int)sdeal[x * rounds + r] : n_ne + s_before[x] + r - s_cnt[x];
     };
-    auto sid_of = [&](int origin) -> int { return (origin >> 16) / SUPER_M * nSupN + (origin & 0xffff) / SUPER_N; };
+    auto sid_of = [&](int origin) -> int { return (origin >> 16) / SUPER_M * sup.n + (origin & 0xffff) / SUPER_N; };
     // computing macro tiles go to the front of the XCD's sequence in order, empty ones to the back: one wave
     // per XCD adds up how many of each come before its r-th super tile
     if (wave < n_xcd) {
@@ -809,18 +840,34 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
         const int x = wave % n_xcd, per = 2 * 16 / n_xcd, slot = lane % (SUPER_M * SUPER_N);
         const int nall = s_nall[x], cnt = deal == DEAL_SNAKE ? 0 : s_cnt[x], rest = deal == DEAL_SNAKE ? 0 : n_ne + s_before[x] - cnt;
         const uint32_t before = (1u << slot) - 1u;
-        for (int r = wave / n_xcd * 2 + lane / (SUPER_M * SUPER_N); r < rounds; r += per) {
-            const int sr = deal == DEAL_SNAKE ? r * n_xcd + ((r & 1) ? n_xcd - 1 - x : x) : (r < cnt ? (int)sdeal[x * rounds + r] : rest + r);
-            if (sr >= n_super) continue;
-            const int origin = srank_id[sr], oi = origin >> 16, oj = origin & 0xffff;
-            const int mi = oi + slot / SUPER_N, mj = oj + slot % SUPER_N;
-            if (mi >= nMacM || mj >= nMacN) continue;
-            const uint32_t comp = scomp[sid_of(origin)];
-            const int c = __builtin_popcount(comp & before);
-            const int wn = nMacN - oj < SUPER_N ? nMacN - oj : SUPER_N;       // (slots before this one that exist, less the computing ones)
-            const int q = (comp >> slot) & 1u ? swork[x * rounds + r] + c
-                                              : nall - 1 - (sempty[x * rounds + r] + (slot / SUPER_N) * wn + slot % SUPER_N - c);
-            g.order[x * P + q] = mi * nMacN + mj;
+        constexpr int UNROLL = 4;                // super tiles whose tables a half wave has in flight
+        for (int r0 = wave / n_xcd * 2 + lane / (SUPER_M * SUPER_N); r0 < rounds; r0 += UNROLL * per) {
+            int at[UNROLL], origin[UNROLL], first[UNROLL], empty[UNROLL];
+            uint32_t comp[UNROLL];
+#pragma unroll
+            for (int u = 0; u < UNROLL; u++) {
+                const int r = r0 + u * per;
+                at[u] = n_super;                 // its rank; n_super: none
+                if (r < rounds) at[u] = deal == DEAL_SNAKE ? r * n_xcd + ((r & 1) ? n_xcd - 1 - x : x) : (r < cnt ? (int)sdeal[x * rounds + r] : rest + r);
+            }
+#pragma unroll
+            for (int u = 0; u < UNROLL; u++) {
+                const int r = r0 + u * per < rounds ? r0 + u * per : 0;
+                origin[u] = srank_id[at[u] < n_super ? at[u] : 0];
+                first[u] = swork[x * rounds + r];
+                empty[u] = sempty[x * rounds + r];
+            }
+#pragma unroll
+            for (int u = 0; u < UNROLL; u++) comp[u] = scomp[sid_of(origin[u])];
+#pragma unroll
+            for (int u = 0; u < UNROLL; u++) {
+                const int oi = origin[u] >> 16, oj = origin[u] & 0xffff;
+                const int mi = oi + slot / SUPER_N, mj = oj + slot % SUPER_N;
+                const int c = __builtin_popcount(comp[u] & before);
+                const int wn = nMacN - oj < SUPER_N ? nMacN - oj : SUPER_N;       // (slots before this one that exist, less the computing ones)
+                const int q = (comp[u] >> slot) & 1u ? first[u] + c : nall - 1 - (empty[u] + (slot / SUPER_N) * wn + slot % SUPER_N - c);
+                if (at[u] < n_super && mi < nMacM && mj < nMacN) g.order[x * P + q] = mi * nMacN + mj;
+            }
         }
     }
 }
@@ -839,50 +886,33 @@ constexpr int ORDER_FEW = 64;
 constexpr int ORDER_FEW_WAVES = 8;
 static_assert(ORDER_FEW <= LPT_GREEDY_MAX && MAX_XCD <= ORDER_FEW_WAVES, "always the greedy deal; a wave for every XCD");
 __global__ __launch_bounds__(ORDER_FEW_WAVES * 64) void k_order_few(const int32_t *macro_work, const int32_t *macro_count, int32_t *order, int32_t *sched,
-                                                                  KeptProducts *kept, int nMacM, int nMacN, int nSupN, uint32_t sup_rec,
+                                                                  KeptProducts *kept, int nMacM, int nMacN, SuperGrid sup,
                                                                   int n_super, int rounds, int xcd_shift) {
-    asm volatile("" : "+s"(macro_work), "+s"(macro_count), "+s"(order), "+s"(sched), "+s"(kept), "+s"(nMacM), "+s"(nMacN), "+s"(nSupN),
-                 "+s"(sup_rec), "+s"(n_super), "+s"(rounds), "+s"(xcd_shift));
-    struct Super {
-        uint32_t len, comp, work;       // entries of its macro tiles' lists, computing macro tiles (bit: slot), kept products
-    };
+    asm volatile("" : "+s"(macro_work), "+s"(macro_count), "+s"(order), "+s"(sched), "+s"(kept), "+s"(nMacM), "+s"(nMacN), "+s"(sup.n),
+                 "+s"(sup.rec), "+s"(n_super), "+s"(rounds), "+s"(xcd_shift));
     __shared__ Super s_super[ORDER_FEW];
     __shared__ u32x4 s_seq[ORDER_FEW + MAX_XCD];     // [n_xcd][rounds] origin, computing macro tiles, of the XCD's ones before it computing | empty << 16
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n_xcd = 1 << xcd_shift, n_macro = nMacM * nMacN, P = rounds * SUPER_M * SUPER_N;
     auto below = [](uint64_t m) { return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)); };
-    auto origin_of = [&](int sid) {                  // first macro tile row, column
-        const int si = (int)__umulhi((uint32_t)sid + 1u, sup_rec);
-        return si * SUPER_M << 16 | (sid - si * nSupN) * SUPER_N;
-    };
-    // eight threads a super tile, four macro tiles a thread; what lies outside C reads as zero
     {
-        static_assert(SUPER_M * SUPER_N == 32, "eight threads of four macro tiles");
-        const int sid = threadIdx.x >> 3, a = threadIdx.x >> 1 & 3, b0 = (threadIdx.x & 1) * 4;
-        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)macro_work, 0, n_macro * 4, 0x00020000);
-        const __amdgpu_buffer_rsrc_t rl = __builtin_amdgcn_make_buffer_rsrc((void *)macro_count, 0, n_macro * 8, 0x00020000);
-        const int origin = origin_of(sid), mi = (origin >> 16) + a, mj = (origin & 0xffff) + b0;
-        const int at = (mi * nMacN + mj) * 4, room = sid < n_super && mi < nMacM ? nMacN - mj : 0;
+        const __amdgpu_buffer_rsrc_t work_of = __builtin_amdgcn_make_buffer_rsrc((void *)macro_work, 0, n_macro * 4, 0x00020000);
+        const __amdgpu_buffer_rsrc_t count_of = __builtin_amdgcn_make_buffer_rsrc((void *)macro_count, 0, n_macro * 8, 0x00020000);
+        const int sid = threadIdx.x >> 3, at = threadIdx.x & 7;
+        const int origin = sup.origin(sid), mi = (origin >> 16) + (at >> 1), mj = (origin & 0xffff) + (at & 1) * 4;
+        const int first = (mi * nMacN + mj) * 4, room = sid < n_super && mi < nMacM ? nMacN - mj : 0;
         uint32_t w[4], l[4];
 #pragma unroll
         for (int b = 0; b < 4; b++) {
-            const int off = b < room ? at + b * 4 : 0x40000000;
-            w[b] = __builtin_amdgcn_raw_buffer_load_b32(rw, off, 0, 0);
-            l[b] = __builtin_amdgcn_raw_buffer_load_b32(rl, off * 2, 0, 0);
+            const int off = b < room ? first + b * 4 : 0x40000000;
+            w[b] = __builtin_amdgcn_raw_buffer_load_b32(work_of, off, 0, 0);
+            l[b] = __builtin_amdgcn_raw_buffer_load_b32(count_of, off * 2, 0, 0);
         }
-        uint32_t len = l[0] + l[1] + l[2] + l[3], work = w[0] + w[1] + w[2] + w[3], comp = 0;
+        Super sp = {l[0] + l[1] + l[2] + l[3], 0, w[0] + w[1] + w[2] + w[3]};
 #pragma unroll
-        for (int b = 0; b < 4; b++) comp |= l[b] ? 1u << b : 0u;
-        comp <<= (threadIdx.x & 7) * 4;
-        auto eight = [&](auto ctrl) {
-            len += (uint32_t)dpp<decltype(ctrl)::value>((int)len);
-            work += (uint32_t)dpp<decltype(ctrl)::value>((int)work);
-            comp |= (uint32_t)dpp<decltype(ctrl)::value>((int)comp);
-        };
-        eight(std::integral_constant<int, 0xB1>{});          // lane ^ 1
-        eight(std::integral_constant<int, 0x4E>{});          // lane ^ 2
-        eight(std::integral_constant<int, 0x141>{});         // 7 - lane: the other four
-        if ((threadIdx.x & 7) == 0) s_super[sid] = {len, comp, work};
+        for (int b = 0; b < 4; b++) sp.comp |= l[b] ? 1u << (at * 4 + b) : 0u;
+        sp = super_of_eight(sp);
+        if (at == 0) s_super[sid] = sp;
     }
     __syncthreads();
     if (wave == ORDER_FEW_WAVES - 1) {
@@ -944,7 +974,7 @@ __global__ __launch_bounds__(ORDER_FEW_WAVES * 64) void k_order_few(const int32_
     const int fill = n_ne + x * rounds - n_less, fill_end = fill + rounds - n_dealt;
     const bool member = work ? dealt == x : lane < n_super && lane >= fill && lane < fill_end;
     const uint64_t members = __ballot(member);
-    const int origin = origin_of(sid), hm = nMacM - (origin >> 16), wn = nMacN - (origin & 0xffff);
+    const int origin = sup.origin(sid), hm = nMacM - (origin >> 16), wn = nMacN - (origin & 0xffff);
     const int n_comp = member ? __builtin_popcount(comp) : 0;
     const int n_empty = member ? (hm < SUPER_M ? hm : SUPER_M) * (wn < SUPER_N ? wn : SUPER_N) - n_comp : 0;
     const uint32_t own = (uint32_t)n_comp | (uint32_t)n_empty << 16, incl = wave_scan(own);      // (at most 2048 of each)
@@ -1051,11 +1081,12 @@ hipError_t launch_gate(const GateBuffers &g, int64_t nbM, int64_t nbK, int64_t n
     const int nSupM = (nMacM + SUPER_M - 1) / SUPER_M, nSupN = (nMacN + SUPER_N - 1) / SUPER_N;
     const int n_super = nSupM * nSupN;
     const int rounds = (n_super + n_xcd - 1) / n_xcd;
+    const SuperGrid sup = {nSupN, 0xffffffffu / (uint32_t)nSupN};
     if (n_super <= ORDER_FEW)
-        k_order_few<<<1, ORDER_FEW_WAVES * 64, 0, s>>>(g.macro_work, g.macro_count, g.order, g.sched, g.kept, nMacM, nMacN, nSupN,
-                                                       0xffffffffu / (uint32_t)nSupN, n_super, rounds, __builtin_ctz((unsigned)n_xcd));
+        k_order_few<<<1, ORDER_FEW_WAVES * 64, 0, s>>>(g.macro_work, g.macro_count, g.order, g.sched, g.kept, nMacM, nMacN, sup, n_super, rounds,
+                                                       __builtin_ctz((unsigned)n_xcd));
     else
-        k_order<<<1, 1024, order_lds_bytes(tile, nbM, nbN), s>>>(g, nMacM, nMacN, nSupN, n_super, rounds, n_xcd);
+        k_order<<<1, 1024, order_lds_bytes(tile, nbM, nbN), s>>>(g, nMacM, nMacN, sup, n_super, rounds, n_xcd);
     return hipGetLastError();
 }
 
