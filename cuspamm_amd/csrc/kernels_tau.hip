@@ -482,12 +482,18 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_tree(const float *__restrict__ 
 // Whole calls, launches of their own -> this: 528 products to a kept fraction 66 -> 42 us, tuned 69 -> 50; 21952
 // products 49 and 59.  At 64 per thread the one CU is the slower: 32768 products tuned 83 against 75 us, 64000 to a
 // kept fraction 72.5 against 71, hence TAU_SMALL_MAX.
+// What bounds it: the chain of three histograms, each two barriers and a scan.  Scans by LDS shuffles, divisions -> by lane moves and
+// reciprocals: a selection of 512 or 4096 products 7.45 -> 6.35 us.
 template <int E>
-__device__ __forceinline__ void load_products(const float *__restrict__ nA, const float *__restrict__ nBt, int nbK, int nbN, int total,
-                                              float (&p)[E]) {
-    // product idx = (i * nbN + j) * nbK + k; thread t has t, t + 1024, ...
-    int idx = threadIdx.x, k = idx % nbK, j = idx / nbK % nbN, i = idx / nbK / nbN;
-    const int dk = TAU_NTH % nbK, dj = TAU_NTH / nbK % nbN, di = TAU_NTH / nbK / nbN;
+__device__ __forceinline__ void load_products(const float *__restrict__ nA, const float *__restrict__ nBt, int nbK, int nbN, uint32_t rec_k,
+                                              uint32_t rec_n, int total, float (&p)[E]) {
+    // product idx = (i * nbN + j) * nbK + k; thread t has t, t + 1024, ...; quotients by rec_ = floor((2^32 - 1) / nb_), exact
+    // for divisors up to TAU_SMALL_MAX
+    static_assert((TAU_NTH + 1) * TAU_SMALL_MAX < 1ll << 32, "exact quotients");
+    int idx = threadIdx.x;
+    const int row = (int)__umulhi((uint32_t)idx + 1u, rec_k), drow = (int)__umulhi(TAU_NTH + 1u, rec_k);
+    int i = (int)__umulhi((uint32_t)row + 1u, rec_n), j = row - i * nbN, k = idx - row * nbK;
+    const int di = (int)__umulhi((uint32_t)drow + 1u, rec_n), dj = drow - di * nbN, dk = TAU_NTH - drow * nbK;
 #pragma unroll
     for (int e = 0; e < E; e++) {
         const bool live = idx < total;
@@ -504,14 +510,14 @@ __device__ __forceinline__ void load_products(const float *__restrict__ nA, cons
 
 template <int E>
 __global__ __launch_bounds__(TAU_NTH) void k_tau_small_select(const float *__restrict__ nA, const float *__restrict__ nBt, int nbK, int nbN,
-                                                              int total, unsigned int want0, TauState *__restrict__ host_out,
+                                                              uint32_t rec_k, uint32_t rec_n, int total, unsigned int want0, TauState *__restrict__ host_out,
                                                               unsigned long long *__restrict__ host_seq, unsigned long long seq) {
     constexpr int COPIES = 4;
     __shared__ __attribute__((aligned(16))) unsigned int lh[2048 * COPIES];
     __shared__ unsigned int s_sum[TAU_NW], s_found[3];            // prefix, rank inside the bin, products above it
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float p[E];
-    load_products<E>(nA, nBt, nbK, nbN, total, p);
+    load_products<E>(nA, nBt, nbK, nbN, rec_k, rec_n, total, p);
     for (int b = threadIdx.x; b < 2048 * COPIES; b += TAU_NTH) lh[b] = 0;
     unsigned int positive = 0;
 #pragma unroll
@@ -549,12 +555,7 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_small_select(const float *__res
             h[e] = c.x + c.y + c.z + c.w;
             mine += h[e];
         }
-        unsigned int incl = mine;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const unsigned int o = __shfl_up(incl, off, 64);
-            if (lane >= off) incl += o;
-        }
+        const unsigned int incl = wave_scan(mine);
         if (lane == 63) s_sum[wave] = incl;
         __syncthreads();
         unsigned int above = incl - mine;
@@ -587,19 +588,18 @@ __global__ __launch_bounds__(TAU_NTH) void k_tau_small_select(const float *__res
 
 template <int E>
 __global__ __launch_bounds__(TAU_NTH) void k_tau_small_tune(const float *__restrict__ nA, const float *__restrict__ nBt, int nbK, int nbN,
-                                                            int total, double expected, double tol, int max_rounds,
+                                                            uint32_t rec_k, uint32_t rec_n, int total, double expected, double tol, int max_rounds,
                                                             TauResult *__restrict__ host_out, unsigned long long *__restrict__ host_seq,
                                                             unsigned long long seq) {
     __shared__ unsigned int s_cnt[2][TAU_NW];
     __shared__ double s_sum[TAU_NW];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float p[E];
-    load_products<E>(nA, nBt, nbK, nbN, total, p);
+    load_products<E>(nA, nBt, nbK, nbN, rec_k, rec_n, total, p);
     double sum = 0.0;
 #pragma unroll
     for (int e = 0; e < E; e++) sum += (int)threadIdx.x + e * TAU_NTH < total ? (double)p[e] : 0.0;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off, 64);
+    sum = wave_sum(sum);
     if (lane == 0) s_sum[wave] = sum;
     int turn = 0;
     // products >= thr, of all waves
@@ -678,7 +678,7 @@ hipError_t launch_tau_select(const float *nA, const float *nBt, int64_t nbM, int
     TauWorkspace *ws = (TauWorkspace *)workspace;
     const int64_t n = tau_products(nbM, nbK, nbN);
     if (n <= TAU_SMALL_MAX) {
-#define SPAMM_SELECT(E) k_tau_small_select<E><<<1, TAU_NTH, 0, s>>>(nA, nBt, (int)nbK, (int)nbN, (int)n, (unsigned int)want, host_out, host_seq, seq)
+#define SPAMM_SELECT(E) k_tau_small_select<E><<<1, TAU_NTH, 0, s>>>(nA, nBt, (int)nbK, (int)nbN, 0xffffffffu / (uint32_t)nbK, 0xffffffffu / (uint32_t)nbN, (int)n, (unsigned int)want, host_out, host_seq, seq)
         if (n <= 8 * TAU_NTH) SPAMM_SELECT(8);
         else SPAMM_SELECT(24);
 #undef SPAMM_SELECT
@@ -705,7 +705,7 @@ hipError_t launch_tau_count(const float *nA, const float *nBt, int64_t nbM, int6
 hipError_t launch_tau_tune_small(const float *nA, const float *nBt, int64_t nbM, int64_t nbK, int64_t nbN, double expected, double tol,
                                  int max_rounds, TauResult *host_out, unsigned long long *host_seq, unsigned long long seq, hipStream_t s) {
     const int64_t n = tau_products(nbM, nbK, nbN);
-#define SPAMM_TUNE(E) k_tau_small_tune<E><<<1, TAU_NTH, 0, s>>>(nA, nBt, (int)nbK, (int)nbN, (int)n, expected, tol, max_rounds, host_out, host_seq, seq)
+#define SPAMM_TUNE(E) k_tau_small_tune<E><<<1, TAU_NTH, 0, s>>>(nA, nBt, (int)nbK, (int)nbN, 0xffffffffu / (uint32_t)nbK, 0xffffffffu / (uint32_t)nbN, (int)n, expected, tol, max_rounds, host_out, host_seq, seq)
     if (n <= 8 * TAU_NTH) SPAMM_TUNE(8);
     else SPAMM_TUNE(24);
 #undef SPAMM_TUNE
