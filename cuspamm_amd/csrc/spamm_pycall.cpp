@@ -5,8 +5,9 @@
 //
 // Each function takes what api.py's method has been given and answers None -- unless everything is as it usually is: tensors and numbers
 // of exactly the types expected, shapes that fit, one GPU, contiguous -- and api.py goes on by itself then, with its own checks
-// and errors.  Otherwise the ABI's function has been called, with the interpreter released: the answer is its error code, or the
-// shape tuple that the context keeps.
+// and errors.  So it does where torch throws while a tensor is looked at (a size that is a symbol, say): nothing may be thrown through the
+// interpreter's frames.  Otherwise the ABI's function has been called, with the interpreter released: the answer is its error code, or
+// the shape tuple that the context keeps.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -23,52 +24,72 @@ int (*g_multiply_noalloc)(spamm_ctx *, const spamm_params *, const float *, cons
 const at::Tensor *matrix(PyObject *o) {
     if (!THPVariable_CheckExact(o)) return nullptr;
     const at::Tensor &t = THPVariable_Unpack(o);
-    if (t.dim() != 2 || !t.is_cuda() || t.layout() != c10::kStrided || !t.is_contiguous() || !t.has_storage() || t.is_neg() || t.is_conj()) return nullptr;
+    if (t.is_nested() || t.dim() != 2 || !t.is_cuda() || t.layout() != c10::kStrided || !t.is_contiguous() || !t.has_storage() || t.is_neg() || t.is_conj()) return nullptr;
     return &t;
 }
 
-// args: handle, A, B, C, tile, tau, flags (each a truth value: its bit)
-PyObject *call(PyObject *const *args, Py_ssize_t n, Py_ssize_t expected, const uint32_t *flag_bits, bool noalloc) {
-    if (n != expected || !g_multiply) Py_RETURN_NONE;
-    if (!PyLong_CheckExact(args[0]) || !PyLong_CheckExact(args[4]) || !(PyFloat_CheckExact(args[5]) || PyLong_CheckExact(args[5]))) Py_RETURN_NONE;
+struct Call {
+    spamm_ctx *ctx;
+    spamm_params p;
+    const void *a, *b;
+    float *c;
+    bool half;
+};
+
+// args: handle, A, B, C, tile, tau, flags (each a truth value: its bit).  False: not the usual arguments, or none that Python numbers
+// or truth values can be had of (its error is set).
+bool usual(PyObject *const *args, Py_ssize_t n, Py_ssize_t expected, const uint32_t *flag_bits, bool noalloc, Call &out) {
+    if (n != expected || !g_multiply) return false;
+    if (!PyLong_CheckExact(args[0]) || !PyLong_CheckExact(args[4]) || !(PyFloat_CheckExact(args[5]) || PyLong_CheckExact(args[5]))) return false;
     const at::Tensor *A = matrix(args[1]), *B = matrix(args[2]), *C = matrix(args[3]);
-    if (!A || !B || !C) Py_RETURN_NONE;
+    if (!A || !B || !C) return false;
     const int64_t M = A->size(0), K = A->size(1), N = B->size(1);
-    if (B->size(0) != K || C->size(0) != M || C->size(1) != N || A->device() != B->device() || A->device() != C->device()) Py_RETURN_NONE;
+    if (B->size(0) != K || C->size(0) != M || C->size(1) != N || A->device() != B->device() || A->device() != C->device()) return false;
     const at::ScalarType type = A->scalar_type();
-    if (B->scalar_type() != type || C->scalar_type() != at::kFloat || (type != at::kFloat && (noalloc || type != at::kHalf))) Py_RETURN_NONE;
-    spamm_ctx *ctx = static_cast<spamm_ctx *>(PyLong_AsVoidPtr(args[0]));
+    if (B->scalar_type() != type || C->scalar_type() != at::kFloat || (type != at::kFloat && (noalloc || type != at::kHalf))) return false;
+    out.ctx = static_cast<spamm_ctx *>(PyLong_AsVoidPtr(args[0]));
     const long tile = PyLong_AsLong(args[4]);
     const double tau = PyFloat_AsDouble(args[5]);
-    if (PyErr_Occurred()) {
+    if (PyErr_Occurred() || !out.ctx || tile < 1 || tile > 128) return false;
+    out.p = {};
+    out.p.M = M;
+    out.p.K = K;
+    out.p.N = N;
+    out.p.tile = (int32_t)tile;
+    out.p.tau = (float)tau;
+    for (Py_ssize_t i = 6; i < expected; i++) {
+        const int on = PyObject_IsTrue(args[i]);
+        if (on < 0) return false;
+        if (on) out.p.flags |= flag_bits[i - 6];
+    }
+    out.a = A->const_data_ptr();
+    out.b = B->const_data_ptr();
+    out.c = static_cast<float *>(C->data_ptr());
+    out.half = type == at::kHalf;
+    return true;
+}
+
+PyObject *call(PyObject *const *args, Py_ssize_t n, Py_ssize_t expected, const uint32_t *flag_bits, bool noalloc) {
+    Call k;
+    bool go = false;
+    try {
+        go = usual(args, n, expected, flag_bits, noalloc, k);
+    } catch (...) {
+    }
+    if (!go) {
         PyErr_Clear();
         Py_RETURN_NONE;
     }
-    if (!ctx || tile < 1 || tile > 128) Py_RETURN_NONE;
-    spamm_params p = {};
-    p.M = M;
-    p.K = K;
-    p.N = N;
-    p.tile = (int32_t)tile;
-    p.tau = (float)tau;
-    for (Py_ssize_t i = 6; i < expected; i++) {
-        const int on = PyObject_IsTrue(args[i]);
-        if (on < 0) {
-            PyErr_Clear();
-            Py_RETURN_NONE;
-        }
-        if (on) p.flags |= flag_bits[i - 6];
-    }
-    const void *a = A->const_data_ptr(), *b = B->const_data_ptr();
-    float *c = static_cast<float *>(C->data_ptr());
     int code;
     Py_BEGIN_ALLOW_THREADS
-    if (noalloc) code = g_multiply_noalloc(ctx, &p, static_cast<const float *>(a), static_cast<const float *>(b), c);
-    else if (type == at::kHalf) code = g_multiply_f16(ctx, &p, a, b, c);
-    else code = g_multiply(ctx, &p, static_cast<const float *>(a), static_cast<const float *>(b), c);
+    if (noalloc) code = g_multiply_noalloc(k.ctx, &k.p, static_cast<const float *>(k.a), static_cast<const float *>(k.b), k.c);
+    else if (k.half) code = g_multiply_f16(k.ctx, &k.p, k.a, k.b, k.c);
+    else code = g_multiply(k.ctx, &k.p, static_cast<const float *>(k.a), static_cast<const float *>(k.b), k.c);
     Py_END_ALLOW_THREADS
     if (code != SPAMM_OK) return PyLong_FromLong(code);
-    return Py_BuildValue("(LLLlLLL)", (long long)(M / tile), (long long)(K / tile), (long long)(N / tile), tile, (long long)M, (long long)K, (long long)N);
+    const long long M = k.p.M, K = k.p.K, N = k.p.N;
+    const long tile = k.p.tile;
+    return Py_BuildValue("(LLLlLLL)", M / tile, K / tile, N / tile, tile, M, K, N);
 }
 
 PyObject *multiply(PyObject *, PyObject *const *args, Py_ssize_t n) {

@@ -560,3 +560,19 @@ def test_native_multiply_call_answers_as_the_checks_in_python(ctx):
             assert first == second, (i, first, second)
     assert seen == 10
     assert native.multiply(None, A, B, C, tile, 4.0, False, False, False, False, False) is None and native.multiply(1, A, B) is None
+
+
+@pytest.mark.parametrize("lengths", [(256,) * 256, (256,) * 255 + (128,)], ids=["even rows", "ragged rows"])
+def test_nested_matrices_are_refused(ctx, lengths):
+    """Nested tensors of exactly torch's type, strided, contiguous and two-dimensional: torch throws at their sizes, or answers."""
+    import torch
+    X = torch.randn((256, 256), device="cuda")
+    C = torch.full((256, 256), 7.0, device="cuda")
+    nested = torch.nested.nested_tensor([X[i, :n] for i, n in enumerate(lengths)])
+    assert type(nested) is torch.Tensor and nested.dim() == 2 and nested.is_cuda
+    for A, B, out in ((nested, X, C), (X, nested, C), (X, X, nested)):
+        for multiply in (ctx.multiply, ctx.multiply_noalloc):
+            with pytest.raises((RuntimeError, ValueError)) as e:
+                multiply(A, B, 32, 4.0, out)
+            assert not hasattr(e.value, "code")                   # (by torch or the checks: the engine was not called)
+    assert (C == 7.0).all()
