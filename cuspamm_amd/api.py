@@ -5,6 +5,7 @@ provider); every call goes through the C ABI with raw device pointers.
 """
 import ctypes
 import os
+import warnings
 
 import numpy as np
 
@@ -48,7 +49,17 @@ class SpammError(RuntimeError):
 _lib = None
 _torch = None       # the module, and its types by name, once the library is loaded
 _dtypes = {}
-_call = None        # _spamm_call (csrc/spamm_pycall.cpp): the multiply calls for the usual arguments
+_call = None        # _spamm_call (csrc/spamm_pycall.cpp): the multiply calls for the usual arguments, or PythonCalls
+
+
+class PythonCalls:
+    """What stands in for _spamm_call where it has not been built for this interpreter and torch: all arguments are left to the checks here."""
+
+    @staticmethod
+    def multiply(*args):
+        return None
+
+    multiply_noalloc = multiply
 
 
 def library_path():
@@ -108,10 +119,14 @@ def load_library():
     L.spamm_version.restype = ctypes.c_int
     try:
         from . import _spamm_call
+        built_with = getattr(_spamm_call, "torch_version", None)
+        if built_with != str(torch.__version__):
+            raise ImportError("_spamm_call was built with torch %s, this is %s" % (built_with, torch.__version__))
         _spamm_call.bind(*(ctypes.cast(f, vp).value for f in (L.spamm_multiply, L.spamm_multiply_f16, L.spamm_multiply_noalloc)))
         _call = _spamm_call
     except ImportError as e:
-        raise ImportError("%s: build it with `python -m cuspamm_amd.build`" % e) from e
+        warnings.warn("multiply calls take some 2 us longer of the host: %s (`python -m cuspamm_amd.build`)" % e, RuntimeWarning)
+        _call = PythonCalls
     _torch = torch
     _dtypes.update(float16=torch.float16, float32=torch.float32)
     _lib = L

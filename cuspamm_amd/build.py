@@ -6,13 +6,16 @@ The library is cross-compiled for gfx950 and needs no GPU to build.
 import os
 import subprocess
 import sys
+import sysconfig
+import warnings
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_PATH = os.path.join(HERE, "libspamm_gfx950.so")
 DEV_LIB_PATH = os.path.join(HERE, "libspamm_dev_gfx950.so")   # measurement aids (csrc/dev_probe.hip), not the engine
-CALL_PATH = os.path.join(HERE, "_spamm_call.so")                # the Python mirror's multiply calls (csrc/spamm_pycall.cpp)
+# the Python mirror's multiply calls (csrc/spamm_pycall.cpp); of this interpreter only, by its name
+CALL_PATH = os.path.join(HERE, "_spamm_call" + sysconfig.get_config_var("EXT_SUFFIX"))
 MAIN_PATH = os.path.join(HERE, "spamm_main")     # the reference's main() on top of the C ABI (csrc/spamm_main.cpp)
 
 SOURCES = ["kernels_normmap.hip", "kernels_gate.hip", "kernels_gemm.hip", "kernels_small.hip", "kernels_tau.hip", "kernels_tools.hip",
@@ -93,15 +96,22 @@ def build_library(verbose=False):
             log = "\n".join(keep)
         return log
 
+    # (without it multiplies go through the checks in Python: no reason to be without the engine)
     def compile_call():
-        import sysconfig
-        import torch
-        from torch.utils import cpp_extension
-        dirs = cpp_extension.include_paths() + [sysconfig.get_paths()["include"]]
-        lib = os.path.join(os.path.dirname(torch.__file__), "lib")
-        return _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
-                     "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi()] + ["-I" + d for d in dirs] +
-                    [os.path.join(CSRC, "spamm_pycall.cpp"), "-o", CALL_PATH, "-L" + lib, "-ltorch_python", "-ltorch_cpu", "-lc10"])
+        try:
+            import torch
+            from torch.utils import cpp_extension
+            dirs = cpp_extension.include_paths() + [sysconfig.get_paths()["include"]]
+            lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+            return _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+                         "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(),
+                         '-DSPAMM_TORCH_VERSION="%s"' % torch.__version__] + ["-I" + d for d in dirs] +
+                        [os.path.join(CSRC, "spamm_pycall.cpp"), "-o", CALL_PATH, "-L" + lib, "-ltorch_python", "-ltorch_cpu", "-lc10"])
+        except (RuntimeError, OSError, ImportError) as e:
+            if os.path.exists(CALL_PATH):
+                os.remove(CALL_PATH)
+            warnings.warn("multiply calls will go through the checks in Python: %s" % e)
+            return ""
 
     with ThreadPoolExecutor(max_workers=4) as ex:
         call = ex.submit(compile_call)

@@ -123,4 +123,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_spamm_call", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__spamm_call(void) { return PyModule_Create(&module); }
+// torch_version: of the torch whose headers this was built with; with another one its tensors are not to be looked into
+PyMODINIT_FUNC PyInit__spamm_call(void) {
+    PyObject *m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_version", SPAMM_TORCH_VERSION) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}
