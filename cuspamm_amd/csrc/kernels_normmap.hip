@@ -400,6 +400,8 @@ __global__ __launch_bounds__(64 * NWV) void k_normmap_pair(const void *__restric
 // tau-aware 23.0 -> 20.6, fp16 5024^2 20.5 -> 19.3, tau-aware 17.8 -> 16.2, 12032^2 155 -> 153.5; fp32 tile 64 4096^2 A = B 25.9 -> 24.2, both operands in
 // one launch 33.6 -> 32.4, 8192^2 61.7 -> 61.0.  Reads alone reach 6.8 to 7.2 TB/s there; as soon as one workgroup in sixteen writes its
 // tile the whole comes to 5.5 to 5.8, in whatever order or policy (4 GiB read, 1/16, 3/16, all of the copies written: 624 -> 770, 870, 1090 us).
+// Buffer loads are of whole 32-bit words (an address's lowest two bits need not count): a matrix of halves that begins between two
+// of them (whole_words) stays with the streaming kernel, whose loads are global ones and take any address.
 //
 // Sum over the 64 lanes, in every lane: the same additions as butterfly64.  (Behind the steps of 1 and 2 all lanes of a quad hold one sum, so
 // that a mirrored quad is the neighbour; likewise for 8.)
@@ -707,12 +709,15 @@ constexpr int64_t KEEP_INPUT_MAX = 32ll << 20, KEEP_COPY_MAX = 448ll << 20;
 static bool keep_input(int64_t bytes) { return bytes <= KEEP_INPUT_MAX; }
 static bool keep_copy(int64_t bytes) { return bytes <= KEEP_COPY_MAX; }
 
+// The lean strips' buffer loads are of whole 32-bit words.  (Rows are multiples of 64 bytes: where the first begins decides.  Floats always do.)
+static bool whole_words(const void *X) { return ((uintptr_t)X & 3u) == 0; }
+
 template <int ROLE, bool IN16>
 static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int tile, void *packed, float *nm,
                                  float *nmT, hipStream_t s, void *packed2 = nullptr, float *nm2 = nullptr,
                                  const float *rowmax = nullptr, float tau_skip = 0.0f) {
     const int64_t nbr = rows / tile, nbc = cols / tile;
-    const bool keep = keep_input(rows * cols * (IN16 ? 2 : 4));
+    const bool keep = keep_input(rows * cols * (IN16 ? 2 : 4)), words = !IN16 || whole_words(X);
     const auto strips = [&](int64_t sw) { return (unsigned)(nbr * ((cols + sw - 1) / sw)); };
 #define SPAMM_NORMMAP(T, SW, PH, NWV)                                                                                              \
     k_normmap<T, ROLE, SW, IN16, PH, NWV><<<strips(SW), 64 * NWV, 0, s>>>(X, cols, cols, nbr, nbc, (cols + SW - 1) / SW, (uint4 *)packed, \
@@ -725,15 +730,16 @@ static hipError_t launch_normmap(const void *X, int64_t rows, int64_t cols, int 
             X, (uint32_t)cols, (uint32_t)nbr, (uint32_t)nbc, ns, strip_reciprocal(strips(SW), ns), packed, nm, nmT, packed2, nm2, rowmax, \
             tau_skip, keep_copy(rows * cols * 2));                                                                                        \
     } while (0)
-#define SPAMM_LEAN(T, SW, NWV)                    \
-    do {                                          \
-        if (keep) SPAMM_LEAN_(T, SW, NWV, true);  \
-        else SPAMM_LEAN_(T, SW, NWV, false);      \
+#define SPAMM_LEAN(T, SW, NWV)                            \
+    do {                                                  \
+        if (keep && words) SPAMM_LEAN_(T, SW, NWV, true); \
+        else if (words) SPAMM_LEAN_(T, SW, NWV, false);   \
+        else if constexpr (IN16) SPAMM_NORMMAP(T, SW, 1, NWV); \
     } while (0)
-#define SPAMM_LEAN_IF_KEPT(T, SW, NWV)            \
-    do {                                          \
-        if (keep) SPAMM_LEAN_(T, SW, NWV, true);  \
-        else SPAMM_NORMMAP(T, SW, 1, NWV);        \
+#define SPAMM_LEAN_IF_KEPT(T, SW, NWV)                    \
+    do {                                                  \
+        if (keep && words) SPAMM_LEAN_(T, SW, NWV, true); \
+        else SPAMM_NORMMAP(T, SW, 1, NWV);                \
     } while (0)
     // strip widths and waves: one 8-row group per lane, at most ~42 KiB of LDS and so three workgroups or more per CU.
     // fp16 input: 256 columns, two rows per load (512 in phases before: tile 64 1024^2, both passes, 6.2 -> 4.1 us, 4096^2
@@ -795,18 +801,22 @@ static void launch_pair(const void *A, const void *Bm, int64_t nbM, int64_t nbK,
     const int64_t strips_a = (nbK * B + SW - 1) / SW, strips_b = (nbN * B + SW - 1) / SW;
     const unsigned n_b = (unsigned)(nbK * strips_b), n_a = (unsigned)(nbM * strips_a);
     const int64_t a = nbM * nbK * B * B, b = nbK * nbN * B * B;
-    const bool keep = keep_input((a + b) * (IN16 ? 2 : 4));
+    const bool keep = keep_input((a + b) * (IN16 ? 2 : 4)), words = !IN16 || (whole_words(A) && whole_words(Bm));
     const bool cached = keep_copy(2 * (a > b ? a : b));
     auto lean = [&](auto kept) {
         k_normmap_pair_lean<B, SW, IN16, NWV, decltype(kept)::value><<<n_a + n_b, 64 * NWV, 0, s>>>(
             A, Bm, (uint32_t)nbM, (uint32_t)nbK, (uint32_t)nbN, n_b, (uint32_t)strips_a, strip_reciprocal(n_a, (uint32_t)strips_a),
             (uint32_t)strips_b, strip_reciprocal(n_b, (uint32_t)strips_b), packedA, packedB, nmA, nmB, nmBt, tau_skip, cached);
     };
-    if (keep) lean(std::true_type{});
-    else if constexpr (B == 32 || (B == 64 && !IN16)) lean(std::false_type{});          // (as launch_normmap)
-    else
+    auto streaming = [&](auto) {                                   // (a kernel only where it is called)
         k_normmap_pair<B, SW, IN16, PH, NWV><<<n_a + n_b, 64 * NWV, 0, s>>>(A, Bm, nbM, nbK, nbN, n_b, strips_a, strips_b, (uint4 *)packedA,
                                                                             (uint4 *)packedB, nmA, nmB, nmBt, tau_skip, cached);
+    };
+    if (keep && words) lean(std::true_type{});
+    else if constexpr (B == 32 || (B == 64 && !IN16)) {            // (as launch_normmap)
+        if (words) lean(std::false_type{});
+        else if constexpr (IN16) streaming(0);
+    } else streaming(0);
 }
 
 // Where the two passes are worth running as one, by the strips of both operands, counted as tile rows of 1 KiB (256

@@ -134,7 +134,8 @@ SPAMM_API int spamm_multiply(spamm_ctx *ctx, const spamm_params *p, const float 
 
 /* The same multiply for operands that already are fp16 (the reference's actual
  * input type, para.h:1, cuSpAMM.cu:486): dAh, dBh are row-major fp16 device
- * arrays.  The norm-map stage then only packs and takes norms. */
+ * arrays, which need begin at no more than a multiple of 2 bytes (of 4: shorter norm-map passes).
+ * The norm-map stage then only packs and takes norms. */
 SPAMM_API int spamm_multiply_f16(spamm_ctx *ctx, const spamm_params *p, const void *dAh, const void *dBh,
                                  float *dC);
 

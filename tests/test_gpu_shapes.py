@@ -573,3 +573,64 @@ def test_passes_over_inputs_beyond_the_cache_line(orc, ctx, tile, half, n):
     ctx.multiply(X, X, tile, tau, a_eq_b=True)
     same(0, X)
     same(1, X)
+
+
+@pytest.mark.parametrize("tile,half,M,K,N", [(32, True, 288, 352, 544), (64, True, 320, 192, 448), (128, True, 384, 256, 640),      # one launch
+                                             (32, True, 4064, 4128, 1056), (64, True, 4032, 4160, 1088), (64, True, 4096, 4096, 576),
+                                             (128, True, 4224, 4096, 1152),
+                                             (32, False, 288, 352, 544), (64, False, 320, 192, 448), (128, False, 384, 256, 640),
+                                             (32, False, 3104, 2848, 1056), (64, False, 3136, 2816, 1088), (64, False, 2816, 8192, 2112)])
+def test_matrices_begin_anywhere(ctx, tile, half, M, K, N):
+    """Operands that begin at any element of a buffer, halves between two 32-bit words among them, and C at any float: bit for bit as where all
+    begin at 256 bytes, in passes of their own, both in one launch, A = B, tau-aware, small and beyond 32 MiB."""
+    import torch
+    tab = np.exp(-0.005 * np.arange(max(M, K, N))).astype(np.float32)
+
+    def filled(rows, cols, seed):
+        X = torch.empty((rows, cols), dtype=torch.float32, device="cuda")
+        ctx.fill_decay(X, tab, seed)
+        return X.half() if half else X
+
+    def at(X, offset):
+        buffer = torch.full((X.numel() + 8,), float("nan"), dtype=X.dtype, device="cuda")
+        view = buffer[offset:offset + X.numel()].view(X.shape)
+        view.copy_(X)
+        return view, buffer
+
+    def state(*roles):
+        return [ctx.get_normmap(r).view(np.uint32) for r in roles] + [ctx.get_fp16(r) for r in roles]
+
+    def same(got, want):
+        assert all(np.array_equal(g, w) for g, w in zip(got, want))
+
+    A, B = filled(M, K, 1), filled(K, N, 2)
+    alone = ctx.normmap_f16 if half else ctx.normmap_f32
+    alone(1, B, tile)
+    alone(0, A, tile)
+    tau = ctx.tau_for_ratio(0.2)[0]
+    C = ctx.multiply(A, B, tile, tau)
+    want, mask = state(0, 1), ctx.get_mask()
+    n = min(M, K)
+    S = A[:n, :n].contiguous()
+    square = ctx.multiply(S, S, tile, tau, a_eq_b=True)
+    want_square = state(0, 1)
+    for a, b, c in ((1, 0, 0), (0, 1, 1), (3, 2, 3), (2, 5, 0)):
+        (Av, _), (Bv, _), (Cv, buffer) = at(A, a), at(B, b), at(torch.empty_like(C), c)
+        assert Av.data_ptr() % 16 == (a * A.element_size()) % 16 and Av.is_contiguous()
+        alone(1, Bv, tile)
+        alone(0, Av, tile)
+        same(state(0, 1), want)
+        ctx.multiply(Av, Bv, tile, tau, C=Cv)
+        same(state(0, 1), want)
+        assert torch.equal(Cv, C) and np.array_equal(ctx.get_mask(), mask)
+        assert buffer[:c].isnan().all() and buffer[c + C.numel():].isnan().all()
+        Cv.fill_(float("nan"))
+        ctx.multiply(Av, Bv, tile, tau, C=Cv, prune=True)
+        assert torch.equal(Cv, C) and np.array_equal(ctx.get_mask(), mask)
+        if not half and max(M * K, K * N) * 2 <= 16 << 20:
+            Cv.fill_(float("nan"))
+            ctx.multiply_noalloc(Av, Bv, tile, tau, Cv)
+            assert torch.equal(Cv, C)
+        Sv, _ = at(S, a)
+        assert torch.equal(ctx.multiply(Sv, Sv, tile, tau, a_eq_b=True), square)
+        same(state(0, 1), want_square)

@@ -237,6 +237,41 @@ def test_lines_of_the_small_kernel_are_by_work_per_cu(run, cus):
     run("multiply_on_a_partition", cus)
 
 
+def passes_over_halves(e, tile, n):
+    h = e.context()
+    memory = ctypes.create_string_buffer(64)
+    start = -(-ctypes.addressof(memory) // 16) * 16
+
+    def kernels(call, *args):
+        e.launches()
+        assert call(h, *args) == 0
+        return [name for name, _ in e.launches() if name.startswith("k_normmap")]
+
+    C = ctypes.c_void_p(start)
+    for a in range(0, 16, 2):
+        A = ctypes.c_void_p(start + a)
+        passes = kernels(e.L.spamm_normmap_f16, 0, A, i64(n), i64(n), tile) + kernels(e.L.spamm_normmap_f16, 1, A, i64(n), i64(n), tile)
+        square = kernels(e.L.spamm_multiply_f16, p(Params(n, n, n, tile, 0.5, 1, 0)), A, A, C)
+        assert passes and square
+        for name in passes + square:
+            assert a % 4 == 0 or "lean" not in name, (name, a)
+        if n * n * 2 <= 32 * MIB:
+            assert a % 4 or all("lean" in name for name in passes)
+        for b in range(0, 16, 2):
+            pair = kernels(e.L.spamm_multiply_f16, p(Params(n, n, n, tile, 0.5, 0, 0)), A, ctypes.c_void_p(start + b), C)
+            assert len(pair) == 1
+            assert (a % 4 == 0 and b % 4 == 0) or "lean" not in pair[0], (pair, a, b)
+            if 2 * n * n * 2 <= 32 * MIB:
+                assert a % 4 or b % 4 or "lean" in pair[0]
+
+
+@pytest.mark.parametrize("n", [256, 1024, 5120])
+@pytest.mark.parametrize("tile", [32, 64, 128])
+def test_halves_between_two_words_are_not_read_by_buffer_loads(run, tile, n):
+    """Buffer loads are of whole 32-bit words: passes that read their input by them take no matrix of halves that begins at an odd half."""
+    run("passes_over_halves", tile, n)
+
+
 if __name__ == "__main__":
     globals()[sys.argv[3]](Engine(*sys.argv[1:3]), *map(int, sys.argv[4:]))
     print("ok")
