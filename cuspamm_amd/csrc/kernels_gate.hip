@@ -539,6 +539,10 @@ struct SuperGrid {
     }
 };
 
+// Offset of a macro tile beyond C in the buffer of kept products, and, doubled (which leaves 31 bits, so it is unsigned), in that of the
+// lists' lengths: neither holds it, and zero comes back.
+constexpr uint32_t NO_MACRO = 0x40000000u;
+
 struct Super {
     uint32_t len, comp, work;       // entries of its macro tiles' lists, computing macro tiles (bit: slot), kept products
 };
@@ -605,9 +609,9 @@ __global__ __launch_bounds__(1024) void k_order(GateBuffers g, int nMacM, int nM
             uint32_t w[SUPER_M], l[SUPER_M];
 #pragma unroll
             for (int a = 0; a < SUPER_M; a++) {
-                const int off = mi0 + a < nMacM && mj < nMacN ? ((mi0 + a) * nMacN + mj) * 4 : 0x40000000;      // beyond C: zero
-                w[a] = __builtin_amdgcn_raw_buffer_load_b32(work_of, off, 0, 0);
-                l[a] = __builtin_amdgcn_raw_buffer_load_b32(count_of, off * 2, 0, 0);
+                const uint32_t off = mi0 + a < nMacM && mj < nMacN ? (uint32_t)((mi0 + a) * nMacN + mj) * 4u : NO_MACRO;
+                w[a] = __builtin_amdgcn_raw_buffer_load_b32(work_of, (int)off, 0, 0);
+                l[a] = __builtin_amdgcn_raw_buffer_load_b32(count_of, (int)(off * 2u), 0, 0);
             }
             Super sp = {0, 0, 0};
 #pragma unroll
@@ -900,13 +904,14 @@ __global__ __launch_bounds__(ORDER_FEW_WAVES * 64) void k_order_few(const int32_
         const __amdgpu_buffer_rsrc_t count_of = __builtin_amdgcn_make_buffer_rsrc((void *)macro_count, 0, n_macro * 8, 0x00020000);
         const int sid = threadIdx.x >> 3, at = threadIdx.x & 7;
         const int origin = sup.origin(sid), mi = (origin >> 16) + (at >> 1), mj = (origin & 0xffff) + (at & 1) * 4;
-        const int first = (mi * nMacN + mj) * 4, room = sid < n_super && mi < nMacM ? nMacN - mj : 0;
+        const uint32_t first = (uint32_t)(mi * nMacN + mj) * 4u;
+        const int room = sid < n_super && mi < nMacM ? nMacN - mj : 0;
         uint32_t w[4], l[4];
 #pragma unroll
         for (int b = 0; b < 4; b++) {
-            const int off = b < room ? first + b * 4 : 0x40000000;
-            w[b] = __builtin_amdgcn_raw_buffer_load_b32(work_of, off, 0, 0);
-            l[b] = __builtin_amdgcn_raw_buffer_load_b32(count_of, off * 2, 0, 0);
+            const uint32_t off = b < room ? first + b * 4u : NO_MACRO;
+            w[b] = __builtin_amdgcn_raw_buffer_load_b32(work_of, (int)off, 0, 0);
+            l[b] = __builtin_amdgcn_raw_buffer_load_b32(count_of, (int)(off * 2u), 0, 0);
         }
         Super sp = {l[0] + l[1] + l[2] + l[3], 0, w[0] + w[1] + w[2] + w[3]};
 #pragma unroll

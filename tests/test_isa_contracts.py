@@ -432,3 +432,28 @@ def test_one_word_kernels_keep_the_same_contracts(tmp_path):
         assert not other and not any(mn.startswith("scratch_") for mn, _, _ in ins), (name, other)
         loads = re.findall(r"s_load_dword(?:x(\d+))?\s+\S+, s\[\d+:\d+\], (0x[0-9a-f]+)", body)
         assert loads and max(int(at, 16) + 4 * int(n or 1) for n, at in loads) <= 128, (name, loads)
+
+
+@pytest.mark.parametrize("src", ["kernels_gate.hip", "kernels_normmap.hip"])
+def test_offsets_that_no_buffer_holds_stay_within_their_type(src, tmp_path):
+    """A lane with nothing to load gets an offset beyond its buffer.  Signed arithmetic on it that leaves 31 bits may be taken by the compiler
+    as never happening, and with it the offset: looked for in the optimised intermediate code, where a value that is one of two has a
+    large constant among them and goes into a signed operation with another constant."""
+    from cuspamm_amd import build
+    out = os.path.join(str(tmp_path), "ir.ll")
+    cmd = [build.HIPCC] + [f for f in build.CFLAGS if f != "-Wall"] + build.EXTRA_FLAGS.get(src, []) + ["-S", "-emit-llvm", "--cuda-device-only",
+                                                                                                    os.path.join(CSRC, src), "-o", out]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert proc.returncode == 0, proc.stdout[-2000:]
+    wrong, selects = [], 0
+    operate = {"add": lambda x, y: x + y, "mul": lambda x, y: x * y, "shl": lambda x, y: x << y}
+    for function in open(out).read().split("\ndefine ")[1:]:
+        chosen = {}
+        for name, rest in re.findall(r"(%\S+) = (?:select|phi) (.*)", function):
+            large = [int(c) for c in re.findall(r"i32 (-?\d{9,})", rest) + re.findall(r"\[ (-?\d{9,}), ", rest)]
+            if large:
+                chosen[name] = large
+        selects += len(chosen)
+        for op, name, c in re.findall(r"= (add|mul|shl) (?:nuw )?nsw i32 (%\S+), (-?\d+)", function):
+            wrong += [(op, v, int(c)) for v in chosen.get(name, []) if not -2 ** 31 <= operate[op](v, int(c)) < 2 ** 31]
+    assert selects and not wrong, wrong
