@@ -1,4 +1,4 @@
-// Device code shared by the multiply kernels (kernels_gemm.hip, kernels_small.hip).
+// Device code shared by the multiply kernels, the gate and the selection of tau (kernels_gemm.hip, kernels_small.hip, kernels_gate.hip, kernels_tau.hip).
 #pragma once
 #include <type_traits>
 #include <utility>

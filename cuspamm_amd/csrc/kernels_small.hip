@@ -11,10 +11,8 @@
 //
 // Two forms: K / tile up to 64 (small_word_body, the list in a register) and beyond (small_unit_body, the list in LDS).
 //
-// A unit's life with its list in LDS, measured on fp16 2048^3 at tile 32, 5 % kept, us: gate 2.0 (most of it the norms' round trip), list 0.3, first
-// stages 0.8, 9 to 14 stages 3.4 to 6, C 1.5.  With 64-bit places, divisions by the grid's sizes, a scan for the one word of 64 k that most lists
-// are, and counts formed behind C's stores it was 1 us longer (whole calls: 256^3 10.5 -> 9.8 us, 1024^3 11.6 -> 10.6, 1056 x 1568 x
-// 1312 16.3 -> 15.5, this one 19.5 -> 18.4, 4096^2 of a band 57.9 -> 56.2).
+// A unit's life with its list in LDS, measured on fp16 2048^3 at tile 32, 5 % kept (which has its list in a register since), us: gate 2.0 (most
+// of it the norms' round trip), list 0.3, first stages 0.8, 9 to 14 stages 3.4 to 6, C 1.5.
 //
 // Of the k loop's 0.285 us per stage on 256 CUs (2048^3 dense) the loads alone take 0.2 (a bare copy of the same panels into
 // LDS, 21 TB/s over the chip), all else without them 0.18; without the MFMAs 0.27, without the LDS reads 0.285.  Two stages
@@ -28,10 +26,10 @@
 // What bounds it: a chain of latencies -- norms in, first stages in, one sync per 32 k,
 // results out -- of which units of 128 (16 KiB a stage, two workgroups per CU, or three) make
 // the k loop shortest and units of 64 spread a small C over more CUs.  Gate, schedule
-// and GEMM as launches of their own -> this kernel, whole multiplies: 256^3 24.6 -> 14.7 us
-// (today, with one launch for both norm-map passes too: 10.3), 1056 x 1568 x 1312 38.2 -> 22.8
-// (17.4), fp16 2048^3 at tile 32, 5 % kept, 38.5 -> 26.3 (21.8), 2048^3 dense 63 -> 38 (36), 1024 rows
-// against a resident 8192^2 50.3 -> 36.5 (35.8).
+// and GEMM as launches of their own -> this kernel, whole multiplies, when it took their place: 256^3 24.6 -> 14.7 us, 1056 x 1568 x
+// 1312 38.2 -> 22.8, fp16 2048^3 at tile 32, 5 % kept, 38.5 -> 26.3, 2048^3 dense 63 -> 38, 1024 rows against a resident 8192^2
+// 50.3 -> 36.5.  With both norm-map passes in one launch, the copies in the memory-side cache and the list in a register they take
+// 8.1, 12.4, 14.4, 33 and 30.5.
 #include "gemm_device.h"
 
 namespace spamm {
@@ -827,24 +825,26 @@ SPAMM_WORD_THREE(128)
 static int64_t per_256_cus(int64_t units, int n_cu) { return (units * 256 + n_cu - 1) / n_cu; }
 static int64_t units_of_128(int64_t M, int64_t N, int n_cu) { return per_256_cus(((M + 127) / 128) * ((N + 127) / 128), n_cu); }
 
-// Unit by units of 128 in C: the wide one from half a unit per CU on.  Resident operands, K = 2048 at tile 32 (64 within
-// 10 %), 2 %, 10 %, 30 % kept and dense, narrow -> wide: 256 units 13.7 -> 12.4, 17.9 -> 15.3, 27.2 -> 20.0, 37.1 -> 24.9 us;
-// 196 units 12.3 -> 12.4, 15.7 -> 15.2, 20.7 -> 19.4, 36.1 -> 23.7; 144 units 10.0 -> 12.2, 13.4 -> 14.5, 17.8 -> 18.5,
-// 28.0 -> 22.9; 128 units 9.9 -> 12.4, 12.8 -> 15.0, 16.0 -> 19.8, 23.8 -> 22.9.  So between 128 and 196 units the line is a
-// choice: a sparse product pays some 2 us there for the 5 to 12 that a dense one, or one of more k, saves (144 units,
-// K = 6144: 30 % kept 28.7 -> 24.7, dense 62.8 -> 47.8).  Below it the narrow one (whole calls, wide -> narrow: 99 units
-// 20.1 -> 18.4, 64 units 15.4 -> 13.1 and, dense, 21.7 -> 20.6).
+// Unit by units of 128 in C: the wide one from half a unit per CU on.  Whole fp16 multiplies of inputs that change, 2 %, 10 %, 30 %
+// kept and dense, narrow -> wide.  K = 2048 at tile 32 (K = 4096 at tiles 64 and 128 alike): 100 units 9.7 -> 11.7, 11.6 -> 14.1, 13.7 -> 17.3, 19.5 ->
+// 21.6 us; 128 units 10.5 -> 12.6, 12.2 -> 14.9, 14.5 -> 18.5, 20.3 -> 22.0; 144 units 10.5 -> 12.3, 12.5 -> 14.5, 16.4 -> 18.0, 24.9 -> 22.1;
+// 196 units 11.7 -> 13.2, 13.5 -> 15.5, 18.2 -> 19.0, 31.4 -> 23.8; 256 units 12.5 -> 13.7, 15.0 -> 16.1, 20.2 -> 20.3, 33.1 -> 26.9.  K = 6144
+// at tile 32: 128 units 23.8 -> 26.1, 27.7 -> 31.4, 32.9 -> 35.5, 53.5 -> 55.6; 144 units 24.3 -> 25.6, 29.3 -> 30.3, 36.8 -> 34.5, 69.8 -> 54.9; 256
+// units 29.8 -> 29.7, 41.1 -> 35.6, 49.4 -> 43.2, 94.1 -> 69.2.  Beyond 128 units, where four narrow ones a unit no longer run at once, two per CU,
+// the line is a choice: a sparse product of few k pays up to 2 us for the 3 to 35 that a dense one, or one of more k, saves.  At 128
+// units themselves, where the line was drawn before the list was a register, the narrow one is ahead by 1 to 4 us.
 static int small_unit(int64_t units128) { return units128 >= 128 ? 128 : 64; }
 
 // Clearly more than two units of 128 per CU: a ring of three stages leaves room for a third workgroup on the CU, whose loads
-// and syncs fill the others' waits.  Ring of four, two workgroups -> this, whole multiplies, fp16: 640 units, K = 2048 at tile
-// 32, 10 % kept 45.8 -> 41.0 us, 40 % 60.2 -> 54.5, dense 75.6 -> 69; 768 units 48.5 -> 44.7, 65.4 -> 58.7, 79.6 -> 75.7; 1024
-// units, 5 % 47.4 -> 45.2, 40 % 75.7 -> 78.7.  From 513 to 600 units, where a second turn of two per CU is short, neither is the
-// better one: over 120 calls (K of 1024 to 4096, all tiles, 3.5 % kept to dense) this takes 0.99 of the time in the geometric
-// mean, 0.85 to 1.16 of it.  Bands, whose few long lists want the longer ring, lose (576 units, K = 2048 at tile 64, 10 %
-// 32.9 -> 38.1 us; 600 units at tile 32, 3.5 % 31.3 -> 34.3), slow decay gains (576 units, 30 % algebraic 50.8 -> 45.0, 550 units,
-// 10 % 42.4 -> 38.9): the host cannot tell them apart, and bands are the usual operands.  A list too long for three in a CU's LDS
-// keeps the ring of four.
+// and syncs fill the others' waits.  Ring of four, two workgroups -> this, whole fp16 multiplies of inputs that change, band of 10 % | 1 / (1 + d)^2,
+// 40 % | dense.  K = 2048 at tile 32: 522 units 24.0 -> 25.3 | 35.6 -> 36.4 | 56.4 -> 53.5 us; 550 units 25.8 -> 24.7 | 38.5 -> 37.3 |
+// 60.5 -> 55.3; 600 units 27.4 -> 26.1 | 43.2 -> 39.6 | 64.2 -> 57.3; 640 units 26.9 -> 27.1 | 47.4 -> 45.0 | 58.6 -> 56.1; 768 units 30.3 -> 29.1 | 50.2 ->
+// 47.1 | 63.6 -> 61.7; 1024 units 36.2 -> 36.5 | 57.0 -> 58.2; 1296 units 47.9 -> 47.2 | 77.2 -> 72.6.  K = 4096 at tile 64: 522 units 38.0 -> 36.5 | 62.1 ->
+// 64.5 | 111 -> 105; 600 units 37.9 -> 36.5 | 68.6 -> 62.8 | 121 -> 109; 768 units 43.6 -> 41.9 | 76.7 -> 71.4 | 118 -> 115; 1024 units 52.8 -> 51.5 | 89.5 ->
+// 95.5.  K = 8192 at tile 128: 576 units 59.2 -> 62.5 | 102 -> 98.8 | 202 -> 195; 640 units 64.8 -> 67.5 | 114 -> 111 | 209 -> 205; 768 units 74.5 -> 70.8 | 126 -> 115 |
+// 222 -> 219.  From 513 to some 540 units, where a second turn of two per CU is short, neither is the better one, and bands, whose few
+// long lists want the longer ring, lose up to 1.5 us; from 550 on this one is ahead but for bands at tile 128.  The line is at 600 from when the
+// list was not in a register and bands lost up to there.  A list too long for three in a CU's LDS keeps the ring of four.
 static bool small_three(int64_t units128, int64_t nbK) {
     return units128 > 600 && 3 * (small_lds_bytes_(16384, 3, nbK) + 2048) <= 160 * 1024;
 }
@@ -905,42 +905,38 @@ hipError_t small_init() {
     return small_attrs<128>();
 }
 
-// Whole multiplies on fp16 operands, gate, schedule and GEMM apart -> this kernel, by units of 128 in C; "m" is the number of
-// macro tiles (four units each), of which k_gemm runs 256 at a time.
+// Gate, schedule and GEMM apart -> this kernel, by units of 128 in C; "m" is the number of macro tiles (four units each), of which k_gemm runs
+// 256 at a time.  Whole fp16 multiplies, three sets of operands and workspaces in turn on one stream; "from HBM": on operands converted
+// before, 768 MiB of other writes since.
 //
-// tau > 0, at most 6 units per CU; 1 / (1 + d)^2, 10 % | 40 % kept, passes and all (their copies lie in the memory-side cache).  K =
-// 2048 at tile 32: 768 units 33.1 -> 28.4 | 44.4 -> 41.5 us; 840 units 37.4 -> 30.3 | 47.3 -> 44.2; 1024 units 40.3 -> 32.9 | 50.7 ->
-// 52.8; 1296 units 46.5 -> 41.3 | 58.9 -> 66.1; 1444 units 48.7 -> 43.5 | 64.0 -> 74.4.  K = 4096 at tile 64: 768 units 46.0 -> 41.7 |
-// 67.3 -> 72.4; 840 units 52.3 -> 44.8 | 76.0 -> 79.6; 1024 units 55.0 -> 50.1 | 81.9 -> 91.6; 1296 units 63.1 -> 61.7 | 98.1 ->
-// 117.2; 1444 units 70.1 -> 66.7 | 108.6 -> 129.3.  K = 8192 at tile 128: 840 units 76.0 -> 74.9 | 120.6 -> 146.6; 1024 units 84.3 ->
-// 86.5 | 131.1 -> 173.5; 1296 units 100.9 -> 103.5 | 163.8 -> 221.1.  What decides is how many macro tiles compute, which the host
-// does not know: the fewer, the more CUs k_gemm leaves idle.  Operands that lie there already and come from HBM (converted before,
-// other work since), where three workgroups per CU hide more of the latency: 1024 units, K = 4096 94.8 -> 76.7 | 124.3 -> 112.3,
-// K = 8192 102.7 -> 84.4 | 156.8 -> 157.5; 1296 units, K = 8192 136.4 -> 94.7 | 227.1 -> 188.3.
-// In the one round that k_gemm fills (833 to 1024 units) K ends at 8192, where neither gains any more, few kept with the
-// passes or many from HBM.  Beyond it, 5 % | 40 %: 840 units, K = 16384 112.4 -> 110.5 | 214.3 -> 309.4 and, from HBM, 100.7 -> 78.0 |
-// 237.7 -> 263.9; 1024 units, K = 12288 100.6 -> 102.3 | 186.5 -> 290.3 and 101.3 -> 83.7 | 198.5 -> 225.3, K = 16384 129.7 -> 134.6 |
-// 237.8 -> 353.1 and 114.0 -> 94.3 | 251.9 -> 287.6.
-// Beyond 6 units, 10 % | 40 %, with the passes: 1600 units, K = 3072 88.6 -> 76.1 | 131 -> 150; 1936 units, K = 5120 114 -> 102 |
-// 203 -> 218; 2304 units, K = 5120 130 -> 113 | 228 -> 231, and 30 % at K = 8192 268 -> 284.
+// tau > 0, at most 6 units per CU; exponential decay, 5 % kept | 1 / (1 + d)^2, 10 % | 25 % | 40 %.  K = 2048 at tile 32: 640 units 40.3 -> 24.4 |
+// 43.3 -> 27.4 | 55.4 -> 36.0 | 63.4 -> 45.0 us; 840 units 45.0 -> 28.6 | 48.7 -> 33.7 | 62.5 -> 44.1 | 66.3 -> 50.6; 1024 units 48.0 -> 29.7 | 52.0 ->
+// 35.6 | 65.8 -> 48.1 | 66.5 -> 58.5; 1444 units 53.7 -> 43.3 | 58.3 -> 49.6 | 71.0 -> 67.9 | 72.6 -> 78.4.  K = 4096 at tile 64: 840 units 56.6 ->
+// 39.3 | 57.1 -> 47.3 | 72.7 -> 65.2 | 83.3 -> 81.2; 1024 units 60.8 -> 43.2 | 60.3 -> 53.1 | 79.4 -> 77.3 | 93.0 -> 95.5; 1296 units 62.2 -> 49.7 |
+// 80.3 -> 64.3 | 106 -> 91 | 122 -> 122; 1444 units 66.2 -> 54.9 | 85.4 -> 70.8 | 112 -> 98 | 131 -> 126.  K = 8192 at tile 64: 840 units 80.8 -> 63.6 |
+// 88.3 -> 78.9 | 113 -> 112 | 135 -> 136; 1024 units 84.6 -> 71.8 | 94.7 -> 91.4 | 121 -> 126 | 147 -> 153; 1296 units 92.2 -> 85.6 | 124 -> 114 | 173 -> 164 |
+// 219 -> 200; 1444 units 97.5 -> 93.4 | 129 -> 123 | 178 -> 172 | 224 -> 222.  From HBM, K = 8192 at tile 64: 1024 units 57 -> 47 | 72 -> 68 | 99 -> 101 | 123 ->
+// 138; 1296 units 62 -> 57 | 94 -> 79 | 134 -> 128 | 183 -> 168.
+// In the one round that k_gemm fills (833 to 1024 units) K ends at 8192, where a quarter kept is even: beyond, 5 % | 10 % | 40 %: 840 units, K = 12288
+// 112 -> 95 | 118 -> 111 | 180 -> 207, K = 16384 138 -> 123 | 146 -> 138 | 233 -> 266; 1024 units, K = 12288 119 -> 107 | 130 -> 129 | 192 -> 217, K = 16384
+// 149 -> 136 | 165 -> 164 | 260 -> 297.  Beyond 6 units per CU: 1600 units, K = 3072 60.6 -> 51.6 | 70.3 -> 62.6 | 113 -> 116; 1936 units, K = 5120 86 -> 78 |
+// 107 -> 102 | 179 -> 192; 2304 units, K = 5120 94 -> 85 | 127 -> 118 | 200 -> 223, K = 8192 130 -> 130 | 179 -> 178 | 324 -> 331.
 //
-// tau <= 0, everything is kept and the rounds are known.  Tile 64, whole multiplies | operands from HBM, K = 2048 and 4096.  With m = 160
-// to 192 a round is a third empty: 640 units 64.5 -> 53.8 | 108.1 -> 79.4 and 111.8 -> 112.1 | 152.3 -> 124.8; 704 units 64.9 -> 59.7 |
-// 108.9 -> 81.7 and 116.7 -> 119.6 | 153.4 -> 130.3; 768 units 62.0 -> 64.5 | 108.4 -> 86.7 and 115.2 -> 124.8 | 153.5 -> 134.7; but 600
-// units 101.9 -> 107.7 | 152.6 -> 130.6 and 841 units 63.4 -> 74.8 | 109.0 -> 99.1 and 117.8 -> 157.3 | 153.4 -> 156.8.  With m = 257 to 324
-// a second round is mostly empty, which pays from HBM only: 1088 units, K = 1024 56.6 -> 47.7 | 113.6 -> 76.4, K = 2048 80.4 -> 91.2 |
-// 154.1 -> 113.2, K = 4096 145.4 -> 175.7 | 231.3 -> 182.7, K = 8192 268.4 -> 397.2 | 383.2 -> 332.7; 1296 units 91.4 -> 108.0 | 154.7 ->
-// 121.7 and 165.5 -> 236.7 | 230.9 -> 205.7; 1444 units 104.3 -> 121.8 | 157.6 -> 133.3 and 184.3 -> 257.9 | 236.9 -> 220.9.  (The lines were
-// drawn when every multiply read its operands from HBM; whether the passes have just run is not asked here.)
-// Gate and multiply called apart (`stages`) form mask and list twice, which costs less than the schedule does up to 1200 units
-// (fp32 passes, tau to a fraction, both stages, 10 % | 40 % kept: 1120 units, K = 2048 at tile 32 98.3 -> 89.8 | 109.4 -> 109.7 us, K =
-// 4096 at tile 64 122.0 -> 110.6 | 150.5 -> 149.3; 1200 units 97.2 -> 92.4 | 105.9 -> 113.8, 118.7 -> 114.2 | 150.8 -> 156.9; but 1444
-// units 125.6 -> 123.8 | 159.8 -> 175.9).  In the round that k_gemm fills (833 to 1024 units) it pays for one word of 64 k and up to
-// K = 4096 (10 % | 40 % | 75 %: 840 units, K = 2048 at tile 32 98.0 -> 87.4 | 105.6 -> 100.5 | 107.5 -> 112.2; 1024 units 101.7 -> 91.6 |
-// 110.2 -> 108.4 | 112.7 -> 121.9, K = 4096 at tile 64 118.8 -> 106.5 | 138.9 -> 138.5 | 161.0 -> 167.5, at tile 128 116.1 -> 103.7 |
-// 137.7 -> 133.8 | 160.7 -> 163.4); beyond that few kept still gain, a quarter is even, and more lose more (10 % | 25 % | 50 %: 1000
-// units at tile 32, K = 4128 120.5 -> 112.7 | 131.1 -> 132.5 | 147.1 -> 165.2; 10 % | 50 % at tile 128, 1024 units, K = 8192 157.1 -> 146.8 |
-// 209.0 -> 224.3; passes and stages alone, 1024 units at tile 64, K = 8192, 10 % | 40 % 86.0 -> 91.9 | 129.7 -> 169.6).
+// tau <= 0, everything is kept and the rounds are known.  Tile 64, K = 1024 | 2048 | 4096 | 8192.  With m = 160 to 192 a round is a third empty: 640
+// units 42.2 -> 31.9 | 66.3 -> 55.2 | 116 -> 108 | 210 -> 209; 704 units 43.8 -> 33.3 | 68.3 -> 57.6 | 120 -> 111 | 215 -> 211; 768 units 44.6 -> 35.2 |
+// 70.6 -> 60.0 | 123 -> 114 | 220 -> 218; but 600 units 41.0 -> 35.9 | 64.5 -> 62.2 | 112 -> 122 | 206 -> 233; 841 units 48.4 -> 43.2 | 75.4 -> 77.8 | 131 -> 157 |
+// 237 -> 298; 1024 units 52.0 -> 44.1 | 82.4 -> 77.2 | 141 -> 147 | 247 -> 281.  With m = 257 to 324 a second round is mostly empty: 1088 units 74.8 -> 49.2 | 121 ->
+// 91 | 210 -> 168 | 383 -> 321; 1296 units 77.9 -> 58.5 | 125 -> 108 | 216 -> 200 | 398 -> 394; 1444 units 78.7 -> 60.0 | 127 -> 111 | 223 -> 208 | 407 -> 424.  (The
+// lines were drawn by K = 2048 and more, and by the schedule before k_order_few, which took 4 us more of the other side: K = 1024 gains at every
+// one of these sizes now, and so do 520 and 576 units: 62.1 -> 54.9 and 62.5 -> 55.3 at K = 2048, even at 8192.)
+//
+// Gate and multiply called apart (`stages`) form mask and list twice, which costs less than the schedule does (fp32 passes, tau to a fraction, both
+// stages, 1 / (1 + d)^2, 10 % | 25 % | 40 % kept): 1120 units, K = 2048 at tile 32 104 -> 83 | 120 -> 94 | 120 -> 103, K = 4096 at tile 64 130 -> 105 | 153 -> 129 |
+// 170 -> 149; 1200 units 106 -> 86 | 120 -> 99 | 120 -> 109 and 134 -> 111 | 150 -> 132 | 173 -> 155; 1444 units 110 -> 94 | 122 -> 113 | 125 -> 123 and 141 ->
+// 119 | 167 -> 146 | 187 -> 174.  In the round that k_gemm fills: 840 units, K = 2048 at tile 32 99.7 -> 77.4 | 114 -> 88 | 118 -> 95, K = 4128 117 -> 103 | 132 ->
+// 119 | 144 -> 138, K = 8192 at tile 64 152 -> 137 | 177 -> 170 | 196 -> 194; 1024 units 103 -> 80 | 119 -> 93 | 118 -> 103, 123 -> 111 | 142 -> 134 | 154 -> 152 and 162 ->
+// 152 | 186 -> 183 | 212 -> 213.  (Its lines -- 1200 units, and in that round one word of 64 k and K = 4096 -- are from before the list was a register and
+// the gate of few instructions; up to 1536 units and K = 8192 this kernel is ahead, or even, throughout.)
 bool small_fits(int64_t M, int64_t K, int64_t N, int tile, float tau, bool stages, int n_cu) {
     const int64_t units128 = units_of_128(M, N, n_cu), m = per_256_cus(((M + 255) / 256) * ((N + 255) / 256), n_cu);
     if (K / tile > SMALL_MAX_NBK || n_cu > 256) return false;
