@@ -272,6 +272,42 @@ def test_halves_between_two_words_are_not_read_by_buffer_loads(run, tile, n):
     run("passes_over_halves", tile, n)
 
 
+def forms_of_the_one_launch_kernel(e, tile):
+    h = e.context()
+    X = ctypes.create_string_buffer(16)
+    for M, N, name, unit in ((1024, 1024, "k_small", 64), (2048, 2048, "k_small", 128), (3072, 3584, "k_small_three", 128)):
+        for k_tiles in (1, 63, 64, 65, 128):
+            e.launches()
+            assert e.L.spamm_multiply(h, p(Params(M, k_tiles * tile, N, tile, 0.5, 0, 0)), X, X, X) == 0
+            full = [item.rsplit(" ", 1)[0] for item in e.fake.fake_launches().decode().split(";")[:-1] if "k_small" in item]
+            sizes = "ILi%dELi%dE" % (tile, unit)
+            word = "_ZN5spamm%d%sENS_8WordArgs%sEE" % (len(name), name, sizes)
+            general = "_ZN5spamm%d%s%s" % (len(name), name, sizes if unit == 64 or name == "k_small" else "ILi%dE" % tile)
+            assert len(full) == 1 and full[0].startswith(word if k_tiles <= 64 else general), (full, k_tiles)
+
+
+@pytest.mark.parametrize("tile", [32, 64, 128])
+def test_the_list_is_a_register_up_to_one_word_of_k_tiles(run, tile):
+    """Both forms of the one-launch kernel go by one name and give the same bits: which of them ran shows in its arguments."""
+    run("forms_of_the_one_launch_kernel", tile)
+
+
+def forms_of_the_gate(e, nbM, nbK, nbN, tile, chunks, few):
+    h = e.context()
+    maps = ctypes.create_string_buffer(4 * max(nbM, nbN) * nbK)
+    assert e.L.spamm_set_normmaps(h, maps, maps, i64(nbM), i64(nbK), i64(nbN), tile) == 0
+    e.launches()
+    assert e.L.spamm_gate(h, ctypes.c_float(0.5)) == 0
+    assert [name for name, _ in e.launches()] == ["k_gate_chunks" if chunks else "k_gate", "k_order_few" if few else "k_order"]
+
+
+@pytest.mark.parametrize("shape", [(512, 1, 16, 128, 0, 1), (513, 1, 16, 128, 0, 0), (16, 1, 1024, 128, 0, 0), (2048, 2, 64, 32, 0, 1), (2049, 2, 64, 32, 0, 0),
+                                   (8, 19392, 8, 32, 0, 1), (8, 19393, 8, 32, 1, 1), (4, 65535, 4, 64, 0, 1), (2, 65535, 2, 128, 0, 1)])
+def test_lines_of_gate_and_schedule(run, shape):
+    """64 super tiles of C are a wave's lanes; a macro tile's sets of k fill a CU's LDS up to 19392 k tiles of 32, and fit at the others."""
+    run("forms_of_the_gate", *shape)
+
+
 if __name__ == "__main__":
     globals()[sys.argv[3]](Engine(*sys.argv[1:3]), *map(int, sys.argv[4:]))
     print("ok")
