@@ -789,8 +789,9 @@ __device__ __forceinline__ void small_word_body(const unsigned char *pA, const u
 template <int U>
 static constexpr int WORD_RING = U == 128 ? 4 : 5;
 
-// The arguments, in the order of their use; a kernel for each tile size and unit (functions of the names of the other form's templates: whoever
-// lists a call's kernels sees the one-launch kernel, and three to a CU).
+// The arguments, in the order of their use; a kernel for each tile size and unit.  They are functions of the names of the other form's templates, so
+// that whoever lists a call's kernels sees the one-launch kernel, and three to a CU; B and U tell them apart, by which a list of full names shows
+// the form.
 template <int B, int U>
 struct WordArgs {
     const unsigned char *pA, *pB;
