@@ -694,17 +694,17 @@ __global__ __launch_bounds__(256) void k_fill_decay(float *__restrict__ X, int64
 constexpr unsigned NARROW_STRIPS = 512;     // of 256 columns, in a launch: two per CU
 
 // Which of a pass's accesses leave their lines in the 256 MB memory-side cache.  Whole calls on three sets of operands and
-// workspaces in turn, so that nothing of a call is there when the set comes round again.
+// workspaces in turn, on one stream, so that nothing of a call is there when the set comes round again; bands, 10 % kept.
 // Copies, written through (sc1) instead of non-temporally up to 448 MiB an operand: the multiply reads them, or what of them
-// still lies there, from that cache.  1056 x 1568 x 1312 17.4 -> 17.0 us, 2048^3 24.7 -> 23.0, 3072^3 47.0 -> 41.7, 4096^3 76 -> 64,
-// 6144^3 179 -> 169, 7168^3 238 -> 219, dense 8192^3 911 -> 888, 10240^3 513 -> 480, 12288^3 728 -> 706; fp16 4096^3 69.4 -> 56.8,
-// 8192^3 270 -> 257, 10048^3 425 -> 418, 14336^3 912 -> 890; A = B 4096^2 66 -> 57, 7168^2 202 -> 182, 9216^2 332 -> 312.  Beyond, the
-// copies drive each other out: 16384^3 1205 on both sides, tau-aware 1252 -> 1274; 20032^3 2052 -> 2067, tau-aware 1929 -> 1966.
+// still lies there, from that cache.  1056 x 1568 x 1312 13.2 -> 12.3 us, 2048^3 19.4 -> 18.2, 3072^3 43.6 -> 37.6, 4096^3 71 -> 59,
+// 6144^3 168 -> 157, 7168^3 225 -> 202, dense 8192^3 884 -> 865, 10240^3 492 -> 459, 12288^3 703 -> 673; fp16 4096^3 61 -> 50,
+// 8192^3 224 -> 209, 10048^3 402 -> 371, 14336^3 876 -> 844; A = B 4096^2 63 -> 51, 7168^2 192 -> 171, 9216^2 320 -> 297.  Beyond, the
+// copies drive each other out: 16384^3 1309 -> 1297, tau-aware 1206 -> 1213; 20032^3 2195 -> 2210, tau-aware 2013 -> 2012.
 // Strips of nothing but zeros, most of a narrow band's operands, are written past it all the same: left out of that rule, and
-// then with it, 8192^3 of a band 278 -> 276 -> 261, A = B 235 -> 237 to 246 -> 224, 9216^2 332 -> 317 -> 309.
-// Input, by ordinary loads up to 32 MiB a launch: a producer's output of that size may be there.  2048^3 23.0 -> 21.8, fp16
-// 20.9 -> 19.6, 1056 x 1568 x 1312 17.0 -> 16.3, 1024 rows against a resident 8192^2 34.6 -> 33.1; beyond it takes the copies'
-// place (3072^3 41.8 -> 45.0, 4096^3 63.9 -> 69.3).
+// then with it, by the strips before the lean ones, 8192^3 of a band 278 -> 276 -> 261, A = B 235 -> 237 to 246 -> 224, 9216^2 332 -> 317 -> 309.
+// Input, by ordinary loads up to 32 MiB a launch: a producer's output of that size may be there.  2048^3 19.4 -> 18.2, fp16
+// 16.8 -> 15.4, 1056 x 1568 x 1312 13.1 -> 12.2; beyond it takes the copies' place (4096^3 58.8 -> 61.3, 6144^3 157 -> 163, 7168^3 203 ->
+// 226, 8192^3 248 -> 267; fp16 4096^3 49.4 -> 48.6, 8192^3 208 -> 217).
 constexpr int64_t KEEP_INPUT_MAX = 32ll << 20, KEEP_COPY_MAX = 448ll << 20;
 static bool keep_input(int64_t bytes) { return bytes <= KEEP_INPUT_MAX; }
 static bool keep_copy(int64_t bytes) { return bytes <= KEEP_COPY_MAX; }
