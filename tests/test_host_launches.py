@@ -5,6 +5,7 @@ import os
 import re
 import subprocess
 import sys
+import time
 
 import pytest
 
@@ -306,6 +307,23 @@ def forms_of_the_gate(e, nbM, nbK, nbN, tile, chunks, few):
 def test_lines_of_gate_and_schedule(run, shape):
     """64 super tiles of C are a wave's lanes; a macro tile's sets of k fill a CU's LDS up to 19392 k tiles of 32, and fit at the others."""
     run("forms_of_the_gate", *shape)
+
+
+def time_looked_for_a_result(e):
+    h = e.context()
+    maps = ctypes.create_string_buffer(4 * 64 * 64)
+    assert e.L.spamm_set_normmaps(h, maps, maps, i64(64), i64(64), i64(64), 32) == 0
+    times = []
+    for _ in range(20):
+        start = time.perf_counter()
+        assert e.L.spamm_count_kept(h, f64(0.5), p(i64()), p(f64())) == -3               # (no kernel writes it: the runtime says the stream has ended)
+        times.append(time.perf_counter() - start)
+    assert min(times) >= 100e-6, "%.1f us" % (min(times) * 1e6)
+
+
+def test_a_result_is_looked_for_some_100_us_before_the_stream_is_asked(run):
+    """Whatever the core: asking the stream costs 6 us more, and most calls that wait have their result after 10 to 60."""
+    run("time_looked_for_a_result")
 
 
 if __name__ == "__main__":
